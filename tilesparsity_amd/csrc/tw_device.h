@@ -14,6 +14,9 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 #define TW_LDS(T) __attribute__((address_space(3))) T *
 #define TW_GLOBAL(T) __attribute__((address_space(1))) T *
@@ -34,6 +37,11 @@ template <> struct Elem<TW_F16> {
     {
         return __builtin_bit_cast(uint16_t, (_Float16)f);
     }
+    // two neighbours in one register: v_cvt_pk_f16_f32, nearest even
+    static __device__ __forceinline__ uint32_t to_bits2(float lo, float hi)
+    {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), f16x2));
+    }
     static __device__ __forceinline__ float from_bits(uint16_t h)
     {
         return (float)__builtin_bit_cast(_Float16, h);
@@ -48,6 +56,10 @@ template <> struct Elem<TW_BF16> {
     static __device__ __forceinline__ uint32_t to_bits(float f)
     {
         return __builtin_bit_cast(uint16_t, (__bf16)f); // v_cvt_pk_bf16_f32, nearest even
+    }
+    static __device__ __forceinline__ uint32_t to_bits2(float lo, float hi)
+    {
+        return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
     }
     static __device__ __forceinline__ float from_bits(uint16_t h)
     {
@@ -82,14 +94,18 @@ __device__ __forceinline__ float tw_activate(float v, int act)
 {
     if (act == TW_ACT_RELU)
         return v > 0.0f ? v : 0.0f;
-    // tanh(u) = 1 - 2 / (exp(2u) + 1) with the hardware exponential and reciprocal (1 ulp each):
-    // exact limits at +-inf, ~1e-6 relative error in between, far below the 16-bit rounding
+    // v_exp_f32 (a power of two) and v_rcp_f32, 1 ulp each, with log2(e) folded into the constants:
+    // exact limits at +-inf, ~1e-6 relative error in between, far below the 16-bit rounding.  An
+    // epilogue is bound by these instructions once its stores are not (33.5 M GELUs are 0.5 M
+    // wave-instructions of each kind, a quarter-rate one taking 16 cycles), so GELU is
+    //   0.5 v (1 + tanh u) = v / (1 + exp(-2u)),  u = sqrt(2/pi) (v + 0.044715 v^3):
+    // five full-rate instructions and the two quarter-rate ones.
     if (act == TW_ACT_GELU) {
-        const float u = 0.7978845608028654f * (v + 0.044715f * v * v * v);
-        return v - v * __builtin_amdgcn_rcpf(__expf(2.0f * u) + 1.0f); // 0.5 v (1 + tanh u)
+        const float t = v * __builtin_fmaf(-0.1029432396f, v * v, -2.302208198f); // -2u log2(e)
+        return v * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
     }
     if (act == TW_ACT_TANH)
-        return 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * v) + 1.0f);
+        return 1.0f - 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(2.885390082f * v) + 1.0f);
     return v;
 }
 // the same for a handful of values with the test of `act` outside the loop over them

@@ -472,10 +472,8 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN * WGS) / 4)
 #pragma unroll
                     for (int r4 = 0; r4 < 4; ++r4) {
                         u32x2 pk;
-                        pk.x = E::to_bits(scale * acc[mi][ni][r4 * 4 + 0]) |
-                               (E::to_bits(scale * acc[mi][ni][r4 * 4 + 1]) << 16);
-                        pk.y = E::to_bits(scale * acc[mi][ni][r4 * 4 + 2]) |
-                               (E::to_bits(scale * acc[mi][ni][r4 * 4 + 3]) << 16);
+                        pk.x = E::to_bits2(scale * acc[mi][ni][r4 * 4 + 0], scale * acc[mi][ni][r4 * 4 + 1]);
+                        pk.y = E::to_bits2(scale * acc[mi][ni][r4 * 4 + 2], scale * acc[mi][ni][r4 * 4 + 3]);
                         *reinterpret_cast<u32x2 *>(smem + j * CPITCH + mloc + r4 * 8) = pk;
                     }
                 }
@@ -1344,8 +1342,8 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                                         for (int e = 0; e < 4; ++e)
                                             v[e] = tw_fp32_value(tw_activate(scale * acc[mi][ni][r4 * 4 + e] + bj, ACT));
                                         u32x2 pk;
-                                        pk.x = E::to_bits(v[0]) | (E::to_bits(v[1]) << 16);
-                                        pk.y = E::to_bits(v[2]) | (E::to_bits(v[3]) << 16);
+                                        pk.x = E::to_bits2(v[0], v[1]);
+                                        pk.y = E::to_bits2(v[2], v[3]);
                                         *reinterpret_cast<u32x2 *>(ctile + j * CPITCH + mloc + r4 * 8) = pk;
                                     }
                                 }
@@ -1375,10 +1373,8 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
 #pragma unroll
                                 for (int r4 = 0; r4 < 4; ++r4) {
                                     u32x2 pk;
-                                    pk.x = E::to_bits(scale * acc[mi][ni][r4 * 4 + 0]) |
-                                           (E::to_bits(scale * acc[mi][ni][r4 * 4 + 1]) << 16);
-                                    pk.y = E::to_bits(scale * acc[mi][ni][r4 * 4 + 2]) |
-                                           (E::to_bits(scale * acc[mi][ni][r4 * 4 + 3]) << 16);
+                                    pk.x = E::to_bits2(scale * acc[mi][ni][r4 * 4 + 0], scale * acc[mi][ni][r4 * 4 + 1]);
+                                    pk.y = E::to_bits2(scale * acc[mi][ni][r4 * 4 + 2], scale * acc[mi][ni][r4 * 4 + 3]);
                                     *reinterpret_cast<u32x2 *>(ctile + j * CPITCH + mloc + r4 * 8) = pk;
                                 }
                             }
@@ -1773,13 +1769,9 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
             tw_activate_all(v, p.act); // the test of the activation outside the loop over the elements
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
-                uint32_t h[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    h[e] = E::to_bits(tw_fp32_value(v[r4 * 4 + e]));
                 u32x2 pk;
-                pk.x = h[0] | (h[1] << 16);
-                pk.y = h[2] | (h[3] << 16);
+                pk.x = E::to_bits2(tw_fp32_value(v[r4 * 4]), tw_fp32_value(v[r4 * 4 + 1]));
+                pk.y = E::to_bits2(tw_fp32_value(v[r4 * 4 + 2]), tw_fp32_value(v[r4 * 4 + 3]));
                 *reinterpret_cast<u32x2 *>(cst + j * CP + mloc + r4 * 8) = pk;
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -2129,11 +2121,10 @@ __global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const 
             for (int e = 0; e < 8; ++e)
                 v[e] += out_bias;
             tw_activate_all(v, p.act);
-            uint32_t h[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                h[e] = E::to_bits(tw_fp32_value(v[e]));
-            store_chunk(dst, u32x4{h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)},
+                v[e] = tw_fp32_value(v[e]);
+            store_chunk(dst, u32x4{E::to_bits2(v[0], v[1]), E::to_bits2(v[2], v[3]), E::to_bits2(v[4], v[5]), E::to_bits2(v[6], v[7])},
                         m0 + m8, m_end, false);
         }
     }

@@ -275,13 +275,9 @@ __global__ void __launch_bounds__(64 * kBsWaves, 4)
         for (int mi = 0; mi < 2; ++mi) {
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
-                uint32_t h[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    h[e] = E::to_bits(tw_fp32_value(acc[mi][r4 * 4 + e]));
                 u32x2 pk;
-                pk.x = h[0] | (h[1] << 16);
-                pk.y = h[2] | (h[3] << 16);
+                pk.x = E::to_bits2(tw_fp32_value(acc[mi][r4 * 4]), tw_fp32_value(acc[mi][r4 * 4 + 1]));
+                pk.y = E::to_bits2(tw_fp32_value(acc[mi][r4 * 4 + 2]), tw_fp32_value(acc[mi][r4 * 4 + 3]));
                 *reinterpret_cast<u32x2 *>(cst + j * kBsCPitch + mi * 32 + (lane >> 5) * 4 + r4 * 8) = pk;
             }
         }
