@@ -87,6 +87,31 @@ def test_mix_ties_and_extremes(twprune, po):
             assert np.array_equal(a, b), (sp, g1)
 
 
+@pytest.mark.parametrize("values", ["normal", "few_values", "mostly_zero", "extreme_scales"])
+def test_mix_selection_narrowed_by_a_sample(twprune, po, values):
+    """Enough elements for the sampled bracket (more than 2^17): it holds the threshold ("normal"), or
+    it cannot be narrow because the values around the threshold repeat ("few_values",
+    "mostly_zero") and the selection walks all elements; squares that leave the normal range
+    ("extreme_scales") take the square root.  Masks are integers: bit for bit the oracle's."""
+    rng = np.random.default_rng(43)
+    shapes = [(577, 300), (64, 1000), (33, 7)]     # whole items, ragged ones, a layer off 16 bytes
+    w = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    if values == "few_values":
+        w = [(np.round(x * 2) / 2).astype(np.float32) for x in w]
+    elif values == "mostly_zero":
+        w = [np.where(rng.random(x.shape) < 0.9, 0, x).astype(np.float32) for x in w]
+    elif values == "extreme_scales":
+        w = [(x * 10.0 ** rng.integers(-25, 18, x.shape)).astype(np.float32) for x in w]
+    scores = twprune.img2col_forward(w)
+    masks = [rng.random(s) < 0.3 for s in shapes]
+    for g1 in (5, 0.01, 50, 100):
+        want, thr = po.tw_mix_fn(scores, g1, masks)
+        got = twprune.tw_mix_fn(scores, g1, masks)
+        assert np.float64(thr) == twprune.tw_mix_fn.last_threshold, (values, g1)
+        for a, b in zip(want, got):
+            assert np.array_equal(a, b), (values, g1)
+
+
 def test_mix_error_paths(tw, twprune):
     with pytest.raises(tw.TwError):
         twprune.tiled_wise_1d_mix([np.ones((4, 4), np.float32)], 50, 2, 120)   # percentile < 0

@@ -140,6 +140,21 @@ def test_wide_tiles_use_the_recursive_sum(twprune, po):
         assert np.array_equal(want[0], got[0]), g
 
 
+@pytest.mark.parametrize("shapes, g", [
+    ([(33, 7 + 5 * i) for i in range(70)], 16),       # more layers than a wave's lanes, rows off 16 bytes
+    ([(40, 5000), (31, 260)], 4500),                  # sums of many blocks; a remainder of rows
+    ([(520, 13000)], 128),                            # more columns than the column stage keeps in LDS
+])
+def test_layer_and_tile_table_edges(twprune, po, shapes, g):
+    rng = np.random.default_rng(25)
+    scores = twprune.img2col_forward([rng.standard_normal(s).astype(np.float32) for s in shapes])
+    for a, b in zip(po.tiled_wise_1d(scores, 60, g)[0], twprune.tiled_wise_1d(scores, 60, g)):
+        assert np.array_equal(a, b)
+    want = po.tiled_wise_2d(scores, 60, g)[0]
+    for a, b in zip(want, twprune.tiled_wise_2d(scores, 60, g)):
+        assert np.array_equal(a, b)
+
+
 def test_masks_feed_plans(tw, twprune, po, oracle):
     """1-D masks go through tw_plan_from_mask, 2-D masks through tw_plan_from_mask_tiles with
     the kept-column tile table; the plans hold the lists the oracle derives from the mask."""

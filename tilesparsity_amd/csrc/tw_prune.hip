@@ -17,7 +17,7 @@
 // would not do: their bodies live in a header outside the pragma and are fused after inlining.
 // sqrtf and the division are the compiler's correctly rounded ones (the __fsqrt_rn / __fdiv_rn
 // intrinsics map to the approximate hardware instructions).
-#include "tw_internal.h"
+#include "tw_device.h"
 
 #include <cmath>
 #include <cstring>
@@ -27,170 +27,293 @@
 
 namespace tw {
 
-__device__ __forceinline__ float sq_term(const float *x, const uint8_t *keep, int i)
-{
-    const float v = (!keep || keep[i]) ? x[i] : 0.0f;
-    return v * v;
-}
+// A pointer that comes out of a table in memory is not known to point to global memory, and a load
+// through it is a flat one, which waits for LDS as well.
+template <class T> __device__ __forceinline__ TW_GLOBAL(T) as_global(T *p) { return (TW_GLOBAL(T))p; }
 
-// NumPy's pairwise sum for n <= 128 terms, by a group of 8 adjacent lanes: lane j keeps NumPy's
-// running sum r[j] (terms j, j+8, j+16, ...), the three shuffle steps are NumPy's
+// NumPy's pairwise sum of the squares of n <= 128 terms, by a group of 8 adjacent lanes: lane j keeps
+// NumPy's running sum r[j] (terms j, j+8, j+16, ...), the three shuffle steps are NumPy's
 // ((r0+r1)+(r2+r3)) + ((r4+r5)+(r6+r7)), lane 0 then adds the n % 8 trailing terms.  The result
-// is valid in lane 0 of the group.
-__device__ float pairwise_block(const float *x, const uint8_t *keep, int n, int l8)
+// is valid in lane 0 of the group.  All reads leave before the chain of additions starts.
+__device__ __forceinline__ float pairwise_block(const float *x, int n, int l8)
 {
     if (n < 8) {
         float r = 0.0f;
         for (int i = 0; i < n; ++i)
-            r = r + sq_term(x, keep, i);
+            r = r + x[i] * x[i];
         return r;
     }
-    float r = sq_term(x, keep, l8);
-    int i = 8;
-    for (; i < n - (n % 8); i += 8)
-        r = r + sq_term(x, keep, i + l8);
+    const int n8 = n >> 3;
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        v[i] = x[(i < n8 ? i : 0) * 8 + l8]; // (the others are not added)
+    float r = v[0] * v[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) {
+        const float sq = v[i] * v[i];
+        r = i < n8 ? r + sq : r;
+    }
     r = r + __shfl_down(r, 1, 8);
     r = r + __shfl_down(r, 2, 8);
     r = r + __shfl_down(r, 4, 8);
-    for (; i < n; ++i)
-        r = r + sq_term(x, keep, i);
+    for (int i = n8 * 8; i < n; ++i)
+        r = r + x[i] * x[i];
     return r;
 }
 
-// ... and for any n: halves (the first a multiple of 8) are summed separately and added
-__device__ float pairwise_sq_sum(const float *x, const uint8_t *keep, int n, int l8)
-{
-    if (n <= 128)
-        return pairwise_block(x, keep, n, l8);
-    struct Frame {
-        int off, n, stage;
-        float left;
-    };
-    Frame st[32];
-    int sp = 0;
-    float ret = 0.0f;
-    st[sp++] = Frame{0, n, 0, 0.0f};
-    while (sp > 0) {
-        Frame &f = st[sp - 1];
-        if (f.n <= 128) {
-            ret = pairwise_block(x + f.off, keep ? keep + f.off : nullptr, f.n, l8);
-            --sp;
-            continue;
+// ... and for any n: halves (the first a multiple of 8) are summed separately and added.  PairWalk
+// walks the blocks of that tree from left to right; `left` (kPairDepth floats of LDS for each group
+// of eight lanes) holds the sums of the left halves whose right halves are still open, one per level,
+// and bit d of `path` says that the walk is in the right half at level d.
+constexpr int kPairDepth = 26; // 2^31 columns in blocks of 57 and more
+struct PairWalk {
+    int n, off, size; // all columns; the block the walk stands at
+    uint32_t path = 0;
+    int depth = 0;
+    __device__ explicit PairWalk(int n_) : n(n_) { descend(); }
+    __device__ void descend()
+    {
+        off = 0;
+        size = n;
+        for (int d = 0; d < depth; ++d) {
+            const int n2 = size / 2 - size / 2 % 8;
+            const bool right = path >> d & 1u;
+            off += right ? n2 : 0;
+            size = right ? size - n2 : n2;
         }
-        int n2 = f.n / 2;
-        n2 -= n2 % 8;
-        if (f.stage == 0) {
-            f.stage = 1;
-            st[sp++] = Frame{f.off, n2, 0, 0.0f};
-        } else if (f.stage == 1) {
-            f.left = ret;
-            f.stage = 2;
-            st[sp++] = Frame{f.off + n2, f.n - n2, 0, 0.0f};
-        } else {
-            ret = f.left + ret;
-            --sp;
-        }
+        for (; size > 128; ++depth)
+            size = size / 2 - size / 2 % 8;
     }
-    return ret;
-}
+    // takes the block's sum (lane 0 of the group); true, with everything in `sum`, after the last block
+    __device__ bool add(float &sum, float *left, int l8)
+    {
+        for (; depth > 0 && (path >> (depth - 1) & 1u); --depth) {
+            sum = left[depth - 1] + sum;
+            path &= ~(1u << (depth - 1));
+        }
+        if (depth == 0)
+            return true;
+        if (l8 == 0)
+            left[depth - 1] = sum;
+        path |= 1u << (depth - 1);
+        descend();
+        return false;
+    }
+};
 
 constexpr int kNormNotDivided = 1;   // norms are not divided by the tile width
 constexpr int kPerTileThreshold = 2; // tile t compares with selection state t, not with state 0
 
-// One entry per layer of a producer call; all layers run in one launch per stage.
+// One entry per layer of a producer call; all layers run in one launch per stage.  The host fills
+// the table, and for the 2-D producer plan_2d_kernel fills in what depends on the kept columns
+// (n_tiles, norms, rt_begin and the tile table itself).
 struct PruneLayer {
     const float *score;
     uint8_t *mask;
-    const uint8_t *colkeep; // nullptr: every column counts
-    const int32_t *tcol0;   // n_tiles + 1 entries
-    float *norms;           // [n_tiles][K]
-    int32_t K, N, n_tiles;
-    int32_t flags;          // kNormNotDivided, kPerTileThreshold
-    int64_t rt_begin;       // first (row, tile) pair of this layer in the launch-wide numbering
-    int64_t el_begin;       // first item of the mask fill likewise (ceil(K/4) x ceil(N/16) items)
+    uint8_t *colkeep;     // nullptr: every column counts
+    uint8_t *colout;      // the caller's copy of colkeep, or nullptr
+    int32_t *tcol0;       // n_tiles + 1 entries, or nullptr: tiles of `granularity` columns
+    float *norms;         // [n_tiles][K]
+    int32_t K, N, n_tiles, granularity;
+    int32_t flags;        // kNormNotDivided, kPerTileThreshold
+    int32_t pad_;
+    int64_t rt_begin;     // first (row block, tile) item of this layer in the launch-wide numbering
+    int64_t el_begin;     // first workgroup of the mask fill likewise (kFillUnits of ceil(K/4) x ceil(N/16) units)
+    int64_t col_begin;    // first column of this layer among the pooled column norms
 };
 
-__device__ __forceinline__ int find_layer(const PruneLayer *layers, int n_layers, int64_t idx,
-                                          bool by_elements)
+__device__ __forceinline__ int tile_begin(const PruneLayer &L, int t)
 {
-    int lo = 0, hi = n_layers;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if ((by_elements ? layers[mid].el_begin : layers[mid].rt_begin) <= idx)
-            lo = mid;
-        else
-            hi = mid;
+    return L.tcol0 ? as_global(L.tcol0)[t] : min(t * L.granularity, L.N);
+}
+
+// The layer that owns item `idx`, given the layers' first items (`stride` bytes apart), for wave-uniform
+// items: each lane of a wave keeps one layer's first item in a register, so a look-up is a ballot, and
+// the first one a single trip to memory instead of a chain of dependent ones.
+class LayerFinder {
+public:
+    __device__ LayerFinder(const int64_t *begin, size_t stride, int n_layers) : begin_(begin), stride_(stride), n_(n_layers)
+    {
+        mine_ = at(0);
     }
-    return lo;
-}
+    __device__ int operator()(int64_t idx) const
+    {
+        int n = __popcll(__ballot(mine_ <= idx));
+        for (int base = 64; base < n_ && n == base; base += 64) // (beyond 64 layers)
+            n += __popcll(__ballot(at(base) <= idx));
+        return __builtin_amdgcn_readfirstlane(n - 1);
+    }
 
-// norms[t*K + k] = ||score[k][tcol0[t] .. tcol0[t+1])|| / width, pruned columns counting as 0;
-// 8 lanes per (row, tile), neighbouring groups take neighbouring tiles of a row
-__global__ void __launch_bounds__(256)
-    tile_row_norms_kernel(const PruneLayer *layers, int n_layers, int64_t n_pairs)
+private:
+    __device__ int64_t at(int base) const
+    {
+        const int l = base + (int)(threadIdx.x & 63);
+        return l < n_ ? *(TW_GLOBAL(const int64_t))(reinterpret_cast<const char *>(begin_) + (size_t)l * stride_)
+                      : (int64_t)0x7fffffffffffffff;
+    }
+    const int64_t *begin_;
+    size_t stride_;
+    int n_;
+    int64_t mine_;
+};
+
+// norms[t*K + k] = ||score[k][tile t]|| / width, pruned columns counting as 0.  A workgroup takes
+// one tile of up to 32 rows.  NumPy's order of summation gives every eighth column to one running
+// sum, so lanes that read what they add would touch eight 32-byte pieces per load: instead the rows
+// go through LDS a block of the sum (at most 128 columns) at a time, loaded along the row (16 bytes a
+// lane where the rows are aligned), pruned columns replaced by zeros on the way, and eight lanes per
+// row add from there.  The pitch of a staged row is 8 floats past 128, so the eight rows a wave adds
+// at a time lie in eight different groups of banks.  The pointers out of the layer table are known to
+// be global and no load is conditional: flat or predicated loads wait for each other.  Bound by the
+// read: the feed-forward weights of twelve BERT-base layers (226 MB) in 43 us, 5.2 TB/s (a kernel
+// that only reads them 35); 92 us when every lane loaded what it added.
+constexpr int kNormRows = 32;     // rows of an item: eight lanes each
+constexpr int kNormPitch = 136;   // floats; a block of 128 columns with up to 3 before it
+__global__ void __launch_bounds__(256, 6)
+    tile_row_norms_kernel(const PruneLayer *layers, int n_layers, const int64_t *n_items)
 {
-    const int64_t gid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
-    const int l8 = threadIdx.x & 7;
-    if (gid >= n_pairs)
-        return; // whole groups leave together
-    const PruneLayer L = layers[find_layer(layers, n_layers, gid, false)];
-    const int64_t idx = gid - L.rt_begin;
-    const int t = (int)(idx % L.n_tiles);
-    const int k = (int)(idx / L.n_tiles);
-    const int c0 = L.tcol0[t], w = L.tcol0[t + 1] - c0;
-    const float s = pairwise_sq_sum(L.score + (int64_t)k * L.N + c0,
-                                    L.colkeep ? L.colkeep + c0 : nullptr, w, l8);
-    if (l8 == 0)
-        L.norms[(int64_t)t * L.K + k] =
-            (L.flags & kNormNotDivided) ? sqrtf(s) : sqrtf(s) / (float)w; // both correctly rounded
+    __shared__ __align__(16) float stage[kNormRows * kNormPitch];
+    __shared__ float s_left[kNormRows][kPairDepth];
+    const int64_t item = blockIdx.x;
+    if (n_items && item >= *n_items)
+        return; // (a grid sized for the most tiles the layers can have)
+    const PruneLayer L = layers[LayerFinder(&layers->rt_begin, sizeof(PruneLayer), n_layers)(item)];
+    const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a launch has fewer than 2^31 items)
+    const int rblk = (int)(idx / (uint32_t)L.n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)L.n_tiles);
+    const int k0 = rblk * kNormRows, nr = min(kNormRows, L.K - k0);
+    const int c0 = tile_begin(L, t), w = tile_begin(L, t + 1) - c0;
+    const int tid = (int)threadIdx.x, l8 = tid & 7, grp = tid >> 3;
+    TW_GLOBAL(const float) const src = as_global(L.score) + (int64_t)k0 * L.N;
+    TW_GLOBAL(const uint8_t) const keep = as_global((const uint8_t *)L.colkeep);
+    // rows whose starts are aligned are loaded from the 16-byte piece that holds the block's first
+    // column to the one that holds its last (which does not reach past the row: N is a multiple of 4)
+    const bool vec = (L.N & 3) == 0 && ((uintptr_t)L.score & 15) == 0;
+    PairWalk walk(w);
+    for (;;) {
+        const int c = c0 + walk.off, n = walk.size;
+        const int lead = vec ? c & 3 : 0;
+        // (loads and LDS writes are unconditional, so that they all leave at once: rows past the
+        // item's last repeat that one)
+        if (vec) {
+            const int r0 = tid >> 5, q0 = tid & 31, w4 = (lead + n + 3) >> 2;
+            for (int q = q0; q < w4; q += 32) {
+                const int cq = c - lead + q * 4;
+                float4 v[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    v[i] = __builtin_bit_cast(float4, *(TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, nr - 1) * L.N + cq));
+                bool kp[4] = {true, true, true, true};
+                if (keep) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        kp[e] = keep[cq + e] != 0;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    *reinterpret_cast<float4 *>(stage + (r0 + i * 8) * kNormPitch + q * 4) =
+                        float4{kp[0] ? v[i].x : 0.0f, kp[1] ? v[i].y : 0.0f, kp[2] ? v[i].z : 0.0f, kp[3] ? v[i].w : 0.0f};
+            }
+        } else {
+            const int r0 = tid >> 6, q0 = tid & 63;
+            for (int q = q0; q < n; q += 64) {
+                const bool kp = !keep || keep[c + q];
+                float v[kNormRows / 4];
+#pragma unroll
+                for (int i = 0; i < kNormRows / 4; ++i)
+                    v[i] = src[(int64_t)min(r0 + i * 4, nr - 1) * L.N + c + q];
+#pragma unroll
+                for (int i = 0; i < kNormRows / 4; ++i)
+                    stage[(r0 + i * 4) * kNormPitch + q] = kp ? v[i] : 0.0f;
+            }
+        }
+        __syncthreads();
+        float s = pairwise_block(stage + grp * kNormPitch + lead, n, l8); // (rows past the last: unused)
+        if (walk.add(s, s_left[grp], l8)) {
+            if (l8 == 0 && grp < nr) // both operations correctly rounded
+                as_global(L.norms)[(int64_t)t * L.K + k0 + grp] = (L.flags & kNormNotDivided) ? sqrtf(s) : sqrtf(s) / (float)w;
+            return;
+        }
+        __syncthreads(); // the stage is written again
+    }
 }
 
-// One entry per layer for the column stage.
+// cnorm[pooled c] = ||score[:, c]|| / K, the rows accumulated in order.  The chain of K additions
+// per column is sequential by definition; everything around it is not: a workgroup takes 32
+// columns; four waves load 64 rows at a time (eight such groups in flight in registers: 64 KB a
+// workgroup, as much as hides the way to memory), square them and leave them in LDS as [column][row];
+// a fifth adds, four rows per LDS read.
+// All layers share one launch; a column block belongs to one layer (blk_begin: its first block).
+// 31 us for the 126 MB of VGG16's layers (4.1 TB/s, the chain of 4608 additions being about as long);
+// 117 us with a thread per column that loads 32 rows ahead of its additions.
 struct ColLayer {
     const float *score;
     int32_t K, N;
     int64_t col_begin; // first column of this layer in the pooled numbering
+    int64_t blk_begin; // first block of 32 columns likewise
 };
-
-// cnorm[pooled c] = ||score[:, c]|| / K, the rows accumulated in order.  The chain of additions
-// is sequential by definition; the loads are not, so they are issued 32 rows at a time, and all
-// layers share one launch.
-__global__ void col_norms_kernel(const ColLayer *layers, int n_layers, int64_t n_cols, float *cnorm)
+constexpr int kColRows = 64, kColCols = 32, kColPitch = kColRows + 4, kColDeep = 8;
+constexpr int kColThreads = 320; // four waves that load, one that adds
+__global__ void __launch_bounds__(kColThreads) col_norms_kernel(const ColLayer *layers, int n_layers, float *cnorm)
 {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= n_cols)
-        return;
-    int lo = 0, hi = n_layers;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (layers[mid].col_begin <= g)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    const ColLayer L = layers[lo];
+    __shared__ __align__(16) float sq[2][kColCols * kColPitch];
+    const ColLayer L = layers[LayerFinder(&layers->blk_begin, sizeof(ColLayer), n_layers)(blockIdx.x)];
+    const int c0 = (int)((int64_t)blockIdx.x - L.blk_begin) * kColCols;
+    const int tid = (int)threadIdx.x, col = tid & 31;
     const int K = L.K, N = L.N;
-    constexpr int U = 32;
-    const float *p = L.score + (g - L.col_begin);
-    float acc = 0.0f;
-    int k = 0;
-    for (; k + U <= K; k += U) {
-        float v[U];
+    const int n_grp = (K + kColRows * kColDeep - 1) / (kColRows * kColDeep) * kColDeep; // in whole rounds of kColDeep
+    if (tid >= 256) { // the adding wave: lanes 0 - 31 and, as an unused copy, 32 - 63
+        float acc = 0.0f;
+        const float *const x = sq[0] + col * kColPitch;
+        for (int g = 0; g < n_grp; ++g) {
+            __syncthreads(); // group g is staged
+            const float *const s = x + (g & 1) * (kColCols * kColPitch);
+            float4 a[kColRows / 4];
 #pragma unroll
-        for (int j = 0; j < U; ++j)
-            v[j] = p[(int64_t)(k + j) * N];
+            for (int j = 0; j < kColRows / 4; ++j)
+                a[j] = *reinterpret_cast<const float4 *>(s + j * 4);
 #pragma unroll
-        for (int j = 0; j < U; ++j) {
-            const float sq = v[j] * v[j];
-            acc = acc + sq;
+            for (int j = 0; j < kColRows / 4; ++j) {
+                acc = acc + a[j].x;
+                acc = acc + a[j].y;
+                acc = acc + a[j].z;
+                acc = acc + a[j].w;
+            }
+        }
+        if (tid < 256 + kColCols && c0 + col < N)
+            cnorm[L.col_begin + c0 + col] = sqrtf(acc) / (float)K;
+        return;
+    }
+    const int r0 = tid >> 5;
+    // (a column past the layer's last repeats that one and is dropped at the end)
+    TW_GLOBAL(const float) const p = as_global(L.score) + min(c0 + col, N - 1);
+    float v[kColDeep][8];
+    auto load = [&](int g, float (&d)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            d[i] = p[(int64_t)min(g * kColRows + r0 + i * 8, K - 1) * N];
+        }
+    };
+    // (groups past the last repeat its last row and count as zeros: no load is conditional, so the
+    // waits for them are exact counts)
+#pragma unroll
+    for (int d = 0; d < kColDeep; ++d)
+        load(d, v[d]);
+    for (int g0 = 0; g0 < n_grp; g0 += kColDeep) {
+#pragma unroll
+        for (int d = 0; d < kColDeep; ++d) {
+            const int g = g0 + d;
+            // (the adding wave has read this stage: it read group g - 2 before barrier g - 1)
+            float *const s = sq[d & 1];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float x = g * kColRows + r0 + i * 8 < K ? v[d][i] : 0.0f; // (a zero leaves a sum of squares alone)
+                s[col * kColPitch + r0 + i * 8] = x * x;
+            }
+            load(g + kColDeep, v[d]);
+            __syncthreads();
         }
     }
-    for (; k < K; ++k) {
-        const float v = p[(int64_t)k * N];
-        const float sq = v * v;
-        acc = acc + sq;
-    }
-    cnorm[g] = sqrtf(acc) / (float)K;
 }
 
 // order-preserving map float -> uint32
@@ -199,96 +322,217 @@ __device__ __forceinline__ uint32_t sort_key(float v)
     const uint32_t b = __float_as_uint(v);
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
-// Selection state in device memory, so that the passes follow each other on the stream without
-// a host round trip.  Pass p (p = 0..3) counts, among the values whose key agrees with the digits
-// fixed by the passes before it, the digit at bit 24 - 8 p; which digit holds the rank is worked
-// out from the histograms by whoever needs it next (resolve_prefix).
+__device__ __forceinline__ float key_to_float(uint32_t key)
+{
+    return __uint_as_float((key & 0x80000000u) ? (key & 0x7FFFFFFFu) : ~key);
+}
+
+// np.percentile with linear interpolation, on the device: a radix select of the k-th smallest key in
+// three passes over the values (11 + 11 + 10 bits of the key), and what the interpolation needs
+// beside it, its upper neighbour, out of the same passes: the values above the digits fixed so far
+// leave their minimum, those that share all digits but the last leave it in the last histogram.
+// (A first digit of 11 bits - sign, exponent, two bits of mantissa - also spreads the values of a
+// layer over a few dozen counters; with 8 bits, two octaves a digit, most lanes of a wave met in one
+// or two LDS counters: 38 us a pass over 31.5 M values.)
+// Pass p counts the values that agree with the digits before it; which digit holds the rank is
+// worked out of the histogram by every workgroup of the next pass, and the workgroup of the last
+// pass that finishes last works out the threshold.
+constexpr int kSelBins = 2048;
+struct SelectHead {               // the wanted rank and the interpolation above it
+    int64_t n;                    // number of values
+    unsigned long long rank0;     // 0-based rank of the wanted value
+    double gamma64;
+    float gamma32;
+    int32_t top;                  // the percentile is the largest value
+    int32_t f64;                  // the interpolation runs in float64
+    int32_t pad_;
+};
 struct SelectState {
-    unsigned long long hist[4][256];
-    unsigned long long rank0;     // rank (0-based) of the wanted value
-    unsigned long long count_le;  // values <= the k-th smallest
-    uint32_t prefix;              // key of the k-th smallest (written with the threshold)
-    uint32_t min_gt;              // smallest key above the k-th smallest's (0xFFFFFFFF: none)
-    int32_t lost;                 // set if a pass found no digit (cannot happen for rank < n)
-    float thr32;                  // the threshold, for the kernels that follow
+    unsigned long long hist[3][kSelBins];
+    SelectHead head;
+    unsigned long long rank[3];   // rank among the values that match before pass p (from pass 1 on)
+    uint32_t prefix[3];           // their common leading bits, as the value of the bits above pass p's digit
+    uint32_t min_gt;              // smallest key above the group the passes so far narrowed down to (0xFFFFFFFF: none)
+    // mixed masks: the selection first narrows the elements down to those between two values
+    float lo, hi;                 // the bracket
+    uint32_t room;                // values inside it that a wave can keep aside
+    uint32_t key_base;            // the passes' digits are those of key - key_base,
+    int32_t key_bits;             // which has this many bits
+    float thr32;                  // the threshold, where select_finish_kernel has run
     double thr64;
 };
 
-// The selection kernels work on segments of equal length laid end to end (one segment for the
-// network-wide thresholds, one per tile for per-tile thresholds): segment g = blockIdx.y (or
-// blockIdx.x for the one-workgroup kernels) uses state st[g] and values v[g*n .. g*n+n).
-__global__ void __launch_bounds__(256) select_init_kernel(SelectState *st, unsigned long long rank)
+// Rank and weight of np.percentile(v[0..n), q): with q_is_f64 == 0 (q was a Python number) the
+// quantile q/100, the virtual index (n-1)*quantile and the interpolation are float32; with 1 (q was
+// a NumPy float64) they are float64, only the difference of the two neighbours stays float32.
+__device__ void select_rank(SelectHead *h, int64_t n, double q, int q_is_f64)
 {
-    st += blockIdx.x;
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-        st->hist[p][threadIdx.x] = 0;
-    if (threadIdx.x == 0) {
-        st->rank0 = rank;
-        st->count_le = 0;
-        st->prefix = 0;
-        st->min_gt = 0xFFFFFFFFu;
-        st->lost = 0;
+    int64_t lo;
+    bool top;
+    h->gamma32 = 0.0f;
+    h->gamma64 = 0.0;
+    if (q_is_f64) {
+        const double quant = q / 100.0;
+        const double virt = (double)(n - 1) * quant;
+        top = virt >= (double)(n - 1);
+        lo = top ? n - 1 : (int64_t)floor(virt);
+        h->gamma64 = virt - floor(virt);
+    } else {
+        const float quant = (float)q / 100.0f;
+        const float virt = (float)(n - 1) * quant;
+        top = virt >= (float)(n - 1);
+        lo = top ? n - 1 : (int64_t)floorf(virt);
+        h->gamma32 = virt - floorf(virt);
     }
+    h->n = n;
+    h->top = top;
+    h->f64 = q_is_f64;
+    h->rank0 = (unsigned long long)min(lo, n - 1);
+}
+__device__ void select_begin(SelectState *st, int64_t n, double q, int q_is_f64)
+{
+    select_rank(&st->head, n, q, q_is_f64);
+    st->min_gt = 0xFFFFFFFFu;
+    st->lo = -INFINITY;
+    st->hi = INFINITY;
+    st->key_base = 0;
+    st->key_bits = 32;
 }
 
-// The key digits that passes 0 .. npass-1 have fixed, the rank that is left among the values
-// matching them, and whether a pass found no digit.  Called by all 256 threads of a workgroup
-// (an inclusive scan of each histogram finds the digit whose count range holds the rank); every
-// thread returns the same values.
-__device__ void resolve_prefix(const SelectState *st, int npass, uint32_t &prefix, uint32_t &mask,
-                               unsigned long long &rank, bool &lost)
+// The digits are those of key - base, for keys known to lie within `bits` bits above `base` (all keys:
+// 0 and 32): 11 bits, 11 bits and what is left of them.
+struct KeyRange {
+    uint32_t base;
+    int shift[3]; // of each pass's digit
+    __device__ KeyRange(uint32_t base_, int bits) : base(base_), shift{max(bits - 11, 0), max(bits - 22, 0), 0} {}
+    __device__ int lead_shift(int pass) const { return pass == 0 ? 32 : shift[pass - 1]; } // the digits before: key >> this
+    __device__ uint32_t digit(int pass, uint32_t k) const
+    {
+        return (k >> shift[pass]) & (pass == 0 ? kSelBins - 1u : (1u << (shift[pass - 1] - shift[pass])) - 1u);
+    }
+};
+
+// The digit of a finished pass whose counts (NB of them) hold `rank`, the rank among the values with
+// that digit and how many those are, and (NEXT) the next digit any value has (0xFFFFFFFF: none); called by
+// all NT threads of a workgroup, the same values come back to every one.
+struct Digit {
+    unsigned long long rest, count;
+    uint32_t digit, next;
+};
+template <int NT, int NB, bool NEXT = false, class T> __device__ Digit find_digit(const T *hist, unsigned long long rank)
 {
-    __shared__ unsigned long long s_wave[4];
-    __shared__ unsigned long long s_before;
-    __shared__ int s_digit;
+    constexpr int PER = NB / NT;
+    __shared__ unsigned long long s_wave[NT / 64];
+    __shared__ Digit s_d;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    prefix = 0;
-    mask = 0;
-    rank = st->rank0;
-    lost = false;
-    for (int p = 0; p < npass; ++p) {
-        const int shift = 24 - 8 * p;
-        const unsigned long long c = st->hist[p][tid];
-        unsigned long long incl = c;
-        for (int off = 1; off < 64; off <<= 1) {
-            const unsigned long long up = __shfl_up(incl, off);
-            if (lane >= off)
-                incl += up;
-        }
-        if (lane == 63)
-            s_wave[wave] = incl;
-        if (tid == 0)
-            s_digit = -1;
-        __syncthreads();
-        for (int w = 0; w < wave; ++w)
-            incl += s_wave[w];
-        const unsigned long long excl = incl - c;
-        if (c > 0 && excl <= rank && rank < incl) { // exactly one digit, if any
-            s_digit = tid;
-            s_before = excl;
-        }
-        __syncthreads();
-        int d = s_digit;
-        if (d < 0) {
-            lost = true;
-            d = 255;
-        } else {
-            rank -= s_before;
-        }
-        prefix |= (uint32_t)d << shift;
-        mask |= 255u << shift;
-        __syncthreads(); // the shared words are rewritten by the next pass
+    T c[PER];
+    unsigned long long sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        c[i] = hist[tid * PER + i];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        sum += c[i];
+    unsigned long long incl = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const unsigned long long up = __shfl_up(incl, off);
+        if (lane >= off)
+            incl += up;
     }
+    if (lane == 63)
+        s_wave[wave] = incl;
+    if (tid == 0) // (a rank below the sum of the counts is always found)
+        s_d = Digit{0, 1, (uint32_t)NB - 1u, 0xFFFFFFFFu};
+    __syncthreads();
+    for (int w = 0; w < wave; ++w)
+        incl += s_wave[w];
+    unsigned long long before = incl - sum;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (before <= rank && rank < before + c[i]) { // exactly one digit
+            s_d.digit = tid * PER + i;
+            s_d.rest = rank - before;
+            s_d.count = c[i];
+        }
+        before += c[i];
+    }
+    __syncthreads();
+    if (NEXT) { // (one LDS atomic per wave: hundreds on one word take microseconds)
+        const uint32_t digit = s_d.digit;
+        uint32_t next = 0xFFFFFFFFu;
+#pragma unroll
+        for (int i = PER - 1; i >= 0; --i)
+            if (c[i] && (uint32_t)(tid * PER + i) > digit)
+                next = tid * PER + i;
+        for (int off = 32; off > 0; off >>= 1)
+            next = min(next, (uint32_t)__shfl_down(next, off));
+        if (lane == 0)
+            atomicMin(&s_d.next, next);
+        __syncthreads();
+    }
+    const Digit d = s_d;
+    __syncthreads(); // the shared words are written again by the next call
+    return d;
 }
 
-// Calls f(value) for every element of v[0..n) once, the workgroups of blockIdx.x sharing the
+// A threshold in both types; values of the type of NumPy's result are compared with it, strictly.
+struct Threshold {
+    double v64;
+    float v32;
+    bool f64;
+    __device__ bool passed_by(float v) const { return f64 ? (double)v > v64 : v > v32; }
+};
+
+// NumPy's two-sided linear interpolation between the k-th smallest value a and its upper
+// neighbour b (a again if it is repeated, or if the index is the last one): float32 throughout
+// for a float32 gamma, float64 with a float32 difference b - a otherwise.
+__device__ Threshold interpolate(const SelectHead *st, uint32_t key_a, uint32_t key_b)
+{
+    const float a = key_to_float(key_a);
+    const float b = st->top || key_b == 0xFFFFFFFFu ? a : key_to_float(key_b);
+    const float diff = b - a;
+    if (st->f64) {
+        const double g = st->gamma64;
+        const double prod = g >= 0.5 ? (double)diff * (1.0 - g) : (double)diff * g;
+        const double r = g >= 0.5 ? (double)b - prod : (double)a + prod;
+        return Threshold{r, (float)r, true};
+    }
+    const float g = st->gamma32;
+    const float prod = g >= 0.5f ? diff * (1.0f - g) : diff * g;
+    const float r = g >= 0.5f ? b - prod : a + prod;
+    return Threshold{(double)r, r, false};
+}
+
+// The threshold out of the counts of the finished last pass, by all NT threads of a workgroup: the key
+// of the wanted value, and the key above it where that value is not repeated.  Whatever uses a
+// threshold works it out itself: a kernel of its own for it, or a last workgroup of the last pass,
+// is a chain of trips to memory of 5 to 10 us with the chip idle.
+template <int NT> __device__ Threshold threshold_of(const SelectState *st)
+{
+    __shared__ Threshold s_t;
+    const uint32_t min_gt = st->min_gt;
+    const uint32_t base = st->key_base;
+    const KeyRange range(base, st->key_bits);
+    const uint32_t lead = st->prefix[2] << range.lead_shift(2);
+    const Digit d = find_digit<NT, 1024, true>(st->hist[2], st->rank[2]);
+    if (threadIdx.x == 0) {
+        const uint32_t key_a = base + (lead | d.digit);
+        uint32_t key_b = key_a;
+        if (d.rest + 1 >= d.count) // the wanted value is the last of its kind
+            key_b = d.next != 0xFFFFFFFFu ? base + (lead | d.next) : min_gt;
+        s_t = interpolate(&st->head, key_a, key_b);
+    }
+    __syncthreads();
+    return s_t;
+}
+
+// Calls f(value) for every element of v[0..n) once, the first `workgroups` of blockIdx.x sharing the
 // work: 16-byte loads over the aligned middle (four of them in flight per thread), single
 // elements at the ragged ends.
-template <class F> __device__ __forceinline__ void for_each_value(const float *v, int64_t n, F f)
+template <class F> __device__ __forceinline__ void for_each_value(const float *v, int64_t n, int workgroups, F f)
 {
     const int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t nthr = (int64_t)gridDim.x * blockDim.x;
+    const int64_t nthr = (int64_t)workgroups * blockDim.x;
     const int64_t head = min(n, (int64_t)((16 - ((uintptr_t)v & 15)) & 15) >> 2);
     const int64_t nvec = (n - head) >> 2;
     const float4 *v4 = reinterpret_cast<const float4 *>(v + head);
@@ -310,223 +554,378 @@ template <class F> __device__ __forceinline__ void for_each_value(const float *v
         f(v[j < head ? j : tail0 + (j - head)]);
 }
 
-// hist[pass][d] += number of values whose key matches the digits fixed so far and has digit d
-// at bit 24 - 8 pass
-__global__ void __launch_bounds__(256)
-    select_hist_kernel(const float *v, int64_t n, int pass, SelectState *st)
+// One value of pass PASS: counted where it agrees with the digits before, remembered as the
+// smallest above them where it lies above.
+template <int PASS>
+__device__ __forceinline__ void select_count(uint32_t key, const KeyRange &r, uint32_t prefix, unsigned int *s_h, uint32_t &mn)
 {
-    st += blockIdx.y;
-    v += (int64_t)blockIdx.y * n;
-    __shared__ unsigned int s_h[256];
-    s_h[threadIdx.x] = 0;
-    uint32_t prefix, mask;
-    unsigned long long rank;
-    bool lost;
-    resolve_prefix(st, pass, prefix, mask, rank, lost);
-    __syncthreads(); // s_h is zeroed
-    const int shift = 24 - 8 * pass;
-    for_each_value(v, n, [&](float x) {
-        const uint32_t key = sort_key(x);
-        if ((key & mask) == prefix)
-            atomicAdd(&s_h[(key >> shift) & 255u], 1u);
-    });
-    __syncthreads();
-    if (s_h[threadIdx.x])
-        atomicAdd(&st->hist[pass][threadIdx.x], (unsigned long long)s_h[threadIdx.x]);
+    const uint32_t k = key - r.base;
+    const uint32_t lead = PASS == 0 ? 0u : k >> r.lead_shift(PASS);
+    if (PASS == 0 || lead == prefix)
+        atomicAdd(&s_h[r.digit(PASS, k)], 1u);
+    else if (lead > prefix)
+        mn = min(mn, key);
 }
 
-// count_le = number of values <= the selected one, min_gt = smallest key above it
-__global__ void __launch_bounds__(256) rank_stats_kernel(const float *v, int64_t n, SelectState *st)
+// What a workgroup of pass PASS does before it counts: the digits so far (its first workgroup
+// leaves them for the next pass), cleared counters.  rank0: the rank before the first pass.
+template <int PASS, int NT>
+__device__ void select_enter(SelectState *st, const KeyRange &range, unsigned int *s_h, uint32_t *s_min, unsigned long long rank0,
+                             uint32_t &prefix, unsigned long long &rank)
 {
-    st += blockIdx.y;
-    v += (int64_t)blockIdx.y * n;
-    uint32_t key_a, mask;
-    unsigned long long rank;
-    bool lost;
-    resolve_prefix(st, 4, key_a, mask, rank, lost);
-    unsigned long long cnt = 0;
-    unsigned int mn = 0xFFFFFFFFu;
-    for_each_value(v, n, [&](float x) {
-        const uint32_t key = sort_key(x);
-        if (key <= key_a)
-            ++cnt;
-        else
-            mn = min(mn, key);
-    });
-    // one pair of atomics per workgroup
-    __shared__ unsigned long long s_cnt;
-    __shared__ unsigned int s_min;
-    if (threadIdx.x == 0) {
-        s_cnt = 0;
-        s_min = 0xFFFFFFFFu;
+    for (int i = (int)threadIdx.x; i < kSelBins; i += NT)
+        s_h[i] = 0;
+    if (threadIdx.x == 0)
+        *s_min = 0xFFFFFFFFu;
+    prefix = 0;
+    rank = rank0;
+    if (PASS > 0) {
+        const Digit d = find_digit<NT, kSelBins>(st->hist[PASS > 0 ? PASS - 1 : 0], PASS == 2 ? st->rank[1] : rank0);
+        prefix = PASS == 2 ? st->prefix[1] << (range.shift[0] - range.shift[1]) | d.digit : d.digit;
+        rank = d.rest;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            st->prefix[PASS] = prefix;
+            st->rank[PASS] = rank;
+        }
     }
     __syncthreads();
+}
+
+// ... and after it has counted: its counts join those of the others.
+template <int PASS, int NT> __device__ void select_leave(SelectState *st, unsigned int *s_h, uint32_t *s_min, uint32_t mn)
+{
+    if (PASS > 0) {
+        for (int off = 32; off > 0; off >>= 1)
+            mn = min(mn, (uint32_t)__shfl_down(mn, off));
+        if ((threadIdx.x & 63) == 0 && mn != 0xFFFFFFFFu)
+            atomicMin(s_min, mn);
+    }
+    __syncthreads();
+    for (int i = (int)threadIdx.x; i < kSelBins; i += NT)
+        if (s_h[i])
+            atomicAdd(&st->hist[PASS][i], (unsigned long long)s_h[i]);
+    if (PASS > 0 && threadIdx.x == 0 && *s_min != 0xFFFFFFFFu)
+        atomicMin(&st->min_gt, *s_min);
+}
+
+// Pass PASS over v[0 .. st->n).  The selection works on segments of equal length laid end to end
+// (one segment for the network-wide thresholds, one per tile for per-tile thresholds): segment g =
+// blockIdx.y uses state st[g] and values v[g*n .. g*n+n).
+template <int PASS> __global__ void __launch_bounds__(256) select_hist_kernel(const float *v, SelectState *st)
+{
+    __shared__ unsigned int s_h[kSelBins];
+    __shared__ uint32_t s_min;
+    st += blockIdx.y;
+    const int64_t n = st->head.n;
+    uint32_t prefix, mn = 0xFFFFFFFFu;
+    unsigned long long rank;
+    const KeyRange range(0, 32);
+    select_enter<PASS, 256>(st, range, s_h, &s_min, st->head.rank0, prefix, rank);
+    for_each_value(v + (int64_t)blockIdx.y * n, n, (int)gridDim.x, [&](float x) { select_count<PASS>(sort_key(x), range, prefix, s_h, mn); });
+    select_leave<PASS, 256>(st, s_h, &s_min, mn);
+}
+
+// The selection in one workgroup and its LDS, for a few ten thousand values (the columns of a network, a
+// sample).  The digits are those of the keys' own range, so that the values spread over all counters:
+// lanes of a wave that meet in one LDS counter take turns.
+template <int NT, class V> __device__ KeyRange key_range_in_block(V key, int n)
+{
+    __shared__ uint32_t s_lo, s_hi;
+    if (threadIdx.x == 0) {
+        s_lo = 0xFFFFFFFFu;
+        s_hi = 0;
+    }
+    __syncthreads();
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+    for (int i = (int)threadIdx.x; i < n; i += NT) {
+        const uint32_t k = key(i);
+        lo = min(lo, k);
+        hi = max(hi, k);
+    }
     for (int off = 32; off > 0; off >>= 1) {
-        cnt += __shfl_down(cnt, off);
-        mn = min(mn, (unsigned int)__shfl_down(mn, off));
+        lo = min(lo, (uint32_t)__shfl_down(lo, off));
+        hi = max(hi, (uint32_t)__shfl_down(hi, off));
     }
     if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&s_cnt, cnt);
-        atomicMin(&s_min, mn);
+        atomicMin(&s_lo, lo);
+        atomicMax(&s_hi, hi);
     }
+    __syncthreads();
+    return KeyRange(s_lo, s_hi > s_lo ? 32 - __clz(s_hi - s_lo) : 1);
+}
+// one pass: rank becomes the rank among the values that share the digits so far
+template <int PASS, int NT, class V>
+__device__ Digit count_in_block(V key, int n, const KeyRange &range, unsigned long long &rank, uint32_t &prefix, unsigned int *s_h,
+                                uint32_t &mn)
+{
+    for (int i = (int)threadIdx.x; i < kSelBins; i += NT)
+        s_h[i] = 0;
+    __syncthreads();
+    for (int i = (int)threadIdx.x; i < n; i += NT)
+        select_count<PASS>(key(i), range, prefix, s_h, mn);
+    __syncthreads();
+    const Digit d = find_digit<NT, PASS == 2 ? 1024 : kSelBins, PASS != 0>(s_h, rank);
+    prefix = PASS == 0 ? d.digit : prefix << (range.lead_shift(PASS) - range.shift[PASS]) | d.digit;
+    rank = d.rest;
+    return d;
+}
+template <int NT, class V> __device__ Threshold select_in_block(V key, const SelectHead *h, unsigned int *s_h)
+{
+    __shared__ uint32_t s_min;
+    __shared__ Threshold s_t;
+    if (threadIdx.x == 0)
+        s_min = 0xFFFFFFFFu;
+    const int n = (int)h->n;
+    const KeyRange range = key_range_in_block<NT>(key, n);
+    uint32_t prefix = 0, mn = 0xFFFFFFFFu;
+    unsigned long long rank = h->rank0;
+    count_in_block<0, NT>(key, n, range, rank, prefix, s_h, mn);
+    Digit d = count_in_block<1, NT>(key, n, range, rank, prefix, s_h, mn);
+    if (range.shift[1] > 0) // (else two digits hold all of the range)
+        d = count_in_block<2, NT>(key, n, range, rank, prefix, s_h, mn);
+    for (int off = 32; off > 0; off >>= 1)
+        mn = min(mn, (uint32_t)__shfl_down(mn, off));
+    if ((threadIdx.x & 63) == 0)
+        atomicMin(&s_min, mn);
     __syncthreads();
     if (threadIdx.x == 0) {
-        if (s_cnt)
-            atomicAdd(&st->count_le, s_cnt);
-        if (s_min != 0xFFFFFFFFu)
-            atomicMin(&st->min_gt, s_min);
+        const uint32_t a = range.base + prefix;
+        s_t = interpolate(h, a, d.rest + 1 < d.count ? a : d.next != 0xFFFFFFFFu ? a - d.digit + d.next : s_min);
     }
+    __syncthreads();
+    return s_t;
 }
 
-__device__ __forceinline__ float key_to_float(uint32_t key)
-{
-    return __uint_as_float((key & 0x80000000u) ? (key & 0x7FFFFFFFu) : ~key);
-}
-
-// NumPy's two-sided linear interpolation between the k-th smallest value a and its upper
-// neighbour b (a again if it is repeated, or if the index is the last one): float32 throughout
-// for a float32 gamma, float64 with a float32 difference b - a otherwise.
-__global__ void __launch_bounds__(256)
-    select_lerp_kernel(SelectState *st, unsigned long long k, int top, int f64, float gamma32,
-                       double gamma64)
+// the thresholds of several segments, or one that only the host wants
+__global__ void __launch_bounds__(256) select_finish_kernel(SelectState *st)
 {
     st += blockIdx.x;
-    uint32_t key_a, mask;
-    unsigned long long rank;
-    bool lost;
-    resolve_prefix(st, 4, key_a, mask, rank, lost);
-    if (threadIdx.x != 0)
-        return;
-    st->prefix = key_a;
-    st->lost = lost ? 1 : 0;
-    const float a = key_to_float(key_a);
-    float b = a;
-    if (!top && st->count_le <= k + 1 && st->min_gt != 0xFFFFFFFFu)
-        b = key_to_float(st->min_gt);
-    const float diff = b - a;
-    if (f64) {
-        const double prod = gamma64 >= 0.5 ? (double)diff * (1.0 - gamma64) : (double)diff * gamma64;
-        const double r = gamma64 >= 0.5 ? (double)b - prod : (double)a + prod;
-        st->thr64 = r;
-        st->thr32 = (float)r;
-    } else {
-        const float prod = gamma32 >= 0.5f ? diff * (1.0f - gamma32) : diff * gamma32;
-        const float r = gamma32 >= 0.5f ? b - prod : a + prod;
-        st->thr32 = r;
-        st->thr64 = (double)r;
+    const Threshold t = threshold_of<256>(st);
+    if (threadIdx.x == 0) {
+        st->thr32 = t.v32;
+        st->thr64 = t.v64;
     }
 }
 
-// keep[c] = cnorm[c] > threshold
-__global__ void col_keep_kernel(const float *cnorm, int N, const SelectState *st, int f64,
-                                uint8_t *keep)
+// Between the column stage and the row stage of the 2-D producer, one workgroup: the threshold over
+// all column norms, the column masks, every layer's tiles (they end after every `granularity` kept
+// columns) and where its norms and its row-norm items begin, and the state of the row selection.
+// All on the device, so that the call needs no trip to the host between its stages.
+constexpr int kPlanThreads = 1024;
+constexpr int kPlanStage = 12288; // column norms kept in LDS; more of them are read from memory in every pass
+__global__ void __launch_bounds__(kPlanThreads)
+    plan_2d_kernel(PruneLayer *layers, int n_layers, const float *cnorm, int64_t n_cols, float *norms,
+                   double *thr_cols, SelectState *st_rows, int64_t *n_items, double q, int q_is_f64)
 {
-    const float thr32 = st->thr32;
-    const double thr64 = st->thr64;
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < N)
-        keep[c] = (f64 ? (double)cnorm[c] > thr64 : cnorm[c] > thr32) ? 1 : 0;
-}
-
-// mask[k][c] = (norm of row k in c's tile > threshold) and column c kept.  One thread per 16
-// consecutive columns of kFillRows consecutive rows: one 16-byte store per row where the chunk
-// is whole and aligned; the layer and tile look-ups are shared by the rows.
-constexpr int kFillRows = 4;
-__global__ void __launch_bounds__(256)
-    fill_mask_kernel(const PruneLayer *layers, int n_layers, int64_t n_chunks,
-                     const SelectState *st, int f64)
-{
-    // the first chunk of every layer, so that a thread finds its layer without a chain of
-    // global loads (the first kFillCached layers; a search beyond them reads the table itself)
-    constexpr int kFillCached = 128;
-    __shared__ int64_t s_begin[kFillCached];
-    const int n_cached = min(n_layers, kFillCached);
-    for (int i = (int)threadIdx.x; i < n_cached; i += (int)blockDim.x)
-        s_begin[i] = layers[i].el_begin;
+    __shared__ unsigned int s_h[kSelBins];
+    __shared__ SelectHead s_head;
+    __shared__ int64_t s_norm[kPlanThreads], s_item[kPlanThreads];
+    __shared__ float s_cn[kPlanStage];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const bool staged = n_cols <= kPlanStage;
+    if (staged) {
+        constexpr int PER = kPlanStage / kPlanThreads;
+        float v[PER];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (tid + i * kPlanThreads < n_cols)
+                v[i] = cnorm[tid + i * kPlanThreads];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            if (tid + i * kPlanThreads < n_cols)
+                s_cn[tid + i * kPlanThreads] = v[i];
+    }
+    if (tid == 0)
+        select_rank(&s_head, n_cols, q, q_is_f64);
     __syncthreads();
-    const int64_t gidx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gidx >= n_chunks)
-        return;
-    int li;
-    if (n_layers > kFillCached && layers[kFillCached].el_begin <= gidx) {
-        li = kFillCached + find_layer(layers + kFillCached, n_layers - kFillCached, gidx, true);
-    } else {
-        int lo = 0, hi = n_cached;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (s_begin[mid] <= gidx)
-                lo = mid;
-            else
-                hi = mid;
+    auto norm_of = [&](int64_t i) -> float {
+        if (staged)
+            return s_cn[i];
+        return as_global(cnorm)[i];
+    };
+    const Threshold thr = select_in_block<kPlanThreads>([&](int i) { return sort_key(norm_of(i)); }, &s_head, s_h);
+    if (tid == 0)
+        *thr_cols = thr.v64;
+    int64_t norm_carry = 0, item_carry = 0;
+    for (int base = 0; base < n_layers; base += kPlanThreads) {
+        const int cnt = min(kPlanThreads, n_layers - base);
+        for (int l = wave; l < cnt; l += kPlanThreads / 64) {
+            PruneLayer &L = layers[base + l];
+            const int64_t first = L.col_begin;
+            TW_GLOBAL(uint8_t) const colkeep = as_global(L.colkeep);
+            TW_GLOBAL(uint8_t) const colout = as_global(L.colout);
+            TW_GLOBAL(int32_t) const tcol0 = as_global(L.tcol0);
+            const int N = L.N, G = L.granularity;
+            int kept = 0;           // columns kept before this group of 64
+            int tile = 1, end = G;  // the next tile starts behind kept column number `end`
+            for (int c0 = 0; c0 < N; c0 += 64) {
+                const int c = c0 + lane;
+                const float v = c < N ? norm_of(first + c) : 0.0f;
+                const bool keep = c < N && thr.passed_by(v);
+                const unsigned long long b = __ballot(keep);
+                const int mine = kept + __popcll(b & ((2ull << lane) - 1ull)); // kept columns up to this one
+                if (c < N) {
+                    colkeep[c] = keep ? 1 : 0;
+                    if (colout)
+                        colout[c] = keep ? 1 : 0;
+                }
+                kept += __popcll(b);
+                for (; end <= kept; end += G, ++tile)
+                    if (keep && mine == end && c + 1 < N)
+                        tcol0[tile] = c + 1;
+            }
+            if (lane == 0) {
+                // tiles that ended before the last column, and the one that takes the rest
+                const bool last_col_ends = kept > 0 && kept % G == 0 &&
+                                           thr.passed_by(norm_of(first + N - 1));
+                const int nt = kept / G - (last_col_ends ? 1 : 0) + 1;
+                tcol0[0] = 0;
+                tcol0[nt] = N;
+                L.n_tiles = nt;
+                s_norm[l] = (int64_t)L.K * nt;
+                s_item[l] = (int64_t)((L.K + kNormRows - 1) / kNormRows) * nt;
+            }
         }
-        li = lo;
+        __syncthreads();
+        const int64_t my_norm = tid < cnt ? s_norm[tid] : 0, my_item = tid < cnt ? s_item[tid] : 0;
+        for (int off = 1; off < cnt; off <<= 1) { // inclusive sums over the layers
+            const int64_t a = tid >= off && tid < cnt ? s_norm[tid - off] : 0;
+            const int64_t b = tid >= off && tid < cnt ? s_item[tid - off] : 0;
+            __syncthreads();
+            if (tid < cnt) {
+                s_norm[tid] += a;
+                s_item[tid] += b;
+            }
+            __syncthreads();
+        }
+        if (tid < cnt) {
+            layers[base + tid].norms = norms + norm_carry + s_norm[tid] - my_norm;
+            layers[base + tid].rt_begin = item_carry + s_item[tid] - my_item;
+        }
+        norm_carry += s_norm[cnt - 1];
+        item_carry += s_item[cnt - 1];
+        __syncthreads();
     }
-    const PruneLayer L = layers[li];
+    if (tid == 0) {
+        *n_items = item_carry;
+        select_begin(st_rows, norm_carry, q, q_is_f64);
+    }
+}
+
+// Start of a call: up to kBlobWords words of the call's tables, handed over in the kernel arguments, go
+// to device memory, the histograms of `n_states` selections are cleared and, where n > 0, their ranks
+// worked out.  One launch (or a few, for tables of more than some twenty layers) instead of a copy
+// from host memory and the wait for it.
+constexpr int kBlobWords = 640;
+struct Blob {
+    uint32_t w[kBlobWords];
+};
+__global__ void __launch_bounds__(256)
+    prune_setup_kernel(const Blob a, uint32_t *dst, int words, SelectState *st, int n_states, int64_t n, double q, int q_is_f64,
+                       uint32_t room)
+{
+    const auto *src = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    const int gtid = (int)(blockIdx.x * blockDim.x + threadIdx.x), nthr = (int)(gridDim.x * blockDim.x);
+    for (int i = gtid; i < words; i += nthr)
+        dst[i] = src[i];
+    for (int g = 0; g < n_states; ++g) {
+        for (int i = gtid; i < 3 * kSelBins; i += nthr)
+            (&st[g].hist[0][0])[i] = 0;
+        if (gtid == 0 && n > 0) {
+            select_begin(&st[g], n, q, q_is_f64);
+            st[g].room = room;
+        }
+    }
+}
+
+// mask[k][c] = (norm of row k in c's tile > threshold) and column c kept.  A unit of work is 16
+// consecutive columns of four consecutive rows: one 16-byte store per row where the chunk is whole and
+// aligned; a workgroup takes 1024 units of one layer, four per thread.  15 us for the 57 MB of masks of
+// twelve BERT-base feed-forward layers, of which 3 are the threshold.
+constexpr int kFillRows = 4, kFillUnits = 1024;
+__global__ void __launch_bounds__(256)
+    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const double *thr_cols, double *mail)
+{
+    const PruneLayer L = layers[LayerFinder(&layers->el_begin, sizeof(PruneLayer), n_layers)(blockIdx.x)];
     const bool per_tile = (L.flags & kPerTileThreshold) != 0;
-    float thr32 = st->thr32;
-    double thr64 = st->thr64;
-    const int64_t idx = gidx - L.el_begin;
-    const int cpr = (L.N + 15) >> 4; // chunks per row
-    // (a 32-bit division where the layer's item count allows it: the 64-bit one is long)
-    const int kg = (idx >> 31) == 0 ? (int)((uint32_t)idx / (uint32_t)cpr) : (int)(idx / cpr);
-    const int c0 = (int)(idx - (int64_t)kg * cpr) << 4;
-    const int k0 = kg * kFillRows;
-    const int nrows = min(kFillRows, L.K - k0);
-    // the tile of column c0: start near where tiles of equal width would put it, then walk
-    int t = min(L.n_tiles - 1, (int)((float)c0 * (float)L.n_tiles / (float)L.N));
-    while (L.tcol0[t] > c0)
-        --t;
-    while (L.tcol0[t + 1] <= c0)
-        ++t;
-    int t_end = L.tcol0[t + 1];
-    bool row_keep[kFillRows];
-    auto enter_tile = [&]() { // the rows' norms in tile t against its threshold
-        if (per_tile) {
-            thr32 = st[t].thr32;
-            thr64 = st[t].thr64;
+    const Threshold thr = per_tile ? Threshold{} : threshold_of<256>(st);
+    if (blockIdx.x == 0 && threadIdx.x == 0) { // the thresholds, to host memory
+        mail[0] = per_tile ? st->thr64 : thr.v64;
+        mail[1] = thr_cols ? *thr_cols : 0.0;
+    }
+    const uint32_t cpr = (uint32_t)(L.N + 15) >> 4; // chunks per row
+    const int64_t n_units = (int64_t)cpr * ((L.K + kFillRows - 1) / kFillRows);
+    const int64_t first = (blockIdx.x - L.el_begin) * kFillUnits;
+    TW_GLOBAL(const float) const norms = as_global((const float *)L.norms);
+    TW_GLOBAL(const int32_t) const tcol0 = as_global((const int32_t *)L.tcol0);
+    TW_GLOBAL(const uint8_t) const colkeep = as_global((const uint8_t *)L.colkeep);
+    auto begin_of = [&](int t) { return tcol0 ? tcol0[t] : min(t * L.granularity, L.N); };
+#pragma unroll
+    for (int i = 0; i < kFillUnits / 256; ++i) {
+        const int64_t unit = first + i * 256 + threadIdx.x;
+        if (unit >= n_units)
+            break;
+        // (a 32-bit division where the layer's units allow it: the 64-bit one is long)
+        const int kg = (unit >> 31) == 0 ? (int)((uint32_t)unit / cpr) : (int)(unit / cpr);
+        const int c0 = (int)(unit - (int64_t)kg * cpr) << 4, n = min(16, L.N - c0), k0 = kg * kFillRows;
+        uint32_t cols[4]; // the chunk's columns: a byte of 1 where kept
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            cols[w] = 0x01010101u;
+            if (colkeep) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (!colkeep[min(c0 + w * 4 + e, L.N - 1)])
+                        cols[w] &= ~(1u << (e * 8));
+            }
+        }
+        // the tile of column c0: start near where tiles of equal width would put it, then walk
+        int t = tcol0 ? min(L.n_tiles - 1, (int)((float)c0 * (float)L.n_tiles / (float)L.N)) : c0 / L.granularity;
+        if (tcol0) {
+            while (tcol0[t] > c0)
+                --t;
+            while (tcol0[t + 1] <= c0)
+                ++t;
+        }
+        uint32_t out[kFillRows][4];
+#pragma unroll
+        for (int r = 0; r < kFillRows; ++r)
+            out[r][0] = out[r][1] = out[r][2] = out[r][3] = 0u;
+        for (int cb = c0; cb < c0 + n; ++t) { // the tiles the chunk touches: one, or a few
+            const int ce = min(begin_of(t + 1), c0 + n);
+            Threshold tt = thr;
+            if (per_tile)
+                tt = Threshold{st[t].thr64, st[t].thr32, st[t].head.f64 != 0};
+            float nv[kFillRows];
+#pragma unroll
+            for (int r = 0; r < kFillRows; ++r)
+                nv[r] = norms[(int64_t)t * L.K + min(k0 + r, L.K - 1)];
+            uint32_t in_tile[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int lo = min(max(cb - c0 - w * 4, 0), 4), hi = min(max(ce - c0 - w * 4, 0), 4);
+                in_tile[w] = cols[w] & (uint32_t)((1ull << (hi * 8)) - 1ull) & ~(uint32_t)((1ull << (lo * 8)) - 1ull);
+            }
+#pragma unroll
+            for (int r = 0; r < kFillRows; ++r) {
+                const bool keep = tt.passed_by(nv[r]);
+#pragma unroll
+                for (int w = 0; w < 4; ++w)
+                    out[r][w] |= keep ? in_tile[w] : 0u;
+            }
+            cb = ce;
         }
 #pragma unroll
         for (int r = 0; r < kFillRows; ++r) {
-            const float nv = r < nrows ? L.norms[(int64_t)t * L.K + k0 + r] : 0.0f;
-            row_keep[r] = r < nrows && (f64 ? (double)nv > thr64 : nv > thr32);
-        }
-    };
-    enter_tile();
-    uint32_t w[kFillRows][4];
-#pragma unroll
-    for (int r = 0; r < kFillRows; ++r)
-        w[r][0] = w[r][1] = w[r][2] = w[r][3] = 0u;
-    const int n = min(16, L.N - c0);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        if (e < n) {
-            const int c = c0 + e;
-            if (c >= t_end) {
-                ++t;
-                t_end = L.tcol0[t + 1];
-                enter_tile();
+            if (k0 + r >= L.K)
+                break;
+            TW_GLOBAL(uint8_t) const dst = as_global(L.mask) + (int64_t)(k0 + r) * L.N + c0;
+            if (n == 16 && (((uintptr_t)dst) & 15) == 0) {
+                *(TW_GLOBAL(u32x4))dst = u32x4{out[r][0], out[r][1], out[r][2], out[r][3]};
+            } else {
+                for (int e = 0; e < n; ++e)
+                    dst[e] = (uint8_t)(out[r][e >> 2] >> ((e & 3) * 8));
             }
-            const bool col = !L.colkeep || L.colkeep[c];
-#pragma unroll
-            for (int r = 0; r < kFillRows; ++r)
-                w[r][e >> 2] |= (col && row_keep[r] ? 1u : 0u) << ((e & 3) * 8);
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kFillRows; ++r) {
-        if (r >= nrows)
-            break;
-        uint8_t *dst = L.mask + (int64_t)(k0 + r) * L.N + c0;
-        if (n == 16 && (((uintptr_t)dst) & 15) == 0) {
-            uint4 v;
-            v.x = w[r][0];
-            v.y = w[r][1];
-            v.z = w[r][2];
-            v.w = w[r][3];
-            *reinterpret_cast<uint4 *>(dst) = v;
-        } else {
-            for (int e = 0; e < n; ++e)
-                dst[e] = (uint8_t)(w[r][e >> 2] >> ((e & 3) * 8));
         }
     }
 }
@@ -538,105 +937,350 @@ struct MixLayer {
     const float *score;
     const uint8_t *mask0; // the TW mask of the layer
     uint8_t *out;         // may be mask0 itself
-    int64_t begin;        // first element of the layer in the pooled vector
+    int64_t n;            // elements of the layer
+    int64_t begin;        // its first element among all layers'
+    int64_t item_begin;   // its first item in the launch-wide numbering
 };
 
-__device__ inline int find_mix_layer(const MixLayer *layers, int n_layers, int64_t idx)
+// ||x|| of a single element (sqrt(x*x) / 1, the reference's norm over a tile of one column) minus 1
+// where the TW mask already keeps it (prune_algo.py:159-161).  The square root of a rounded square
+// is |x| again as long as the square is a normal number (or zero).
+__device__ __forceinline__ bool mix_plain(float ax) { return (ax >= 1e-18f && ax <= 1e18f) || ax == 0.0f; }
+__device__ __forceinline__ float mix_value(float x, uint32_t m0)
 {
+    float nrm = fabsf(x);
+    if (!mix_plain(nrm)) {
+        const float sq = x * x;
+        nrm = sqrtf(sq);
+    }
+    return m0 ? nrm - 1.0f : nrm;
+}
+
+// The kernels of the mixed producer walk items of 4096 consecutive elements of a layer, sixteen per
+// thread, as vectors where score, mask and output are aligned alike.  The element scores are worked
+// out anew from weight and mask in every pass (five bytes an element, 158 MB for the layers of VGG16,
+// which the memory-side cache holds) rather than written to a pool and read back (eight bytes more,
+// once, and four in every pass).  At five bytes an element the vector instructions count as much as
+// the memory: a dozen per element are 10 us for 31.5 M elements.
+constexpr int kMixItem = 4096;
+struct MixFetched {
+    TW_GLOBAL(const float) sc;
+    TW_GLOBAL(const uint8_t) mk;
+    uint8_t *out;
+    int n;
+    bool vec;
+    float4 x[4];
+    uint32_t m[4];
+};
+__device__ __forceinline__ void mix_fetch(const MixLayer &L, int64_t item, const float *safe, MixFetched &d)
+{
+    const int64_t e0 = (item - L.item_begin) * kMixItem;
+    d.n = (int)min((int64_t)kMixItem, L.n - e0);
+    d.sc = as_global(L.score) + e0;
+    d.mk = as_global(L.mask0) + e0;
+    d.out = L.out + e0;
+    d.vec = d.n == kMixItem && ((uintptr_t)d.sc & 15) == 0 && (((uintptr_t)d.mk | (uintptr_t)d.out) & 3) == 0;
+    // (an item that cannot be loaded in vectors loads something else in its place: with no load on a
+    // condition the waits for them are exact counts)
+    TW_GLOBAL(const u32x4) const x = d.vec ? (TW_GLOBAL(const u32x4))d.sc : (TW_GLOBAL(const u32x4))safe;
+    TW_GLOBAL(const uint32_t) const m = d.vec ? (TW_GLOBAL(const uint32_t))d.mk : (TW_GLOBAL(const uint32_t))safe;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        d.x[i] = __builtin_bit_cast(float4, x[threadIdx.x + i * 256]);
+        d.m[i] = m[threadIdx.x + i * 256];
+    }
+}
+// f(values, mask bytes, output, count) per four (or single) elements
+template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d, F f)
+{
+    if (d.vec) {
+        float ax[4][4];
+        float hi = 0.0f, lo = 1.0f; // largest and (zeros aside) smallest
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            ax[i][0] = fabsf(d.x[i].x);
+            ax[i][1] = fabsf(d.x[i].y);
+            ax[i][2] = fabsf(d.x[i].z);
+            ax[i][3] = fabsf(d.x[i].w);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                hi = ax[i][e] <= hi ? hi : ax[i][e]; // (a NaN stays)
+                lo = fminf(lo, ax[i][e] == 0.0f ? 1.0f : ax[i][e]);
+            }
+        }
+        if (!(mix_plain(hi) && mix_plain(lo))) { // one test for all sixteen
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    ax[i][e] = mix_value(ax[i][e], 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) // (the mask byte, any value but 0 counting as 1)
+                v[e] = ax[i][e] - fminf((float)(d.m[i] >> (e * 8) & 255u), 1.0f);
+            f(v, d.m[i], d.out + (threadIdx.x + i * 256) * 4, 4);
+        }
+    } else {
+        // (whole waves make every round: f may look at its wave)
+        for (int i0 = 0; i0 < d.n; i0 += 256) {
+            const int i = i0 + (int)threadIdx.x, j = min(i, d.n - 1);
+            const uint32_t m0 = d.mk[j];
+            float v[4] = {mix_value(d.sc[j], m0), 0.0f, 0.0f, 0.0f};
+            f(v, m0, d.out + j, i < d.n ? 1 : 0);
+        }
+    }
+}
+// All items of a launch, shared out over its workgroups, the next item's loads in flight while one is
+// worked on.  done() after every item;
+// safe: 16 KB of device memory that can be read.
+template <class F, class D>
+__device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layers, int64_t n_items, const float *safe, F f, D done)
+{
+    const LayerFinder find(&layers->item_begin, sizeof(MixLayer), n_layers);
+    MixFetched a, b;
+    const int64_t step = gridDim.x, last = n_items - 1;
+    int64_t item = blockIdx.x; // (a launch has at most n_items workgroups)
+    mix_fetch(layers[find(item)], item, safe, a);
+    for (;;) {
+        const int64_t i1 = min(item + step, last), i2 = min(item + 2 * step, last);
+        mix_fetch(layers[find(i1)], i1, safe, b);
+        mix_apply(a, f);
+        done();
+        if (item + step > last)
+            break;
+        mix_fetch(layers[find(i2)], i2, safe, a);
+        mix_apply(b, f);
+        done();
+        item += 2 * step;
+        if (item > last)
+            break;
+    }
+}
+
+// The selection over the element scores.  Three passes with a histogram over all elements cost three
+// reads of everything and, most elements sharing a few dozen digits, as many conflicts in LDS (60, 90
+// and 67 us over the 31.5 M elements of VGG16).  So the wanted value is bracketed first: 8192 elements
+// drawn evenly (one at a random place of every stretch) give two keys between which it lies but for
+// one case in a million, one pass over the elements counts what is below and keeps aside what is
+// between (2 - 3 % of the elements), and the three passes run over what was kept.
+// Where the bracket missed or does not fit - the counts tell, for certain - they run over the
+// elements.
+// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 15 + 32 + 40 us.
+constexpr int kMixSamples = 8192;
+constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
+__global__ void __launch_bounds__(256) mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, uint32_t *sample)
+{
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); // kMixSamples threads
+    const int64_t at = total / kMixSamples * i;
+    uint32_t h = (uint32_t)i * 0x9E3779B9u;
+    h = (h ^ (h >> 16)) * 0x85EBCA6Bu;
+    h ^= h >> 13;
+    const int64_t e = at + (int64_t)(h % (uint32_t)min(total / kMixSamples, (int64_t)0x7FFFFFFF));
     int lo = 0, hi = n_layers;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (layers[mid].begin <= idx)
+        if (layers[mid].begin <= e)
             lo = mid;
         else
             hi = mid;
     }
-    return lo;
+    const int64_t j = e - layers[lo].begin;
+    sample[i] = sort_key(mix_value(layers[lo].score[j], layers[lo].mask0[j]));
 }
 
-// Both mixed-mask kernels walk the pooled element numbering in groups of four: a group that lies
-// in one layer and is 16-byte aligned there moves as vectors, any other group element by element.
-struct MixGroup {
-    MixLayer L;
-    int64_t e;   // first element inside the layer
-    bool vec;
+// The bracket out of the sample, one workgroup: the sample's values five standard deviations of their
+// rank to either side of the wanted one, widened to 22 bits of the sample's range.
+constexpr int kBracketThreads = 1024;
+__global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint32_t *sample, SelectState *st)
+{
+    constexpr int PER = kMixSamples / kBracketThreads;
+    __shared__ unsigned int s_h[kSelBins];
+    __shared__ uint32_t s_key[kMixSamples];
+    const int tid = (int)threadIdx.x;
+    uint32_t key[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        key[i] = sample[tid + i * kBracketThreads];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        s_key[tid + i * kBracketThreads] = key[i];
+    const double f = (double)st->head.rank0 / (double)st->head.n;
+    const double mid = f * kMixSamples, dev = 5.0 * sqrt((double)kMixSamples * f * (1.0 - f)) + 2.0;
+    const double want[2] = {mid - dev, mid + dev};
+    auto key_of = [&](int i) { return s_key[i]; };
+    const KeyRange range = key_range_in_block<kBracketThreads>(key_of, kMixSamples); // (its barrier: s_key is whole)
+    uint32_t edge[2];
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        if (want[w] < 0.0 || want[w] >= (double)kMixSamples) { // workgroup-uniform
+            edge[w] = w ? 0xFFFFFFFFu : 0u;
+            continue;
+        }
+        uint32_t prefix = 0, mn = 0xFFFFFFFFu;
+        unsigned long long rank = (unsigned long long)want[w];
+        count_in_block<0, kBracketThreads>(key_of, kMixSamples, range, rank, prefix, s_h, mn);
+        count_in_block<1, kBracketThreads>(key_of, kMixSamples, range, rank, prefix, s_h, mn);
+        const unsigned long long at = ((unsigned long long)prefix + w) << range.shift[1];
+        edge[w] = (uint32_t)min((unsigned long long)range.base + at - w, 0xFFFFFFFFull);
+    }
+    if (tid == 0) {
+        st->lo = edge[0] == 0u ? -INFINITY : key_to_float(edge[0]);
+        st->hi = edge[1] == 0xFFFFFFFFu ? INFINITY : key_to_float(edge[1]);
+    }
+}
+
+// Below, between, above.  Every wave of the launch keeps the values between in a piece of the
+// candidates of its own and leaves its counts beside it: nothing is added up with atomics, of which the
+// memory takes one in 15 ns on one address (a counter per workgroup that all add to was 25 us of this
+// kernel, one per wave 90).
+constexpr int kMixWgs = 1024, kMixWaves = kMixWgs * 4; // most workgroups and waves of a pass over the elements
+struct MixCounts {
+    uint32_t between, below;
 };
-
-__device__ __forceinline__ MixGroup mix_group(const MixLayer *layers, int n_layers, int64_t total,
-                                              int64_t i)
-{
-    MixGroup g;
-    const int l = find_mix_layer(layers, n_layers, i);
-    g.L = layers[l];
-    g.e = i - g.L.begin;
-    const int64_t end = l + 1 < n_layers ? layers[l + 1].begin : total;
-    g.vec = i + 4 <= end && (((uintptr_t)(g.L.score + g.e)) & 15) == 0 &&
-            (((uintptr_t)(g.L.mask0 + g.e)) & 3) == 0 && (((uintptr_t)(g.L.out + g.e)) & 3) == 0;
-    return g;
-}
-
-__device__ __forceinline__ float mix_value(float x, uint8_t m0)
-{
-    const float sq = x * x;
-    const float nrm = sqrtf(sq) / 1.0f;
-    return nrm - (m0 ? 1.0f : 0.0f);
-}
-
-// pool[i] = ||x|| of the single element (sqrt(x*x) / 1, the reference's norm over a tile of one
-// column) minus 1 where the TW mask already keeps it (prune_algo.py:159-161)
 __global__ void __launch_bounds__(256)
-    mix_values_kernel(const MixLayer *layers, int n_layers, int64_t total, float *pool)
+    mix_narrow_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, float *cand, MixCounts *counts)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
-    for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < total; i += stride) {
-        const MixGroup g = mix_group(layers, n_layers, total, i);
-        if (g.vec) {
-            const float4 x = *reinterpret_cast<const float4 *>(g.L.score + g.e);
-            const uint32_t m = *reinterpret_cast<const uint32_t *>(g.L.mask0 + g.e);
-            float4 r;
-            r.x = mix_value(x.x, (uint8_t)(m & 255u));
-            r.y = mix_value(x.y, (uint8_t)((m >> 8) & 255u));
-            r.z = mix_value(x.z, (uint8_t)((m >> 16) & 255u));
-            r.w = mix_value(x.w, (uint8_t)(m >> 24));
-            *reinterpret_cast<float4 *>(pool + i) = r; // the pool is 256-byte aligned, i = 0 mod 4
-        } else {
-            for (int64_t j = i; j < min(i + 4, total); ++j) {
-                const MixLayer L = layers[find_mix_layer(layers, n_layers, j)];
-                const int64_t e = j - L.begin;
-                pool[j] = mix_value(L.score[e], L.mask0[e]);
+    const float lo = st->lo, hi = st->hi;
+    const uint32_t room = st->room;
+    const int lane = (int)(threadIdx.x & 63);
+    const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    TW_GLOBAL(float) const keep = as_global(cand) + (int64_t)w * room;
+    uint32_t kept = 0, below = 0; // wave-uniform
+    auto narrow = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const unsigned long long under = __ballot(e < cnt && v[e] < lo);
+            const unsigned long long in = __ballot(e < cnt && v[e] >= lo && v[e] <= hi);
+            below += __popcll(under);
+            if (in) {
+                const uint32_t at = kept + __popcll(in & ((1ull << lane) - 1ull));
+                if ((in >> lane & 1ull) && at < room) // (the count tells of an overflow)
+                    keep[at] = v[e];
+                kept += __popcll(in);
             }
         }
-    }
+    };
+    mix_for_each(layers, n_layers, n_items, cand, narrow, []() {});
+    if (lane == 0)
+        counts[w] = MixCounts{kept, below};
 }
 
-// out = mask0 | (pool > threshold)   (prune_algo.py:171-176)
-__global__ void __launch_bounds__(256)
-    mix_mask_kernel(const MixLayer *layers, int n_layers, int64_t total, const float *pool,
-                    const SelectState *st, int f64)
+// the counts of all waves of the narrowing pass added up, and whether every piece held its values; called by all 256
+// threads of a workgroup
+__device__ bool mix_totals(const MixCounts *counts, int waves, uint32_t room, unsigned long long &between, unsigned long long &below)
 {
-    const float thr32 = st->thr32;
-    const double thr64 = st->thr64;
-    auto above = [&](float v) { return f64 ? (double)v > thr64 : v > thr32; };
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x * 4;
-    for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; i < total; i += stride) {
-        const MixGroup g = mix_group(layers, n_layers, total, i);
-        if (g.vec) {
-            const float4 v = *reinterpret_cast<const float4 *>(pool + i);
-            const uint32_t m = *reinterpret_cast<const uint32_t *>(g.L.mask0 + g.e);
-            uint32_t o = 0;
-            o |= ((m & 0x000000FFu) || above(v.x)) ? 0x00000001u : 0u;
-            o |= ((m & 0x0000FF00u) || above(v.y)) ? 0x00000100u : 0u;
-            o |= ((m & 0x00FF0000u) || above(v.z)) ? 0x00010000u : 0u;
-            o |= ((m & 0xFF000000u) || above(v.w)) ? 0x01000000u : 0u;
-            *reinterpret_cast<uint32_t *>(g.L.out + g.e) = o;
-        } else {
-            for (int64_t j = i; j < min(i + 4, total); ++j) {
-                const MixLayer L = layers[find_mix_layer(layers, n_layers, j)];
-                const int64_t e = j - L.begin;
-                L.out[e] = (L.mask0[e] || above(pool[j])) ? 1 : 0;
+    __shared__ unsigned long long s_sum[2];
+    __shared__ uint32_t s_most;
+    if (threadIdx.x == 0) {
+        s_sum[0] = s_sum[1] = 0;
+        s_most = 0;
+    }
+    __syncthreads();
+    unsigned long long a = 0, b = 0;
+    uint32_t most = 0;
+#pragma unroll
+    for (int i = 0; i < kMixWaves / 256; ++i) {
+        const int w = (int)threadIdx.x + i * 256;
+        const MixCounts c = counts[min(w, waves - 1)];
+        a += w < waves ? c.between : 0u;
+        b += w < waves ? c.below : 0u;
+        most = max(most, c.between);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        a += __shfl_down(a, off);
+        b += __shfl_down(b, off);
+        most = max(most, (uint32_t)__shfl_down(most, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&s_sum[0], a);
+        atomicAdd(&s_sum[1], b);
+        atomicMax(&s_most, most);
+    }
+    __syncthreads();
+    between = s_sum[0];
+    below = s_sum[1];
+    return s_most <= room;
+}
+
+constexpr int kMixHistWgs = 96; // workgroups that count what was kept (each adds up to 2048 counters to the others')
+template <int PASS>
+__global__ void __launch_bounds__(256)
+    mix_hist_kernel(const MixLayer *layers, int n_layers, int64_t n_items, SelectState *st, const float *cand,
+                    const MixCounts *counts, int waves)
+{
+    __shared__ unsigned int s_h[kSelBins];
+    __shared__ uint32_t s_min;
+    uint32_t prefix, mn = 0xFFFFFFFFu;
+    unsigned long long rank;
+    const unsigned long long want = st->head.rank0;
+    const uint32_t room = st->room;
+    unsigned long long n_cand, below;
+    const bool whole = mix_totals(counts, waves, room, n_cand, below);
+    // the wanted value and the one above it lie inside the bracket, and all of that was kept
+    const bool narrowed = whole && below <= want && (want - below) + 1 < n_cand;
+    if (narrowed && blockIdx.x >= kMixHistWgs)
+        return;
+    // (-0 and +0 are one value to the comparisons with the bracket, and two keys)
+    const uint32_t lo = narrowed ? sort_key(st->lo == 0.0f ? -0.0f : st->lo) : 0u;
+    const uint32_t span = narrowed ? sort_key(st->hi == 0.0f ? 0.0f : st->hi) - lo : 0xFFFFFFFFu;
+    const int bits = span ? 32 - __clz(span) : 1;
+    const KeyRange range(lo, bits);
+    select_enter<PASS, 256>(st, range, s_h, &s_min, narrowed ? want - below : want, prefix, rank);
+    if (PASS == 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+        st->key_base = lo;
+        st->key_bits = bits;
+    }
+    if (narrowed) {
+        const int per = min((int)gridDim.x, kMixHistWgs) * 4;
+        for (int w = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)); w < waves; w += per) {
+            const uint32_t n = counts[w].between;
+            TW_GLOBAL(const float) const v = as_global(cand) + (int64_t)w * room;
+            for (uint32_t i = threadIdx.x & 63; i < n; i += 256) { // four loads in flight
+                float x[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    x[e] = v[min(i + e * 64, n - 1)];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (i + e * 64 < n)
+                        select_count<PASS>(sort_key(x[e]), range, prefix, s_h, mn);
             }
         }
+    } else {
+        auto count = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e < cnt)
+                    select_count<PASS>(sort_key(v[e]), range, prefix, s_h, mn);
+        };
+        mix_for_each(layers, n_layers, n_items, cand, count, []() {});
     }
+    select_leave<PASS, 256>(st, s_h, &s_min, mn);
+}
+
+// out = mask0 | (score > threshold)   (prune_algo.py:171-176)
+__global__ void __launch_bounds__(256)
+    mix_mask_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, const float *safe, double *mail)
+{
+    const Threshold thr = threshold_of<256>(st);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        mail[0] = thr.v64;
+    auto above = [&](float v) { return thr.passed_by(v); };
+    auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt) {
+        if (cnt == 4) {
+            uint32_t o = ((m & 0x7F7F7F7Fu) + 0x7F7F7F7Fu | m) >> 7 & 0x01010101u; // mask bytes that are not 0
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                o |= above(v[e]) ? 1u << (e * 8) : 0u;
+            *(TW_GLOBAL(uint32_t))out = o;
+        } else if (cnt == 1) {
+            *as_global(out) = (m || above(v[0])) ? 1 : 0;
+        }
+    };
+    mix_for_each(layers, n_layers, n_items, safe, mark, []() {});
 }
 
 // ---------------------------------------------------------------------------------
@@ -645,12 +1289,14 @@ __global__ void __launch_bounds__(256)
 namespace {
 
 // Temporaries of one producer call come from a process-wide device buffer that only grows, so
-// that a steady stream of calls does not pay for hipMalloc / hipFree.  The arena holds the
-// buffer's lock for the duration of the call (producer calls are serialised).
+// that a steady stream of calls does not pay for hipMalloc / hipFree, and its thresholds come back
+// through a page of pinned host memory that its last kernel writes.  The arena holds the lock of
+// both for the duration of the call (producer calls are serialised).
 std::mutex g_ws_mutex;
 void *g_ws = nullptr;
 size_t g_ws_size = 0;
 int g_ws_device = -1; // the device the buffer lives on; calls on another device do not use it
+double *g_mail = nullptr;
 
 class Arena {
 public:
@@ -667,11 +1313,12 @@ public:
     }
     ~Arena()
     {
-        (void)hipStreamSynchronize(stream_);
+        if (!idle_)
+            (void)hipStreamSynchronize(stream_);
         for (void *p : extras_)
-            hipFree(p);
+            (void)hipFree(p);
         if (usable_ && need_ > g_ws_size) { // grow for the next call
-            hipFree(g_ws);
+            (void)hipFree(g_ws);
             g_ws = nullptr;
             g_ws_size = 0;
             const size_t want = need_ + need_ / 2;
@@ -695,87 +1342,69 @@ public:
         return p;
     }
     template <class T> T *alloc_n(size_t n) { return static_cast<T *>(alloc(sizeof(T) * std::max<size_t>(n, 1))); }
+    // the pinned page, or nullptr
+    double *mail()
+    {
+        if (!g_mail && hipHostMalloc((void **)&g_mail, 4096, hipHostMallocPortable) != hipSuccess)
+            g_mail = nullptr;
+        return g_mail;
+    }
+    // waits for the call's kernels; nothing may be queued behind this
+    int wait()
+    {
+        TW_HIP(hipStreamSynchronize(stream_));
+        idle_ = true;
+        return TW_OK;
+    }
 
 private:
     std::lock_guard<std::mutex> lock_;
     hipStream_t stream_;
     int device_ = -1;
-    bool usable_ = false;
+    bool usable_ = false, idle_ = false;
     size_t off_ = 0, need_ = 0;
     std::vector<void *> extras_;
 };
 
-// The k-th (0-based) smallest of v[0..n) and its upper neighbour in sorted order.
-struct Threshold {
-    SelectState *state; // device; thr32 / thr64 are valid once the stream has run
-    int is_f64;
-};
+// `bytes` of a host table to the device through kernel arguments, and the selections cleared
+int put_table(const void *table, size_t bytes, void *dst, SelectState *st, int n_states, int64_t n, double q,
+              int q_is_f64, hipStream_t s, uint32_t room = 0)
+{
+    size_t off = 0;
+    do {
+        Blob a;
+        const size_t take = std::min(bytes - off, sizeof(a.w));
+        std::memcpy(a.w, static_cast<const char *>(table) + off, take);
+        hipLaunchKernelGGL(prune_setup_kernel, dim3(n_states > 4 ? 128 : 16), dim3(256), 0, s, a,
+                           reinterpret_cast<uint32_t *>(static_cast<char *>(dst) + off), (int)((take + 3) / 4), st, n_states,
+                           n, q, q_is_f64, room);
+        n_states = 0; // (the selections once)
+        off += take;
+    } while (off < bytes);
+    TW_HIP(hipGetLastError());
+    return TW_OK;
+}
 
-// np.percentile(v, q) with linear interpolation for a float32 vector on the device, queued on the
-// stream: four histogram passes of a radix select for the k-th smallest value, its upper
-// neighbour, then the interpolation.  With q_is_f64 == 0 (q was a Python number) the quantile
-// q/100, the virtual index (n-1)*quantile and the interpolation are float32; with 1 (q was a
-// NumPy float64) they are float64, only the difference of the two neighbours stays float32.
-int percentile_linear(Arena &ar, const float *d_v, int64_t n, double q, int q_is_f64, hipStream_t s,
-                      Threshold *out, int n_segments = 1)
+int check_percentile(int64_t n, double q)
 {
     if (n <= 0)
         return fail(TW_ERR_SHAPE, "percentile of an empty set");
     if (!(q >= 0.0 && q <= 100.0))
         return fail(TW_ERR_SHAPE, "percentile %g is outside [0, 100]", q);
-    int64_t lo;
-    double gamma64 = 0.0;
-    float gamma32 = 0.0f;
-    bool top;
-    if (q_is_f64) {
-        const double quant = q / 100.0;
-        const double virt = (double)(n - 1) * quant;
-        top = virt >= (double)(n - 1);
-        lo = top ? n - 1 : (int64_t)std::floor(virt);
-        gamma64 = virt - std::floor(virt);
-    } else {
-        const float quant = (float)q / 100.0f;
-        const float virt = (float)(n - 1) * quant;
-        top = virt >= (float)(n - 1);
-        lo = top ? n - 1 : (int64_t)std::floor(virt);
-        gamma32 = virt - std::floor(virt);
-    }
-    const unsigned long long k = (unsigned long long)std::min(lo, n - 1);
-    SelectState *st = ar.alloc_n<SelectState>(n_segments);
-    if (!st)
-        return fail(TW_ERR_ALLOC, "hipMalloc of the selection state failed");
-    const int grid = (int)std::min<int64_t>(n_segments > 1 ? 64 : 1024, (n + 255) / 256);
-    const dim3 g2(grid, n_segments), g1(n_segments);
-    hipLaunchKernelGGL(select_init_kernel, g1, dim3(256), 0, s, st, k);
-    for (int pass = 0; pass < 4; ++pass)
-        hipLaunchKernelGGL(select_hist_kernel, g2, dim3(256), 0, s, d_v, n, pass, st);
-    hipLaunchKernelGGL(rank_stats_kernel, g2, dim3(256), 0, s, d_v, n, st);
-    hipLaunchKernelGGL(select_lerp_kernel, g1, dim3(256), 0, s, st, k, top ? 1 : 0, q_is_f64,
-                       gamma32, gamma64);
-    TW_HIP(hipGetLastError());
-    out->state = st;
-    out->is_f64 = q_is_f64;
     return TW_OK;
 }
 
-// waits for the stream and returns the threshold as a double
-int read_threshold(const Threshold &t, hipStream_t s, double *value)
+// The three passes over `n` values (at most, where the state holds the exact number) in each of
+// n_segments segments.  Two workgroups per compute unit at most: every workgroup starts by
+// working out a digit from 16 KB of counters and ends with an atomic on every counter it has used.
+int queue_select(const float *d_v, int64_t n, SelectState *st, int n_segments, hipStream_t s)
 {
-    // the words behind the histograms are all the host needs
-    struct Tail {
-        int32_t lost;
-        float thr32;
-        double thr64;
-    } h;
-    static_assert(offsetof(SelectState, thr64) - offsetof(SelectState, lost) == offsetof(Tail, thr64) &&
-                      sizeof(SelectState) - offsetof(SelectState, lost) == sizeof(Tail),
-                  "Tail mirrors the end of SelectState");
-    TW_HIP(hipMemcpyAsync(&h, reinterpret_cast<const char *>(t.state) + offsetof(SelectState, lost),
-                          sizeof(h), hipMemcpyDeviceToHost, s));
-    TW_HIP(hipStreamSynchronize(s));
-    if (h.lost)
-        return fail(TW_ERR_DEVICE, "radix select lost its rank");
-    *value = h.thr64;
+    const int grid = (int)std::min<int64_t>(n_segments > 1 ? 64 : 256, (n + 4095) / 4096);
+    const dim3 g(std::max(1, grid), n_segments);
+    hipLaunchKernelGGL(select_hist_kernel<0>, g, dim3(256), 0, s, d_v, st);
+    hipLaunchKernelGGL(select_hist_kernel<1>, g, dim3(256), 0, s, d_v, st);
+    hipLaunchKernelGGL(select_hist_kernel<2>, g, dim3(256), 0, s, d_v, st);
+    TW_HIP(hipGetLastError());
     return TW_OK;
 }
 
@@ -796,70 +1425,87 @@ int check_layers(int n_layers, const int32_t *K, const int32_t *N, const float *
     return TW_OK;
 }
 
-// per layer: the tile table on the device, offsets of the layer's norms in the pooled vector
-struct LayerTiles {
-    std::vector<int32_t> tcol0; // n_tiles + 1 entries
-    int64_t norm_off = 0;
+// The table of a call whose tiles are every `granularity` columns, or (tile_tables != nullptr) at most
+// that many tiles, found on the device.
+struct CallTable {
+    std::vector<PruneLayer> layers;
+    int64_t n_norms = 0, n_items = 0, n_fill = 0, n_tcol = 0, n_cols = 0; // sums over the layers (upper bounds)
 };
-
-// norms of all layers into one pooled vector, one threshold, masks
-int rows_stage(Arena &ar, int n_layers, const int32_t *K, const int32_t *N,
-               const float *const *scores, std::vector<LayerTiles> &lt,
-               const std::vector<uint8_t *> &d_colkeep, double q, int q_is_f64,
-               uint8_t *const *masks, Threshold *thr, hipStream_t s, int flags = 0)
+CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
+                     uint8_t *const *masks, int granularity, int flags)
 {
-    int64_t total = 0, tab = 0;
+    CallTable c;
+    c.layers.resize(n_layers);
     for (int l = 0; l < n_layers; ++l) {
-        lt[l].norm_off = total;
-        total += (int64_t)K[l] * ((int64_t)lt[l].tcol0.size() - 1);
-        tab += (int64_t)lt[l].tcol0.size();
-    }
-    float *d_norms = ar.alloc_n<float>(total);
-    // the layer table and the tile tables behind it share one buffer: one upload
-    const size_t table_bytes = (sizeof(PruneLayer) * n_layers + 15) / 16 * 16;
-    char *d_both = static_cast<char *>(ar.alloc(table_bytes + sizeof(int32_t) * tab));
-    if (!d_norms || !d_both)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %lld norms failed", (long long)total);
-    PruneLayer *d_table = reinterpret_cast<PruneLayer *>(d_both);
-    int32_t *d_tables = reinterpret_cast<int32_t *>(d_both + table_bytes);
-    std::vector<char> both(table_bytes + sizeof(int32_t) * tab, 0);
-    PruneLayer *pl = reinterpret_cast<PruneLayer *>(both.data());
-    int32_t *flat = reinterpret_cast<int32_t *>(both.data() + table_bytes);
-    size_t n_flat = 0;
-    int64_t n_pairs = 0, n_elems = 0;
-    for (int l = 0; l < n_layers; ++l) {
-        PruneLayer e;
+        PruneLayer &e = c.layers[l];
+        std::memset(&e, 0, sizeof(e));
         e.score = scores[l];
-        e.mask = masks ? masks[l] : nullptr;
-        e.colkeep = d_colkeep.empty() ? nullptr : d_colkeep[l];
-        e.tcol0 = d_tables + n_flat;
-        e.norms = d_norms + lt[l].norm_off;
+        e.mask = masks[l];
         e.K = K[l];
         e.N = N[l];
-        e.n_tiles = (int32_t)lt[l].tcol0.size() - 1;
+        e.granularity = granularity;
+        e.n_tiles = (int32_t)(((int64_t)N[l] + granularity - 1) / granularity);
         e.flags = flags;
-        e.rt_begin = n_pairs;
-        e.el_begin = n_elems;
-        n_pairs += (int64_t)e.K * e.n_tiles;
-        n_elems += (int64_t)((e.K + kFillRows - 1) / kFillRows) * ((e.N + 15) / 16);
-        std::memcpy(&pl[l], &e, sizeof(e));
-        std::memcpy(flat + n_flat, lt[l].tcol0.data(), sizeof(int32_t) * lt[l].tcol0.size());
-        n_flat += lt[l].tcol0.size();
+        e.rt_begin = c.n_items;
+        e.el_begin = c.n_fill;
+        e.col_begin = c.n_cols;
+        c.n_norms += (int64_t)e.K * e.n_tiles;
+        c.n_items += (int64_t)((e.K + kNormRows - 1) / kNormRows) * e.n_tiles;
+        c.n_fill += (((int64_t)e.K + kFillRows - 1) / kFillRows * (((int64_t)e.N + 15) / 16) + kFillUnits - 1) / kFillUnits;
+        c.n_tcol += e.n_tiles + 1;
+        c.n_cols += e.N;
     }
-    TW_HIP(hipMemcpyAsync(d_both, both.data(), both.size(), hipMemcpyHostToDevice, s));
-    TW_HIP(hipStreamSynchronize(s)); // `both` is pageable host memory
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)((n_pairs * 8 + 255) / 256)), dim3(256),
-                       0, s, d_table, n_layers, n_pairs);
-    TW_HIP(hipGetLastError());
-    // per-tile thresholds (one layer): every tile's K norms are one segment
-    const int n_seg = (flags & kPerTileThreshold) ? (int)lt[0].tcol0.size() - 1 : 1;
-    int st = percentile_linear(ar, d_norms, total / n_seg, q, q_is_f64, s, thr, n_seg);
+    return c;
+}
+
+int too_large(int64_t workgroups)
+{
+    return workgroups > 0x7fffffff ? fail(TW_ERR_SHAPE, "%lld workgroups: a launch takes at most 2^31 - 1", (long long)workgroups)
+                                   : TW_OK;
+}
+
+// tiles of `granularity` columns: norms of all layers into one pooled vector, one threshold (or, with
+// kPerTileThreshold, one per tile of the only layer), masks.  *threshold receives it.
+int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double q, int q_is_f64,
+                 int granularity, uint8_t *const *masks, double *threshold, hipStream_t s, int flags)
+{
+    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, flags);
+    const int n_seg = (flags & kPerTileThreshold) ? c.layers[0].n_tiles : 1;
+    int st = check_percentile(c.n_norms / n_seg, q);
+    if (!st)
+        st = too_large(std::max(c.n_items, c.n_fill));
     if (st)
         return st;
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)((n_elems + 255) / 256)), dim3(256), 0, s,
-                       d_table, n_layers, n_elems, thr->state, thr->is_f64);
+    Arena ar(s);
+    float *d_norms = ar.alloc_n<float>(c.n_norms);
+    PruneLayer *d_table = ar.alloc_n<PruneLayer>(n_layers);
+    SelectState *d_st = ar.alloc_n<SelectState>(n_seg);
+    double *mail = ar.mail();
+    if (!d_norms || !d_table || !d_st || !mail)
+        return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
+    int64_t off = 0;
+    for (PruneLayer &e : c.layers) {
+        e.norms = d_norms + off;
+        off += (int64_t)e.K * e.n_tiles;
+    }
+    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, d_st, n_seg, c.n_norms / n_seg, q, q_is_f64, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers,
+                       (const int64_t *)nullptr);
+    // per-tile thresholds (one layer): every tile's K norms are one segment
+    st = queue_select(d_norms, c.n_norms / n_seg, d_st, n_seg, s);
+    if (st)
+        return st;
+    if (flags & kPerTileThreshold)
+        hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st);
+    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st,
+                       (const double *)nullptr, mail);
     TW_HIP(hipGetLastError());
-    return TW_OK; // the caller reads the threshold back, which waits for the stream
+    st = ar.wait();
+    if (!st && threshold)
+        *threshold = mail[0];
+    return st;
 }
 
 } // namespace
@@ -928,6 +1574,10 @@ try {
     if (c != N)
         return fail(TW_ERR_TILE_TABLE, "tiles cover %d columns, N=%d", c, N);
     tcol0[n_tiles] = N;
+    const int64_t n_items = (int64_t)((K + kNormRows - 1) / kNormRows) * n_tiles;
+    int st = too_large(n_items);
+    if (st)
+        return st;
     hipStream_t s = (hipStream_t)stream;
     Arena ar(s);
     int32_t *d_tab = ar.alloc_n<int32_t>(n_tiles + 1);
@@ -935,26 +1585,22 @@ try {
     if (!d_tab || !d_table)
         return fail(TW_ERR_ALLOC, "hipMalloc of the tile table failed");
     PruneLayer e;
+    std::memset(&e, 0, sizeof(e));
     e.score = scores;
-    e.mask = nullptr;
-    e.colkeep = col_keep;
+    e.colkeep = const_cast<uint8_t *>(col_keep); // (read only)
     e.tcol0 = d_tab;
     e.norms = norms;
     e.K = K;
     e.N = N;
     e.n_tiles = n_tiles;
-    e.flags = 0;
-    e.rt_begin = 0;
-    e.el_begin = 0;
-    TW_HIP(hipMemcpyAsync(d_tab, tcol0.data(), sizeof(int32_t) * (n_tiles + 1), hipMemcpyHostToDevice, s));
-    TW_HIP(hipMemcpyAsync(d_table, &e, sizeof(e), hipMemcpyHostToDevice, s));
-    TW_HIP(hipStreamSynchronize(s));
-    const int64_t n_pairs = (int64_t)K * n_tiles;
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)((n_pairs * 8 + 255) / 256)), dim3(256), 0, s,
-                       d_table, 1, n_pairs);
+    st = put_table(tcol0.data(), sizeof(int32_t) * (n_tiles + 1), d_tab, nullptr, 0, 0, 0.0, 0, s);
+    if (!st)
+        st = put_table(&e, sizeof(e), d_table, nullptr, 0, 0, 0.0, 0, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)n_items), dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr);
     TW_HIP(hipGetLastError());
-    TW_HIP(hipStreamSynchronize(s));
-    return TW_OK;
+    return ar.wait();
 }
 TW_CATCH_TO_STATUS
 
@@ -969,13 +1615,13 @@ try {
     ColLayer *d_cl = ar.alloc_n<ColLayer>(1);
     if (!d_cl)
         return fail(TW_ERR_ALLOC, "hipMalloc of the layer table failed");
-    const ColLayer cl{scores, K, N, 0};
-    TW_HIP(hipMemcpyAsync(d_cl, &cl, sizeof(cl), hipMemcpyHostToDevice, s));
-    TW_HIP(hipStreamSynchronize(s));
-    hipLaunchKernelGGL(col_norms_kernel, dim3((N + 63) / 64), dim3(64), 0, s, d_cl, 1, (int64_t)N, norms);
+    const ColLayer cl{scores, K, N, 0, 0};
+    const int st = put_table(&cl, sizeof(cl), d_cl, nullptr, 0, 0, 0.0, 0, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(col_norms_kernel, dim3((N + kColCols - 1) / kColCols), dim3(kColThreads), 0, s, d_cl, 1, norms);
     TW_HIP(hipGetLastError());
-    TW_HIP(hipStreamSynchronize(s));
-    return TW_OK;
+    return ar.wait();
 }
 TW_CATCH_TO_STATUS
 
@@ -986,12 +1632,23 @@ try {
         return fail(TW_ERR_NULL, "a pointer is NULL");
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
-    Threshold t;
-    Arena ar((hipStream_t)stream);
-    int st = percentile_linear(ar, values, n, q, q_type, (hipStream_t)stream, &t);
+    hipStream_t s = (hipStream_t)stream;
+    int st = check_percentile(n, q);
+    if (st)
+        return st;
+    Arena ar(s);
+    SelectState *d_st = ar.alloc_n<SelectState>(1);
+    if (!d_st)
+        return fail(TW_ERR_ALLOC, "hipMalloc of the selection state failed");
+    st = put_table(nullptr, 0, d_st, d_st, 1, n, q, q_type, s);
     if (!st)
-        st = read_threshold(t, (hipStream_t)stream, result);
-    return st;
+        st = queue_select(values, n, d_st, 1, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(256), 0, s, d_st);
+    TW_HIP(hipGetLastError());
+    TW_HIP(hipMemcpyAsync(result, &d_st->thr64, sizeof(double), hipMemcpyDeviceToHost, s));
+    return ar.wait();
 }
 TW_CATCH_TO_STATUS
 
@@ -1004,22 +1661,7 @@ try {
         return st;
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
-    std::vector<LayerTiles> lt(n_layers);
-    for (int l = 0; l < n_layers; ++l) {
-        for (int c = 0; c < N[l]; c += granularity)
-            lt[l].tcol0.push_back(c);
-        lt[l].tcol0.push_back(N[l]);
-    }
-    Threshold thr;
-    Arena ar((hipStream_t)stream);
-    st = rows_stage(ar, n_layers, K, N, scores, lt, {}, sparsity, q_type, masks, &thr,
-                    (hipStream_t)stream);
-    double value = 0.0;
-    if (!st)
-        st = read_threshold(thr, (hipStream_t)stream, &value); // also: the masks are complete
-    if (!st && threshold)
-        *threshold = value;
-    return st;
+    return uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, masks, threshold, (hipStream_t)stream, 0);
 }
 TW_CATCH_TO_STATUS
 
@@ -1035,17 +1677,8 @@ try {
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
     if (N % granularity != 0)
         return fail(TW_ERR_SHAPE, "N=%d is not a multiple of the granularity %d", N, granularity);
-    std::vector<LayerTiles> lt(1);
-    for (int c = 0; c <= N; c += granularity)
-        lt[0].tcol0.push_back(c);
-    Threshold thr;
-    Arena ar((hipStream_t)stream);
-    st = rows_stage(ar, 1, &K, &N, sc, lt, {}, sparsity, q_type, mk, &thr, (hipStream_t)stream,
-                    kNormNotDivided | kPerTileThreshold);
-    double value = 0.0;
-    if (!st)
-        st = read_threshold(thr, (hipStream_t)stream, &value); // waits for the mask
-    return st;
+    return uniform_rows(1, &K, &N, sc, sparsity, q_type, granularity, mk, nullptr, (hipStream_t)stream,
+                        kNormNotDivided | kPerTileThreshold);
 }
 TW_CATCH_TO_STATUS
 
@@ -1068,65 +1701,59 @@ try {
         q = 100.0 - std::sqrt(10000.0 - sparsity * 100.0);
         q_type = TW_Q_F64;
     }
-    // columns: one pooled vector of column norms, one threshold
-    int64_t total_n = 0;
-    std::vector<int64_t> coff(n_layers);
-    for (int l = 0; l < n_layers; ++l) {
-        coff[l] = total_n;
-        total_n += N[l];
-    }
-    Arena ar((hipStream_t)stream);
-    float *d_cnorm = ar.alloc_n<float>(total_n);
-    uint8_t *d_ckeep = ar.alloc_n<uint8_t>(total_n);
-    ColLayer *d_cl = ar.alloc_n<ColLayer>(n_layers);
-    if (!d_cnorm || !d_ckeep || !d_cl)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %lld column norms failed", (long long)total_n);
-    std::vector<ColLayer> cl(n_layers);
-    for (int l = 0; l < n_layers; ++l)
-        cl[l] = ColLayer{scores[l], K[l], N[l], coff[l]};
-    TW_HIP(hipMemcpyAsync(d_cl, cl.data(), sizeof(ColLayer) * n_layers, hipMemcpyHostToDevice, s));
-    TW_HIP(hipStreamSynchronize(s)); // `cl` is pageable host memory
-    hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)((total_n + 63) / 64)), dim3(64), 0, s, d_cl,
-                       n_layers, total_n, d_cnorm);
-    TW_HIP(hipGetLastError());
-    Threshold thr_c;
-    st = percentile_linear(ar, d_cnorm, total_n, q, q_type, s, &thr_c);
+    // columns: one pooled vector of column norms, one threshold; then, without a trip to the host,
+    // the tiles and the rows
+    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, 0);
+    st = check_percentile(c.n_cols, q);
+    if (!st)
+        st = too_large(std::max({c.n_items, c.n_fill, c.n_cols}));
     if (st)
         return st;
-    hipLaunchKernelGGL(col_keep_kernel, dim3((unsigned)((total_n + 255) / 256)), dim3(256), 0, s,
-                       d_cnorm, (int)total_n, thr_c.state, thr_c.is_f64, d_ckeep);
-    TW_HIP(hipGetLastError());
-    std::vector<uint8_t> h_keep(total_n);
-    TW_HIP(hipMemcpyAsync(h_keep.data(), d_ckeep, (size_t)total_n, hipMemcpyDeviceToHost, s));
-    TW_HIP(hipStreamSynchronize(s));
-    // tiles end after every `granularity` kept columns
-    std::vector<LayerTiles> lt(n_layers);
-    std::vector<uint8_t *> d_colkeep(n_layers);
-    std::vector<int32_t> col0, width;
+    Arena ar(s);
+    float *d_cnorm = ar.alloc_n<float>(c.n_cols);
+    uint8_t *d_ckeep = ar.alloc_n<uint8_t>(c.n_cols);
+    int32_t *d_tcol = ar.alloc_n<int32_t>(c.n_tcol);
+    float *d_norms = ar.alloc_n<float>(c.n_norms);
+    int64_t *d_items = ar.alloc_n<int64_t>(2); // the number of items; the columns' threshold
+    double *d_thr_cols = reinterpret_cast<double *>(d_items + 1);
+    SelectState *d_st = ar.alloc_n<SelectState>(1);
+    // both layer tables in one buffer: one upload
+    const size_t table_bytes = sizeof(PruneLayer) * n_layers;
+    char *d_tables = static_cast<char *>(ar.alloc(table_bytes + sizeof(ColLayer) * n_layers));
+    double *mail = ar.mail();
+    if (!d_cnorm || !d_ckeep || !d_tcol || !d_norms || !d_items || !d_st || !d_tables || !mail)
+        return fail(TW_ERR_ALLOC, "allocation for %lld columns and %lld norms failed", (long long)c.n_cols, (long long)c.n_norms);
+    PruneLayer *d_table = reinterpret_cast<PruneLayer *>(d_tables);
+    ColLayer *d_cl = reinterpret_cast<ColLayer *>(d_tables + table_bytes);
+    std::vector<char> both(table_bytes + sizeof(ColLayer) * n_layers);
+    int64_t n_blk = 0, n_tcol = 0;
     for (int l = 0; l < n_layers; ++l) {
-        col0.resize(N[l]);
-        width.resize(N[l]);
-        int32_t nt = 0;
-        st = tw_tiles_every_g_kept_columns(N[l], granularity, h_keep.data() + coff[l], col0.data(),
-                                           width.data(), &nt);
-        if (st)
-            return st;
-        lt[l].tcol0.assign(col0.begin(), col0.begin() + nt);
-        lt[l].tcol0.push_back(N[l]);
-        d_colkeep[l] = d_ckeep + coff[l];
-        if (col_masks && col_masks[l])
-            TW_HIP(hipMemcpyAsync(col_masks[l], d_colkeep[l], (size_t)N[l], hipMemcpyDeviceToDevice, s));
+        PruneLayer &e = c.layers[l];
+        e.colkeep = d_ckeep + e.col_begin;
+        e.colout = col_masks ? col_masks[l] : nullptr;
+        e.tcol0 = d_tcol + n_tcol;
+        n_tcol += e.n_tiles + 1;
+        const ColLayer cl{scores[l], K[l], N[l], e.col_begin, n_blk};
+        std::memcpy(both.data() + table_bytes + sizeof(ColLayer) * l, &cl, sizeof(cl));
+        n_blk += (N[l] + kColCols - 1) / kColCols;
     }
-    Threshold thr_r;
-    st = rows_stage(ar, n_layers, K, N, scores, lt, d_colkeep, q, q_type, masks, &thr_r, s);
-    double vc = 0.0, vr = 0.0;
-    if (!st)
-        st = read_threshold(thr_c, s, &vc);
-    if (!st)
-        st = read_threshold(thr_r, s, &vr);
+    std::memcpy(both.data(), c.layers.data(), table_bytes);
+    st = put_table(both.data(), both.size(), d_tables, d_st, 1, 0, q, q_type, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)n_blk), dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm);
+    hipLaunchKernelGGL(plan_2d_kernel, dim3(1), dim3(kPlanThreads), 0, s, d_table, n_layers, d_cnorm, c.n_cols, d_norms,
+                       d_thr_cols, d_st, d_items, q, q_type);
+    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, d_items);
+    st = queue_select(d_norms, c.n_norms, d_st, 1, s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_thr_cols, mail);
+    TW_HIP(hipGetLastError());
+    st = ar.wait();
     if (!st && thresholds) {
-        thresholds[0] = vc;
-        thresholds[1] = vr;
+        thresholds[0] = mail[1];
+        thresholds[1] = mail[0];
     }
     return st;
 }
@@ -1145,38 +1772,49 @@ try {
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
     hipStream_t s = (hipStream_t)stream;
     std::vector<MixLayer> ml(n_layers);
-    int64_t total = 0;
+    int64_t total = 0, n_items = 0;
     for (int l = 0; l < n_layers; ++l) {
         if (!layer_masks[l])
             return fail(TW_ERR_NULL, "layer %d: layer mask pointer is NULL", l);
-        ml[l].score = scores[l];
-        ml[l].mask0 = layer_masks[l];
-        ml[l].out = masks[l];
-        ml[l].begin = total;
-        total += (int64_t)K[l] * N[l];
+        ml[l] = MixLayer{scores[l], layer_masks[l], masks[l], (int64_t)K[l] * N[l], total, n_items};
+        total += ml[l].n;
+        n_items += (ml[l].n + kMixItem - 1) / kMixItem;
     }
-    Arena ar(s);
-    float *d_pool = ar.alloc_n<float>(total);
-    MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
-    if (!d_pool || !d_layers)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %lld element scores failed", (long long)total);
-    TW_HIP(hipMemcpyAsync(d_layers, ml.data(), sizeof(MixLayer) * n_layers, hipMemcpyHostToDevice, s));
-    TW_HIP(hipStreamSynchronize(s)); // `ml` is pageable host memory
-    const unsigned grid = (unsigned)std::min<int64_t>((total + 1023) / 1024, 256 * 32);
-    hipLaunchKernelGGL(mix_values_kernel, dim3(grid), dim3(256), 0, s, d_layers, n_layers, total,
-                       d_pool);
-    TW_HIP(hipGetLastError());
-    Threshold thr;
-    st = percentile_linear(ar, d_pool, total, 100.0 - g1percent, q_type, s, &thr);
+    const double q = 100.0 - g1percent;
+    st = check_percentile(total, q);
     if (st)
         return st;
-    hipLaunchKernelGGL(mix_mask_kernel, dim3(grid), dim3(256), 0, s, d_layers, n_layers, total,
-                       d_pool, thr.state, thr.is_f64);
+    Arena ar(s);
+    // room for the values inside the bracket: an eighth of the elements, and all of a small network's
+    const int wgs = (int)std::min<int64_t>(n_items, kMixWgs), waves = wgs * 4;
+    const int64_t share = (n_items + wgs - 1) / wgs * (kMixItem / 4); // elements of a wave
+    const uint32_t room = (uint32_t)(total > kMixSampleFrom ? std::max<int64_t>(share / 8, 512) : share);
+    float *d_cand = ar.alloc_n<float>((size_t)waves * room);
+    MixCounts *d_counts = ar.alloc_n<MixCounts>(waves);
+    uint32_t *d_sample = ar.alloc_n<uint32_t>(kMixSamples);
+    MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
+    SelectState *d_st = ar.alloc_n<SelectState>(1);
+    double *mail = ar.mail();
+    if (!d_cand || !d_counts || !d_sample || !d_layers || !d_st || !mail)
+        return fail(TW_ERR_ALLOC, "allocation for %lld element scores failed", (long long)total);
+    st = put_table(ml.data(), sizeof(MixLayer) * n_layers, d_layers, d_st, 1, total, q, q_type, s, room);
+    if (st)
+        return st;
+    if (total > kMixSampleFrom) {
+        hipLaunchKernelGGL(mix_sample_kernel, dim3(kMixSamples / 256), dim3(256), 0, s, d_layers, n_layers, total, d_sample);
+        hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample, d_st);
+    }
+    hipLaunchKernelGGL(mix_narrow_kernel, dim3(wgs), dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts);
+    const dim3 grid((unsigned)std::min<int64_t>(n_items, 512));
+    hipLaunchKernelGGL(mix_hist_kernel<0>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
+    hipLaunchKernelGGL(mix_hist_kernel<1>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
+    hipLaunchKernelGGL(mix_hist_kernel<2>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
+    hipLaunchKernelGGL(mix_mask_kernel, dim3((unsigned)std::min<int64_t>(n_items, 2048)), dim3(256), 0, s, d_layers, n_layers,
+                       n_items, d_st, d_cand, mail);
     TW_HIP(hipGetLastError());
-    double value = 0.0;
-    st = read_threshold(thr, s, &value); // waits for the masks
+    st = ar.wait();
     if (!st && threshold)
-        *threshold = value;
+        *threshold = mail[0];
     return st;
 }
 TW_CATCH_TO_STATUS

@@ -34,37 +34,62 @@ def img2col_forward(accumulated_scores):
 
 
 class _DeviceLayers:
-    """Scores uploaded to the GPU and mask buffers, as pointer tables for the C ABI."""
+    """Scores on the GPU (uploaded where they are not there yet) and mask buffers, as pointer tables
+    for the C ABI.  The masks of a call are views of one allocation, each starting at a multiple of
+    256 bytes, and so are the column masks, made when they are first asked for."""
 
     def __init__(self, scores):
         import torch
         self.torch = torch
-        self.shapes = []
-        self.d_scores, self.d_masks, self.d_cols = [], [], []
+        self.d_scores = d_scores = []
         for s in scores:
             if isinstance(s, torch.Tensor):
-                t = s.detach().to(device="cuda", dtype=torch.float32)
+                if s.is_cuda and s.dtype is torch.float32:
+                    t = s.detach() if s.requires_grad else s
+                else:
+                    t = s.detach().to(device="cuda", dtype=torch.float32)
             else:
                 t = torch.from_numpy(np.ascontiguousarray(s, dtype=np.float32)).cuda()
             if t.dim() == 4:
                 t = t.reshape(-1, t.shape[-1])
             if t.dim() != 2:
                 raise tw.TwError(tw.ERR_SHAPE, "a score tensor must be 2-D or 4-D")
-            t = t.contiguous()
-            self.shapes.append(tuple(t.shape))
-            self.d_scores.append(t)
-            self.d_masks.append(torch.empty(t.shape, dtype=torch.uint8, device="cuda"))
-            self.d_cols.append(torch.empty(t.shape[1], dtype=torch.uint8, device="cuda"))
-        n = len(scores)
-        self.K = np.array([s[0] for s in self.shapes], np.int32)
-        self.N = np.array([s[1] for s in self.shapes], np.int32)
-        self.p_scores = (ctypes.c_void_p * n)(*[t.data_ptr() for t in self.d_scores])
-        self.p_masks = (ctypes.c_void_p * n)(*[t.data_ptr() for t in self.d_masks])
-        self.p_cols = (ctypes.c_void_p * n)(*[t.data_ptr() for t in self.d_cols])
+            d_scores.append(t if t.is_contiguous() else t.contiguous())
+        n = len(d_scores)
+        self.shapes = [tuple(t.shape) for t in d_scores]
+        self.K = np.array([k for k, _ in self.shapes], np.int32)
+        self.N = np.array([w for _, w in self.shapes], np.int32)
+        self.p_scores = (ctypes.c_void_p * n)(*[t.data_ptr() for t in d_scores])
+        self.d_masks, self.p_masks = self._views([(k, w) for k, w in self.shapes], n)
+        self._cols = None
         self.stream = torch.cuda.current_stream().cuda_stream
+
+    def _views(self, shapes, n):
+        torch = self.torch
+        offsets, total = [], 0
+        for shape in shapes:
+            offsets.append(total)
+            total += -(-(shape[0] * (shape[1] if len(shape) == 2 else 1)) // 256) * 256
+        flat = torch.empty(total, dtype=torch.uint8, device="cuda")
+        base, cut = flat.data_ptr(), torch.as_strided
+        views = [cut(flat, s, (s[1], 1) if len(s) == 2 else (1,), o) for s, o in zip(shapes, offsets)]
+        return views, (ctypes.c_void_p * n)(*[base + o for o in offsets])
+
+    def _make_cols(self):
+        if self._cols is None:
+            self._cols = self._views([(w,) for _, w in self.shapes], len(self.shapes))
+        return self._cols
+
+    d_cols = property(lambda self: self._make_cols()[0])
+    p_cols = property(lambda self: self._make_cols()[1])
 
     def masks(self):
         return [m.cpu().numpy().astype(bool) for m in self.d_masks]
+
+    def host_cols(self):
+        """The column masks in host memory: one copy for all layers."""
+        host = self.torch.cat(self.d_cols).cpu().numpy()
+        return np.split(host, np.cumsum(self.N)[:-1])
 
 
 def tiled_wise_1d(accumulated_scores, sparsity, granularity=128, return_device=False):
@@ -99,7 +124,7 @@ def tiled_wise_2d(accumulated_scores, sparsity, granularity=128, transform=True,
     masks = d.d_masks if return_device else d.masks()
     if not return_tiles:
         return masks
-    tables = [tiles_every_g_kept_columns(c.cpu().numpy(), granularity) for c in d.d_cols]
+    tables = [tiles_every_g_kept_columns(c, granularity) for c in d.host_cols()]
     return masks, tables
 
 
@@ -146,8 +171,7 @@ def tiled_wise_2d_mix(accumulated_scores, sparsity, granularity=128, g1percent=1
     tw._check(tw.lib().tw_prune_tiled_wise_2d(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
         ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(q), _q_type(q), 1,
-        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)),
-        ctypes.cast(d.p_cols, ctypes.POINTER(ctypes.c_void_p)), None, d.stream))
+        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), None, None, d.stream))
     return _mix(d, g1percent, return_device)
 
 
@@ -184,7 +208,7 @@ def tiles_every_g_kept_columns(col_mask, granularity):
     tw._check(L.tw_tiles_every_g_kept_columns(cm.size, int(granularity), tw._ptr(cm, ctypes.c_uint8),
                                               tw._ptr(col0, ctypes.c_int32),
                                               tw._ptr(width, ctypes.c_int32), ctypes.byref(n)))
-    return [(int(col0[i]), int(width[i])) for i in range(n.value)]
+    return list(zip(col0[:n.value].tolist(), width[:n.value].tolist()))
 
 
 def tile_row_norms(score, tile_table, col_keep=None):
