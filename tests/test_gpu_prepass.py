@@ -75,6 +75,41 @@ def test_plan_from_mask_full_size_configurations(tw, oracle, name):
         assert inf["kept_elems"] == int(mask.sum()) and inf["total_width"] == N
 
 
+@pytest.mark.parametrize("K,N,widths,offset", [
+    (300, 256, [135, 121], 0),             # a tile that starts and ends inside a 16-byte piece
+    (65, 640, [5, 123, 510, 2], 0),        # one, two and three windows of columns; a slab of one row
+    (130, 4400, [4300, 100], 0),           # more columns than one window of the list kernel
+    (9000, 48, [17, 1, 30], 0),            # more rows than one round of it
+    (200, 131, [64, 67], 0),               # rows off 4 bytes
+    (200, 132, [60, 72], 4),               # rows on 4 bytes, not on 16
+    (200, 128, [60, 68], 1),               # a mask off 4 bytes
+])
+def test_plan_from_device_mask_tile_edges(tw, oracle, K, N, widths, offset):
+    """Tile tables and mask addresses that fall outside the aligned cases, bit for bit.  The device
+    memory around the call is dirtied first: nothing the kernels read may be left over."""
+    import torch
+    rng = np.random.default_rng(K + N + offset)
+    table, tiles, c = [], [], 0
+    for w in widths:
+        kk = np.sort(rng.choice(K, max(1, K // 3), replace=False))
+        kn = np.sort(rng.choice(w, max(1, 2 * w // 3), replace=False))
+        tiles.append(dict(col0=c, width=w, kept_k=kk.astype(np.int32), kept_n=kn.astype(np.int32)))
+        table.append((c, w))
+        c += w
+    mask = oracle.plan_mask(K, N, tiles)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    junk = [torch.full((1 << 20,), 0xFF, dtype=torch.uint8, device="cuda") for _ in range(4)]
+    del junk
+    torch.cuda.empty_cache()
+    buf = torch.full((K * N + 64,), 7, dtype=torch.uint8, device="cuda")
+    buf[offset:offset + K * N] = torch.from_numpy(np.ascontiguousarray(mask, np.uint8)).cuda().reshape(-1)
+    dB = torch.from_numpy(B).cuda()
+    for _ in range(2):
+        with tw.Plan.from_device_mask(K, N, buf.data_ptr() + offset, table, "bf16", dB.data_ptr(),
+                                      stream=torch.cuda.current_stream().cuda_stream) as plan:
+            check_export(oracle, plan, tiles, B, "bf16")
+
+
 def test_plan_from_mask_rejects_non_tw_mask(tw):
     K, N, G = 64, 128, 32
     mask = np.zeros((K, N), np.uint8)

@@ -116,7 +116,7 @@ struct tw_plan {
     int K = 0, N = 0, dtype = 0, n_tiles = 0;
     int device = 0;
     // host copies
-    std::vector<int32_t> tile_col0, tile_width, kept_k_ptr, kept_k_idx, kept_n_ptr, kept_n_idx;
+    std::vector<int32_t> tile_col0, tile_width, kept_k_ptr, kept_n_ptr;
     std::vector<int32_t> k_pad, n_pad;
     std::vector<int64_t> b_off; // element offset of each tile's packed weight
     int64_t packed_elems = 0;
@@ -135,13 +135,9 @@ struct tw_plan {
     int32_t *d_blocks = nullptr;
     int n_blocks = 0;
     uint32_t *d_kept_pairs = nullptr; // GemmArgs::kept_pairs
-    // Ownership: every pointer above points into one of these two allocations.  d_lists holds the
-    // four index arrays when the pre-pass compacted them on the device (else they sit in d_slab);
-    // d_slab holds the unit / tile tables, the pruned-column and padded kept-K lists, the packing
-    // table, the ticket slots and the packed weight.
-    void *d_lists = nullptr;
+    // Ownership: every pointer above points into this one allocation.
     void *d_slab = nullptr;
-    void *d_pack_tiles = nullptr; // tw::PackTile[n_tiles] for packing from a dense weight
+    void *d_plan_tiles = nullptr; // tw_plan.hip's table of the tiles
     mutable unsigned next_slot = 0, next_capture_slot = 0;
     int blocks_per_unit = 0; // 32-column blocks of every unit where all units have the same number, else 0
     int n_halves = 0;   // pieces of 64 compact columns over all units (the skinny kernel's work per row block)
@@ -183,15 +179,6 @@ int validate_lists(int K, int N, int n_tiles, const int32_t *tile_col0, const in
                    const int32_t *kept_k_ptr, const int32_t *kept_k_idx,
                    const int32_t *kept_n_ptr, const int32_t *kept_n_idx);
 
-// fills the host-side geometry (k_pad, n_pad, b_off, packed_elems) of a plan whose
-// lists are set, uploads lists/units/tiles and allocates the packed weight (zeroed); the copies
-// run on `s`, which is waited for.
-int finalize_plan_geometry(tw_plan *p, hipStream_t s);
-
-// device pack: packed weight from a row-major fp32 [K,N] device buffer
-int pack_from_dense(tw_plan *p, const float *d_B, hipStream_t s, const uint8_t *d_mask = nullptr);
-// device pack: packed weight from the reference's compacted stream layout (16-bit, device)
-int pack_from_stream(tw_plan *p, const void *d_Bs, const int64_t *off_B, hipStream_t s);
 // true when tw_gemm_ex takes a row-major A and a row-major C of this plan with a kernel of its own
 // (no layout-generic kernel, no staging): K short enough for a panel of A in LDS and C not read
 bool takes_row_major_directly(const tw_plan *p, float beta);
@@ -200,7 +187,5 @@ bool takes_row_major_directly(const tw_plan *p, float beta);
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
 int launch_bs(const tw_plan *p, const GemmArgs &a, int per_cu, hipStream_t s);
 double bs_fill(const tw_plan *p, int M); // share of the chip's workgroup slots its launch fills
-// device unpack: compacted stream layout (K*N 16-bit, zero elsewhere) from the packed weight
-int unpack_to_stream(const tw_plan *p, uint16_t *d_Bs, hipStream_t s);
 
 } // namespace tw

@@ -11,15 +11,24 @@
 #include "tw_internal.h"
 
 #include <algorithm>
+#include <atomic>
+#include <climits>
 #include <cstring>
+#include <map>
 #include <mutex>
 
 namespace tw {
 
 constexpr int kPackKS = kBlockK / kMfmaK; // MFMA k steps per packed step
 
-struct PackTile {
-    int32_t col0, k_kept, n_kept, k_pad, n_pad, kk_off, kn_off, pad_;
+// One tile of a plan being built: its geometry, where its lists lie among the ones they are made from
+// (kk_src, kn_src, pn_src) and where they go (kk_dst ...; see GemmArgs for the padded copies).
+struct PlanTile {
+    int32_t col0, k_kept, n_kept, k_pad, n_pad, n_pruned;
+    int32_t kk_dst, kn_dst, pn_dst;
+    int32_t kkp_dst, kkp_len;  // its stretch of the padded list of rows
+    int32_t pad_;
+    int64_t kk_src, kn_src, pn_src;
     int64_t b_off;
     int64_t src_off; // stream layout only: element offset of the tile in B_stream
 };
@@ -47,427 +56,432 @@ __device__ __forceinline__ uint16_t cast16(float f, int dtype)
 // ---------------------------------------------------------------------------------
 // packing
 
-// `mask` (optional, K x N bytes): elements whose mask byte is zero are stored as zeros (covering
-// plans of masks that are not rows x columns per tile)
-__global__ void pack_dense_kernel(const PackTile *tiles, const int32_t *kept_k,
-                                  const int32_t *kept_n, const float *B, int N, int dtype,
-                                  uint16_t *Bp, const uint8_t *mask)
+// Group g of a tile's packed weight: eight k rows of one column, the sixteen bytes of one lane.
+struct PackPos {
+    int n, kk0; // compact column, first compact row
+    bool any;   // inside the tile's packed weight
+};
+__device__ __forceinline__ PackPos pack_pos(const PlanTile &t, int64_t g)
 {
-    const PackTile t = tiles[blockIdx.y];
-    const int64_t groups = (int64_t)t.k_pad * t.n_pad / 8;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= groups)
-        return;
+    PackPos q;
+    q.any = g < (int64_t)t.k_pad * t.n_pad / 8;
     const int lane = (int)(g & 63);
-    const int64_t blk = g >> 6; // ((step * nblk + nb) * kPackKS + ks)
-    const int nblk = t.n_pad / kMfmaN;
-    const int ks = (int)(blk % kPackKS);
-    const int nb = (int)((blk / kPackKS) % nblk);
-    const int k16 = (int)((blk / kPackKS) / nblk) * kPackKS + ks;
-    const int n = nb * kMfmaN + (lane & 31);
-    const int kk0 = k16 * kMfmaK + (lane >> 5) * 8;
-    uint16_t v[8];
-    int col = -1;
-    if (n < t.n_kept)
-        col = t.col0 + kept_n[t.kn_off + n];
+    const uint32_t blk = (uint32_t)(g >> 6); // ((step * nblk + nb) * kPackKS + ks)
+    const uint32_t nblk = max(t.n_pad / kMfmaN, 1);
+    const uint32_t step = blk / kPackKS / nblk;
+    q.n = (int)(blk / kPackKS - step * nblk) * kMfmaN + (lane & 31);
+    q.kk0 = (int)(step * kPackKS + blk % kPackKS) * kMfmaK + (lane >> 5) * 8;
+    return q;
+}
+__device__ __forceinline__ void pack_put(uint16_t *Bp, const PlanTile &t, int64_t g, const uint16_t (&v)[8])
+{
+    uint4 out;
+    out.x = v[0] | ((uint32_t)v[1] << 16);
+    out.y = v[2] | ((uint32_t)v[3] << 16);
+    out.z = v[4] | ((uint32_t)v[5] << 16);
+    out.w = v[6] | ((uint32_t)v[7] << 16);
+    *reinterpret_cast<uint4 *>(Bp + t.b_off + g * 8) = out;
+}
+
+// From the dense fp32 weight.  `mask` (optional, K x N bytes): elements whose mask byte is zero are
+// stored as zeros (covering plans of masks that are not rows x columns per tile).
+__device__ __forceinline__ void pack_dense(const PlanTile &t, int64_t g, const int32_t *kept_k, const int32_t *kept_n,
+                                           const float *B, int N, int dtype, uint16_t *Bp, const uint8_t *mask)
+{
+    const PackPos q = pack_pos(t, g);
+    if (!q.any)
+        return;
+    const int col = q.n < t.n_kept ? t.col0 + kept_n[t.kn_src + q.n] : -1;
+    int64_t src[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const int kk = kk0 + e;
+        const int kk = q.kk0 + e;
+        src[e] = col >= 0 && kk < t.k_kept ? (int64_t)kept_k[t.kk_src + kk] * N + col : -1;
+    }
+    uint16_t v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
         float f = 0.0f;
-        if (col >= 0 && kk < t.k_kept) {
-            const int64_t src = (int64_t)kept_k[t.kk_off + kk] * N + col;
-            if (!mask || mask[src])
-                f = B[src];
-        }
+        if (src[e] >= 0 && (!mask || mask[src[e]]))
+            f = B[src[e]];
         v[e] = cast16(f, dtype);
     }
-    uint4 out;
-    out.x = v[0] | ((uint32_t)v[1] << 16);
-    out.y = v[2] | ((uint32_t)v[3] << 16);
-    out.z = v[4] | ((uint32_t)v[5] << 16);
-    out.w = v[6] | ((uint32_t)v[7] << 16);
-    *reinterpret_cast<uint4 *>(Bp + t.b_off + g * 8) = out;
+    pack_put(Bp, t, g, v);
 }
 
-// Source is the reference's compacted layout: tile column j, row i at
-// Bs[src_off + j*K + i] (gen_masked_stream_weight, basic_nn.cu:765).
-__global__ void pack_stream_kernel(const PackTile *tiles, const uint16_t *Bs, int K, uint16_t *Bp)
+// From the reference's compacted layout: tile column j, row i at Bs[src_off + j*K + i]
+// (gen_masked_stream_weight, basic_nn.cu:765).
+__device__ __forceinline__ void pack_stream(const PlanTile &t, int64_t g, const uint16_t *Bs, int K, uint16_t *Bp)
 {
-    const PackTile t = tiles[blockIdx.y];
-    const int64_t groups = (int64_t)t.k_pad * t.n_pad / 8;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= groups)
+    const PackPos q = pack_pos(t, g);
+    if (!q.any)
         return;
-    const int lane = (int)(g & 63);
-    const int64_t blk = g >> 6; // ((step * nblk + nb) * kPackKS + ks)
-    const int nblk = t.n_pad / kMfmaN;
-    const int ks = (int)(blk % kPackKS);
-    const int nb = (int)((blk / kPackKS) % nblk);
-    const int k16 = (int)((blk / kPackKS) / nblk) * kPackKS + ks;
-    const int n = nb * kMfmaN + (lane & 31);
-    const int kk0 = k16 * kMfmaK + (lane >> 5) * 8;
     uint16_t v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const int kk = kk0 + e;
-        v[e] = (n < t.n_kept && kk < t.k_kept) ? Bs[t.src_off + (int64_t)n * K + kk] : (uint16_t)0;
+        const int kk = q.kk0 + e;
+        v[e] = (q.n < t.n_kept && kk < t.k_kept) ? Bs[t.src_off + (int64_t)q.n * K + kk] : (uint16_t)0;
     }
-    uint4 out;
-    out.x = v[0] | ((uint32_t)v[1] << 16);
-    out.y = v[2] | ((uint32_t)v[3] << 16);
-    out.z = v[4] | ((uint32_t)v[5] << 16);
-    out.w = v[6] | ((uint32_t)v[7] << 16);
-    *reinterpret_cast<uint4 *>(Bp + t.b_off + g * 8) = out;
+    pack_put(Bp, t, g, v);
 }
 
-// Inverse of the packing into the reference's compacted layout at K*col0.
-__global__ void unpack_stream_kernel(const PackTile *tiles, const uint16_t *Bp, int K, uint16_t *Bs)
+// Everything of a plan that is not known on the host.  Row t of the grid packs tile t's weight, row
+// n_tiles + t writes its lists, the last row copies the tables the host has made (units, tiles, blocks and
+// the PlanTile table itself) out of pinned host memory and clears the ticket slots.  The tiles of most
+// plans fit the kernel arguments, and then this is one launch; a plan of more runs it twice, once for
+// the lists and tables (a workgroup reads its tile's entry across the bus, next to its other first
+// loads) and once for the weight, out of the table the first has copied.
+constexpr int kArgTiles = 24;
+struct BuildArgs {
+    const PlanTile *tiles; // null: arg_tiles
+    int32_t row0;          // first row of this launch
+    int32_t n_tiles, K, N, dtype;
+    const int32_t *kk, *kn, *pn; // lists the plan is made from
+    const float *B;              // dense weight, or
+    const uint16_t *Bs;          // compacted weight in the stream layout
+    const uint8_t *mask;
+    const uint4 *header; // host
+    uint4 *header_dst;
+    int32_t *kept_k, *rel_k, *kept_n, *rel_n, *pruned_n, *kept_k_pad;
+    uint32_t *kept_pairs;
+    int32_t *tickets;
+    uint16_t *Bp;
+    int32_t header_chunks; // of 16 bytes
+    int32_t ticket_words;
+    PlanTile arg_tiles[kArgTiles];
+};
+__device__ __forceinline__ PlanTile build_tile(const BuildArgs &a, int t)
 {
-    const PackTile t = tiles[blockIdx.y];
-    const int64_t groups = (int64_t)t.k_pad * t.n_pad / 8;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= groups)
+    constexpr int W = sizeof(PlanTile) / 4;
+    int32_t w[W];
+    if (a.tiles) {
+        const auto *g = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)(a.tiles + t);
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+            w[i] = g[i];
+    } else {
+        const auto *ka = (const __attribute__((address_space(4))) int32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+#pragma unroll
+        for (int i = 0; i < W; ++i)
+            w[i] = ka[offsetof(BuildArgs, arg_tiles) / 4 + t * W + i];
+    }
+    PlanTile q;
+    __builtin_memcpy(&q, w, sizeof(q));
+    return q;
+}
+__global__ void __launch_bounds__(256) plan_build_kernel(const BuildArgs a)
+{
+    const int y = a.row0 + (int)blockIdx.y;
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+    if (y < a.n_tiles) {
+        const PlanTile t = build_tile(a, y);
+        const int64_t groups = (int64_t)t.k_pad * t.n_pad / 8;
+        for (int64_t g = i0; g < groups; g += step) {
+            if (a.B)
+                pack_dense(t, g, a.kk, a.kn, a.B, a.N, a.dtype, a.Bp, a.mask);
+            else
+                pack_stream(t, g, a.Bs, a.K, a.Bp);
+        }
         return;
-    const int lane = (int)(g & 63);
-    const int64_t blk = g >> 6; // ((step * nblk + nb) * kPackKS + ks)
-    const int nblk = t.n_pad / kMfmaN;
-    const int ks = (int)(blk % kPackKS);
-    const int nb = (int)((blk / kPackKS) % nblk);
-    const int k16 = (int)((blk / kPackKS) / nblk) * kPackKS + ks;
-    const int n = nb * kMfmaN + (lane & 31);
-    const int kk0 = k16 * kMfmaK + (lane >> 5) * 8;
-    if (n >= t.n_kept)
+    }
+    if (y == 2 * a.n_tiles) {
+        for (int64_t i = i0; i < a.header_chunks; i += step)
+            a.header_dst[i] = a.header[i];
+        for (int64_t i = i0; i < a.ticket_words; i += step)
+            a.tickets[i] = 0;
+        return;
+    }
+    const PlanTile t = build_tile(a, y - a.n_tiles);
+    for (int64_t i = i0; i < t.k_kept; i += step) {
+        const int k = a.kk[t.kk_src + i];
+        a.kept_k[t.kk_dst + i] = k;
+        a.rel_k[t.kk_dst + i] = k - (int)i;
+    }
+    for (int64_t i = i0; i < t.n_kept; i += step) {
+        const int c = a.kn[t.kn_src + i];
+        a.kept_n[t.kn_dst + i] = c;
+        a.rel_n[t.kn_dst + i] = c - (int)i;
+    }
+    for (int64_t i = i0; i < t.n_pruned; i += step)
+        a.pruned_n[t.pn_dst + i] = a.pn[t.pn_src + i];
+    for (int64_t i = i0; i < t.kkp_len; i += step)
+        a.kept_k_pad[t.kkp_dst + i] = i < t.k_kept ? a.kk[t.kk_src + i] : 0;
+    // pairs of rows (GemmArgs::kept_pairs); the padding names row K there (a row of zeros behind the
+    // A-stationary kernel's panel), not row 0.  A tile without columns has no unit and its list
+    // counts as padding.
+    if (a.kept_pairs) {
+        const int kept = t.n_kept > 0 ? t.k_kept : 0;
+        for (int64_t i = i0; i < t.kkp_len / 2; i += step) {
+            const int in = (int)(i & 31), e = in >> 2, g16 = in & 3;
+            const int lo = (int)(i >> 5) * 64 + g16 * 16 + (e >> 2) * 8 + (e & 3);
+            const uint32_t r_lo = lo < kept ? (uint32_t)a.kk[t.kk_src + lo] : (uint32_t)a.K;
+            const uint32_t r_hi = lo + 4 < kept ? (uint32_t)a.kk[t.kk_src + lo + 4] : (uint32_t)a.K;
+            a.kept_pairs[t.kkp_dst / 2 + i] = r_lo | r_hi << 16;
+        }
+    }
+}
+// Inverse of the packing into the reference's compacted layout at K*col0.
+__global__ void unpack_stream_kernel(const PlanTile *tiles, const uint16_t *Bp, int K, uint16_t *Bs)
+{
+    const PlanTile t = tiles[blockIdx.y];
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const PackPos q = pack_pos(t, g);
+    if (!q.any || q.n >= t.n_kept)
         return;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const int kk = kk0 + e;
+        const int kk = q.kk0 + e;
         if (kk < t.k_kept)
-            Bs[(int64_t)(t.col0 + n) * K + kk] = Bp[t.b_off + g * 8 + e];
+            Bs[(int64_t)(t.col0 + q.n) * K + kk] = Bp[t.b_off + g * 8 + e];
     }
 }
 
 // ---------------------------------------------------------------------------------
 // mask -> flags -> lists  (integer pre-pass)
 
-// The tile table on the device: tcol0[t] is the first column of tile t, tcol0[n_tiles] == N.
+// A tile keeps row k where any byte of mask[k][its columns] is non-zero, and a column likewise.  Two
+// kernels: mask_flags_kernel reads the mask once, mask_lists_kernel turns the flags into ascending
+// lists.  Whether the mask is rows x columns in every tile needs no second pass over it: its non-zero
+// elements lie in that product, so it is exactly when they are as many as rows times columns.
 
-// Both flag kernels walk the mask in 16-byte column chunks: thread (slice, chunk) of a block
-// handles chunk `chunk` of the rows slice, slice + 256/cw, ... of a 64-row slab, so that the cw
-// lanes next to each other read cw * 16 contiguous bytes of one row.  A chunk usually lies inside
-// one tile; chunks that straddle a tile boundary, ragged ends and unaligned masks take the
-// byte-wise path.
-
-struct ChunkPos {
-    int c0, w;       // first column and width (1..16) of the chunk
-    int t0;          // tile of the chunk's first column
-    bool one_tile;   // the whole chunk lies in tile t0
-    bool vec;        // 16-byte loads are possible
-    int k_begin, k_end, k_step;
+// Rows of one tile and slab, and what a slab of kFlagRows rows of it says about the columns.
+constexpr int kFlagRows = 128, kFlagPasses = kFlagRows / 8; // passes over the rows at 32 lanes a row
+constexpr int kMaxTileRows = 32768; // tiles of one launch, where they are the rows of its grid
+struct FlagArgs {
+    const uint8_t *mask;
+    const int32_t *tcol0; // host memory (pinned): first column of each tile, N behind the last
+    int32_t K, N, n_slabs, tile0;
+    uint8_t *rowflag;     // [tile][K]
+    uint8_t *colpart;     // per tile [slab][width, rounded up to 4], see colpart_at
+    uint32_t *nnz;        // [tile][slab]: non-zero elements
+    __device__ int64_t colpart_at(int t, int c0) const { return (int64_t)(((int64_t)c0 + 3 * t + 3) & ~(int64_t)3) * n_slabs; }
 };
 
-__device__ __forceinline__ bool chunk_pos(const uint8_t *mask, int K, int N, const int32_t *tcol0,
-                                          int n_tiles, int cw, ChunkPos &q)
+// Workgroup (slab, tile): kFlagRows rows of one tile, so every flag has one writer and nothing has to
+// be cleared first.  Each row is taken by 8, 16 or 32 lanes of 16 bytes (windows of 32 lanes for wider
+// tiles), all loads of a window in flight at once; a row's lanes vote, the rows of a column are
+// joined with shuffles and through LDS.
+__global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
 {
-    const int nchunk = (N + 15) >> 4;
-    const int chunk = blockIdx.x * cw + (int)(threadIdx.x % cw);
-    if (chunk >= nchunk)
-        return false;
-    q.c0 = chunk << 4;
-    q.w = min(16, N - q.c0);
-    int lo = 0, hi = n_tiles; // the tile with tcol0[t] <= c0 < tcol0[t+1]
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (tcol0[mid] <= q.c0)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    q.t0 = lo;
-    q.one_tile = tcol0[lo + 1] >= q.c0 + q.w;
-    q.vec = q.w == 16 && (N & 15) == 0 && ((uintptr_t)mask & 15) == 0;
-    q.k_step = 256 / cw;
-    q.k_begin = blockIdx.y * 64 + (int)(threadIdx.x / cw);
-    q.k_end = min(K, (int)blockIdx.y * 64 + 64);
-    return true;
-}
-
-// the chunk's bytes as four words, byte j of the chunk in bits 8*(j%4) of word j/4; 0 beyond w
-__device__ __forceinline__ void load_chunk(const uint8_t *src, const ChunkPos &q, uint32_t (&v)[4])
-{
-    if (q.vec) {
-        const uint4 x = *reinterpret_cast<const uint4 *>(src);
-        v[0] = x.x;
-        v[1] = x.y;
-        v[2] = x.z;
-        v[3] = x.w;
-    } else {
-        v[0] = v[1] = v[2] = v[3] = 0u;
-        for (int j = 0; j < q.w; ++j)
-            v[j >> 2] |= (uint32_t)src[j] << ((j & 3) * 8);
-    }
-}
-
-__device__ __forceinline__ uint32_t chunk_byte(const uint32_t (&v)[4], int j)
-{
-    return (v[j >> 2] >> ((j & 3) * 8)) & 0xFFu;
-}
-
-// Rows a thread loads before it looks at any of them, so that this many 16-byte loads are in
-// flight per lane.
-constexpr int kFlagBatch = 8;
-
-// rowflag[t*K + k] = 1 where any byte of mask[k][tcol0[t] .. tcol0[t+1]) is non-zero,
-// colflag[c] = 1 where any byte of column c is; both arrays start zeroed and only receive ones.
-__global__ void __launch_bounds__(256)
-    mask_flags_kernel(const uint8_t *__restrict__ mask, int K, int N,
-                      const int32_t *__restrict__ tcol0, int n_tiles, int cw,
-                      uint8_t *__restrict__ rowflag, uint8_t *__restrict__ colflag)
-{
-    ChunkPos q;
-    if (!chunk_pos(mask, K, N, tcol0, n_tiles, cw, q))
-        return;
-    // Of the lanes that hold chunks of one row inside one tile, only the lowest one with a
-    // non-zero chunk stores the row flag.  seg_mask: the lanes below this one from the tile's
-    // first whole chunk in this row on (they all lie in tile t0 when this chunk does).
-    const int lane = (int)(threadIdx.x & 63u);
-    unsigned long long seg_mask = 0ull;
-    if (q.one_tile) {
-        const int in_row = (int)(threadIdx.x % cw);
-        const int first_chunk = (tcol0[q.t0] + 15) >> 4;
-        const int seg_lane = lane - in_row + max(0, first_chunk - (int)blockIdx.x * cw);
-        seg_mask = ((1ull << lane) - 1ull) & ~((1ull << seg_lane) - 1ull);
-    }
-    uint32_t acc[4] = {0u, 0u, 0u, 0u};
-    for (int k0 = q.k_begin; k0 < q.k_end; k0 += kFlagBatch * q.k_step) {
-        uint32_t v[kFlagBatch][4];
+    __shared__ uint32_t s_col[4][128]; // per wave, a window's columns
+    __shared__ uint32_t s_nnz;
+    const int slab = (int)blockIdx.x, t = a.tile0 + (int)blockIdx.y;
+    const int c0 = a.tcol0[t], w = a.tcol0[t + 1] - c0;
+    const int k0 = slab * kFlagRows, nr = min(kFlagRows, a.K - k0);
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // the widest aligned load the mask allows: 16 bytes, 4 or 1
+    const int unit = (a.N & 15) == 0 && ((uintptr_t)a.mask & 15) == 0 ? 16 : (a.N & 3) == 0 && ((uintptr_t)a.mask & 3) == 0 ? 4 : 1;
+    const int a0 = c0 & -unit, chunks = (c0 + w - a0 + 15) >> 4;
+    const int lpr = chunks <= 8 ? 8 : chunks <= 16 ? 16 : 32; // lanes of a row
+    const int lg = lpr == 8 ? 3 : lpr == 16 ? 4 : 5;
+    const int rpp = 256 >> lg;                                // rows the workgroup takes at a time
+    const int l = tid & (lpr - 1), r0 = tid >> lg;
+    const uint8_t *const base = a.mask + (int64_t)k0 * a.N;
+    uint32_t row_any = 0; // bit p: row r0 + p * rpp has an element (this lane's chunks)
+    uint32_t nnz = 0;
+    if (tid == 0)
+        s_nnz = 0;
+    for (int win = 0; win * lpr < chunks; ++win) {
+        const int cc = a0 + (win * lpr + l) * 16; // first column of this lane's chunk
+        uint32_t v[kFlagPasses][4];
 #pragma unroll
-        for (int i = 0; i < kFlagBatch; ++i) {
-            const int k = k0 + i * q.k_step;
-            if (k < q.k_end)
-                load_chunk(mask + (int64_t)k * N + q.c0, q, v[i]);
-            else
-                v[i][0] = v[i][1] = v[i][2] = v[i][3] = 0u;
-        }
+        for (int p = 0; p < kFlagPasses; ++p) {
+            if (p * rpp >= kFlagRows)
+                break;
+            const uint8_t *const src = base + (int64_t)min(r0 + p * rpp, nr - 1) * a.N + cc;
+            if (unit == 16) {
+                const uint4 x = cc < a.N ? *reinterpret_cast<const uint4 *>(src) : uint4{0u, 0u, 0u, 0u};
+                v[p][0] = x.x, v[p][1] = x.y, v[p][2] = x.z, v[p][3] = x.w;
+            } else if (unit == 4) {
 #pragma unroll
-        for (int i = 0; i < kFlagBatch; ++i) {
-            const int k = k0 + i * q.k_step;
-            const bool nz = (v[i][0] | v[i][1] | v[i][2] | v[i][3]) != 0u;
-            // lanes of one row run the same iterations, so a row's lanes all vote here
-            const unsigned long long votes = __ballot(nz && q.one_tile);
-            if (!nz)
-                continue; // also every row past k_end
-            if (q.one_tile) {
-                if ((votes & seg_mask) == 0ull)
-                    rowflag[(int64_t)q.t0 * K + k] = 1;
+                for (int j = 0; j < 4; ++j)
+                    v[p][j] = cc + j * 4 < a.N ? *reinterpret_cast<const uint32_t *>(src + j * 4) : 0u;
             } else {
-                int t = q.t0, t_end = tcol0[t + 1];
-                uint32_t any = 0;
-                for (int j = 0; j < q.w; ++j) {
-                    if (q.c0 + j >= t_end) {
-                        if (any)
-                            rowflag[(int64_t)t * K + k] = 1;
-                        any = 0;
-                        ++t;
-                        t_end = tcol0[t + 1];
-                    }
-                    any |= chunk_byte(v[i], j);
-                }
-                if (any)
-                    rowflag[(int64_t)t * K + k] = 1;
-            }
-            acc[0] |= v[i][0];
-            acc[1] |= v[i][1];
-            acc[2] |= v[i][2];
-            acc[3] |= v[i][3];
-        }
-    }
-    for (int j = 0; j < q.w; ++j)
-        if (chunk_byte(acc, j))
-            colflag[q.c0 + j] = 1;
-}
-
-// counts the elements where mask != rowflag & colflag (a TW mask has none)
-__global__ void __launch_bounds__(256)
-    validate_tw_kernel(const uint8_t *__restrict__ mask, int K, int N,
-                       const int32_t *__restrict__ tcol0, int n_tiles, int cw,
-                       const uint8_t *__restrict__ rowflag, const uint8_t *__restrict__ colflag,
-                       unsigned long long *__restrict__ mismatch)
-{
-    ChunkPos q;
-    unsigned bad = 0;
-    if (chunk_pos(mask, K, N, tcol0, n_tiles, cw, q)) {
-        // 0x01 in every byte of the chunk whose column is kept
-        uint32_t cf[4] = {0u, 0u, 0u, 0u};
-        for (int j = 0; j < q.w; ++j)
-            cf[j >> 2] |= (colflag[q.c0 + j] ? 1u : 0u) << ((j & 3) * 8);
-        for (int k0 = q.k_begin; k0 < q.k_end; k0 += kFlagBatch * q.k_step) {
-            uint32_t v[kFlagBatch][4];
-            uint32_t rf[kFlagBatch]; // all ones where the row of tile t0 is kept
 #pragma unroll
-            for (int i = 0; i < kFlagBatch; ++i) {
-                const int k = k0 + i * q.k_step;
-                if (k < q.k_end) {
-                    load_chunk(mask + (int64_t)k * N + q.c0, q, v[i]);
-                    rf[i] = rowflag[(int64_t)q.t0 * K + k] ? 0xFFFFFFFFu : 0u;
-                } else {
-                    v[i][0] = v[i][1] = v[i][2] = v[i][3] = 0u;
-                    rf[i] = 0u;
-                }
-            }
+                for (int j = 0; j < 4; ++j) {
+                    v[p][j] = 0u;
 #pragma unroll
-            for (int i = 0; i < kFlagBatch; ++i) {
-                const int k = k0 + i * q.k_step;
-                if (q.one_tile) {
-                    // byte-parallel: 0x01 where the mask byte is non-zero, against (row kept) & cf;
-                    // a row past k_end has v == 0 and rf == 0 and adds nothing
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        const uint32_t x = v[i][w];
-                        const uint32_t nz =
-                            ((x | ((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu)) >> 7) & 0x01010101u;
-                        bad += __popc(nz ^ (cf[w] & rf[i]));
-                    }
-                } else if (k < q.k_end) {
-                    int t = q.t0, t_end = tcol0[t + 1];
-                    bool r = rf[i] != 0u;
-                    for (int j = 0; j < q.w; ++j) {
-                        if (q.c0 + j >= t_end) {
-                            ++t;
-                            t_end = tcol0[t + 1];
-                            r = rowflag[(int64_t)t * K + k] != 0;
-                        }
-                        const bool m = chunk_byte(v[i], j) != 0;
-                        const bool e = r && chunk_byte(cf, j);
-                        bad += m != e;
-                    }
+                    for (int e = 0; e < 4; ++e)
+                        if (cc + j * 4 + e < a.N)
+                            v[p][j] |= (uint32_t)src[j * 4 + e] << (e * 8);
                 }
             }
         }
+        uint32_t in_tile[4], acc[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int lo = min(max(c0 - cc - j * 4, 0), 4), hi = min(max(c0 + w - cc - j * 4, 0), 4);
+            in_tile[j] = (uint32_t)((1ull << (hi * 8)) - 1ull) & ~(uint32_t)((1ull << (lo * 8)) - 1ull);
+        }
+#pragma unroll
+        for (int p = 0; p < kFlagPasses; ++p) {
+            if (p * rpp >= kFlagRows)
+                break;
+            uint32_t any = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t x = r0 + p * rpp < nr ? v[p][j] & in_tile[j] : 0u;
+                const uint32_t nz = ((x | ((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu)) >> 7) & 0x01010101u;
+                any |= nz;
+                acc[j] |= nz;
+                nnz += __popc(nz);
+            }
+            row_any |= (any ? 1u : 0u) << p;
+        }
+        // the window's columns over all rows of the slab
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            for (int off = lpr; off < 64; off <<= 1)
+                acc[j] |= __shfl_xor(acc[j], off);
+        if (lane < lpr) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                s_col[wave][l * 4 + j] = acc[j];
+        }
+        __syncthreads();
+        const int wp = (w + 3) & ~3; // width of the slab's row of column flags
+        uint8_t *const part = a.colpart + a.colpart_at(t, c0) + (int64_t)slab * wp;
+        for (int j = tid; j < lpr * 16; j += 256) {
+            const int rel = a0 + win * lpr * 16 + j - c0;
+            const uint32_t x = s_col[0][j >> 2] | s_col[1][j >> 2] | s_col[2][j >> 2] | s_col[3][j >> 2];
+            if (rel >= 0 && rel < w)
+                part[rel] = (uint8_t)(x >> ((j & 3) * 8));
+        }
+        __syncthreads();
     }
-    // one atomic per wave that saw a mismatch
+#pragma unroll
+    for (int p = 0; p < kFlagPasses; ++p) {
+        if (p * rpp >= kFlagRows)
+            break;
+        const unsigned long long votes = __ballot(row_any >> p & 1u);
+        const unsigned long long mine = (lpr == 32 ? 0xFFFFFFFFull : (1ull << lpr) - 1ull) << (lane & -lpr);
+        if (l == 0 && r0 + p * rpp < nr)
+            a.rowflag[(int64_t)t * a.K + k0 + r0 + p * rpp] = (votes & mine) != 0ull;
+    }
     for (int off = 32; off > 0; off >>= 1)
-        bad += __shfl_down(bad, off);
-    if ((threadIdx.x & 63) == 0 && bad)
-        atomicAdd(mismatch, (unsigned long long)bad);
+        nnz += __shfl_down(nnz, off);
+    if (lane == 0)
+        atomicAdd(&s_nnz, nnz);
+    __syncthreads();
+    if (tid == 0)
+        a.nnz[(int64_t)t * a.n_slabs + slab] = s_nnz;
 }
 
-// Counting and compaction work on segments of kSegFlags flags (rows of one tile, or columns of
-// one tile), one workgroup per segment: grid (n_tiles, n_seg_k + n_seg_n), y < n_seg_k rows.
-// seg_counts holds the kept flags per segment, tile-major: first the n_tiles * n_seg_k row
-// entries, then the n_tiles * n_seg_n column entries.
-constexpr int kSegFlags = 1024;
-constexpr int kSegRounds = kSegFlags / 256;
-
-struct FlagSegment {
-    const uint8_t *flag; // the tile's flag vector
-    int n;               // its length
-    int first;           // first flag of this segment
-    int entry;           // index of this segment among the row (or column) entries
-    bool rows;
+// What the host needs to know of a tile before it can lay the plan out, in pinned memory.
+struct TileCounts {
+    unsigned long long nnz;
+    int32_t k_kept, n_kept;
+    uint32_t stamp; // the build's number, written last
+    uint32_t pad_[3];
 };
 
-__device__ __forceinline__ FlagSegment flag_segment(const uint8_t *rowflag, const uint8_t *colflag,
-                                                    int K, const int32_t *tcol0, int n_seg_k,
-                                                    int n_seg_n)
+// One workgroup per tile: ascending lists of the kept rows (at kk + t * K), of the kept columns and of
+// the pruned ones (both at the tile's first column), and the counts.  Every thread takes a run of
+// neighbouring flags, so one scan orders all of them.
+constexpr int kListThreads = 512;
+__global__ void __launch_bounds__(kListThreads)
+    mask_lists_kernel(const FlagArgs a, int32_t *kk, int32_t *kn, int32_t *pn, TileCounts *counts, uint32_t stamp)
 {
-    FlagSegment g;
-    const int t = blockIdx.x;
-    g.rows = (int)blockIdx.y < n_seg_k;
-    const int seg = g.rows ? (int)blockIdx.y : (int)blockIdx.y - n_seg_k;
-    g.flag = g.rows ? rowflag + (int64_t)t * K : colflag + tcol0[t];
-    g.n = g.rows ? K : tcol0[t + 1] - tcol0[t];
-    g.first = seg * kSegFlags;
-    g.entry = t * (g.rows ? n_seg_k : n_seg_n) + seg;
-    return g;
-}
-
-__global__ void __launch_bounds__(256)
-    count_flags_kernel(const uint8_t *__restrict__ rowflag, const uint8_t *__restrict__ colflag,
-                       int K, const int32_t *__restrict__ tcol0, int n_tiles, int n_seg_k,
-                       int n_seg_n, int32_t *__restrict__ seg_counts)
-{
-    __shared__ int s_wave[4];
-    const FlagSegment g = flag_segment(rowflag, colflag, K, tcol0, n_seg_k, n_seg_n);
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j) {
-        const int i = g.first + j * 256 + (int)threadIdx.x;
-        if (i < g.n)
-            c += g.flag[i] != 0;
-    }
-    for (int off = 32; off > 0; off >>= 1)
-        c += __shfl_down(c, off);
-    if ((threadIdx.x & 63) == 0)
-        s_wave[threadIdx.x >> 6] = c;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        seg_counts[(g.rows ? 0 : n_tiles * n_seg_k) + g.entry] =
-            s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
-}
-
-// Ordered compaction of one segment: the ascending kept indices and the relative offsets
-// kept[i] - i land where the segments before it (seg_counts, tile-major) leave off.
-__global__ void __launch_bounds__(256)
-    compact_lists_kernel(const uint8_t *__restrict__ rowflag, const uint8_t *__restrict__ colflag,
-                         int K, const int32_t *__restrict__ tcol0, int n_tiles, int n_seg_k,
-                         int n_seg_n, const int32_t *__restrict__ seg_counts,
-                         int32_t *__restrict__ kept_k, int32_t *__restrict__ rel_k,
-                         int32_t *__restrict__ kept_n, int32_t *__restrict__ rel_n)
-{
-    __shared__ int s_sum[2][4];
-    __shared__ int s_round[kSegRounds][4];
-    const FlagSegment g = flag_segment(rowflag, colflag, K, tcol0, n_seg_k, n_seg_n);
-    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
-    bool f[kSegRounds];
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j) {
-        const int i = g.first + j * 256 + (int)threadIdx.x;
-        f[j] = i < g.n && g.flag[i] != 0;
-    }
-    // kept flags before this segment: in the tiles before (a) and earlier in this tile (b)
-    const int32_t *cnt = seg_counts + (g.rows ? 0 : n_tiles * n_seg_k);
-    const int tile_first = (int)blockIdx.x * (g.rows ? n_seg_k : n_seg_n);
-    int a = 0, b = 0;
-    for (int i = (int)threadIdx.x; i < g.entry; i += 256) {
-        const int v = cnt[i];
-        if (i < tile_first)
-            a += v;
-        else
-            b += v;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_down(a, off);
-        b += __shfl_down(b, off);
-    }
-    int before[kSegRounds];
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j) {
-        const unsigned long long votes = __ballot(f[j]);
-        before[j] = __popcll(votes & ((1ull << lane) - 1ull));
-        if (lane == 0)
-            s_round[j][wave] = __popcll(votes);
-    }
-    if (lane == 0) {
-        s_sum[0][wave] = a;
-        s_sum[1][wave] = b;
-    }
-    __syncthreads();
-    const int in_tile = s_sum[1][0] + s_sum[1][1] + s_sum[1][2] + s_sum[1][3];
-    const int tile_base = s_sum[0][0] + s_sum[0][1] + s_sum[0][2] + s_sum[0][3];
-    int32_t *kept = (g.rows ? kept_k : kept_n) + tile_base;
-    int32_t *rel = (g.rows ? rel_k : rel_n) + tile_base;
-    int rank = in_tile; // position in the tile's list of this round's first kept flag
-#pragma unroll
-    for (int j = 0; j < kSegRounds; ++j) {
-        int mine = rank + before[j];
-        for (int w = 0; w < wave; ++w)
-            mine += s_round[j][w];
-        if (f[j]) {
-            const int i = g.first + j * 256 + (int)threadIdx.x;
-            kept[mine] = i;
-            rel[mine] = i - mine;
+    constexpr int NW = kListThreads / 64;
+    __shared__ int s_wave[NW];
+    __shared__ uint32_t s_cols[1024]; // flags of a window of 4096 columns
+    __shared__ unsigned long long s_nnz;
+    const int t = (int)blockIdx.x, tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c0 = a.tcol0[t], w = a.tcol0[t + 1] - c0;
+    // position of this thread's first one among all ones of the workgroup, and their number
+    auto scan = [&](int mine, int &total) {
+        int incl = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int up = __shfl_up(incl, off);
+            if (lane >= off)
+                incl += up;
         }
-        rank += s_round[j][0] + s_round[j][1] + s_round[j][2] + s_round[j][3];
+        if (lane == 63)
+            s_wave[wave] = incl;
+        __syncthreads();
+        int before = incl - mine;
+        total = 0;
+#pragma unroll
+        for (int v = 0; v < NW; ++v) {
+            before += v < wave ? s_wave[v] : 0;
+            total += s_wave[v];
+        }
+        __syncthreads();
+        return before;
+    };
+    if (tid == 0)
+        s_nnz = 0;
+    unsigned long long nnz = 0;
+    for (int i = tid; i < a.n_slabs; i += kListThreads)
+        nnz += a.nnz[(int64_t)t * a.n_slabs + i];
+    for (int off = 32; off > 0; off >>= 1)
+        nnz += __shfl_down(nnz, off);
+
+    // rows
+    const uint8_t *const flag = a.rowflag + (int64_t)t * a.K;
+    int32_t *const rows = kk + (int64_t)t * a.K;
+    int k_kept = 0;
+    for (int base = 0; base < a.K; base += kListThreads * 16) { // sixteen rows a thread at a time
+        const int run = min(16, (a.K - base + kListThreads - 1) / kListThreads);
+        const int first = base + tid * run;
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i < run && first + i < a.K)
+                bits |= (flag[first + i] ? 1u : 0u) << i;
+        int total;
+        int at = k_kept + scan(__popc(bits), total);
+        for (; bits; bits &= bits - 1u)
+            rows[at++] = first + __ffs(bits) - 1;
+        k_kept += total;
+    }
+    if (lane == 0)
+        atomicAdd(&s_nnz, nnz);
+
+    // columns: kept where any slab says so
+    const int words = ((w + 3) & ~3) >> 2;
+    const uint32_t *const part = reinterpret_cast<const uint32_t *>(a.colpart + a.colpart_at(t, c0));
+    int n_kept = 0;
+    for (int base = 0; base < words; base += 1024) {
+        const int nw = min(1024, words - base);
+        for (int i = tid; i < nw; i += kListThreads)
+            s_cols[i] = 0;
+        __syncthreads();
+        for (int i = tid; i < nw * a.n_slabs; i += kListThreads) {
+            const int slab = i / nw, j = i - slab * nw;
+            const uint32_t x = part[(int64_t)slab * words + base + j];
+            if (x)
+                atomicOr(&s_cols[j], x);
+        }
+        __syncthreads();
+        // (four columns, one word, per thread and round)
+        for (int r = 0; r < nw; r += kListThreads) {
+            const int j = r + tid;
+            const int here = min(max(w - (base + j) * 4, 0), 4); // columns of this word (what lies behind them was not written)
+            const uint32_t x = (j < nw ? s_cols[j] : 0u) & (uint32_t)((1ull << (here * 8)) - 1ull);
+            int total;
+            int at = n_kept + scan(__popc(x), total);
+            const int col = (base + j) * 4;
+            int pruned = col - at; // pruned columns before this word
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (j >= nw || col + e >= w)
+                    break;
+                if (x >> (e * 8) & 0xFFu)
+                    kn[c0 + at++] = col + e;
+                else
+                    pn[c0 + pruned++] = col + e;
+            }
+            n_kept += total;
+        }
+    }
+    if (tid == 0) {
+        volatile TileCounts *const c = counts + t;
+        c->nnz = s_nnz;
+        c->k_kept = k_kept;
+        c->n_kept = n_kept;
+        __threadfence_system(); // the counts are in host memory before the stamp that announces them
+        c->stamp = stamp;
     }
 }
 
@@ -475,64 +489,192 @@ __global__ void __launch_bounds__(256)
 
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-static std::vector<PackTile> pack_tiles(const tw_plan *p, const int64_t *src_off)
-{
-    std::vector<PackTile> v(p->n_tiles);
-    for (int t = 0; t < p->n_tiles; ++t) {
-        PackTile &q = v[t];
-        q.col0 = p->tile_col0[t];
-        q.k_kept = p->kept_k_ptr[t + 1] - p->kept_k_ptr[t];
-        q.n_kept = p->kept_n_ptr[t + 1] - p->kept_n_ptr[t];
-        q.k_pad = p->k_pad[t];
-        q.n_pad = p->n_pad[t];
-        q.kk_off = p->kept_k_ptr[t];
-        q.kn_off = p->kept_n_ptr[t];
-        q.pad_ = 0;
-        q.b_off = p->b_off[t];
-        q.src_off = src_off ? src_off[t] : 0;
-    }
-    return v;
-}
-
-static int64_t max_groups(const tw_plan *p)
-{
-    int64_t g = 0;
-    for (int t = 0; t < p->n_tiles; ++t)
-        g = std::max<int64_t>(g, (int64_t)p->k_pad[t] * p->n_pad[t] / 8);
-    return g;
-}
-
-template <typename T> static int upload(T **dst, const std::vector<T> &src)
-{
-    *dst = nullptr;
-    size_t bytes = std::max<size_t>(src.size(), 1) * sizeof(T);
-    if (hipMalloc((void **)dst, bytes) != hipSuccess)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes failed", bytes);
-    if (!src.empty()) {
-        hipError_t e = hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice);
-        if (e != hipSuccess) {
-            hipFree(*dst);
-            *dst = nullptr;
-            return fail(TW_ERR_DEVICE, "upload of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+// Device memory of plans and of builds.  The runtime hands out and takes back pieces of up to a
+// megabyte in half a microsecond, but maps and unmaps larger ones anew: 25 us for a hipMalloc of 4 MB,
+// 20 - 240 for its hipFree.  Those are kept here when they are given back, up to kPoolBytes a process,
+// and go to the next that asks for about as much on that device; what does not fit is freed, and all
+// of it when an allocation fails.  A piece is given back only when no kernel uses it any more.
+constexpr size_t kPoolFrom = 1 << 20, kPoolBytes = 256u << 20;
+class DevicePool {
+public:
+    void *get(size_t bytes, int device)
+    {
+        if (bytes > kPoolFrom) {
+            std::lock_guard<std::mutex> lock(mu_);
+            size_t best = free_.size();
+            for (size_t i = 0; i < free_.size(); ++i)
+                if (free_[i].device == device && free_[i].bytes >= bytes && free_[i].bytes <= 2 * bytes &&
+                    (best == free_.size() || free_[i].bytes < free_[best].bytes))
+                    best = i;
+            if (best < free_.size()) {
+                const Piece p = free_[best];
+                free_.erase(free_.begin() + best);
+                held_ -= p.bytes;
+                used_[p.ptr] = p.bytes;
+                return p.ptr;
+            }
         }
+        void *p = nullptr;
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            drop_all();
+            if (hipMalloc(&p, bytes) != hipSuccess)
+                return nullptr;
+        }
+        if (bytes > kPoolFrom) {
+            std::lock_guard<std::mutex> lock(mu_);
+            used_[p] = bytes;
+        }
+        return p;
     }
-    return TW_OK;
+    // no kernel uses `p` any more, or (idle == false) what is queued on the device may
+    void put(void *p, int device, bool idle)
+    {
+        if (!p)
+            return;
+        size_t bytes = 0;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            auto it = used_.find(p);
+            if (it != used_.end()) {
+                bytes = it->second;
+                used_.erase(it);
+            }
+        }
+        int now = -1;
+        if (bytes && (hipGetDevice(&now) != hipSuccess || now != device || (!idle && hipDeviceSynchronize() != hipSuccess)))
+            bytes = 0; // (another device is current, or a capture forbids to wait)
+        if (bytes) {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (held_ + bytes <= kPoolBytes) {
+                free_.push_back(Piece{p, bytes, device});
+                held_ += bytes;
+                return;
+            }
+        }
+        (void)hipFree(p);
+    }
+
+private:
+    struct Piece {
+        void *ptr;
+        size_t bytes;
+        int device;
+    };
+    void drop_all()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (const Piece &p : free_)
+            (void)hipFree(p.ptr);
+        free_.clear();
+        held_ = 0;
+    }
+    std::mutex mu_;
+    std::vector<Piece> free_;
+    std::map<void *, size_t> used_;
+    size_t held_ = 0;
+};
+// (never destroyed: plans may be, by a host program's own destructors, after the library's)
+static DevicePool &device_pool()
+{
+    static DevicePool *const pool = new DevicePool;
+    return *pool;
 }
 
-static void free_plan(tw_plan *p);
+// Pinned host memory of a build, on a list of a few pieces between builds.
+class PinnedPool {
+public:
+    void *get(size_t bytes, size_t *size)
+    {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            for (size_t i = 0; i < free_.size(); ++i)
+                if (free_[i].second >= bytes) {
+                    const auto p = free_[i];
+                    free_.erase(free_.begin() + i);
+                    *size = p.second;
+                    return p.first;
+                }
+        }
+        void *p = nullptr;
+        *size = std::max<size_t>(bytes, 64 << 10);
+        return hipHostMalloc(&p, *size, hipHostMallocPortable) == hipSuccess ? p : nullptr;
+    }
+    void put(void *p, size_t size)
+    {
+        if (!p)
+            return;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            if (size <= (1u << 20) && free_.size() < 8) {
+                free_.emplace_back(p, size);
+                return;
+            }
+        }
+        (void)hipHostFree(p);
+    }
+
+private:
+    std::mutex mu_;
+    std::vector<std::pair<void *, size_t>> free_;
+};
+static PinnedPool &pinned_pool()
+{
+    static PinnedPool *const pool = new PinnedPool;
+    return *pool;
+}
+
+static void free_plan(tw_plan *p)
+{
+    if (!p)
+        return;
+    device_pool().put(p->d_slab, p->device, false);
+    delete p;
+}
 
 // Owners of what a builder holds until it succeeds: whatever path leaves the builder (an error
-// return, an exception on its way to the status conversion), the device buffer and the
-// half-built plan are released.
+// return, an exception on its way to the status conversion), its buffers and the half-built plan are
+// released.  The stream of a build is waited for first: its kernels use them.
 struct DeviceBuffer {
     void *ptr = nullptr;
+    int device = 0;
     DeviceBuffer() = default;
     DeviceBuffer(const DeviceBuffer &) = delete;
     DeviceBuffer &operator=(const DeviceBuffer &) = delete;
     ~DeviceBuffer()
     {
-        if (ptr)
-            (void)hipFree(ptr);
+        device_pool().put(ptr, device, true);
+    }
+    bool get(size_t bytes, int dev)
+    {
+        device = dev;
+        ptr = device_pool().get(bytes, dev);
+        return ptr != nullptr;
+    }
+};
+struct PinnedBuffer {
+    void *ptr = nullptr;
+    size_t size = 0;
+    PinnedBuffer() = default;
+    PinnedBuffer(const PinnedBuffer &) = delete;
+    PinnedBuffer &operator=(const PinnedBuffer &) = delete;
+    ~PinnedBuffer()
+    {
+        pinned_pool().put(ptr, size);
+    }
+    bool get(size_t bytes)
+    {
+        ptr = pinned_pool().get(bytes, &size);
+        return ptr != nullptr;
+    }
+};
+struct StreamWait { // declared behind the buffers it protects
+    hipStream_t s;
+    bool done = false;
+    ~StreamWait()
+    {
+        if (!done)
+            (void)hipStreamSynchronize(s);
     }
 };
 struct PlanOwner {
@@ -553,20 +695,35 @@ struct PlanOwner {
     }
 };
 
-int finalize_plan_geometry(tw_plan *p, hipStream_t s)
+// What a plan is made from besides its counts (kept_k_ptr, kept_n_ptr): lists in device memory (tile
+// t's kept rows at kk + kk_src[t], and so on) and one of the two forms of the weight.
+struct PlanSource {
+    const int32_t *kk = nullptr, *kn = nullptr, *pn = nullptr;
+    std::vector<int64_t> kk_src, kn_src, pn_src;
+    const float *B = nullptr;
+    const uint8_t *mask = nullptr;
+    const uint16_t *Bs = nullptr;
+    const int64_t *off_B = nullptr;
+};
+
+// Lays out a plan whose tile table and counts are set, and builds everything it owns on the device
+// with one launch on `s`; returns when that has run.
+static int build_plan(tw_plan *p, const PlanSource &src, hipStream_t s)
 {
     const int dst = prepare_device();
     if (dst != TW_OK)
         return dst;
+    TW_HIP(hipGetDevice(&p->device));
     const int nt = p->n_tiles;
     p->k_pad.assign(nt, 0);
     p->n_pad.assign(nt, 0);
     p->b_off.assign(nt, 0);
-    int64_t off = 0;
-    std::vector<UnitDev> units;
+    int64_t off = 0, kkp = 0, groups = 1, longest_list = 1;
+    int32_t n_pruned = 0;
+    std::vector<UnitDev> &units = p->h_units;
     std::vector<TileDev> ztiles;
-    std::vector<int32_t> pruned_n;
-    std::vector<int32_t> kept_k_pad; // the GEMM kernel's copy: k_pad entries per tile
+    std::vector<PlanTile> tiles(nt);
+    units.clear();
     p->max_unit_n = 0;
     p->n_halves = 0;
     for (int t = 0; t < nt; ++t) {
@@ -579,14 +736,29 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
             p->k_pad[t] = 0;
             p->n_pad[t] = ntk > 0 ? round_up(ntk, kMfmaN) : 0;
         }
-        const int32_t kkp_off = (int32_t)kept_k_pad.size();
-        kept_k_pad.insert(kept_k_pad.end(), p->kept_k_idx.begin() + p->kept_k_ptr[t],
-                          p->kept_k_idx.begin() + p->kept_k_ptr[t + 1]);
-        // padding past k_pad: the kernel prefetches the index list up to eight 64-row steps ahead
-        kept_k_pad.resize(kkp_off + p->k_pad[t] + 8 * kBlockK, 0);
-        p->b_off[t] = off;
+        PlanTile &q = tiles[t];
+        std::memset(&q, 0, sizeof(q));
+        q.col0 = p->tile_col0[t];
+        q.k_kept = kt;
+        q.n_kept = ntk;
+        q.k_pad = p->k_pad[t];
+        q.n_pad = p->n_pad[t];
+        q.n_pruned = p->tile_width[t] - ntk;
+        q.kk_dst = p->kept_k_ptr[t];
+        q.kn_dst = p->kept_n_ptr[t];
+        q.pn_dst = n_pruned;
+        // the padded list: the kernels prefetch it up to eight 64-row steps ahead
+        q.kkp_dst = (int32_t)kkp;
+        q.kkp_len = p->k_pad[t] + 8 * kBlockK;
+        q.kk_src = src.kk_src[t];
+        q.kn_src = src.kn_src[t];
+        q.pn_src = src.pn_src[t];
+        q.src_off = src.off_B ? src.off_B[t] : 0;
+        kkp += q.kkp_len;
+        longest_list = std::max<int64_t>(longest_list, std::max(q.kkp_len, p->tile_width[t]));
+        q.b_off = p->b_off[t] = off; // (a multiple of 64 x 32 elements: every tile is 1 KiB aligned)
         off += (int64_t)p->k_pad[t] * p->n_pad[t];
-        off = (off + 511) / 512 * 512; // keep every tile 1 KiB aligned
+        groups = std::max<int64_t>(groups, (int64_t)p->k_pad[t] * p->n_pad[t] / 8);
         for (int nc0 = 0; nc0 < ntk; nc0 += kMaxUnitN) {
             UnitDev u;
             u.col0 = p->tile_col0[t];
@@ -595,7 +767,7 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
             u.n_cnt = std::min(kMaxUnitN, ntk - nc0);
             u.nb0 = nc0 / kMfmaN;
             u.nb_cnt = (u.n_cnt + kMfmaN - 1) / kMfmaN;
-            u.kk_off = kkp_off;
+            u.kk_off = q.kkp_dst;
             u.kn_off = p->kept_n_ptr[t] + nc0;
             u.b_off = p->b_off[t];
             u.tile = t;
@@ -604,29 +776,23 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
             p->max_unit_n = std::max(p->max_unit_n, u.n_cnt);
             p->n_halves += (u.n_cnt + 63) / 64;
         }
-        if (ntk < p->tile_width[t]) {
+        if (q.n_pruned > 0) {
             TileDev z;
             z.col0 = p->tile_col0[t];
-            z.n_pruned = p->tile_width[t] - ntk;
-            z.pn_off = (int32_t)pruned_n.size();
+            z.n_pruned = q.n_pruned;
+            z.pn_off = n_pruned;
             z.pad_ = 0;
-            const int32_t *kn = p->kept_n_idx.data() + p->kept_n_ptr[t];
-            int j = 0;
-            for (int c = 0; c < p->tile_width[t]; ++c) {
-                if (j < ntk && kn[j] == c)
-                    ++j;
-                else
-                    pruned_n.push_back(c);
-            }
             ztiles.push_back(z);
+            n_pruned += q.n_pruned;
         }
     }
+    if (kkp > INT32_MAX)
+        return fail(TW_ERR_SHAPE, "the plan keeps %lld rows in all its tiles: at most 2^31 - 1", (long long)kkp);
     // work queue order: heaviest kept-K first, ties keep a tile's pieces adjacent
     std::stable_sort(units.begin(), units.end(),
                      [](const UnitDev &a, const UnitDev &b) { return a.k_kept > b.k_kept; });
     p->packed_elems = off;
     p->n_units = (int)units.size();
-    p->h_units = units;
     p->n_pipe_units = 0;
     for (const UnitDev &u : units)
         p->n_pipe_units += u.k_pad > 0;
@@ -636,7 +802,7 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
     for (int t = 0; t < nt; ++t)
         tiles_with_rows += p->kept_k_ptr[t + 1] > p->kept_k_ptr[t];
     p->rows_shared = tiles_with_rows > 1 && p->n_pipe_units > 0 &&
-                     (int64_t)p->kept_k_idx.size() * 10 >= (int64_t)p->K * tiles_with_rows * 9;
+                     (int64_t)p->kept_k_ptr[nt] * 10 >= (int64_t)p->K * tiles_with_rows * 9;
     p->n_zero_tiles = (int)ztiles.size();
     p->max_k_pad = 0;
     p->pipe_steps = 0;
@@ -644,99 +810,111 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
         p->max_k_pad = std::max(p->max_k_pad, u.k_pad);
         p->pipe_steps += u.k_pad / kBlockK;
     }
-
-    // One device allocation for everything the plan owns besides lists that were compacted on
-    // the device: [staged tables, uploaded with one copy][ticket slots][packed weight], the last
-    // two zeroed with one memset.
-    std::vector<int32_t> rel_k, rel_n;
-    const bool lists_here = p->d_kept_k == nullptr;
-    if (lists_here) {
-        rel_k.resize(p->kept_k_idx.size());
-        rel_n.resize(p->kept_n_idx.size());
-        for (int t = 0; t < nt; ++t) {
-            for (int i = p->kept_k_ptr[t]; i < p->kept_k_ptr[t + 1]; ++i)
-                rel_k[i] = p->kept_k_idx[i] - (i - p->kept_k_ptr[t]);
-            for (int i = p->kept_n_ptr[t]; i < p->kept_n_ptr[t + 1]; ++i)
-                rel_n[i] = p->kept_n_idx[i] - (i - p->kept_n_ptr[t]);
-        }
-    }
-    const std::vector<PackTile> ptab = pack_tiles(p, nullptr);
-    std::vector<char> stage;
-    auto put = [&stage](const void *src, size_t bytes) { // returns the 256-aligned offset
-        const size_t off = (stage.size() + 255) / 256 * 256;
-        stage.resize(off + std::max<size_t>(bytes, 4), 0);
-        if (bytes)
-            std::memcpy(stage.data() + off, src, bytes);
-        return off;
-    };
-    const size_t o_units = put(units.data(), units.size() * sizeof(UnitDev));
-    const size_t o_tiles = put(ztiles.data(), ztiles.size() * sizeof(TileDev));
-    const size_t o_pruned = put(pruned_n.data(), pruned_n.size() * sizeof(int32_t));
-    const size_t o_kkpad = put(kept_k_pad.data(), kept_k_pad.size() * sizeof(int32_t));
-    const size_t o_ptab = put(ptab.data(), ptab.size() * sizeof(PackTile));
-    std::vector<int32_t> blocks;
-    for (size_t ui = 0; ui < units.size(); ++ui)
-        for (int nb = 0; nb < units[ui].nb_cnt; ++nb)
-            blocks.push_back((int32_t)ui * 4 + nb);
-    p->n_blocks = (int)blocks.size();
+    p->n_blocks = 0;
     p->blocks_per_unit = units.empty() ? 0 : units[0].nb_cnt;
-    for (const UnitDev &u : units)
+    for (const UnitDev &u : units) {
+        p->n_blocks += u.nb_cnt;
         if (u.nb_cnt != p->blocks_per_unit)
             p->blocks_per_unit = 0;
-    const size_t o_blocks = put(blocks.data(), blocks.size() * sizeof(int32_t));
-    std::vector<uint32_t> kpairs; // see GemmArgs::kept_pairs
-    if (p->K < 0xFFFF) {
-        // the padding names row K here (a row of zeros behind the kernel's panel of A), not row 0
-        std::vector<uint16_t> padded(kept_k_pad.size(), (uint16_t)p->K);
-        for (const UnitDev &u : units)
-            for (int i = 0; i < u.k_kept; ++i)
-                padded[u.kk_off + i] = (uint16_t)kept_k_pad[u.kk_off + i];
-        kpairs.resize(kept_k_pad.size() / 2);
-        for (size_t st = 0; st < kept_k_pad.size() / 64; ++st)
-            for (int g16 = 0; g16 < 4; ++g16)
-                for (int e = 0; e < 8; ++e) {
-                    const size_t lo = st * 64 + g16 * 16 + (e >> 2) * 8 + (e & 3);
-                    kpairs[st * 32 + e * 4 + g16] = (uint32_t)padded[lo] | ((uint32_t)padded[lo + 4] << 16);
-                }
     }
-    const size_t o_kpairs = put(kpairs.data(), kpairs.size() * sizeof(uint32_t));
-    size_t o_kk = 0, o_kn = 0, o_rk = 0, o_rn = 0;
-    if (lists_here) {
-        o_kk = put(p->kept_k_idx.data(), p->kept_k_idx.size() * sizeof(int32_t));
-        o_kn = put(p->kept_n_idx.data(), p->kept_n_idx.size() * sizeof(int32_t));
-        o_rk = put(rel_k.data(), rel_k.size() * sizeof(int32_t));
-        o_rn = put(rel_n.data(), rel_n.size() * sizeof(int32_t));
-    }
-    const size_t o_tickets = (stage.size() + 255) / 256 * 256;
-    const size_t ticket_bytes = sizeof(int32_t) * kTicketInts * (kTicketSlots + 1); // (the last: status words)
-    const size_t o_bp = (o_tickets + ticket_bytes + 1023) / 1024 * 1024;
-    const size_t bp_bytes = (size_t)std::max<int64_t>(p->packed_elems, 8) * 2;
-    char *slab = nullptr;
-    if (hipMalloc((void **)&slab, o_bp + bp_bytes) != hipSuccess)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the plan failed", o_bp + bp_bytes);
-    p->d_slab = slab;
-    TW_HIP(hipMemcpyAsync(slab, stage.data(), stage.size(), hipMemcpyHostToDevice, s));
-    // the packing kernel follows on the same stream and the builders wait for it; a plan with
-    // nothing to pack waits here (the staged tables are host memory of this call: wait either way
-    // before they go out of scope)
-    TW_HIP(hipMemsetAsync(slab + o_tickets, 0, o_bp + bp_bytes - o_tickets, s));
-    TW_HIP(hipStreamSynchronize(s));
+
+    // One device allocation for everything the plan owns: the tables the host makes (one copy), then
+    // what the kernel writes.
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    size_t at = 0;
+    auto place = [&](size_t bytes) { // returns the 256-aligned offset
+        const size_t o = at;
+        at = up(at + std::max<size_t>(bytes, 4));
+        return o;
+    };
+    const size_t o_units = place(units.size() * sizeof(UnitDev));
+    const size_t o_ztiles = place(ztiles.size() * sizeof(TileDev));
+    const size_t o_tiles = place(tiles.size() * sizeof(PlanTile));
+    const size_t o_blocks = place(p->n_blocks * sizeof(int32_t));
+    const size_t header_bytes = at;
+    const size_t sk = p->kept_k_ptr[nt], sn = p->kept_n_ptr[nt];
+    const size_t o_kk = place(sk * sizeof(int32_t)), o_rk = place(sk * sizeof(int32_t));
+    const size_t o_kn = place(sn * sizeof(int32_t)), o_rn = place(sn * sizeof(int32_t));
+    const size_t o_pruned = place(n_pruned * sizeof(int32_t));
+    const size_t o_kkpad = place(kkp * sizeof(int32_t));
+    const bool pairs = p->K < 0xFFFF;
+    const size_t o_pairs = place(pairs ? kkp / 2 * sizeof(uint32_t) : 0);
+    const int ticket_words = kTicketInts * (kTicketSlots + 1); // (the last: status words)
+    const size_t o_tickets = place(ticket_words * sizeof(int32_t));
+    at = (at + 1023) / 1024 * 1024;
+    const size_t o_bp = place((size_t)std::max<int64_t>(p->packed_elems, 8) * 2);
+
+    PinnedBuffer header;
+    if (!header.get(header_bytes))
+        return fail(TW_ERR_ALLOC, "hipHostMalloc of %zu bytes for the plan's tables failed", header_bytes);
+    p->d_slab = device_pool().get(at, p->device);
+    if (!p->d_slab)
+        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the plan failed", at);
+    char *const slab = static_cast<char *>(p->d_slab), *const host = static_cast<char *>(header.ptr);
+    std::memcpy(host + o_units, units.data(), units.size() * sizeof(UnitDev));
+    std::memcpy(host + o_ztiles, ztiles.data(), ztiles.size() * sizeof(TileDev));
+    std::memcpy(host + o_tiles, tiles.data(), tiles.size() * sizeof(PlanTile));
+    int32_t *blocks = reinterpret_cast<int32_t *>(host + o_blocks);
+    for (size_t ui = 0; ui < units.size(); ++ui)
+        for (int nb = 0; nb < units[ui].nb_cnt; ++nb)
+            *blocks++ = (int32_t)ui * 4 + nb;
+
     p->d_units = reinterpret_cast<UnitDev *>(slab + o_units);
-    p->d_tiles = reinterpret_cast<TileDev *>(slab + o_tiles);
+    p->d_tiles = reinterpret_cast<TileDev *>(slab + o_ztiles);
+    p->d_plan_tiles = slab + o_tiles;
+    p->d_blocks = reinterpret_cast<int32_t *>(slab + o_blocks);
+    p->d_kept_k = reinterpret_cast<int32_t *>(slab + o_kk);
+    p->d_rel_k = reinterpret_cast<int32_t *>(slab + o_rk);
+    p->d_kept_n = reinterpret_cast<int32_t *>(slab + o_kn);
+    p->d_rel_n = reinterpret_cast<int32_t *>(slab + o_rn);
     p->d_pruned_n = reinterpret_cast<int32_t *>(slab + o_pruned);
     p->d_kept_k_pad = reinterpret_cast<int32_t *>(slab + o_kkpad);
-    p->d_pack_tiles = slab + o_ptab;
-    p->d_blocks = reinterpret_cast<int32_t *>(slab + o_blocks);
-    p->d_kept_pairs = kpairs.empty() ? nullptr : reinterpret_cast<uint32_t *>(slab + o_kpairs);
-    if (lists_here) {
-        p->d_kept_k = reinterpret_cast<int32_t *>(slab + o_kk);
-        p->d_kept_n = reinterpret_cast<int32_t *>(slab + o_kn);
-        p->d_rel_k = reinterpret_cast<int32_t *>(slab + o_rk);
-        p->d_rel_n = reinterpret_cast<int32_t *>(slab + o_rn);
-    }
+    p->d_kept_pairs = pairs ? reinterpret_cast<uint32_t *>(slab + o_pairs) : nullptr;
     p->d_tickets = reinterpret_cast<int32_t *>(slab + o_tickets);
     p->d_Bp = slab + o_bp;
-    TW_HIP(hipGetDevice(&p->device));
+
+    BuildArgs a;
+    a.n_tiles = nt;
+    a.K = p->K;
+    a.N = p->N;
+    a.dtype = p->dtype;
+    a.kk = src.kk;
+    a.kn = src.kn;
+    a.pn = src.pn;
+    a.B = src.B;
+    a.Bs = src.Bs;
+    a.mask = src.mask;
+    a.header = reinterpret_cast<const uint4 *>(host);
+    a.header_dst = reinterpret_cast<uint4 *>(slab);
+    a.kept_k = p->d_kept_k;
+    a.rel_k = p->d_rel_k;
+    a.kept_n = p->d_kept_n;
+    a.rel_n = p->d_rel_n;
+    a.pruned_n = p->d_pruned_n;
+    a.kept_k_pad = p->d_kept_k_pad;
+    a.kept_pairs = p->d_kept_pairs;
+    a.tickets = p->d_tickets;
+    a.Bp = static_cast<uint16_t *>(p->d_Bp);
+    a.header_chunks = (int32_t)(header_bytes / 16);
+    a.ticket_words = ticket_words;
+    const unsigned gl = (unsigned)std::min<int64_t>((longest_list + 1023) / 1024, 1024);
+    const unsigned gp = (unsigned)std::min<int64_t>((groups + 255) / 256, 4096);
+    StreamWait wait{s};
+    auto launch_rows = [&](unsigned gx, int begin, int end) { // (kMaxTileRows rows of a grid at a time)
+        for (a.row0 = begin; a.row0 < end; a.row0 += kMaxTileRows)
+            hipLaunchKernelGGL(plan_build_kernel, dim3(gx, std::min(end - a.row0, kMaxTileRows)), dim3(256), 0, s, a);
+    };
+    if (nt <= kArgTiles) {
+        a.tiles = nullptr;
+        std::memcpy(a.arg_tiles, tiles.data(), tiles.size() * sizeof(PlanTile));
+        launch_rows(std::max(gl, gp), 0, 2 * nt + 1);
+    } else {
+        a.tiles = reinterpret_cast<const PlanTile *>(host + o_tiles);
+        launch_rows(gl, nt, 2 * nt + 1);
+        a.tiles = static_cast<const PlanTile *>(p->d_plan_tiles);
+        launch_rows(gp, 0, nt);
+    }
+    TW_HIP(hipGetLastError());
     {
         // the CU count of a device does not change: ask once per device
         static std::mutex mu;
@@ -751,81 +929,68 @@ int finalize_plan_geometry(tw_plan *p, hipStream_t s)
         }
         p->cu_count = cu_of[p->device];
     }
-    return TW_OK;
-}
-
-int pack_from_dense(tw_plan *p, const float *d_B, hipStream_t s, const uint8_t *d_mask)
-{
-    const int64_t mg = max_groups(p);
-    if (mg == 0)
-        return TW_OK;
-    dim3 grid((unsigned)((mg + 255) / 256), (unsigned)p->n_tiles);
-    hipLaunchKernelGGL(pack_dense_kernel, grid, dim3(256), 0, s,
-                       static_cast<const PackTile *>(p->d_pack_tiles), p->d_kept_k, p->d_kept_n, d_B,
-                       p->N, p->dtype, (uint16_t *)p->d_Bp, d_mask);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
+    const hipError_t e = hipStreamSynchronize(s);
+    wait.done = true;
     if (e != hipSuccess)
-        return fail(TW_ERR_DEVICE, "weight packing kernel failed: %s", hipGetErrorString(e));
+        return fail(TW_ERR_DEVICE, "building the plan on the device failed: %s", hipGetErrorString(e));
     return TW_OK;
 }
 
-int pack_from_stream(tw_plan *p, const void *d_Bs, const int64_t *off_B, hipStream_t s)
+// The same from lists in host memory (tile t's kept rows kept_k_idx[kept_k_ptr[t] ..], likewise the
+// columns), which are uploaded first.
+static int build_plan_from_host_lists(tw_plan *p, const int32_t *kept_k_idx, const int32_t *kept_n_idx, PlanSource &src,
+                                      hipStream_t s)
 {
-    const int64_t mg = max_groups(p);
-    if (mg == 0)
-        return TW_OK;
-    std::vector<PackTile> pt = pack_tiles(p, off_B);
-    PackTile *d_pt = nullptr;
-    int st = upload(&d_pt, pt);
-    if (st)
-        return st;
-    DeviceBuffer pt_owner;
-    pt_owner.ptr = d_pt;
-    dim3 grid((unsigned)((mg + 255) / 256), (unsigned)p->n_tiles);
-    hipLaunchKernelGGL(pack_stream_kernel, grid, dim3(256), 0, s, d_pt, (const uint16_t *)d_Bs,
-                       p->K, (uint16_t *)p->d_Bp);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(s);
-    if (e != hipSuccess)
-        return fail(TW_ERR_DEVICE, "stream-weight packing kernel failed: %s", hipGetErrorString(e));
-    return TW_OK;
+    const int nt = p->n_tiles;
+    const size_t sk = p->kept_k_ptr[nt], sn = p->kept_n_ptr[nt];
+    std::vector<int32_t> lists; // kept rows, kept columns, pruned columns
+    lists.reserve(sk + p->N);
+    lists.insert(lists.end(), kept_k_idx, kept_k_idx + sk);
+    lists.insert(lists.end(), kept_n_idx, kept_n_idx + sn);
+    src.kk_src.resize(nt);
+    src.kn_src.resize(nt);
+    src.pn_src.resize(nt);
+    for (int t = 0; t < nt; ++t) {
+        src.kk_src[t] = p->kept_k_ptr[t];
+        src.kn_src[t] = p->kept_n_ptr[t];
+        src.pn_src[t] = (int64_t)(lists.size() - sk - sn);
+        int j = p->kept_n_ptr[t];
+        for (int c = 0; c < p->tile_width[t]; ++c) {
+            if (j < p->kept_n_ptr[t + 1] && kept_n_idx[j] == c)
+                ++j;
+            else
+                lists.push_back(c);
+        }
+    }
+    int dev = -1;
+    TW_HIP(hipGetDevice(&dev));
+    DeviceBuffer d_lists;
+    const size_t bytes = std::max<size_t>(lists.size(), 1) * sizeof(int32_t);
+    if (!d_lists.get(bytes, dev))
+        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the plan's lists failed", bytes);
+    src.kk = static_cast<const int32_t *>(d_lists.ptr);
+    src.kn = src.kk + sk;
+    src.pn = src.kn + sn;
+    if (!lists.empty())
+        TW_HIP(hipMemcpy(d_lists.ptr, lists.data(), lists.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    return build_plan(p, src, s);
 }
 
-int unpack_to_stream(const tw_plan *p, uint16_t *d_Bs, hipStream_t s)
+static int unpack_to_stream(const tw_plan *p, uint16_t *d_Bs, hipStream_t s)
 {
     TW_HIP(hipMemsetAsync(d_Bs, 0, (size_t)p->K * p->N * 2, s));
-    const int64_t mg = max_groups(p);
+    int64_t mg = 0;
+    for (int t = 0; t < p->n_tiles; ++t)
+        mg = std::max<int64_t>(mg, (int64_t)p->k_pad[t] * p->n_pad[t] / 8);
     if (mg > 0) {
-        std::vector<PackTile> pt = pack_tiles(p, nullptr);
-        PackTile *d_pt = nullptr;
-        int st = upload(&d_pt, pt);
-        if (st)
-            return st;
-        DeviceBuffer pt_owner;
-        pt_owner.ptr = d_pt;
-        dim3 grid((unsigned)((mg + 255) / 256), (unsigned)p->n_tiles);
-        hipLaunchKernelGGL(unpack_stream_kernel, grid, dim3(256), 0, s, d_pt,
-                           (const uint16_t *)p->d_Bp, p->K, d_Bs);
-        hipError_t e = hipGetLastError();
-        if (e == hipSuccess)
-            e = hipStreamSynchronize(s);
-        if (e != hipSuccess)
-            return fail(TW_ERR_DEVICE, "unpack kernel failed: %s", hipGetErrorString(e));
+        for (int t0 = 0; t0 < p->n_tiles; t0 += kMaxTileRows)
+            hipLaunchKernelGGL(unpack_stream_kernel, dim3((unsigned)((mg + 255) / 256), std::min(p->n_tiles - t0, kMaxTileRows)),
+                               dim3(256), 0, s, static_cast<const PlanTile *>(p->d_plan_tiles) + t0, (const uint16_t *)p->d_Bp,
+                               p->K, d_Bs);
+        TW_HIP(hipGetLastError());
     }
     TW_HIP(hipStreamSynchronize(s));
     return TW_OK;
-}
-
-static void free_plan(tw_plan *p)
-{
-    if (!p)
-        return;
-    hipFree(p->d_lists);
-    hipFree(p->d_slab);
-    delete p;
 }
 
 static int check_dtype(int dtype)
@@ -833,20 +998,6 @@ static int check_dtype(int dtype)
     if (dtype != TW_F16 && dtype != TW_BF16)
         return fail(TW_ERR_DTYPE, "dtype %d is neither TW_F16 nor TW_BF16", dtype);
     return TW_OK;
-}
-
-// uploads a host fp32 [K,N] weight and packs it
-static int pack_host_weight(tw_plan *p, const float *B)
-{
-    if (p->packed_elems == 0)
-        return TW_OK;
-    DeviceBuffer d_B;
-    size_t bytes = (size_t)p->K * p->N * sizeof(float);
-    if (hipMalloc(&d_B.ptr, bytes) != hipSuccess)
-        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the weight upload failed", bytes);
-    hipError_t e = hipMemcpy(d_B.ptr, B, bytes, hipMemcpyHostToDevice);
-    return e == hipSuccess ? pack_from_dense(p, static_cast<const float *>(d_B.ptr), nullptr)
-                           : fail(TW_ERR_DEVICE, "weight upload failed: %s", hipGetErrorString(e));
 }
 
 } // namespace tw
@@ -884,9 +1035,17 @@ try {
     p->tile_width.assign(tile_width, tile_width + n_tiles);
     p->kept_k_ptr.assign(kept_k_ptr, kept_k_ptr + n_tiles + 1);
     p->kept_n_ptr.assign(kept_n_ptr, kept_n_ptr + n_tiles + 1);
-    p->kept_k_idx.assign(kept_k_idx, kept_k_idx + kept_k_ptr[n_tiles]);
-    p->kept_n_idx.assign(kept_n_idx, kept_n_idx + kept_n_ptr[n_tiles]);
-    if ((st = finalize_plan_geometry(p, nullptr)) || (st = pack_host_weight(p, B)))
+    int dev = -1;
+    TW_HIP(hipGetDevice(&dev));
+    DeviceBuffer d_B;
+    const size_t bytes = (size_t)K * N * sizeof(float);
+    if (!d_B.get(bytes, dev))
+        return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the weight upload failed", bytes);
+    TW_HIP(hipMemcpy(d_B.ptr, B, bytes, hipMemcpyHostToDevice));
+    PlanSource src;
+    src.B = static_cast<const float *>(d_B.ptr);
+    st = build_plan_from_host_lists(p, kept_k_idx, kept_n_idx, src, nullptr);
+    if (st)
         return st;
     *out = owner.release();
     return TW_OK;
@@ -973,123 +1132,112 @@ static int plan_from_device_mask(int K, int N, int dtype, int n_tiles, const int
 
     // one allocation for all temporaries, carved at 256-byte boundaries
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    int max_width = 0;
-    for (int t = 0; t < nt; ++t)
-        max_width = std::max(max_width, tile_width[t]);
-    const int n_seg_k = (K + kSegFlags - 1) / kSegFlags, n_seg_n = (max_width + kSegFlags - 1) / kSegFlags;
-    if ((int64_t)nt * (n_seg_k + n_seg_n) > INT32_MAX || n_seg_k + n_seg_n > 65535)
-        return fail(TW_ERR_SHAPE, "K=%d rows in %d tiles are more than the pre-pass indexes", K, nt);
-    const size_t n_seg = (size_t)nt * (n_seg_k + n_seg_n);
+    const int n_slabs = (K + kFlagRows - 1) / kFlagRows;
     const size_t o_rowflag = 0;
-    const size_t o_colflag = o_rowflag + up((size_t)nt * K);
-    const size_t o_mismatch = o_colflag + up((size_t)N);
-    const size_t o_counts = o_mismatch + up(sizeof(unsigned long long));
-    const size_t o_tcol0 = o_counts + up(sizeof(int32_t) * n_seg);
-    const size_t ws_bytes = o_tcol0 + up(sizeof(int32_t) * (nt + 1));
+    const size_t o_colpart = o_rowflag + up((size_t)nt * K);
+    const size_t o_nnz = o_colpart + up((size_t)(N + 3 * nt + 4) * n_slabs);
+    const size_t o_kk = o_nnz + up(sizeof(uint32_t) * nt * n_slabs);
+    const size_t o_kn = o_kk + up(sizeof(int32_t) * nt * K);
+    const size_t o_pn = o_kn + up(sizeof(int32_t) * N);
+    const size_t ws_bytes = o_pn + up(sizeof(int32_t) * N);
+    int dev = -1;
+    TW_HIP(hipGetDevice(&dev));
     // the workspace and the half-built plan are released on every way out of this function;
     // every kernel and copy runs on the caller's stream, which this function waits for
     DeviceBuffer ws_owner;
+    PinnedBuffer pinned; // the counts, then the tile table
     PlanOwner owner;
-#define TW_TRY(call) TW_HIP(call)
-    TW_TRY(hipMalloc(&ws_owner.ptr, ws_bytes));
+    const size_t counts_bytes = up(sizeof(TileCounts) * nt);
+    if (!ws_owner.get(ws_bytes, dev) || !pinned.get(counts_bytes + sizeof(int32_t) * (nt + 1)))
+        return fail(TW_ERR_ALLOC, "allocation of %zu bytes for the pre-pass failed", ws_bytes);
     char *const ws = static_cast<char *>(ws_owner.ptr);
-    uint8_t *d_rowflag = reinterpret_cast<uint8_t *>(ws + o_rowflag);
-    uint8_t *d_colflag = reinterpret_cast<uint8_t *>(ws + o_colflag);
-    unsigned long long *d_mismatch = reinterpret_cast<unsigned long long *>(ws + o_mismatch);
-    int32_t *d_seg_counts = reinterpret_cast<int32_t *>(ws + o_counts);
-    int32_t *d_tcol0 = reinterpret_cast<int32_t *>(ws + o_tcol0);
-    TW_TRY(hipMemcpyAsync(d_tcol0, tcol0.data(), sizeof(int32_t) * (nt + 1), hipMemcpyHostToDevice, s));
-    // row flags, column flags and the mismatch counter start at zero (adjacent in the workspace)
-    TW_TRY(hipMemsetAsync(ws, 0, o_counts, s));
+    volatile TileCounts *const counts = static_cast<volatile TileCounts *>(pinned.ptr);
+    int32_t *const h_tcol0 = reinterpret_cast<int32_t *>(static_cast<char *>(pinned.ptr) + counts_bytes);
+    std::memcpy(h_tcol0, tcol0.data(), sizeof(int32_t) * (nt + 1));
+    // (never 0, and another number for every build, so that a stamp an earlier build left is not taken for this one's)
+    static std::atomic<uint32_t> builds{0};
+    uint32_t stamp = ++builds;
+    if (stamp == 0)
+        stamp = ++builds;
+    for (int t = 0; t < nt; ++t)
+        counts[t].stamp = 0;
+    FlagArgs fa;
+    fa.mask = d_mask;
+    fa.tcol0 = h_tcol0;
+    fa.K = K;
+    fa.N = N;
+    fa.n_slabs = n_slabs;
+    fa.rowflag = reinterpret_cast<uint8_t *>(ws + o_rowflag);
+    fa.colpart = reinterpret_cast<uint8_t *>(ws + o_colpart);
+    fa.nnz = reinterpret_cast<uint32_t *>(ws + o_nnz);
+    int32_t *const kk = reinterpret_cast<int32_t *>(ws + o_kk);
+    int32_t *const kn = reinterpret_cast<int32_t *>(ws + o_kn);
+    int32_t *const pn = reinterpret_cast<int32_t *>(ws + o_pn);
+    StreamWait wait{s};
+    for (fa.tile0 = 0; fa.tile0 < nt; fa.tile0 += kMaxTileRows)
+        hipLaunchKernelGGL(mask_flags_kernel, dim3(n_slabs, std::min(nt - fa.tile0, kMaxTileRows)), dim3(256), 0, s, fa);
+    hipLaunchKernelGGL(mask_lists_kernel, dim3(nt), dim3(kListThreads), 0, s, fa, kk, kn, pn,
+                       static_cast<TileCounts *>(pinned.ptr), stamp);
+    TW_HIP(hipGetLastError());
 
-    const dim3 seg_grid((unsigned)nt, (unsigned)(n_seg_k + n_seg_n));
-    {
-        // lanes next to each other take the chunks of one row: 64 of them where a row has that
-        // many, else 32 or 16 (two or four rows per wave)
-        const int nchunk = (N + 15) / 16;
-        const int cw = nchunk > 32 ? 64 : (nchunk > 16 ? 32 : 16);
-        const dim3 grid((unsigned)((nchunk + cw - 1) / cw), (unsigned)((K + 63) / 64));
-        hipLaunchKernelGGL(mask_flags_kernel, grid, dim3(256), 0, s, d_mask, K, N, d_tcol0, nt,
-                           cw, d_rowflag, d_colflag);
-        hipLaunchKernelGGL(validate_tw_kernel, grid, dim3(256), 0, s, d_mask, K, N, d_tcol0, nt,
-                           cw, d_rowflag, d_colflag, d_mismatch);
-        hipLaunchKernelGGL(count_flags_kernel, seg_grid, dim3(256), 0, s, d_rowflag, d_colflag,
-                           K, d_tcol0, nt, n_seg_k, n_seg_n, d_seg_counts);
-        TW_TRY(hipGetLastError());
-    }
-    // the mismatch counter and the segment counts come back with one copy (they are adjacent)
-    std::vector<char> back(o_tcol0 - o_mismatch);
-    TW_TRY(hipMemcpyAsync(back.data(), ws + o_mismatch, back.size(), hipMemcpyDeviceToHost, s));
-    TW_TRY(hipStreamSynchronize(s));
+    tw_plan *const p = owner.p = new (std::nothrow) tw_plan;
+    if (!p)
+        return fail(TW_ERR_ALLOC, "out of host memory");
+    p->device = dev;
+    p->K = K;
+    p->N = N;
+    p->dtype = dtype;
+    p->n_tiles = nt;
+    p->tile_col0.assign(tile_col0, tile_col0 + nt);
+    p->tile_width.assign(tile_width, tile_width + nt);
+    p->kept_k_ptr.assign(nt + 1, 0);
+    p->kept_n_ptr.assign(nt + 1, 0);
+    PlanSource src;
+    src.kk = kk;
+    src.kn = kn;
+    src.pn = pn;
+    src.kk_src.resize(nt);
+    src.kn_src.resize(nt);
+    src.pn_src.resize(nt);
+    // The counts arrive in host memory tile by tile: looked at until they are there, which is some 5 us
+    // sooner than the runtime's own wait notices the end of the stream.  The look is bounded by that
+    // wait, taken after a while.
     unsigned long long mismatch = 0;
-    std::memcpy(&mismatch, back.data(), sizeof(mismatch));
-    const int32_t *seg_counts = reinterpret_cast<const int32_t *>(back.data() + (o_counts - o_mismatch));
+    int64_t sum_k = 0;
+    for (int t = 0; t < nt; ++t) {
+        for (long spin = 0; counts[t].stamp != stamp; ++spin) {
+            if (spin < 200000) {
+                __builtin_ia32_pause();
+                continue;
+            }
+            TW_HIP(hipStreamSynchronize(s));
+            if (counts[t].stamp != stamp)
+                return fail(TW_ERR_DEVICE, "the pre-pass left no counts for tile %d", t);
+        }
+        std::atomic_thread_fence(std::memory_order_acquire);
+        const int32_t rows = counts[t].k_kept, cols = counts[t].n_kept;
+        mismatch += (unsigned long long)rows * (unsigned long long)cols - counts[t].nnz;
+        sum_k += rows;
+        p->kept_k_ptr[t + 1] = (int32_t)std::min<int64_t>(sum_k, INT32_MAX);
+        p->kept_n_ptr[t + 1] = p->kept_n_ptr[t] + cols;
+        src.kk_src[t] = (int64_t)t * K;
+        src.kn_src[t] = src.pn_src[t] = tile_col0[t];
+    }
+    if (sum_k > INT32_MAX)
+        return fail(TW_ERR_SHAPE, "K=%d rows in %d tiles are more than the pre-pass indexes", K, nt);
     if (mismatch != 0 && !cover) {
         return fail(TW_ERR_NOT_TW,
                     "%llu mask elements differ from (row kept) & (column kept) of their tile",
                     mismatch);
     }
-
-    tw_plan *const p = owner.p = new (std::nothrow) tw_plan;
-    if (!p)
-        return fail(TW_ERR_ALLOC, "out of host memory");
-    p->K = K;
-    p->N = N;
-    p->dtype = dtype;
-    p->n_tiles = nt;
-    p->tile_col0.resize(nt);
-    p->tile_width.resize(nt);
-    p->kept_k_ptr.assign(nt + 1, 0);
-    p->kept_n_ptr.assign(nt + 1, 0);
-    for (int t = 0; t < nt; ++t) {
-        p->tile_col0[t] = tile_col0[t];
-        p->tile_width[t] = tile_width[t];
-        int rows = 0, cols = 0;
-        for (int g = 0; g < n_seg_k; ++g)
-            rows += seg_counts[(size_t)t * n_seg_k + g];
-        for (int g = 0; g < n_seg_n; ++g)
-            cols += seg_counts[(size_t)nt * n_seg_k + (size_t)t * n_seg_n + g];
-        p->kept_k_ptr[t + 1] = p->kept_k_ptr[t] + rows;
-        p->kept_n_ptr[t + 1] = p->kept_n_ptr[t] + cols;
-    }
-    const size_t sk = std::max(p->kept_k_ptr[nt], 1), sn = std::max(p->kept_n_ptr[nt], 1);
-    // [kept_k | kept_n | rel_k | rel_n], each at a 256-byte boundary: the first two come back
-    // to the host with one copy
-    const size_t l_kn = up(sizeof(int32_t) * sk), l_rk = l_kn + up(sizeof(int32_t) * sn);
-    const size_t l_rn = l_rk + up(sizeof(int32_t) * sk);
-    char *lists = nullptr;
-    TW_TRY(hipMalloc((void **)&lists, l_rn + up(sizeof(int32_t) * sn)));
-    p->d_lists = lists;
-    p->d_kept_k = reinterpret_cast<int32_t *>(lists);
-    p->d_kept_n = reinterpret_cast<int32_t *>(lists + l_kn);
-    p->d_rel_k = reinterpret_cast<int32_t *>(lists + l_rk);
-    p->d_rel_n = reinterpret_cast<int32_t *>(lists + l_rn);
-    hipLaunchKernelGGL(compact_lists_kernel, seg_grid, dim3(256), 0, s, d_rowflag, d_colflag, K,
-                       d_tcol0, nt, n_seg_k, n_seg_n, d_seg_counts, p->d_kept_k, p->d_rel_k,
-                       p->d_kept_n, p->d_rel_n);
-    TW_TRY(hipGetLastError());
-    p->kept_k_idx.resize(p->kept_k_ptr[nt]);
-    p->kept_n_idx.resize(p->kept_n_ptr[nt]);
-    {
-        std::vector<char> both(l_kn + sizeof(int32_t) * sn);
-        TW_TRY(hipMemcpyAsync(both.data(), lists, both.size(), hipMemcpyDeviceToHost, s));
-        TW_TRY(hipStreamSynchronize(s));
-        if (!p->kept_k_idx.empty())
-            std::memcpy(p->kept_k_idx.data(), both.data(), sizeof(int32_t) * p->kept_k_idx.size());
-        if (!p->kept_n_idx.empty())
-            std::memcpy(p->kept_n_idx.data(), both.data() + l_kn, sizeof(int32_t) * p->kept_n_idx.size());
-    }
-#undef TW_TRY
-    st = validate_lists(K, N, nt, p->tile_col0.data(), p->tile_width.data(), p->kept_k_ptr.data(),
-                        p->kept_k_idx.data(), p->kept_n_ptr.data(), p->kept_n_idx.data());
-    if (!st)
-        st = finalize_plan_geometry(p, s);
     // rows and columns of a covering tile are the union of its elements: the elements the mask
     // drops inside that cover are stored as zeros
-    if (!st && p->packed_elems > 0)
-        st = pack_from_dense(p, d_B, s, cover && mismatch != 0 ? d_mask : nullptr);
+    src.B = d_B;
+    src.mask = mismatch != 0 ? d_mask : nullptr;
+    st = build_plan(p, src, s);
     if (st)
         return st;
+    wait.done = true; // (the build has waited)
     *out = owner.release();
     return TW_OK;
 }
@@ -1109,8 +1257,10 @@ static int plan_from_mask_impl(int K, int N, int dtype, int n_tiles, const int32
     if (!mask || !B || !tile_col0 || !tile_width)
         return fail(TW_ERR_NULL, "mask, B or the tile table is NULL");
     const size_t b_bytes = (size_t)K * N * sizeof(float), m_bytes = (size_t)K * N;
+    int dev = -1;
+    TW_HIP(hipGetDevice(&dev));
     DeviceBuffer upload_buf;
-    if (hipMalloc(&upload_buf.ptr, b_bytes + m_bytes) != hipSuccess)
+    if (!upload_buf.get(b_bytes + m_bytes, dev))
         return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes for the mask and weight upload failed",
                     b_bytes + m_bytes);
     char *const buf = static_cast<char *>(upload_buf.ptr);
@@ -1251,10 +1401,11 @@ try {
     p->tile_width = width;
     p->kept_k_ptr = kp;
     p->kept_n_ptr = np;
-    p->kept_k_idx = ki;
-    p->kept_n_idx = ni;
-    if ((st = finalize_plan_geometry(p, nullptr)) ||
-        (st = pack_from_stream(p, B_stream, off_B, nullptr)))
+    PlanSource src;
+    src.Bs = static_cast<const uint16_t *>(B_stream);
+    src.off_B = off_B;
+    st = build_plan_from_host_lists(p, ki.data(), ni.data(), src, nullptr);
+    if (st)
         return st;
     *out = owner.release();
     return TW_OK;
@@ -1302,7 +1453,7 @@ try {
         memcpy(kept_k_ptr, p->kept_k_ptr.data(), sizeof(int32_t) * (nt + 1));
     if (kept_n_ptr)
         memcpy(kept_n_ptr, p->kept_n_ptr.data(), sizeof(int32_t) * (nt + 1));
-    const size_t sk = p->kept_k_idx.size(), sn = p->kept_n_idx.size();
+    const size_t sk = p->kept_k_ptr[nt], sn = p->kept_n_ptr[nt];
     // the index lists come back from the device copies the kernels read
     if (kept_k_idx && sk)
         TW_HIP(hipMemcpy(kept_k_idx, p->d_kept_k, sizeof(int32_t) * sk, hipMemcpyDeviceToHost));
@@ -1313,9 +1464,11 @@ try {
     if (mask_n_rel && sn)
         TW_HIP(hipMemcpy(mask_n_rel, p->d_rel_n, sizeof(int32_t) * sn, hipMemcpyDeviceToHost));
     if (B_stream) {
+        int dev = -1;
+        TW_HIP(hipGetDevice(&dev));
         DeviceBuffer d_Bs;
         const size_t bytes = (size_t)p->K * p->N * 2;
-        if (hipMalloc(&d_Bs.ptr, bytes) != hipSuccess)
+        if (!d_Bs.get(bytes, dev))
             return fail(TW_ERR_ALLOC, "hipMalloc of %zu bytes failed", bytes);
         if (int st = unpack_to_stream(p, static_cast<uint16_t *>(d_Bs.ptr), nullptr))
             return st;
