@@ -964,6 +964,36 @@ def test_skinny_kernel_many_units(tw, oracle):
         tw.set_option(tw.OPT_PIECE, -1)
 
 
+@pytest.mark.parametrize("n_units", [1, 2, 3, 4, 5, 7, 8, 11])
+@pytest.mark.parametrize("M", [1, 33, 500])
+@pytest.mark.parametrize("k_max, width", [(256, 128), (700, 128), (256, 64)])
+def test_skinny_work_split(tw, oracle, n_units, M, k_max, width):
+    """How the skinny kernel hands its work out: units in groups of eight, the ones left over on a
+    set of dies each (row blocks in turn, so workgroups of a row block past the last leave at once),
+    one half or two per unit, four waves (256 kept rows at most) or eight.  Against the oracle, with
+    nothing written outside."""
+    rng = np.random.default_rng([n_units, M, k_max, width])
+    K, N = 720, n_units * width
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    tiles = [dict(col0=t * width, width=width,
+                  kept_k=np.sort(rng.choice(K, size=k_max if t == 0 else int(rng.integers(0, k_max)),
+                                            replace=False)).astype(np.int32),
+                  kept_n=np.sort(rng.choice(width, size=int(rng.integers(1, width + 1)),
+                                            replace=False)).astype(np.int32)) for t in range(n_units)]
+    keep = kept_columns(tiles, N)
+    try:
+        with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+            tw.set_option(tw.OPT_SHAPE, tw.SHAPE_SKINNY)
+            print("skinny split", n_units, M, k_max, width, flush=True)
+            C, bits = run_gemm(tw, oracle, plan, A, "f16", N, pad=8)
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+    ref = reference(oracle, A, B, tiles, "f16")
+    assert oracle.rel_error(C[:, keep], ref[:, keep]) <= TOL["f16"]
+    assert np.all(bits[~keep, :] == SENTINEL) and np.all(bits[:, M:] == SENTINEL)
+
+
 def test_operand_beyond_four_gib(tw, oracle):
     """A of 4.4 GiB: byte offsets into A no longer fit 32 bits, the launch falls back to the
     kernel with 64-bit addressing.  Checked on sampled rows (a row of C depends on the same row

@@ -1865,76 +1865,101 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 }
 
 // ---------------------------------------------------------------------------------
-// Skinny kernel for a handful of rows of A (one time step of a recurrent cell: M = 128): the
+// Skinny kernel for few rows of A (one time step of a recurrent cell: M = 128; a small batch): the
 // launch is then a chain of dependent trips to memory on an almost empty chip, and the streaming
-// kernels walk a tile's kept rows 64 at a time, one trip per step.  Here a workgroup takes
-// 32 rows m of one half of a unit (up to 64 compact columns) and its four waves split the kept
-// rows between them: wave w takes the steps w, w + 4, ... of 64 kept rows, two at a time: it
-// fetches their row numbers, then their 8 KB of A and 16 KB of weight fragments in one go, turns
-// A through its own piece of LDS (no barrier: nobody else reads it) and multiplies.  The four
-// partial products meet in LDS once, are added in wave order (so the result does not depend on
-// timing) and leave through one rounding.  A tile of 512 kept rows is one trip to memory for the
-// numbers and one for the operands.
-//   work:  workgroup (x, y): die x % 8, unit (x / 16) * 8 + die, half (x / 8) % 2, row block y
-//          (a plan without units wider than 64 columns is launched without second halves);
+// kernels walk a tile's kept rows 64 at a time, one trip per step.  Here a workgroup takes 32 rows m
+// of one half of a unit (up to 64 compact columns) and its NW waves split the kept rows between them:
+// wave w takes the steps w, w + NW, ... of 64 kept rows: it fetches their row numbers, then their 4 KB
+// of A and 8 KB of weight fragments in one go, turns A through its own piece of LDS (no barrier:
+// nobody else reads it) and multiplies, each fragment's registers taking the next step's as soon as it
+// is used.  The NW partial products meet in LDS once, are added in wave order (so the result does not
+// depend on timing) and leave through one rounding.  With eight waves a tile of 512 kept rows is one
+// trip to memory for the numbers and one for the operands, and at 128 registers a wave two workgroups
+// share a compute unit.
+//   work:  workgroup b runs on die b % 8.  Units in whole groups of eight have a die each, where their
+//          halves and row blocks share their rows of A and their weight in the L2.  The units left
+//          over (all of them, in a plan of fewer than eight) get as many dies each as there are, a
+//          row block in turn on each of them: with one die each and the others idle the 512 columns
+//          of VGG16 conv4_1 at M 980 took 14.4 us, on all dies 7.7;
 //          the unit comes from the kernel arguments at an offset that depends on the workgroup
-//          number alone, so that it arrives with the other arguments; the halves and row blocks
-//          of a unit sit on one die and share its rows of A in that L2; workgroups of a half the
+//          number alone, so that it arrives with the other arguments; workgroups of a half the
 //          unit does not have fill pruned columns (TW_PRUNED_ZERO) or leave
-//   stage: per wave 2 x 64 rows k of 32 rows m (64 bytes each), then reused for the wave's
+//   stage: per wave 64 rows k of 32 rows m (64 bytes each), then reused for the wave's
 //          partial product [64 columns][32 + 4 rows m] in fp32
-// K-major A and C; any beta.  The sum over k runs in four slices, so the result can differ from
+// K-major A and C; any beta.  The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
-constexpr int kSkWaves = 4;
 constexpr int kSkRows = 32;                            // rows m of a workgroup
 constexpr int kSkCols = 64;                            // compact columns of a workgroup
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
-constexpr int kSkStage = kSkCols * kSkPitch * 4;       // 9216 bytes >= 2 * 64 * 64
-constexpr int kSkLdsBytes = kSkWaves * kSkStage;
+constexpr int kSkStage = kSkCols * kSkPitch * 4;       // 9216 bytes >= 64 * 64
+struct SkinnyWork {
+    int32_t n_units, halves, n_rowblk;
+    int32_t grouped;       // items of a row block in whole groups of eight units
+    int32_t grouped_items; // n_rowblk times that
+    uint32_t magic;        // 2^32 / grouped, rounded up
+    int32_t left;          // units left over
+    int32_t dies_per_unit; // kXcd / left
+};
 
-template <int DT>
-__global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const GemmArgs p, int n_units, int halves)
+template <int DT, int NW>
+__global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
 {
-    constexpr int NT = 64 * kSkWaves;
+    constexpr int NT = 64 * NW;
+    constexpr int RPT = kSkRows * kSkCols / NT; // rows of a column a thread adds up and stores: 8 or 4
     using E = Elem<DT>;
-    __shared__ __align__(16) unsigned char sk_smem[kSkLdsBytes];
+    __shared__ __align__(16) unsigned char sk_smem[NW * kSkStage];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int die = blockIdx.x % kXcd, rest = blockIdx.x / kXcd;
-    // (halves: 2, or 1 for a plan whose units all have at most 64 compact columns)
-    const int half = halves == 2 ? rest & 1 : 0, ui = (halves == 2 ? rest >> 1 : rest) * kXcd + die;
+    // (w.halves: 2, or 1 for a plan whose units all have at most 64 compact columns)
+    const int die = blockIdx.x % kXcd;
+    int half, ui, yblk;
+    bool in_range = true;
+    if ((int)blockIdx.x < w.grouped_items) {
+        yblk = (int)__umulhi(blockIdx.x, w.magic);
+        const int rest = ((int)blockIdx.x - yblk * w.grouped) / kXcd;
+        half = w.halves == 2 ? rest & 1 : 0;
+        ui = (w.halves == 2 ? rest >> 1 : rest) * kXcd + die;
+    } else {
+        const int rest = ((int)blockIdx.x - w.grouped_items) / kXcd;
+        half = w.halves == 2 ? rest & 1 : 0;
+        yblk = (w.halves == 2 ? rest >> 1 : rest) * w.dies_per_unit;
+        int v = die; // unit v of those left over, and which of its dies this is
+        for (; v >= w.left; v -= w.left)
+            ++yblk;
+        in_range = die < w.left * w.dies_per_unit && yblk < w.n_rowblk;
+        ui = w.n_units - w.left + v;
+    }
     // the arguments the first loads need, asked for together with the unit
     // (as integers: a pointer that has been through an asm statement is no longer known to
     // point to global memory)
     uintptr_t A_i = (uintptr_t)p.A, kk_i = (uintptr_t)p.kept_k, kn_i = (uintptr_t)p.kept_n, Bp_i = (uintptr_t)p.Bp;
     int64_t lda = p.lda, ldc = p.ldc;
     int M = p.M;
-    const bool in_range = ui < n_units;
-    const int m0 = blockIdx.y * kSkRows;
+    const int m0 = yblk * kSkRows;
     // the unit: asked for from the kernel arguments before anything else has arrived
     UnitDev u;
     {
         const auto *ka = (const __attribute__((address_space(4))) int32_t *)__builtin_amdgcn_kernarg_segment_ptr();
         const int ua = ui < kMaxArgUnits ? ui : 0;
-        int32_t w[12];
+        int32_t uw[12];
 #pragma unroll
         for (int i = 0; i < 12; ++i)
-            w[i] = ka[offsetof(GemmArgs, arg_units) / 4 + ua * 12 + i];
+            uw[i] = ka[offsetof(GemmArgs, arg_units) / 4 + ua * 12 + i];
         const int n_arg_units = p.n_arg_units;
 #pragma unroll
         for (int i = 0; i < 12; ++i)
-            asm volatile("" : "+s"(w[i])); // asked for here, not behind the test below
+            asm volatile("" : "+s"(uw[i])); // asked for here, not behind the test below
         asm volatile("" : "+s"(A_i), "+s"(kk_i), "+s"(kn_i), "+s"(Bp_i), "+s"(lda), "+s"(ldc), "+s"(M));
         if (!n_arg_units) {
-            const auto *gu = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)(p.units + (in_range ? ui : 0));
+            const auto *gu = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)(p.units + ui);
 #pragma unroll
             for (int i = 0; i < 12; ++i)
-                w[i] = gu[i];
+                uw[i] = gu[i];
         }
 #pragma unroll
         for (int i = 0; i < 12; ++i)
-            w[i] = __builtin_amdgcn_readfirstlane(w[i]);
-        __builtin_memcpy(&u, w, sizeof(UnitDev));
+            uw[i] = __builtin_amdgcn_readfirstlane(uw[i]);
+        __builtin_memcpy(&u, uw, sizeof(UnitDev));
     }
     const int m_end = m0 + kSkRows < M ? m0 + kSkRows : M;
     TW_GLOBAL(const uint16_t) const A = (TW_GLOBAL(const uint16_t))A_i;
@@ -1943,19 +1968,18 @@ __global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const 
     TW_GLOBAL(const int32_t) const kept_n = (TW_GLOBAL(const int32_t))kn_i;
     TW_GLOBAL(const unsigned char) const Bp = (TW_GLOBAL(const unsigned char))Bp_i;
 
-    if (in_range && half * 2 < u.nb_cnt) {
+    if (!in_range)
+        return;
+    if (half * 2 < u.nb_cnt) {
         const int nsteps = u.k_pad / kBlockK;
         const bool two_blocks = half * 2 + 1 < u.nb_cnt;
         unsigned char *const stage = sk_smem + wave * kSkStage;
-        // the reducing role of this lane: column jj of the half, rows m8 .. m8 + 7
-        const int jj = wave * 16 + (lane >> 2), m8 = (lane & 3) * 8;
+        // the reducing role of this lane: column jj of the half, rows mr .. mr + RPT - 1
+        const int jj = tid / (kSkRows / RPT), mr = tid % (kSkRows / RPT) * RPT;
         const int cnt = min(kSkCols, u.n_cnt - half * kSkCols);
 
         struct Numbers {
-            int row[2][4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of step t
-        };
-        struct Loads {
-            u32x4 a[2][4], b[2][2][4];
+            int row[4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of the step
         };
         TW_GLOBAL(const unsigned char) const bsrc = Bp + u.b_off * 2 +
                                           (int64_t)(u.nb0 + half * 2) * 4096 + lane * 16;
@@ -1963,41 +1987,27 @@ __global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const 
         const int ch = lane & 3, row16 = lane >> 2;
         // Nothing on the way to the operands is conditional, so that the waits between the loads
         // are exact counts: a chunk of rows past M is fetched from the row block's first chunk
-        // instead (those rows of the product are never stored), a second step past the end and a
-        // second block the half does not have repeat the first (and are not multiplied, or not
-        // stored).
+        // instead (those rows of the product are never stored), and a second block the half does not
+        // have repeats the first (and is not stored).
         TW_GLOBAL(const uint16_t) const a_lane = A + m0 + (m0 + ch * 8 < M ? ch * 8 : 0);
         const int cb_off = two_blocks ? 4096 : 0;
-        // a pair of steps: s and s + kSkWaves (the second may be past the end)
+        u32x4 av[4], bv[2][4];
         auto numbers = [&](int s) {
             Numbers n;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int st = s + t * kSkWaves < nsteps ? s + t * kSkWaves : s;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    n.row[t][i] = kept_k[u.kk_off + st * kBlockK + i * 16 + row16];
-            }
+            for (int i = 0; i < 4; ++i)
+                n.row[i] = kept_k[u.kk_off + s * kBlockK + i * 16 + row16];
             return n;
         };
-        // (the weight fragments first: they do not wait for the row numbers, so on a wave's
-        // first pair they travel while the numbers are still on their way)
-        auto issue = [&](int s, const Numbers &n, Loads &l) {
+        auto load_b = [&](int s, int k16) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int st = s + t * kSkWaves < nsteps ? s + t * kSkWaves : s;
+            for (int cb = 0; cb < 2; ++cb)
+                bv[cb][k16] = *(TW_GLOBAL(const u32x4))(bsrc + s * step_b + cb * cb_off + k16 * 1024);
+        };
+        auto load_a = [&](const Numbers &n) {
 #pragma unroll
-                for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-                    for (int k16 = 0; k16 < 4; ++k16)
-                        l.b[t][cb][k16] =
-                            *(TW_GLOBAL(const u32x4))(bsrc + st * step_b + cb * cb_off + k16 * 1024);
-            }
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    l.a[t][i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[t][i] * lda);
+            for (int i = 0; i < 4; ++i)
+                av[i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[i] * lda);
         };
         f32x16 acc[2];
 #pragma unroll
@@ -2009,78 +2019,63 @@ __global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const 
         const int pair_e = (lane >> 5) * 4 + (L >> 2);
         const int lane_b = ((lane >> 4) & 1) * 32 + (L & 3) * 8;
         const uint32_t r_first = (uint32_t)((pair_e >> 2) * 8 + (pair_e & 3));
+        TW_LDS(unsigned char) const lds_lane = (TW_LDS(unsigned char))stage + lane_b + r_first * 64;
 
-        // the steps of the pair at s out of one register set: A through the stage, the products
+        // step s out of the registers, which take step s + NW where there is one (MORE; its row numbers
+        // are `n`, which takes those of the step after it)
         // (the tile's list of kept rows is padded to whole steps with row 0: what was fetched for
         // the padding is replaced by zeros here, so that no value of a row the tile does not keep,
         // finite or not, ever reaches a product)
         const int k_lim = u.k_kept - row16;
-        auto multiply = [&](int s, const Loads &l) {
+        auto multiply = [&](int s, Numbers &n, auto more_tag) {
+            constexpr bool MORE = decltype(more_tag)::value;
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int k0 = (s + t * kSkWaves) * kBlockK;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const uint32_t keep = k0 + i * 16 < k_lim ? 0xFFFFFFFFu : 0u;
-                    const u32x4 v = l.a[t][i];
-                    *reinterpret_cast<u32x4 *>(stage + (t * 64 + i * 16 + row16) * 64 + ch * 16) =
-                        u32x4{v.x & keep, v.y & keep, v.z & keep, v.w & keep};
-                }
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t keep = s * kBlockK + i * 16 < k_lim ? 0xFFFFFFFFu : 0u;
+                const u32x4 v = av[i];
+                *reinterpret_cast<u32x4 *>(stage + (i * 16 + row16) * 64 + ch * 16) =
+                    u32x4{v.x & keep, v.y & keep, v.z & keep, v.w & keep};
+            }
+            if (MORE) {
+                load_a(n);
+                n = numbers(s + 2 * NW < nsteps ? s + 2 * NW : s);
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the rows are in the stage
-            TW_LDS(unsigned char) lds_lane = (TW_LDS(unsigned char))stage + lane_b;
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
-                if (s + t * kSkWaves < nsteps) {
-#pragma unroll
-                    for (int k16 = 0; k16 < 4; ++k16) {
-                        const uint32_t r_lo = t * 64 + r_first + k16 * 16, r_hi = r_lo + 4;
-                        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + r_lo * 64));
-                        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + r_hi * 64));
-                        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
-                        const u32x4 af = u32x4{l2.x, l2.y, h2.x, h2.y};
-                        acc[0] = E::mfma(af, l.b[t][0][k16], acc[0]);
-                        acc[1] = E::mfma(af, l.b[t][1][k16], acc[1]);
-                    }
-                }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read before the next steps overwrite it
+            for (int k16 = 0; k16 < 4; ++k16) {
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + k16 * 1024));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + k16 * 1024 + 256));
+                const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+                const u32x4 af = u32x4{l2.x, l2.y, h2.x, h2.y};
+                acc[0] = E::mfma(af, bv[0][k16], acc[0]);
+                acc[1] = E::mfma(af, bv[1][k16], acc[1]);
+                if (MORE)
+                    load_b(s + NW, k16);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // read before the next step overwrites it
         };
-        // One pair is multiplied out of one register set while the operands of the wave's next
-        // pair fill the other and the row numbers of the pair after that are on their way.
-        constexpr int kPair = 2 * kSkWaves;
         int s = wave;
-        int out_col = 0;
-        float out_bias = 0.0f;
-        Loads l0, l1;
-        Numbers n;
+        Numbers n{};
+        // where this lane's sums go, and the bias there: asked for ahead of what takes as long
+        const int out_n = kept_n[u.kn_off + half * kSkCols + (jj < cnt ? jj : 0)];
         if (s < nsteps) {
+            // (the weight fragments first: they do not wait for the row numbers)
             n = numbers(s);
-            issue(s, n, l0);
-            if (s + kPair < nsteps)
-                n = numbers(s + kPair);
+#pragma unroll
+            for (int k16 = 0; k16 < 4; ++k16)
+                load_b(s, k16);
         }
-        // behind the first operands on their way: where this lane's sums go
-        out_col = u.col0 + kept_n[u.kn_off + half * kSkCols + (jj < cnt ? jj : 0)];
-        while (s < nsteps) {
-            if (s + kPair < nsteps) {
-                issue(s + kPair, n, l1);
-                if (s + 2 * kPair < nsteps)
-                    n = numbers(s + 2 * kPair);
-            }
-            multiply(s, l0);
-            s += kPair;
-            if (s >= nsteps)
-                break;
-            if (s + kPair < nsteps) {
-                issue(s + kPair, n, l0);
-                if (s + 2 * kPair < nsteps)
-                    n = numbers(s + 2 * kPair);
-            }
-            multiply(s, l1);
-            s += kPair;
+        const int out_col = u.col0 + out_n;
+        const float out_bias = p.bias ? p.bias[out_col] : 0.0f;
+        if (s < nsteps) {
+            load_a(n);
+            n = numbers(s + NW < nsteps ? s + NW : s);
         }
-        if (p.bias)
-            out_bias = p.bias[out_col];
+        if (s < nsteps) {
+            for (; s + NW < nsteps; s += NW)
+                multiply(s, n, std::true_type());
+            multiply(s, n, std::false_type());
+        }
         // the partial product of this wave: column cb * 32 + lane % 32, rows r4 * 8 + (lane / 32) * 4 + e
         float *const part = reinterpret_cast<float *>(stage);
 #pragma unroll
@@ -2094,57 +2089,63 @@ __global__ void __launch_bounds__(64 * kSkWaves, 1) tw_gemm_skinny_kernel(const 
             }
         __syncthreads();
         // (a wave without steps has written zeros)
-        float sum[8];
+        float sum[RPT];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < RPT; ++e)
             sum[e] = 0.0f;
 #pragma unroll
-        for (int w = 0; w < kSkWaves; ++w) {
-            const float *const src = reinterpret_cast<const float *>(sk_smem + w * kSkStage) + jj * kSkPitch + m8;
+        for (int v = 0; v < NW; ++v) {
+            const float *const src = reinterpret_cast<const float *>(sk_smem + v * kSkStage) + jj * kSkPitch + mr;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < RPT; ++e)
                 sum[e] += src[e];
         }
-        if (jj < cnt && m0 + m8 < m_end) {
-            uint16_t *const dst = C + (int64_t)out_col * ldc + m0 + m8;
-            float v[8];
+        if (jj < cnt && m0 + mr < m_end) {
+            uint16_t *const dst = C + (int64_t)out_col * ldc + m0 + mr;
+            float v[RPT];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < RPT; ++e)
                 v[e] = p.alpha * sum[e];
             if (p.beta != 0.0f) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (m0 + m8 + e < m_end)
+                for (int e = 0; e < RPT; ++e)
+                    if (m0 + mr + e < m_end)
                         v[e] += p.beta * E::from_bits(dst[e]);
             }
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
+            for (int e = 0; e < RPT; ++e)
                 v[e] += out_bias;
             tw_activate_all(v, p.act);
+            uint32_t h[RPT / 2];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                v[e] = tw_fp32_value(v[e]);
-            store_chunk(dst, u32x4{E::to_bits2(v[0], v[1]), E::to_bits2(v[2], v[3]), E::to_bits2(v[4], v[5]), E::to_bits2(v[6], v[7])},
-                        m0 + m8, m_end, false);
+            for (int e = 0; e < RPT / 2; ++e)
+                h[e] = E::to_bits2(tw_fp32_value(v[2 * e]), tw_fp32_value(v[2 * e + 1]));
+            if (m0 + mr + RPT <= m_end) {
+                if constexpr (RPT == 8)
+                    *reinterpret_cast<u32x4 *>(dst) = u32x4{h[0], h[1], h[2], h[3]};
+                else
+                    *reinterpret_cast<u32x2 *>(dst) = u32x2{h[0], h[1]};
+            } else {
+                for (int e = 0; m0 + mr + e < m_end; ++e)
+                    dst[e] = (uint16_t)(h[e >> 1] >> ((e & 1) * 16));
+            }
         }
     }
 
     // ---- TW_PRUNED_ZERO: pruned columns receive act(beta * C + bias); shared out over the
     // workgroups of a row block
-    if (in_range) {
-        for (int z = p.n_gemm_u + ui * halves + half; z < p.n_all_u; z += n_units * halves) {
-            const TileDev t = p.tiles[z - p.n_gemm_u];
-            for (int i = tid; i < t.n_pruned * 4; i += NT) {
-                const int jz = i >> 2, m = m0 + (i & 3) * 8;
-                const int c = t.col0 + p.pruned_n[t.pn_off + jz];
-                uint16_t *const dst = C + (int64_t)c * ldc + m;
-                uint32_t w[4] = {0u, 0u, 0u, 0u};
-                for (int e = 0; e < 8 && m + e < m_end; ++e) {
-                    const float old = p.beta != 0.0f ? p.beta * E::from_bits(dst[e]) : 0.0f;
-                    w[e >> 1] |= E::to_bits(tw_finish(old, p.bias, c, p.act)) << ((e & 1) * 16);
-                }
-                store_chunk(dst, u32x4{w[0], w[1], w[2], w[3]}, m, m_end, false);
+    for (int z = p.n_gemm_u + ui * w.halves + half; z < p.n_all_u; z += w.n_units * w.halves) {
+        const TileDev t = p.tiles[z - p.n_gemm_u];
+        for (int i = tid; i < t.n_pruned * 4; i += NT) {
+            const int jz = i >> 2, m = m0 + (i & 3) * 8;
+            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
+            uint16_t *const dst = C + (int64_t)c * ldc + m;
+            uint32_t h[4] = {0u, 0u, 0u, 0u};
+            for (int e = 0; e < 8 && m + e < m_end; ++e) {
+                const float old = p.beta != 0.0f ? p.beta * E::from_bits(dst[e]) : 0.0f;
+                h[e >> 1] |= E::to_bits(tw_finish(old, p.bias, c, p.act)) << ((e & 1) * 16);
             }
+            store_chunk(dst, u32x4{h[0], h[1], h[2], h[3]}, m, m_end, false);
         }
     }
 }
@@ -2444,6 +2445,26 @@ static int option(int o)
 
 int get_option(int option_id) { return option(option_id); }
 
+// The skinny kernel's work on M rows and its number of workgroups, or -1 where that is more than it
+// numbers: it divides a workgroup's number by `grouped` with a multiplication, exact while number *
+// grouped stays below 2^32.
+static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w)
+{
+    w->n_units = plan->n_units;
+    w->halves = plan->max_unit_n > kSkCols ? 2 : 1;
+    w->n_rowblk = (M + kSkRows - 1) / kSkRows;
+    w->left = plan->n_units % kXcd;
+    w->dies_per_unit = w->left ? kXcd / w->left : 1;
+    const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->halves, grouped_items = grouped * w->n_rowblk;
+    const int64_t left_items = w->left ? (int64_t)kXcd * w->halves * ((w->n_rowblk + w->dies_per_unit - 1) / w->dies_per_unit) : 0;
+    if (grouped_items + left_items > 0x7fffffff || grouped_items * grouped >= (1ll << 32))
+        return -1;
+    w->grouped = (int32_t)grouped;
+    w->grouped_items = (int32_t)grouped_items;
+    w->magic = grouped ? (uint32_t)(((1ull << 32) + grouped - 1) / grouped) : 0u;
+    return grouped_items + left_items;
+}
+
 static int round_up32(int v) { return (v + 31) / 32 * 32; }
 
 // What a launch runs with: kernel shape, columns of a unit piece, workgroups per CU.
@@ -2482,14 +2503,24 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
         return ws_ok && !reads_c && plan->n_blocks > 0 && plan->d_kept_pairs &&
                as_lds_bytes(plan->K, kShapes[shape].bm) <= kLdsBytes;
     };
-    // The skinny kernel where it gives a compute unit at most two workgroups: the launch is then
-    // a chain of trips to memory, which it keeps shortest (measured on M 16 .. 512 of the grid
-    // above, replayed from a graph: 1.6 - 3 x faster up to one workgroup per unit, 1.1 - 1.5 x
-    // up to two).
-    const bool skinny_ok = plan->n_units > 0 && (M + 31) / 32 <= 65535; // its grid: units x row blocks
-    // (not beyond 1024 rows: M 2048, N 512 would still be two workgroups per unit, but each then
-    // walks a whole tile's kept rows for 32 rows of A: 10 - 24 us against 6 - 15)
-    const bool skinny = skinny_ok && M <= 1024 && (int64_t)plan->n_halves * ((M + 31) / 32) <= 2 * (int64_t)cu;
+    // The skinny kernel while its workgroups are few to a compute unit (w) and the tiles not long
+    // (steps): each of them walks a tile's kept rows for 32 rows of A and 64 columns only.  Against
+    // every other shape, replayed from a graph, M 256 .. 4096, N 512 .. 4096, 10 / 25 / 50 % of the
+    // rows kept.  Where the streaming kernels are the alternative it is ahead everywhere below w = 3
+    // (K 4608, N 512, M 2048, 36 steps: 22.9 against 27.5 us; at w = 3, M 3072, 30.8 against 28.7),
+    // to w = 4 while w * steps <= 70 (K 4096, N 1024, M 2048, 16 steps: 18.0 against 19.6) and to w = 6
+    // while w * steps <= 24 (K 2048, N 2048, M 1500, 4 steps: 8.7 against 13.4; K 3072, N 768, M 3072, w 4.5,
+    // 6 steps: 12.2 against 11.3).  Where a panel of A fits LDS, up to w = 3 (K 768, N 3072, M 512: 5.1
+    // against 8.0; K 1024, N 1024, M 1536: 7.3 against 8.3) and to w = 5 while w * steps <= 18 (K 768, N 3072,
+    // M 768, w 4.5, 3 steps: 6.9 against 7.7; M 1024, w 6: 6.8 against 6.0).
+    SkinnyWork sk_work;
+    const int64_t sk_items = plan->n_units > 0 ? skinny_work(plan, M, &sk_work) : -1;
+    const bool skinny_ok = sk_items >= 0;
+    const double sk_w = (double)plan->n_halves * ((M + 31) / 32) / cu, sk_steps = (double)plan->pipe_steps / (double)units;
+    const double sk_cost = sk_w * sk_steps;
+    const bool skinny = skinny_ok && (as_ok(TW_SHAPE_AS64)
+                                          ? sk_w <= 3.0 || (sk_w <= 5.0 && sk_cost <= 18.0)
+                                          : sk_w < 3.0 || (sk_w <= 4.0 && sk_cost <= 70.0) || (sk_w <= 6.0 && sk_cost <= 24.0));
     // The weight-stationary kernel where a tile keeps at most 192 rows under many rows of A, tiles
     // wider than 64 columns.  Measured on M 512 .. 16384, K 768 / 1024 / 4096, N 1024 / 4096 with
     // 64 .. 192 kept rows a tile against the choice below: from 2048 rows of A on it takes 0.58 -
@@ -2522,11 +2553,15 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
                (!plan->rows_shared || width <= 64 || items(256, 128) * 2 <= 3 * cu) && !long_tiles) {
         // (a 0 %-sparse plan with many 256-row items is better off streaming with one queue per
         // die: M 12800, K 768, N 3072: 87 against 96 us)
-        // 64-row panels where they still give three quarters of the compute units a workgroup
-        const int mblk64 = (M + 63) / 64;
+        // 64-row panels where they still give three quarters of the compute units a workgroup, or where
+        // a wave then has fewer blocks to work off one after the other (K 1024, N 4096, half the rows
+        // kept, M 1024: one against two, 13.6 against 16.3 us)
         constexpr int tw64 = as_task_waves(64, false);
-        const int groups64 = std::min(std::max(1, cu / mblk64), (plan->n_blocks + tw64 - 1) / tw64);
-        c.shape = (int64_t)mblk64 * groups64 * 4 >= (int64_t)cu * 3 ? TW_SHAPE_AS64 : TW_SHAPE_AS32;
+        auto groups = [&](int mblk) { return std::min(std::max(1, cu / mblk), (plan->n_blocks + tw64 - 1) / tw64); };
+        auto rounds = [&](int mblk) { return (plan->n_blocks + groups(mblk) * tw64 - 1) / (groups(mblk) * tw64); };
+        const int mblk64 = (M + 63) / 64, mblk32 = (M + 31) / 32;
+        c.shape = (int64_t)mblk64 * groups(mblk64) * 4 >= (int64_t)cu * 3 || rounds(mblk64) < rounds(mblk32) ? TW_SHAPE_AS64
+                                                                                                         : TW_SHAPE_AS32;
     } else if (!as_ok(TW_SHAPE_AS64) && as_ok(TW_SHAPE_AS32) && M > 128 &&
                (M <= 512 || (M <= 1024 && plan->n_blocks <= as_task_waves(32, false) * std::max(1, cu / ((M + 31) / 32))))) {
         // (up to 1024 rows where every wave still has at most one block: M 1024, K 2048, N 2048:
@@ -2616,17 +2651,18 @@ template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, co
     return TW_OK;
 }
 
-// the skinny kernel: one workgroup per (half of a unit, 32-row block)
+// the skinny kernel: one workgroup per (half of a unit, 32-row block); four waves where no tile has
+// more than four steps for them
 template <int DT> static int launch_skinny(const tw_plan *plan, const GemmArgs &a, hipStream_t s)
 {
-    const int halves = plan->max_unit_n > kSkCols ? 2 : 1;
-    const int64_t gx = ((int64_t)plan->n_units + kXcd - 1) / kXcd * kXcd * halves;
-    const int64_t gy = (a.M + kSkRows - 1) / kSkRows;
-    if (gx > (int64_t)0x7fffffff || gy > 65535)
-        return fail(TW_ERR_SHAPE, "%lld x %lld workgroups (M=%d): the skinny kernel takes at most 65535 row blocks",
-                    (long long)gx, (long long)gy, a.M);
-    hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT>), dim3((unsigned)gx, (unsigned)gy), dim3(64 * kSkWaves), 0, s, a,
-                       plan->n_units, halves);
+    SkinnyWork w;
+    const int64_t items = skinny_work(plan, a.M, &w);
+    if (items < 0)
+        return fail(TW_ERR_SHAPE, "M=%d: more row blocks than the skinny kernel numbers", a.M);
+    if (plan->max_k_pad <= 4 * kBlockK)
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
+    else
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
