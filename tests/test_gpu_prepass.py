@@ -263,3 +263,39 @@ def test_long_rows_and_wide_tiles_span_several_segments(tw, oracle):
         assert np.array_equal(got[2]["kept_k"], [5]) and np.array_equal(got[2]["kept_n"], [2090])
         assert np.array_equal(got[2]["mask_k"], [5]) and np.array_equal(got[2]["mask_n"], [2090])
         assert len(got[3]["kept_k"]) == 0
+
+
+def test_plan_destroyed_during_a_capture(tw, oracle):
+    """A plan above a megabyte may be destroyed while a stream is being captured (a host program drops
+    its old plans whenever it likes): the capture goes on, and the plan that takes the memory next is
+    right, also while the graph is replayed."""
+    import torch
+    rng = np.random.default_rng(5)
+    K, N, M = 1024, 1024, 64
+    tiles = random_tiles(rng, K, N, 128, k_keep=0.9, n_keep=1.0)
+    mask = torch.from_numpy(np.ascontiguousarray(oracle.plan_mask(K, N, tiles), np.uint8)).cuda()
+    table = [(t["col0"], t["width"]) for t in tiles]
+    B = [rng.standard_normal((K, N)).astype(np.float32) for _ in range(3)]
+    dB = [torch.from_numpy(b).cuda() for b in B]
+
+    def build(i):
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "bf16", dB[i].data_ptr(),
+                                        stream=torch.cuda.current_stream().cuda_stream)
+
+    x = torch.randn((K, M), device="cuda").to(torch.bfloat16)
+    y, want = (torch.zeros((N, M), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    old = build(0)
+    with build(1) as plan:
+        plan.gemm(x.data_ptr(), want.data_ptr(), M, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(g, stream=s):
+            old.destroy()
+            plan.gemm(x.data_ptr(), y.data_ptr(), M, stream=s.cuda_stream)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            with build(2) as new:
+                check_export(oracle, new, tiles, B[2], "bf16")
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)

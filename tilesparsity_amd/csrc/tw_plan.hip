@@ -493,14 +493,17 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // megabyte in half a microsecond, but maps and unmaps larger ones anew: 25 us for a hipMalloc of 4 MB,
 // 20 - 240 for its hipFree.  Those are kept here when they are given back, up to kPoolBytes a process,
 // and go to the next that asks for about as much on that device; what does not fit is freed, and all
-// of it when an allocation fails.  A piece is given back only when no kernel uses it any more.
+// of it when an allocation fails.  Kernels of a plan that is destroyed may still be queued, on any stream
+// or in a graph: its piece is handed out again only behind a wait for the whole device, made by the build
+// that takes it (a build waits anyway) and not by the destruction, which may come in the middle of a
+// stream capture: a wait would end that.
 constexpr size_t kPoolFrom = 1 << 20, kPoolBytes = 256u << 20;
 class DevicePool {
 public:
     void *get(size_t bytes, int device)
     {
         if (bytes > kPoolFrom) {
-            std::lock_guard<std::mutex> lock(mu_);
+            std::unique_lock<std::mutex> lock(mu_);
             size_t best = free_.size();
             for (size_t i = 0; i < free_.size(); ++i)
                 if (free_[i].device == device && free_[i].bytes >= bytes && free_[i].bytes <= 2 * bytes &&
@@ -511,7 +514,21 @@ public:
                 free_.erase(free_.begin() + best);
                 held_ -= p.bytes;
                 used_[p.ptr] = p.bytes;
-                return p.ptr;
+                if (p.idle)
+                    return p.ptr;
+                const unsigned long long before = ++waits_;
+                lock.unlock();
+                const bool waited = hipDeviceSynchronize() == hipSuccess;
+                if (!waited)
+                    (void)hipGetLastError();
+                lock.lock();
+                if (waited) {
+                    for (Piece &q : free_) // what was given back before that wait
+                        q.idle |= q.device == device && q.wait < before;
+                    return p.ptr;
+                }
+                lock.unlock();
+                put(p.ptr, device, false); // (a capture forbids to wait)
             }
         }
         void *p = nullptr;
@@ -527,7 +544,7 @@ public:
         }
         return p;
     }
-    // no kernel uses `p` any more, or (idle == false) what is queued on the device may
+    // `device` is p's; no kernel uses `p` any more, or (idle == false) what is queued on the device may
     void put(void *p, int device, bool idle)
     {
         if (!p)
@@ -541,13 +558,10 @@ public:
                 used_.erase(it);
             }
         }
-        int now = -1;
-        if (bytes && (hipGetDevice(&now) != hipSuccess || now != device || (!idle && hipDeviceSynchronize() != hipSuccess)))
-            bytes = 0; // (another device is current, or a capture forbids to wait)
         if (bytes) {
             std::lock_guard<std::mutex> lock(mu_);
             if (held_ + bytes <= kPoolBytes) {
-                free_.push_back(Piece{p, bytes, device});
+                free_.push_back(Piece{p, bytes, device, idle, waits_});
                 held_ += bytes;
                 return;
             }
@@ -560,6 +574,8 @@ private:
         void *ptr;
         size_t bytes;
         int device;
+        bool idle;
+        unsigned long long wait; // waits begun before it was given back
     };
     void drop_all()
     {
@@ -573,6 +589,7 @@ private:
     std::vector<Piece> free_;
     std::map<void *, size_t> used_;
     size_t held_ = 0;
+    unsigned long long waits_ = 0;
 };
 // (never destroyed: plans may be, by a host program's own destructors, after the library's)
 static DevicePool &device_pool()
