@@ -195,7 +195,7 @@ def _i32(a):
 
 def _tile_table(table):
     """[(col0, width), ...] as two contiguous int32 arrays and their number."""
-    t = np.array(table, dtype=np.int32).reshape(-1, 2).T.copy()
+    t = np.array([(row[0], row[1]) for row in table], dtype=np.int32).reshape(-1, 2).T.copy()
     return t, len(table)
 
 

@@ -42,9 +42,10 @@ class _DeviceLayers:
         import torch
         self.torch = torch
         self.d_scores = d_scores = []
+        current = torch.cuda.current_device()
         for s in scores:
             if isinstance(s, torch.Tensor):
-                if s.is_cuda and s.dtype is torch.float32:
+                if s.is_cuda and s.dtype is torch.float32 and s.device.index == current:
                     t = s.detach() if s.requires_grad else s
                 else:
                     t = s.detach().to(device="cuda", dtype=torch.float32)
