@@ -964,6 +964,53 @@ def test_skinny_kernel_many_units(tw, oracle):
         tw.set_option(tw.OPT_PIECE, -1)
 
 
+@pytest.mark.parametrize("M, K, n_units, width, k_max, dtype", [
+    (1, 720, 1, 128, 700, "f16"),       # one row: 31 of the 32 repeat it
+    (31, 65, 3, 128, 65, "bf16"),       # a step of one kept row behind a whole one
+    (33, 129, 8, 64, 129, "f16"),       # one half per unit, four waves, one row in the last row block
+    (500, 720, 5, 128, 256, "bf16"),    # four waves with a step each
+    (200, 3001, 9, 128, 2000, "f16"),   # eight waves with several steps, K too long for a panel of A
+])
+def test_skinny_row_major_gives_the_k_major_bits(tw, oracle, M, K, n_units, width, k_max, dtype):
+    """The skinny kernel on row-major A and C: bit for bit its result on K-major copies, with NaN in the
+    rows no tile keeps, beta, bias and filled pruned columns; nothing written outside M x N."""
+    import torch
+    rng = np.random.default_rng([M, K, n_units])
+    N = n_units * width
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    tiles = [dict(col0=t * width, width=width,
+                  kept_k=np.sort(rng.choice(K, size=k_max if t == 0 else int(rng.integers(0, k_max)),
+                                            replace=False)).astype(np.int32),
+                  kept_n=np.sort(rng.choice(width, size=int(rng.integers(1, width + 1)),
+                                            replace=False)).astype(np.int32)) for t in range(n_units)]
+    A[:, np.setdiff1d(np.arange(K), np.concatenate([t["kept_k"] for t in tiles]))] = np.nan
+    Ab, Cb = oracle.cast_bits(A, dtype).reshape(M, K), oracle.cast_bits(C0, dtype).reshape(M, N)
+    lda, ldc, ldm = round_up(K, 8) + 8, round_up(N, 8) + 8, round_up(M, 8)
+    Ar, Cr = np.zeros((M, lda), np.uint16), np.full((M, ldc), SENTINEL, np.uint16)
+    Ak, Ck = np.zeros((K, ldm), np.uint16), np.full((N, ldm), SENTINEL, np.uint16)
+    Ar[:, :K], Cr[:, :N], Ak[:, :M], Ck[:, :M] = Ab, Cb, Ab.T, Cb.T
+    bias = torch.randn(N, device="cuda")
+    try:
+        tw.set_option(tw.OPT_SHAPE, tw.SHAPE_SKINNY)
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            for kw in (dict(pruned_cols=tw.PRUNED_UNTOUCHED),
+                       dict(pruned_cols=tw.PRUNED_ZERO, alpha=0.5, beta=2.0, bias_ptr=bias.data_ptr(),
+                            activation=tw.ACT_GELU)):
+                print("skinny row-major", M, K, n_units, flush=True)
+                dA, dC, dAk, dCk = (to_device_bits(x, x.shape) for x in (Ar, Cr, Ak, Ck))
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, a_layout=tw.ROWMAJOR,
+                          c_layout=tw.ROWMAJOR, **kw)
+                plan.gemm(dAk.data_ptr(), dCk.data_ptr(), M, lda=ldm, ldc=ldm, **kw)
+                torch.cuda.synchronize()
+                have, want = from_device_bits(dC), from_device_bits(dCk)
+                assert np.array_equal(have[:, :N], np.ascontiguousarray(want[:, :M].T))
+                assert np.all(have[:, N:] == SENTINEL)
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+
+
 @pytest.mark.parametrize("n_units", [1, 2, 3, 4, 5, 7, 8, 11])
 @pytest.mark.parametrize("M", [1, 33, 500])
 @pytest.mark.parametrize("k_max, width", [(256, 128), (700, 128), (256, 64)])

@@ -1886,7 +1886,11 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 //          unit does not have fill pruned columns (TW_PRUNED_ZERO) or leave
 //   stage: per wave 64 rows k of 32 rows m (64 bytes each), then reused for the wave's
 //          partial product [64 columns][32 + 4 rows m] in fp32
-// K-major A and C; any beta.  The sum over k runs in NW slices, so the result can differ from
+// K-major A and C, or (RM) row-major ones; any beta.  A kept row of a row-major A is one 2-byte element
+// per m: a lane then takes one kept row of the step and fetches its 32 elements, 64 lanes together a few
+// neighbouring lines of each row m (a quarter kept: four), packs them into the same 64 bytes of the stage,
+// and everything behind it is the same, bit for bit.  C leaves with the lanes along its columns.
+//   The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
 constexpr int kSkRows = 32;                            // rows m of a workgroup
 constexpr int kSkCols = 64;                            // compact columns of a workgroup
@@ -1901,7 +1905,7 @@ struct SkinnyWork {
     int32_t dies_per_unit; // kXcd / left
 };
 
-template <int DT, int NW>
+template <int DT, int NW, bool RM>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
 {
     constexpr int NT = 64 * NW;
@@ -1975,11 +1979,11 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         const bool two_blocks = half * 2 + 1 < u.nb_cnt;
         unsigned char *const stage = sk_smem + wave * kSkStage;
         // the reducing role of this lane: column jj of the half, rows mr .. mr + RPT - 1
-        const int jj = tid / (kSkRows / RPT), mr = tid % (kSkRows / RPT) * RPT;
+        const int jj = RM ? lane : tid / (kSkRows / RPT), mr = RM ? wave * RPT : tid % (kSkRows / RPT) * RPT;
         const int cnt = min(kSkCols, u.n_cnt - half * kSkCols);
 
         struct Numbers {
-            int row[4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of the step
+            int row[RM ? 1 : 4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of the step (RM: kept row `lane`)
         };
         TW_GLOBAL(const unsigned char) const bsrc = Bp + u.b_off * 2 +
                                           (int64_t)(u.nb0 + half * 2) * 4096 + lane * 16;
@@ -1991,12 +1995,17 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         // have repeats the first (and is not stored).
         TW_GLOBAL(const uint16_t) const a_lane = A + m0 + (m0 + ch * 8 < M ? ch * 8 : 0);
         const int cb_off = two_blocks ? 4096 : 0;
-        u32x4 av[4], bv[2][4];
+        u32x4 av[RM ? 1 : 4], bv[2][4];
+        uint32_t ae[RM ? kSkRows : 1];
         auto numbers = [&](int s) {
             Numbers n;
+            if constexpr (RM) {
+                n.row[0] = kept_k[u.kk_off + s * kBlockK + lane];
+            } else {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                n.row[i] = kept_k[u.kk_off + s * kBlockK + i * 16 + row16];
+                for (int i = 0; i < 4; ++i)
+                    n.row[i] = kept_k[u.kk_off + s * kBlockK + i * 16 + row16];
+            }
             return n;
         };
         auto load_b = [&](int s, int k16) {
@@ -2005,9 +2014,15 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                 bv[cb][k16] = *(TW_GLOBAL(const u32x4))(bsrc + s * step_b + cb * cb_off + k16 * 1024);
         };
         auto load_a = [&](const Numbers &n) {
+            if constexpr (RM) { // (rows past M repeat the last one; those of the product are not stored)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                av[i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[i] * lda);
+                for (int i = 0; i < kSkRows; ++i)
+                    ae[i] = (A + (int64_t)(m0 + i < M ? m0 + i : M - 1) * lda)[(uint32_t)n.row[0]];
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    av[i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[i] * lda);
+            }
         };
         f32x16 acc[2];
 #pragma unroll
@@ -2029,6 +2044,17 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         const int k_lim = u.k_kept - row16;
         auto multiply = [&](int s, Numbers &n, auto more_tag) {
             constexpr bool MORE = decltype(more_tag)::value;
+            if constexpr (RM) {
+                const uint32_t keep = s * kBlockK + lane < u.k_kept ? 0xFFFFFFFFu : 0u;
+                uint32_t w2[kSkRows / 2];
+#pragma unroll
+                for (int i = 0; i < kSkRows / 2; ++i)
+                    w2[i] = (ae[2 * i] | (ae[2 * i + 1] << 16)) & keep;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    *reinterpret_cast<u32x4 *>(stage + lane * 64 + i * 16) =
+                        u32x4{w2[4 * i], w2[4 * i + 1], w2[4 * i + 2], w2[4 * i + 3]};
+            } else
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint32_t keep = s * kBlockK + i * 16 < k_lim ? 0xFFFFFFFFu : 0u;
@@ -2101,7 +2127,8 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                 sum[e] += src[e];
         }
         if (jj < cnt && m0 + mr < m_end) {
-            uint16_t *const dst = C + (int64_t)out_col * ldc + m0 + mr;
+            uint16_t *const dst = RM ? C + (int64_t)(m0 + mr) * ldc + out_col : C + (int64_t)out_col * ldc + m0 + mr;
+            const int64_t step_m = RM ? ldc : 1;
             float v[RPT];
 #pragma unroll
             for (int e = 0; e < RPT; ++e)
@@ -2110,7 +2137,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
 #pragma unroll
                 for (int e = 0; e < RPT; ++e)
                     if (m0 + mr + e < m_end)
-                        v[e] += p.beta * E::from_bits(dst[e]);
+                        v[e] += p.beta * E::from_bits(dst[e * step_m]);
             }
 #pragma unroll
             for (int e = 0; e < RPT; ++e)
@@ -2120,7 +2147,12 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
 #pragma unroll
             for (int e = 0; e < RPT / 2; ++e)
                 h[e] = E::to_bits2(tw_fp32_value(v[2 * e]), tw_fp32_value(v[2 * e + 1]));
-            if (m0 + mr + RPT <= m_end) {
+            if constexpr (RM) {
+#pragma unroll
+                for (int e = 0; e < RPT; ++e)
+                    if (m0 + mr + e < m_end)
+                        dst[e * step_m] = (uint16_t)(h[e >> 1] >> ((e & 1) * 16));
+            } else if (m0 + mr + RPT <= m_end) {
                 if constexpr (RPT == 8)
                     *reinterpret_cast<u32x4 *>(dst) = u32x4{h[0], h[1], h[2], h[3]};
                 else
@@ -2136,6 +2168,18 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     // workgroups of a row block
     for (int z = p.n_gemm_u + ui * w.halves + half; z < p.n_all_u; z += w.n_units * w.halves) {
         const TileDev t = p.tiles[z - p.n_gemm_u];
+        if constexpr (RM) {
+            for (int i = tid; i < t.n_pruned * kSkRows; i += NT) {
+                const int m = m0 + i / t.n_pruned;
+                if (m >= m_end)
+                    break;
+                const int c = t.col0 + p.pruned_n[t.pn_off + i % t.n_pruned];
+                uint16_t *const dst = C + (int64_t)m * ldc + c;
+                const float old = p.beta != 0.0f ? p.beta * E::from_bits(*dst) : 0.0f;
+                *dst = (uint16_t)E::to_bits(tw_finish(old, p.bias, c, p.act));
+            }
+            continue;
+        }
         for (int i = tid; i < t.n_pruned * 4; i += NT) {
             const int jz = i >> 2, m = m0 + (i & 3) * 8;
             const int c = t.col0 + p.pruned_n[t.pn_off + jz];
@@ -2631,6 +2675,16 @@ bool takes_row_major_directly(const tw_plan *plan, float beta)
     return beta == 0.0f && plan->d_kept_pairs && plan->n_blocks > 0 && as_lds_bytes(plan->K, 32) <= kLdsBytes;
 }
 
+// the skinny kernel in its row-major form: where it is taken for K-major copies of the operands
+bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
+{
+    // (where a panel of 64 rows of A fits LDS and C is not read the A-stationary kernel's row-major form stays)
+    if (takes_row_major_directly(plan, beta) && as_lds_bytes(plan->K, 64) <= kLdsBytes && option(TW_OPT_SHAPE) != TW_SHAPE_SKINNY)
+        return false;
+    const int64_t ld = ((int64_t)M + 63) / 64 * 64;
+    return choose_shape(plan, M, ld, ld, beta != 0.0f).shape == TW_SHAPE_SKINNY;
+}
+
 template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, const GemmArgs &a, int M, hipStream_t s)
 {
     const int pst = prepare_device();
@@ -2653,16 +2707,16 @@ template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, co
 
 // the skinny kernel: one workgroup per (half of a unit, 32-row block); four waves where no tile has
 // more than four steps for them
-template <int DT> static int launch_skinny(const tw_plan *plan, const GemmArgs &a, hipStream_t s)
+template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const GemmArgs &a, hipStream_t s)
 {
     SkinnyWork w;
     const int64_t items = skinny_work(plan, a.M, &w);
     if (items < 0)
         return fail(TW_ERR_SHAPE, "M=%d: more row blocks than the skinny kernel numbers", a.M);
     if (plan->max_k_pad <= 4 * kBlockK)
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
     else
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
@@ -2901,7 +2955,7 @@ int launch_gemm(const tw_plan *plan, GemmArgs &a, const Choice &c, int32_t *tick
                                         : launch_as<TW_BF16, 32, false>(plan, a, a.M, s);
     }
     if (c.shape == TW_SHAPE_SKINNY)
-        return plan->dtype == TW_F16 ? launch_skinny<TW_F16>(plan, a, s) : launch_skinny<TW_BF16>(plan, a, s);
+        return plan->dtype == TW_F16 ? launch_skinny<TW_F16, false>(plan, a, s) : launch_skinny<TW_BF16, false>(plan, a, s);
     if (c.shape == TW_SHAPE_BS)
         return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), s);
     // queue 0 is the longest: one workgroup per entry, up to the chip's share of a queue
@@ -2954,6 +3008,16 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return st;
     GemmArgs a;
     fill_common(a, plan, A, lda, C, ldc, M, alpha, beta, ep);
+    if (a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR && skinny_takes_row_major(plan, M, beta)) {
+        fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false);
+        if (a.n_all_u == 0)
+            return TW_OK;
+        a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
+        for (int i = 0; i < a.n_arg_units; ++i)
+            a.arg_units[i] = plan->h_units[i];
+        hipStream_t s = (hipStream_t)stream;
+        return plan->dtype == TW_F16 ? launch_skinny<TW_F16, true>(plan, a, s) : launch_skinny<TW_BF16, true>(plan, a, s);
+    }
     if (a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR && takes_row_major_directly(plan, beta)) {
         // both operands row-major, K short enough for a panel of A in LDS, C not read: the
         // A-stationary kernel in its row-major form (64-row panels where they fit and still give

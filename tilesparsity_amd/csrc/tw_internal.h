@@ -182,6 +182,8 @@ int validate_lists(int K, int N, int n_tiles, const int32_t *tile_col0, const in
 // true when tw_gemm_ex takes a row-major A and a row-major C of this plan with a kernel of its own
 // (no layout-generic kernel, no staging): K short enough for a panel of A in LDS and C not read
 bool takes_row_major_directly(const tw_plan *p, float beta);
+// ... and where its kernel for few rows of A takes them, whatever K and beta
+bool skinny_takes_row_major(const tw_plan *p, int M, float beta);
 // the weight-stationary kernel (tw_gemm_bs.hip): whether it takes the plan, and its launch with
 // `per_cu` workgroups meant to share a compute unit
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
