@@ -2678,8 +2678,14 @@ bool takes_row_major_directly(const tw_plan *plan, float beta)
 // the skinny kernel in its row-major form: where it is taken for K-major copies of the operands
 bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
 {
-    // (where a panel of 64 rows of A fits LDS and C is not read the A-stationary kernel's row-major form stays)
-    if (takes_row_major_directly(plan, beta) && as_lds_bytes(plan->K, 64) <= kLdsBytes && option(TW_OPT_SHAPE) != TW_SHAPE_SKINNY)
+    // Against the staged copies it is ahead wherever the rule takes it (K 3072, N 768, M 128: 6.7 against
+    // 10.5 us; M 2048: 21.0 against 26.5).  Against the A-stationary kernel's row-major form, while its
+    // workgroups are at most two to a compute unit (K 768, N 3072, M 128: 4.7 against 7.2; K 1024, N 1024,
+    // M 1024, w 2: 9.4 against 10.3; K 1024, N 4096, M 512, w 4: 7.8 against 7.2; K 2048, N 4096, M 512, w 4: 15.2
+    // against 14.2), and from K 512 on (below, the panel is a few trips: K 320, N 512, M 128 5.0 against 4.1,
+    // N 2048, M 1024 6.3 against 6.3; results there keep the panel kernel's order of sums).
+    if (takes_row_major_directly(plan, beta) && option(TW_OPT_SHAPE) != TW_SHAPE_SKINNY &&
+        (plan->K <= 512 || (double)plan->n_halves * ((M + 31) / 32) > 2.0 * plan->cu_count))
         return false;
     const int64_t ld = ((int64_t)M + 63) / 64 * 64;
     return choose_shape(plan, M, ld, ld, beta != 0.0f).shape == TW_SHAPE_SKINNY;
