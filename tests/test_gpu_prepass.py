@@ -299,3 +299,34 @@ def test_plan_destroyed_during_a_capture(tw, oracle):
                 check_export(oracle, new, tiles, B[2], "bf16")
             torch.cuda.synchronize()
             assert torch.equal(y, want)
+
+
+def test_plans_destroyed_during_a_capture_beyond_what_is_kept(tw):
+    """Plans that are together more than the memory kept for the next builds are destroyed while a stream
+    is being captured: some of it is freed there and then, and the capture goes on."""
+    import torch
+    K, N, M = 4096, 8192, 64
+    mask = torch.ones((K, N), dtype=torch.uint8, device="cuda")
+    W = torch.randn((K, N), device="cuda")
+    table = [(c, 128) for c in range(0, N, 128)]
+
+    def build():
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "f16", W.data_ptr(),
+                                        stream=torch.cuda.current_stream().cuda_stream)
+
+    x = torch.randn((K, M), device="cuda").half()
+    y, want = (torch.zeros((N, M), dtype=torch.float16, device="cuda") for _ in range(2))
+    olds = [build() for _ in range(6)]      # 64 MB of weight each
+    with build() as plan:
+        plan.gemm(x.data_ptr(), want.data_ptr(), M, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(g, stream=s):
+            for old in olds:
+                old.destroy()
+            plan.gemm(x.data_ptr(), y.data_ptr(), M, stream=s.cuda_stream)
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)

@@ -566,10 +566,20 @@ public:
                 return;
             }
         }
-        (void)hipFree(p);
+        free_now(p);
     }
 
 private:
+    // A plan may be destroyed in the middle of a capture, and hipFree in a thread's own mode ends that (or
+    // any global one); in relaxed mode it does not.
+    static void free_now(void *p)
+    {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        if (hipFree(p) != hipSuccess)
+            (void)hipGetLastError();
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
     struct Piece {
         void *ptr;
         size_t bytes;
@@ -581,7 +591,7 @@ private:
     {
         std::lock_guard<std::mutex> lock(mu_);
         for (const Piece &p : free_)
-            (void)hipFree(p.ptr);
+            free_now(p.ptr);
         free_.clear();
         held_ = 0;
     }
