@@ -330,3 +330,96 @@ def test_plans_destroyed_during_a_capture_beyond_what_is_kept(tw):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("mode, threaded", [("thread_local", True), ("relaxed", True), ("relaxed", False)])
+def test_builds_beside_a_capture(tw, oracle, mode, threaded):
+    """While one thread captures a stream, another builds plans out of the memory of destroyed ones (and in
+    relaxed mode the capturing thread does): the capture goes on, its replays and the new plans are right."""
+    import threading
+    import torch
+    rng = np.random.default_rng(6)
+    K, N, M = 1024, 1024, 64
+    tiles = random_tiles(rng, K, N, 128, k_keep=0.9, n_keep=1.0)
+    mask = torch.from_numpy(np.ascontiguousarray(oracle.plan_mask(K, N, tiles), np.uint8)).cuda()
+    table = [(t["col0"], t["width"]) for t in tiles]
+    B = [rng.standard_normal((K, N)).astype(np.float32) for _ in range(2)]
+    dB = [torch.from_numpy(b).cuda() for b in B]
+    side, s = torch.cuda.Stream(), torch.cuda.Stream()
+
+    def build(i):
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "bf16", dB[i].data_ptr(), stream=side.cuda_stream)
+
+    x = torch.randn((K, M), device="cuda").to(torch.bfloat16)
+    y, want = (torch.zeros((N, M), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    made, failed = [], []
+
+    def work():
+        try:
+            for old in olds:
+                old.destroy()
+            made.extend(build(1) for _ in range(3))
+        except Exception as e:
+            failed.append(e)
+
+    olds = [build(1) for _ in range(3)]
+    with build(0) as plan:
+        plan.gemm(x.data_ptr(), want.data_ptr(), M, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s, capture_error_mode=mode):
+            plan.gemm(x.data_ptr(), y.data_ptr(), M, stream=s.cuda_stream)
+            if threaded:
+                t = threading.Thread(target=work)
+                t.start()
+                t.join()
+            else:
+                work()
+        assert not failed, failed
+        for _ in range(3):
+            y.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, want)
+        for p in made:
+            check_export(oracle, p, tiles, B[1], "bf16")
+            p.destroy()
+
+
+@pytest.mark.parametrize("K", [256, 2048])     # a plan below the size whose memory is kept, and one above it
+def test_plan_destroyed_with_products_queued(tw, oracle, K):
+    """Products of a plan are still queued on another stream when it is destroyed and a plan of the same
+    mask with another weight takes its memory: every queued product is the old plan's."""
+    import torch
+    rng = np.random.default_rng(8)
+    N, M = 1024, 512
+    tiles = random_tiles(rng, K, N, 128, k_keep=0.9, n_keep=1.0)
+    mask = torch.from_numpy(np.ascontiguousarray(oracle.plan_mask(K, N, tiles), np.uint8)).cuda()
+    table = [(t["col0"], t["width"]) for t in tiles]
+    dB = [torch.from_numpy(rng.standard_normal((K, N)).astype(np.float32)).cuda() for _ in range(2)]
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def build(i):
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "f16", dB[i].data_ptr(), stream=stream)
+
+    x = (torch.randn((K, M), device="cuda") * 0.1).half()
+    want = torch.zeros((N, M), dtype=torch.float16, device="cuda")
+    ys = [torch.zeros_like(want) for _ in range(60)]
+    big = torch.randn((8192, 8192), device="cuda").half()
+    side = torch.cuda.Stream()
+    old = build(0)
+    old.gemm(x.data_ptr(), want.data_ptr(), M, stream=stream)
+    torch.mm(big, big)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):            # some 20 ms ahead of the products
+            torch.mm(big, big)
+    for y in ys:
+        old.gemm(x.data_ptr(), y.data_ptr(), M, stream=side.cuda_stream)
+    old.destroy()
+    news = [build(1) for _ in range(4)]
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want) for y in ys)
+    for p in news:
+        p.destroy()

@@ -493,10 +493,13 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // megabyte in half a microsecond, but maps and unmaps larger ones anew: 25 us for a hipMalloc of 4 MB,
 // 20 - 240 for its hipFree.  Those are kept here when they are given back, up to kPoolBytes a process,
 // and go to the next that asks for about as much on that device; what does not fit is freed, and all
-// of it when an allocation fails.  Kernels of a plan that is destroyed may still be queued, on any stream
-// or in a graph: its piece is handed out again only behind a wait for the whole device, made by the build
-// that takes it (a build waits anyway) and not by the destruction, which may come in the middle of a
-// stream capture: a wait would end that.
+// of it when an allocation fails.  Kernels of a plan that is destroyed may still be queued, on any
+// stream or in a graph: its piece is handed out again only behind a wait for the whole device, made by
+// the build that takes it (a build waits anyway) and not by the destruction, which may come in the
+// middle of a stream capture.  Nor may that wait be hipDeviceSynchronize: it ends every capture under way
+// in the process, whichever thread and mode it was begun in, and another thread may be capturing while
+// this one builds.  hipFree waits for the device as well, by contract, and leaves the captures of other
+// threads (and relaxed ones) alone, so the wait is the freeing of a small piece.
 constexpr size_t kPoolFrom = 1 << 20, kPoolBytes = 256u << 20;
 class DevicePool {
 public:
@@ -518,9 +521,7 @@ public:
                     return p.ptr;
                 const unsigned long long before = ++waits_;
                 lock.unlock();
-                const bool waited = hipDeviceSynchronize() == hipSuccess;
-                if (!waited)
-                    (void)hipGetLastError();
+                const bool waited = wait_for_device();
                 lock.lock();
                 if (waited) {
                     for (Piece &q : free_) // what was given back before that wait
@@ -579,6 +580,15 @@ private:
         if (hipFree(p) != hipSuccess)
             (void)hipGetLastError();
         (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    // everything queued on the current device has run; false where a capture forbids to wait
+    static bool wait_for_device()
+    {
+        void *p = nullptr;
+        if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess)
+            return true;
+        (void)hipGetLastError();
+        return false;
     }
     struct Piece {
         void *ptr;
