@@ -112,6 +112,28 @@ def test_mix_selection_narrowed_by_a_sample(twprune, po, values):
             assert np.array_equal(a, b), (values, g1)
 
 
+@pytest.mark.parametrize("g1", [50, 9.76, 7])       # the rank among normal scores, below an infinite one, among those
+def test_mix_nan_beside_huge_values(twprune, g1):
+    """A NaN next to a score whose square overflows: every element's score is its own, sqrt(x x), whatever
+    stands beside it.  NaNs rank above everything; the expectation is NumPy's float32 arithmetic on that order."""
+    rng = np.random.default_rng(44)
+    x = rng.random((64, 64)).astype(np.float32)
+    flat = x.reshape(-1)
+    flat[0:800:4], flat[1:800:4] = 1e20, np.nan        # 200 neighbouring pairs, each in one lane's group
+    mask0 = np.zeros(x.shape, bool)
+    with np.errstate(over="ignore", invalid="ignore"):
+        score = np.sqrt(flat * flat)
+        s = np.sort(score)                             # (NaNs last)
+        virt = np.float32(s.size - 1) * (np.float32(100 - g1) / np.float32(100))
+        k = int(np.floor(virt))
+        g, a, b = np.float32(virt - np.floor(virt)), s[k], s[k + 1]
+        thr = b - (b - a) * (np.float32(1) - g) if g >= 0.5 else a + (b - a) * g
+        want = (score > thr).reshape(x.shape)
+    got = twprune.tw_mix_fn([x], g1, [mask0])[0]
+    assert np.array_equal(np.float64(thr), np.float64(twprune.tw_mix_fn.last_threshold), equal_nan=True)
+    assert np.array_equal(want, got)
+
+
 def test_mix_error_paths(tw, twprune):
     with pytest.raises(tw.TwError):
         twprune.tiled_wise_1d_mix([np.ones((4, 4), np.float32)], 50, 2, 120)   # percentile < 0

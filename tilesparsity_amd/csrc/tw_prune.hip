@@ -945,7 +945,8 @@ struct MixLayer {
 // ||x|| of a single element (sqrt(x*x) / 1, the reference's norm over a tile of one column) minus 1
 // where the TW mask already keeps it (prune_algo.py:159-161).  The square root of a rounded square
 // is |x| again as long as the square is a normal number (or zero).
-__device__ __forceinline__ bool mix_plain(float ax) { return (ax >= 1e-18f && ax <= 1e18f) || ax == 0.0f; }
+constexpr float kMixPlainMin = 1e-18f, kMixPlainMax = 1e18f;
+__device__ __forceinline__ bool mix_plain(float ax) { return (ax >= kMixPlainMin && ax <= kMixPlainMax) || ax == 0.0f; }
 __device__ __forceinline__ float mix_value(float x, uint32_t m0)
 {
     float nrm = fabsf(x);
@@ -995,7 +996,9 @@ template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d
 {
     if (d.vec) {
         float ax[4][4];
-        float hi = 0.0f, lo = 1.0f; // largest and (zeros aside) smallest
+        // largest and (zeros aside: 0 - 1 wraps) smallest of the sixteen, by the bits of |x|, where a NaN is
+        // larger than every number
+        uint32_t hi = 0u, lo_less_1 = 0xFFFFFFFFu;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             ax[i][0] = fabsf(d.x[i].x);
@@ -1004,11 +1007,13 @@ template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d
             ax[i][3] = fabsf(d.x[i].w);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                hi = ax[i][e] <= hi ? hi : ax[i][e]; // (a NaN stays)
-                lo = fminf(lo, ax[i][e] == 0.0f ? 1.0f : ax[i][e]);
+                const uint32_t bits = __float_as_uint(ax[i][e]);
+                hi = max(hi, bits);
+                lo_less_1 = min(lo_less_1, bits - 1u);
             }
         }
-        if (!(mix_plain(hi) && mix_plain(lo))) { // one test for all sixteen
+        // mix_plain for all sixteen
+        if (hi > __float_as_uint(kMixPlainMax) || lo_less_1 < __float_as_uint(kMixPlainMin) - 1u) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
