@@ -195,6 +195,31 @@ def test_granularity_pruning_matches_oracle(twprune, po):
     assert np.array_equal(twprune.granularity_pruning(s, 60, 8), po.granularity_pruning(s, 60, 8))
 
 
+@pytest.mark.parametrize("K", [1, 255, 1024, 1025, 8192, 8193])   # around the sizes where the selection changes form
+@pytest.mark.parametrize("values", ["normal", "ties"])
+def test_granularity_pruning_long_tiles(twprune, po, K, values):
+    rng = np.random.default_rng(K)
+    s = np.abs(rng.standard_normal((K, 6))).astype(np.float32)
+    if values == "ties":
+        s = (np.round(s * 2) / 2).astype(np.float32)
+    for sp in (75, np.float64(33.3), 0, 100):
+        assert np.array_equal(twprune.granularity_pruning(s, sp, 2), po.granularity_pruning(s, sp, 2)), sp
+
+
+def test_granularity_pruning_of_single_columns_stays_small(twprune, po):
+    """Tiles of one column: the memory of a call is a small multiple of its scores' (1 MB here), not tens of
+    kilobytes a tile."""
+    import torch
+    rng = np.random.default_rng(26)
+    s = np.abs(rng.standard_normal((16, 16384))).astype(np.float32)
+    twprune.granularity_pruning(s[:, :64], 75, 1)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    got = twprune.granularity_pruning(s, 75, 1)
+    assert free - torch.cuda.mem_get_info()[0] < 100 << 20
+    assert np.array_equal(got, po.granularity_pruning(s, 75, 1))
+
+
 def test_error_paths(tw, twprune):
     with pytest.raises(tw.TwError):
         twprune.tiled_wise_1d([np.ones((4, 4), np.float32)], 150, 2)

@@ -103,7 +103,7 @@ struct PairWalk {
 };
 
 constexpr int kNormNotDivided = 1;   // norms are not divided by the tile width
-constexpr int kPerTileThreshold = 2; // tile t compares with selection state t, not with state 0
+constexpr int kPerTileThreshold = 2; // tile t compares with a threshold of its own (one layer only)
 
 // One entry per layer of a producer call; all layers run in one launch per stage.  The host fills
 // the table, and for the 2-D producer plan_2d_kernel fills in what depends on the kept columns
@@ -358,8 +358,6 @@ struct SelectState {
     uint32_t room;                // values inside it that a wave can keep aside
     uint32_t key_base;            // the passes' digits are those of key - key_base,
     int32_t key_bits;             // which has this many bits
-    float thr32;                  // the threshold, where select_finish_kernel has run
-    double thr64;
 };
 
 // Rank and weight of np.percentile(v[0..n), q): with q_is_f64 == 0 (q was a Python number) the
@@ -697,14 +695,41 @@ template <int NT, class V> __device__ Threshold select_in_block(V key, const Sel
 }
 
 // the thresholds of several segments, or one that only the host wants
-__global__ void __launch_bounds__(256) select_finish_kernel(SelectState *st)
+__global__ void __launch_bounds__(256) select_finish_kernel(const SelectState *st, Threshold *out)
 {
-    st += blockIdx.x;
-    const Threshold t = threshold_of<256>(st);
-    if (threadIdx.x == 0) {
-        st->thr32 = t.v32;
-        st->thr64 = t.v64;
+    const Threshold t = threshold_of<256>(st + blockIdx.x);
+    if (threadIdx.x == 0)
+        out[blockIdx.x] = t;
+}
+
+// One threshold per tile: workgroup t selects among the K norms of tile t, which it keeps in LDS.  The
+// passes over all tiles with counters in memory took 49 KB of them a tile, cleared and read again for
+// a few hundred norms: K 768, N 4096 in tiles of one column 245 against 861 us a call, in tiles of
+// eight 63 against 145.  They remain for tiles of more than kTileSelect norms.
+constexpr int kTileSelect = 8192;
+template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(const float *norms, int K, double q, int q_is_f64, Threshold *out)
+{
+    __shared__ unsigned int s_h[kSelBins];
+    __shared__ SelectHead s_head;
+    __shared__ float s_v[STAGE];
+    const float *const v = norms + (int64_t)blockIdx.x * K;
+    const int tid = (int)threadIdx.x;
+    for (int i0 = tid; i0 < K; i0 += 256 * 4) { // four loads in flight
+        float x[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            x[e] = v[min(i0 + e * 256, K - 1)];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (i0 + e * 256 < K)
+                s_v[i0 + e * 256] = x[e];
     }
+    if (tid == 0)
+        select_rank(&s_head, K, q, q_is_f64);
+    __syncthreads();
+    const Threshold t = select_in_block<256>([&](int i) { return sort_key(s_v[i]); }, &s_head, s_h);
+    if (tid == 0)
+        out[blockIdx.x] = t;
 }
 
 // Between the column stage and the row stage of the 2-D producer, one workgroup: the threshold over
@@ -844,13 +869,13 @@ __global__ void __launch_bounds__(256)
 // twelve BERT-base feed-forward layers, of which 3 are the threshold.
 constexpr int kFillRows = 4, kFillUnits = 1024;
 __global__ void __launch_bounds__(256)
-    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const double *thr_cols, double *mail)
+    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const Threshold *tile_thr, const double *thr_cols,
+                     double *mail)
 {
     const PruneLayer L = layers[LayerFinder(&layers->el_begin, sizeof(PruneLayer), n_layers)(blockIdx.x)];
-    const bool per_tile = (L.flags & kPerTileThreshold) != 0;
-    const Threshold thr = per_tile ? Threshold{} : threshold_of<256>(st);
+    const Threshold thr = tile_thr ? *tile_thr : threshold_of<256>(st); // (tile_thr: one per tile)
     if (blockIdx.x == 0 && threadIdx.x == 0) { // the thresholds, to host memory
-        mail[0] = per_tile ? st->thr64 : thr.v64;
+        mail[0] = thr.v64;
         mail[1] = thr_cols ? *thr_cols : 0.0;
     }
     const uint32_t cpr = (uint32_t)(L.N + 15) >> 4; // chunks per row
@@ -893,9 +918,7 @@ __global__ void __launch_bounds__(256)
             out[r][0] = out[r][1] = out[r][2] = out[r][3] = 0u;
         for (int cb = c0; cb < c0 + n; ++t) { // the tiles the chunk touches: one, or a few
             const int ce = min(begin_of(t + 1), c0 + n);
-            Threshold tt = thr;
-            if (per_tile)
-                tt = Threshold{st[t].thr64, st[t].thr32, st[t].head.f64 != 0};
+            const Threshold tt = tile_thr ? tile_thr[t] : thr;
             float nv[kFillRows];
 #pragma unroll
             for (int r = 0; r < kFillRows; ++r)
@@ -1475,7 +1498,9 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
                  int granularity, uint8_t *const *masks, double *threshold, hipStream_t s, int flags)
 {
     CallTable c = make_table(n_layers, K, N, scores, masks, granularity, flags);
-    const int n_seg = (flags & kPerTileThreshold) ? c.layers[0].n_tiles : 1;
+    const bool per_tile = (flags & kPerTileThreshold) != 0;
+    const int n_seg = per_tile ? c.layers[0].n_tiles : 1;
+    const bool in_blocks = per_tile && K[0] <= kTileSelect; // a workgroup a tile, no counters in memory
     int st = check_percentile(c.n_norms / n_seg, q);
     if (!st)
         st = too_large(std::max(c.n_items, c.n_fill));
@@ -1484,27 +1509,34 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
     Arena ar(s);
     float *d_norms = ar.alloc_n<float>(c.n_norms);
     PruneLayer *d_table = ar.alloc_n<PruneLayer>(n_layers);
-    SelectState *d_st = ar.alloc_n<SelectState>(n_seg);
+    SelectState *d_st = ar.alloc_n<SelectState>(in_blocks ? 0 : n_seg);
+    Threshold *d_tile_thr = per_tile ? ar.alloc_n<Threshold>(n_seg) : nullptr;
     double *mail = ar.mail();
-    if (!d_norms || !d_table || !d_st || !mail)
+    if (!d_norms || !d_table || !d_st || (per_tile && !d_tile_thr) || !mail)
         return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
     int64_t off = 0;
     for (PruneLayer &e : c.layers) {
         e.norms = d_norms + off;
         off += (int64_t)e.K * e.n_tiles;
     }
-    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, d_st, n_seg, c.n_norms / n_seg, q, q_is_f64, s);
+    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q,
+                   q_is_f64, s);
     if (st)
         return st;
     hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers,
                        (const int64_t *)nullptr);
     // per-tile thresholds (one layer): every tile's K norms are one segment
-    st = queue_select(d_norms, c.n_norms / n_seg, d_st, n_seg, s);
-    if (st)
-        return st;
-    if (flags & kPerTileThreshold)
-        hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st);
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st,
+    if (in_blocks) {
+        auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
+        hipLaunchKernelGGL(kernel, dim3(n_seg), dim3(256), 0, s, d_norms, K[0], q, q_is_f64, d_tile_thr);
+    } else {
+        st = queue_select(d_norms, c.n_norms / n_seg, d_st, n_seg, s);
+        if (st)
+            return st;
+        if (per_tile)
+            hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st, d_tile_thr);
+    }
+    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_tile_thr,
                        (const double *)nullptr, mail);
     TW_HIP(hipGetLastError());
     st = ar.wait();
@@ -1643,16 +1675,17 @@ try {
         return st;
     Arena ar(s);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
-    if (!d_st)
+    Threshold *d_thr = ar.alloc_n<Threshold>(1);
+    if (!d_st || !d_thr)
         return fail(TW_ERR_ALLOC, "hipMalloc of the selection state failed");
     st = put_table(nullptr, 0, d_st, d_st, 1, n, q, q_type, s);
     if (!st)
         st = queue_select(values, n, d_st, 1, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(256), 0, s, d_st);
+    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(256), 0, s, d_st, d_thr);
     TW_HIP(hipGetLastError());
-    TW_HIP(hipMemcpyAsync(result, &d_st->thr64, sizeof(double), hipMemcpyDeviceToHost, s));
+    TW_HIP(hipMemcpyAsync(result, &d_thr->v64, sizeof(double), hipMemcpyDeviceToHost, s));
     return ar.wait();
 }
 TW_CATCH_TO_STATUS
@@ -1753,7 +1786,8 @@ try {
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_thr_cols, mail);
+    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st,
+                       (const Threshold *)nullptr, d_thr_cols, mail);
     TW_HIP(hipGetLastError());
     st = ar.wait();
     if (!st && thresholds) {
