@@ -220,6 +220,20 @@ def test_granularity_pruning_of_single_columns_stays_small(twprune, po):
     assert np.array_equal(got, po.granularity_pruning(s, 75, 1))
 
 
+def test_device_masks_have_storage_of_their_own(twprune):
+    """return_device=True: a mask that is kept (or saved) keeps its own bytes alive and no other layer's."""
+    import torch
+    scores = [torch.rand(s, device="cuda") for s in ((64, 96), (33, 7), (128, 40))]
+    calls = [lambda: twprune.tiled_wise_1d(scores, 60, 16, return_device=True),
+             lambda: twprune.tiled_wise_2d(scores, 60, 16, return_device=True),
+             lambda: twprune.tiled_wise_1d_mix(scores, 60, 16, return_device=True),
+             lambda: twprune.tiled_wise_2d_mix(scores, 60, 16, return_device=True)]
+    for call in calls:
+        masks = call()
+        assert [tuple(m.shape) for m in masks] == [tuple(s.shape) for s in scores]
+        assert all(m.untyped_storage().nbytes() == m.numel() for m in masks)
+
+
 def test_error_paths(tw, twprune):
     with pytest.raises(tw.TwError):
         twprune.tiled_wise_1d([np.ones((4, 4), np.float32)], 150, 2)

@@ -35,8 +35,8 @@ def img2col_forward(accumulated_scores):
 
 class _DeviceLayers:
     """Scores on the GPU (uploaded where they are not there yet) and mask buffers, as pointer tables
-    for the C ABI.  The masks of a call are views of one allocation, each starting at a multiple of
-    256 bytes, and so are the column masks, made when they are first asked for."""
+    for the C ABI.  Every mask is a tensor with storage of its own, so that a caller who keeps one keeps
+    no other layer's memory; the column masks are made when they are first asked for."""
 
     def __init__(self, scores):
         import torch
@@ -61,24 +61,18 @@ class _DeviceLayers:
         self.K = np.array([k for k, _ in self.shapes], np.int32)
         self.N = np.array([w for _, w in self.shapes], np.int32)
         self.p_scores = (ctypes.c_void_p * n)(*[t.data_ptr() for t in d_scores])
-        self.d_masks, self.p_masks = self._views([(k, w) for k, w in self.shapes], n)
+        self.d_masks, self.p_masks = self._buffers(self.shapes)
         self._cols = None
         self.stream = torch.cuda.current_stream().cuda_stream
 
-    def _views(self, shapes, n):
-        torch = self.torch
-        offsets, total = [], 0
-        for shape in shapes:
-            offsets.append(total)
-            total += -(-(shape[0] * (shape[1] if len(shape) == 2 else 1)) // 256) * 256
-        flat = torch.empty(total, dtype=torch.uint8, device="cuda")
-        base, cut = flat.data_ptr(), torch.as_strided
-        views = [cut(flat, s, (s[1], 1) if len(s) == 2 else (1,), o) for s, o in zip(shapes, offsets)]
-        return views, (ctypes.c_void_p * n)(*[base + o for o in offsets])
+    def _buffers(self, shapes):
+        empty, u8 = self.torch.empty, self.torch.uint8
+        bufs = [empty(s, dtype=u8, device="cuda") for s in shapes]
+        return bufs, (ctypes.c_void_p * len(bufs))(*[b.data_ptr() for b in bufs])
 
     def _make_cols(self):
         if self._cols is None:
-            self._cols = self._views([(w,) for _, w in self.shapes], len(self.shapes))
+            self._cols = self._buffers([(w,) for _, w in self.shapes])
         return self._cols
 
     d_cols = property(lambda self: self._make_cols()[0])
