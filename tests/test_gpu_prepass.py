@@ -423,3 +423,58 @@ def test_plan_destroyed_with_products_queued(tw, oracle, K):
     assert all(torch.equal(y, want) for y in ys)
     for p in news:
         p.destroy()
+
+
+def test_plan_memory_is_given_back(tw):
+    """What the library keeps of destroyed plans goes back to the device when asked for, behind the work
+    that is queued on it; plans are built beside that and afterwards as before."""
+    import threading
+    import torch
+    K, N, M = 4096, 8192, 64
+    mask = torch.ones((K, N), dtype=torch.uint8, device="cuda")
+    W = torch.randn((K, N), device="cuda")
+    table = [(c, 128) for c in range(0, N, 128)]
+    side = torch.cuda.Stream()
+
+    def build(stream):
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "f16", W.data_ptr(), stream=stream.cuda_stream)
+
+    main = torch.cuda.current_stream()
+    x = torch.randn((K, M), device="cuda").half()
+    want, last = (torch.zeros((N, M), dtype=torch.float16, device="cuda") for _ in range(2))
+    ys = [torch.zeros_like(want) for _ in range(40)]
+    plan = build(main)
+    plan.gemm(x.data_ptr(), want.data_ptr(), M, stream=main.cuda_stream)
+    torch.cuda.synchronize()
+    tw.release_memory()
+    free = torch.cuda.mem_get_info()[0]
+    for y in ys:                                  # queued, then the plan goes
+        plan.gemm(x.data_ptr(), y.data_ptr(), M, stream=side.cuda_stream)
+    plan.destroy()
+    assert torch.cuda.mem_get_info()[0] - free < 64 << 20      # kept for the next build
+    tw.release_memory()
+    assert torch.cuda.mem_get_info()[0] - free >= 64 << 20     # the plan's 64 MB of weight
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want) for y in ys)
+
+    failed = []
+
+    def work():
+        try:
+            s = torch.cuda.Stream()
+            for _ in range(4):
+                build(s).destroy()
+        except Exception as e:
+            failed.append(e)
+
+    t = threading.Thread(target=work)
+    t.start()
+    while t.is_alive():
+        tw.release_memory()
+        t.join(0.001)
+    assert not failed, failed
+    with build(main) as plan:
+        plan.gemm(x.data_ptr(), last.data_ptr(), M, stream=main.cuda_stream)
+        torch.cuda.synchronize()
+    assert torch.equal(last, want)
+    tw.release_memory()

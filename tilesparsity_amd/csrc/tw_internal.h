@@ -179,6 +179,8 @@ int validate_lists(int K, int N, int n_tiles, const int32_t *tile_col0, const in
                    const int32_t *kept_k_ptr, const int32_t *kept_k_idx,
                    const int32_t *kept_n_ptr, const int32_t *kept_n_idx);
 
+// frees the buffer that producer calls leave for the next one
+void release_producer_memory();
 // true when tw_gemm_ex takes a row-major A and a row-major C of this plan with a kernel of its own
 // (no layout-generic kernel, no staging): K short enough for a panel of A in LDS and C not read
 bool takes_row_major_directly(const tw_plan *p, float beta);

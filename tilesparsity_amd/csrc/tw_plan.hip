@@ -493,7 +493,7 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // megabyte in half a microsecond, but maps and unmaps larger ones anew: 25 us for a hipMalloc of 4 MB,
 // 20 - 240 for its hipFree.  Those are kept here when they are given back, up to kPoolBytes a process,
 // and go to the next that asks for about as much on that device; what does not fit is freed, and all
-// of it when an allocation fails.  Kernels of a plan that is destroyed may still be queued, on any
+// of it when an allocation fails or the host program asks for it (tw_release_memory).  Kernels of a plan that is destroyed may still be queued, on any
 // stream or in a graph: its piece is handed out again only behind a wait for the whole device, made by
 // the build that takes it (a build waits anyway) and not by the destruction, which may come in the
 // middle of a stream capture.  Nor may that wait be hipDeviceSynchronize: it ends every capture under way
@@ -569,6 +569,15 @@ public:
         }
         free_now(p);
     }
+    // what is kept goes back to the device (hipFree waits for work still queued on a destroyed plan)
+    void drop_all()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (const Piece &p : free_)
+            free_now(p.ptr);
+        free_.clear();
+        held_ = 0;
+    }
 
 private:
     // A plan may be destroyed in the middle of a capture, and hipFree in a thread's own mode ends that (or
@@ -597,14 +606,6 @@ private:
         bool idle;
         unsigned long long wait; // waits begun before it was given back
     };
-    void drop_all()
-    {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (const Piece &p : free_)
-            free_now(p.ptr);
-        free_.clear();
-        held_ = 0;
-    }
     std::mutex mu_;
     std::vector<Piece> free_;
     std::map<void *, size_t> used_;
@@ -649,6 +650,13 @@ public:
             }
         }
         (void)hipHostFree(p);
+    }
+    void drop_all()
+    {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (const auto &p : free_)
+            (void)hipHostFree(p.first);
+        free_.clear();
     }
 
 private:
@@ -1522,5 +1530,18 @@ int tw_plan_destroy(tw_plan *plan)
     free_plan(plan);
     return TW_OK;
 }
+
+int tw_release_memory(void)
+try {
+    // (another stream, or another thread's, may be under capture)
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    device_pool().drop_all();
+    pinned_pool().drop_all();
+    release_producer_memory();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return TW_OK;
+}
+TW_CATCH_TO_STATUS
 
 } // extern "C"

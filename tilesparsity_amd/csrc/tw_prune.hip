@@ -1316,10 +1316,10 @@ __global__ void __launch_bounds__(256)
 
 namespace {
 
-// Temporaries of one producer call come from a process-wide device buffer that only grows, so
-// that a steady stream of calls does not pay for hipMalloc / hipFree, and its thresholds come back
-// through a page of pinned host memory that its last kernel writes.  The arena holds the lock of
-// both for the duration of the call (producer calls are serialised).
+// Temporaries of one producer call come from a process-wide device buffer that grows (until
+// tw_release_memory gives it back), so that a steady stream of calls does not pay for hipMalloc / hipFree,
+// and its thresholds come back through a page of pinned host memory that its last kernel writes.  The arena
+// holds the lock of both for the duration of the call (producer calls are serialised).
 std::mutex g_ws_mutex;
 void *g_ws = nullptr;
 size_t g_ws_size = 0;
@@ -1546,6 +1546,17 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
 }
 
 } // namespace
+
+void release_producer_memory()
+{
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    if (g_ws && hipFree(g_ws) != hipSuccess)
+        (void)hipGetLastError();
+    g_ws = nullptr;
+    g_ws_size = 0;
+    g_ws_device = -1; // the device of the next call
+}
+
 } // namespace tw
 
 using namespace tw;

@@ -48,7 +48,7 @@ EXPORTED_SYMBOLS = (
     "tw_version", "tw_last_error", "tw_status_string",
     "tw_mask_to_offsets", "tw_offsets_to_kept", "tw_tile_partition",
     "tw_plan_create", "tw_plan_create_dense", "tw_plan_from_mask",
-    "tw_plan_from_stream_operands", "tw_plan_info", "tw_plan_export", "tw_plan_destroy",
+    "tw_plan_from_stream_operands", "tw_plan_info", "tw_plan_export", "tw_plan_destroy", "tw_release_memory",
     "tw_gemm", "tw_stream_gemm_nn", "tw_cast_f32", "tw_delete_row", "tw_insert_row",
     "tw_plan_from_mask_tiles", "tw_prune_tiled_wise_1d", "tw_prune_tiled_wise_2d",
     "tw_tiles_every_g_columns", "tw_tiles_every_g_kept_columns",
@@ -127,6 +127,7 @@ def lib():
         "tw_plan_info": (c_int, [vp, i64p, c_int]),
         "tw_plan_export": (c_int, [vp, i32p, i32p, i32p, i32p, i32p, i32p, i32p, i32p, u16p]),
         "tw_plan_destroy": (c_int, [vp]),
+        "tw_release_memory": (c_int, []),
         "tw_gemm": (c_int, [vp, vp, c_int, c_i64, vp, c_int, c_i64, c_int, c_f, c_f, c_int, vp]),
         "tw_gemm_ex": (c_int, [vp, vp, c_int, c_i64, vp, c_int, c_i64, c_int, c_f, c_f, c_int,
                                ctypes.POINTER(Epilogue), vp]),
@@ -187,6 +188,12 @@ def _check(status):
 def set_option(option, value):
     """tw_set_option: process-wide tuning switch of the GEMM launches (OPT_*), -1 = automatic."""
     _check(lib().tw_set_option(int(option), int(value)))
+
+
+def release_memory():
+    """tw_release_memory: what the library keeps of destroyed plans and between producer calls goes
+    back to the device."""
+    _check(lib().tw_release_memory())
 
 
 def _i32(a):
