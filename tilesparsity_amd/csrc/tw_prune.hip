@@ -412,7 +412,10 @@ struct KeyRange {
 
 // The digit of a finished pass whose counts (NB of them) hold `rank`, the rank among the values with
 // that digit and how many those are, and (NEXT) the next digit any value has (0xFFFFFFFF: none); called by
-// all NT threads of a workgroup, the same values come back to every one.
+// all NT threads of a workgroup, the same values come back to every one.  A rank that is not below the sum of
+// the counts cannot happen; it comes back as kLostRank, which no later pass finds either, and ends the
+// call with an error.
+constexpr unsigned long long kLostRank = ~0ull;
 struct Digit {
     unsigned long long rest, count;
     uint32_t digit, next;
@@ -439,8 +442,8 @@ template <int NT, int NB, bool NEXT = false, class T> __device__ Digit find_digi
     }
     if (lane == 63)
         s_wave[wave] = incl;
-    if (tid == 0) // (a rank below the sum of the counts is always found)
-        s_d = Digit{0, 1, (uint32_t)NB - 1u, 0xFFFFFFFFu};
+    if (tid == 0)
+        s_d = Digit{kLostRank, 1, (uint32_t)NB - 1u, 0xFFFFFFFFu};
     __syncthreads();
     for (int w = 0; w < wave; ++w)
         incl += s_wave[w];
@@ -478,6 +481,7 @@ struct Threshold {
     double v64;
     float v32;
     bool f64;
+    bool lost; // no value had the wanted rank
     __device__ bool passed_by(float v) const { return f64 ? (double)v > v64 : v > v32; }
 };
 
@@ -493,12 +497,12 @@ __device__ Threshold interpolate(const SelectHead *st, uint32_t key_a, uint32_t 
         const double g = st->gamma64;
         const double prod = g >= 0.5 ? (double)diff * (1.0 - g) : (double)diff * g;
         const double r = g >= 0.5 ? (double)b - prod : (double)a + prod;
-        return Threshold{r, (float)r, true};
+        return Threshold{r, (float)r, true, false};
     }
     const float g = st->gamma32;
     const float prod = g >= 0.5f ? diff * (1.0f - g) : diff * g;
     const float r = g >= 0.5f ? b - prod : a + prod;
-    return Threshold{(double)r, r, false};
+    return Threshold{(double)r, r, false, false};
 }
 
 // The threshold out of the counts of the finished last pass, by all NT threads of a workgroup: the key
@@ -519,6 +523,7 @@ template <int NT> __device__ Threshold threshold_of(const SelectState *st)
         if (d.rest + 1 >= d.count) // the wanted value is the last of its kind
             key_b = d.next != 0xFFFFFFFFu ? base + (lead | d.next) : min_gt;
         s_t = interpolate(&st->head, key_a, key_b);
+        s_t.lost = d.rest == kLostRank;
     }
     __syncthreads();
     return s_t;
@@ -689,17 +694,27 @@ template <int NT, class V> __device__ Threshold select_in_block(V key, const Sel
     if (threadIdx.x == 0) {
         const uint32_t a = range.base + prefix;
         s_t = interpolate(h, a, d.rest + 1 < d.count ? a : d.next != 0xFFFFFFFFu ? a - d.digit + d.next : s_min);
+        s_t.lost = d.rest == kLostRank;
     }
     __syncthreads();
     return s_t;
 }
 
+// What a call leaves for the host in its page of pinned memory.
+struct Mail {
+    double thr_rows, thr_cols;
+    int32_t lost; // cleared by the host, set by whoever's selection lost its rank
+};
+
 // the thresholds of several segments, or one that only the host wants
-__global__ void __launch_bounds__(256) select_finish_kernel(const SelectState *st, Threshold *out)
+__global__ void __launch_bounds__(256) select_finish_kernel(const SelectState *st, Threshold *out, Mail *mail)
 {
     const Threshold t = threshold_of<256>(st + blockIdx.x);
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         out[blockIdx.x] = t;
+        if (t.lost)
+            mail->lost = 1;
+    }
 }
 
 // One threshold per tile: workgroup t selects among the K norms of tile t, which it keeps in LDS.  The
@@ -707,7 +722,8 @@ __global__ void __launch_bounds__(256) select_finish_kernel(const SelectState *s
 // a few hundred norms: K 768, N 4096 in tiles of one column 245 against 861 us a call, in tiles of
 // eight 63 against 145.  They remain for tiles of more than kTileSelect norms.
 constexpr int kTileSelect = 8192;
-template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(const float *norms, int K, double q, int q_is_f64, Threshold *out)
+template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(const float *norms, int K, double q, int q_is_f64,
+                                                                               Threshold *out, Mail *mail)
 {
     __shared__ unsigned int s_h[kSelBins];
     __shared__ SelectHead s_head;
@@ -728,8 +744,11 @@ template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(c
         select_rank(&s_head, K, q, q_is_f64);
     __syncthreads();
     const Threshold t = select_in_block<256>([&](int i) { return sort_key(s_v[i]); }, &s_head, s_h);
-    if (tid == 0)
+    if (tid == 0) {
         out[blockIdx.x] = t;
+        if (t.lost)
+            mail->lost = 1;
+    }
 }
 
 // Between the column stage and the row stage of the 2-D producer, one workgroup: the threshold over
@@ -740,7 +759,7 @@ constexpr int kPlanThreads = 1024;
 constexpr int kPlanStage = 12288; // column norms kept in LDS; more of them are read from memory in every pass
 __global__ void __launch_bounds__(kPlanThreads)
     plan_2d_kernel(PruneLayer *layers, int n_layers, const float *cnorm, int64_t n_cols, float *norms,
-                   double *thr_cols, SelectState *st_rows, int64_t *n_items, double q, int q_is_f64)
+                   SelectState *st_rows, int64_t *n_items, double q, int q_is_f64, Mail *mail)
 {
     __shared__ unsigned int s_h[kSelBins];
     __shared__ SelectHead s_head;
@@ -769,8 +788,11 @@ __global__ void __launch_bounds__(kPlanThreads)
         return as_global(cnorm)[i];
     };
     const Threshold thr = select_in_block<kPlanThreads>([&](int i) { return sort_key(norm_of(i)); }, &s_head, s_h);
-    if (tid == 0)
-        *thr_cols = thr.v64;
+    if (tid == 0) {
+        mail->thr_cols = thr.v64;
+        if (thr.lost)
+            mail->lost = 1;
+    }
     int64_t norm_carry = 0, item_carry = 0;
     for (int base = 0; base < n_layers; base += kPlanThreads) {
         const int cnt = min(kPlanThreads, n_layers - base);
@@ -869,14 +891,14 @@ __global__ void __launch_bounds__(256)
 // twelve BERT-base feed-forward layers, of which 3 are the threshold.
 constexpr int kFillRows = 4, kFillUnits = 1024;
 __global__ void __launch_bounds__(256)
-    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const Threshold *tile_thr, const double *thr_cols,
-                     double *mail)
+    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const Threshold *tile_thr, Mail *mail)
 {
     const PruneLayer L = layers[LayerFinder(&layers->el_begin, sizeof(PruneLayer), n_layers)(blockIdx.x)];
     const Threshold thr = tile_thr ? *tile_thr : threshold_of<256>(st); // (tile_thr: one per tile)
-    if (blockIdx.x == 0 && threadIdx.x == 0) { // the thresholds, to host memory
-        mail[0] = thr.v64;
-        mail[1] = thr_cols ? *thr_cols : 0.0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        mail->thr_rows = thr.v64;
+        if (thr.lost)
+            mail->lost = 1;
     }
     const uint32_t cpr = (uint32_t)(L.N + 15) >> 4; // chunks per row
     const int64_t n_units = (int64_t)cpr * ((L.K + kFillRows - 1) / kFillRows);
@@ -1291,11 +1313,14 @@ __global__ void __launch_bounds__(256)
 
 // out = mask0 | (score > threshold)   (prune_algo.py:171-176)
 __global__ void __launch_bounds__(256)
-    mix_mask_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, const float *safe, double *mail)
+    mix_mask_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, const float *safe, Mail *mail)
 {
     const Threshold thr = threshold_of<256>(st);
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        mail[0] = thr.v64;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        mail->thr_rows = thr.v64;
+        if (thr.lost)
+            mail->lost = 1;
+    }
     auto above = [&](float v) { return thr.passed_by(v); };
     auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt) {
         if (cnt == 4) {
@@ -1324,7 +1349,7 @@ std::mutex g_ws_mutex;
 void *g_ws = nullptr;
 size_t g_ws_size = 0;
 int g_ws_device = -1; // the device the buffer lives on; calls on another device do not use it
-double *g_mail = nullptr;
+Mail *g_mail = nullptr;
 
 class Arena {
 public:
@@ -1370,18 +1395,23 @@ public:
         return p;
     }
     template <class T> T *alloc_n(size_t n) { return static_cast<T *>(alloc(sizeof(T) * std::max<size_t>(n, 1))); }
-    // the pinned page, or nullptr
-    double *mail()
+    // the pinned page for this call, or nullptr
+    Mail *mail()
     {
         if (!g_mail && hipHostMalloc((void **)&g_mail, 4096, hipHostMallocPortable) != hipSuccess)
             g_mail = nullptr;
-        return g_mail;
+        mail_ = g_mail;
+        if (mail_)
+            mail_->lost = 0;
+        return mail_;
     }
     // waits for the call's kernels; nothing may be queued behind this
     int wait()
     {
         TW_HIP(hipStreamSynchronize(stream_));
         idle_ = true;
+        if (mail_ && mail_->lost)
+            return fail(TW_ERR_DEVICE, "radix select lost its rank");
         return TW_OK;
     }
 
@@ -1390,6 +1420,7 @@ private:
     hipStream_t stream_;
     int device_ = -1;
     bool usable_ = false, idle_ = false;
+    Mail *mail_ = nullptr;
     size_t off_ = 0, need_ = 0;
     std::vector<void *> extras_;
 };
@@ -1511,7 +1542,7 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
     PruneLayer *d_table = ar.alloc_n<PruneLayer>(n_layers);
     SelectState *d_st = ar.alloc_n<SelectState>(in_blocks ? 0 : n_seg);
     Threshold *d_tile_thr = per_tile ? ar.alloc_n<Threshold>(n_seg) : nullptr;
-    double *mail = ar.mail();
+    Mail *mail = ar.mail();
     if (!d_norms || !d_table || !d_st || (per_tile && !d_tile_thr) || !mail)
         return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
     int64_t off = 0;
@@ -1528,20 +1559,20 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
     // per-tile thresholds (one layer): every tile's K norms are one segment
     if (in_blocks) {
         auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
-        hipLaunchKernelGGL(kernel, dim3(n_seg), dim3(256), 0, s, d_norms, K[0], q, q_is_f64, d_tile_thr);
+        hipLaunchKernelGGL(kernel, dim3(n_seg), dim3(256), 0, s, d_norms, K[0], q, q_is_f64, d_tile_thr, mail);
     } else {
         st = queue_select(d_norms, c.n_norms / n_seg, d_st, n_seg, s);
         if (st)
             return st;
         if (per_tile)
-            hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st, d_tile_thr);
+            hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st, d_tile_thr, mail);
     }
     hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_tile_thr,
-                       (const double *)nullptr, mail);
+                       mail);
     TW_HIP(hipGetLastError());
     st = ar.wait();
     if (!st && threshold)
-        *threshold = mail[0];
+        *threshold = mail->thr_rows;
     return st;
 }
 
@@ -1687,14 +1718,15 @@ try {
     Arena ar(s);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
     Threshold *d_thr = ar.alloc_n<Threshold>(1);
-    if (!d_st || !d_thr)
-        return fail(TW_ERR_ALLOC, "hipMalloc of the selection state failed");
+    Mail *mail = ar.mail();
+    if (!d_st || !d_thr || !mail)
+        return fail(TW_ERR_ALLOC, "allocation of the selection state failed");
     st = put_table(nullptr, 0, d_st, d_st, 1, n, q, q_type, s);
     if (!st)
         st = queue_select(values, n, d_st, 1, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(256), 0, s, d_st, d_thr);
+    hipLaunchKernelGGL(select_finish_kernel, dim3(1), dim3(256), 0, s, d_st, d_thr, mail);
     TW_HIP(hipGetLastError());
     TW_HIP(hipMemcpyAsync(result, &d_thr->v64, sizeof(double), hipMemcpyDeviceToHost, s));
     return ar.wait();
@@ -1763,13 +1795,12 @@ try {
     uint8_t *d_ckeep = ar.alloc_n<uint8_t>(c.n_cols);
     int32_t *d_tcol = ar.alloc_n<int32_t>(c.n_tcol);
     float *d_norms = ar.alloc_n<float>(c.n_norms);
-    int64_t *d_items = ar.alloc_n<int64_t>(2); // the number of items; the columns' threshold
-    double *d_thr_cols = reinterpret_cast<double *>(d_items + 1);
+    int64_t *d_items = ar.alloc_n<int64_t>(1);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
     // both layer tables in one buffer: one upload
     const size_t table_bytes = sizeof(PruneLayer) * n_layers;
     char *d_tables = static_cast<char *>(ar.alloc(table_bytes + sizeof(ColLayer) * n_layers));
-    double *mail = ar.mail();
+    Mail *mail = ar.mail();
     if (!d_cnorm || !d_ckeep || !d_tcol || !d_norms || !d_items || !d_st || !d_tables || !mail)
         return fail(TW_ERR_ALLOC, "allocation for %lld columns and %lld norms failed", (long long)c.n_cols, (long long)c.n_norms);
     PruneLayer *d_table = reinterpret_cast<PruneLayer *>(d_tables);
@@ -1792,18 +1823,18 @@ try {
         return st;
     hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)n_blk), dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm);
     hipLaunchKernelGGL(plan_2d_kernel, dim3(1), dim3(kPlanThreads), 0, s, d_table, n_layers, d_cnorm, c.n_cols, d_norms,
-                       d_thr_cols, d_st, d_items, q, q_type);
+                       d_st, d_items, q, q_type, mail);
     hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, d_items);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
     hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st,
-                       (const Threshold *)nullptr, d_thr_cols, mail);
+                       (const Threshold *)nullptr, mail);
     TW_HIP(hipGetLastError());
     st = ar.wait();
     if (!st && thresholds) {
-        thresholds[0] = mail[1];
-        thresholds[1] = mail[0];
+        thresholds[0] = mail->thr_cols;
+        thresholds[1] = mail->thr_rows;
     }
     return st;
 }
@@ -1844,7 +1875,7 @@ try {
     uint32_t *d_sample = ar.alloc_n<uint32_t>(kMixSamples);
     MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
-    double *mail = ar.mail();
+    Mail *mail = ar.mail();
     if (!d_cand || !d_counts || !d_sample || !d_layers || !d_st || !mail)
         return fail(TW_ERR_ALLOC, "allocation for %lld element scores failed", (long long)total);
     st = put_table(ml.data(), sizeof(MixLayer) * n_layers, d_layers, d_st, 1, total, q, q_type, s, room);
@@ -1864,7 +1895,7 @@ try {
     TW_HIP(hipGetLastError());
     st = ar.wait();
     if (!st && threshold)
-        *threshold = mail[0];
+        *threshold = mail->thr_rows;
     return st;
 }
 TW_CATCH_TO_STATUS
