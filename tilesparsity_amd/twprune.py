@@ -43,6 +43,7 @@ class _DeviceLayers:
         self.torch = torch
         self.d_scores = d_scores = []
         current = torch.cuda.current_device()
+        self.device = torch.device("cuda", current)
         for s in scores:
             if isinstance(s, torch.Tensor):
                 if s.is_cuda and s.dtype is torch.float32 and s.device.index == current:
@@ -66,8 +67,9 @@ class _DeviceLayers:
         self.stream = torch.cuda.current_stream().cuda_stream
 
     def _buffers(self, shapes):
-        empty, u8 = self.torch.empty, self.torch.uint8
-        bufs = [empty(s, dtype=u8, device="cuda") for s in shapes]
+        # (empty_strided with a device object: 1.3 us a tensor, empty with its name 1.8)
+        empty, u8, device = self.torch.empty_strided, self.torch.uint8, self.device
+        bufs = [empty(s, (s[-1], 1) if len(s) == 2 else (1,), dtype=u8, device=device) for s in shapes]
         return bufs, (ctypes.c_void_p * len(bufs))(*[b.data_ptr() for b in bufs])
 
     def _make_cols(self):
