@@ -636,7 +636,10 @@ public:
         }
         void *p = nullptr;
         *size = std::max<size_t>(bytes, 64 << 10);
-        return hipHostMalloc(&p, *size, hipHostMallocPortable) == hipSuccess ? p : nullptr;
+        if (hipHostMalloc(&p, *size, hipHostMallocPortable) == hipSuccess)
+            return p;
+        (void)hipGetLastError(); // (or the next call's check of its launches would find it)
+        return nullptr;
     }
     void put(void *p, size_t size)
     {

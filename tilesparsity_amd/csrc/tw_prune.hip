@@ -1375,8 +1375,12 @@ public:
             g_ws = nullptr;
             g_ws_size = 0;
             const size_t want = need_ + need_ / 2;
-            if (hipMalloc(&g_ws, want) == hipSuccess)
+            if (hipMalloc(&g_ws, want) == hipSuccess) {
                 g_ws_size = want;
+            } else {
+                (void)hipGetLastError();
+                g_ws = nullptr;
+            }
         }
     }
     void *alloc(size_t bytes)
@@ -1389,8 +1393,10 @@ public:
             return p;
         }
         void *p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess)
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError(); // (or the next call's check of its launches would find it)
             return nullptr;
+        }
         extras_.push_back(p);
         return p;
     }
@@ -1398,8 +1404,10 @@ public:
     // the pinned page for this call, or nullptr
     Mail *mail()
     {
-        if (!g_mail && hipHostMalloc((void **)&g_mail, 4096, hipHostMallocPortable) != hipSuccess)
+        if (!g_mail && hipHostMalloc((void **)&g_mail, 4096, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
             g_mail = nullptr;
+        }
         mail_ = g_mail;
         if (mail_)
             mail_->lost = 0;
