@@ -233,8 +233,9 @@ def test_gemm_row_major_layouts(tw, oracle, a_layout, c_layout, dtype, staged):
                                                         N * (c_layout == tw.ROWMAJOR))
                 ws = torch.full((nbytes // 2 + 64,), 0x7bcd, dtype=torch.int16, device="cuda")
                 kw = dict(workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes)
-                # (beta != 0: C is read, so the launch has to stage whatever the layouts are; with
-                # beta == 0 and this short K two row-major operands need no workspace at all)
+                # (beta != 0: a workspace is asked for whatever the layouts are; with beta == 0 and this short K two
+                # row-major operands need none.  At these sizes the few-rows kernel takes two row-major operands as
+                # they are all the same; both staged: test_gemm_both_row_major_operands_staged)
                 with pytest.raises(tw.TwError) as e:
                     plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, beta=1.0, a_layout=a_layout,
                               c_layout=c_layout, workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes - 2)
@@ -270,6 +271,60 @@ def test_gemm_row_major_layouts(tw, oracle, a_layout, c_layout, dtype, staged):
         else:
             expect = oracle.cast_bits(beta * oracle.quantize(C0, dtype)[:, ~keep], dtype)
             assert np.array_equal(np.ascontiguousarray(got)[:, ~keep], expect.reshape(M, -1))
+
+
+@pytest.mark.parametrize("M,K,N", [(203, 150, 330), (100, 2200, 200)])     # a panel of A fits LDS, or does not
+@pytest.mark.parametrize("alpha,beta,pruned", [(1.0, 0.0, 0), (0.5, 2.0, 1)])
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_gemm_both_row_major_operands_staged(tw, oracle, dtype, alpha, beta, pruned, M, K, N):
+    """Row-major A and C where no kernel takes them directly (a streaming shape is forced): tw_gemm_staged
+    turns both through one workspace, A in front and C's old values behind it, and gives the bits of the same
+    shape on K-major operands; tw_gemm_ex takes the layout-generic kernel.  (K 150 with beta == 0 is a
+    panel that fits: taken directly whatever shape is forced.)"""
+    import torch
+    rng = np.random.default_rng(37)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    tiles = random_tiles(rng, K, N, 128, k_keep=0.4, n_keep=0.8)
+    keep = kept_columns(tiles, N)
+    Ab, Cb = oracle.cast_bits(A, dtype).reshape(M, K), oracle.cast_bits(C0, dtype).reshape(M, N)
+    lda, ldc, ldm = round_up(K, 8) + 8, round_up(N, 8) + 8, round_up(M, 8)
+    Ah, Ch = np.zeros((M, lda), np.uint16), np.full((M, ldc), SENTINEL, np.uint16)
+    Ah[:, :K], Ch[:, :N] = Ab, Cb
+    Ak, Ck = np.zeros((K, ldm), np.uint16), np.full((N, ldm), SENTINEL, np.uint16)
+    Ak[:, :M], Ck[:, :M] = Ab.T, Cb.T
+    dA, dAk, dCk = (to_device_bits(x, x.shape) for x in (Ah, Ak, Ck))
+    direct = beta == 0.0 and K == 150
+    ref = reference(oracle, A, B, tiles, dtype, alpha, beta, C0)
+    tw.set_option(tw.OPT_SHAPE, tw.SHAPE_128x128)
+    try:
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            nbytes = plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR)
+            assert nbytes == 2 * round_up(M, 64) * (K + N)
+            ws = torch.full((nbytes // 2 + 64,), 0x7bcd, dtype=torch.int16, device="cuda")
+            kw = dict(alpha=alpha, beta=beta, pruned_cols=pruned)
+            row = dict(lda=lda, ldc=ldc, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+            got = {}
+            for name, extra in (("staged", dict(workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes)), ("generic", {})):
+                dC = to_device_bits(Ch, Ch.shape)
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), M, **kw, **row, **extra)
+                torch.cuda.synchronize()
+                got[name] = from_device_bits(dC)
+            plan.gemm(dAk.data_ptr(), dCk.data_ptr(), M, lda=ldm, ldc=ldm, **kw)
+            torch.cuda.synchronize()
+            want = from_device_bits(dCk)[:, :M].T
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+    assert torch.all(ws[nbytes // 2:] == 0x7bcd)                      # nothing beyond the stated size
+    assert torch.all(ws[:nbytes // 2] == 0x7bcd) == direct            # the workspace was used, or not needed
+    for name, out in got.items():
+        assert np.all(out[:, N:] == SENTINEL)
+        Cf = oracle.bits_to_f32(np.ascontiguousarray(out[:, :N]), dtype).reshape(M, N)
+        assert oracle.rel_error(Cf[:, keep], ref[:, keep]) <= TOL[dtype], name
+        assert np.array_equal(np.ascontiguousarray(out[:, :N])[:, ~keep], np.ascontiguousarray(want)[:, ~keep]), name
+    if not direct:
+        assert np.array_equal(got["staged"][:, :N], want)
 
 
 def test_gemm_degenerate_plans(tw, oracle):
