@@ -1164,3 +1164,27 @@ def test_concurrent_host_threads_and_streams(tw, oracle):
         assert not errors, errors
         for o in outs:
             assert torch.equal(o, want)
+
+
+@pytest.mark.parametrize("M,K,N,kept,skinny", [
+    # workgroups of the kernel for few rows to a compute unit of the fullest of eight dies (of 32 units each): w
+    (1024, 768, 2048, 192, True),       # w 4, four-wave form, a panel of A fits LDS
+    (1280, 768, 2048, 192, False),      # w 5
+    (3072, 768, 768, 192, False),       # w 6: six units leave two dies without work
+    (4096, 384, 512, 250, False),       # w 4, more than 2048 rows, tiles not short
+    (512, 768, 3072, 448, True),        # w 3, eight-wave form
+    (3072, 512, 512, 300, False),       # w 3, more than 1536 rows
+    (2048, 512, 1024, 300, False),      # w 4
+    (768, 2048, 2048, 1024, True),      # w 3, a 32-row panel fits
+    (768, 1536, 3072, 384, False),      # w 4.5
+    (2560, 2048, 768, 500, True),       # w 5, streaming items of 64 columns
+    (2560, 4608, 1024, 460, False),     # w 5, streaming items of 256 x 128
+    (1536, 1536, 2048, 150, True),      # w 6, four-wave form
+    (3072, 3072, 768, 310, False),      # w 6
+])
+def test_kernel_for_few_rows_is_taken_where_it_is_ahead(tw, M, K, N, kept, skinny):
+    """Both sides of the lines of the launch's rule, at problems whose two kernels were timed."""
+    tiles = [dict(col0=c, width=128, kept_k=np.arange(kept, dtype=np.int32), kept_n=np.arange(128, dtype=np.int32))
+             for c in range(0, N, 128)]
+    with tw.Plan.create(K, N, "f16", tiles, np.zeros((K, N), np.float32)) as plan:
+        assert (plan.choice(M, round_up(M, 64), round_up(M, 64))["shape"] == tw.SHAPE_SKINNY) == skinny

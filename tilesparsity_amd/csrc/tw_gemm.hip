@@ -2489,6 +2489,8 @@ static int option(int o)
 
 int get_option(int option_id) { return option(option_id); }
 
+constexpr int kSkFewSteps = 4; // steps of the longest tile up to which the skinny kernel runs with four waves
+
 // The skinny kernel's work on M rows and its number of workgroups, or -1 where that is more than it
 // numbers: it divides a workgroup's number by `grouped` with a multiplication, exact while number *
 // grouped stays below 2^32.
@@ -2507,6 +2509,14 @@ static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w)
     w->grouped_items = (int32_t)grouped_items;
     w->magic = grouped ? (uint32_t)(((1ull << 32) + grouped - 1) / grouped) : 0u;
     return grouped_items + left_items;
+}
+
+// Its workgroups to a compute unit of the die that has most of them (second halves that a unit narrower than the
+// others does not have leave at once and are not counted).
+static double skinny_load(const tw_plan *plan, const SkinnyWork &w)
+{
+    const int per_die = w.grouped / kXcd * w.n_rowblk + (w.left ? w.halves * ((w.n_rowblk + w.dies_per_unit - 1) / w.dies_per_unit) : 0);
+    return (double)per_die * kXcd / plan->cu_count * plan->n_halves / (plan->n_units * w.halves);
 }
 
 static int round_up32(int v) { return (v + 31) / 32 * 32; }
@@ -2547,24 +2557,39 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
         return ws_ok && !reads_c && plan->n_blocks > 0 && plan->d_kept_pairs &&
                as_lds_bytes(plan->K, kShapes[shape].bm) <= kLdsBytes;
     };
-    // The skinny kernel while its workgroups are few to a compute unit (w) and the tiles not long
-    // (steps): each of them walks a tile's kept rows for 32 rows of A and 64 columns only.  Against
-    // every other shape, replayed from a graph, M 256 .. 4096, N 512 .. 4096, 10 / 25 / 50 % of the
-    // rows kept.  Where the streaming kernels are the alternative it is ahead everywhere below w = 3
-    // (K 4608, N 512, M 2048, 36 steps: 22.9 against 27.5 us; at w = 3, M 3072, 30.8 against 28.7),
-    // to w = 4 while w * steps <= 70 (K 4096, N 1024, M 2048, 16 steps: 18.0 against 19.6) and to w = 6
-    // while w * steps <= 24 (K 2048, N 2048, M 1500, 4 steps: 8.7 against 13.4; K 3072, N 768, M 3072, w 4.5,
-    // 6 steps: 12.2 against 11.3).  Where a panel of A fits LDS, up to w = 3 (K 768, N 3072, M 512: 5.1
-    // against 8.0; K 1024, N 1024, M 1536: 7.3 against 8.3) and to w = 5 while w * steps <= 18 (K 768, N 3072,
-    // M 768, w 4.5, 3 steps: 6.9 against 7.7; M 1024, w 6: 6.8 against 6.0).
+    // The skinny kernel while its workgroups are few to a compute unit of the die that has most of them (w:
+    // units left over from groups of eight may leave dies without any) and the tiles not long (steps): each of
+    // them walks a tile's kept rows for 32 rows of A and 64 columns only.  `few`: its form with four waves, of
+    // which four share a compute unit instead of two.  The lines lie where the other shapes, replayed from a
+    // graph, get ahead on M 64 .. 8192, K 256 .. 4608, N 512 .. 4096, 10 / 25 / 50 % of the rows kept:
+    // Where a panel of A fits LDS (against the A-stationary kernel), few: to w = 4 (M 1024, K 768, N 2048, 3 steps:
+    // 6.0 against 7.0 us; w = 5, M 1280: 7.2 against 6.6; w = 6, M 3072, K 768, N 768: 8.4 against 7.2), with
+    // more than 2048 rows only short tiles (M 4096, K 384, N 512, w 4, 3.5 steps: 7.0 against 6.5).  Not few: to
+    // w = 2, and to w = 3 up to 1536 rows (M 512, K 768, N 3072, 6.5 steps: 7.5 against 8.9; M 3072, K 512, N 512,
+    // w 3, 4.5 steps: 8.2 against 6.9; M 2048, K 512, N 1024, w 4: 8.6 against 7.1).
+    // Where it does not, against the streaming kernels: below w = 3 whatever the tiles (K 4608, N 512, M 2048, 36
+    // steps: 22.9 against 27.5), to w = 4 while w * steps <= 70 (K 4096, N 1024, M 2048, 16 steps: 18.0 against
+    // 19.6), to w = 5 while w * steps <= 65 where those have 64-column items (K 2048, N 768, M 2560, 8 steps: 0.93 of
+    // the time; 16 steps: 20.7 against 19.5) and <= 25 against 256 x 128 items (K 4608, N 1024, M 2560, 7 steps: 14.0
+    // against 13.2), and few to w = 6 (K 1536, N 2048, M 1536, 3 steps: 0.81 of the time; K 3072, N 768, M 3072, 5
+    // steps, not few: 12.5 against 10.8).  Against the 32-row panel, which fills the chip above 512 rows: to w = 3
+    // (K 2048, N 2048, M 768, 16 steps: 0.81 of the time), to w = 4 while w * steps <= 40 (K 1536, N 2048, M 1024,
+    // 6 steps: 0.96; 12 steps: 14.3 against 13.3; K 1536, N 3072, M 768, w 4.5, 6 steps: 11.3 against 10.0).
     SkinnyWork sk_work;
     const int64_t sk_items = plan->n_units > 0 ? skinny_work(plan, M, &sk_work) : -1;
     const bool skinny_ok = sk_items >= 0;
-    const double sk_w = (double)plan->n_halves * ((M + 31) / 32) / cu, sk_steps = (double)plan->pipe_steps / (double)units;
+    const double sk_w = skinny_ok ? skinny_load(plan, sk_work) : 0.0, sk_steps = (double)plan->pipe_steps / (double)units;
     const double sk_cost = sk_w * sk_steps;
-    const bool skinny = skinny_ok && (as_ok(TW_SHAPE_AS64)
-                                          ? sk_w <= 3.0 || (sk_w <= 5.0 && sk_cost <= 18.0)
-                                          : sk_w < 3.0 || (sk_w <= 4.0 && sk_cost <= 70.0) || (sk_w <= 6.0 && sk_cost <= 24.0));
+    const bool few = plan->max_k_pad <= kSkFewSteps * kBlockK, panel32 = as_ok(TW_SHAPE_AS32) && M > 512 && M <= 1024;
+    bool skinny;
+    if (as_ok(TW_SHAPE_AS64))
+        skinny = few ? sk_w <= 4.0 && (M <= 2048 || sk_cost <= 12.0) : sk_w <= 2.0 || (sk_w <= 3.0 && M <= 1536);
+    else if (panel32)
+        skinny = sk_w <= 3.0 || (sk_w <= 4.0 && sk_cost <= 40.0) || (few && sk_w <= 6.0);
+    else
+        skinny = sk_w < 3.0 || (sk_w <= 4.0 && sk_cost <= 70.0) || (sk_w <= 5.0 && sk_cost <= (items(256, 128) * 4 <= cu ? 65.0 : 25.0)) ||
+                 (few && sk_w <= 6.0);
+    skinny = skinny && skinny_ok;
     // The weight-stationary kernel where a tile keeps at most 192 rows under many rows of A, tiles
     // wider than 64 columns.  Measured on M 512 .. 16384, K 768 / 1024 / 4096, N 1024 / 4096 with
     // 64 .. 192 kept rows a tile against the choice below: from 2048 rows of A on it takes 0.58 -
@@ -2681,11 +2706,13 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
     // Against the staged copies it is ahead wherever the rule takes it (K 3072, N 768, M 128: 6.7 against
     // 10.5 us; M 2048: 21.0 against 26.5).  Against the A-stationary kernel's row-major form, while its
     // workgroups are at most two to a compute unit (K 768, N 3072, M 128: 4.7 against 7.2; K 1024, N 1024,
-    // M 1024, w 2: 9.4 against 10.3; K 1024, N 4096, M 512, w 4: 7.8 against 7.2; K 2048, N 4096, M 512, w 4: 15.2
-    // against 14.2), and from K 512 on (below, the panel is a few trips: K 320, N 512, M 128 5.0 against 4.1,
-    // N 2048, M 1024 6.3 against 6.3; results there keep the panel kernel's order of sums).
+    // M 1024, w 2: 9.4 against 10.3; K 768, N 768, M 1280, w 2.5: 11.7 against 9.3; K 1024, N 4096, M 512, w 4: 7.8
+    // against 7.2), and beyond K 512 (up to there the panel is a few trips: K 320, N 512, M 128 5.0 against 4.1;
+    // K 512, N 768, M 128, half the rows kept, would be 5.3 against 8.0; results there keep the panel kernel's
+    // order of sums).
+    SkinnyWork w;
     if (takes_row_major_directly(plan, beta) && option(TW_OPT_SHAPE) != TW_SHAPE_SKINNY &&
-        (plan->K <= 512 || (double)plan->n_halves * ((M + 31) / 32) > 2.0 * plan->cu_count))
+        (plan->K <= 512 || plan->n_units <= 0 || skinny_work(plan, M, &w) < 0 || skinny_load(plan, w) > 2.0))
         return false;
     const int64_t ld = ((int64_t)M + 63) / 64 * 64;
     return choose_shape(plan, M, ld, ld, beta != 0.0f).shape == TW_SHAPE_SKINNY;
@@ -2719,7 +2746,7 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     const int64_t items = skinny_work(plan, a.M, &w);
     if (items < 0)
         return fail(TW_ERR_SHAPE, "M=%d: more row blocks than the skinny kernel numbers", a.M);
-    if (plan->max_k_pad <= 4 * kBlockK)
+    if (plan->max_k_pad <= kSkFewSteps * kBlockK)
         hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
     else
         hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
