@@ -289,7 +289,8 @@ int tw_gemm_static(const tw_plan *plan, const void *A, int a_layout, int64_t lda
 /* tw_gemm_ex for row-major operands at the speed of the K-major kernels.  The reference's Python
  * operator multiplies a row-major x[M,K] into a row-major result (mask_dense,
  * Pruning/BERT/utils/modeling.py:992-1007).  tw_gemm_ex takes such operands as they are when both
- * are row-major, K <= 2128 and beta == 0 (a kernel that keeps a panel of A in LDS), and else
+ * are row-major and either K <= 2128 and beta == 0 (a kernel that keeps a panel of A in LDS) or M is small
+ * enough for the kernel for few rows (any K and beta; a rule on workgroups per compute unit), and else
  * through a layout-generic kernel that gathers 2-byte elements.  Here, in those other cases, a row-major A is first turned into
  * its K-major copy and a row-major C is produced K-major and turned back, both in `workspace`
  * (device memory, 16-byte aligned, at least tw_gemm_staged_workspace(plan, M, a_layout, c_layout)
@@ -297,7 +298,8 @@ int tw_gemm_static(const tw_plan *plan, const void *A, int a_layout, int64_t lda
  * each staged operand at the memory rate.  C's old values go through the workspace as well
  * whenever the K-major kernel would leave some of them in place (beta != 0, untouched pruned
  * columns, columns no tile covers).  Same arguments, results and errors as tw_gemm_ex; TW_ERR_BUFFER
- * for a workspace that is missing or too small.  Allocates nothing; with both layouts K-major it is
+ * for a workspace that is missing or too small: unless both are row-major, K <= 2128 and beta == 0 it is asked for
+ * whatever M is, also where the kernel for few rows then does without.  Allocates nothing; with both layouts K-major it is
  * tw_gemm_ex.  Calls that share a workspace must not overlap. */
 int64_t tw_gemm_staged_workspace(const tw_plan *plan, int M, int a_layout, int c_layout);
 int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda, void *C,

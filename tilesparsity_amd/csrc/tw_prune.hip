@@ -9,8 +9,8 @@
 //     halves combined above that);
 //   * a column norm accumulates the rows one after the other;
 //   * np.percentile with linear interpolation: the two neighbouring order statistics are found
-//     here with a radix select, the interpolation runs on the host in the arithmetic type
-//     NumPy would use for the given kind of `q`;
+//     here with a radix select, and interpolated here in the arithmetic type NumPy would
+//     use for the given kind of `q`;
 //   * comparisons are strict.
 // This file is compiled with floating-point contraction off (pragma below): a product and the sum
 // that takes it stay two rounded operations, as in NumPy.  The __fmul_rn / __fadd_rn intrinsics
@@ -166,7 +166,7 @@ private:
 // row add from there.  The pitch of a staged row is 8 floats past 128, so the eight rows a wave adds
 // at a time lie in eight different groups of banks.  The pointers out of the layer table are known to
 // be global and no load is conditional: flat or predicated loads wait for each other.  Bound by the
-// read: the feed-forward weights of twelve BERT-base layers (226 MB) in 43 us, 5.2 TB/s (a kernel
+// read: the feed-forward weights of twelve BERT-base layers (226 MB) in 40 us, 5.6 TB/s (a kernel
 // that only reads them 35); 92 us when every lane loaded what it added.
 constexpr int kNormRows = 32;     // rows of an item: eight lanes each
 constexpr int kNormPitch = 136;   // floats; a block of 128 columns with up to 3 before it
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(256, 6)
 // workgroup, as much as hides the way to memory), square them and leave them in LDS as [column][row];
 // a fifth adds, four rows per LDS read.
 // All layers share one launch; a column block belongs to one layer (blk_begin: its first block).
-// 31 us for the 126 MB of VGG16's layers (4.1 TB/s, the chain of 4608 additions being about as long);
+// 26 us for the 126 MB of VGG16's layers (4.8 TB/s, the chain of 4608 additions being about as long);
 // 117 us with a thread per column that loads 32 rows ahead of its additions.
 struct ColLayer {
     const float *score;
@@ -335,8 +335,8 @@ __device__ __forceinline__ float key_to_float(uint32_t key)
 // layer over a few dozen counters; with 8 bits, two octaves a digit, most lanes of a wave met in one
 // or two LDS counters: 38 us a pass over 31.5 M values.)
 // Pass p counts the values that agree with the digits before it; which digit holds the rank is
-// worked out of the histogram by every workgroup of the next pass, and the workgroup of the last
-// pass that finishes last works out the threshold.
+// worked out of the histogram by every workgroup of the next pass, and the threshold out of the
+// last one by whatever uses it (threshold_of).
 constexpr int kSelBins = 2048;
 struct SelectHead {               // the wanted rank and the interpolation above it
     int64_t n;                    // number of values
@@ -1118,7 +1118,7 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // between (2 - 3 % of the elements), and the three passes run over what was kept.
 // Where the bracket missed or does not fit - the counts tell, for certain - they run over the
 // elements.
-// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 15 + 32 + 40 us.
+// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 14 + 31 + 39 us.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
 __global__ void __launch_bounds__(256) mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, uint32_t *sample)
@@ -1492,8 +1492,8 @@ int check_layers(int n_layers, const int32_t *K, const int32_t *N, const float *
     return TW_OK;
 }
 
-// The table of a call whose tiles are every `granularity` columns, or (tile_tables != nullptr) at most
-// that many tiles, found on the device.
+// The table of a call whose tiles are every `granularity` columns, or (2-D) at most that many tiles, found on
+// the device.
 struct CallTable {
     std::vector<PruneLayer> layers;
     int64_t n_norms = 0, n_items = 0, n_fill = 0, n_tcol = 0, n_cols = 0; // sums over the layers (upper bounds)
