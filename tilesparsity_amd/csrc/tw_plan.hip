@@ -569,14 +569,18 @@ public:
         }
         free_now(p);
     }
-    // what is kept goes back to the device (hipFree waits for work still queued on a destroyed plan)
+    // what is kept goes back to the device (hipFree waits for work still queued on a destroyed plan: not
+    // under the lock, other threads build and destroy plans meanwhile)
     void drop_all()
     {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (const Piece &p : free_)
+        std::vector<Piece> pieces;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            pieces.swap(free_);
+            held_ = 0;
+        }
+        for (const Piece &p : pieces)
             free_now(p.ptr);
-        free_.clear();
-        held_ = 0;
     }
 
 private:
@@ -656,10 +660,13 @@ public:
     }
     void drop_all()
     {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (const auto &p : free_)
+        std::vector<std::pair<void *, size_t>> pieces;
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            pieces.swap(free_);
+        }
+        for (const auto &p : pieces)
             (void)hipHostFree(p.first);
-        free_.clear();
     }
 
 private:
