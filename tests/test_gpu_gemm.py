@@ -1188,3 +1188,85 @@ def test_kernel_for_few_rows_is_taken_where_it_is_ahead(tw, M, K, N, kept, skinn
              for c in range(0, N, 128)]
     with tw.Plan.create(K, N, "f16", tiles, np.zeros((K, N), np.float32)) as plan:
         assert (plan.choice(M, round_up(M, 64), round_up(M, 64))["shape"] == tw.SHAPE_SKINNY) == skinny
+
+
+@pytest.mark.parametrize("M,K,N,G,k_keep,n_keep,dtype", [
+    (1100, 2203, 1530, 128, 0.25, 1.0, "f16"),    # ragged M, K and N; whole octets of columns
+    (1100, 2203, 1530, 128, 0.25, 0.8, "bf16"),   # element-wise stores
+    (1600, 2136, 1000, 64, 0.3, 1.0, "f16"),      # units of at most 64 columns: a wave each
+    (1300, 3000, 1290, 128, 0.01, 0.9, "f16"),    # groups of 16 kept rows over many chunks: cut
+    (3080, 2400, 520, 128, 0.6, 0.9, "bf16"),     # a last group of units that is not full
+    (4096, 1024, 1024, 128, 0.25, 1.0, "f16"),    # where a panel of A would fit
+])
+def test_row_major_streaming(tw, oracle, M, K, N, G, k_keep, n_keep, dtype):
+    """Row-major A and C through the row-major streaming kernel (its workgroups fill three eighths of the chip): alpha, bias
+    and ReLU, pruned columns left alone, then beta and pruned columns filled; tiles without kept rows; padding and
+    the workspace untouched (nothing is staged).  Sampled rows against the oracle."""
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    tiles = random_tiles(rng, K, N, G, k_keep=k_keep, n_keep=n_keep, empty_every=5)
+    keep = kept_columns(tiles, N)
+    lda, ldc = round_up(K, 8) + 8, round_up(N, 8) + 8
+    Ah, Ch = np.full((M, lda), 0x7e00 if dtype == "f16" else 0x7fc0, np.uint16), np.full((M, ldc), SENTINEL, np.uint16)
+    Ah[:, :K] = oracle.cast_bits(A, dtype).reshape(M, K)       # NaN in the padding of the rows of A
+    Ch[:, :N] = oracle.cast_bits(C0, dtype).reshape(M, N)
+    dA, d_bias = to_device_bits(Ah, Ah.shape), torch.from_numpy(bias).cuda()
+    rows = np.unique(np.concatenate([np.arange(5), np.arange(M - 70, M), rng.choice(M, 40)]))
+    with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+        nbytes = max(plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR), 16)
+        ws = torch.full((nbytes // 2,), 0x7bcd, dtype=torch.int16, device="cuda")
+        for alpha, beta, pruned in ((0.75, 0.0, tw.PRUNED_UNTOUCHED), (1.0, 0.5, tw.PRUNED_ZERO)):
+            if beta and K < 2128:
+                continue                                       # (a panel does not read C: staged there)
+            dC = to_device_bits(Ch, Ch.shape)
+            plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=alpha, beta=beta, a_layout=tw.ROWMAJOR,
+                      c_layout=tw.ROWMAJOR, pruned_cols=pruned, bias_ptr=d_bias.data_ptr(), activation=tw.ACT_RELU,
+                      workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes)
+            torch.cuda.synchronize()
+            assert torch.all(ws == 0x7bcd)
+            out = from_device_bits(dC)
+            assert np.all(out[:, N:] == SENTINEL)
+            pre = alpha * reference(oracle, A[rows], B, tiles, dtype)
+            want = np.maximum(pre + beta * oracle.quantize(C0[rows], dtype) + bias, 0.0)
+            got = oracle.bits_to_f32(np.ascontiguousarray(out[rows, :N]), dtype).reshape(rows.size, N)
+            assert oracle.rel_error(got[:, keep], want[:, keep]) <= TOL[dtype]
+            if pruned == tw.PRUNED_UNTOUCHED:
+                assert np.array_equal(out[:, :N][:, ~keep], Ch[:, :N][:, ~keep])
+            elif not np.all(keep):
+                assert oracle.rel_error(got[:, ~keep], want[:, ~keep]) <= TOL[dtype]
+
+
+def test_row_major_streaming_nonfinite(tw, oracle):
+    """Inf and NaN in columns of A that a tile prunes do not reach it, and an infinite weight in a group of kept rows that
+    is cut gives what it gives uncut: the row-major streaming kernel and the K-major one agree on where the result is finite."""
+    import torch
+    rng = np.random.default_rng(5)
+    M, K, N, G = 1100, 2500, 1536, 128
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    tiles = random_tiles(rng, K, N, G, k_keep=0.02, n_keep=1.0)
+    free = np.setdiff1d(np.arange(K), np.concatenate([t["kept_k"] for t in tiles[:6]]))
+    A[:, free[::3]], A[:, free[1::3]] = np.inf, np.nan         # (kept by other tiles: those become non-finite)
+    A[A == 0] = 1.0
+    for t in tiles[:3]:
+        B[t["kept_k"][7], t["col0"] + 11] = 1e9                # infinite in f16
+    Ak = np.zeros((K, round_up(M, 8)), np.uint16)
+    Ab = oracle.cast_bits(A, "f16").reshape(M, K)
+    Ak[:, :M] = Ab.T
+    Ar = np.zeros((M, round_up(K, 8)), np.uint16)
+    Ar[:, :K] = Ab
+    dAk, dAr = to_device_bits(Ak, Ak.shape), to_device_bits(Ar, Ar.shape)
+    dCk, dCr = (torch.zeros(s, dtype=torch.int16, device="cuda") for s in ((N, Ak.shape[1]), (M, N)))
+    with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+        plan.gemm(dAr.data_ptr(), dCr.data_ptr(), M, lda=Ar.shape[1], ldc=N, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+        plan.gemm(dAk.data_ptr(), dCk.data_ptr(), M, lda=Ak.shape[1], ldc=Ak.shape[1])
+        torch.cuda.synchronize()
+    r, k = dCr.view(torch.float16), dCk.view(torch.float16)[:, :M].T
+    assert torch.equal(torch.isnan(r), torch.isnan(k)) and torch.equal(torch.isinf(r), torch.isinf(k))
+    assert bool(torch.isfinite(r[:, :6 * G]).any()) and bool(torch.isinf(r[:, 11]).all())
+    fin = torch.isfinite(r)
+    assert float((r[fin].float() - k[fin].float()).abs().max()) <= 2e-3 * float(k[fin].float().abs().max())

@@ -2718,6 +2718,29 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
     return choose_shape(plan, M, ld, ld, beta != 0.0f).shape == TW_SHAPE_SKINNY;
 }
 
+// The row-major streaming kernel for row-major operands.  Measured (us a launch of a replayed graph, before and with it)
+// on M 256 .. 16384, K 768 .. 4608, N 256 .. 3072, 10 / 25 / 50 % of the rows kept, tiles of 64 and 128 columns.  Its time
+// is that of a round of workgroups (64 rows x 256 columns: 13 - 25 us by K and kept rows) times rounds:
+// Against the skinny kernel and the copies around the streaming kernels (no panel of A in LDS), from 96 workgroups on
+// (K 3072, N 768, M 2048, a quarter kept: 22 -> 15; M 4096: 33 -> 17; K 4608, N 512, M 12544: 82 -> 46; 64 workgroups,
+// K 4608, N 512, M 2048: 18 -> 20), 128 where tiles of 64 columns keep more than 1024 rows (K 4096, N 1024, half kept,
+// 96 workgroups: 1.06 of the time); not for many columns under many rows, where turning A once is cheaper than
+// streaming all of it for every 256 columns (K 2560, N 2560, M 16384: 141 -> 165; M 4096, 640 workgroups: 49 -> 41).
+// Against the panel, where one round fills the chip (K 2048, N 1024, M 4096: 20 -> 16; K 1024, N 1024, M 4096: 14 -> 12;
+// 128 workgroups: 1.05 of the time; two rounds, M 8192: 1.0 - 1.14) and the tiles are no shorter than a fifth of K (a tenth
+// kept: 0.92 - 1.3 of the time).
+bool streams_row_major(const tw_plan *plan, int M, int64_t lda, float beta)
+{
+    if (option(TW_OPT_SHAPE) != -1 || !rm_takes(plan, lda)) // (a forced shape keeps the paths around the K-major kernels)
+        return false;
+    const int64_t groups = rm_groups(plan), wgs = (((int64_t)M + kRmRowsPerWg - 1) / kRmRowsPerWg) * groups;
+    if (takes_row_major_directly(plan, beta))
+        return plan->K >= 1024 && wgs * 8 >= (int64_t)plan->cu_count * 5 && wgs <= plan->cu_count &&
+               plan->pipe_steps * kBlockK * 5 >= (int64_t)plan->K * std::max(1, plan->n_pipe_units);
+    const bool long_narrow = plan->max_unit_n <= 64 && plan->pipe_steps * kBlockK > (int64_t)1024 * std::max(1, plan->n_pipe_units);
+    return wgs * 8 >= (int64_t)plan->cu_count * (long_narrow ? 4 : 3) && (groups <= 6 || wgs <= 4 * (int64_t)plan->cu_count);
+}
+
 template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, const GemmArgs &a, int M, hipStream_t s)
 {
     const int pst = prepare_device();
@@ -2796,6 +2819,9 @@ int prepare_device()
     };
     for (const void *k : as_kernels)
         TW_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
+    const int rst = prepare_rm();
+    if (rst != TW_OK)
+        return rst;
     void *p = nullptr;
     TW_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
     g_scratch_ptr[dev] = static_cast<int32_t *>(p);
@@ -3041,7 +3067,9 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return st;
     GemmArgs a;
     fill_common(a, plan, A, lda, C, ldc, M, alpha, beta, ep);
-    if (a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR && skinny_takes_row_major(plan, M, beta)) {
+    const bool row_major = a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR;
+    const bool streams = row_major && streams_row_major(plan, M, lda, beta);
+    if (row_major && !streams && skinny_takes_row_major(plan, M, beta)) {
         fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false);
         if (a.n_all_u == 0)
             return TW_OK;
@@ -3051,7 +3079,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         hipStream_t s = (hipStream_t)stream;
         return plan->dtype == TW_F16 ? launch_skinny<TW_F16, true>(plan, a, s) : launch_skinny<TW_BF16, true>(plan, a, s);
     }
-    if (a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR && takes_row_major_directly(plan, beta)) {
+    if (row_major && !streams && takes_row_major_directly(plan, beta)) {
         // both operands row-major, K short enough for a panel of A in LDS, C not read: the
         // A-stationary kernel in its row-major form (64-row panels where they fit and still give
         // three quarters of the compute units a workgroup)
@@ -3068,6 +3096,17 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         if (plan->dtype == TW_F16)
             return b64 ? launch_as<TW_F16, 64, true>(plan, a, M, s) : launch_as<TW_F16, 32, true>(plan, a, M, s);
         return b64 ? launch_as<TW_BF16, 64, true>(plan, a, M, s) : launch_as<TW_BF16, 32, true>(plan, a, M, s);
+    }
+    if (streams || (row_major && option(TW_OPT_SHAPE) == -1 && rm_takes(plan, lda))) {
+        // (off the rule's range too: the layout-generic kernel is several times slower everywhere)
+        fill_queues(a, plan, M, kRmRowsPerWg, 128, pruned_cols, false);
+        if (a.n_all_u == 0)
+            return TW_OK;
+        a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
+        for (int i = 0; i < a.n_arg_units; ++i)
+            a.arg_units[i] = plan->h_units[i];
+        const int pst = prepare_device();
+        return pst != TW_OK ? pst : launch_rm(plan, a, (hipStream_t)stream);
     }
     if (a_layout != TW_LAYOUT_KMAJOR || c_layout != TW_LAYOUT_KMAJOR) {
         // layout-generic path (element strides), 128-row blocks, one workgroup per item

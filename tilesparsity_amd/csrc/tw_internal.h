@@ -191,5 +191,14 @@ bool skinny_takes_row_major(const tw_plan *p, int M, float beta);
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
 int launch_bs(const tw_plan *p, const GemmArgs &a, int per_cu, hipStream_t s);
 double bs_fill(const tw_plan *p, int M); // share of the chip's workgroup slots its launch fills
+// the row-major streaming kernel (tw_gemm_rm.hip): whether it can take the plan, its workgroups per block of rows of A,
+// its launch, its set-up per device
+constexpr int kRmRowsPerWg = 64;
+int rm_groups(const tw_plan *p);
+bool rm_takes(const tw_plan *p, int64_t lda);
+int launch_rm(const tw_plan *p, const GemmArgs &a, hipStream_t s);
+int prepare_rm();
+// true where tw_gemm_ex takes a row-major A and a row-major C of this plan with it
+bool streams_row_major(const tw_plan *p, int M, int64_t lda, float beta);
 
 } // namespace tw
