@@ -152,8 +152,7 @@ def lib():
         "tw_prune_granularity": (c_int, [c_int, c_int, vp, ctypes.c_double, c_int, c_int, vp, vp]),
         "tw_percentile_linear": (c_int, [vp, c_i64, ctypes.c_double, c_int,
                                          ctypes.POINTER(ctypes.c_double), vp]),
-        "tw_tiles_every_g_kept_columns": (c_int, [c_int, c_int, u8p, i32p, i32p,
-                                                  ctypes.POINTER(c_int)]),
+        "tw_tiles_every_g_kept_columns": (c_int, [c_int, c_int, vp, vp, vp, ctypes.POINTER(c_int)]),
         "tw_prune_mix": (c_int, [c_int, i32p, i32p, pp, pp, ctypes.c_double, c_int, pp,
                                  ctypes.POINTER(ctypes.c_double), vp]),
         "tw_lstm_gates": (c_int, [c_int, c_int, c_int, vp, c_i64, c_f, vp, c_i64, vp, c_i64, vp, c_i64, vp]),
