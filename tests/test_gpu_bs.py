@@ -119,3 +119,77 @@ def test_weight_stationary_kernel_declines(tw, oracle):
     finally:
         tw.set_option(tw.OPT_SHAPE, -1)
     assert np.array_equal(out[0], out[1])
+
+
+# M, K, G, (kept rows, kept columns) per tile: the wider form where the launch takes it by itself, one to six steps, units of one
+# to four blocks of columns, tiles without a kept row, ranges of two blocks of 64 rows and of many, M off every grain; the last
+# one's output is stored in lines
+WIDE_CASES = [
+    (4101, 1100, 128, ((256, 128), (200, 100), (0, 128), (255, 65), (193, 7), (220, 33))),
+    (1031, 1200, 128, ((384, 128), (257, 97), (321, 32), (0, 5), (380, 128)) * 5),
+    (97, 600, 128, tuple((300 + t % 64, 128 if t % 3 else 64) for t in range(256))),
+    (2600, 1100, 128, tuple((230 + 13 * (t % 12), 128 - t) for t in range(40))),
+    (6001, 130, 128, tuple((60 + t % 68, 128 - t % 31) for t in range(64))),
+]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("case", range(len(WIDE_CASES)))
+def test_weight_stationary_wide_form(tw, oracle, dtype, case):
+    """Bit for bit the streaming 256 x 128 kernel (both add a tile's kept rows up in the order of its list, in fp32), with every
+    activation and either treatment of the pruned columns, the padding of C's rows untouched.  GELU and tanh: the kernels build
+    them from the same sum in a different order of instructions, so one unit in the last place of the result (2^-10, 2^-7)."""
+    import torch
+    M, K, G, spec = WIDE_CASES[case]
+    N = G * len(spec)
+    rng = np.random.default_rng(1300 + case)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    dbias = torch.from_numpy(rng.standard_normal(N).astype(np.float32)).cuda()
+    tiles = make_tiles(rng, K, G, spec)
+    used = np.unique(np.concatenate([t["kept_k"] for t in tiles]))
+    lda = ldc = (M + 7) // 8 * 8 + 8
+    At = np.zeros((K, lda), np.uint16)
+    At[:, :M] = oracle.cast_bits(A, dtype).reshape(M, K).T
+    At[np.setdiff1d(np.arange(K), used)] = 0x7fff       # NaN in the rows that no tile keeps: they reach no product
+    dA = to_device_bits(At, At.shape)
+    s = torch.cuda.current_stream().cuda_stream
+    tdt = torch.float16 if dtype == "f16" else torch.bfloat16
+    ulp = 2.0 ** -10 if dtype == "f16" else 2.0 ** -7
+
+    def launch(plan, shape, alpha, pruned, with_bias, act):
+        dC = torch.full((N, ldc), SENTINEL, dtype=torch.int16, device="cuda")
+        tw.set_option(tw.OPT_SHAPE, shape)
+        print("wide form: case", case, "shape", shape, alpha, pruned, with_bias, act, dtype, flush=True)
+        assert plan.choice(M, lda=lda, ldc=ldc)["shape"] == (tw.SHAPE_BS if shape == -1 else shape)
+        plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=alpha, pruned_cols=pruned,
+                  bias_ptr=dbias.data_ptr() if with_bias else None, activation=act, stream=s)
+        torch.cuda.synchronize()
+        return dC
+
+    try:
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            for (alpha, pruned, with_bias, act) in ((1.0, tw.PRUNED_UNTOUCHED, False, tw.ACT_NONE),
+                                                    (0.5, tw.PRUNED_ZERO, True, tw.ACT_RELU),
+                                                    (1.0, tw.PRUNED_ZERO, True, tw.ACT_GELU),
+                                                    (1.0, tw.PRUNED_UNTOUCHED, True, tw.ACT_TANH)):
+                want = launch(plan, tw.SHAPE_256x128, alpha, pruned, with_bias, act)
+                got = launch(plan, -1, alpha, pruned, with_bias, act)
+                if act in (tw.ACT_GELU, tw.ACT_TANH):
+                    a, b = got[:, :M].view(tdt).float(), want[:, :M].view(tdt).float()
+                    assert bool(((a - b).abs() <= ulp * b.abs() + 1e-7).all())
+                    assert torch.equal(got[:, M:], want[:, M:])
+                else:
+                    assert torch.equal(got, want), (alpha, pruned, with_bias, act)
+                assert torch.equal(got, launch(plan, -1, alpha, pruned, with_bias, act))
+            if case == 2:   # (the smallest)
+                out = from_device_bits(launch(plan, -1, 1.0, tw.PRUNED_ZERO, False, tw.ACT_NONE))
+                keep = np.zeros(N, bool)
+                for t in tiles:
+                    keep[t["col0"] + t["kept_n"]] = True
+                ref = oracle.stream_gemm_nn(oracle.quantize(A, dtype), oracle.quantize(B, dtype), tiles, 1.0)
+                Cf = oracle.bits_to_f32(out[:, :M], dtype).reshape(N, M).T
+                assert oracle.rel_error(Cf[:, keep], ref[:, keep]) <= TOL[dtype]
+                assert not Cf[:, ~keep].any()
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)

@@ -2533,7 +2533,7 @@ struct Choice {
 // workgroups of a die then share the rows of A in their L2 (measured on the 0 %-sparse plan of
 // the headline shape: a third of the reads from memory), but no benchmark shape ran faster for
 // it and the stress shape, whose 512-row block of A fills an L2, ran 13 % slower.
-static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc, bool reads_c)
+static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc, bool reads_c, bool row_major = false)
 {
     Choice c;
     const int width = std::max(32, round_up32(plan->max_unit_n)); // 32, 64, 96 or 128
@@ -2590,17 +2590,31 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
         skinny = sk_w < 3.0 || (sk_w <= 4.0 && sk_cost <= 70.0) || (sk_w <= 5.0 && sk_cost <= (items(256, 128) * 4 <= cu ? 65.0 : 25.0)) ||
                  (few && sk_w <= 6.0);
     skinny = skinny && skinny_ok;
-    // The weight-stationary kernel where a tile keeps at most 192 rows under many rows of A, tiles
-    // wider than 64 columns.  Measured on M 512 .. 16384, K 768 / 1024 / 4096, N 1024 / 4096 with
-    // 64 .. 192 kept rows a tile against the choice below: from 2048 rows of A on it takes 0.58 -
-    // 1.05 of the time (median 0.79 - 0.86; most where K is too long for a panel of A in LDS),
-    // below that, and on tiles of 64 columns, it is as often slower as faster.
-    // Its workgroups (unit x range of rows) have to fill the chip's slots evenly: BERT-base's 24
-    // units give 384 workgroups for 512 slots, and the kernel is then 1 us slower than the
-    // A-stationary one (15 against 14), where 32 units (BERT-large FFN1 at 90 %) gain 12 %.
-    // With K = 512 the panel of A is small and the A-stationary kernel stays ahead (M 16384, N 4096:
-    // 43 against 49 - 54 us), so the kernel is taken from K = 1024 on.
-    const bool bs = bs_takes(plan, lda, ldc, reads_c) && width > 64 && M >= 2048 && plan->K >= 1024 && bs_fill(plan, M) >= 0.9;
+    // The weight-stationary kernels: tiles of at most 384 kept rows, wider than 64 columns, under units * rows of A above 24576
+    // (96 rows to a workgroup with one on every compute unit).  Against the choice without the wider of them, us of a replayed
+    // graph before and after, on M 256 .. 16384, K 512 .. 4096, N 512 .. 8192, 60 .. 380 kept rows, all alike or within 40 % of
+    // each other, without activation, with ReLU and GELU: 0.88 of the time over 1700 problems from there on (BERT-large FFN1 at
+    // 75 % 34.1 -> 26.2, with GELU 39.5 -> 32.5; M 4096, K 3072, N 3072, 60 kept 16.2 -> 10.9; M 512, N 8192 0.83, M 1024, N 4096
+    // 0.90; below the line M 2048, N 1024 1.0 - 1.08, M 1024, N 2048 1.07).  A unit multiplies as many steps as the longest has,
+    // so beyond three steps the tiles have to be of about a length (within 40 %: 0.85 - 0.93 at 250 kept, K from 1024 on).  Their
+    // workgroups (unit x range of rows, one to a compute unit) have to give three quarters of the chip work (5 .. 130 units:
+    // 0.77 - 0.89 of the time from there on; 17 and 130 units, half the chip: to 1.2 and 1.34); where no panel fits LDS two
+    // thirds (0.81 - 0.86), and up to three steps any share (0.71 - 0.76).
+    // Not where a 64-row panel of A fits LDS and
+    // - there are few units and K is short (M 8192, K 768, N 512: 0.98 - 1.07), or
+    // - the tiles are long and K is 512 (190 kept within 40 %: 1.02 in the mean, to 1.10) or the workgroups leave more than a
+    //   tenth of the chip without one (24 units, 300 kept, M 2048: 1.10 - 1.15), or
+    // - the launch is little but its stores (K 512, N 8192, M 16384, 60 kept within 40 %: 73 -> 102; 120: 83.5 -> 93; 60 kept,
+    //   M 8192, N 5632: 27.8 -> 32.5).
+    const bool panel64 = as_ok(TW_SHAPE_AS64);
+    const double chip = bs_fill(plan, M);
+    const int64_t out_mb = (int64_t)M * plan->N * 2 >> 20;
+    const bool bs = !row_major && bs_takes(plan, lda, ldc, reads_c) && width > 64 && (int64_t)plan->n_units * M > 24576 &&
+                    (plan->max_k_pad <= 192 || plan->pipe_steps * kBlockK * 10 >= 6 * units * plan->max_k_pad) &&
+                    (chip >= 0.75 || (!panel64 && (plan->max_k_pad <= 192 || chip >= 0.65))) &&
+                    !(panel64 && ((plan->K < 1024 && plan->n_units < 8) || (plan->max_k_pad > 256 && plan->K <= 512) ||
+                                  (plan->max_k_pad > 256 && M < 16384 && chip < 0.9) ||
+                                  (plan->K < 1024 && out_mb > (plan->max_k_pad <= 64 ? 32 : plan->max_k_pad <= 128 ? 200 : INT64_MAX))));
     // Tiles of six steps and more on average, wide, with 256-row items for three quarters of the
     // chip: the streaming 256 x 128 kernel, whose loads write LDS directly, is ahead of the panel
     // (M 8192, K 1024, N 2048, half the rows kept: 28.4 against 33.2 us; BERT-large FFN1 at 50 %
@@ -2612,10 +2626,10 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
     const int64_t it256 = items(256, 128);
     const bool long_tiles = ws_ok && width > 64 && plan->pipe_steps >= 6 * units && it256 * 4 >= 3 * cu &&
                             it256 * 10 >= (it256 + cu - 1) / cu * cu * 9;
-    if (skinny) {
-        c.shape = TW_SHAPE_SKINNY;
-    } else if (bs) {
+    if (bs) {
         c.shape = TW_SHAPE_BS;
+    } else if (skinny) {
+        c.shape = TW_SHAPE_SKINNY;
     } else if (!ws_ok) {
         c.shape = TW_SHAPE_WIDE;
     } else if (as_ok(TW_SHAPE_AS64) && (M > 128 || plan->n_blocks >= 96) &&
@@ -2677,7 +2691,8 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
         if (skinny_ok)
             c.shape = f_shape;
     } else if (f_shape == TW_SHAPE_BS) {
-        if (bs_takes(plan, lda, ldc, reads_c))
+        // (forced, up to 192 kept rows as ever; longer tiles are the rule's to give)
+        if (plan->max_k_pad <= 192 && bs_takes(plan, lda, ldc, reads_c))
             c.shape = f_shape;
     } else if (f_shape >= 0 && (f_shape != TW_SHAPE_WIDE ? ws_ok : true)) {
         const int piece = f_piece > 0 ? f_piece : std::min(128, kShapes[f_shape].bn);
@@ -2715,7 +2730,7 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
         (plan->K <= 512 || plan->n_units <= 0 || skinny_work(plan, M, &w) < 0 || skinny_load(plan, w) > 2.0))
         return false;
     const int64_t ld = ((int64_t)M + 63) / 64 * 64;
-    return choose_shape(plan, M, ld, ld, beta != 0.0f).shape == TW_SHAPE_SKINNY;
+    return choose_shape(plan, M, ld, ld, beta != 0.0f, true).shape == TW_SHAPE_SKINNY;
 }
 
 // The row-major streaming kernel for row-major operands.  Measured (us a launch of a replayed graph, before and with it)

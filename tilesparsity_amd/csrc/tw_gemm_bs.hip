@@ -1,5 +1,5 @@
 // Weight-stationary kernel of the tile-wise-sparse GEMM (TW_SHAPE_BS), for tiles that keep few
-// rows (at most 192) under many rows of A: BERT-like layers at 75 % sparsity and more.
+// rows (at most 192; 384 in its wider form below) under many rows of A: BERT-like layers at 75 % sparsity and more.
 //
 // A workgroup takes one unit (up to 128 compact columns of a tile) and a range of rows of A.  Its
 // four multiplying waves own one block of 32 compact columns each and keep that block's packed
@@ -37,6 +37,7 @@
 #include "tw_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace tw {
 
@@ -318,6 +319,322 @@ __global__ void __launch_bounds__(64 * kBsWaves, 4)
     }
 }
 
+// ---------------------------------------------------------------------------------
+// The same with eight multiplying waves, for tiles of up to 384 kept rows (instantiations of two, three, four and six steps).
+// What bounds it is C on its way out (M 8192, N 4096: 64 MB, 14 us at 4.5 TB/s, what such stores alone reach) beside the
+// gathered reads of A, and how well a block's epilogue hides beneath the next one's products.  A wave that holds 32 columns of
+// four steps and multiplies 64 rows at a time has room for nobody beside it, so here eight waves multiply 32 rows x 32 columns
+// each (the two of a block of columns hold its weight twice), two to four load, and one workgroup has the compute unit (168
+// registers a wave).  Two waves a SIMD are too few to fill each other's waits, so a wave's own work is laid out to overlap:
+// the vector instructions of a block's epilogue (GELU: 250 of them) stand between the products of the next block, which need
+// the matrix pipe for 32 cycles each, and the reads of a product's rows three products ahead.  For that a block is one piece
+// of straight code: all of its steps have landed when it begins (words in LDS instead of a barrier per step: a loading wave
+// says which of its steps are there, a multiplying wave how many it has read), tiles with fewer steps multiply zeros in the
+// missing ones, and the activation is a template argument.  The multiplying waves' memory queue holds stores only and nothing
+// in the loop waits for it.
+// A wave's 32 rows are 64 bytes of a column.  Stored a further block later through the stage that the two waves of a block of
+// columns share, they go out as whole 128-byte lines (`lines`): ahead where C leaves the last-level cache (134 MB 61 -> 47.6
+// us), level below (64 MB: 26.2 without, 26.8 with), crossing at 90 - 96 MB.
+// Measured (bf16, us of a replayed graph, the panel kernel or the four-wave one -> this): M 8192, K 1024, N 4096, 256 kept rows
+// 34.2 -> 26.2, with GELU 39.7 -> 32.5; M 12288 61.3 -> 37.0, with GELU 69.5 -> 43.5; M 4096, K 768, N 3072, 192 kept 15.1 ->
+// 13.0, with GELU 16.9 -> 16.1.  Bit for bit what those give.
+constexpr int kBwMulWaves = 8;
+constexpr int bw_load_waves(int ns) { return ns <= 4 ? ns : 3; } // (three and four waves a SIMD have 168 and 128 registers)
+constexpr int bw_threads(int ns) { return 64 * (kBwMulWaves + bw_load_waves(ns)); }
+constexpr int kBwRing = 14;                          // stages of 8 KiB
+constexpr int kBwCPitch = kBsRows + 4;               // elements per column of a C stage
+constexpr int kBwCStage = 32 * kBwCPitch * 2;        // bytes; two of them for the two waves of a block of columns
+constexpr int64_t kBwLineBytes = 90 << 20;           // outputs from here on are stored in whole lines
+constexpr uint64_t kBwMaxBytes = 0xFFFF0000u;        // of C, which is stored through a buffer descriptor
+constexpr int kBwSteps = 6;                          // most steps of an instantiation
+
+template <int DT, int ACT, int NS>
+__global__ void __launch_bounds__(bw_threads(NS), 3)
+    tw_gemm_bw_kernel(const GemmArgs p, int n_units, int n_ranges, int row_units, int affine, uint32_t a_bytes,
+                      uint32_t c_bytes, int lines)
+{
+    using E = Elem<DT>;
+    constexpr int LW = bw_load_waves(NS), SPW = NS / LW; // loading waves, steps of a block each
+    static_assert(LW * SPW == NS, "whole steps a wave");
+    __shared__ __align__(1024) unsigned char ring[kBwRing * kBsStage];
+    __shared__ __align__(16) unsigned char cstage[kBwMulWaves * kBwCStage];
+    __shared__ uint32_t row_off[NS * kBlockK]; // byte offset of each kept row in A, beyond the buffer for the list's padding
+    __shared__ int flags[16];                  // first step that is not there of each loading wave's, steps each multiplying wave has read
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int ui, r;
+    if (affine) {
+        const int die = blockIdx.x % kXcd, i = blockIdx.x / kXcd;
+        ui = i % n_units;
+        r = die + kXcd * (i / n_units);
+    } else {
+        r = blockIdx.x % n_ranges;
+        ui = blockIdx.x / n_ranges;
+    }
+    if (r >= n_ranges)
+        return;
+    const int m_lo = (int)((int64_t)r * row_units / n_ranges) * 32;
+    const int m_hi = min((int)((int64_t)(r + 1) * row_units / n_ranges) * 32, p.M);
+    if (m_lo >= m_hi)
+        return;
+    const UnitDev u = load_unit(p, ui);
+    const int nsteps = u.k_pad / kBlockK; // <= NS (host check)
+    const int n_mb = (m_hi - m_lo + kBsRows - 1) / kBsRows;
+    TW_LDS(volatile int) const landed = (TW_LDS(volatile int))flags;
+    TW_LDS(volatile int) const done = landed + 4;
+    if (tid < 4 + kBwMulWaves)
+        flags[tid] = tid < LW ? 0 : tid < 4 ? 0x7fffffff : 0;
+    uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
+
+    if (wave >= kBwMulWaves) {
+        // ================= loading waves: the same SPW steps of every block each =============
+        const int w = wave - kBwMulWaves;
+        const uint32_t lda_b = (uint32_t)p.lda * 2u;
+#pragma unroll
+        for (int q = 0; q < SPW; ++q) {
+            const int i = (w * SPW + q) * kBlockK + lane;
+            row_off[i] = i < u.k_kept ? (uint32_t)p.kept_k[u.kk_off + i] * lda_b : 0xFFFFFF00u;
+        }
+        TW_LDS_BARRIER(); // the row offsets, and the flags
+        const __amdgpu_buffer_rsrc_t a_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p.A), 0, (int)a_bytes, kBsRsrcFlags);
+        const int rr = lane >> 3, pos = lane & 7;
+        // load j of a step covers its kept rows 8 j .. 8 j + 7, lane l 16 bytes of row 8 j + l / 8; halves swapped as above
+        uint32_t off[SPW][8];
+#pragma unroll
+        for (int q = 0; q < SPW; ++q)
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                off[q][j] = row_off[(w * SPW + q) * kBlockK + j * 8 + rr] + (uint32_t)(pos ^ ((rr >> 1 & 1) << 2)) * 16u;
+        TW_LDS(unsigned char) const lds0 = (TW_LDS(unsigned char))ring;
+        // two blocks in flight: what a block takes to arrive is more than what it takes to multiply
+        auto issue = [&](int mb) {
+            const int m0b = (m_lo + mb * kBsRows) * 2;
+#pragma unroll
+            for (int q = 0; q < SPW; ++q) {
+                const int g = mb * NS + w * SPW + q;
+                if (g >= kBwRing)
+                    while (!__all(done[lane & 7] > g - kBwRing))
+                        __builtin_amdgcn_s_sleep(1);
+                TW_LDS(unsigned char) const dst = lds0 + g % kBwRing * kBsStage;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, (TW_LDS(void))(dst + j * 1024), 16, (int)off[q][j], m0b, 0, 0);
+            }
+        };
+        issue(0);
+        for (int mb = 0; mb < n_mb; ++mb) {
+            if (NS <= kBwRing / 3 && mb + 1 < n_mb) { // (a block ahead of the one waited for, where three fit the ring)
+                issue(mb + 1);
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(8 * SPW) : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
+            if (lane == 0)
+                landed[w] = (mb + 1) * NS;
+            if (NS > kBwRing / 3 && mb + 1 < n_mb)
+                issue(mb + 1);
+        }
+        return;
+    }
+
+    // ================= multiplying waves ====================================================
+    const int cb = wave & 3, mi = wave >> 2;
+    const bool active = cb < u.nb_cnt;
+    const int nb = active ? cb : 0;
+    const int cnt = min(32, u.n_cnt - nb * 32);
+    const int L = lane & 15, j = lane & 31;
+    TW_LDS_BARRIER(); // the row offsets, and the flags (before anything is fetched here: the loading waves stand behind it)
+    const int out_n = p.kept_n[u.kn_off + nb * 32 + (j < cnt ? j : 0)];
+    u32x4 bq[NS][4];
+    {
+        const unsigned char *const bsrc = reinterpret_cast<const unsigned char *>(p.Bp) +
+                                          (nsteps ? u.b_off * 2 + (int64_t)(u.nb0 + nb) * 4096 : 0) + lane * 16;
+        const int64_t step_b = (int64_t)u.nblk * 4096;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+#pragma unroll
+            for (int k16 = 0; k16 < 4; ++k16) {
+                bq[s][k16] = *reinterpret_cast<const u32x4 *>(bsrc + (s < nsteps ? s : 0) * step_b + k16 * 1024);
+                if (s >= nsteps) // (zeros times zeros: the loading waves' rows there are beyond the buffer)
+                    bq[s][k16] = u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+    }
+    int out_col = u.col0 + out_n;
+    float out_bias = p.bias ? p.bias[out_col] : 0.0f;
+    const uint32_t swap = (uint32_t)((L >> 3) & 1);
+    const uint32_t lane_a = (uint32_t)((lane >> 5) * 8 + (L >> 2)) * 128u + (uint32_t)(((lane >> 4) & 1) * 32 + (L & 3) * 8) +
+                            (mi ? 1u - swap : swap) * 64u;
+    TW_LDS(unsigned char) const lds0 = (TW_LDS(unsigned char))ring + lane_a;
+    TW_LDS(unsigned char) const cst = (TW_LDS(unsigned char))cstage + cb * 2 * kBwCStage;
+    int slot = 0;
+    f32x16 acc{};
+    // Both waves of a block of columns put their 32 rows of a product into one stage.  With `lines` each takes 16 of its columns
+    // out, 64 rows, whole 128-byte lines of C, for which it waits until the other is as far; else each takes its own 32 rows out
+    // again, 64 bytes a column.  This lane's two 16-byte pieces:
+    const int jq[2] = {lines ? mi * 16 + (lane >> 3) : lane >> 2, lines ? mi * 16 + (lane >> 3) + 8 : (lane >> 2) + 16};
+    const int row_q = lines ? (lane & 7) * 8 : mi * 32 + (lane & 3) * 8;
+    uint32_t o_q[2]; // byte offset of the column, and of the row inside a block (set once the column numbers are there)
+    // a block's epilogue goes to stage `parity`
+    auto stage_put = [&](int parity, int r4, const float (&e)[4]) {
+        *(TW_LDS(u32x2))(cst + parity * kBwCStage + (j * kBwCPitch + mi * 32 + (lane >> 5) * 4 + r4 * 8) * 2) =
+            u32x2{E::to_bits2(e[0], e[1]), E::to_bits2(e[2], e[3])};
+    };
+    auto stage_get = [&](int parity, int q) {
+        const u32x2 lo = *(TW_LDS(const u32x2))(cst + parity * kBwCStage + (jq[q] * kBwCPitch + row_q) * 2);
+        const u32x2 hi = *(TW_LDS(const u32x2))(cst + parity * kBwCStage + (jq[q] * kBwCPitch + row_q + 4) * 2);
+        return u32x4{lo.x, lo.y, hi.x, hi.y};
+    };
+    // the pieces of block mb, out of the stage, to C
+    auto put = [&](int mb, const u32x4 (&v)[2]) {
+        const int m0 = m_lo + mb * kBsRows;
+        const int m_end = min(m0 + kBsRows, m_hi);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            if (jq[q] < cnt)
+                store_chunk(reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(C) + o_q[q]) + m0, v[q], m0 + row_q, m_end,
+                            p.store_through != 0);
+    };
+    // The products of block mb, whose steps have landed.  Between them (`older` blocks before it: 0, 1, or 2 and more) the
+    // epilogue of the block before (`prev`) goes to one stage, and the block before that from the other one to C: whole
+    // blocks, through a buffer descriptor that drops the columns the unit does not have, and through to memory (as
+    // store_chunk).  `land` is what the flags said in the middle of the block.
+    const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(C + m_lo, 0, (int)c_bytes, kBsRsrcFlags);
+    const bool other = lines && (lane & 4); // what this lane watches: the other wave, or the loads
+    TW_LDS(volatile int) const flag = other ? done + (wave ^ 4) : landed + (lane & 3);
+    const int flag_add = other ? NS : 0;
+    int land = 0;
+    auto block = [&](const f32x16 &prev, int mb, auto older_tag) {
+        constexpr int OLDER = decltype(older_tag)::value;
+        const int parity = (mb - 1) & 1;
+        u32x4 out[2];
+        f32x16 sum;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            sum[e] = 0.0f;
+        u32x4 af[NS * 4];
+        auto fetch = [&](int i) {
+            const int sl = slot + (i >> 2);
+            TW_LDS(unsigned char) const st = lds0 + (sl >= kBwRing ? sl - kBwRing : sl) * kBsStage + (i & 3) * 2048;
+            const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(st));
+            const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(st + 512));
+            const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+            af[i] = u32x4{l2.x, l2.y, h2.x, h2.y};
+        };
+        constexpr int AHEAD = NS == 6 ? 2 : 3; // (registers)
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            fetch(i);
+        __builtin_amdgcn_sched_barrier(0);
+        float epi[4];
+#pragma unroll
+        for (int i = 0; i < NS * 4; ++i) {
+            if (i + AHEAD < NS * 4)
+                fetch(i + AHEAD);
+            if (i == NS)
+                land = *flag;
+            if (OLDER > 1 && (i == 2 || i == 3))
+                out[i - 2] = stage_get(parity ^ 1, i - 2);
+            sum = E::mfma(af[i], bq[i >> 2][i & 3], sum);
+            if (OLDER > 1 && (i == NS * 4 - 2 || i == NS * 4 - 1))
+                __builtin_amdgcn_raw_buffer_store_b128(out[i - (NS * 4 - 2)], c_rsrc, (int)o_q[i - (NS * 4 - 2)], (mb - 2) * kBsRows * 2,
+                                                       1 | 2 | 16);
+            if constexpr (OLDER > 0) {
+                // this product's share of the sixteen values of the block before; four of them go to the stage together
+                constexpr int P = NS < 4 ? NS * 4 : 16;
+#pragma unroll
+                for (int e = 16 * i / P; e < 16 * (i + 1) / P && e < 16; ++e) {
+                    epi[e & 3] = tw_fp32_value(tw_activate(p.alpha * prev[e] + out_bias, ACT));
+                    if ((e & 3) == 3)
+                        stage_put(parity, e >> 2, epi);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        slot += NS;
+        slot = slot >= kBwRing ? slot - kBwRing : slot;
+        return sum;
+    };
+    // All steps of block mb have landed, and with `lines` the other wave of these columns has the block before behind it (it
+    // has put its rows of the one before that into the stage, and taken its columns of the one before that out of it).
+    auto await = [&](int mb) {
+        for (int l = land;; l = *flag)
+            if (__all(l >= (mb + 1) * NS - flag_add))
+                break;
+        asm volatile("" ::: "memory"); // (no read of the stages before this)
+    };
+    // (every read of the block's stages has been waited for by its product)
+    auto say = [&](int mb) {
+        asm volatile("" ::: "memory");
+        if (lane == 0)
+            done[wave] = (mb + 1) * NS;
+    };
+    if (active) {
+        await(0);
+        acc = block(acc, 0, std::integral_constant<int, 0>());
+        say(0);
+        // (the weight has arrived: nothing in the loop waits for it, which would be to wait for stores as well)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int k16 = 0; k16 < 4; ++k16)
+                asm volatile("" : "+v"(bq[s][k16]));
+        asm volatile("" : "+v"(out_col), "+v"(out_bias));
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const uint32_t col = (uint32_t)__shfl(out_col, jq[q]);
+            o_q[q] = jq[q] < cnt ? col * ((uint32_t)p.ldc * 2u) + (uint32_t)row_q * 2u : 0xFFFFFF00u;
+        }
+        if (n_mb > 1) {
+            await(1);
+            acc = block(acc, 1, std::integral_constant<int, 1>());
+            say(1);
+        }
+        for (int mb = 2; mb < n_mb; ++mb) {
+            await(mb);
+            acc = block(acc, mb, std::integral_constant<int, 2>());
+            say(mb);
+        }
+        while (lines && done[wave ^ 4] < n_mb * NS) // (the other wave has taken out what was in the last block's stage)
+            ;
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = tw_fp32_value(tw_activate(p.alpha * acc[r4 * 4 + e] + out_bias, ACT));
+            stage_put((n_mb - 1) & 1, r4, v);
+        }
+        asm volatile("" ::: "memory");
+        if (lane == 0)
+            done[wave] = 0x7fffffff;
+        while (lines && done[wave ^ 4] != 0x7fffffff)
+            ;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        for (int mb = max(n_mb - 2, 0); mb < n_mb; ++mb) {
+            const u32x4 out[2] = {stage_get(mb & 1, 0), stage_get(mb & 1, 1)};
+            put(mb, out);
+        }
+    }
+    if (lane == 0)
+        done[wave] = 0x7fffffff;
+
+    // ---- TW_PRUNED_ZERO: the pruned columns of this unit's share of the tiles receive act(bias)
+    for (int z = p.n_gemm_u + ui; z < p.n_all_u; z += n_units) {
+        const TileDev t = p.tiles[z - p.n_gemm_u];
+        const int chunks = (m_hi - m_lo + 7) / 8;
+        for (int i = tid; i < t.n_pruned * chunks; i += 64 * kBwMulWaves) {
+            const int jz = i / chunks, ch = i - jz * chunks;
+            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
+            const uint32_t hb = E::to_bits(tw_finish(0.0f, p.bias, c, ACT));
+            const uint32_t w = hb | (hb << 16);
+            store_chunk(C + (int64_t)c * p.ldc + m_lo + ch * 8, u32x4{w, w, w, w}, m_lo + ch * 8, m_hi, p.store_through != 0);
+        }
+    }
+}
+
 bool bs_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
 {
     if (reads_c || plan->n_units == 0 || plan->n_pipe_units == 0)
@@ -325,8 +642,9 @@ bool bs_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
     // A is addressed through a buffer descriptor with 32-bit offsets
     if ((uint64_t)plan->K * (uint64_t)lda * 2u >= (1ull << 32))
         return false;
-    (void)ldc;
-    return plan->max_k_pad <= kBsMaxSteps * kBlockK;
+    // (and the wider form stores C through one)
+    return plan->max_k_pad <= kBsMaxSteps * kBlockK ||
+           (plan->max_k_pad <= kBwSteps * kBlockK && (uint64_t)plan->N * (uint64_t)ldc * 2u < kBwMaxBytes);
 }
 
 // ranges of rows of A a launch is cut into: as many as give every compute unit `per_cu`
@@ -345,13 +663,19 @@ int bs_ranges(const tw_plan *plan, int M, int per_cu)
     return r;
 }
 
-// share of the compute units' workgroup slots the launch fills, over a whole number of rounds
+// the wider form's: as many as fit one workgroup on each compute unit; below the number of dies whatever that is
+int bw_ranges(const tw_plan *plan, int M, int per_cu)
+{
+    const int r = std::min(std::max(1, plan->cu_count * std::max(1, per_cu) / std::max(1, plan->n_units)), std::max(1, (M + 31) / 64));
+    return r >= kXcd ? r / kXcd * kXcd : r;
+}
+
+// share of the compute units the launch fills with one workgroup each, over a whole number of rounds
 double bs_fill(const tw_plan *plan, int M)
 {
-    const int64_t wgs = (int64_t)plan->n_units * bs_ranges(plan, M, 0);
-    const int64_t slots = (int64_t)plan->cu_count * kBsPerCu;
-    const int64_t rounds = (wgs + slots - 1) / slots;
-    return (double)wgs / (double)(rounds * slots);
+    const int64_t wgs = (int64_t)plan->n_units * bw_ranges(plan, M, 1), cu = plan->cu_count;
+    const int64_t rounds = (wgs + cu - 1) / cu;
+    return (double)wgs / (double)(rounds * cu);
 }
 
 template <int DT, int NS> static int launch_bs_t(const tw_plan *plan, const GemmArgs &a, int per_cu, hipStream_t s)
@@ -368,27 +692,54 @@ template <int DT, int NS> static int launch_bs_t(const tw_plan *plan, const Gemm
     return TW_OK;
 }
 
+template <int DT, int NS> static int launch_bw(const tw_plan *plan, const GemmArgs &a, int per_cu, hipStream_t s)
+{
+    const int n_ranges = bw_ranges(plan, a.M, per_cu);
+    const int affine = n_ranges >= kXcd;
+    const int64_t grid = affine ? (int64_t)kXcd * plan->n_units * (n_ranges / kXcd) : (int64_t)n_ranges * plan->n_units;
+    if (grid > (int64_t)0x7fffffff)
+        return fail(TW_ERR_SHAPE, "%lld workgroups (M=%d): a launch takes at most %lld", (long long)grid, a.M,
+                    (long long)(int64_t)0x7fffffff);
+    const auto kernel = a.act == TW_ACT_RELU   ? tw_gemm_bw_kernel<DT, TW_ACT_RELU, NS>
+                        : a.act == TW_ACT_GELU ? tw_gemm_bw_kernel<DT, TW_ACT_GELU, NS>
+                        : a.act == TW_ACT_TANH ? tw_gemm_bw_kernel<DT, TW_ACT_TANH, NS>
+                                               : tw_gemm_bw_kernel<DT, TW_ACT_NONE, NS>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(bw_threads(NS)), 0, s, a, plan->n_units, n_ranges, (a.M + 31) / 32, affine,
+                       (uint32_t)((uint64_t)plan->K * (uint64_t)a.lda * 2u), (uint32_t)((uint64_t)plan->N * (uint64_t)a.ldc * 2u),
+                       (int64_t)a.M * plan->N * 2 > kBwLineBytes);
+    TW_HIP(hipGetLastError());
+    return TW_OK;
+}
+
 int launch_bs(const tw_plan *plan, const GemmArgs &a, int per_cu, hipStream_t s)
 {
     // (per_cu <= 0: as many workgroups per compute unit as the kernel is built for)
     const int ns = std::max(1, plan->max_k_pad / kBlockK);
     const int pc = per_cu > 0 ? per_cu : kBsPerCu;
-    if (plan->dtype == TW_F16) {
-        switch (ns) {
-        case 1:
-        case 2:
-            return launch_bs_t<TW_F16, 2>(plan, a, pc, s);
-        default:
-            return launch_bs_t<TW_F16, 3>(plan, a, pc, s);
-        }
+    const bool f16 = plan->dtype == TW_F16;
+    // Up to three steps either kernel takes the plan.  Without a long activation, where the launch is little but its stores, the
+    // one whose waves store 64 rows themselves is ahead where its workgroups, two to a compute unit, come out even: beyond 112
+    // MB of output (M 16384, N 4096, 120 kept rows: 38.5 against 47.1 us; M 14336: 34.5 against 29.5; with GELU 54.9 against
+    // 50.1; 34, 39 or 44 units, which leave it a third of the chip, 1.1 - 1.4 of the time of what ran before), and with one step
+    // from 32 MB on (60 kept: M 8192, N 4096 18.9 against 22.7, M 8192, N 2048 12.1 against 13.9; M 8192, N 3072, not even, 19.9
+    // against 16.9).
+    const int64_t out_bytes = (int64_t)a.M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, a.M, 2);
+    const int64_t slots2 = 2 * (int64_t)plan->cu_count, all2 = (wgs2 + slots2 - 1) / slots2 * slots2;
+    const bool stores_only = (a.act == TW_ACT_NONE || a.act == TW_ACT_RELU) &&
+                             ((out_bytes > (int64_t)112 << 20 && wgs2 * 4 >= all2 * 3) ||
+                              (ns == 1 && out_bytes >= (int64_t)32 << 20 && wgs2 * 10 >= all2 * 9));
+    if (ns <= 3 && (stores_only || (uint64_t)plan->N * (uint64_t)a.ldc * 2u >= kBwMaxBytes)) {
+        if (ns <= 2)
+            return f16 ? launch_bs_t<TW_F16, 2>(plan, a, pc, s) : launch_bs_t<TW_BF16, 2>(plan, a, pc, s);
+        return f16 ? launch_bs_t<TW_F16, 3>(plan, a, pc, s) : launch_bs_t<TW_BF16, 3>(plan, a, pc, s);
     }
-    switch (ns) {
-    case 1:
-    case 2:
-        return launch_bs_t<TW_BF16, 2>(plan, a, pc, s);
-    default:
-        return launch_bs_t<TW_BF16, 3>(plan, a, pc, s);
-    }
+    if (ns <= 2)
+        return f16 ? launch_bw<TW_F16, 2>(plan, a, per_cu, s) : launch_bw<TW_BF16, 2>(plan, a, per_cu, s);
+    if (ns == 3)
+        return f16 ? launch_bw<TW_F16, 3>(plan, a, per_cu, s) : launch_bw<TW_BF16, 3>(plan, a, per_cu, s);
+    if (ns == 4)
+        return f16 ? launch_bw<TW_F16, 4>(plan, a, per_cu, s) : launch_bw<TW_BF16, 4>(plan, a, per_cu, s);
+    return f16 ? launch_bw<TW_F16, 6>(plan, a, per_cu, s) : launch_bw<TW_BF16, 6>(plan, a, per_cu, s);
 }
 
 } // namespace tw

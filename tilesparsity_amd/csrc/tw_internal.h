@@ -190,7 +190,7 @@ bool skinny_takes_row_major(const tw_plan *p, int M, float beta);
 // `per_cu` workgroups meant to share a compute unit
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
 int launch_bs(const tw_plan *p, const GemmArgs &a, int per_cu, hipStream_t s);
-double bs_fill(const tw_plan *p, int M); // share of the chip's workgroup slots its launch fills
+double bs_fill(const tw_plan *p, int M); // share of the compute units its launch gives a workgroup
 // the row-major streaming kernel (tw_gemm_rm.hip): whether it can take the plan, its workgroups per block of rows of A,
 // its launch, its set-up per device
 constexpr int kRmRowsPerWg = 64;
