@@ -209,6 +209,25 @@ def test_full_size_network_all_producers(twprune, po):
     assert all(np.array_equal(w, g) for w, g in zip(want, got))
 
 
+
+@pytest.mark.parametrize("g1", [5, 50])
+def test_mix_selection_with_uneven_pieces(twprune, po, g1):
+    """The values inside the bracket lie together: a third of a few thousand consecutive elements, so that the pieces of the waves
+    that read these hold some three hundred values each and most others few or none.  Bit for bit the oracle's."""
+    rng = np.random.default_rng(47)
+    shapes = [(577, 300), (64, 1000), (33, 7)]
+    scores = [np.abs(rng.standard_normal(s)).astype(np.float32) for s in shapes]
+    masks = [np.zeros(s, bool) for s in shapes]
+    flat = scores[0].reshape(-1)
+    at = np.quantile(np.concatenate([s.reshape(-1) for s in scores]), 1 - g1 / 100)
+    near = np.flatnonzero(rng.random(20480) < 0.35) + 8192
+    flat[near] = at * (1 + 0.002 * (rng.random(near.size) - 0.5))
+    want, thr = po.tw_mix_fn(scores, g1, masks)
+    got = twprune.tw_mix_fn(scores, g1, masks)
+    assert np.float64(thr) == twprune.tw_mix_fn.last_threshold
+    for a, b in zip(want, got):
+        assert np.array_equal(a, b)
+
 def _mixed_layer(rng, twprune, K, N, G, sparsity, g1, structured):
     """Weight, the TW mask of the mixed producer's first stage and the mixed mask."""
     W = (rng.standard_normal((K, N)) * 0.1).astype(np.float32)

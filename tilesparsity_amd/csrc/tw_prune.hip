@@ -1118,7 +1118,7 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // between (2 - 3 % of the elements), and the three passes run over what was kept.
 // Where the bracket missed or does not fit - the counts tell, for certain - they run over the
 // elements.
-// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 14 + 31 + 39 us.
+// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 11 + 31 + 31 us.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
 __global__ void __launch_bounds__(256) mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, uint32_t *sample)
@@ -1162,19 +1162,44 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
     const double want[2] = {mid - dev, mid + dev};
     auto key_of = [&](int i) { return s_key[i]; };
     const KeyRange range = key_range_in_block<kBracketThreads>(key_of, kMixSamples); // (its barrier: s_key is whole)
-    uint32_t edge[2];
+    // both edges out of one count of the first digit and one of the second, with counters for each: an edge is a chain of trips
+    // through LDS and barriers, which is all that this kernel waits for (one edge after the other: 14.6 us, so 11)
+    __shared__ unsigned int s_h2[kSelBins];
+    bool inside[2];
+    uint32_t prefix[2], edge[2];
+    unsigned long long rank[2];
+    for (int i = tid; i < kSelBins; i += kBracketThreads)
+        s_h[i] = s_h2[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        atomicAdd(&s_h[range.digit(0, key[i] - range.base)], 1u);
+    __syncthreads();
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-        if (want[w] < 0.0 || want[w] >= (double)kMixSamples) { // workgroup-uniform
-            edge[w] = w ? 0xFFFFFFFFu : 0u;
-            continue;
-        }
-        uint32_t prefix = 0, mn = 0xFFFFFFFFu;
-        unsigned long long rank = (unsigned long long)want[w];
-        count_in_block<0, kBracketThreads>(key_of, kMixSamples, range, rank, prefix, s_h, mn);
-        count_in_block<1, kBracketThreads>(key_of, kMixSamples, range, rank, prefix, s_h, mn);
-        const unsigned long long at = ((unsigned long long)prefix + w) << range.shift[1];
-        edge[w] = (uint32_t)min((unsigned long long)range.base + at - w, 0xFFFFFFFFull);
+        inside[w] = want[w] >= 0.0 && want[w] < (double)kMixSamples; // workgroup-uniform
+        const Digit d = find_digit<kBracketThreads, kSelBins>(s_h, inside[w] ? (unsigned long long)want[w] : 0ull);
+        prefix[w] = d.digit;
+        rank[w] = d.rest;
+    }
+    for (int i = tid; i < kSelBins; i += kBracketThreads)
+        s_h[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const uint32_t k = key[i] - range.base, lead = k >> range.lead_shift(1);
+        if (lead == prefix[0])
+            atomicAdd(&s_h[range.digit(1, k)], 1u);
+        if (lead == prefix[1])
+            atomicAdd(&s_h2[range.digit(1, k)], 1u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const Digit d = find_digit<kBracketThreads, kSelBins>(w ? s_h2 : s_h, rank[w]);
+        const uint32_t both = prefix[w] << (range.lead_shift(1) - range.shift[1]) | d.digit;
+        const unsigned long long at = ((unsigned long long)both + w) << range.shift[1];
+        edge[w] = inside[w] ? (uint32_t)min((unsigned long long)range.base + at - w, 0xFFFFFFFFull) : w ? 0xFFFFFFFFu : 0u;
     }
     if (tid == 0) {
         st->lo = edge[0] == 0u ? -INFINITY : key_to_float(edge[0]);
@@ -1256,6 +1281,7 @@ __device__ bool mix_totals(const MixCounts *counts, int waves, uint32_t room, un
 }
 
 constexpr int kMixHistWgs = 96; // workgroups that count what was kept (each adds up to 2048 counters to the others')
+static_assert(kMixWaves <= 64 * 4 * kMixHistWgs, "a lane for each piece of a wave");
 template <int PASS>
 __global__ void __launch_bounds__(256)
     mix_hist_kernel(const MixLayer *layers, int n_layers, int64_t n_items, SelectState *st, const float *cand,
@@ -1267,6 +1293,10 @@ __global__ void __launch_bounds__(256)
     unsigned long long rank;
     const unsigned long long want = st->head.rank0;
     const uint32_t room = st->room;
+    // this wave's pieces (at most 64, see below): w0, w0 + per, ..; lane l has the count of number l
+    const int per = min((int)gridDim.x, kMixHistWgs) * 4, w0 = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+    const int mine = w0 < min(per, waves) ? (waves - w0 + per - 1) / per : 0;
+    const uint32_t held = lane < mine ? counts[w0 + lane * per].between : 0u;
     unsigned long long n_cand, below;
     const bool whole = mix_totals(counts, waves, room, n_cand, below);
     // the wanted value and the one above it lie inside the bracket, and all of that was kept
@@ -1284,19 +1314,38 @@ __global__ void __launch_bounds__(256)
         st->key_bits = bits;
     }
     if (narrowed) {
-        const int per = min((int)gridDim.x, kMixHistWgs) * 4;
-        for (int w = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)); w < waves; w += per) {
-            const uint32_t n = counts[w].between;
-            TW_GLOBAL(const float) const v = as_global(cand) + (int64_t)w * room;
-            for (uint32_t i = threadIdx.x & 63; i < n; i += 256) { // four loads in flight
-                float x[4];
+        // four pieces at a time, sixteen loads in flight: a piece holds some two hundred values, and one piece after the other,
+        // each behind the load of its count, was eleven pairs of trips to memory (the three passes 18 + 12 + 12 us, so 9 + 11 +
+        // 11; what is left are the counts of all waves, the digits so far and the counters' atomics: 48 workgroups 12 + 15 + 15,
+        // 192 10 + 10 + 10, 256 12 + 10 + 10)
+        for (int q0 = 0; q0 < mine; q0 += 4) {
+            TW_GLOBAL(const float) v[4];
+            uint32_t n[4];
+            float x[4][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                n[q] = q0 + q < mine ? (uint32_t)__builtin_amdgcn_readlane((int)held, q0 + q) : 0u;
+                v[q] = as_global(cand) + (int64_t)(w0 + min(q0 + q, mine - 1) * per) * room;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    x[e] = v[min(i + e * 64, n - 1)];
+                    x[q][e] = v[q][min((uint32_t)(lane + e * 64), max(n[q], 1u) - 1u)];
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (i + e * 64 < n)
-                        select_count<PASS>(sort_key(x[e]), range, prefix, s_h, mn);
+                    if ((uint32_t)(lane + e * 64) < n[q])
+                        select_count<PASS>(sort_key(x[q][e]), range, prefix, s_h, mn);
+                for (uint32_t i = 256 + lane; i < n[q]; i += 256) { // (the rest of a long one)
+                    float y[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        y[e] = v[q][min(i + e * 64, n[q] - 1)];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (i + e * 64 < n[q])
+                            select_count<PASS>(sort_key(y[e]), range, prefix, s_h, mn);
+                }
             }
         }
     } else {
