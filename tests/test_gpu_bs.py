@@ -193,3 +193,33 @@ def test_weight_stationary_wide_form(tw, oracle, dtype, case):
                 assert not Cf[:, ~keep].any()
     finally:
         tw.set_option(tw.OPT_SHAPE, -1)
+
+
+@pytest.mark.parametrize("kept", [100, 350])
+def test_weight_stationary_padding_lies_beyond_the_largest_a(tw, oracle, kept):
+    """The padding of a tile's row list is fetched from beyond A's buffer, which delivers zeros - also where A ends 16 bytes
+    short of 4 GiB: NaN in the last 256 bytes of A (padding behind row K - 1) reaches no product.  Bit for bit what the same
+    rows of A give in a small buffer."""
+    import torch
+    M, K, G, N = 4096, 3741, 128, 1024
+    rng = np.random.default_rng(91 + kept)
+    tiles = make_tiles(rng, K - 1, G, ((kept, G),) * (N // G))
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    Ab = torch.randn((K, M), generator=torch.Generator("cuda").manual_seed(kept), device="cuda").half()
+    s = torch.cuda.current_stream().cuda_stream
+    out = []
+    with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+        for lda in (M, 574040):
+            dA = torch.zeros((K, lda), dtype=torch.float16, device="cuda")
+            dA[:, :M] = Ab
+            if lda > M:
+                assert dA.numel() * 2 == 2 ** 32 - 16
+                dA[K - 1, lda - 128:] = float("nan")
+            assert plan.choice(M, lda=lda, ldc=M)["shape"] == tw.SHAPE_BS
+            dC = torch.zeros((N, M), dtype=torch.float16, device="cuda")
+            print("padding beyond A: kept", kept, "lda", lda, flush=True)
+            plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=M, stream=s)
+            torch.cuda.synchronize()
+            out.append(dC.view(torch.int16))
+            del dA
+    assert torch.equal(out[0], out[1])

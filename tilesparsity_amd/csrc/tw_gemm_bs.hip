@@ -347,6 +347,7 @@ constexpr int kBwCStage = 32 * kBwCPitch * 2;        // bytes; two of them for t
 constexpr int64_t kBwLineBytes = 90 << 20;           // outputs from here on are stored in whole lines
 constexpr uint64_t kBwMaxBytes = 0xFFFF0000u;        // of C, which is stored through a buffer descriptor
 constexpr int kBwSteps = 6;                          // most steps of an instantiation
+constexpr uint32_t kBwNoRow = 0xFFFFFFFFu;           // (offsets of rows are multiples of 16)
 
 template <int DT, int ACT, int NS>
 __global__ void __launch_bounds__(bw_threads(NS), 3)
@@ -358,7 +359,7 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
     static_assert(LW * SPW == NS, "whole steps a wave");
     __shared__ __align__(1024) unsigned char ring[kBwRing * kBsStage];
     __shared__ __align__(16) unsigned char cstage[kBwMulWaves * kBwCStage];
-    __shared__ uint32_t row_off[NS * kBlockK]; // byte offset of each kept row in A, beyond the buffer for the list's padding
+    __shared__ uint32_t row_off[NS * kBlockK]; // byte offset of each kept row in A, kBwNoRow for the list's padding
     __shared__ int flags[16];                  // first step that is not there of each loading wave's, steps each multiplying wave has read
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -393,7 +394,7 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
 #pragma unroll
         for (int q = 0; q < SPW; ++q) {
             const int i = (w * SPW + q) * kBlockK + lane;
-            row_off[i] = i < u.k_kept ? (uint32_t)p.kept_k[u.kk_off + i] * lda_b : 0xFFFFFF00u;
+            row_off[i] = i < u.k_kept ? (uint32_t)p.kept_k[u.kk_off + i] * lda_b : kBwNoRow;
         }
         TW_LDS_BARRIER(); // the row offsets, and the flags
         const __amdgpu_buffer_rsrc_t a_rsrc =
@@ -404,8 +405,11 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
 #pragma unroll
         for (int q = 0; q < SPW; ++q)
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                off[q][j] = row_off[(w * SPW + q) * kBlockK + j * 8 + rr] + (uint32_t)(pos ^ ((rr >> 1 & 1) << 2)) * 16u;
+            for (int j = 0; j < 8; ++j) {
+                // (a row that is not there: 16 bytes short of 4 GiB whatever the piece, beyond every buffer bs_takes admits)
+                const uint32_t row = row_off[(w * SPW + q) * kBlockK + j * 8 + rr];
+                off[q][j] = row == kBwNoRow ? 0xFFFFFFF0u : row + (uint32_t)(pos ^ ((rr >> 1 & 1) << 2)) * 16u;
+            }
         TW_LDS(unsigned char) const lds0 = (TW_LDS(unsigned char))ring;
         // two blocks in flight: what a block takes to arrive is more than what it takes to multiply
         auto issue = [&](int mb) {
