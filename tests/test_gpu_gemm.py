@@ -1270,3 +1270,29 @@ def test_row_major_streaming_nonfinite(tw, oracle):
     assert bool(torch.isfinite(r[:, :6 * G]).any()) and bool(torch.isinf(r[:, 11]).all())
     fin = torch.isfinite(r)
     assert float((r[fin].float() - k[fin].float()).abs().max()) <= 2e-3 * float(k[fin].float().abs().max())
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged):
+    """262208 tiles of one column: more groups of units than the second dimension of a grid has.  Row-major calls of such a
+    plan run on the kernels that number their workgroups in one dimension, with a workspace and without."""
+    import torch
+    M, K, N = 8, 16, 262208
+    gen = torch.Generator("cuda").manual_seed(3)
+    A = torch.randn((M, K), generator=gen, device="cuda").half()
+    B = torch.randn((K, N), generator=gen, device="cuda")
+    C0 = torch.randn((M, N), generator=gen, device="cuda").half()
+    kept = torch.arange(N, device="cuda") % K                # the one kept row of every tile
+    mask = torch.zeros((K, N), dtype=torch.uint8, device="cuda")
+    mask[kept, torch.arange(N, device="cuda")] = 1
+    want = A.double()[:, kept] * B.half().double()[kept, torch.arange(N, device="cuda")] + 0.5 * C0.double()
+    s = torch.cuda.current_stream().cuda_stream
+    with tw.Plan.from_device_mask(K, N, mask.data_ptr(), [(c, 1) for c in range(N)], "f16", B.data_ptr(), stream=s) as plan:
+        nbytes = plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR) if staged else 0
+        ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda") if staged else None
+        C = C0.clone()
+        plan.gemm(A.data_ptr(), C.data_ptr(), M, lda=K, ldc=N, beta=0.5, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR, stream=s,
+                  workspace_ptr=ws.data_ptr() if staged else None, workspace_bytes=nbytes)
+        torch.cuda.synchronize()
+    # one product in fp32, one rounding to f16
+    assert bool(((C.double() - want).abs() <= 2.0 ** -11 * want.abs() * 1.01 + 1e-6).all())

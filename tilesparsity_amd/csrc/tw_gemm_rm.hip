@@ -462,17 +462,19 @@ __global__ void __launch_bounds__(kRmThreads, 2)
     }
 }
 
-// Whether the kernel can take the plan: its lists fit beside the ring, its offsets 32 bits.
-bool rm_takes(const tw_plan *plan, int64_t lda)
-{
-    return plan->n_units > 0 && rm_lds_bytes(plan) <= kRmMaxLds && lda * 2 * kRmRows < (1ll << 31) &&
-           plan->packed_elems * 2 < (1ll << 31);
-}
-
 int rm_groups(const tw_plan *plan)
 {
     const int units = rm_units(rm_narrow(plan));
     return (plan->n_units + units - 1) / units;
+}
+
+// Whether the kernel can take the plan: its lists fit beside the ring, its offsets 32 bits, its groups of units the second
+// dimension of a grid.
+constexpr int kRmMaxGroups = 65535;
+bool rm_takes(const tw_plan *plan, int64_t lda)
+{
+    return plan->n_units > 0 && rm_lds_bytes(plan) <= kRmMaxLds && lda * 2 * kRmRows < (1ll << 31) &&
+           plan->packed_elems * 2 < (1ll << 31) && rm_groups(plan) <= kRmMaxGroups;
 }
 
 template <int DT, bool NARROW> static int launch_rm_t(const tw_plan *plan, const GemmArgs &a, hipStream_t s)
@@ -481,8 +483,6 @@ template <int DT, bool NARROW> static int launch_rm_t(const tw_plan *plan, const
     // (a row block to a die where that leaves no die more than a tenth behind)
     const int padded = (n_rowblk + kXcd - 1) / kXcd * kXcd;
     const int gx = (int64_t)padded * 10 <= (int64_t)n_rowblk * 11 ? padded : n_rowblk;
-    if (n_groups > 65535)
-        return fail(TW_ERR_SHAPE, "%d units: a launch takes at most %d groups of them", plan->n_units, 65535);
     hipLaunchKernelGGL((tw_gemm_rm_kernel<DT, NARROW>), dim3((unsigned)gx, (unsigned)n_groups), dim3(kRmThreads),
                        (size_t)rm_lds_bytes(plan), s, a, plan->K, n_rowblk, plan->max_k_pad);
     TW_HIP(hipGetLastError());
