@@ -1296,3 +1296,23 @@ def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged):
         torch.cuda.synchronize()
     # one product in fp32, one rounding to f16
     assert bool(((C.double() - want).abs() <= 2.0 ** -11 * want.abs() * 1.01 + 1e-6).all())
+
+
+def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw):
+    """2^29 + 70 rows: a workgroup of 512 threads for every 64 of them is beyond 2^32 threads; C is read, so that no panel
+    kernel applies."""
+    import torch
+    M, K, N = (1 << 29) + 70, 8, 8
+    B = torch.full((K, N), 0.5, device="cuda")
+    mask = torch.zeros((K, N), dtype=torch.uint8, device="cuda")
+    mask[2:5] = 1
+    s = torch.cuda.current_stream().cuda_stream
+    A = torch.ones((M, K), dtype=torch.float16, device="cuda")
+    A[-3:] = 2.0
+    A[:, 0] = 7.0                                            # (not kept)
+    C = torch.ones((M, N), dtype=torch.float16, device="cuda")
+    with tw.Plan.from_device_mask(K, N, mask.data_ptr(), [(0, N)], "f16", B.data_ptr(), stream=s) as plan:
+        plan.gemm(A.data_ptr(), C.data_ptr(), M, lda=K, ldc=N, beta=2.0, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR, stream=s)
+        torch.cuda.synchronize()
+    assert bool((C[-3:] == 5.0).all()) and bool((C[:100] == 3.5).all()) and bool((C[M - 200:-3] == 3.5).all())
+    assert int((C != 3.5).sum(dtype=torch.int64)) == 3 * N

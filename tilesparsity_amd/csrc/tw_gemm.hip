@@ -2746,7 +2746,7 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
 // kept: 0.92 - 1.3 of the time).
 bool streams_row_major(const tw_plan *plan, int M, int64_t lda, float beta)
 {
-    if (option(TW_OPT_SHAPE) != -1 || !rm_takes(plan, lda)) // (a forced shape keeps the paths around the K-major kernels)
+    if (option(TW_OPT_SHAPE) != -1 || !rm_takes(plan, M, lda)) // (a forced shape keeps the paths around the K-major kernels)
         return false;
     const int64_t groups = rm_groups(plan), wgs = (((int64_t)M + kRmRowsPerWg - 1) / kRmRowsPerWg) * groups;
     if (takes_row_major_directly(plan, beta))
@@ -3112,7 +3112,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
             return b64 ? launch_as<TW_F16, 64, true>(plan, a, M, s) : launch_as<TW_F16, 32, true>(plan, a, M, s);
         return b64 ? launch_as<TW_BF16, 64, true>(plan, a, M, s) : launch_as<TW_BF16, 32, true>(plan, a, M, s);
     }
-    if (streams || (row_major && option(TW_OPT_SHAPE) == -1 && rm_takes(plan, lda))) {
+    if (streams || (row_major && option(TW_OPT_SHAPE) == -1 && rm_takes(plan, M, lda))) {
         // (off the rule's range too: the layout-generic kernel is several times slower everywhere)
         fill_queues(a, plan, M, kRmRowsPerWg, 128, pruned_cols, false);
         if (a.n_all_u == 0)

@@ -468,13 +468,14 @@ int rm_groups(const tw_plan *plan)
     return (plan->n_units + units - 1) / units;
 }
 
-// Whether the kernel can take the plan: its lists fit beside the ring, its offsets 32 bits, its groups of units the second
-// dimension of a grid.
+// Whether the kernel can take the call: its lists fit beside the ring, its offsets 32 bits, its blocks of rows (a row block
+// to a die, see launch_rm_t) and groups of units the two dimensions of a grid.
 constexpr int kRmMaxGroups = 65535;
-bool rm_takes(const tw_plan *plan, int64_t lda)
+bool rm_takes(const tw_plan *plan, int M, int64_t lda)
 {
     return plan->n_units > 0 && rm_lds_bytes(plan) <= kRmMaxLds && lda * 2 * kRmRows < (1ll << 31) &&
-           plan->packed_elems * 2 < (1ll << 31) && rm_groups(plan) <= kRmMaxGroups;
+           plan->packed_elems * 2 < (1ll << 31) && rm_groups(plan) <= kRmMaxGroups &&
+           ((int64_t)M / kRmRows + kXcd) * kRmThreads <= kMaxGridThreads;
 }
 
 template <int DT, bool NARROW> static int launch_rm_t(const tw_plan *plan, const GemmArgs &a, hipStream_t s)

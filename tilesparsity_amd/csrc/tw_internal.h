@@ -59,6 +59,9 @@ struct TileDev {
 constexpr int kXcd = 8;
 constexpr int kTicketInts = 16; // per slot: [0, kXcd) next index of each queue, [kXcd] workgroups done
 
+// Threads of a grid's first dimension: a launch of more reports no error and runs nothing.
+constexpr int64_t kMaxGridThreads = 0xFFFFFFFFll;
+
 struct GemmArgs {
     const UnitDev *units;   // sorted by k_kept descending
     const TileDev *tiles;
@@ -195,7 +198,7 @@ double bs_fill(const tw_plan *p, int M); // share of the compute units its launc
 // its launch, its set-up per device
 constexpr int kRmRowsPerWg = 64;
 int rm_groups(const tw_plan *p);
-bool rm_takes(const tw_plan *p, int64_t lda);
+bool rm_takes(const tw_plan *p, int M, int64_t lda);
 int launch_rm(const tw_plan *p, const GemmArgs &a, hipStream_t s);
 int prepare_rm();
 // true where tw_gemm_ex takes a row-major A and a row-major C of this plan with it
