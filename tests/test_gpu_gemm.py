@@ -1272,12 +1272,13 @@ def test_row_major_streaming_nonfinite(tw, oracle):
     assert float((r[fin].float() - k[fin].float()).abs().max()) <= 2e-3 * float(k[fin].float().abs().max())
 
 
-@pytest.mark.parametrize("staged", [False, True])
-def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged):
+@pytest.mark.parametrize("staged,M", [(False, 8), (True, 8), (False, 8200)])
+def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged, M):
     """262208 tiles of one column: more groups of units than the second dimension of a grid has.  Row-major calls of such a
-    plan run on the kernels that number their workgroups in one dimension, with a workspace and without."""
+    plan run on the kernels that number their workgroups in one dimension, with a workspace and without; 8200 rows are more
+    work items than one launch takes."""
     import torch
-    M, K, N = 8, 16, 262208
+    K, N = 16, 262208
     gen = torch.Generator("cuda").manual_seed(3)
     A = torch.randn((M, K), generator=gen, device="cuda").half()
     B = torch.randn((K, N), generator=gen, device="cuda")
@@ -1285,7 +1286,8 @@ def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged):
     kept = torch.arange(N, device="cuda") % K                # the one kept row of every tile
     mask = torch.zeros((K, N), dtype=torch.uint8, device="cuda")
     mask[kept, torch.arange(N, device="cuda")] = 1
-    want = A.double()[:, kept] * B.half().double()[kept, torch.arange(N, device="cuda")] + 0.5 * C0.double()
+    rows = torch.unique(torch.tensor([0, 1, 2, 3, 4, 5, 6, 7, 127, 128, 8063, 8064, 8191, 8192, 8199], device="cuda").clamp(max=M - 1))
+    want = A[rows].double()[:, kept] * B.half().double()[kept, torch.arange(N, device="cuda")] + 0.5 * C0[rows].double()
     s = torch.cuda.current_stream().cuda_stream
     with tw.Plan.from_device_mask(K, N, mask.data_ptr(), [(c, 1) for c in range(N)], "f16", B.data_ptr(), stream=s) as plan:
         nbytes = plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR) if staged else 0
@@ -1295,12 +1297,13 @@ def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged):
                   workspace_ptr=ws.data_ptr() if staged else None, workspace_bytes=nbytes)
         torch.cuda.synchronize()
     # one product in fp32, one rounding to f16
-    assert bool(((C.double() - want).abs() <= 2.0 ** -11 * want.abs() * 1.01 + 1e-6).all())
+    assert bool(((C[rows].double() - want).abs() <= 2.0 ** -11 * want.abs() * 1.01 + 1e-6).all())
 
 
-def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw):
-    """2^29 + 70 rows: a workgroup of 512 threads for every 64 of them is beyond 2^32 threads; C is read, so that no panel
-    kernel applies."""
+@pytest.mark.parametrize("beta", [2.0, 0.0])
+def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw, beta):
+    """2^29 + 70 rows: a workgroup for every 64 of them is beyond 2^32 threads, with C read (no panel of A in LDS then) and not
+    read (a panel)."""
     import torch
     M, K, N = (1 << 29) + 70, 8, 8
     B = torch.full((K, N), 0.5, device="cuda")
@@ -1312,7 +1315,7 @@ def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw):
     A[:, 0] = 7.0                                            # (not kept)
     C = torch.ones((M, N), dtype=torch.float16, device="cuda")
     with tw.Plan.from_device_mask(K, N, mask.data_ptr(), [(0, N)], "f16", B.data_ptr(), stream=s) as plan:
-        plan.gemm(A.data_ptr(), C.data_ptr(), M, lda=K, ldc=N, beta=2.0, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR, stream=s)
+        plan.gemm(A.data_ptr(), C.data_ptr(), M, lda=K, ldc=N, beta=beta, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR, stream=s)
         torch.cuda.synchronize()
-    assert bool((C[-3:] == 5.0).all()) and bool((C[:100] == 3.5).all()) and bool((C[M - 200:-3] == 3.5).all())
-    assert int((C != 3.5).sum(dtype=torch.int64)) == 3 * N
+    assert bool((C[-3:] == 3.0 + beta).all()) and bool((C[:100] == 1.5 + beta).all()) and bool((C[M - 200:-3] == 1.5 + beta).all())
+    assert int((C != 1.5 + beta).sum(dtype=torch.int64)) == 3 * N

@@ -2503,7 +2503,7 @@ static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w)
     w->dies_per_unit = w->left ? kXcd / w->left : 1;
     const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->halves, grouped_items = grouped * w->n_rowblk;
     const int64_t left_items = w->left ? (int64_t)kXcd * w->halves * ((w->n_rowblk + w->dies_per_unit - 1) / w->dies_per_unit) : 0;
-    if (grouped_items + left_items > 0x7fffffff || grouped_items * grouped >= (1ll << 32))
+    if ((grouped_items + left_items) * 64 * 8 > kMaxGridThreads || grouped_items * grouped >= (1ll << 32))
         return -1;
     w->grouped = (int32_t)grouped;
     w->grouped_items = (int32_t)grouped_items;
@@ -2761,16 +2761,26 @@ template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, co
     const int pst = prepare_device();
     if (pst != TW_OK)
         return pst;
+    constexpr int kThreads = 64 * as_waves(BMS, RM), kMaxRows = (int)(kMaxGridThreads / kThreads * BMS / 256 * 256);
+    if (M > kMaxRows) { // (more rows than a grid takes threads: several launches)
+        for (int64_t m0 = 0; m0 < M; m0 += kMaxRows) {
+            GemmArgs part = a;
+            part.M = (int)std::min<int64_t>(M - m0, kMaxRows);
+            part.A = static_cast<const uint16_t *>(a.A) + m0 * (RM ? a.lda : 1);
+            part.C = static_cast<uint16_t *>(a.C) + m0 * (RM ? a.ldc : 1);
+            const int st = launch_as<DT, BMS, RM>(plan, part, part.M, s);
+            if (st != TW_OK)
+                return st;
+        }
+        return TW_OK;
+    }
     const int n_mblk = (M + BMS - 1) / BMS;
     // as many groups as keep every compute unit at one workgroup, each wave with a block or more
     const int per_wg = as_task_waves(BMS, RM);
     int n_groups = std::max(1, plan->cu_count / n_mblk);
     n_groups = std::min(n_groups, std::max(1, (plan->n_blocks + per_wg - 1) / per_wg));
-    if ((int64_t)n_mblk * n_groups > (int64_t)0x7fffffff)
-        return fail(TW_ERR_SHAPE, "%lld workgroups (M=%d): a launch takes at most %lld",
-                    (long long)n_mblk * n_groups, M, (long long)(int64_t)0x7fffffff);
-    hipLaunchKernelGGL((tw_gemm_as_kernel<DT, BMS, RM>), dim3((unsigned)(n_mblk * n_groups)),
-                       dim3(64 * as_waves(BMS, RM)), (size_t)as_lds_bytes(plan->K, BMS), s, a, plan->d_blocks, plan->n_blocks, n_groups,
+    hipLaunchKernelGGL((tw_gemm_as_kernel<DT, BMS, RM>), dim3((unsigned)(n_mblk * n_groups)), dim3(kThreads),
+                       (size_t)as_lds_bytes(plan->K, BMS), s, a, plan->d_blocks, plan->n_blocks, n_groups,
                        n_mblk, plan->K, plan->blocks_per_unit);
     TW_HIP(hipGetLastError());
     return TW_OK;
@@ -3124,25 +3134,31 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return pst != TW_OK ? pst : launch_rm(plan, a, (hipStream_t)stream);
     }
     if (a_layout != TW_LAYOUT_KMAJOR || c_layout != TW_LAYOUT_KMAJOR) {
-        // layout-generic path (element strides), 128-row blocks, one workgroup per item
+        // layout-generic path (element strides), 128-row blocks, one workgroup per item; as many launches as the
+        // grid's threads ask for
         fill_queues(a, plan, M, 128, 128, pruned_cols, false);
-        const int64_t n_items = (int64_t)a.n_all_u * a.n_mblk;
-        if (n_items == 0)
+        if (a.n_all_u == 0)
             return TW_OK;
-        if (n_items > kMaxItems)
-            return fail(TW_ERR_SHAPE, "%lld work items (M=%d): a launch takes at most %lld",
-                        (long long)n_items, M, (long long)kMaxItems);
+        const int64_t max_mblk = kMaxGridThreads / 256 / a.n_all_u;
+        if (max_mblk == 0)
+            return fail(TW_ERR_SHAPE, "%d units and tiles: a launch takes at most %lld", a.n_all_u, (long long)(kMaxGridThreads / 256));
         const int64_t sa_m = a_layout == TW_LAYOUT_KMAJOR ? 1 : lda;
         const int64_t sa_k = a_layout == TW_LAYOUT_KMAJOR ? lda : 1;
         const int64_t sc_m = c_layout == TW_LAYOUT_KMAJOR ? 1 : ldc;
         const int64_t sc_n = c_layout == TW_LAYOUT_KMAJOR ? ldc : 1;
-        if (plan->dtype == TW_F16)
-            hipLaunchKernelGGL((tw_gemm_generic_kernel<TW_F16>), dim3((unsigned)n_items), dim3(256), 0,
-                               (hipStream_t)stream, a, sa_m, sa_k, sc_m, sc_n);
-        else
-            hipLaunchKernelGGL((tw_gemm_generic_kernel<TW_BF16>), dim3((unsigned)n_items), dim3(256), 0,
-                               (hipStream_t)stream, a, sa_m, sa_k, sc_m, sc_n);
-        TW_HIP(hipGetLastError());
+        for (int64_t m0 = 0; m0 < M; m0 += max_mblk * 128) {
+            const int rows = (int)std::min<int64_t>(M - m0, max_mblk * 128);
+            a.A = static_cast<const uint16_t *>(A) + m0 * sa_m;
+            a.C = static_cast<uint16_t *>(C) + m0 * sc_m;
+            a.M = rows;
+            fill_queues(a, plan, rows, 128, 128, pruned_cols, false);
+            const dim3 grid((unsigned)(a.n_all_u * a.n_mblk));
+            if (plan->dtype == TW_F16)
+                hipLaunchKernelGGL((tw_gemm_generic_kernel<TW_F16>), grid, dim3(256), 0, (hipStream_t)stream, a, sa_m, sa_k, sc_m, sc_n);
+            else
+                hipLaunchKernelGGL((tw_gemm_generic_kernel<TW_BF16>), grid, dim3(256), 0, (hipStream_t)stream, a, sa_m, sa_k, sc_m, sc_n);
+            TW_HIP(hipGetLastError());
+        }
         return TW_OK;
     }
 

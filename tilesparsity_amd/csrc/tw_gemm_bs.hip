@@ -641,7 +641,7 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
 
 bool bs_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
 {
-    if (reads_c || plan->n_units == 0 || plan->n_pipe_units == 0)
+    if (reads_c || plan->n_units == 0 || plan->n_pipe_units == 0 || (int64_t)plan->n_units * 1024 > kMaxGridThreads)
         return false;
     // A is addressed through a buffer descriptor with 32-bit offsets
     if ((uint64_t)plan->K * (uint64_t)lda * 2u >= (1ull << 32))
