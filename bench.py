@@ -33,14 +33,14 @@ PREWARM_SECONDS = 0.03  # untimed launches before a configuration's warm-up step
 
 MEASURED_TRAFFIC = {
     "vgg16_conv4_2_im2col": ((2 * 62014 + 11282) * 1024, "profiles/tw_gemm_ws_kernel__vgg16_conv4_2.md (tw_gemm_ws_kernel 256x128)"),
-    "bert_base_ffn_in": ((2 * 7880 + 24576) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bs_kernel)"),
+    "bert_base_ffn_in": ((2 * 7880 + 24576) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bw_kernel)"),
     "nmt_lstm_gates": ((2 * 3558.5 + 1024) * 1024, "profiles/tw_gemm_skinny_kernel__nmt_lstm_gates.md (tw_gemm_skinny_kernel)"),
     "imbalance_stress": ((2 * 922921 + 209150) * 1024, "profiles/tw_gemm_ws_kernel__imbalance_stress.md (tw_gemm_ws_kernel 256x64)"),
     "bert_large_ffn1_keep50": ((2 * 25220 + 65570) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn1_50.md (tw_gemm_ws_kernel 256x128)"),
     "bert_large_ffn2_keep10": ((2 * 22280 + 16400) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn2.md (tw_gemm_ws_kernel 256x128)"),
     "bert_large_ffn2_keep50": ((2 * 49480 + 16400) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn2.md (tw_gemm_ws_kernel 256x128)"),
-    "bert_large_ffn1_keep25": ((2 * 16671 + 65536) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bs_kernel)"),
-    "bert_large_ffn1_keep10": ((2 * 12295 + 65536) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bs_kernel)"),
+    "bert_large_ffn1_keep25": ((2 * 16671 + 65536) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bw_kernel)"),
+    "bert_large_ffn1_keep10": ((2 * 12295 + 65536) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bw_kernel)"),
     "bert_large_ffn2_keep25": ((2 * 38160 + 16400) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn2.md (tw_gemm_ws_kernel 256x128)"),
 }
 
@@ -284,7 +284,7 @@ def run_workload(wl, steps, warmup, torch, rotate_bytes=768 << 20, repeats=5, gr
             for i in range(n_sets)]
     sparse = tw.Plan.create(K, N, dtype, tiles, B)
     dense = tw.Plan.dense(K, N, G, dtype, B)
-    kernel_sparse, kernel_dense = sparse.choice(M)["name"], dense.choice(M)["name"]
+    kernel_sparse, kernel_dense = sparse.kernel_name(M), dense.kernel_name(M)
     timer = time_plan_graph if graph else time_plan
     # After an idle stretch (the plans were just built on the host) the GPU's clocks take ~10 ms of
     # work to come back up: the first 100 launches of the headline shape then read 32.0 us instead

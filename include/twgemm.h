@@ -350,13 +350,20 @@ int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda
 #define TW_SHAPE_AS64 7    /* A-stationary, 64 rows of all K in LDS: K up to 1064, beta == 0 */
 #define TW_SHAPE_AS32 8    /* A-stationary, 32 rows: K up to 2128, beta == 0 */
 #define TW_SHAPE_SKINNY 9  /* 64 rows x 32 columns per workgroup, the kept rows split over its waves: few rows of A */
-#define TW_SHAPE_BS 10     /* weight-stationary: a unit's packed weight in registers, A streamed: tiles of at most 384 kept rows (192 where it is forced), beta == 0 */
-#define TW_N_SHAPES 11
+#define TW_SHAPE_BS 10     /* weight-stationary: a unit's packed weight in registers, A streamed: tiles of at most 384 kept rows (192 where it is forced), beta == 0; which of the two kernels below follows from the plan and the call */
+#define TW_SHAPE_BS4 11    /* forced only: the weight-stationary kernel of four multiplying waves, tiles of at most 192 kept rows */
+#define TW_SHAPE_BS8 12    /* forced only: the one of eight, tiles of at most 384 kept rows */
+#define TW_SHAPE_RM 13     /* forced only: the row-major streaming kernel, where A and C are row-major (K-major calls run as without it) */
+#define TW_N_SHAPES 14
 /* What a K-major launch of `plan` on M rows would run with, under the options in force:
  * choice[0] the TW_SHAPE_* kernel, [1] the columns of a unit piece, [2] workgroups per compute
  * unit, [3] 1 for one work queue per die.  (No counterpart in the reference, whose kernel is
  * fixed at compile time, basic_nn.cu:250-259; benchmarks name the kernel they timed with it.) */
 int tw_gemm_choice(const tw_plan *plan, int M, int64_t lda, int64_t ldc, float beta, int32_t *choice);
+/* Name of the kernel tw_gemm_ex runs for these arguments, in any layout, under the options in force (a static string; NULL
+ * for a NULL plan, M < 0 or an unknown layout).  tw_gemm_staged runs the same one where it stages nothing. */
+const char *tw_gemm_kernel_name(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, int64_t ldc, float beta,
+                                int activation);
 int tw_set_option(int option, int value);
 
 /* One-shot drop-in for Stream_Gemm_NN (basic_nn.cu:378-393), same argument

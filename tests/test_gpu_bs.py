@@ -223,3 +223,74 @@ def test_weight_stationary_padding_lies_beyond_the_largest_a(tw, oracle, kept):
             out.append(dC.view(torch.int16))
             del dA
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("case", range(len(CASES) + len(WIDE_CASES)))
+def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
+    """The kernel of four multiplying waves (up to 192 kept rows) and the one of eight (up to 384), forced in turn: without
+    activation and with ReLU bit for bit the streaming 256 x 128 kernel, with GELU and tanh one unit in the last place of the
+    result (2^-10, 2^-7: the same sum, its activation from a different order of instructions), pruned columns filled and
+    left alone, few and many ranges of rows, the padding of C's rows untouched."""
+    import torch
+    M, K, G, spec = (CASES + WIDE_CASES)[case]
+    N = G * len(spec)
+    rng = np.random.default_rng(1700 + case)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    dbias = torch.from_numpy(rng.standard_normal(N).astype(np.float32)).cuda()
+    tiles = make_tiles(rng, K, G, spec)
+    lda = ldc = (M + 7) // 8 * 8 + 8
+    At = np.zeros((K, lda), np.uint16)
+    At[:, :M] = oracle.cast_bits(A, dtype).reshape(M, K).T
+    dA = to_device_bits(At, At.shape)
+    s = torch.cuda.current_stream().cuda_stream
+    tdt = torch.float16 if dtype == "f16" else torch.bfloat16
+    ulp = 2.0 ** -10 if dtype == "f16" else 2.0 ** -7
+    names = {tw.SHAPE_BS4: "tw_gemm_bs_kernel", tw.SHAPE_BS8: "tw_gemm_bw_kernel", tw.SHAPE_256x128: "tw_gemm_ws_kernel 256x128"}
+
+    def launch(plan, shape, pruned, act, per_cu=-1):
+        dC = torch.full((N, ldc), SENTINEL, dtype=torch.int16, device="cuda")
+        tw.set_option(tw.OPT_SHAPE, shape)
+        tw.set_option(tw.OPT_WGS_PER_CU, per_cu)
+        print("weight-stationary kernels: case", case, "shape", shape, pruned, act, per_cu, dtype, flush=True)
+        assert plan.kernel_name(M, lda, ldc, activation=act) == names[shape]
+        plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=0.5, pruned_cols=pruned, bias_ptr=dbias.data_ptr(),
+                  activation=act, stream=s)
+        torch.cuda.synchronize()
+        return dC
+
+    try:
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            for pruned, act in ((tw.PRUNED_UNTOUCHED, tw.ACT_NONE), (tw.PRUNED_ZERO, tw.ACT_RELU), (tw.PRUNED_ZERO, tw.ACT_GELU),
+                                (tw.PRUNED_UNTOUCHED, tw.ACT_TANH)):
+                want = launch(plan, tw.SHAPE_256x128, pruned, act)
+                for shape in (tw.SHAPE_BS4, tw.SHAPE_BS8):
+                    if shape == tw.SHAPE_BS4 and max(kt for kt, _ in spec) > 192:
+                        continue
+                    for per_cu in (-1, 1, 4):
+                        got = launch(plan, shape, pruned, act, per_cu)
+                        if act in (tw.ACT_GELU, tw.ACT_TANH):
+                            a, b = got[:, :M].view(tdt).float(), want[:, :M].view(tdt).float()
+                            assert bool(((a - b).abs() <= ulp * b.abs() + 1e-7).all())
+                            assert torch.equal(got[:, M:], want[:, M:])
+                        else:
+                            assert torch.equal(got, want), (shape, pruned, act, per_cu)
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+        tw.set_option(tw.OPT_WGS_PER_CU, -1)
+
+
+@pytest.mark.parametrize("M,N,kept,act,kernel", [
+    (8192, 4096, 60, "none", "tw_gemm_bs_kernel"),    # one step, 64 MB of output, little but stores
+    (8192, 4096, 60, "gelu", "tw_gemm_bw_kernel"),
+    (16384, 4096, 120, "relu", "tw_gemm_bs_kernel"),  # 128 MB
+    (8192, 4096, 256, "none", "tw_gemm_bw_kernel"),   # four steps
+])
+def test_which_weight_stationary_kernel_runs(tw, M, N, kept, act, kernel):
+    """The automatic choice between the two (what test_both_weight_stationary_kernels forces runs by itself at these sizes)."""
+    K, G = 1024, 128
+    tiles = make_tiles(np.random.default_rng(3), K, G, ((kept, G),) * (N // G))
+    with tw.Plan.create(K, N, "bf16", tiles, np.zeros((K, N), np.float32)) as plan:
+        assert plan.choice(M)["shape"] == tw.SHAPE_BS
+        assert plan.kernel_name(M, activation={"none": tw.ACT_NONE, "relu": tw.ACT_RELU, "gelu": tw.ACT_GELU}[act]) == kernel

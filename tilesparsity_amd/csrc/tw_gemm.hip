@@ -2371,6 +2371,9 @@ static const Shape kShapes[TW_N_SHAPES] = {
     {32, 128, 1},  // TW_SHAPE_AS32
     {32, 128, 1},  // TW_SHAPE_SKINNY
     {64, 128, 3},  // TW_SHAPE_BS
+    {64, 128, 2},  // TW_SHAPE_BS4
+    {64, 128, 1},  // TW_SHAPE_BS8
+    {64, 128, 1},  // TW_SHAPE_RM
 };
 
 // LDS of the A-stationary kernel: the panel (all K rows, BMS rows m) and a C stage per wave
@@ -2381,7 +2384,7 @@ static bool is_as_shape(int shape) { return shape == TW_SHAPE_AS64 || shape == T
 // shapes that walk the plan's units themselves: no work queue, no unit pieces
 static bool is_queueless_shape(int shape)
 {
-    return is_as_shape(shape) || shape == TW_SHAPE_SKINNY || shape == TW_SHAPE_BS;
+    return is_as_shape(shape) || (shape >= TW_SHAPE_SKINNY && shape <= TW_SHAPE_BS8);
 }
 
 // Steps of loads a moving wave keeps in flight, per shape (bounded by its 256 registers: a step
@@ -2694,7 +2697,13 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
         // (forced, up to 192 kept rows as ever; longer tiles are the rule's to give)
         if (plan->max_k_pad <= 192 && bs_takes(plan, lda, ldc, reads_c))
             c.shape = f_shape;
-    } else if (f_shape >= 0 && (f_shape != TW_SHAPE_WIDE ? ws_ok : true)) {
+    } else if (f_shape == TW_SHAPE_BS4) {
+        if (plan->max_k_pad <= 192 && bs_takes(plan, lda, ldc, reads_c))
+            c.shape = f_shape;
+    } else if (f_shape == TW_SHAPE_BS8) {
+        if (bw_takes(plan, lda, ldc, reads_c))
+            c.shape = f_shape;
+    } else if (f_shape >= 0 && f_shape != TW_SHAPE_RM && (f_shape != TW_SHAPE_WIDE ? ws_ok : true)) {
         const int piece = f_piece > 0 ? f_piece : std::min(128, kShapes[f_shape].bn);
         if (std::min(piece, width) <= kShapes[f_shape].bn) {
             c.shape = f_shape;
@@ -2746,8 +2755,11 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
 // kept: 0.92 - 1.3 of the time).
 bool streams_row_major(const tw_plan *plan, int M, int64_t lda, float beta)
 {
-    if (option(TW_OPT_SHAPE) != -1 || !rm_takes(plan, M, lda)) // (a forced shape keeps the paths around the K-major kernels)
+    const int forced = option(TW_OPT_SHAPE); // (any other forced shape keeps the paths around the K-major kernels)
+    if ((forced != -1 && forced != TW_SHAPE_RM) || !rm_takes(plan, M, lda))
         return false;
+    if (forced == TW_SHAPE_RM)
+        return true;
     const int64_t groups = rm_groups(plan), wgs = (((int64_t)M + kRmRowsPerWg - 1) / kRmRowsPerWg) * groups;
     if (takes_row_major_directly(plan, beta))
         return plan->K >= 1024 && wgs * 8 >= (int64_t)plan->cu_count * 5 && wgs <= plan->cu_count &&
@@ -3040,8 +3052,8 @@ int launch_gemm(const tw_plan *plan, GemmArgs &a, const Choice &c, int32_t *tick
     }
     if (c.shape == TW_SHAPE_SKINNY)
         return plan->dtype == TW_F16 ? launch_skinny<TW_F16, false>(plan, a, s) : launch_skinny<TW_BF16, false>(plan, a, s);
-    if (c.shape == TW_SHAPE_BS)
-        return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), s);
+    if (c.shape == TW_SHAPE_BS || c.shape == TW_SHAPE_BS4 || c.shape == TW_SHAPE_BS8)
+        return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), c.shape == TW_SHAPE_BS ? bs_wide(plan, a.M, a.ldc, a.act) : c.shape == TW_SHAPE_BS8, s);
     // queue 0 is the longest: one workgroup per entry, up to the chip's share of a queue
     const int64_t qlen0 = (int64_t)a.n_own_items + (a.n_tail_items + kXcd - 1) / kXcd;
     const int64_t per_queue = std::max<int64_t>(1, (int64_t)plan->cu_count * c.per_cu / kXcd);
@@ -3080,6 +3092,34 @@ int static_scratch(int32_t **out)
     return TW_OK;
 }
 
+// which of the ways below a call takes
+enum class Route { KMAJOR, STREAM, SKINNY, PANEL, GENERIC };
+Route route_of(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, float beta)
+{
+    if (a_layout == TW_LAYOUT_KMAJOR && c_layout == TW_LAYOUT_KMAJOR)
+        return Route::KMAJOR;
+    if (a_layout != c_layout)
+        return Route::GENERIC;
+    if (streams_row_major(plan, M, lda, beta))
+        return Route::STREAM;
+    if (skinny_takes_row_major(plan, M, beta))
+        return Route::SKINNY;
+    if (takes_row_major_directly(plan, beta))
+        return Route::PANEL;
+    // (off the streaming kernel's range too: the layout-generic kernel is several times slower everywhere)
+    return option(TW_OPT_SHAPE) == -1 && rm_takes(plan, M, lda) ? Route::STREAM : Route::GENERIC;
+}
+
+// the panel kernel for row-major operands: 64-row panels where they fit and still give three quarters of the compute
+// units a workgroup
+bool row_major_panel_of_64(const tw_plan *plan, int M)
+{
+    const int mblk64 = (M + 63) / 64;
+    const int groups64 =
+        std::min(std::max(1, plan->cu_count / mblk64), (plan->n_blocks + as_task_waves(64, true) - 1) / as_task_waves(64, true));
+    return as_lds_bytes(plan->K, 64) <= kLdsBytes && (int64_t)mblk64 * groups64 * 4 >= (int64_t)plan->cu_count * 3;
+}
+
 // tw_gemm_ex and tw_gemm_static: the latter brings the counters (the library's `scratch` array),
 // cleared on the stream before the launch; the former takes a ticket slot of the plan.
 int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, void *C, int c_layout,
@@ -3092,9 +3132,8 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return st;
     GemmArgs a;
     fill_common(a, plan, A, lda, C, ldc, M, alpha, beta, ep);
-    const bool row_major = a_layout == TW_LAYOUT_ROWMAJOR && c_layout == TW_LAYOUT_ROWMAJOR;
-    const bool streams = row_major && streams_row_major(plan, M, lda, beta);
-    if (row_major && !streams && skinny_takes_row_major(plan, M, beta)) {
+    const Route route = route_of(plan, M, a_layout, lda, c_layout, beta);
+    if (route == Route::SKINNY) {
         fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false);
         if (a.n_all_u == 0)
             return TW_OK;
@@ -3104,26 +3143,20 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         hipStream_t s = (hipStream_t)stream;
         return plan->dtype == TW_F16 ? launch_skinny<TW_F16, true>(plan, a, s) : launch_skinny<TW_BF16, true>(plan, a, s);
     }
-    if (row_major && !streams && takes_row_major_directly(plan, beta)) {
+    if (route == Route::PANEL) {
         // both operands row-major, K short enough for a panel of A in LDS, C not read: the
-        // A-stationary kernel in its row-major form (64-row panels where they fit and still give
-        // three quarters of the compute units a workgroup)
+        // A-stationary kernel in its row-major form
         fill_queues(a, plan, M, 64, 128, pruned_cols, false);
         a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
         for (int i = 0; i < a.n_arg_units; ++i)
             a.arg_units[i] = plan->h_units[i];
-        const int mblk64 = (M + 63) / 64;
-        const int groups64 =
-            std::min(std::max(1, plan->cu_count / mblk64), (plan->n_blocks + as_task_waves(64, true) - 1) / as_task_waves(64, true));
-        const bool b64 = as_lds_bytes(plan->K, 64) <= kLdsBytes &&
-                         (int64_t)mblk64 * groups64 * 4 >= (int64_t)plan->cu_count * 3;
+        const bool b64 = row_major_panel_of_64(plan, M);
         hipStream_t s = (hipStream_t)stream;
         if (plan->dtype == TW_F16)
             return b64 ? launch_as<TW_F16, 64, true>(plan, a, M, s) : launch_as<TW_F16, 32, true>(plan, a, M, s);
         return b64 ? launch_as<TW_BF16, 64, true>(plan, a, M, s) : launch_as<TW_BF16, 32, true>(plan, a, M, s);
     }
-    if (streams || (row_major && option(TW_OPT_SHAPE) == -1 && rm_takes(plan, M, lda))) {
-        // (off the rule's range too: the layout-generic kernel is several times slower everywhere)
+    if (route == Route::STREAM) {
         fill_queues(a, plan, M, kRmRowsPerWg, 128, pruned_cols, false);
         if (a.n_all_u == 0)
             return TW_OK;
@@ -3133,7 +3166,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         const int pst = prepare_device();
         return pst != TW_OK ? pst : launch_rm(plan, a, (hipStream_t)stream);
     }
-    if (a_layout != TW_LAYOUT_KMAJOR || c_layout != TW_LAYOUT_KMAJOR) {
+    if (route == Route::GENERIC) {
         // layout-generic path (element strides), 128-row blocks, one workgroup per item; as many launches as the
         // grid's threads ask for
         fill_queues(a, plan, M, 128, 128, pruned_cols, false);
@@ -3233,6 +3266,34 @@ int tw_gemm_choice(const tw_plan *plan, int M, int64_t lda, int64_t ldc, float b
     choice[2] = c.per_cu;
     choice[3] = c.xcd ? 1 : 0;
     return TW_OK;
+}
+
+const char *tw_gemm_kernel_name(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, int64_t ldc, float beta,
+                                int activation)
+{
+    auto unknown = [](int layout) { return layout != TW_LAYOUT_KMAJOR && layout != TW_LAYOUT_ROWMAJOR; };
+    if (!plan || M < 0 || unknown(a_layout) || unknown(c_layout))
+        return nullptr;
+    switch (route_of(plan, M, a_layout, lda, c_layout, beta)) {
+    case Route::STREAM:
+        return "tw_gemm_rm_kernel";
+    case Route::SKINNY:
+        return "tw_gemm_skinny_kernel row-major";
+    case Route::PANEL:
+        return row_major_panel_of_64(plan, M) ? "tw_gemm_as_kernel 64 rows row-major" : "tw_gemm_as_kernel 32 rows row-major";
+    case Route::GENERIC:
+        return "tw_gemm_generic_kernel";
+    case Route::KMAJOR:
+        break;
+    }
+    static const char *const names[] = {"tw_gemm_kmajor_kernel 256x128", "tw_gemm_ws_kernel 128x128", "tw_gemm_ws_kernel 512x64",
+                                        "tw_gemm_ws_kernel 128x64",      "tw_gemm_ws_kernel 256x128", "tw_gemm_ws_kernel 128x32",
+                                        "tw_gemm_ws_kernel 256x64",      "tw_gemm_as_kernel 64 rows", "tw_gemm_as_kernel 32 rows",
+                                        "tw_gemm_skinny_kernel"};
+    const int shape = choose_shape(plan, M, lda, ldc, beta != 0.0f).shape;
+    if (shape < TW_SHAPE_BS)
+        return names[shape];
+    return shape == TW_SHAPE_BS8 || (shape == TW_SHAPE_BS && bs_wide(plan, M, ldc, activation)) ? "tw_gemm_bw_kernel" : "tw_gemm_bs_kernel";
 }
 
 int tw_plan_reset(tw_plan *plan, void *stream)

@@ -639,16 +639,21 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
     }
 }
 
-bool bs_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
+bool bw_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
 {
     if (reads_c || plan->n_units == 0 || plan->n_pipe_units == 0 || (int64_t)plan->n_units * 1024 > kMaxGridThreads)
         return false;
-    // A is addressed through a buffer descriptor with 32-bit offsets
-    if ((uint64_t)plan->K * (uint64_t)lda * 2u >= (1ull << 32))
-        return false;
-    // (and the wider form stores C through one)
-    return plan->max_k_pad <= kBsMaxSteps * kBlockK ||
-           (plan->max_k_pad <= kBwSteps * kBlockK && (uint64_t)plan->N * (uint64_t)ldc * 2u < kBwMaxBytes);
+    // A is addressed, and C stored, through a buffer descriptor with 32-bit offsets
+    return (uint64_t)plan->K * (uint64_t)lda * 2u < (1ull << 32) && plan->max_k_pad <= kBwSteps * kBlockK &&
+           (uint64_t)plan->N * (uint64_t)ldc * 2u < kBwMaxBytes;
+}
+
+bool bs_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)
+{
+    if (bw_takes(plan, lda, ldc, reads_c))
+        return true;
+    // (the four-wave kernel stores C by address: any size of it)
+    return plan->max_k_pad <= kBsMaxSteps * kBlockK && bw_takes(plan, lda, 0, reads_c);
 }
 
 // ranges of rows of A a launch is cut into: as many as give every compute unit `per_cu`
@@ -715,24 +720,30 @@ template <int DT, int NS> static int launch_bw(const tw_plan *plan, const GemmAr
     return TW_OK;
 }
 
-int launch_bs(const tw_plan *plan, const GemmArgs &a, int per_cu, hipStream_t s)
+// Up to three steps either kernel takes the plan.  Without a long activation, where the launch is little but its stores, the
+// one whose waves store 64 rows themselves is ahead where its workgroups, two to a compute unit, come out even: beyond 112
+// MB of output (M 16384, N 4096, 120 kept rows: 38.5 against 47.1 us; M 14336: 34.5 against 29.5; with GELU 54.9 against
+// 50.1; 34, 39 or 44 units, which leave it a third of the chip, 1.1 - 1.4 of the time of what ran before), and with one step
+// from 32 MB on (60 kept: M 8192, N 4096 18.9 against 22.7, M 8192, N 2048 12.1 against 13.9; M 8192, N 3072, not even, 19.9
+// against 16.9).
+bool bs_wide(const tw_plan *plan, int M, int64_t ldc, int act)
+{
+    const int ns = std::max(1, plan->max_k_pad / kBlockK);
+    const int64_t out_bytes = (int64_t)M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, M, 2);
+    const int64_t slots2 = 2 * (int64_t)plan->cu_count, all2 = (wgs2 + slots2 - 1) / slots2 * slots2;
+    const bool stores_only = (act == TW_ACT_NONE || act == TW_ACT_RELU) &&
+                             ((out_bytes > (int64_t)112 << 20 && wgs2 * 4 >= all2 * 3) ||
+                              (ns == 1 && out_bytes >= (int64_t)32 << 20 && wgs2 * 10 >= all2 * 9));
+    return ns > kBsMaxSteps || !(stores_only || (uint64_t)plan->N * (uint64_t)ldc * 2u >= kBwMaxBytes);
+}
+
+int launch_bs(const tw_plan *plan, const GemmArgs &a, int per_cu, bool wide, hipStream_t s)
 {
     // (per_cu <= 0: as many workgroups per compute unit as the kernel is built for)
     const int ns = std::max(1, plan->max_k_pad / kBlockK);
     const int pc = per_cu > 0 ? per_cu : kBsPerCu;
     const bool f16 = plan->dtype == TW_F16;
-    // Up to three steps either kernel takes the plan.  Without a long activation, where the launch is little but its stores, the
-    // one whose waves store 64 rows themselves is ahead where its workgroups, two to a compute unit, come out even: beyond 112
-    // MB of output (M 16384, N 4096, 120 kept rows: 38.5 against 47.1 us; M 14336: 34.5 against 29.5; with GELU 54.9 against
-    // 50.1; 34, 39 or 44 units, which leave it a third of the chip, 1.1 - 1.4 of the time of what ran before), and with one step
-    // from 32 MB on (60 kept: M 8192, N 4096 18.9 against 22.7, M 8192, N 2048 12.1 against 13.9; M 8192, N 3072, not even, 19.9
-    // against 16.9).
-    const int64_t out_bytes = (int64_t)a.M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, a.M, 2);
-    const int64_t slots2 = 2 * (int64_t)plan->cu_count, all2 = (wgs2 + slots2 - 1) / slots2 * slots2;
-    const bool stores_only = (a.act == TW_ACT_NONE || a.act == TW_ACT_RELU) &&
-                             ((out_bytes > (int64_t)112 << 20 && wgs2 * 4 >= all2 * 3) ||
-                              (ns == 1 && out_bytes >= (int64_t)32 << 20 && wgs2 * 10 >= all2 * 9));
-    if (ns <= 3 && (stores_only || (uint64_t)plan->N * (uint64_t)a.ldc * 2u >= kBwMaxBytes)) {
+    if (!wide) {
         if (ns <= 2)
             return f16 ? launch_bs_t<TW_F16, 2>(plan, a, pc, s) : launch_bs_t<TW_BF16, 2>(plan, a, pc, s);
         return f16 ? launch_bs_t<TW_F16, 3>(plan, a, pc, s) : launch_bs_t<TW_BF16, 3>(plan, a, pc, s);
