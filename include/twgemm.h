@@ -290,8 +290,9 @@ int tw_gemm_static(const tw_plan *plan, const void *A, int a_layout, int64_t lda
  * operator multiplies a row-major x[M,K] into a row-major result (mask_dense,
  * Pruning/BERT/utils/modeling.py:992-1007).  tw_gemm_ex takes such operands as they are when both
  * are row-major and either K <= 2128 and beta == 0 (a kernel that keeps a panel of A in LDS) or M is small
- * enough for the kernel for few rows (any K and beta; a rule on workgroups per compute unit), and else
- * through a layout-generic kernel that gathers 2-byte elements.  Here, in those other cases, a row-major A is first turned into
+ * enough for the kernel for few rows (any K and beta; a rule on workgroups per compute unit), else through a
+ * kernel that streams whole rows of A, or a layout-generic one that gathers 2-byte elements (short lists of a long K,
+ * mixed layouts).  Here, in those other cases, the streaming kernel runs where it is estimated to be ahead, and else a row-major A is first turned into
  * its K-major copy and a row-major C is produced K-major and turned back, both in `workspace`
  * (device memory, 16-byte aligned, at least tw_gemm_staged_workspace(plan, M, a_layout, c_layout)
  * bytes: 2 * round_up(M, 64) * (K for a row-major A + N for a row-major C)); one more pass over
@@ -361,7 +362,8 @@ int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda
  * fixed at compile time, basic_nn.cu:250-259; benchmarks name the kernel they timed with it.) */
 int tw_gemm_choice(const tw_plan *plan, int M, int64_t lda, int64_t ldc, float beta, int32_t *choice);
 /* Name of the kernel tw_gemm_ex runs for these arguments, in any layout, under the options in force (a static string; NULL
- * for a NULL plan, M < 0 or an unknown layout).  tw_gemm_staged runs the same one where it stages nothing. */
+ * for a NULL plan, M < 0 or an unknown layout).  tw_gemm_staged, which has its copies to fall back on, runs that kernel or
+ * makes them. */
 const char *tw_gemm_kernel_name(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, int64_t ldc, float beta,
                                 int activation);
 int tw_set_option(int option, int value);

@@ -1272,6 +1272,82 @@ def test_row_major_streaming_nonfinite(tw, oracle):
     assert float((r[fin].float() - k[fin].float()).abs().max()) <= 2e-3 * float(k[fin].float().abs().max())
 
 
+@pytest.mark.parametrize("M,K,N,G,k_keep,n_keep,act,dtype", [
+    (300, 2203, 1530, 128, 0.25, 0.9, "gelu", "f16"),    # ragged; 12 units, read from the arguments
+    (130, 2500, 4400, 128, 0.2, 1.0, "tanh", "bf16"),    # 35 units: read from memory
+    (200, 2300, 2200, 64, 0.02, 0.9, "gelu", "bf16"),    # units of at most 64 columns, a wave each; groups cut
+    (70, 3000, 330, 64, 0.01, 1.0, "relu", "f16"),
+    (64, 100, 128, 128, 0.5, 1.0, "none", "bf16"),       # one chunk of K, one unit: waves and loading waves without work
+    (65, 260, 200, 32, 0.9, 0.8, "tanh", "f16"),
+    (4096, 1024, 1024, 128, 0.25, 1.0, "gelu", "f16"),
+])
+def test_row_major_streaming_forced(tw, oracle, M, K, N, G, k_keep, n_keep, act, dtype):
+    """The row-major streaming kernel wherever it can run, forced and named: every activation, bias, alpha, C read and not read,
+    pruned columns filled and left alone, tiles without kept rows.  Sampled rows against the oracle."""
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    tiles = random_tiles(rng, K, N, G, k_keep=k_keep, n_keep=n_keep, empty_every=5)
+    keep = kept_columns(tiles, N)
+    lda, ldc = round_up(K, 8) + 8, round_up(N, 8) + 8
+    Ah, Ch = np.full((M, lda), 0x7e00 if dtype == "f16" else 0x7fc0, np.uint16), np.full((M, ldc), SENTINEL, np.uint16)
+    Ah[:, :K] = oracle.cast_bits(A, dtype).reshape(M, K)
+    Ch[:, :N] = oracle.cast_bits(C0, dtype).reshape(M, N)
+    dA, d_bias = to_device_bits(Ah, Ah.shape), torch.from_numpy(bias).cuda()
+    code = {"none": tw.ACT_NONE, "relu": tw.ACT_RELU, "gelu": tw.ACT_GELU, "tanh": tw.ACT_TANH}[act]
+    rows = np.unique(np.concatenate([np.arange(min(M, 40)), np.arange(max(0, M - 70), M), rng.choice(M, 20)]))
+    row = dict(a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+    try:
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            tw.set_option(tw.OPT_SHAPE, tw.SHAPE_RM)
+            for alpha, beta, pruned in ((0.75, 0.0, tw.PRUNED_UNTOUCHED), (1.0, 0.5, tw.PRUNED_ZERO)):
+                assert plan.kernel_name(M, lda, ldc, beta=beta, activation=code, **row) == "tw_gemm_rm_kernel"
+                dC = to_device_bits(Ch, Ch.shape)
+                print("row-major streaming, forced:", M, K, N, G, beta, act, dtype, flush=True)
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=alpha, beta=beta, pruned_cols=pruned,
+                          bias_ptr=d_bias.data_ptr(), activation=code, **row)
+                torch.cuda.synchronize()
+                out = from_device_bits(dC)
+                assert np.all(out[:, N:] == SENTINEL)
+                pre = alpha * reference(oracle, A[rows], B, tiles, dtype).astype(np.float64)
+                want = oracle.ACTIVATIONS[act](pre + beta * oracle.quantize(C0[rows], dtype) + bias)
+                got = oracle.bits_to_f32(np.ascontiguousarray(out[rows, :N]), dtype).reshape(rows.size, N)
+                assert oracle.rel_error(got[:, keep], want[:, keep]) <= TOL[dtype]
+                if pruned == tw.PRUNED_UNTOUCHED:
+                    assert np.array_equal(out[:, :N][:, ~keep], Ch[:, :N][:, ~keep])
+                elif not np.all(keep):
+                    assert oracle.rel_error(got[:, ~keep], want[:, ~keep]) <= TOL[dtype]
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+
+
+ROUTES = [
+    # M, K, N, G, kept rows, beta, workspace -> kernel.  The ways a row-major call takes at both sides of their lines
+    (4096, 3072, 768, 128, 768, 0.0, "tw_gemm_rm_kernel"),                 # BERT-base's second layer
+    (4096, 1024, 1024, 128, 256, 0.0, "tw_gemm_as_kernel 64 rows row-major"),
+    (4096, 2048, 1024, 128, 512, 0.0, "tw_gemm_as_kernel 32 rows row-major"),
+    (1863, 3544, 856, 128, 7, 0.0, "tw_gemm_skinny_kernel row-major"),     # (hardly any row kept, short walks)
+    (2048, 3072, 768, 128, 768, 0.0, "tw_gemm_skinny_kernel row-major"),
+    (2600, 3072, 768, 128, 768, 0.0, "tw_gemm_rm_kernel"),
+    (128, 3072, 768, 128, 768, 0.0, "tw_gemm_skinny_kernel row-major"),
+    (6123, 3536, 5248, 128, 18, 0.0, "tw_gemm_generic_kernel"),            # staged where there is a workspace
+    (2968, 3352, 2608, 64, 1676, 0.0, "tw_gemm_rm_kernel"),                # (the same: without one)
+    (6000, 400, 2000, 128, 100, 0.5, "tw_gemm_rm_kernel"),
+    (6000, 3300, 2000, 128, 40, 0.5, "tw_gemm_generic_kernel"),
+]
+
+
+@pytest.mark.parametrize("M,K,N,G,kept,beta,kernel", ROUTES)
+def test_which_kernel_takes_row_major_operands(tw, M, K, N, G, kept, beta, kernel):
+    tiles = [dict(col0=c, width=min(G, N - c), kept_k=np.arange(kept, dtype=np.int32), kept_n=np.arange(min(G, N - c), dtype=np.int32))
+             for c in range(0, N, G)]
+    with tw.Plan.create(K, N, "f16", tiles, np.zeros((K, N), np.float32)) as plan:
+        assert plan.kernel_name(M, K, N, tw.ROWMAJOR, tw.ROWMAJOR, beta=beta) == kernel
+
+
 @pytest.mark.parametrize("staged,M", [(False, 8), (True, 8), (False, 8200)])
 def test_row_major_operands_with_more_units_than_a_grid_has_rows(tw, staged, M):
     """262208 tiles of one column: more groups of units than the second dimension of a grid has.  Row-major calls of such a

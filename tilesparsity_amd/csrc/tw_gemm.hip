@@ -30,6 +30,7 @@
 #include <atomic>
 #include <mutex>
 #include <type_traits>
+#include <cmath>
 #include <cstddef>
 #include <cstdlib>
 
@@ -2725,7 +2726,7 @@ bool takes_row_major_directly(const tw_plan *plan, float beta)
 }
 
 // the skinny kernel in its row-major form: where it is taken for K-major copies of the operands
-bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
+static bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
 {
     // Against the staged copies it is ahead wherever the rule takes it (K 3072, N 768, M 128: 6.7 against
     // 10.5 us; M 2048: 21.0 against 26.5).  Against the A-stationary kernel's row-major form, while its
@@ -2742,30 +2743,58 @@ bool skinny_takes_row_major(const tw_plan *plan, int M, float beta)
     return choose_shape(plan, M, ld, ld, beta != 0.0f, true).shape == TW_SHAPE_SKINNY;
 }
 
-// The row-major streaming kernel for row-major operands.  Measured (us a launch of a replayed graph, before and with it)
-// on M 256 .. 16384, K 768 .. 4608, N 256 .. 3072, 10 / 25 / 50 % of the rows kept, tiles of 64 and 128 columns.  Its time
-// is that of a round of workgroups (64 rows x 256 columns: 13 - 25 us by K and kept rows) times rounds:
-// Against the skinny kernel and the copies around the streaming kernels (no panel of A in LDS), from 96 workgroups on
-// (K 3072, N 768, M 2048, a quarter kept: 22 -> 15; M 4096: 33 -> 17; K 4608, N 512, M 12544: 82 -> 46; 64 workgroups,
-// K 4608, N 512, M 2048: 18 -> 20), 128 where tiles of 64 columns keep more than 1024 rows (K 4096, N 1024, half kept,
-// 96 workgroups: 1.06 of the time); not for many columns under many rows, where turning A once is cheaper than
-// streaming all of it for every 256 columns (K 2560, N 2560, M 16384: 141 -> 165; M 4096, 640 workgroups: 49 -> 41).
-// Against the panel, where one round fills the chip (K 2048, N 1024, M 4096: 20 -> 16; K 1024, N 1024, M 4096: 14 -> 12;
-// 128 workgroups: 1.05 of the time; two rounds, M 8192: 1.0 - 1.14) and the tiles are no shorter than a fifth of K (a tenth
-// kept: 0.92 - 1.3 of the time).
-bool streams_row_major(const tw_plan *plan, int M, int64_t lda, float beta)
+// Whether the row-major streaming kernel is ahead of the other ways for row-major operands that no panel of A takes.  The lines
+// come from 9000 problems, each way timed (replayed graphs): M 64 .. 16384, K 512 .. 5000, N 128 .. 8192, 0.2 - 80 % of
+// the rows kept, all or 80 - 90 % of the columns, tiles of 64, 128 and 256 columns, with and without beta.
+// - A panel of A in LDS (K up to 2128, C not read) is as fast or ahead: the 110 problems where the chip is just full and a fifth
+//   and more of the rows kept take 1.01 of its time in the mean (0.8 - 1.8; K 1024, N 1024, M 4096: 0.9).
+// - The kernel for few rows, where that is taken: from 9 workgroups for 20 compute units and long walks of that
+//   kernel on (38 problems: 0.83 of its time, at most 1.09; everything from 3 for 8 on: 1.09 in the mean, to 3.0), not for units of
+//   64 columns (1.0 - 1.3).
+// - The copies around a K-major kernel: by the estimates below of both, in us, which are within 25 % of what 9 of 10 problems
+//   take.  The margin is for what they do not know: of 1586 problems 1023 are taken at 0.64 of the time in the mean and ten of
+//   them lose more than 4 % (14 % at most; on 3000 others, 13 and 20 %); all from 3 workgroups for 8 compute units on would be 1290 at 0.73, of which 163
+//   lose more than 4 % (to 1.9 of the time: hardly any row kept, or many columns under a long K, where turning A once is
+//   cheaper than streaming all of it for every 256 columns).
+static double streaming_us(const tw_plan *plan, int M, float beta)
+{
+    const bool narrow = plan->max_unit_n <= 64;
+    const double cu = plan->cu_count, fill = (double)((M + kRmRowsPerWg - 1) / kRmRowsPerWg) * rm_groups(plan) / cu;
+    const double rounds = std::max(1.0, 0.5 * (fill + std::ceil(fill))), chunks = (plan->K + 127) / 128;
+    const double steps = (double)plan->pipe_steps / std::max(1, plan->n_pipe_units);
+    const double sparse = std::max(0.0, chunks - 6.0 * steps); // chunks beyond what the lists fill: their groups are cut
+    const int element_wise = (plan->n_zero_tiles > 0) + (beta != 0.0f);
+    return rounds * (13.0 + std::min(1.0, fill) * (0.08 * chunks + 2.5 * element_wise) + (narrow ? 1.1 : 0.65) * steps + 0.3 * sparse);
+}
+
+static double staged_us(const tw_plan *plan, int M, float beta)
+{
+    const double steps = (double)plan->pipe_steps / std::max(1, plan->n_pipe_units);
+    const double items = (double)std::max(1, plan->n_pipe_units) * ((M + 255) / 256) / plan->cu_count;
+    const double rounds = std::max(1.0, 0.5 * (items + std::ceil(items))), m = M * 1e-6;
+    return 19.0 + m * (0.8 * plan->K + (beta != 0.0f ? 5.5 : 1.7) * plan->N) + rounds * steps * (plan->max_unit_n <= 64 ? 0.7 : 0.8);
+}
+
+static bool streaming_is_ahead(const tw_plan *plan, int M, float beta, bool skinny)
+{
+    const bool narrow = plan->max_unit_n <= 64;
+    const int64_t wgs = (((int64_t)M + kRmRowsPerWg - 1) / kRmRowsPerWg) * rm_groups(plan);
+    if (!skinny)
+        return streaming_us(plan, M, beta) < (narrow ? 0.8 : 0.85) * staged_us(plan, M, beta);
+    SkinnyWork w;
+    return !narrow && wgs * 20 >= (int64_t)plan->cu_count * 9 && skinny_work(plan, M, &w) >= 0 &&
+           skinny_load(plan, w) * plan->pipe_steps >= 25.0 * std::max(1, plan->n_pipe_units);
+}
+
+RowMajor row_major_kernel(const tw_plan *plan, int M, int64_t lda, float beta)
 {
     const int forced = option(TW_OPT_SHAPE); // (any other forced shape keeps the paths around the K-major kernels)
-    if ((forced != -1 && forced != TW_SHAPE_RM) || !rm_takes(plan, M, lda))
-        return false;
-    if (forced == TW_SHAPE_RM)
-        return true;
-    const int64_t groups = rm_groups(plan), wgs = (((int64_t)M + kRmRowsPerWg - 1) / kRmRowsPerWg) * groups;
-    if (takes_row_major_directly(plan, beta))
-        return plan->K >= 1024 && wgs * 8 >= (int64_t)plan->cu_count * 5 && wgs <= plan->cu_count &&
-               plan->pipe_steps * kBlockK * 5 >= (int64_t)plan->K * std::max(1, plan->n_pipe_units);
-    const bool long_narrow = plan->max_unit_n <= 64 && plan->pipe_steps * kBlockK > (int64_t)1024 * std::max(1, plan->n_pipe_units);
-    return wgs * 8 >= (int64_t)plan->cu_count * (long_narrow ? 4 : 3) && (groups <= 6 || wgs <= 4 * (int64_t)plan->cu_count);
+    if (forced == TW_SHAPE_RM && rm_takes(plan, M, lda))
+        return RowMajor::STREAM;
+    const bool panel = takes_row_major_directly(plan, beta), skinny = skinny_takes_row_major(plan, M, beta);
+    if (!panel && forced == -1 && rm_takes(plan, M, lda) && streaming_is_ahead(plan, M, beta, skinny))
+        return RowMajor::STREAM;
+    return skinny ? RowMajor::SKINNY : panel ? RowMajor::PANEL : RowMajor::NONE;
 }
 
 template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, const GemmArgs &a, int M, hipStream_t s)
@@ -3092,22 +3121,26 @@ int static_scratch(int32_t **out)
     return TW_OK;
 }
 
-// which of the ways below a call takes
+// which of the ways below a call takes (`staged`: the caller would make copies rather than take the layout-generic kernel)
 enum class Route { KMAJOR, STREAM, SKINNY, PANEL, GENERIC };
-Route route_of(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, float beta)
+Route route_of(const tw_plan *plan, int M, int a_layout, int64_t lda, int c_layout, float beta, bool staged)
 {
     if (a_layout == TW_LAYOUT_KMAJOR && c_layout == TW_LAYOUT_KMAJOR)
         return Route::KMAJOR;
     if (a_layout != c_layout)
         return Route::GENERIC;
-    if (streams_row_major(plan, M, lda, beta))
-        return Route::STREAM;
-    if (skinny_takes_row_major(plan, M, beta))
+    const RowMajor kernel = row_major_kernel(plan, M, lda, beta);
+    if (kernel == RowMajor::SKINNY)
         return Route::SKINNY;
-    if (takes_row_major_directly(plan, beta))
+    if (kernel == RowMajor::PANEL)
         return Route::PANEL;
-    // (off the streaming kernel's range too: the layout-generic kernel is several times slower everywhere)
-    return option(TW_OPT_SHAPE) == -1 && rm_takes(plan, M, lda) ? Route::STREAM : Route::GENERIC;
+    if (option(TW_OPT_SHAPE) != -1 || staged)
+        return kernel == RowMajor::STREAM ? Route::STREAM : Route::GENERIC;
+    // Without a workspace the streaming kernel takes 0.47 of the layout-generic kernel's time (403 problems), but not where the
+    // tiles keep a step of 64 rows or less of a long K: C not read (K is over 2128 then) 1.0 - 1.95, C read 0.4 - 1.1,
+    // from K 2200 on 0.7 - 1.45.
+    const bool few = plan->pipe_steps <= plan->n_pipe_units && (beta == 0.0f || plan->K >= 2200);
+    return !few && rm_takes(plan, M, lda) ? Route::STREAM : Route::GENERIC;
 }
 
 // the panel kernel for row-major operands: 64-row panels where they fit and still give three quarters of the compute
@@ -3124,7 +3157,7 @@ bool row_major_panel_of_64(const tw_plan *plan, int M)
 // cleared on the stream before the launch; the former takes a ticket slot of the plan.
 int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, void *C, int c_layout,
               int64_t ldc, int M, float alpha, float beta, int pruned_cols, const tw_epilogue *ep,
-              void *stream, bool use_static)
+              void *stream, bool use_static, bool staged = false)
 {
     bool run = false;
     const int st = check_gemm_args(plan, A, a_layout, lda, C, c_layout, ldc, M, pruned_cols, ep, &run);
@@ -3132,7 +3165,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return st;
     GemmArgs a;
     fill_common(a, plan, A, lda, C, ldc, M, alpha, beta, ep);
-    const Route route = route_of(plan, M, a_layout, lda, c_layout, beta);
+    const Route route = route_of(plan, M, a_layout, lda, c_layout, beta, staged);
     if (route == Route::SKINNY) {
         fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false);
         if (a.n_all_u == 0)
@@ -3274,7 +3307,7 @@ const char *tw_gemm_kernel_name(const tw_plan *plan, int M, int a_layout, int64_
     auto unknown = [](int layout) { return layout != TW_LAYOUT_KMAJOR && layout != TW_LAYOUT_ROWMAJOR; };
     if (!plan || M < 0 || unknown(a_layout) || unknown(c_layout))
         return nullptr;
-    switch (route_of(plan, M, a_layout, lda, c_layout, beta)) {
+    switch (route_of(plan, M, a_layout, lda, c_layout, beta, false)) {
     case Route::STREAM:
         return "tw_gemm_rm_kernel";
     case Route::SKINNY:
@@ -3395,3 +3428,9 @@ int tw_insert_row(void *matrix, const void *matrix_2, int rows, int columns, con
 }
 
 } // extern "C"
+
+int tw::gemm_staged_in_one_launch(const tw_plan *plan, const void *A, int64_t lda, void *C, int64_t ldc, int M, float alpha, float beta,
+                                  int pruned_cols, const tw_epilogue *ep, void *stream)
+{
+    return gemm_impl(plan, A, TW_LAYOUT_ROWMAJOR, lda, C, TW_LAYOUT_ROWMAJOR, ldc, M, alpha, beta, pruned_cols, ep, stream, false, true);
+}

@@ -187,8 +187,6 @@ void release_producer_memory();
 // true when tw_gemm_ex takes a row-major A and a row-major C of this plan with a kernel of its own
 // (no layout-generic kernel, no staging): K short enough for a panel of A in LDS and C not read
 bool takes_row_major_directly(const tw_plan *p, float beta);
-// ... and where its kernel for few rows of A takes them, whatever K and beta
-bool skinny_takes_row_major(const tw_plan *p, int M, float beta);
 // the weight-stationary kernel (tw_gemm_bs.hip): whether it takes the plan, and its launch with
 // `per_cu` workgroups meant to share a compute unit
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
@@ -204,7 +202,11 @@ int rm_groups(const tw_plan *p);
 bool rm_takes(const tw_plan *p, int M, int64_t lda);
 int launch_rm(const tw_plan *p, const GemmArgs &a, hipStream_t s);
 int prepare_rm();
-// true where tw_gemm_ex takes a row-major A and a row-major C of this plan with it
-bool streams_row_major(const tw_plan *p, int M, int64_t lda, float beta);
+// the kernel that takes a row-major A and a row-major C as they are, ahead of copies around a K-major one; NONE: none does
+enum class RowMajor { NONE, STREAM, SKINNY, PANEL };
+RowMajor row_major_kernel(const tw_plan *p, int M, int64_t lda, float beta);
+// tw_gemm_ex of two row-major operands for which that names a kernel
+int gemm_staged_in_one_launch(const tw_plan *plan, const void *A, int64_t lda, void *C, int64_t ldc, int M, float alpha, float beta,
+                              int pruned_cols, const tw_epilogue *ep, void *stream);
 
 } // namespace tw

@@ -119,8 +119,8 @@ try {
                     (long long)(workspace ? workspace_bytes : 0), (long long)need);
     if ((uintptr_t)workspace & 15)
         return fail(TW_ERR_ALIGNMENT, "the workspace must be 16-byte aligned");
-    if (a_rm && c_rm && (streams_row_major(plan, M, lda, beta) || skinny_takes_row_major(plan, M, beta))) // (one launch instead of three)
-        return tw_gemm_ex(plan, A, a_layout, lda, C, c_layout, ldc, M, alpha, beta, pruned_cols, ep, stream);
+    if (a_rm && c_rm && row_major_kernel(plan, M, lda, beta) != RowMajor::NONE) // (one launch instead of three)
+        return gemm_staged_in_one_launch(plan, A, lda, C, ldc, M, alpha, beta, pruned_cols, ep, stream);
     hipStream_t s = (hipStream_t)stream;
     const int64_t ldw = staged_ld(M);
     uint16_t *ws = static_cast<uint16_t *>(workspace);
