@@ -541,9 +541,14 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
             if (OLDER > 1 && (i == 2 || i == 3))
                 out[i - 2] = stage_get(parity ^ 1, i - 2);
             sum = E::mfma(af[i], bq[i >> 2][i & 3], sum);
-            if (OLDER > 1 && (i == NS * 4 - 2 || i == NS * 4 - 1))
-                __builtin_amdgcn_raw_buffer_store_b128(out[i - (NS * 4 - 2)], c_rsrc, (int)o_q[i - (NS * 4 - 2)], (mb - 2) * kBsRows * 2,
-                                                       1 | 2 | 16);
+            if (OLDER > 1 && (i == NS * 4 - 2 || i == NS * 4 - 1)) {
+                const int q = i - (NS * 4 - 2);
+                __builtin_amdgcn_raw_buffer_store_b128(out[q], c_rsrc, (int)o_q[q], (mb - 2) * kBsRows * 2, 1 | 2 | 16);
+                // Two wait states before the data's registers are written again: the store is still reading them, and the compiler
+                // adds none to a buffer store with a scalar offset (an instruction that wrote the second of the four
+                // at once put its own result into C).
+                asm volatile("s_nop 1" ::"v"(out[q]));
+            }
             if constexpr (OLDER > 0) {
                 // this product's share of the sixteen values of the block before; four of them go to the stage together
                 constexpr int P = NS < 4 ? NS * 4 : 16;
