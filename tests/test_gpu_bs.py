@@ -231,7 +231,7 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
     """The kernel of four multiplying waves (up to 192 kept rows) and the one of eight (up to 384), forced in turn: without
     activation and with ReLU bit for bit the streaming 256 x 128 kernel, with GELU and tanh one unit in the last place of the
     result (2^-10, 2^-7: the same sum, its activation from a different order of instructions), pruned columns filled and
-    left alone, few and many ranges of rows, the padding of C's rows untouched."""
+    left alone, few and many ranges of rows, C's columns at sectors of memory and off them, the padding of its rows untouched."""
     import torch
     M, K, G, spec = (CASES + WIDE_CASES)[case]
     N = G * len(spec)
@@ -240,7 +240,7 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
     B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
     dbias = torch.from_numpy(rng.standard_normal(N).astype(np.float32)).cuda()
     tiles = make_tiles(rng, K, G, spec)
-    lda = ldc = (M + 7) // 8 * 8 + 8
+    lda = (M + 7) // 8 * 8 + 8
     At = np.zeros((K, lda), np.uint16)
     At[:, :M] = oracle.cast_bits(A, dtype).reshape(M, K).T
     dA = to_device_bits(At, At.shape)
@@ -249,11 +249,11 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
     ulp = 2.0 ** -10 if dtype == "f16" else 2.0 ** -7
     names = {tw.SHAPE_BS4: "tw_gemm_bs_kernel", tw.SHAPE_BS8: "tw_gemm_bw_kernel", tw.SHAPE_256x128: "tw_gemm_ws_kernel 256x128"}
 
-    def launch(plan, shape, pruned, act, per_cu=-1):
+    def launch(plan, shape, ldc, pruned, act, per_cu=-1):
         dC = torch.full((N, ldc), SENTINEL, dtype=torch.int16, device="cuda")
         tw.set_option(tw.OPT_SHAPE, shape)
         tw.set_option(tw.OPT_WGS_PER_CU, per_cu)
-        print("weight-stationary kernels: case", case, "shape", shape, pruned, act, per_cu, dtype, flush=True)
+        print("weight-stationary kernels: case", case, "shape", shape, ldc, pruned, act, per_cu, dtype, flush=True)
         assert plan.kernel_name(M, lda, ldc, activation=act) == names[shape]
         plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=0.5, pruned_cols=pruned, bias_ptr=dbias.data_ptr(),
                   activation=act, stream=s)
@@ -262,14 +262,16 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
 
     try:
         with tw.Plan.create(K, N, dtype, tiles, B) as plan:
-            for pruned, act in ((tw.PRUNED_UNTOUCHED, tw.ACT_NONE), (tw.PRUNED_ZERO, tw.ACT_RELU), (tw.PRUNED_ZERO, tw.ACT_GELU),
-                                (tw.PRUNED_UNTOUCHED, tw.ACT_TANH)):
-                want = launch(plan, tw.SHAPE_256x128, pruned, act)
+            sectors, off = (M + 31) // 32 * 32, (M + 7) // 16 * 16 + 8
+            for ldc, pruned, act in ((off, tw.PRUNED_UNTOUCHED, tw.ACT_NONE), (sectors, tw.PRUNED_ZERO, tw.ACT_RELU),
+                                     (sectors, tw.PRUNED_UNTOUCHED, tw.ACT_NONE), (off, tw.PRUNED_ZERO, tw.ACT_GELU),
+                                     (sectors, tw.PRUNED_UNTOUCHED, tw.ACT_TANH)):
+                want = launch(plan, tw.SHAPE_256x128, ldc, pruned, act)
                 for shape in (tw.SHAPE_BS4, tw.SHAPE_BS8):
                     if shape == tw.SHAPE_BS4 and max(kt for kt, _ in spec) > 192:
                         continue
                     for per_cu in (-1, 1, 4):
-                        got = launch(plan, shape, pruned, act, per_cu)
+                        got = launch(plan, shape, ldc, pruned, act, per_cu)
                         if act in (tw.ACT_GELU, tw.ACT_TANH):
                             a, b = got[:, :M].view(tdt).float(), want[:, :M].view(tdt).float()
                             assert bool(((a - b).abs() <= ulp * b.abs() + 1e-7).all())
@@ -284,6 +286,7 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
 @pytest.mark.parametrize("M,N,kept,act,kernel", [
     (8192, 4096, 60, "none", "tw_gemm_bs_kernel"),    # one step, 64 MB of output, little but stores
     (8192, 4096, 60, "gelu", "tw_gemm_bw_kernel"),
+    (8200, 4096, 60, "none", "tw_gemm_bw_kernel"),    # (columns of C off the sectors of memory)
     (16384, 4096, 120, "relu", "tw_gemm_bs_kernel"),  # 128 MB
     (8192, 4096, 256, "none", "tw_gemm_bw_kernel"),   # four steps
 ])

@@ -3082,7 +3082,7 @@ int launch_gemm(const tw_plan *plan, GemmArgs &a, const Choice &c, int32_t *tick
     if (c.shape == TW_SHAPE_SKINNY)
         return plan->dtype == TW_F16 ? launch_skinny<TW_F16, false>(plan, a, s) : launch_skinny<TW_BF16, false>(plan, a, s);
     if (c.shape == TW_SHAPE_BS || c.shape == TW_SHAPE_BS4 || c.shape == TW_SHAPE_BS8)
-        return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), c.shape == TW_SHAPE_BS ? bs_wide(plan, a.M, a.ldc, a.act) : c.shape == TW_SHAPE_BS8, s);
+        return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), c.shape == TW_SHAPE_BS ? bs_wide(plan, a.M, a.C, a.ldc, a.act) : c.shape == TW_SHAPE_BS8, s);
     // queue 0 is the longest: one workgroup per entry, up to the chip's share of a queue
     const int64_t qlen0 = (int64_t)a.n_own_items + (a.n_tail_items + kXcd - 1) / kXcd;
     const int64_t per_queue = std::max<int64_t>(1, (int64_t)plan->cu_count * c.per_cu / kXcd);
@@ -3326,7 +3326,7 @@ const char *tw_gemm_kernel_name(const tw_plan *plan, int M, int a_layout, int64_
     const int shape = choose_shape(plan, M, lda, ldc, beta != 0.0f).shape;
     if (shape < TW_SHAPE_BS)
         return names[shape];
-    return shape == TW_SHAPE_BS8 || (shape == TW_SHAPE_BS && bs_wide(plan, M, ldc, activation)) ? "tw_gemm_bw_kernel" : "tw_gemm_bs_kernel";
+    return shape == TW_SHAPE_BS8 || (shape == TW_SHAPE_BS && bs_wide(plan, M, nullptr, ldc, activation)) ? "tw_gemm_bw_kernel" : "tw_gemm_bs_kernel";
 }
 
 int tw_plan_reset(tw_plan *plan, void *stream)

@@ -332,7 +332,10 @@ __global__ void __launch_bounds__(64 * kBsWaves, 4)
 // says which of its steps are there, a multiplying wave how many it has read), tiles with fewer steps multiply zeros in the
 // missing ones, and the activation is a template argument.  The multiplying waves' memory queue holds stores only and nothing
 // in the loop waits for it.
-// A wave's 32 rows are 64 bytes of a column.  Stored a further block later through the stage that the two waves of a block of
+// A wave's 32 rows are 64 bytes of a column.  Where those are whole sectors of memory they are stored through to it; else they
+// stay in L2, where a sector's two parts meet (`through`: M 5809, N 3515, two thirds of the columns 16 bytes off, 41.5 us
+// through and 17 not; M 12516, N 7222 152 and 58; 1000 such problems 0.47 - 0.71 of what ran before, through 0.92 - 1.18).
+// Stored a further block later through the stage that the two waves of a block of
 // columns share, they go out as whole 128-byte lines (`lines`): ahead where C leaves the last-level cache (134 MB 61 -> 47.6
 // us), level below (64 MB: 26.2 without, 26.8 with), crossing at 90 - 96 MB.
 // Measured (bf16, us of a replayed graph, the panel kernel or the four-wave one -> this): M 8192, K 1024, N 4096, 256 kept rows
@@ -352,7 +355,7 @@ constexpr uint32_t kBwNoRow = 0xFFFFFFFFu;           // (offsets of rows are mul
 template <int DT, int ACT, int NS>
 __global__ void __launch_bounds__(bw_threads(NS), 3)
     tw_gemm_bw_kernel(const GemmArgs p, int n_units, int n_ranges, int row_units, int affine, uint32_t a_bytes,
-                      uint32_t c_bytes, int lines)
+                      uint32_t c_bytes, int lines, int through)
 {
     using E = Elem<DT>;
     constexpr int LW = bw_load_waves(NS), SPW = NS / LW; // loading waves, steps of a block each
@@ -498,11 +501,11 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
         for (int q = 0; q < 2; ++q)
             if (jq[q] < cnt)
                 store_chunk(reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(C) + o_q[q]) + m0, v[q], m0 + row_q, m_end,
-                            p.store_through != 0);
+                            through && p.store_through);
     };
     // The products of block mb, whose steps have landed.  Between them (`older` blocks before it: 0, 1, or 2 and more) the
     // epilogue of the block before (`prev`) goes to one stage, and the block before that from the other one to C: whole
-    // blocks, through a buffer descriptor that drops the columns the unit does not have, and through to memory (as
+    // blocks, through a buffer descriptor that drops the columns the unit does not have, and `through` to memory (as
     // store_chunk).  `land` is what the flags said in the middle of the block.
     const __amdgpu_buffer_rsrc_t c_rsrc = __builtin_amdgcn_make_buffer_rsrc(C + m_lo, 0, (int)c_bytes, kBsRsrcFlags);
     const bool other = lines && (lane & 4); // what this lane watches: the other wave, or the loads
@@ -542,8 +545,11 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
                 out[i - 2] = stage_get(parity ^ 1, i - 2);
             sum = E::mfma(af[i], bq[i >> 2][i & 3], sum);
             if (OLDER > 1 && (i == NS * 4 - 2 || i == NS * 4 - 1)) {
-                const int q = i - (NS * 4 - 2);
-                __builtin_amdgcn_raw_buffer_store_b128(out[q], c_rsrc, (int)o_q[q], (mb - 2) * kBsRows * 2, 1 | 2 | 16);
+                const int q = i - (NS * 4 - 2), row_b = (mb - 2) * kBsRows * 2;
+                if (through)
+                    __builtin_amdgcn_raw_buffer_store_b128(out[q], c_rsrc, (int)o_q[q], row_b, 1 | 2 | 16);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b128(out[q], c_rsrc, (int)o_q[q], row_b, 0);
                 // Two wait states before the data's registers are written again: the store is still reading them, and the compiler
                 // adds none to a buffer store with a scalar offset (an instruction that wrote the second of the four
                 // at once put its own result into C).
@@ -639,7 +645,8 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
             const int c = t.col0 + p.pruned_n[t.pn_off + jz];
             const uint32_t hb = E::to_bits(tw_finish(0.0f, p.bias, c, ACT));
             const uint32_t w = hb | (hb << 16);
-            store_chunk(C + (int64_t)c * p.ldc + m_lo + ch * 8, u32x4{w, w, w, w}, m_lo + ch * 8, m_hi, p.store_through != 0);
+            store_chunk(C + (int64_t)c * p.ldc + m_lo + ch * 8, u32x4{w, w, w, w}, m_lo + ch * 8, m_hi,
+                        through && p.store_through);
         }
     }
 }
@@ -692,6 +699,9 @@ double bs_fill(const tw_plan *plan, int M)
     return (double)wgs / (double)(rounds * cu);
 }
 
+// whether every 32 rows of a column of C are whole 64-byte pieces of memory
+bool bs_whole_sectors(const void *C, int64_t ldc) { return (((uintptr_t)C | (uintptr_t)ldc * 2u) & 63) == 0; }
+
 template <int DT, int NS> static int launch_bs_t(const tw_plan *plan, const GemmArgs &a, int per_cu, hipStream_t s)
 {
     const int n_ranges = bs_ranges(plan, a.M, per_cu);
@@ -714,13 +724,14 @@ template <int DT, int NS> static int launch_bw(const tw_plan *plan, const GemmAr
     if (grid > (int64_t)0x7fffffff)
         return fail(TW_ERR_SHAPE, "%lld workgroups (M=%d): a launch takes at most %lld", (long long)grid, a.M,
                     (long long)(int64_t)0x7fffffff);
+    const int whole = bs_whole_sectors(a.C, a.ldc);
     const auto kernel = a.act == TW_ACT_RELU   ? tw_gemm_bw_kernel<DT, TW_ACT_RELU, NS>
                         : a.act == TW_ACT_GELU ? tw_gemm_bw_kernel<DT, TW_ACT_GELU, NS>
                         : a.act == TW_ACT_TANH ? tw_gemm_bw_kernel<DT, TW_ACT_TANH, NS>
                                                : tw_gemm_bw_kernel<DT, TW_ACT_NONE, NS>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(bw_threads(NS)), 0, s, a, plan->n_units, n_ranges, (a.M + 31) / 32, affine,
                        (uint32_t)((uint64_t)plan->K * (uint64_t)a.lda * 2u), (uint32_t)((uint64_t)plan->N * (uint64_t)a.ldc * 2u),
-                       (int64_t)a.M * plan->N * 2 > kBwLineBytes);
+                       whole && (int64_t)a.M * plan->N * 2 > kBwLineBytes, whole);
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
@@ -731,7 +742,7 @@ template <int DT, int NS> static int launch_bw(const tw_plan *plan, const GemmAr
 // 50.1; 34, 39 or 44 units, which leave it a third of the chip, 1.1 - 1.4 of the time of what ran before), and with one step
 // from 32 MB on (60 kept: M 8192, N 4096 18.9 against 22.7, M 8192, N 2048 12.1 against 13.9; M 8192, N 3072, not even, 19.9
 // against 16.9).
-bool bs_wide(const tw_plan *plan, int M, int64_t ldc, int act)
+bool bs_wide(const tw_plan *plan, int M, const void *C, int64_t ldc, int act)
 {
     const int ns = std::max(1, plan->max_k_pad / kBlockK);
     const int64_t out_bytes = (int64_t)M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, M, 2);
@@ -739,7 +750,8 @@ bool bs_wide(const tw_plan *plan, int M, int64_t ldc, int act)
     const bool stores_only = (act == TW_ACT_NONE || act == TW_ACT_RELU) &&
                              ((out_bytes > (int64_t)112 << 20 && wgs2 * 4 >= all2 * 3) ||
                               (ns == 1 && out_bytes >= (int64_t)32 << 20 && wgs2 * 10 >= all2 * 9));
-    return ns > kBsMaxSteps || !(stores_only || (uint64_t)plan->N * (uint64_t)ldc * 2u >= kBwMaxBytes);
+    // (off the sectors of memory the wider one, which then stores through L2, is ahead)
+    return ns > kBsMaxSteps || !((stores_only && bs_whole_sectors(C, ldc)) || (uint64_t)plan->N * (uint64_t)ldc * 2u >= kBwMaxBytes);
 }
 
 int launch_bs(const tw_plan *plan, const GemmArgs &a, int per_cu, bool wide, hipStream_t s)

@@ -191,7 +191,7 @@ bool takes_row_major_directly(const tw_plan *p, float beta);
 // `per_cu` workgroups meant to share a compute unit
 bool bs_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
 // which of its two kernels (tw_gemm_bs_kernel, tw_gemm_bw_kernel: `wide`) takes a call that bs_takes
-bool bs_wide(const tw_plan *p, int M, int64_t ldc, int act);
+bool bs_wide(const tw_plan *p, int M, const void *C, int64_t ldc, int act);
 bool bw_takes(const tw_plan *p, int64_t lda, int64_t ldc, bool reads_c);
 int launch_bs(const tw_plan *p, const GemmArgs &a, int per_cu, bool wide, hipStream_t s);
 double bs_fill(const tw_plan *p, int M); // share of the compute units its launch gives a workgroup
