@@ -287,7 +287,12 @@ def test_both_weight_stationary_kernels(tw, oracle, dtype, case):
     (8192, 4096, 60, "none", "tw_gemm_bs_kernel"),    # one step, 64 MB of output, little but stores
     (8192, 4096, 60, "gelu", "tw_gemm_bw_kernel"),
     (8200, 4096, 60, "none", "tw_gemm_bw_kernel"),    # (columns of C off the sectors of memory)
-    (16384, 4096, 120, "relu", "tw_gemm_bs_kernel"),  # 128 MB
+    (10240, 3072, 60, "none", "tw_gemm_bw_kernel"),   # (its workgroups not even)
+    (14336, 4096, 60, "none", "tw_gemm_bw_kernel"),   # 112 MB
+    (16384, 4096, 60, "relu", "tw_gemm_bs_kernel"),   # 128 MB, columns of C 32 KB apart
+    (16384, 4096, 120, "relu", "tw_gemm_bs_kernel"),
+    (16320, 4096, 120, "relu", "tw_gemm_bw_kernel"),
+    (16384, 4096, 190, "none", "tw_gemm_bw_kernel"),  # three steps
     (8192, 4096, 256, "none", "tw_gemm_bw_kernel"),   # four steps
 ])
 def test_which_weight_stationary_kernel_runs(tw, M, N, kept, act, kernel):

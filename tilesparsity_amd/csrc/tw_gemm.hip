@@ -2607,7 +2607,11 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
     // Not where a 64-row panel of A fits LDS and
     // - there are few units and K is short (M 8192, K 768, N 512: 0.98 - 1.07), or
     // - the tiles are long and K is 512 (190 kept within 40 %: 1.02 in the mean, to 1.10) or the workgroups leave more than a
-    //   tenth of the chip without one (24 units, 300 kept, M 2048: 1.10 - 1.15), or
+    //   tenth of the chip without one (24 units, 300 kept, M 2048: 1.10 - 1.15; 1.09 in the mean below M 1500, 1.0 to 6000, 0.85
+    //   from there to 16384, which is left to the panel, 0.92 at 16384), or
+    // - C's columns start at sectors of memory (else 0.61 in the mean of 1132 problems, none of them slower by more than 5 %) and the
+    //   launch is small: long tiles under fewer than 1500 rows (0.98, 1.03 and more in 11 of 25), or less than 0.8 of the chip
+    //   under at most 50000 units * rows (0.95, 1.03 and more in 9 of 47, to 1.16), or
     // - the launch is little but its stores (K 512, N 8192, M 16384, 60 kept within 40 %: 73 -> 102; 120: 83.5 -> 93; 60 kept,
     //   M 8192, N 5632: 27.8 -> 32.5).
     const bool panel64 = as_ok(TW_SHAPE_AS64);
@@ -2618,6 +2622,7 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
                     (chip >= 0.75 || (!panel64 && (plan->max_k_pad <= 192 || chip >= 0.65))) &&
                     !(panel64 && ((plan->K < 1024 && plan->n_units < 8) || (plan->max_k_pad > 256 && plan->K <= 512) ||
                                   (plan->max_k_pad > 256 && M < 16384 && chip < 0.9) ||
+                                  (ldc % 32 == 0 && ((plan->max_k_pad > 256 && M < 1500) || (chip < 0.8 && (int64_t)plan->n_units * M <= 50000))) ||
                                   (plan->K < 1024 && out_mb > (plan->max_k_pad <= 64 ? 32 : plan->max_k_pad <= 128 ? 200 : INT64_MAX))));
     // Tiles of six steps and more on average, wide, with 256-row items for three quarters of the
     // chip: the streaming 256 x 128 kernel, whose loads write LDS directly, is ahead of the panel

@@ -736,22 +736,29 @@ template <int DT, int NS> static int launch_bw(const tw_plan *plan, const GemmAr
     return TW_OK;
 }
 
-// Up to three steps either kernel takes the plan.  Without a long activation, where the launch is little but its stores, the
-// one whose waves store 64 rows themselves is ahead where its workgroups, two to a compute unit, come out even: beyond 112
-// MB of output (M 16384, N 4096, 120 kept rows: 38.5 against 47.1 us; M 14336: 34.5 against 29.5; with GELU 54.9 against
-// 50.1; 34, 39 or 44 units, which leave it a third of the chip, 1.1 - 1.4 of the time of what ran before), and with one step
-// from 32 MB on (60 kept: M 8192, N 4096 18.9 against 22.7, M 8192, N 2048 12.1 against 13.9; M 8192, N 3072, not even, 19.9
-// against 16.9).
+// Up to three steps either kernel takes the plan.  The one whose waves store 64 rows themselves is ahead without a long
+// activation, where its workgroups, two to a compute unit, come out even, every 32 rows of a column of C are whole
+// sectors of memory, and (us of it against the wider one, M 4096 .. 16384, N 900 .. 8192, 1500 problems)
+// - one step, 32 to 90 MB of output (0.88 - 0.99 of the time in the mean of a size; N 4096, M 10240: 16.2 against 18.6; from
+//   there on, where the wider one stores whole lines, 1.02 - 1.7), or to 128 MB where C's columns are a multiple of 16 KB apart
+//   (N 8192, M 8192: 0.71; N 4096, M 16384: 0.83);
+// - two steps, the same stride and 112 to 128 MB (N 4096, M 16384 40.9 against 48.3; M 16320 1.09; N 8192, M 8192 0.95; 256 MB 1.15).
+// Three steps: the wider one (1.06 - 1.7, N 4096, M 14336 1.39).
 bool bs_wide(const tw_plan *plan, int M, const void *C, int64_t ldc, int act)
 {
     const int ns = std::max(1, plan->max_k_pad / kBlockK);
-    const int64_t out_bytes = (int64_t)M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, M, 2);
+    if (ns > kBsMaxSteps)
+        return true;
+    if ((uint64_t)plan->N * (uint64_t)ldc * 2u >= kBwMaxBytes)
+        return false;
+    const int64_t mb = (int64_t)1 << 20, out_bytes = (int64_t)M * plan->N * 2, wgs2 = (int64_t)plan->n_units * bs_ranges(plan, M, 2);
     const int64_t slots2 = 2 * (int64_t)plan->cu_count, all2 = (wgs2 + slots2 - 1) / slots2 * slots2;
-    const bool stores_only = (act == TW_ACT_NONE || act == TW_ACT_RELU) &&
-                             ((out_bytes > (int64_t)112 << 20 && wgs2 * 4 >= all2 * 3) ||
-                              (ns == 1 && out_bytes >= (int64_t)32 << 20 && wgs2 * 10 >= all2 * 9));
-    // (off the sectors of memory the wider one, which then stores through L2, is ahead)
-    return ns > kBsMaxSteps || !((stores_only && bs_whole_sectors(C, ldc)) || (uint64_t)plan->N * (uint64_t)ldc * 2u >= kBwMaxBytes);
+    if ((act != TW_ACT_NONE && act != TW_ACT_RELU) || wgs2 * 10 < all2 * 9 || !bs_whole_sectors(C, ldc))
+        return true;
+    const bool far_stride = ldc * 2 % 16384 == 0;
+    if (ns == 1)
+        return !(out_bytes >= 32 * mb && (out_bytes <= kBwLineBytes || (far_stride && out_bytes <= 128 * mb)));
+    return !(ns == 2 && far_stride && out_bytes > 112 * mb && out_bytes <= 128 * mb);
 }
 
 int launch_bs(const tw_plan *plan, const GemmArgs &a, int per_cu, bool wide, hipStream_t s)
