@@ -1199,7 +1199,7 @@ def test_kernel_for_few_rows_is_taken_where_it_is_ahead(tw, M, K, N, kept, skinn
     (4096, 1024, 1024, 128, 0.25, 1.0, "f16"),    # where a panel of A would fit
 ])
 def test_row_major_streaming(tw, oracle, M, K, N, G, k_keep, n_keep, dtype):
-    """Row-major A and C through the row-major streaming kernel (its workgroups fill three eighths of the chip): alpha, bias
+    """Row-major A and C through the row-major streaming kernel (forced: some of these calls take another by themselves): alpha, bias
     and ReLU, pruned columns left alone, then beta and pruned columns filled; tiles without kept rows; padding and
     the workspace untouched (nothing is staged).  Sampled rows against the oracle."""
     import torch
@@ -1216,28 +1216,30 @@ def test_row_major_streaming(tw, oracle, M, K, N, G, k_keep, n_keep, dtype):
     Ch[:, :N] = oracle.cast_bits(C0, dtype).reshape(M, N)
     dA, d_bias = to_device_bits(Ah, Ah.shape), torch.from_numpy(bias).cuda()
     rows = np.unique(np.concatenate([np.arange(5), np.arange(M - 70, M), rng.choice(M, 40)]))
-    with tw.Plan.create(K, N, dtype, tiles, B) as plan:
-        nbytes = max(plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR), 16)
-        ws = torch.full((nbytes // 2,), 0x7bcd, dtype=torch.int16, device="cuda")
-        for alpha, beta, pruned in ((0.75, 0.0, tw.PRUNED_UNTOUCHED), (1.0, 0.5, tw.PRUNED_ZERO)):
-            if beta and K < 2128:
-                continue                                       # (a panel does not read C: staged there)
-            dC = to_device_bits(Ch, Ch.shape)
-            plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=alpha, beta=beta, a_layout=tw.ROWMAJOR,
-                      c_layout=tw.ROWMAJOR, pruned_cols=pruned, bias_ptr=d_bias.data_ptr(), activation=tw.ACT_RELU,
-                      workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes)
-            torch.cuda.synchronize()
-            assert torch.all(ws == 0x7bcd)
-            out = from_device_bits(dC)
-            assert np.all(out[:, N:] == SENTINEL)
-            pre = alpha * reference(oracle, A[rows], B, tiles, dtype)
-            want = np.maximum(pre + beta * oracle.quantize(C0[rows], dtype) + bias, 0.0)
-            got = oracle.bits_to_f32(np.ascontiguousarray(out[rows, :N]), dtype).reshape(rows.size, N)
-            assert oracle.rel_error(got[:, keep], want[:, keep]) <= TOL[dtype]
-            if pruned == tw.PRUNED_UNTOUCHED:
-                assert np.array_equal(out[:, :N][:, ~keep], Ch[:, :N][:, ~keep])
-            elif not np.all(keep):
-                assert oracle.rel_error(got[:, ~keep], want[:, ~keep]) <= TOL[dtype]
+    try:
+        tw.set_option(tw.OPT_SHAPE, tw.SHAPE_RM)
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            nbytes = max(plan.staged_workspace(M, tw.ROWMAJOR, tw.ROWMAJOR), 16)
+            ws = torch.full((nbytes // 2,), 0x7bcd, dtype=torch.int16, device="cuda")
+            for alpha, beta, pruned in ((0.75, 0.0, tw.PRUNED_UNTOUCHED), (1.0, 0.5, tw.PRUNED_ZERO)):
+                dC = to_device_bits(Ch, Ch.shape)
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=lda, ldc=ldc, alpha=alpha, beta=beta, a_layout=tw.ROWMAJOR,
+                          c_layout=tw.ROWMAJOR, pruned_cols=pruned, bias_ptr=d_bias.data_ptr(), activation=tw.ACT_RELU,
+                          workspace_ptr=ws.data_ptr(), workspace_bytes=nbytes)
+                torch.cuda.synchronize()
+                assert torch.all(ws == 0x7bcd)
+                out = from_device_bits(dC)
+                assert np.all(out[:, N:] == SENTINEL)
+                pre = alpha * reference(oracle, A[rows], B, tiles, dtype)
+                want = np.maximum(pre + beta * oracle.quantize(C0[rows], dtype) + bias, 0.0)
+                got = oracle.bits_to_f32(np.ascontiguousarray(out[rows, :N]), dtype).reshape(rows.size, N)
+                assert oracle.rel_error(got[:, keep], want[:, keep]) <= TOL[dtype]
+                if pruned == tw.PRUNED_UNTOUCHED:
+                    assert np.array_equal(out[:, :N][:, ~keep], Ch[:, :N][:, ~keep])
+                elif not np.all(keep):
+                    assert oracle.rel_error(got[:, ~keep], want[:, ~keep]) <= TOL[dtype]
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
 
 
 def test_row_major_streaming_nonfinite(tw, oracle):
@@ -1262,7 +1264,12 @@ def test_row_major_streaming_nonfinite(tw, oracle):
     dAk, dAr = to_device_bits(Ak, Ak.shape), to_device_bits(Ar, Ar.shape)
     dCk, dCr = (torch.zeros(s, dtype=torch.int16, device="cuda") for s in ((N, Ak.shape[1]), (M, N)))
     with tw.Plan.create(K, N, "f16", tiles, B) as plan:
-        plan.gemm(dAr.data_ptr(), dCr.data_ptr(), M, lda=Ar.shape[1], ldc=N, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+        try:
+            tw.set_option(tw.OPT_SHAPE, tw.SHAPE_RM)
+            assert plan.kernel_name(M, Ar.shape[1], N, tw.ROWMAJOR, tw.ROWMAJOR) == "tw_gemm_rm_kernel"
+            plan.gemm(dAr.data_ptr(), dCr.data_ptr(), M, lda=Ar.shape[1], ldc=N, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+        finally:
+            tw.set_option(tw.OPT_SHAPE, -1)
         plan.gemm(dAk.data_ptr(), dCk.data_ptr(), M, lda=Ak.shape[1], ldc=Ak.shape[1])
         torch.cuda.synchronize()
     r, k = dCr.view(torch.float16), dCk.view(torch.float16)[:, :M].T
