@@ -2596,7 +2596,7 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
     skinny = skinny && skinny_ok;
     // The weight-stationary kernels: tiles of at most 384 kept rows, wider than 64 columns, under units * rows of A above 24576
     // (96 rows to a workgroup with one on every compute unit).  Against the choice without the wider of them, us of a replayed
-    // graph before and after, on M 256 .. 16384, K 512 .. 4096, N 512 .. 8192, 60 .. 380 kept rows, all alike or within 40 % of
+    // graph before and after, on M 256 .. 16384 in whole lines, K 512 .. 4096, N 512 .. 8192, 60 .. 380 kept rows, all alike or within 40 % of
     // each other, without activation, with ReLU and GELU: 0.88 of the time over 1700 problems from there on (BERT-large FFN1 at
     // 75 % 34.1 -> 26.2, with GELU 39.5 -> 32.5; M 4096, K 3072, N 3072, 60 kept 16.2 -> 10.9; M 512, N 8192 0.83, M 1024, N 4096
     // 0.90; below the line M 2048, N 1024 1.0 - 1.08, M 1024, N 2048 1.07).  A unit multiplies as many steps as the longest has,

@@ -1,5 +1,6 @@
-// Weight-stationary kernel of the tile-wise-sparse GEMM (TW_SHAPE_BS), for tiles that keep few
-// rows (at most 192; 384 in its wider form below) under many rows of A: BERT-like layers at 75 % sparsity and more.
+// Weight-stationary kernels of the tile-wise-sparse GEMM (TW_SHAPE_BS), for tiles that keep few
+// rows under many rows of A: BERT-like layers at 75 % sparsity and more.  First the one of four multiplying waves
+// (tw_gemm_bs_kernel, at most 192 kept rows), then its wider form of eight (tw_gemm_bw_kernel, at most 384).
 //
 // A workgroup takes one unit (up to 128 compact columns of a tile) and a range of rows of A.  Its
 // four multiplying waves own one block of 32 compact columns each and keep that block's packed
@@ -340,7 +341,8 @@ __global__ void __launch_bounds__(64 * kBsWaves, 4)
 // us), level below (64 MB: 26.2 without, 26.8 with), crossing at 90 - 96 MB.
 // Measured (bf16, us of a replayed graph, the panel kernel or the four-wave one -> this): M 8192, K 1024, N 4096, 256 kept rows
 // 34.2 -> 26.2, with GELU 39.7 -> 32.5; M 12288 61.3 -> 37.0, with GELU 69.5 -> 43.5; M 4096, K 768, N 3072, 192 kept 15.1 ->
-// 13.0, with GELU 16.9 -> 16.1.  Bit for bit what those give.
+// 13.0, with GELU 16.9 -> 16.1.  Without activation and with ReLU bit for bit what those give; GELU and tanh of the same sum come
+// from instructions in another order, within one unit in the last place of the result.
 constexpr int kBwMulWaves = 8;
 constexpr int bw_load_waves(int ns) { return ns <= 4 ? ns : 3; } // (three and four waves a SIMD have 168 and 128 registers)
 constexpr int bw_threads(int ns) { return 64 * (kBwMulWaves + bw_load_waves(ns)); }

@@ -10,7 +10,8 @@
 //   16.4); K 4608, N 512, M 12544: 82 -> 46; K 2304, N 512, M 16384: 57 -> 37.
 // What bounds the first of these: 6300 cycles until the lists are there (arguments, unit, row numbers: trips to memory
 // from cold caches, then the lists themselves), 24 chunks at 735 cycles (a wave's chain of about 70 instructions and 8
-// MFMAs per record; the loads alone take 430, the multiplying side alone 600), 5000 to add up and store.
+// MFMAs per record; the loads alone take 430, the multiplying side alone 600), 5000 to add up and store.  (The compiler keeps 53
+// to 58 scalar registers of the unit and the arguments in lanes of a vector register across the loop; no scratch memory.)
 //
 //   work:  a workgroup takes 64 rows m and two units (four of at most 64 columns): with 256 columns the bytes a
 //          compute unit fetches (128 K for A, 512 K_t for the weight) are near their least, while 4096 rows of 768 columns
