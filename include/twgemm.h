@@ -316,12 +316,11 @@ int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda
  *   TW_OPT_SHAPE        one of the TW_SHAPE_* kernels below
  *   TW_OPT_WGS_PER_CU   workgroups launched per compute unit, 1..8
  *   TW_OPT_PIECE        columns of a tile handed out as one work item: 128, 64 or 32
- *   TW_OPT_XCD_QUEUES   1: one work queue per accelerator die, each owning whole row blocks of A
- *                       (the workgroups of a die then share those rows in their L2);
- *                       0: the work items are dealt out over the dies in turn; automatic: 0
- *                       unless nearly every tile keeps nearly every row (a 0 %-sparse plan);
+ *   TW_OPT_XCD_QUEUES   1 and automatic: one work queue per accelerator die, each owning whole row
+ *                       blocks of A (the workgroups of a die then share those rows in their L2);
+ *                       0: the work items are dealt out over the dies in turn, tile after tile;
  *                       2: dealt out over the dies in turn, row block after row block (all tiles
- *                       of a row block before the next) instead of tile after tile
+ *                       of a row block before the next)
  *   TW_OPT_SPIN_LIMIT   loads a wave of tw_lstm_steps spends looking for a step's h before it gives up
  *   TW_OPT_BALANCE      1: row blocks sized per tile where the items would not fill the chip once
  *   TW_OPT_LDS_DMA      0: the 256-row streaming kernels stage their loads through registers

@@ -1402,3 +1402,43 @@ def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw, beta):
         torch.cuda.synchronize()
     assert bool((C[-3:] == 3.0 + beta).all()) and bool((C[:100] == 1.5 + beta).all()) and bool((C[M - 200:-3] == 1.5 + beta).all())
     assert int((C != 1.5 + beta).sum(dtype=torch.int64)) == 3 * N
+
+
+@pytest.mark.parametrize("blocks", [7, 40, 43])
+@pytest.mark.parametrize("pruned", ["untouched", "zero"])
+def test_queues_of_the_dies_hand_out_every_item_once(tw, oracle, blocks, pruned):
+    """Row blocks owned by the dies give bit for bit what items dealt out in turn give: fewer row blocks
+    than dies (nobody owns one), five to a die in a group of two and one of three, the same with three
+    left over, each with one to a die's share of a launch and with twelve items and more to a workgroup,
+    tiles without kept rows and pruned columns to fill among them."""
+    import torch
+    rng = np.random.default_rng(5 + blocks)
+    K, N, G = 96, 2688, 32
+    tiles = random_tiles(rng, K, N, G, k_keep=0.4, n_keep=0.7, empty_every=20)
+    B = (rng.standard_normal((K, N)) * 0.1).astype(np.float32)
+    code = tw.PRUNED_ZERO if pruned == "zero" else tw.PRUNED_UNTOUCHED
+    M = blocks * 128 - 5
+    ld = round_up(M, 8)
+    dA = torch.from_numpy(oracle.cast_bits(rng.standard_normal((K, ld)).astype(np.float32), "f16").view(np.int16).reshape(K, ld)).cuda()
+    got = {}
+    try:
+        with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+            tw.set_option(tw.OPT_SHAPE, tw.SHAPE_128x32)
+            tw.set_option(tw.OPT_PIECE, 32)
+            for per_cu in (1, 8):
+                tw.set_option(tw.OPT_WGS_PER_CU, per_cu)
+                for xcd in (0, 1, -1):
+                    tw.set_option(tw.OPT_XCD_QUEUES, xcd)
+                    print("queues", blocks, pruned, per_cu, xcd, flush=True)
+                    dC = torch.full((N, ld), 0x1234, dtype=torch.int16, device="cuda")
+                    for _ in range(2):  # (the second launch finds the counters as the first left them)
+                        plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=ld, ldc=ld, pruned_cols=code,
+                                  stream=torch.cuda.current_stream().cuda_stream)
+                    torch.cuda.synchronize()
+                    got[per_cu, xcd] = dC.cpu()
+    finally:
+        for opt in (tw.OPT_SHAPE, tw.OPT_PIECE, tw.OPT_WGS_PER_CU, tw.OPT_XCD_QUEUES):
+            tw.set_option(opt, -1)
+    want = got[1, 0]
+    assert (want[:, :M] != 0x1234).any(1).sum() >= (N if pruned == "zero" else 1)
+    assert all(torch.equal(want, g) for g in got.values())

@@ -47,9 +47,23 @@ struct Work {
     int rows; // rows [m0, m0 + rows) of A and C, cut at M by the caller
 };
 
+// (queue x's share of the first `n` of the items that are dealt out over the queues in turn)
+__device__ __forceinline__ int dealt_to(int n, int x)
+{
+    return (n + kXcd - 1 - x) / kXcd;
+}
+
+// where column `u` starts in the part of queue x that is ordered column after column
+__device__ __forceinline__ int column_start(const GemmArgs &p, int x, int u)
+{
+    return u * p.n_last + dealt_to(u * p.n_tail_mblk, x);
+}
+
 __device__ __forceinline__ int queue_length(const GemmArgs &p, int x)
 {
-    return p.n_own_items + (p.n_tail_items > x ? (p.n_tail_items - x + kXcd - 1) / kXcd : 0);
+    if (p.n_list_items)
+        return dealt_to(p.n_list_items, x);
+    return p.n_lead_items + column_start(p, x, p.n_pipe_u) + dealt_to((p.n_all_u - p.n_pipe_u) * p.n_mblk, x);
 }
 
 // (bm: rows of a row block of this launch)
@@ -60,13 +74,9 @@ __device__ __forceinline__ Work queue_entry(const GemmArgs &p, int x, int q, int
     w.u = 0;
     w.m0 = 0;
     w.rows = bm;
-    if (q < p.n_own_items) {
-        const int i = q / p.n_all_u;
-        w.u = q - i * p.n_all_u;
-        w.m0 = (x * p.n_own + i) * bm;
-    } else {
-        const int j = (q - p.n_own_items) * kXcd + x;
-        if (j >= p.n_tail_items)
+    if (p.n_list_items) {
+        const int j = q * kXcd + x;
+        if (j >= p.n_list_items)
             return w;
         if (p.n_bal > 0) {
             // columns with row blocks of their own height: column u owns the items
@@ -78,14 +88,46 @@ __device__ __forceinline__ Work queue_entry(const GemmArgs &p, int x, int q, int
             w.u = u;
             w.rows = p.bal_rows[u];
             w.m0 = (j - p.bal_first[u]) * w.rows;
-        } else if (p.rb_major) {
+        } else {
             // all columns of a row block (heaviest first) before the next row block
             const int mb = j / p.n_all_u;
             w.u = j - mb * p.n_all_u;
-            w.m0 = (kXcd * p.n_own + mb) * bm;
+            w.m0 = mb * bm;
+        }
+    } else if (q < p.n_lead_items) {
+        const int per = p.n_grp * p.n_pipe_u, g = q / per, r = q - g * per;
+        w.u = r / p.n_grp;
+        w.m0 = (x * p.n_own + g * p.n_grp + (r - w.u * p.n_grp)) * bm;
+    } else {
+        const int r = q - p.n_lead_items;
+        int end;
+        if (r < (end = column_start(p, x, p.n_pipe_u))) {
+            int u, off;
+            if (p.n_last > 0) { // (a column starts within one entry of its mean place)
+                u = r * kXcd / (p.n_last * kXcd + p.n_tail_mblk);
+                if (column_start(p, x, u) > r)
+                    --u;
+                else if (column_start(p, x, u + 1) <= r)
+                    ++u;
+                off = r - column_start(p, x, u);
+            } else {
+                u = (r * kXcd + x) / p.n_tail_mblk;
+                off = r - column_start(p, x, u);
+            }
+            w.u = u;
+            if (off < p.n_last) {
+                w.m0 = (x * p.n_own + p.n_own - p.n_last + off) * bm;
+            } else {
+                const int j = (dealt_to(u * p.n_tail_mblk, x) + off - p.n_last) * kXcd + x;
+                w.m0 = (kXcd * p.n_own + j - u * p.n_tail_mblk) * bm;
+            }
         } else {
-            w.u = j / p.n_tail_mblk;
-            w.m0 = (kXcd * p.n_own + (j - w.u * p.n_tail_mblk)) * bm;
+            const int j = (r - end) * kXcd + x;
+            if (j >= (p.n_all_u - p.n_pipe_u) * p.n_mblk)
+                return w;
+            w.u = j / p.n_mblk;
+            w.m0 = (j - w.u * p.n_mblk) * bm;
+            w.u += p.n_pipe_u;
         }
     }
     w.kind = w.u < p.n_pipe_u ? ITEM_PIPE : (w.u < p.n_gemm_u ? ITEM_NOSTEP : ITEM_ZERO);
@@ -2533,10 +2575,7 @@ struct Choice {
 
 // Picks the shape from the plan and M.  Wide tiles run 256-row items (half the weight traffic
 // per row of A of 128-row items).  Launches with too few items for the chip (skinny M) hand a
-// unit out in pieces of 64 or 32 columns.  One queue per die is an option, not the default: the
-// workgroups of a die then share the rows of A in their L2 (measured on the 0 %-sparse plan of
-// the headline shape: a third of the reads from memory), but no benchmark shape ran faster for
-// it and the stress shape, whose 512-row block of A fills an L2, ran 13 % slower.
+// unit out in pieces of 64 or 32 columns.  Every die has row blocks of its own (see fill_queues).
 static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc, bool reads_c, bool row_major = false)
 {
     Choice c;
@@ -2547,9 +2586,7 @@ static Choice choose_shape(const tw_plan *plan, int M, int64_t lda, int64_t ldc,
     auto items = [&](int bm, int piece) {
         return units * ((width + piece - 1) / piece) * ((M + bm - 1) / bm);
     };
-    // one queue per die where the tiles share their rows (a 0 %-sparse plan reads A once per die
-    // then instead of once per tile); no sparse plan gained from it, see below
-    c.xcd = option(TW_OPT_XCD_QUEUES) == 1 || (option(TW_OPT_XCD_QUEUES) == -1 && plan->rows_shared);
+    c.xcd = option(TW_OPT_XCD_QUEUES) == 1 || (option(TW_OPT_XCD_QUEUES) == -1 && option(TW_OPT_BALANCE) != 1);
     c.piece = 128;
     // The A-stationary kernel (K short enough for a panel of A in LDS, C not read).  Measured on a
     // grid of M 128 .. 16384, K 512 .. 2048, N 512 .. 4096, tiles of 64 and 128 columns, 25 and
@@ -2987,7 +3024,6 @@ void fill_common(GemmArgs &a, const tw_plan *plan, const void *A, int64_t lda, v
     a.store_through = 0;
     a.ticket = nullptr;
     a.n_bal = 0;
-    a.rb_major = 0;
     a.lds_dma = 0;
     a.a_bytes = a.b_bytes = 0;
     a.n_arg_units = 0;
@@ -2996,8 +3032,19 @@ void fill_common(GemmArgs &a, const tw_plan *plan, const void *A, int64_t lda, v
 // work items of a launch are counted in 32-bit integers
 constexpr int64_t kMaxItems = 0x7fffffff;
 
-// item matrix and queues of a launch with `bm`-row items and unit pieces of `piece` columns
-void fill_queues(GemmArgs &a, const tw_plan *plan, int M, int bm, int piece, int pruned_cols, bool xcd)
+// Item matrix and queues of a launch with `bm`-row items and unit pieces of `piece` columns for `wgs`
+// workgroups.  `xcd`: every die owns an eighth of the row blocks, whatever is left over is dealt out in turn.
+// Dealt out all in turn, tile after tile, a row block's items meet on one die only where the row blocks are a
+// multiple of eight: a die then fetched most of A (VGG16 conv4_2, 49 row blocks: 126 MB instead of 95).  Over
+// 15000 random problems (M 300 .. 16384, K 512 .. 4608, N 256 .. 8192, 10 - 95 % of the rows kept) owned row
+// blocks take 0.96 of the time at half an item to one item a workgroup, 0.93 to two, 0.91 to three, 0.88 from
+// four to six, 0.83 from there on; 131 of them lose 3 % and more, four a tenth (to 1.19).
+// Within a die the items go tile after tile, the longest first, so that a workgroup's last item is a short one:
+// row block after row block instead (the same rows for all workgroups of the die at a time) loses 10 % and more
+// in one problem of twenty between one and six items a workgroup (to 1.56).  Where there are twelve and more the
+// last items no longer count and two row blocks at a time are ahead of all at once: 0.80 of the time of dealt-out
+// items against 0.83 from twelve to eighteen, 0.78 against 0.81 above (load-imbalance stress, 29: 320 -> 293 us).
+void fill_queues(GemmArgs &a, const tw_plan *plan, int M, int bm, int piece, int pruned_cols, bool xcd, int64_t wgs)
 {
     const int width = std::max(32, round_up32(plan->max_unit_n));
     a.n_split = (std::min(width, 128) + piece - 1) / piece;
@@ -3007,9 +3054,13 @@ void fill_queues(GemmArgs &a, const tw_plan *plan, int M, int bm, int piece, int
     a.n_gemm_u = plan->n_units * a.n_split;
     a.n_all_u = a.n_gemm_u + (pruned_cols == TW_PRUNED_ZERO ? plan->n_zero_tiles : 0);
     a.n_own = xcd ? a.n_mblk / kXcd : 0;
-    a.n_own_items = a.n_own * a.n_all_u;
+    a.n_grp = (int64_t)a.n_pipe_u * a.n_mblk >= 12 * wgs ? 2 : a.n_own;
+    a.n_grp = std::max(1, std::min(a.n_grp, a.n_own));
+    const int groups = std::max(1, a.n_own / a.n_grp);
+    a.n_last = a.n_own - (groups - 1) * a.n_grp;
+    a.n_lead_items = (groups - 1) * a.n_grp * a.n_pipe_u;
     a.n_tail_mblk = a.n_mblk - kXcd * a.n_own;
-    a.n_tail_items = a.n_tail_mblk * a.n_all_u;
+    a.n_list_items = 0;
 }
 
 // Row blocks sized per column of the item matrix, for launches whose items do not fill the chip
@@ -3064,7 +3115,7 @@ bool balance_items(GemmArgs &a, const tw_plan *plan, int M, int bm, int64_t wgs)
     }
     for (int u = a.n_all_u; u <= kBalColumns; ++u)
         a.bal_first[u] = first;
-    a.n_tail_items = first;
+    a.n_list_items = first;
     return true;
 }
 
@@ -3089,7 +3140,9 @@ int launch_gemm(const tw_plan *plan, GemmArgs &a, const Choice &c, int32_t *tick
     if (c.shape == TW_SHAPE_BS || c.shape == TW_SHAPE_BS4 || c.shape == TW_SHAPE_BS8)
         return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), c.shape == TW_SHAPE_BS ? bs_wide(plan, a.M, a.C, a.ldc, a.act) : c.shape == TW_SHAPE_BS8, s);
     // queue 0 is the longest: one workgroup per entry, up to the chip's share of a queue
-    const int64_t qlen0 = (int64_t)a.n_own_items + (a.n_tail_items + kXcd - 1) / kXcd;
+    const int64_t qlen0 = a.n_list_items ? (a.n_list_items + kXcd - 1) / kXcd
+                                         : (int64_t)a.n_own * a.n_pipe_u + ((int64_t)a.n_tail_mblk * a.n_pipe_u + kXcd - 1) / kXcd +
+                                               ((int64_t)(a.n_all_u - a.n_pipe_u) * a.n_mblk + kXcd - 1) / kXcd;
     const int64_t per_queue = std::max<int64_t>(1, (int64_t)plan->cu_count * c.per_cu / kXcd);
     const int grid = (int)(kXcd * std::min(qlen0, per_queue));
     if (plan->dtype == TW_F16)
@@ -3172,7 +3225,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
     fill_common(a, plan, A, lda, C, ldc, M, alpha, beta, ep);
     const Route route = route_of(plan, M, a_layout, lda, c_layout, beta, staged);
     if (route == Route::SKINNY) {
-        fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false);
+        fill_queues(a, plan, M, kSkRows, 128, pruned_cols, false, 0);
         if (a.n_all_u == 0)
             return TW_OK;
         a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
@@ -3184,7 +3237,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
     if (route == Route::PANEL) {
         // both operands row-major, K short enough for a panel of A in LDS, C not read: the
         // A-stationary kernel in its row-major form
-        fill_queues(a, plan, M, 64, 128, pruned_cols, false);
+        fill_queues(a, plan, M, 64, 128, pruned_cols, false, 0);
         a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
         for (int i = 0; i < a.n_arg_units; ++i)
             a.arg_units[i] = plan->h_units[i];
@@ -3195,7 +3248,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
         return b64 ? launch_as<TW_BF16, 64, true>(plan, a, M, s) : launch_as<TW_BF16, 32, true>(plan, a, M, s);
     }
     if (route == Route::STREAM) {
-        fill_queues(a, plan, M, kRmRowsPerWg, 128, pruned_cols, false);
+        fill_queues(a, plan, M, kRmRowsPerWg, 128, pruned_cols, false, 0);
         if (a.n_all_u == 0)
             return TW_OK;
         a.n_arg_units = plan->n_units <= kMaxArgUnits ? plan->n_units : 0;
@@ -3207,7 +3260,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
     if (route == Route::GENERIC) {
         // layout-generic path (element strides), 128-row blocks, one workgroup per item; as many launches as the
         // grid's threads ask for
-        fill_queues(a, plan, M, 128, 128, pruned_cols, false);
+        fill_queues(a, plan, M, 128, 128, pruned_cols, false, 0);
         if (a.n_all_u == 0)
             return TW_OK;
         const int64_t max_mblk = kMaxGridThreads / 256 / a.n_all_u;
@@ -3222,7 +3275,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
             a.A = static_cast<const uint16_t *>(A) + m0 * sa_m;
             a.C = static_cast<uint16_t *>(C) + m0 * sc_m;
             a.M = rows;
-            fill_queues(a, plan, rows, 128, 128, pruned_cols, false);
+            fill_queues(a, plan, rows, 128, 128, pruned_cols, false, 0);
             const dim3 grid((unsigned)(a.n_all_u * a.n_mblk));
             if (plan->dtype == TW_F16)
                 hipLaunchKernelGGL((tw_gemm_generic_kernel<TW_F16>), grid, dim3(256), 0, (hipStream_t)stream, a, sa_m, sa_k, sc_m, sc_n);
@@ -3234,8 +3287,9 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
     }
 
     const Choice c = choose_shape(plan, M, lda, ldc, beta != 0.0f);
-    fill_queues(a, plan, M, kShapes[c.shape].bm, c.piece, pruned_cols, c.xcd);
-    a.rb_major = option(TW_OPT_XCD_QUEUES) == 2;
+    fill_queues(a, plan, M, kShapes[c.shape].bm, c.piece, pruned_cols, c.xcd, (int64_t)plan->cu_count * c.per_cu);
+    if (option(TW_OPT_XCD_QUEUES) == 2)
+        a.n_list_items = (int)std::min<int64_t>((int64_t)a.n_all_u * a.n_mblk, kMaxItems);
     // 256-row items whose loads write LDS directly (measured faster on every shape tried, with
     // one item per workgroup and with several)
     if ((c.shape == TW_SHAPE_256x128 || c.shape == TW_SHAPE_256x64) && option(TW_OPT_LDS_DMA) != 0 && (uint64_t)plan->packed_elems * 2u < (1ull << 32)) {

@@ -54,8 +54,10 @@ struct TileDev {
 // whose pruned columns are filled) by `n_mblk` blocks of BM rows.  It is handed out through
 // kXcd queues, one per accelerator die: workgroup b runs on die b % kXcd and draws from that
 // die's queue only, so the workgroups that share an L2 work on the same rows of A.  Queue x owns
-// the row blocks [x * n_own, (x + 1) * n_own) (all their items, row block after row block) and
-// every kXcd-th item of the remaining `n_tail_mblk` row blocks (unit after unit).
+// the row blocks [x * n_own, (x + 1) * n_own): first, in groups of n_grp row blocks, column after
+// column of a group; then column after column over the n_last row blocks left of its own and every
+// kXcd-th item of the `n_tail_mblk` row blocks that nobody owns; then every kXcd-th item of the
+// columns without steps.
 constexpr int kXcd = 8;
 constexpr int kTicketInts = 16; // per slot: [0, kXcd) next index of each queue, [kXcd] workgroups done
 
@@ -87,9 +89,11 @@ struct GemmArgs {
     int32_t n_gemm_u;     // + pieces of units without (their columns receive beta * C)
     int32_t n_all_u;      // + tiles with pruned columns to fill
     int32_t n_own;        // row blocks owned by each queue
-    int32_t n_own_items;  // n_own * n_all_u
+    int32_t n_grp;        // ... worked off in groups of so many, tile after tile within a group
+    int32_t n_last;       // ... of which the last group has so many
+    int32_t n_lead_items; // (n_own - n_last) * n_pipe_u
     int32_t n_tail_mblk;  // n_mblk - kXcd * n_own
-    int32_t n_tail_items; // n_tail_mblk * n_all_u
+    int32_t n_list_items; // > 0: one list of so many items is dealt out over the queues instead
     float alpha, beta;
     const float *bias;    // fp32 [N] added to every written column before the activation, or null
     int32_t act;          // TW_ACT_*
@@ -103,7 +107,6 @@ struct GemmArgs {
     // of the packed weight, the sizes of the two buffers its loads are checked against.
     int32_t lds_dma;
     uint32_t a_bytes, b_bytes;
-    int32_t rb_major;     // the items no queue owns are dealt out row block after row block instead of column after column
     int32_t bal_first[kBalColumns + 1];
     int32_t bal_rows[kBalColumns];
     // Copy of `units` inside the kernel arguments for plans of at most kMaxArgUnits units
