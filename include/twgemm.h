@@ -520,6 +520,12 @@ int tw_prune_granularity(int K, int N, const float *scores, double sparsity, int
 int tw_prune_mix(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
                  const uint8_t *const *layer_masks, double g1percent, int q_type,
                  uint8_t *const *masks, double *threshold, void *stream);
+/* tiled_wise_1d_mix (prune_algo.py:182-186) in one call: the masks that tw_prune_tiled_wise_1d at
+ * `sparsity` (already with g1percent added) and tw_prune_mix on them give, without the masks between
+ * the two.  g1_q_type: the type of 100 - g1percent. */
+int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
+                               double sparsity, int q_type, int granularity, double g1percent, int g1_q_type,
+                               uint8_t *const *masks, double *threshold, void *stream);
 
 /* The building blocks of the two producers, on device buffers:
  *   tw_prune_tile_row_norms   norms[t*K + k] = ||scores[k][tile t]|| / width_t in NumPy's float32

@@ -326,3 +326,32 @@ def test_side_edge_cases_and_errors(tw):
             side.gemm(dA.data_ptr() + 2, dC.data_ptr(), M)
     with pytest.raises(ValueError):
         tw.Side(full, "f16", W[:, :3])
+
+
+@pytest.mark.parametrize("values", ["normal", "few_values", "huge"])
+@pytest.mark.parametrize("granularity", [128, 5, 2, 1000])
+def test_1d_mix_in_one_call(twprune, po, granularity, values):
+    """The masks without those of the first stage between the two: rows of whole and of odd numbers of fours,
+    tiles whose last one is one or two columns wide (no vectors), a layer off 16 bytes, layers of less than an
+    item and of whole items; the bracket holds the threshold, or misses (repeated values, the largest or next to
+    nothing kept beside the tiles) and the masks are made again from what the narrowing pass left."""
+    import torch
+    rng = np.random.default_rng(46)
+    shapes = [(512, 384), (577, 301), (64, 1002), (4096, 3), (9, 7)]
+    w = [rng.standard_normal(s).astype(np.float32) for s in shapes]
+    if values == "few_values":
+        w = [(np.round(x * 2) / 2).astype(np.float32) for x in w]
+    elif values == "huge":  # one square in fifty overflows: infinite scores, and a threshold among them
+        w = [np.where(rng.random(x.shape) < 0.02, x * 1e25, x).astype(np.float32) for x in w]
+    scores = twprune.img2col_forward(w)
+    dev = [torch.from_numpy(x).cuda() for x in scores]
+    off = torch.empty(dev[1].numel() + 1, device="cuda")[1:].view(dev[1].shape)  # starts 4 bytes behind a piece of 16
+    off.copy_(dev[1])
+    dev[1] = off
+    for sp, g1 in ((75, 5), (60.0, np.float64(12.5)), (90, 0.01), (40, 60), (50, 0)):
+        with np.errstate(all="ignore"):
+            want = po.tiled_wise_1d_mix(scores, sp, granularity, g1)
+        got = twprune.tiled_wise_1d_mix(dev, sp, granularity, g1, return_device=True)
+        for a, b in zip(want, got):
+            assert np.array_equal(np.asarray(a, bool), b.cpu().numpy().astype(bool)), (sp, g1, a.shape)
+            assert b.max() <= 1

@@ -357,7 +357,9 @@ struct SelectState {
     float lo, hi;                 // the bracket
     uint32_t room;                // values inside it that a wave can keep aside
     uint32_t key_base;            // the passes' digits are those of key - key_base,
-    int32_t key_bits;             // which has this many bits
+    int32_t key_bits;             // which has this many bits (up to 22: two passes hold them all, the third has nothing to do)
+    unsigned long long below;     // elements below the bracket,
+    int32_t narrowed;             // and whether the selection runs over those inside only
 };
 
 // Rank and weight of np.percentile(v[0..n), q): with q_is_f64 == 0 (q was a Python number) the
@@ -515,8 +517,9 @@ template <int NT> __device__ Threshold threshold_of(const SelectState *st)
     const uint32_t min_gt = st->min_gt;
     const uint32_t base = st->key_base;
     const KeyRange range(base, st->key_bits);
-    const uint32_t lead = st->prefix[2] << range.lead_shift(2);
-    const Digit d = find_digit<NT, 1024, true>(st->hist[2], st->rank[2]);
+    const bool two = st->key_bits <= 22;
+    const uint32_t lead = two ? st->prefix[1] << range.lead_shift(1) : st->prefix[2] << range.lead_shift(2);
+    const Digit d = two ? find_digit<NT, kSelBins, true>(st->hist[1], st->rank[1]) : find_digit<NT, 1024, true>(st->hist[2], st->rank[2]);
     if (threadIdx.x == 0) {
         const uint32_t key_a = base + (lead | d.digit);
         uint32_t key_b = key_a;
@@ -863,26 +866,37 @@ __global__ void __launch_bounds__(kPlanThreads)
 // to device memory, the histograms of `n_states` selections are cleared and, where n > 0, their ranks
 // worked out.  One launch (or a few, for tables of more than some twenty layers) instead of a copy
 // from host memory and the wait for it.
-constexpr int kBlobWords = 640;
+constexpr int kBlobWords = 960; // (a launch takes 4 KB of arguments)
 struct Blob {
     uint32_t w[kBlobWords];
 };
+struct SetupSelect {
+    SelectState *st;
+    int64_t n;
+    double q;
+    int32_t n_states, q_is_f64;
+    uint32_t room;
+    int32_t pad_;
+};
 __global__ void __launch_bounds__(256)
-    prune_setup_kernel(const Blob a, uint32_t *dst, int words, SelectState *st, int n_states, int64_t n, double q, int q_is_f64,
-                       uint32_t room)
+    prune_setup_kernel(const Blob a, uint32_t *dst, int words, const SetupSelect first, const SetupSelect second)
 {
     const auto *src = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
     const int gtid = (int)(blockIdx.x * blockDim.x + threadIdx.x), nthr = (int)(gridDim.x * blockDim.x);
     for (int i = gtid; i < words; i += nthr)
         dst[i] = src[i];
-    for (int g = 0; g < n_states; ++g) {
-        for (int i = gtid; i < 3 * kSelBins; i += nthr)
-            (&st[g].hist[0][0])[i] = 0;
-        if (gtid == 0 && n > 0) {
-            select_begin(&st[g], n, q, q_is_f64);
-            st[g].room = room;
+    auto begin = [&](const SetupSelect &p) {
+        for (int g = 0; g < p.n_states; ++g) {
+            for (int i = gtid; i < 3 * kSelBins; i += nthr)
+                (&p.st[g].hist[0][0])[i] = 0;
+            if (gtid == 0 && p.n > 0) {
+                select_begin(&p.st[g], p.n, p.q, p.q_is_f64);
+                p.st[g].room = p.room;
+            }
         }
-    }
+    };
+    begin(first);
+    begin(second);
 }
 
 // mask[k][c] = (norm of row k in c's tile > threshold) and column c kept.  A unit of work is 16
@@ -980,12 +994,24 @@ __global__ void __launch_bounds__(256)
 
 struct MixLayer {
     const float *score;
-    const uint8_t *mask0; // the TW mask of the layer
+    const uint8_t *mask0; // the TW mask of the layer, or nullptr: an element is kept where the norm of its row of its tile passes
+    const float *norms;   // [tiles][K]
     uint8_t *out;         // may be mask0 itself
     int64_t n;            // elements of the layer
     int64_t begin;        // its first element among all layers'
     int64_t item_begin;   // its first item in the launch-wide numbering
+    double per_n;         // 1 / N
+    float per_nf, per_g;  // 1 / N, 1 / G
+    int32_t K, N, G;      // G: columns of a tile
+    int32_t rows_on, cols_on; // 1024 / N, 1024 % N
+    int32_t in_fours;     // whole items are worked off as vectors: score, masks and output are aligned alike, and (norms) no tile is
+                          // narrower than three columns, so that four neighbours lie in two tiles or rows at most;
+                          // 2: in one, rows and tiles being made of fours
 };
+
+// Where the mask bytes of the elements come from: the caller's masks; the norms of the tiles' rows and
+// their threshold, for masks that nobody has written yet; a bit each that the narrowing pass has left.
+enum MixSource { MIX_BYTES, MIX_NORMS, MIX_BITS };
 
 // ||x|| of a single element (sqrt(x*x) / 1, the reference's norm over a tile of one column) minus 1
 // where the TW mask already keeps it (prune_algo.py:159-161).  The square root of a rounded square
@@ -1003,11 +1029,10 @@ __device__ __forceinline__ float mix_value(float x, uint32_t m0)
 }
 
 // The kernels of the mixed producer walk items of 4096 consecutive elements of a layer, sixteen per
-// thread, as vectors where score, mask and output are aligned alike.  The element scores are worked
-// out anew from weight and mask in every pass (five bytes an element, 158 MB for the layers of VGG16,
-// which the memory-side cache holds) rather than written to a pool and read back (eight bytes more,
-// once, and four in every pass).  At five bytes an element the vector instructions count as much as
-// the memory: a dozen per element are 10 us for 31.5 M elements.
+// thread, as vectors where the layer allows it.  The element scores are worked
+// out anew from weight and mask wherever they are needed rather than written to a pool and read back.  At
+// four or five bytes an element the vector instructions count as much as the memory: a dozen per element
+// are 10 us for 31.5 M elements.
 constexpr int kMixItem = 4096;
 struct MixFetched {
     TW_GLOBAL(const float) sc;
@@ -1016,28 +1041,93 @@ struct MixFetched {
     int n;
     bool vec;
     float4 x[4];
-    uint32_t m[4];
+    uint32_t m[4];   // mask bytes, any value but 0 counting as 1 (MIX_NORMS: how many of the four have the first norm)
+    float nv[4][2];  // MIX_NORMS: the norm of the first and of the last of four elements
+    uint32_t bits;   // MIX_BITS: the thread's sixteen elements
+    const MixLayer *layer;
+    int64_t e0;      // the item's first element
+    bool split;      // MIX_NORMS: four elements can lie in two tiles or rows
 };
-__device__ __forceinline__ void mix_fetch(const MixLayer &L, int64_t item, const float *safe, MixFetched &d)
+__device__ __forceinline__ bool mix_in_vectors(const MixLayer &L, int64_t e0) { return L.in_fours && L.n - e0 >= kMixItem; }
+// Layers whose elements are placed in rows and tiles with a multiplication in float: (x + 0.5) / N is off by less than
+// 0.5 / N for x below 2^22, and a product of two numbers below 2^24 is a full-rate instruction.
+constexpr int kMixMaxN = 1 << 21, kMixMaxK = 1 << 23;
+constexpr int64_t kMixMaxNorms = 1 << 29;
+struct MixCell {
+    uint32_t k, c; // row (from the layer's first), column
+    __device__ MixCell(const MixLayer &L, int64_t e0, uint32_t more) // element e0 + more
+    {
+        uint32_t k0 = (uint32_t)((double)e0 * L.per_n); // e0 / N, or one off
+        int32_t r0 = (int32_t)(e0 - (int64_t)k0 * L.N);
+        if (r0 < 0) {
+            --k0;
+            r0 += L.N;
+        } else if (r0 >= L.N) {
+            ++k0;
+            r0 -= L.N;
+        }
+        const uint32_t x = (uint32_t)r0 + more;
+        const uint32_t q = (uint32_t)(((float)x + 0.5f) * L.per_nf);
+        k = k0 + q;
+        c = x - __umul24(q, (uint32_t)L.N);
+    }
+    __device__ void on_1024(const MixLayer &L)
+    {
+        k += L.rows_on;
+        c += L.cols_on;
+        if (c >= (uint32_t)L.N) {
+            c -= L.N;
+            ++k;
+        }
+    }
+    __device__ uint32_t tile(const MixLayer &L) const { return (uint32_t)(((float)c + 0.5f) * L.per_g); }
+    __device__ uint32_t norm(const MixLayer &L, uint32_t t) const { return __umul24(t, (uint32_t)L.K) + k; }
+};
+template <int SRC>
+__device__ __forceinline__ void mix_fetch(const MixLayer &L, int64_t item, const uint16_t *bits, const float *safe, MixFetched &d)
 {
     const int64_t e0 = (item - L.item_begin) * kMixItem;
     d.n = (int)min((int64_t)kMixItem, L.n - e0);
     d.sc = as_global(L.score) + e0;
     d.mk = as_global(L.mask0) + e0;
     d.out = L.out + e0;
-    d.vec = d.n == kMixItem && ((uintptr_t)d.sc & 15) == 0 && (((uintptr_t)d.mk | (uintptr_t)d.out) & 3) == 0;
+    d.vec = mix_in_vectors(L, e0);
     // (an item that cannot be loaded in vectors loads something else in its place: with no load on a
     // condition the waits for them are exact counts)
     TW_GLOBAL(const u32x4) const x = d.vec ? (TW_GLOBAL(const u32x4))d.sc : (TW_GLOBAL(const u32x4))safe;
-    TW_GLOBAL(const uint32_t) const m = d.vec ? (TW_GLOBAL(const uint32_t))d.mk : (TW_GLOBAL(const uint32_t))safe;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 4; ++i)
         d.x[i] = __builtin_bit_cast(float4, x[threadIdx.x + i * 256]);
-        d.m[i] = m[threadIdx.x + i * 256];
+    if constexpr (SRC == MIX_BYTES) {
+        TW_GLOBAL(const uint32_t) const m = d.vec ? (TW_GLOBAL(const uint32_t))d.mk : (TW_GLOBAL(const uint32_t))safe;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            d.m[i] = m[threadIdx.x + i * 256];
+    } else if constexpr (SRC == MIX_BITS) {
+        d.bits = as_global(bits)[item * 256 + threadIdx.x];
+    } else {
+        d.layer = &L;
+        d.e0 = e0;
+        d.split = L.in_fours != 2;
+        TW_GLOBAL(const float) const nm = as_global(L.norms);
+        MixCell p(L, e0, d.vec ? threadIdx.x * 4 : 0u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t t = p.tile(L), at = p.norm(L, t);
+            d.nv[i][0] = nm[at];
+            if (d.split) {
+                const uint32_t end = min((t + 1) * (uint32_t)L.G, (uint32_t)L.N); // of the tile
+                d.m[i] = min(end - p.c, 4u);
+                d.nv[i][1] = nm[d.vec && d.m[i] < 4 ? (end == (uint32_t)L.N ? p.k + 1 : at + L.K) : at];
+            }
+            if (d.vec && i < 3)
+                p.on_1024(L);
+        }
     }
 }
-// f(values, mask bytes, output, count) per four (or single) elements
-template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d, F f)
+// f(values, mask bytes, output, count, place) per four (or single) elements; `place` and what is in sixty-fourths of it
+// tell the first one's place among the wave's elements of the item (see mix_place)
+template <int SRC, class F> __device__ __forceinline__ void mix_apply(const MixFetched &d, const Threshold &rows, F f)
 {
     if (d.vec) {
         float ax[4][4];
@@ -1068,42 +1158,74 @@ template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float v[4];
+            uint32_t m;
+            if constexpr (SRC == MIX_NORMS) {
+                const bool in = rows.passed_by(d.nv[i][0]);
+                m = in ? 0x01010101u : 0u;
+                if (d.split) {
+                    const uint32_t first = (uint32_t)((1ull << (d.m[i] * 8)) - 1ull); // bytes of the first tile
+                    m = (m & first) | (rows.passed_by(d.nv[i][1]) ? ~first & 0x01010101u : 0u);
+                }
+            } else if constexpr (SRC == MIX_BITS) {
+                m = ((d.bits >> (i * 4) & 15u) * 0x204081u) & 0x01010101u;
+            } else {
+                m = d.m[i];
+            }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) // (the mask byte, any value but 0 counting as 1)
-                v[e] = ax[i][e] - fminf((float)(d.m[i] >> (e * 8) & 255u), 1.0f);
-            f(v, d.m[i], d.out + (threadIdx.x + i * 256) * 4, 4);
+            for (int e = 0; e < 4; ++e) { // (the mask byte, any value but 0 counting as 1)
+                const float one = (float)(m >> (e * 8) & 255u);
+                v[e] = ax[i][e] - (SRC == MIX_BYTES ? fminf(one, 1.0f) : one);
+            }
+            f(v, m, d.out + (threadIdx.x + i * 256) * 4, 4, i << 8);
         }
     } else {
         // (whole waves make every round: f may look at its wave)
         for (int i0 = 0; i0 < d.n; i0 += 256) {
             const int i = i0 + (int)threadIdx.x, j = min(i, d.n - 1);
-            const uint32_t m0 = d.mk[j];
+            uint32_t m0;
+            if constexpr (SRC == MIX_NORMS) {
+                const MixCell p(*d.layer, d.e0, (uint32_t)j);
+                m0 = rows.passed_by(as_global(d.layer->norms)[p.norm(*d.layer, p.tile(*d.layer))]) ? 1u : 0u;
+            } else if constexpr (SRC == MIX_BITS) {
+                m0 = d.bits >> (i0 >> 8) & 1u;
+            } else {
+                m0 = d.mk[j];
+            }
             float v[4] = {mix_value(d.sc[j], m0), 0.0f, 0.0f, 0.0f};
-            f(v, m0, d.out + j, i < d.n ? 1 : 0);
+            f(v, m0, d.out + j, i < d.n ? 1 : 0, i0 >> 2);
         }
     }
 }
+// an element's place in its item, from its wave and the ten bits that `place` and the element's number among the four
+// (times 64) and its lane make
+__device__ __forceinline__ int mix_place(bool vec, int wave, uint32_t code)
+{
+    const int thread = wave * 64 + (int)(code & 63u);
+    return vec ? (thread + (int)(code >> 8 & 3u) * 256) * 4 + (int)(code >> 6 & 3u) : (int)(code >> 6 & 15u) * 256 + thread;
+}
 // All items of a launch, shared out over its workgroups, the next item's loads in flight while one is
-// worked on.  done() after every item;
-// safe: 16 KB of device memory that can be read.
-template <class F, class D>
-__device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layers, int64_t n_items, const float *safe, F f, D done)
+// worked on.  done(item) after every item;
+// bits: MIX_BITS; safe: 16 KB of device memory that can be read; rows(): MIX_NORMS, asked for once, after the first loads.
+template <int SRC, class R, class F, class D>
+__device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layers, int64_t n_items, const uint16_t *bits, const float *safe,
+                                             R rows_of, F f, D done)
 {
     const LayerFinder find(&layers->item_begin, sizeof(MixLayer), n_layers);
     MixFetched a, b;
     const int64_t step = gridDim.x, last = n_items - 1;
     int64_t item = blockIdx.x; // (a launch has at most n_items workgroups)
-    mix_fetch(layers[find(item)], item, safe, a);
+    mix_fetch<SRC>(layers[find(item)], item, bits, safe, a);
+    const Threshold rows = rows_of();
     for (;;) {
         const int64_t i1 = min(item + step, last), i2 = min(item + 2 * step, last);
-        mix_fetch(layers[find(i1)], i1, safe, b);
-        mix_apply(a, f);
-        done();
+        mix_fetch<SRC>(layers[find(i1)], i1, bits, safe, b);
+        mix_apply<SRC>(a, rows, f);
+        done(item);
         if (item + step > last)
             break;
-        mix_fetch(layers[find(i2)], i2, safe, a);
-        mix_apply(b, f);
-        done();
+        mix_fetch<SRC>(layers[find(i2)], i2, bits, safe, a);
+        mix_apply<SRC>(b, rows, f);
+        done(item + step);
         item += 2 * step;
         if (item > last)
             break;
@@ -1117,11 +1239,15 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // one case in a million, one pass over the elements counts what is below and keeps aside what is
 // between (2 - 3 % of the elements), and the three passes run over what was kept.
 // Where the bracket missed or does not fit - the counts tell, for certain - they run over the
-// elements.
+// elements.  The narrowing pass also writes the masks: what lies outside the bracket is decided
+// already, and the few per cent inside are marked one by one when the threshold is known, from the places kept
+// beside their values.
 // Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 11 + 31 + 31 us.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
-__global__ void __launch_bounds__(256) mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, uint32_t *sample)
+template <int SRC>
+__global__ void __launch_bounds__(256)
+    mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, const SelectState *st_rows, uint32_t *sample)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); // kMixSamples threads
     const int64_t at = total / kMixSamples * i;
@@ -1137,8 +1263,22 @@ __global__ void __launch_bounds__(256) mix_sample_kernel(const MixLayer *layers,
         else
             hi = mid;
     }
-    const int64_t j = e - layers[lo].begin;
-    sample[i] = sort_key(mix_value(layers[lo].score[j], layers[lo].mask0[j]));
+    const MixLayer &L = layers[lo];
+    const int64_t j = e - L.begin;
+    const float x = as_global(L.score)[j];
+    uint32_t m0;
+    if constexpr (SRC == MIX_NORMS) {
+        int64_t k = (int64_t)((double)j * L.per_n);
+        if (k * L.N > j)
+            --k;
+        else if ((k + 1) * L.N <= j)
+            ++k;
+        const float norm = as_global(L.norms)[(int64_t)((int)(j - k * L.N) / L.G) * L.K + k];
+        m0 = threshold_of<256>(st_rows).passed_by(norm) ? 1u : 0u;
+    } else {
+        m0 = L.mask0[j];
+    }
+    sample[i] = sort_key(mix_value(x, m0));
 }
 
 // The bracket out of the sample, one workgroup: the sample's values five standard deviations of their
@@ -1207,38 +1347,85 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
     }
 }
 
-// Below, between, above.  Every wave of the launch keeps the values between in a piece of the
-// candidates of its own and leaves its counts beside it: nothing is added up with atomics, of which the
+// Below, between, above.  Every wave of the launch keeps the values between, and where they are, in a piece
+// of the candidates of its own and leaves its counts beside it: nothing is added up with atomics, of which the
 // memory takes one in 15 ns on one address (a counter per workgroup that all add to was 25 us of this
-// kernel, one per wave 90).
+// kernel, one per wave 90).  The masks leave with it, as if nothing between were above the threshold; and a bit for
+// each element's mask0, which nobody can read any more where the masks are written in place, should the
+// bracket have missed.
 constexpr int kMixWgs = 1024, kMixWaves = kMixWgs * 4; // most workgroups and waves of a pass over the elements
 struct MixCounts {
     uint32_t between, below;
 };
-__global__ void __launch_bounds__(256)
-    mix_narrow_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, float *cand, MixCounts *counts)
+template <int SRC>
+__global__ void __launch_bounds__(256, 4)
+    mix_narrow_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st_rows, const SelectState *st, u32x2 *cand,
+                      MixCounts *counts, uint16_t *bits, Mail *mail)
 {
     const float lo = st->lo, hi = st->hi;
     const uint32_t room = st->room;
     const int lane = (int)(threadIdx.x & 63);
     const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-    TW_GLOBAL(float) const keep = as_global(cand) + (int64_t)w * room;
-    uint32_t kept = 0, below = 0; // wave-uniform
-    auto narrow = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const unsigned long long under = __ballot(e < cnt && v[e] < lo);
-            const unsigned long long in = __ballot(e < cnt && v[e] >= lo && v[e] <= hi);
-            below += __popcll(under);
-            if (in) {
-                const uint32_t at = kept + __popcll(in & ((1ull << lane) - 1ull));
-                if ((in >> lane & 1ull) && at < room) // (the count tells of an overflow)
-                    keep[at] = v[e];
-                kept += __popcll(in);
-            }
+    TW_GLOBAL(u32x2) const keep = as_global(cand) + (int64_t)w * room;
+    __shared__ __align__(16) float s_v[kMixItem];
+    uint32_t kept = 0, below = 0, round = 0; // wave-uniform
+    uint32_t mine = 0, inside = 0;           // mask0 of the thread's sixteen elements of the item; which are candidates
+    auto rows_of = [&]() {
+        if constexpr (SRC == MIX_NORMS) {
+            const Threshold t = threshold_of<256>(st_rows);
+            if (blockIdx.x == 0 && threadIdx.x == 0 && t.lost)
+                mail->lost = 1;
+            return t;
+        } else {
+            return Threshold{};
         }
     };
-    mix_for_each(layers, n_layers, n_items, cand, narrow, []() {});
+    auto narrow = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt, int at0) {
+        const int slot = at0 >> 6; // of the thread's sixteen
+        float *const sv = s_v + ((slot >> 2) * 256 + (int)threadIdx.x) * 4;
+        if (cnt == 4) {
+            *reinterpret_cast<float4 *>(sv) = float4{v[0], v[1], v[2], v[3]};
+            uint32_t in = 0, over = 0; // a bit an element, the last one lowest
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                below += __popcll(__ballot(v[e] < lo));
+                in = in + in + (v[e] >= lo && v[e] <= hi ? 1u : 0u);
+                over = over + over + (v[e] > hi ? 1u : 0u);
+            }
+            inside |= (__brev(in) >> 28) << slot;
+            const uint32_t o = SRC == MIX_NORMS ? m : ((m & 0x7F7F7F7Fu) + 0x7F7F7F7Fu | m) >> 7 & 0x01010101u; // mask bytes that are not 0
+            mine |= (o * 0x10204080u >> 28) << slot;
+            *(TW_GLOBAL(uint32_t))out = o | (((__brev(over) >> 28) * 0x204081u) & 0x01010101u);
+        } else {
+            sv[slot & 3] = v[0];
+            below += __popcll(__ballot(cnt && v[0] < lo));
+            inside |= (cnt && v[0] >= lo && v[0] <= hi ? 1u : 0u) << slot;
+            mine |= (m ? 1u : 0u) << slot;
+            if (cnt)
+                *as_global(out) = m || v[0] > hi ? 1 : 0;
+        }
+    };
+    // The candidates of an item, one of every lane that has one left at a time: a lane has half of one among its
+    // sixteen elements, so that three or four rounds do for what were sixteen (46 us so, 72 with the test behind each
+    // element).
+    auto item_done = [&](int64_t item) {
+        for (;;) {
+            const bool some = inside != 0;
+            const unsigned long long in = __ballot(some);
+            if (!in)
+                break;
+            const uint32_t slot = some ? (uint32_t)__builtin_ctz(inside) : 0u;
+            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, kept));
+            if (some && at < room) // (the count tells of an overflow)
+                keep[at] = u32x2{__float_as_uint(s_v[((slot >> 2) * 256 + threadIdx.x) * 4 + (slot & 3)]), round << 10 | slot << 6 | (uint32_t)lane};
+            kept += __popcll(in);
+            inside &= inside - 1;
+        }
+        as_global(bits)[item * 256 + threadIdx.x] = (uint16_t)mine;
+        mine = 0;
+        ++round;
+    };
+    mix_for_each<SRC>(layers, n_layers, n_items, nullptr, reinterpret_cast<const float *>(cand), rows_of, narrow, item_done);
     if (lane == 0)
         counts[w] = MixCounts{kept, below};
 }
@@ -1284,9 +1471,11 @@ constexpr int kMixHistWgs = 96; // workgroups that count what was kept (each add
 static_assert(kMixWaves <= 64 * 4 * kMixHistWgs, "a lane for each piece of a wave");
 template <int PASS>
 __global__ void __launch_bounds__(256)
-    mix_hist_kernel(const MixLayer *layers, int n_layers, int64_t n_items, SelectState *st, const float *cand,
-                    const MixCounts *counts, int waves)
+    mix_hist_kernel(const MixLayer *layers, int n_layers, int64_t n_items, SelectState *st, const u32x2 *cand,
+                    const MixCounts *counts, int waves, const uint16_t *bits)
 {
+    if (PASS == 2 && st->key_bits <= 22)
+        return; // (two digits hold all of the range)
     __shared__ unsigned int s_h[kSelBins];
     __shared__ uint32_t s_min;
     uint32_t prefix, mn = 0xFFFFFFFFu;
@@ -1298,20 +1487,28 @@ __global__ void __launch_bounds__(256)
     const int mine = w0 < min(per, waves) ? (waves - w0 + per - 1) / per : 0;
     const uint32_t held = lane < mine ? counts[w0 + lane * per].between : 0u;
     unsigned long long n_cand, below;
-    const bool whole = mix_totals(counts, waves, room, n_cand, below);
-    // the wanted value and the one above it lie inside the bracket, and all of that was kept
-    const bool narrowed = whole && below <= want && (want - below) + 1 < n_cand;
+    bool narrowed;
+    if (PASS == 0) {
+        const bool whole = mix_totals(counts, waves, room, n_cand, below);
+        // the wanted value and the one above it lie inside the bracket, and all of that was kept
+        narrowed = whole && below <= want && (want - below) + 1 < n_cand;
+    } else {
+        below = st->below;
+        narrowed = st->narrowed != 0;
+    }
     if (narrowed && blockIdx.x >= kMixHistWgs)
         return;
     // (-0 and +0 are one value to the comparisons with the bracket, and two keys)
     const uint32_t lo = narrowed ? sort_key(st->lo == 0.0f ? -0.0f : st->lo) : 0u;
     const uint32_t span = narrowed ? sort_key(st->hi == 0.0f ? 0.0f : st->hi) - lo : 0xFFFFFFFFu;
-    const int bits = span ? 32 - __clz(span) : 1;
-    const KeyRange range(lo, bits);
+    const int key_bits = span ? 32 - __clz(span) : 1;
+    const KeyRange range(lo, key_bits);
     select_enter<PASS, 256>(st, range, s_h, &s_min, narrowed ? want - below : want, prefix, rank);
-    if (PASS == 2 && blockIdx.x == 0 && threadIdx.x == 0) {
+    if (PASS == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
         st->key_base = lo;
-        st->key_bits = bits;
+        st->key_bits = key_bits;
+        st->below = below;
+        st->narrowed = narrowed;
     }
     if (narrowed) {
         // four pieces at a time, sixteen loads in flight: a piece holds some two hundred values, and one piece after the other,
@@ -1319,7 +1516,7 @@ __global__ void __launch_bounds__(256)
         // 11; what is left are the counts of all waves, the digits so far and the counters' atomics: 48 workgroups 12 + 15 + 15,
         // 192 10 + 10 + 10, 256 12 + 10 + 10)
         for (int q0 = 0; q0 < mine; q0 += 4) {
-            TW_GLOBAL(const float) v[4];
+            TW_GLOBAL(const u32x2) v[4];
             uint32_t n[4];
             float x[4][4];
 #pragma unroll
@@ -1328,7 +1525,7 @@ __global__ void __launch_bounds__(256)
                 v[q] = as_global(cand) + (int64_t)(w0 + min(q0 + q, mine - 1) * per) * room;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    x[q][e] = v[q][min((uint32_t)(lane + e * 64), max(n[q], 1u) - 1u)];
+                    x[q][e] = __uint_as_float(v[q][min((uint32_t)(lane + e * 64), max(n[q], 1u) - 1u)].x);
             }
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -1340,7 +1537,7 @@ __global__ void __launch_bounds__(256)
                     float y[4];
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        y[e] = v[q][min(i + e * 64, n[q] - 1)];
+                        y[e] = __uint_as_float(v[q][min(i + e * 64, n[q] - 1)].x);
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
                         if (i + e * 64 < n[q])
@@ -1349,40 +1546,98 @@ __global__ void __launch_bounds__(256)
             }
         }
     } else {
-        auto count = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt) {
+        auto count = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt, int) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (e < cnt)
                     select_count<PASS>(sort_key(v[e]), range, prefix, s_h, mn);
         };
-        mix_for_each(layers, n_layers, n_items, cand, count, []() {});
+        mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() { return Threshold{}; }, count, [](int64_t) {});
     }
     select_leave<PASS, 256>(st, s_h, &s_min, mn);
 }
 
-// out = mask0 | (score > threshold)   (prune_algo.py:171-176)
+constexpr int kMarkLayers = 128;
+// out = mask0 | (score > threshold)   (prune_algo.py:171-176): the candidates above the threshold, a wave for each
+// piece of them; all elements where the selection ran over all
 __global__ void __launch_bounds__(256)
-    mix_mask_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, const float *safe, Mail *mail)
+    mix_mark_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st, const u32x2 *cand,
+                    const MixCounts *counts, const uint16_t *bits, Mail *mail)
 {
+    // what a candidate's place is worked out from, for the first kMarkLayers layers: a look-up is a few reads of LDS then,
+    // instead of as many trips to memory
+    __shared__ int64_t s_item[kMarkLayers], s_n[kMarkLayers];
+    __shared__ uint8_t *s_out[kMarkLayers];
+    __shared__ int s_fours[kMarkLayers];
+    const int staged = min(n_layers, kMarkLayers);
+    for (int l = (int)threadIdx.x; l < staged; l += 256) {
+        s_item[l] = layers[l].item_begin;
+        s_n[l] = layers[l].n;
+        s_out[l] = layers[l].out;
+        s_fours[l] = layers[l].in_fours;
+    }
     const Threshold thr = threshold_of<256>(st);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         mail->thr_rows = thr.v64;
         if (thr.lost)
             mail->lost = 1;
     }
-    auto above = [&](float v) { return thr.passed_by(v); };
-    auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt) {
-        if (cnt == 4) {
-            uint32_t o = ((m & 0x7F7F7F7Fu) + 0x7F7F7F7Fu | m) >> 7 & 0x01010101u; // mask bytes that are not 0
+    if (st->narrowed) { // (the grid is the narrowing pass's)
+        const int wave = (int)(threadIdx.x >> 6), lane = (int)(threadIdx.x & 63);
+        const int64_t w = (int64_t)blockIdx.x * 4 + wave;
+        const uint32_t room = st->room, n = counts[w].between;
+        TW_GLOBAL(const u32x2) const v = as_global(cand) + w * room;
+        for (uint32_t i0 = 0; i0 < n; i0 += 256) {
+            u32x2 c[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                o |= above(v[e]) ? 1u << (e * 8) : 0u;
-            *(TW_GLOBAL(uint32_t))out = o;
+                c[e] = v[min(i0 + e * 64 + lane, n - 1)];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (i0 + e * 64 + lane >= n || !thr.passed_by(__uint_as_float(c[e].x)))
+                    continue;
+                const int64_t item = blockIdx.x + (int64_t)(c[e].y >> 10) * gridDim.x;
+                int lo = 0, hi = staged;
+                while (hi - lo > 1) {
+                    const int mid = (lo + hi) >> 1;
+                    if (s_item[mid] <= item)
+                        lo = mid;
+                    else
+                        hi = mid;
+                }
+                int64_t e0 = (item - s_item[lo]) * kMixItem, left = s_n[lo] - e0;
+                uint8_t *out = s_out[lo];
+                int fours = s_fours[lo];
+                if (left <= 0) { // (beyond the staged layers)
+                    hi = n_layers;
+                    while (hi - lo > 1) {
+                        const int mid = (lo + hi) >> 1;
+                        if (layers[mid].item_begin <= item)
+                            lo = mid;
+                        else
+                            hi = mid;
+                    }
+                    e0 = (item - layers[lo].item_begin) * kMixItem;
+                    left = layers[lo].n - e0;
+                    out = layers[lo].out;
+                    fours = layers[lo].in_fours;
+                }
+                as_global(out)[e0 + mix_place(fours && left >= kMixItem, wave, c[e].y)] = 1;
+            }
+        }
+        return;
+    }
+    auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt, int) {
+        if (cnt == 4) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                m |= thr.passed_by(v[e]) ? 1u << (e * 8) : 0u;
+            *(TW_GLOBAL(uint32_t))out = m;
         } else if (cnt == 1) {
-            *as_global(out) = (m || above(v[0])) ? 1 : 0;
+            *as_global(out) = (m || thr.passed_by(v[0])) ? 1 : 0;
         }
     };
-    mix_for_each(layers, n_layers, n_items, safe, mark, []() {});
+    mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() { return Threshold{}; }, mark, [](int64_t) {});
 }
 
 // ---------------------------------------------------------------------------------
@@ -1483,22 +1738,24 @@ private:
 };
 
 // `bytes` of a host table to the device through kernel arguments, and the selections cleared
-int put_table(const void *table, size_t bytes, void *dst, SelectState *st, int n_states, int64_t n, double q,
-              int q_is_f64, hipStream_t s, uint32_t room = 0)
+int put_table(const void *table, size_t bytes, void *dst, SetupSelect first, SetupSelect second, hipStream_t s)
 {
     size_t off = 0;
     do {
         Blob a;
         const size_t take = std::min(bytes - off, sizeof(a.w));
         std::memcpy(a.w, static_cast<const char *>(table) + off, take);
-        hipLaunchKernelGGL(prune_setup_kernel, dim3(n_states > 4 ? 128 : 16), dim3(256), 0, s, a,
-                           reinterpret_cast<uint32_t *>(static_cast<char *>(dst) + off), (int)((take + 3) / 4), st, n_states,
-                           n, q, q_is_f64, room);
-        n_states = 0; // (the selections once)
+        hipLaunchKernelGGL(prune_setup_kernel, dim3(first.n_states > 4 ? 128 : 16), dim3(256), 0, s, a,
+                           reinterpret_cast<uint32_t *>(static_cast<char *>(dst) + off), (int)((take + 3) / 4), first, second);
+        first.n_states = second.n_states = 0; // (the selections once)
         off += take;
     } while (off < bytes);
     TW_HIP(hipGetLastError());
     return TW_OK;
+}
+SetupSelect setup_of(SelectState *st, int n_states, int64_t n, double q, int q_is_f64, uint32_t room = 0)
+{
+    return SetupSelect{st, n, q, n_states, q_is_f64, room, 0};
 }
 
 int check_percentile(int64_t n, double q)
@@ -1607,8 +1864,8 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
         e.norms = d_norms + off;
         off += (int64_t)e.K * e.n_tiles;
     }
-    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q,
-                   q_is_f64, s);
+    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table,
+                   setup_of(d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q, q_is_f64), SetupSelect{}, s);
     if (st)
         return st;
     hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers,
@@ -1632,6 +1889,96 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
         *threshold = mail->thr_rows;
     return st;
 }
+
+// The second stage of the mixed producers (tw_mix_fn): its buffers, its table of the layers, and the launches behind it.
+class MixCall {
+public:
+    // `masks0` or, where that is nullptr, `rows`: the table of a first stage whose masks nobody has written (norms and tiles)
+    int plan(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, const uint8_t *const *masks0,
+             const CallTable *rows, uint8_t *const *masks, double q, int q_type)
+    {
+        layers_.resize(n_layers);
+        for (int l = 0; l < n_layers; ++l) {
+            MixLayer &e = layers_[l];
+            std::memset(&e, 0, sizeof(e));
+            e.score = scores[l];
+            e.mask0 = masks0 ? masks0[l] : nullptr;
+            e.out = masks[l];
+            e.n = (int64_t)K[l] * N[l];
+            e.begin = total_;
+            e.item_begin = n_items_;
+            e.K = K[l];
+            e.N = N[l];
+            e.G = rows ? rows->layers[l].granularity : 1;
+            e.per_n = 1.0 / N[l];
+            e.per_nf = 1.0f / (float)N[l];
+            e.per_g = 1.0f / (float)e.G;
+            e.rows_on = kMixItem / 4 / N[l];
+            e.cols_on = kMixItem / 4 % N[l];
+            const bool wide = masks0 || (e.G >= 3 && N[l] >= 3 && (N[l] % e.G == 0 || N[l] % e.G >= 3));
+            if (((uintptr_t)e.score & 15) == 0 && (((uintptr_t)e.mask0 | (uintptr_t)e.out) & 3) == 0 && wide)
+                e.in_fours = N[l] % 4 == 0 && e.G % 4 == 0 ? 2 : 1;
+            total_ += e.n;
+            n_items_ += (e.n + kMixItem - 1) / kMixItem;
+        }
+        q_ = q;
+        q_type_ = q_type;
+        return check_percentile(total_, q);
+    }
+    int alloc(Arena &ar)
+    {
+        // room for the values inside the bracket: an eighth of the elements, and all of a small network's
+        wgs_ = (int)std::min<int64_t>(n_items_, kMixWgs);
+        const int64_t share = (n_items_ + wgs_ - 1) / wgs_ * (kMixItem / 4); // elements of a wave
+        room_ = (uint32_t)(total_ > kMixSampleFrom ? std::max<int64_t>(share / 8, 512) : share);
+        d_cand_ = ar.alloc_n<u32x2>((size_t)wgs_ * 4 * room_);
+        d_counts_ = ar.alloc_n<MixCounts>(wgs_ * 4);
+        d_bits_ = ar.alloc_n<uint16_t>((size_t)n_items_ * 256);
+        d_sample_ = ar.alloc_n<uint32_t>(kMixSamples);
+        d_st_ = ar.alloc_n<SelectState>(1);
+        if (!d_cand_ || !d_counts_ || !d_bits_ || !d_sample_ || !d_st_)
+            return fail(TW_ERR_ALLOC, "allocation for %lld element scores failed", (long long)total_);
+        return TW_OK;
+    }
+    size_t table_bytes() const { return sizeof(MixLayer) * layers_.size(); }
+    std::vector<MixLayer> &table() { return layers_; }
+    SetupSelect setup() const { return setup_of(d_st_, 1, total_, q_, q_type_, room_); }
+    // behind put_table of the table (at d_layers on the device) and, with SRC == MIX_NORMS, the passes of the selection of `st_rows`
+    template <int SRC> int queue(const MixLayer *d_layers, const SelectState *st_rows, Mail *mail, hipStream_t s)
+    {
+        const int n_layers = (int)layers_.size(), waves = wgs_ * 4;
+        if (total_ > kMixSampleFrom) {
+            hipLaunchKernelGGL(mix_sample_kernel<SRC>, dim3(kMixSamples / 256), dim3(256), 0, s, d_layers, n_layers, total_, st_rows,
+                               d_sample_);
+            hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample_, d_st_);
+        }
+        hipLaunchKernelGGL(mix_narrow_kernel<SRC>, dim3(wgs_), dim3(256), 0, s, d_layers, n_layers, n_items_, st_rows, d_st_, d_cand_,
+                           d_counts_, d_bits_, mail);
+        const dim3 grid((unsigned)std::min<int64_t>(n_items_, 512));
+        hipLaunchKernelGGL(mix_hist_kernel<0>, grid, dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_, d_counts_, waves,
+                           d_bits_);
+        hipLaunchKernelGGL(mix_hist_kernel<1>, grid, dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_, d_counts_, waves,
+                           d_bits_);
+        hipLaunchKernelGGL(mix_hist_kernel<2>, grid, dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_, d_counts_, waves,
+                           d_bits_);
+        hipLaunchKernelGGL(mix_mark_kernel, dim3(wgs_), dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_,
+                           d_counts_, d_bits_, mail);
+        TW_HIP(hipGetLastError());
+        return TW_OK;
+    }
+
+private:
+    std::vector<MixLayer> layers_;
+    int64_t total_ = 0, n_items_ = 0;
+    double q_ = 0.0;
+    int q_type_ = 0, wgs_ = 0;
+    uint32_t room_ = 0;
+    u32x2 *d_cand_ = nullptr;
+    uint32_t *d_sample_ = nullptr;
+    MixCounts *d_counts_ = nullptr;
+    uint16_t *d_bits_ = nullptr;
+    SelectState *d_st_ = nullptr;
+};
 
 } // namespace
 
@@ -1729,9 +2076,9 @@ try {
     e.K = K;
     e.N = N;
     e.n_tiles = n_tiles;
-    st = put_table(tcol0.data(), sizeof(int32_t) * (n_tiles + 1), d_tab, nullptr, 0, 0, 0.0, 0, s);
+    st = put_table(tcol0.data(), sizeof(int32_t) * (n_tiles + 1), d_tab, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (!st)
-        st = put_table(&e, sizeof(e), d_table, nullptr, 0, 0, 0.0, 0, s);
+        st = put_table(&e, sizeof(e), d_table, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (st)
         return st;
     hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)n_items), dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr);
@@ -1752,7 +2099,7 @@ try {
     if (!d_cl)
         return fail(TW_ERR_ALLOC, "hipMalloc of the layer table failed");
     const ColLayer cl{scores, K, N, 0, 0};
-    const int st = put_table(&cl, sizeof(cl), d_cl, nullptr, 0, 0, 0.0, 0, s);
+    const int st = put_table(&cl, sizeof(cl), d_cl, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (st)
         return st;
     hipLaunchKernelGGL(col_norms_kernel, dim3((N + kColCols - 1) / kColCols), dim3(kColThreads), 0, s, d_cl, 1, norms);
@@ -1778,7 +2125,7 @@ try {
     Mail *mail = ar.mail();
     if (!d_st || !d_thr || !mail)
         return fail(TW_ERR_ALLOC, "allocation of the selection state failed");
-    st = put_table(nullptr, 0, d_st, d_st, 1, n, q, q_type, s);
+    st = put_table(nullptr, 0, d_st, setup_of(d_st, 1, n, q, q_type), SetupSelect{}, s);
     if (!st)
         st = queue_select(values, n, d_st, 1, s);
     if (st)
@@ -1875,7 +2222,7 @@ try {
         n_blk += (N[l] + kColCols - 1) / kColCols;
     }
     std::memcpy(both.data(), c.layers.data(), table_bytes);
-    st = put_table(both.data(), both.size(), d_tables, d_st, 1, 0, q, q_type, s);
+    st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, 0, q, q_type), SetupSelect{}, s);
     if (st)
         return st;
     hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)n_blk), dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm);
@@ -1908,48 +2255,88 @@ try {
         return fail(TW_ERR_NULL, "layer_masks is NULL");
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
-    hipStream_t s = (hipStream_t)stream;
-    std::vector<MixLayer> ml(n_layers);
-    int64_t total = 0, n_items = 0;
-    for (int l = 0; l < n_layers; ++l) {
+    for (int l = 0; l < n_layers; ++l)
         if (!layer_masks[l])
             return fail(TW_ERR_NULL, "layer %d: layer mask pointer is NULL", l);
-        ml[l] = MixLayer{scores[l], layer_masks[l], masks[l], (int64_t)K[l] * N[l], total, n_items};
-        total += ml[l].n;
-        n_items += (ml[l].n + kMixItem - 1) / kMixItem;
-    }
-    const double q = 100.0 - g1percent;
-    st = check_percentile(total, q);
+    hipStream_t s = (hipStream_t)stream;
+    MixCall mix;
+    st = mix.plan(n_layers, K, N, scores, layer_masks, nullptr, masks, 100.0 - g1percent, q_type);
     if (st)
         return st;
     Arena ar(s);
-    // room for the values inside the bracket: an eighth of the elements, and all of a small network's
-    const int wgs = (int)std::min<int64_t>(n_items, kMixWgs), waves = wgs * 4;
-    const int64_t share = (n_items + wgs - 1) / wgs * (kMixItem / 4); // elements of a wave
-    const uint32_t room = (uint32_t)(total > kMixSampleFrom ? std::max<int64_t>(share / 8, 512) : share);
-    float *d_cand = ar.alloc_n<float>((size_t)waves * room);
-    MixCounts *d_counts = ar.alloc_n<MixCounts>(waves);
-    uint32_t *d_sample = ar.alloc_n<uint32_t>(kMixSamples);
+    st = mix.alloc(ar);
     MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
-    SelectState *d_st = ar.alloc_n<SelectState>(1);
     Mail *mail = ar.mail();
-    if (!d_cand || !d_counts || !d_sample || !d_layers || !d_st || !mail)
-        return fail(TW_ERR_ALLOC, "allocation for %lld element scores failed", (long long)total);
-    st = put_table(ml.data(), sizeof(MixLayer) * n_layers, d_layers, d_st, 1, total, q, q_type, s, room);
+    if (!st && (!d_layers || !mail))
+        st = fail(TW_ERR_ALLOC, "allocation for %d layers failed", n_layers);
+    if (!st)
+        st = put_table(mix.table().data(), mix.table_bytes(), d_layers, mix.setup(), SetupSelect{}, s);
+    if (!st)
+        st = mix.queue<MIX_BYTES>(d_layers, nullptr, mail, s);
     if (st)
         return st;
-    if (total > kMixSampleFrom) {
-        hipLaunchKernelGGL(mix_sample_kernel, dim3(kMixSamples / 256), dim3(256), 0, s, d_layers, n_layers, total, d_sample);
-        hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample, d_st);
+    st = ar.wait();
+    if (!st && threshold)
+        *threshold = mail->thr_rows;
+    return st;
+}
+TW_CATCH_TO_STATUS
+
+int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double sparsity,
+                               int q_type, int granularity, double g1percent, int g1_q_type, uint8_t *const *masks,
+                               double *threshold, void *stream)
+try {
+    int st = check_layers(n_layers, K, N, scores, masks, granularity);
+    if (st)
+        return st;
+    if ((q_type != TW_Q_F32 && q_type != TW_Q_F64) || (g1_q_type != TW_Q_F32 && g1_q_type != TW_Q_F64))
+        return fail(TW_ERR_LAYOUT, "q_type=%d, %d: unknown", q_type, g1_q_type);
+    for (int l = 0; l < n_layers; ++l)
+        if (N[l] > kMixMaxN || K[l] > kMixMaxK || (N[l] + (int64_t)granularity - 1) / granularity * K[l] > kMixMaxNorms) { // one stage after the other
+            st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, masks, nullptr, (hipStream_t)stream, 0);
+            return st ? st : tw_prune_mix(n_layers, K, N, scores, masks, g1percent, g1_q_type, masks, threshold, stream);
+        }
+    hipStream_t s = (hipStream_t)stream;
+    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, 0);
+    MixCall mix;
+    st = check_percentile(c.n_norms, sparsity);
+    if (!st)
+        st = too_large(c.n_items);
+    if (!st)
+        st = mix.plan(n_layers, K, N, scores, nullptr, &c, masks, 100.0 - g1percent, g1_q_type);
+    if (st)
+        return st;
+    Arena ar(s);
+    float *d_norms = ar.alloc_n<float>(c.n_norms);
+    SelectState *d_st = ar.alloc_n<SelectState>(1);
+    const size_t table_bytes = sizeof(PruneLayer) * n_layers;
+    char *d_tables = static_cast<char *>(ar.alloc(table_bytes + mix.table_bytes()));
+    Mail *mail = ar.mail();
+    if (!d_norms || !d_st || !d_tables || !mail)
+        return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
+    st = mix.alloc(ar);
+    if (st)
+        return st;
+    const PruneLayer *d_table = reinterpret_cast<const PruneLayer *>(d_tables);
+    const MixLayer *d_layers = reinterpret_cast<const MixLayer *>(d_tables + table_bytes);
+    int64_t off = 0;
+    for (int l = 0; l < n_layers; ++l) {
+        c.layers[l].norms = d_norms + off;
+        mix.table()[l].norms = d_norms + off;
+        off += (int64_t)K[l] * c.layers[l].n_tiles;
     }
-    hipLaunchKernelGGL(mix_narrow_kernel, dim3(wgs), dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts);
-    const dim3 grid((unsigned)std::min<int64_t>(n_items, 512));
-    hipLaunchKernelGGL(mix_hist_kernel<0>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
-    hipLaunchKernelGGL(mix_hist_kernel<1>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
-    hipLaunchKernelGGL(mix_hist_kernel<2>, grid, dim3(256), 0, s, d_layers, n_layers, n_items, d_st, d_cand, d_counts, waves);
-    hipLaunchKernelGGL(mix_mask_kernel, dim3((unsigned)std::min<int64_t>(n_items, 2048)), dim3(256), 0, s, d_layers, n_layers,
-                       n_items, d_st, d_cand, mail);
-    TW_HIP(hipGetLastError());
+    std::vector<char> both(table_bytes + mix.table_bytes());
+    std::memcpy(both.data(), c.layers.data(), table_bytes);
+    std::memcpy(both.data() + table_bytes, mix.table().data(), mix.table_bytes());
+    st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
+    if (st)
+        return st;
+    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, (const int64_t *)nullptr);
+    st = queue_select(d_norms, c.n_norms, d_st, 1, s);
+    if (!st)
+        st = mix.queue<MIX_NORMS>(d_layers, d_st, mail, s);
+    if (st)
+        return st;
     st = ar.wait();
     if (!st && threshold)
         *threshold = mail->thr_rows;

@@ -166,12 +166,14 @@ def tw_mix_fn(accumulated_scores, g1percent, layer_mask, return_device=False):
 def tiled_wise_1d_mix(accumulated_scores, sparsity, granularity=128, g1percent=5, return_device=False):
     """prune_algo.py:182-186: tiled_wise_1d at sparsity + g1percent, then tw_mix_fn."""
     d = _DeviceLayers(accumulated_scores)
-    q = sparsity + g1percent
-    tw._check(tw.lib().tw_prune_tiled_wise_1d(
+    q, thr = sparsity + g1percent, ctypes.c_double()
+    tw._check(tw.lib().tw_prune_tiled_wise_1d_mix(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
-        ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(q), _q_type(q),
-        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), None, d.stream))
-    return _mix(d, g1percent, return_device)
+        ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(q), _q_type(q), int(granularity),
+        float(g1percent), _q_type(100 - g1percent), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)),
+        ctypes.byref(thr), d.stream))
+    tw_mix_fn.last_threshold = thr.value
+    return d.d_masks if return_device else d.masks()
 
 
 def tiled_wise_2d_mix(accumulated_scores, sparsity, granularity=128, g1percent=1, return_device=False):
