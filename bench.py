@@ -436,7 +436,7 @@ def bench_producers(steps, warmup, torch):
     rng = np.random.default_rng(20200615)
     scores = [np.abs(rng.standard_normal(s)).astype(np.float32) for s in PRODUCER_LAYERS]
     elems = sum(k * n for k, n in PRODUCER_LAYERS)
-    d = twprune._DeviceLayers(scores)
+    d = twprune._DeviceLayers(scores).make_masks()
     L = tw.lib()
     pp = ctypes.POINTER(ctypes.c_void_p)
     i32 = ctypes.c_int32

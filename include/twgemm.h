@@ -527,6 +527,23 @@ int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N,
                                double sparsity, int q_type, int granularity, double g1percent, int g1_q_type,
                                uint8_t *const *masks, double *threshold, void *stream);
 
+/* The three with masks that the caller allocates while the first kernels run: `ready(user)` is called once,
+ * on the calling thread, when those are queued, and has put the masks' addresses into `masks` when it
+ * returns 0; any other value ends the call with TW_ERR_ALLOC.  It calls no producer itself.  ready ==
+ * NULL: as above. */
+typedef int (*tw_masks_ready)(void *user);
+int tw_prune_tiled_wise_1d_late(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
+                                double sparsity, int q_type, int granularity, uint8_t *const *masks,
+                                tw_masks_ready ready, void *user, double *threshold, void *stream);
+int tw_prune_tiled_wise_2d_late(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
+                                double sparsity, int q_type, int transform, int granularity,
+                                uint8_t *const *masks, tw_masks_ready ready, void *user,
+                                uint8_t *const *col_masks, double *thresholds, void *stream);
+int tw_prune_tiled_wise_1d_mix_late(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
+                                    double sparsity, int q_type, int granularity, double g1percent,
+                                    int g1_q_type, uint8_t *const *masks, tw_masks_ready ready, void *user,
+                                    double *threshold, void *stream);
+
 /* The building blocks of the two producers, on device buffers:
  *   tw_prune_tile_row_norms   norms[t*K + k] = ||scores[k][tile t]|| / width_t in NumPy's float32
  *                             summation order; col_keep (optional, N bytes) zeroes pruned

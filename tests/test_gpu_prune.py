@@ -243,3 +243,32 @@ def test_error_paths(tw, twprune):
         twprune.granularity_pruning(np.ones((4, 6), np.float32), 50, 4)
     with pytest.raises(tw.TwError):
         tw.Plan.from_mask_tiles(np.ones((4, 8), np.uint8), [(0, 4), (5, 3)], "f16", np.ones((4, 8), np.float32))
+
+
+@pytest.mark.parametrize("n_layers", [1, 128, 129])
+def test_masks_of_many_layers_made_during_the_call(twprune, po, n_layers):
+    """As many layers as a launch takes addresses of masks, and one more (whose addresses go to the table)."""
+    rng = np.random.default_rng(n_layers)
+    scores = twprune.img2col_forward([rng.standard_normal((int(rng.integers(3, 40)), int(rng.integers(3, 50)))).astype(np.float32)
+                                      for _ in range(n_layers)])
+    for fn in ("tiled_wise_1d", "tiled_wise_2d", "tiled_wise_1d_mix"):
+        want = getattr(po, fn)(scores, 60, 16)
+        want = want[0] if fn != "tiled_wise_1d_mix" else want
+        got = getattr(twprune, fn)(scores, 60, 16)
+        assert len(got) == n_layers and all(np.array_equal(w, g) for w, g in zip(want, got)), fn
+
+
+@pytest.mark.parametrize("fn", ["tiled_wise_1d", "tiled_wise_2d", "tiled_wise_1d_mix"])
+def test_masks_that_cannot_be_made_end_the_call(tw, twprune, monkeypatch, fn):
+    """An exception while the masks are made comes out of the producer, and the next call is as ever."""
+    rng = np.random.default_rng(3)
+    scores = [rng.random((64, 96)).astype(np.float32)]
+    want = getattr(twprune, fn)(scores, 50, 32)
+
+    def fails(self):
+        raise MemoryError("no masks")
+    with monkeypatch.context() as m:
+        m.setattr(twprune._DeviceLayers, "make_masks", fails)
+        with pytest.raises(MemoryError):
+            getattr(twprune, fn)(scores, 50, 32)
+    assert all(np.array_equal(a, b) for a, b in zip(want, getattr(twprune, fn)(scores, 50, 32)))

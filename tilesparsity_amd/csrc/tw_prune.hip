@@ -903,11 +903,20 @@ __global__ void __launch_bounds__(256)
 // consecutive columns of four consecutive rows: one 16-byte store per row where the chunk is whole and
 // aligned; a workgroup takes 1024 units of one layer, four per thread.  15 us for the 57 MB of masks of
 // twelve BERT-base feed-forward layers, of which 3 are the threshold.
+// The masks' addresses come with the launch, so that the caller can allocate them while the kernels before run (a
+// network of more layers: in the table, at the start).
 constexpr int kFillRows = 4, kFillUnits = 1024;
+constexpr int kLateMasks = 128;
+struct MaskTable {
+    uint8_t *m[kLateMasks];
+};
 __global__ void __launch_bounds__(256)
-    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const Threshold *tile_thr, Mail *mail)
+    fill_mask_kernel(const PruneLayer *layers, int n_layers, const SelectState *st, const Threshold *tile_thr, Mail *mail,
+                     const MaskTable masks)
 {
-    const PruneLayer L = layers[LayerFinder(&layers->el_begin, sizeof(PruneLayer), n_layers)(blockIdx.x)];
+    const int layer = LayerFinder(&layers->el_begin, sizeof(PruneLayer), n_layers)(blockIdx.x);
+    const PruneLayer L = layers[layer];
+    TW_GLOBAL(uint8_t) const mask = as_global(n_layers <= kLateMasks ? masks.m[layer] : L.mask);
     const Threshold thr = tile_thr ? *tile_thr : threshold_of<256>(st); // (tile_thr: one per tile)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         mail->thr_rows = thr.v64;
@@ -978,7 +987,7 @@ __global__ void __launch_bounds__(256)
         for (int r = 0; r < kFillRows; ++r) {
             if (k0 + r >= L.K)
                 break;
-            TW_GLOBAL(uint8_t) const dst = as_global(L.mask) + (int64_t)(k0 + r) * L.N + c0;
+            TW_GLOBAL(uint8_t) const dst = mask + (int64_t)(k0 + r) * L.N + c0;
             if (n == 16 && (((uintptr_t)dst) & 15) == 0) {
                 *(TW_GLOBAL(u32x4))dst = u32x4{out[r][0], out[r][1], out[r][2], out[r][3]};
             } else {
@@ -1242,7 +1251,8 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // elements.  The narrowing pass also writes the masks: what lies outside the bracket is decided
 // already, and the few per cent inside are marked one by one when the threshold is known, from the places kept
 // beside their values.
-// Over the elements of VGG16: sample, bracket, narrowing, three passes 4 + 11 + 31 + 31 us.
+// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 42 + 27 + 10 us; with those masks
+// written and read and the elements read once more at the end 13 + 4 + 11 + 31 + 31 + 32, and the host's wait between the stages.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
 template <int SRC>
@@ -1406,8 +1416,8 @@ __global__ void __launch_bounds__(256, 4)
         }
     };
     // The candidates of an item, one of every lane that has one left at a time: a lane has half of one among its
-    // sixteen elements, so that three or four rounds do for what were sixteen (46 us so, 72 with the test behind each
-    // element).
+    // sixteen elements, so that three or four rounds do for sixteen tests and as many stores (42 us for the 31.5 M elements
+    // of VGG16 with masks out of norms, 46 with a test behind each element).
     auto item_done = [&](int64_t item) {
         for (;;) {
             const bool some = inside != 0;
@@ -1781,18 +1791,37 @@ int queue_select(const float *d_v, int64_t n, SelectState *st, int n_segments, h
     return TW_OK;
 }
 
+// The caller's masks: there from the start, or (`ready`) once that has been called, when the first kernels are queued.
+struct Masks {
+    uint8_t *const *m;
+    tw_masks_ready ready = nullptr;
+    void *user = nullptr;
+
+    // asks for them and checks them
+    int get(int n_layers)
+    {
+        if (ready && ready(user))
+            return fail(TW_ERR_ALLOC, "the caller has no masks");
+        ready = nullptr;
+        for (int l = 0; l < n_layers; ++l)
+            if (!m[l])
+                return fail(TW_ERR_NULL, "layer %d: scores or mask pointer is NULL", l);
+        return TW_OK;
+    }
+};
+
 int check_layers(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
-                 uint8_t *const *masks, int granularity)
+                 const Masks &masks, int granularity)
 {
     if (n_layers <= 0 || granularity <= 0)
         return fail(TW_ERR_SHAPE, "n_layers=%d granularity=%d must be positive", n_layers,
                     granularity);
-    if (!K || !N || !scores || !masks)
+    if (!K || !N || !scores || !masks.m)
         return fail(TW_ERR_NULL, "K, N, scores or masks is NULL");
     for (int l = 0; l < n_layers; ++l) {
         if (K[l] <= 0 || N[l] <= 0)
             return fail(TW_ERR_SHAPE, "layer %d: K=%d N=%d must be positive", l, K[l], N[l]);
-        if (!scores[l] || !masks[l])
+        if (!scores[l] || (!masks.ready && !masks.m[l]))
             return fail(TW_ERR_NULL, "layer %d: scores or mask pointer is NULL", l);
     }
     return TW_OK;
@@ -1804,8 +1833,7 @@ struct CallTable {
     std::vector<PruneLayer> layers;
     int64_t n_norms = 0, n_items = 0, n_fill = 0, n_tcol = 0, n_cols = 0; // sums over the layers (upper bounds)
 };
-CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
-                     uint8_t *const *masks, int granularity, int flags)
+CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, int granularity, int flags)
 {
     CallTable c;
     c.layers.resize(n_layers);
@@ -1813,7 +1841,6 @@ CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const flo
         PruneLayer &e = c.layers[l];
         std::memset(&e, 0, sizeof(e));
         e.score = scores[l];
-        e.mask = masks[l];
         e.K = K[l];
         e.N = N[l];
         e.granularity = granularity;
@@ -1831,6 +1858,33 @@ CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const flo
     return c;
 }
 
+// masks of more layers than a launch takes addresses: into the table, before it goes to the device
+int early_masks(CallTable &c, Masks &masks)
+{
+    const int n_layers = (int)c.layers.size();
+    if (n_layers <= kLateMasks)
+        return TW_OK;
+    const int st = masks.get(n_layers);
+    for (int l = 0; !st && l < n_layers; ++l)
+        c.layers[l].mask = masks.m[l];
+    return st;
+}
+int queue_fill(const CallTable &c, Masks &masks, const PruneLayer *d_table, const SelectState *d_st, const Threshold *d_tile_thr, Mail *mail,
+               hipStream_t s)
+{
+    const int n_layers = (int)c.layers.size();
+    const int st = masks.get(n_layers);
+    if (st)
+        return st;
+    MaskTable m;
+    std::memset(&m, 0, sizeof(m));
+    for (int l = 0; l < std::min(n_layers, kLateMasks); ++l)
+        m.m[l] = masks.m[l];
+    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_tile_thr, mail, m);
+    TW_HIP(hipGetLastError());
+    return TW_OK;
+}
+
 int too_large(int64_t workgroups)
 {
     return workgroups > 0x7fffffff ? fail(TW_ERR_SHAPE, "%lld workgroups: a launch takes at most 2^31 - 1", (long long)workgroups)
@@ -1840,15 +1894,17 @@ int too_large(int64_t workgroups)
 // tiles of `granularity` columns: norms of all layers into one pooled vector, one threshold (or, with
 // kPerTileThreshold, one per tile of the only layer), masks.  *threshold receives it.
 int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double q, int q_is_f64,
-                 int granularity, uint8_t *const *masks, double *threshold, hipStream_t s, int flags)
+                 int granularity, Masks masks, double *threshold, hipStream_t s, int flags)
 {
-    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, flags);
+    CallTable c = make_table(n_layers, K, N, scores, granularity, flags);
     const bool per_tile = (flags & kPerTileThreshold) != 0;
     const int n_seg = per_tile ? c.layers[0].n_tiles : 1;
     const bool in_blocks = per_tile && K[0] <= kTileSelect; // a workgroup a tile, no counters in memory
     int st = check_percentile(c.n_norms / n_seg, q);
     if (!st)
         st = too_large(std::max(c.n_items, c.n_fill));
+    if (!st)
+        st = early_masks(c, masks);
     if (st)
         return st;
     Arena ar(s);
@@ -1881,9 +1937,9 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
         if (per_tile)
             hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st, d_tile_thr, mail);
     }
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st, d_tile_thr,
-                       mail);
-    TW_HIP(hipGetLastError());
+    st = queue_fill(c, masks, d_table, d_st, d_tile_thr, mail, s);
+    if (st)
+        return st;
     st = ar.wait();
     if (!st && threshold)
         *threshold = mail->thr_rows;
@@ -1895,7 +1951,7 @@ class MixCall {
 public:
     // `masks0` or, where that is nullptr, `rows`: the table of a first stage whose masks nobody has written (norms and tiles)
     int plan(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, const uint8_t *const *masks0,
-             const CallTable *rows, uint8_t *const *masks, double q, int q_type)
+             const CallTable *rows, double q, int q_type)
     {
         layers_.resize(n_layers);
         for (int l = 0; l < n_layers; ++l) {
@@ -1903,7 +1959,6 @@ public:
             std::memset(&e, 0, sizeof(e));
             e.score = scores[l];
             e.mask0 = masks0 ? masks0[l] : nullptr;
-            e.out = masks[l];
             e.n = (int64_t)K[l] * N[l];
             e.begin = total_;
             e.item_begin = n_items_;
@@ -1915,15 +1970,22 @@ public:
             e.per_g = 1.0f / (float)e.G;
             e.rows_on = kMixItem / 4 / N[l];
             e.cols_on = kMixItem / 4 % N[l];
-            const bool wide = masks0 || (e.G >= 3 && N[l] >= 3 && (N[l] % e.G == 0 || N[l] % e.G >= 3));
-            if (((uintptr_t)e.score & 15) == 0 && (((uintptr_t)e.mask0 | (uintptr_t)e.out) & 3) == 0 && wide)
-                e.in_fours = N[l] % 4 == 0 && e.G % 4 == 0 ? 2 : 1;
             total_ += e.n;
             n_items_ += (e.n + kMixItem - 1) / kMixItem;
         }
         q_ = q;
         q_type_ = q_type;
         return check_percentile(total_, q);
+    }
+    void write_to(uint8_t *const *masks)
+    {
+        for (size_t l = 0; l < layers_.size(); ++l) {
+            MixLayer &e = layers_[l];
+            e.out = masks[l];
+            const bool wide = e.mask0 || (e.G >= 3 && e.N >= 3 && (e.N % e.G == 0 || e.N % e.G >= 3));
+            if (((uintptr_t)e.score & 15) == 0 && (((uintptr_t)e.mask0 | (uintptr_t)e.out) & 3) == 0 && wide)
+                e.in_fours = e.N % 4 == 0 && e.G % 4 == 0 ? 2 : 1;
+        }
     }
     int alloc(Arena &ar)
     {
@@ -2137,32 +2199,41 @@ try {
 }
 TW_CATCH_TO_STATUS
 
-int tw_prune_tiled_wise_1d(int n_layers, const int32_t *K, const int32_t *N,
-                           const float *const *scores, double sparsity, int q_type,
-                           int granularity, uint8_t *const *masks, double *threshold, void *stream)
+int tw_prune_tiled_wise_1d_late(int n_layers, const int32_t *K, const int32_t *N,
+                                const float *const *scores, double sparsity, int q_type,
+                                int granularity, uint8_t *const *masks, tw_masks_ready ready, void *user, double *threshold, void *stream)
 try {
-    int st = check_layers(n_layers, K, N, scores, masks, granularity);
+    const Masks m{masks, ready, user};
+    int st = check_layers(n_layers, K, N, scores, m, granularity);
     if (st)
         return st;
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
-    return uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, masks, threshold, (hipStream_t)stream, 0);
+    return uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, m, threshold, (hipStream_t)stream, 0);
 }
 TW_CATCH_TO_STATUS
+
+int tw_prune_tiled_wise_1d(int n_layers, const int32_t *K, const int32_t *N,
+                           const float *const *scores, double sparsity, int q_type,
+                           int granularity, uint8_t *const *masks, double *threshold, void *stream)
+{
+    return tw_prune_tiled_wise_1d_late(n_layers, K, N, scores, sparsity, q_type, granularity, masks, nullptr, nullptr, threshold, stream);
+}
 
 int tw_prune_granularity(int K, int N, const float *scores, double sparsity, int q_type,
                          int granularity, uint8_t *mask, void *stream)
 try {
     const float *const sc[1] = {scores};
     uint8_t *const mk[1] = {mask};
-    int st = check_layers(1, &K, &N, sc, mk, granularity);
+    const Masks m{mk};
+    int st = check_layers(1, &K, &N, sc, m, granularity);
     if (st)
         return st;
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
         return fail(TW_ERR_LAYOUT, "q_type=%d: unknown", q_type);
     if (N % granularity != 0)
         return fail(TW_ERR_SHAPE, "N=%d is not a multiple of the granularity %d", N, granularity);
-    return uniform_rows(1, &K, &N, sc, sparsity, q_type, granularity, mk, nullptr, (hipStream_t)stream,
+    return uniform_rows(1, &K, &N, sc, sparsity, q_type, granularity, m, nullptr, (hipStream_t)stream,
                         kNormNotDivided | kPerTileThreshold);
 }
 TW_CATCH_TO_STATUS
@@ -2171,8 +2242,18 @@ int tw_prune_tiled_wise_2d(int n_layers, const int32_t *K, const int32_t *N,
                            const float *const *scores, double sparsity, int q_type, int transform,
                            int granularity, uint8_t *const *masks, uint8_t *const *col_masks,
                            double *thresholds, void *stream)
+{
+    return tw_prune_tiled_wise_2d_late(n_layers, K, N, scores, sparsity, q_type, transform, granularity, masks, nullptr, nullptr, col_masks,
+                                       thresholds, stream);
+}
+
+int tw_prune_tiled_wise_2d_late(int n_layers, const int32_t *K, const int32_t *N,
+                                const float *const *scores, double sparsity, int q_type, int transform,
+                                int granularity, uint8_t *const *masks, tw_masks_ready ready, void *user, uint8_t *const *col_masks,
+                                double *thresholds, void *stream)
 try {
-    int st = check_layers(n_layers, K, N, scores, masks, granularity);
+    Masks m{masks, ready, user};
+    int st = check_layers(n_layers, K, N, scores, m, granularity);
     if (st)
         return st;
     if (q_type != TW_Q_F32 && q_type != TW_Q_F64)
@@ -2188,10 +2269,12 @@ try {
     }
     // columns: one pooled vector of column norms, one threshold; then, without a trip to the host,
     // the tiles and the rows
-    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, 0);
+    CallTable c = make_table(n_layers, K, N, scores, granularity, 0);
     st = check_percentile(c.n_cols, q);
     if (!st)
         st = too_large(std::max({c.n_items, c.n_fill, c.n_cols}));
+    if (!st)
+        st = early_masks(c, m);
     if (st)
         return st;
     Arena ar(s);
@@ -2232,9 +2315,9 @@ try {
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(fill_mask_kernel, dim3((unsigned)c.n_fill), dim3(256), 0, s, d_table, n_layers, d_st,
-                       (const Threshold *)nullptr, mail);
-    TW_HIP(hipGetLastError());
+    st = queue_fill(c, m, d_table, d_st, nullptr, mail, s);
+    if (st)
+        return st;
     st = ar.wait();
     if (!st && thresholds) {
         thresholds[0] = mail->thr_cols;
@@ -2248,7 +2331,7 @@ int tw_prune_mix(int n_layers, const int32_t *K, const int32_t *N, const float *
                  const uint8_t *const *layer_masks, double g1percent, int q_type,
                  uint8_t *const *masks, double *threshold, void *stream)
 try {
-    int st = check_layers(n_layers, K, N, scores, masks, 1);
+    int st = check_layers(n_layers, K, N, scores, Masks{masks}, 1);
     if (st)
         return st;
     if (!layer_masks)
@@ -2260,9 +2343,10 @@ try {
             return fail(TW_ERR_NULL, "layer %d: layer mask pointer is NULL", l);
     hipStream_t s = (hipStream_t)stream;
     MixCall mix;
-    st = mix.plan(n_layers, K, N, scores, layer_masks, nullptr, masks, 100.0 - g1percent, q_type);
+    st = mix.plan(n_layers, K, N, scores, layer_masks, nullptr, 100.0 - g1percent, q_type);
     if (st)
         return st;
+    mix.write_to(masks);
     Arena ar(s);
     st = mix.alloc(ar);
     MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
@@ -2282,57 +2366,61 @@ try {
 }
 TW_CATCH_TO_STATUS
 
-int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double sparsity,
-                               int q_type, int granularity, double g1percent, int g1_q_type, uint8_t *const *masks,
-                               double *threshold, void *stream)
+int tw_prune_tiled_wise_1d_mix_late(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double sparsity,
+                                    int q_type, int granularity, double g1percent, int g1_q_type, uint8_t *const *masks,
+                                    tw_masks_ready ready, void *user, double *threshold, void *stream)
 try {
-    int st = check_layers(n_layers, K, N, scores, masks, granularity);
+    Masks m{masks, ready, user};
+    int st = check_layers(n_layers, K, N, scores, m, granularity);
     if (st)
         return st;
     if ((q_type != TW_Q_F32 && q_type != TW_Q_F64) || (g1_q_type != TW_Q_F32 && g1_q_type != TW_Q_F64))
         return fail(TW_ERR_LAYOUT, "q_type=%d, %d: unknown", q_type, g1_q_type);
     for (int l = 0; l < n_layers; ++l)
         if (N[l] > kMixMaxN || K[l] > kMixMaxK || (N[l] + (int64_t)granularity - 1) / granularity * K[l] > kMixMaxNorms) { // one stage after the other
-            st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, masks, nullptr, (hipStream_t)stream, 0);
+            st = m.get(n_layers);
+            if (!st)
+                st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, m, nullptr, (hipStream_t)stream, 0);
             return st ? st : tw_prune_mix(n_layers, K, N, scores, masks, g1percent, g1_q_type, masks, threshold, stream);
         }
     hipStream_t s = (hipStream_t)stream;
-    CallTable c = make_table(n_layers, K, N, scores, masks, granularity, 0);
+    CallTable c = make_table(n_layers, K, N, scores, granularity, 0);
     MixCall mix;
     st = check_percentile(c.n_norms, sparsity);
     if (!st)
         st = too_large(c.n_items);
     if (!st)
-        st = mix.plan(n_layers, K, N, scores, nullptr, &c, masks, 100.0 - g1percent, g1_q_type);
+        st = mix.plan(n_layers, K, N, scores, nullptr, &c, 100.0 - g1percent, g1_q_type);
     if (st)
         return st;
     Arena ar(s);
     float *d_norms = ar.alloc_n<float>(c.n_norms);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
-    const size_t table_bytes = sizeof(PruneLayer) * n_layers;
-    char *d_tables = static_cast<char *>(ar.alloc(table_bytes + mix.table_bytes()));
+    PruneLayer *d_table = ar.alloc_n<PruneLayer>(n_layers);
+    MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
     Mail *mail = ar.mail();
-    if (!d_norms || !d_st || !d_tables || !mail)
+    if (!d_norms || !d_st || !d_table || !d_layers || !mail)
         return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
     st = mix.alloc(ar);
     if (st)
         return st;
-    const PruneLayer *d_table = reinterpret_cast<const PruneLayer *>(d_tables);
-    const MixLayer *d_layers = reinterpret_cast<const MixLayer *>(d_tables + table_bytes);
     int64_t off = 0;
     for (int l = 0; l < n_layers; ++l) {
         c.layers[l].norms = d_norms + off;
         mix.table()[l].norms = d_norms + off;
         off += (int64_t)K[l] * c.layers[l].n_tiles;
     }
-    std::vector<char> both(table_bytes + mix.table_bytes());
-    std::memcpy(both.data(), c.layers.data(), table_bytes);
-    std::memcpy(both.data() + table_bytes, mix.table().data(), mix.table_bytes());
-    st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
+    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
     if (st)
         return st;
     hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, (const int64_t *)nullptr);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
+    if (!st)
+        st = m.get(n_layers);
+    if (st)
+        return st;
+    mix.write_to(masks);
+    st = put_table(mix.table().data(), mix.table_bytes(), d_layers, SetupSelect{}, SetupSelect{}, s);
     if (!st)
         st = mix.queue<MIX_NORMS>(d_layers, d_st, mail, s);
     if (st)
@@ -2343,5 +2431,13 @@ try {
     return st;
 }
 TW_CATCH_TO_STATUS
+
+int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double sparsity,
+                               int q_type, int granularity, double g1percent, int g1_q_type, uint8_t *const *masks,
+                               double *threshold, void *stream)
+{
+    return tw_prune_tiled_wise_1d_mix_late(n_layers, K, N, scores, sparsity, q_type, granularity, g1percent, g1_q_type, masks, nullptr,
+                                           nullptr, threshold, stream);
+}
 
 } // extern "C"

@@ -54,7 +54,8 @@ EXPORTED_SYMBOLS = (
     "tw_tiles_every_g_columns", "tw_tiles_every_g_kept_columns",
     "tw_prune_tile_row_norms", "tw_prune_col_norms", "tw_percentile_linear", "tw_gemm_ex",
     "tw_prune_granularity", "tw_plan_from_export", "tw_plan_from_mask_cover", "tw_tiles_from_mask",
-    "tw_prune_mix", "tw_prune_tiled_wise_1d_mix", "tw_lstm_gates", "tw_plan_from_device_mask", "tw_set_option", "tw_gemm_static",
+    "tw_prune_mix", "tw_prune_tiled_wise_1d_mix", "tw_prune_tiled_wise_1d_late", "tw_prune_tiled_wise_2d_late",
+    "tw_prune_tiled_wise_1d_mix_late", "tw_lstm_gates", "tw_plan_from_device_mask", "tw_set_option", "tw_gemm_static",
     "tw_gemm_staged", "tw_gemm_staged_workspace",
     "tw_side_create", "tw_side_destroy", "tw_side_nnz", "tw_side_gemm", "tw_plan_reset", "tw_lstm_step",
     "tw_lstm_steps", "tw_lstm_steps_status", "tw_gemm_choice", "tw_gemm_kernel_name",
@@ -69,6 +70,9 @@ class TwError(RuntimeError):
         self.status = status
         self.message = message
 
+
+# tw_masks_ready: the caller's object comes back to it
+MASKS_READY = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.py_object)
 
 _lib = None
 
@@ -153,6 +157,12 @@ def lib():
         "tw_percentile_linear": (c_int, [vp, c_i64, ctypes.c_double, c_int,
                                          ctypes.POINTER(ctypes.c_double), vp]),
         "tw_tiles_every_g_kept_columns": (c_int, [c_int, c_int, vp, vp, vp, ctypes.POINTER(c_int)]),
+        "tw_prune_tiled_wise_1d_late": (c_int, [c_int, i32p, i32p, pp, ctypes.c_double, c_int, c_int, pp, MASKS_READY, ctypes.py_object,
+                                                ctypes.POINTER(ctypes.c_double), vp]),
+        "tw_prune_tiled_wise_2d_late": (c_int, [c_int, i32p, i32p, pp, ctypes.c_double, c_int, c_int, c_int, pp, MASKS_READY,
+                                                ctypes.py_object, pp, ctypes.POINTER(ctypes.c_double), vp]),
+        "tw_prune_tiled_wise_1d_mix_late": (c_int, [c_int, i32p, i32p, pp, ctypes.c_double, c_int, c_int, ctypes.c_double, c_int,
+                                                    pp, MASKS_READY, ctypes.py_object, ctypes.POINTER(ctypes.c_double), vp]),
         "tw_prune_tiled_wise_1d_mix": (c_int, [c_int, i32p, i32p, pp, ctypes.c_double, c_int, c_int, ctypes.c_double, c_int,
                                                pp, ctypes.POINTER(ctypes.c_double), vp]),
         "tw_prune_mix": (c_int, [c_int, i32p, i32p, pp, pp, ctypes.c_double, c_int, pp,

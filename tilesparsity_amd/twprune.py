@@ -36,7 +36,9 @@ def img2col_forward(accumulated_scores):
 class _DeviceLayers:
     """Scores on the GPU (uploaded where they are not there yet) and mask buffers, as pointer tables
     for the C ABI.  Every mask is a tensor with storage of its own, so that a caller who keeps one keeps
-    no other layer's memory; the column masks are made when they are first asked for."""
+    no other layer's memory.  The masks are made when the library asks for them, its first kernels
+    running by then (twelve BERT-base layers' 24 masks are 33 us of the host's time), the column masks when
+    they are first asked for."""
 
     def __init__(self, scores):
         import torch
@@ -58,19 +60,26 @@ class _DeviceLayers:
                 raise tw.TwError(tw.ERR_SHAPE, "a score tensor must be 2-D or 4-D")
             d_scores.append(t if t.is_contiguous() else t.contiguous())
         n = len(d_scores)
-        self.shapes = [tuple(t.shape) for t in d_scores]
-        self.K = np.array([k for k, _ in self.shapes], np.int32)
-        self.N = np.array([w for _, w in self.shapes], np.int32)
+        self.shapes = [t.shape for t in d_scores]
+        self.K = np.array([s[0] for s in self.shapes], np.int32)
+        self.N = np.array([s[1] for s in self.shapes], np.int32)
         self.p_scores = (ctypes.c_void_p * n)(*[t.data_ptr() for t in d_scores])
-        self.d_masks, self.p_masks = self._buffers(self.shapes)
+        self.d_masks, self.p_masks = None, (ctypes.c_void_p * n)()
+        self.error = None
         self._cols = None
         self.stream = torch.cuda.current_stream().cuda_stream
 
-    def _buffers(self, shapes):
+    def make_masks(self):
         # (empty_strided with a device object: 1.3 us a tensor, empty with its name 1.8)
         empty, u8, device = self.torch.empty_strided, self.torch.uint8, self.device
-        bufs = [empty(s, (s[1], 1), dtype=u8, device=device) for s in shapes]
-        return bufs, (ctypes.c_void_p * len(bufs))(*[b.data_ptr() for b in bufs])
+        self.d_masks = [empty(s, (s[1], 1), dtype=u8, device=device) for s in self.shapes]
+        self.p_masks[:] = [m.data_ptr() for m in self.d_masks]
+        return self
+
+    def check(self, status):
+        if self.error is not None:
+            raise self.error
+        tw._check(status)
 
     def _make_cols(self):
         # (one buffer: the column masks stay in here, and come to the host in one copy)
@@ -103,16 +112,28 @@ class _DeviceLayers:
         return out
 
 
+def _masks_ready(d):
+    try:
+        d.make_masks()
+    except BaseException as e:  # (raised again behind the call, whose frames it cannot cross)
+        d.error = e
+        return 1
+    return 0
+
+
+_READY = tw.MASKS_READY(_masks_ready)
+
+
 def tiled_wise_1d(accumulated_scores, sparsity, granularity=128, return_device=False):
     """prune_algo.py:114-148.  Returns the list of masks (bool arrays; uint8 CUDA tensors with
     return_device=True)."""
     L = tw.lib()
     d = _DeviceLayers(accumulated_scores)
     thr = ctypes.c_double()
-    tw._check(L.tw_prune_tiled_wise_1d(
+    d.check(L.tw_prune_tiled_wise_1d_late(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
         ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(sparsity), _q_type(sparsity),
-        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)),
+        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), _READY, d,
         ctypes.byref(thr), d.stream))
     tiled_wise_1d.last_threshold = thr.value
     return d.d_masks if return_device else d.masks()
@@ -125,11 +146,11 @@ def tiled_wise_2d(accumulated_scores, sparsity, granularity=128, transform=True,
     L = tw.lib()
     d = _DeviceLayers(accumulated_scores)
     thr = (ctypes.c_double * 2)()
-    tw._check(L.tw_prune_tiled_wise_2d(
+    d.check(L.tw_prune_tiled_wise_2d_late(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
         ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(sparsity), _q_type(sparsity),
         1 if transform else 0, int(granularity),
-        ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)),
+        ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), _READY, d,
         ctypes.cast(d.p_cols, ctypes.POINTER(ctypes.c_void_p)), thr, d.stream))
     tiled_wise_2d.last_thresholds = (thr[0], thr[1])
     masks = d.d_masks if return_device else d.masks()
@@ -153,7 +174,7 @@ def _mix(d, g1percent, return_device):
 def tw_mix_fn(accumulated_scores, g1percent, layer_mask, return_device=False):
     """prune_algo.py:151-179: the elements whose |score| (minus 1 where ``layer_mask`` keeps
     them) lies above the (100 - g1percent)-th percentile of the whole network join the masks."""
-    d = _DeviceLayers(accumulated_scores)
+    d = _DeviceLayers(accumulated_scores).make_masks()
     for dst, m in zip(d.d_masks, layer_mask):
         if isinstance(m, d.torch.Tensor):
             dst.copy_(m.reshape(dst.shape).to(device="cuda", dtype=d.torch.uint8))
@@ -167,10 +188,10 @@ def tiled_wise_1d_mix(accumulated_scores, sparsity, granularity=128, g1percent=5
     """prune_algo.py:182-186: tiled_wise_1d at sparsity + g1percent, then tw_mix_fn."""
     d = _DeviceLayers(accumulated_scores)
     q, thr = sparsity + g1percent, ctypes.c_double()
-    tw._check(tw.lib().tw_prune_tiled_wise_1d_mix(
+    d.check(tw.lib().tw_prune_tiled_wise_1d_mix_late(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
         ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(q), _q_type(q), int(granularity),
-        float(g1percent), _q_type(100 - g1percent), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)),
+        float(g1percent), _q_type(100 - g1percent), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), _READY, d,
         ctypes.byref(thr), d.stream))
     tw_mix_fn.last_threshold = thr.value
     return d.d_masks if return_device else d.masks()
@@ -180,10 +201,10 @@ def tiled_wise_2d_mix(accumulated_scores, sparsity, granularity=128, g1percent=1
     """prune_algo.py:189-193: tiled_wise_2d at sparsity + g1percent, then tw_mix_fn."""
     d = _DeviceLayers(accumulated_scores)
     q = sparsity + g1percent
-    tw._check(tw.lib().tw_prune_tiled_wise_2d(
+    d.check(tw.lib().tw_prune_tiled_wise_2d_late(
         len(d.shapes), tw._ptr(d.K, ctypes.c_int32), tw._ptr(d.N, ctypes.c_int32),
         ctypes.cast(d.p_scores, ctypes.POINTER(ctypes.c_void_p)), float(q), _q_type(q), 1,
-        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), None, None, d.stream))
+        int(granularity), ctypes.cast(d.p_masks, ctypes.POINTER(ctypes.c_void_p)), _READY, d, None, None, d.stream))
     return _mix(d, g1percent, return_device)
 
 
