@@ -272,3 +272,18 @@ def test_masks_that_cannot_be_made_end_the_call(tw, twprune, monkeypatch, fn):
         with pytest.raises(MemoryError):
             getattr(twprune, fn)(scores, 50, 32)
     assert all(np.array_equal(a, b) for a, b in zip(want, getattr(twprune, fn)(scores, 50, 32)))
+
+
+@pytest.mark.parametrize("shapes", [[(8448, 4096)], [(4224, 8192), (33, 4)], [(8448, 4099)]])
+def test_scores_beyond_the_caches(twprune, shapes):
+    """More than 128 MB of scores are read past the caches, by either kernel of the row norms: the same masks
+    as from the norms and the percentile one at a time."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    scores = [torch.randn(s, generator=gen, device="cuda").abs_() for s in shapes]
+    got = twprune.tiled_wise_1d(scores, 75, 128, return_device=True)
+    norms = [twprune.tile_row_norms(s.cpu().numpy(), twprune.tiles_every_g_columns(s.shape[1], 128)) for s in scores]
+    thr = twprune.percentile(np.concatenate([n.ravel() for n in norms]), 75)
+    for s, n, m in zip(scores, norms, got):
+        keep = torch.from_numpy(n > thr).cuda().t().repeat_interleave(128, 1)[:, :s.shape[1]]
+        assert torch.equal(m.bool(), keep)

@@ -31,6 +31,15 @@ namespace tw {
 // through it is a flat one, which waits for LDS as well.
 template <class T> __device__ __forceinline__ TW_GLOBAL(T) as_global(T *p) { return (TW_GLOBAL(T))p; }
 
+// A load of data that nothing reads again soon (ONCE): it does not push other lines out of the caches.
+template <bool ONCE, class T> __device__ __forceinline__ T load_global(TW_GLOBAL(const T) p)
+{
+    if constexpr (ONCE)
+        return __builtin_nontemporal_load(p);
+    else
+        return *p;
+}
+
 // NumPy's pairwise sum of the squares of n <= 128 terms, by a group of 8 adjacent lanes: lane j keeps
 // NumPy's running sum r[j] (terms j, j+8, j+16, ...), the three shuffle steps are NumPy's
 // ((r0+r1)+(r2+r3)) + ((r4+r5)+(r6+r7)), lane 0 then adds the n % 8 trailing terms.  The result
@@ -170,6 +179,7 @@ private:
 // that only reads them 35); 92 us when every lane loaded what it added.
 constexpr int kNormRows = 32;     // rows of an item: eight lanes each
 constexpr int kNormPitch = 136;   // floats; a block of 128 columns with up to 3 before it
+template <bool ONCE>
 __global__ void __launch_bounds__(256, 6)
     tile_row_norms_kernel(const PruneLayer *layers, int n_layers, const int64_t *n_items)
 {
@@ -202,7 +212,7 @@ __global__ void __launch_bounds__(256, 6)
                 float4 v[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    v[i] = __builtin_bit_cast(float4, *(TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, nr - 1) * L.N + cq));
+                    v[i] = __builtin_bit_cast(float4, load_global<ONCE>((TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, nr - 1) * L.N + cq)));
                 bool kp[4] = {true, true, true, true};
                 if (keep) {
 #pragma unroll
@@ -221,7 +231,7 @@ __global__ void __launch_bounds__(256, 6)
                 float v[kNormRows / 4];
 #pragma unroll
                 for (int i = 0; i < kNormRows / 4; ++i)
-                    v[i] = src[(int64_t)min(r0 + i * 4, nr - 1) * L.N + c + q];
+                    v[i] = load_global<ONCE>(src + (int64_t)min(r0 + i * 4, nr - 1) * L.N + c + q);
 #pragma unroll
                 for (int i = 0; i < kNormRows / 4; ++i)
                     stage[(r0 + i * 4) * kNormPitch + q] = kp ? v[i] : 0.0f;
@@ -236,6 +246,56 @@ __global__ void __launch_bounds__(256, 6)
         }
         __syncthreads(); // the stage is written again
     }
+}
+
+// The same where every tile of every layer is one block of the sum whose rows are made of whole pieces of 16 bytes
+// (queue_norms): the second item's rows are on their way while the first is added up (226 MB of BERT-base, read past the
+// caches: 37 us, 6.1 TB/s; four items 38, the kernel above 40; through the caches 43, 45 and 46).
+constexpr int kNormItems = 2; // of a workgroup, in a row
+template <bool ONCE>
+__global__ void __launch_bounds__(256, 5)
+    block_row_norms_kernel(const PruneLayer *layers, int n_layers, int64_t n_items)
+{
+    __shared__ __align__(16) float stage[kNormRows * kNormPitch];
+    const LayerFinder find(&layers->rt_begin, sizeof(PruneLayer), n_layers);
+    const int tid = (int)threadIdx.x, l8 = tid & 7, grp = tid >> 3, r0 = tid >> 5, q = tid & 31;
+    struct Item {
+        u32x4 v[4]; // the thread's pieces of rows r0 + 8 i
+        TW_GLOBAL(float) out;
+        int nr, w, divide;
+    };
+    auto fetch = [&](int64_t item, Item &d) {
+        const PruneLayer &L = layers[find(item)];
+        const int K = L.K, N = L.N, G = L.granularity, n_tiles = L.n_tiles;
+        const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a launch has fewer than 2^31 items)
+        const int rblk = (int)(idx / (uint32_t)n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)n_tiles);
+        const int k0 = rblk * kNormRows, c0 = t * G;
+        d.nr = min(kNormRows, K - k0);
+        d.w = min(G, N - c0);
+        d.divide = !(L.flags & kNormNotDivided);
+        d.out = as_global(L.norms) + (int64_t)t * K + k0;
+        TW_GLOBAL(const float) const src = as_global(L.score) + (int64_t)k0 * N + c0 + min(q * 4, d.w - 4); // (pieces past the last repeat it)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) // (so do rows)
+            d.v[i] = load_global<ONCE>((TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, d.nr - 1) * N));
+    };
+    auto add = [&](const Item &d) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<u32x4 *>(stage + (r0 + i * 8) * kNormPitch + q * 4) = d.v[i];
+        TW_LDS_BARRIER();
+        const float s = pairwise_block(stage + grp * kNormPitch, d.w, l8);
+        if (l8 == 0 && grp < d.nr) // both operations correctly rounded
+            d.out[grp] = d.divide ? sqrtf(s) / (float)d.w : sqrtf(s);
+        TW_LDS_BARRIER(); // the stage is written again
+    };
+    const int64_t first = (int64_t)blockIdx.x * kNormItems, last = n_items - 1;
+    Item a, b;
+    fetch(first, a);
+    fetch(min(first + 1, last), b);
+    add(a);
+    if (first < last)
+        add(b);
 }
 
 // cnorm[pooled c] = ||score[:, c]|| / K, the rows accumulated in order.  The chain of K additions
@@ -1914,6 +1974,31 @@ CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const flo
     return c;
 }
 
+// The row norms of all layers' tiles; n_items: tiles of kept columns, *n_items items of them.  `last`: the call does not read the
+// scores again.  Scores of more than half the memory-side cache (256 MB) are then read past it: they would not stay
+// there beside what comes next (226 MB of BERT-base: 43 -> 37 us; but where the call reads them again, or the next one
+// builds plans out of the same matrices, they have to stay: narrowing VGG16's 126 MB 42.5 -> 46.7 us, fourteen plans 93 ->
+// 111).
+constexpr int64_t kStayingBytes = 128 << 20;
+void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n_items, bool last, hipStream_t s)
+{
+    bool blocks = n_items == nullptr;
+    int64_t bytes = 0;
+    for (const PruneLayer &e : c.layers)
+        bytes += (int64_t)e.K * e.N * 4;
+    const bool once = last && bytes > kStayingBytes;
+    for (const PruneLayer &e : c.layers)
+        blocks &= (e.N & 3) == 0 && (e.granularity & 3) == 0 && e.granularity <= 128 && ((uintptr_t)e.score & 15) == 0;
+    const int n_layers = (int)c.layers.size();
+    if (blocks) {
+        auto kernel = once ? block_row_norms_kernel<true> : block_row_norms_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((c.n_items + kNormItems - 1) / kNormItems)), dim3(256), 0, s, d_table, n_layers, c.n_items);
+    } else {
+        auto kernel = once ? tile_row_norms_kernel<true> : tile_row_norms_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, n_items);
+    }
+}
+
 // masks of more layers than a launch takes addresses: into the table, before it goes to the device
 int early_masks(CallTable &c, Masks &masks)
 {
@@ -1980,8 +2065,7 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
                    setup_of(d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q, q_is_f64), SetupSelect{}, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers,
-                       (const int64_t *)nullptr);
+    queue_norms(c, d_table, nullptr, true, s);
     // per-tile thresholds (one layer): every tile's K norms are one segment
     if (in_blocks) {
         auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
@@ -2199,7 +2283,7 @@ try {
         st = put_table(&e, sizeof(e), d_table, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)n_items), dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr);
+    hipLaunchKernelGGL(tile_row_norms_kernel<false>, dim3((unsigned)n_items), dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr);
     TW_HIP(hipGetLastError());
     return ar.wait();
 }
@@ -2367,7 +2451,7 @@ try {
     hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)n_blk), dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm);
     hipLaunchKernelGGL(plan_2d_kernel, dim3(1), dim3(kPlanThreads), 0, s, d_table, n_layers, d_cnorm, c.n_cols, d_norms,
                        d_st, d_items, q, q_type, mail);
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, d_items);
+    queue_norms(c, d_table, d_items, false, s);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
@@ -2469,7 +2553,7 @@ try {
     st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
     if (st)
         return st;
-    hipLaunchKernelGGL(tile_row_norms_kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, (const int64_t *)nullptr);
+    queue_norms(c, d_table, nullptr, false, s);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (!st)
         st = m.get(n_layers);
