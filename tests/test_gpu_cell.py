@@ -362,6 +362,34 @@ def test_multi_step_launch(tw, oracle, dtype, M, I, H, G, k_keep, T):
     assert np.array_equal(outs[2][0][:, :I, :], A[:, :I, :])
 
 
+@pytest.mark.parametrize("M,H", [(100, 96), (250, 96), (70, 160), (32, 224), (256, 1024)])
+def test_multi_step_launch_places(tw, oracle, M, H):
+    """Numbers of workgroups that do and do not divide by the eight dies they are dealt to (12, 24, 15, 7, 256):
+    the multi-step launch against one launch a step."""
+    import torch
+    rng = np.random.default_rng(M + H)
+    I, G, T, dtype = 48, 32, 4, "f16"
+    K, ld = I + H, (M + 7) // 8 * 8
+    W, bias, tiles, xs, h0, c0, A, c = _sequence_problem(rng, oracle, M, I, H, G, 0.3, T, dtype, ld)
+    dbias = torch.from_numpy(bias).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    with tw.Plan.create(K, 4 * H, dtype, tiles, W) as plan:
+        print("multi-step launch, places", M, H, flush=True)
+        dA, dC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        plan.lstm_steps(T, dA.data_ptr(), M, dC.data_ptr(), lda=ld, a_step=K * ld, ldc=ld,
+                        bias_ptr=dbias.data_ptr(), stream=s)
+        plan.lstm_steps_status(s)
+        oA, oC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        for t in range(T):
+            plan.lstm_step(oA[t].data_ptr(), M, oC.data_ptr(), oC.data_ptr(), oA[t + 1, I].data_ptr(), lda=ld,
+                           ldc_prev=ld, ldc_new=ld, ldh=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        torch.cuda.synchronize()
+        got = oracle.bits_to_f32(dA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+        want = oracle.bits_to_f32(oA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+    assert oracle.rel_error(got, want) <= 2 * TOL[dtype]
+    assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
+
+
 def test_multi_step_launch_in_a_graph(tw, oracle):
     """tw_lstm_steps records into a HIP graph (its fill of the rows of h is a kernel, not a memset):
     the graph is replayed four times on inputs restored in between, with eager launches of the same
