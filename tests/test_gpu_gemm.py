@@ -1066,6 +1066,46 @@ def test_skinny_row_major_gives_the_k_major_bits(tw, oracle, M, K, n_units, widt
         tw.set_option(tw.OPT_SHAPE, -1)
 
 
+@pytest.mark.parametrize("row_major", [False, True])
+@pytest.mark.parametrize("n_units, width, k_max, rows, dtype", [
+    (11, 128, 700, 33, "f16"), (8, 128, 250, 32, "bf16"), (3, 96, 1000, 50, "f16"), (16, 64, 130, 64, "bf16"), (5, 40, 600, 7, "f16")])
+def test_skinny_pieces_give_the_same_bits(tw, oracle, n_units, width, k_max, rows, dtype, row_major):
+    """Few rows run in pieces of 32 columns, many in pieces of 64: the first rows of a launch with enough of them to
+    fill the chip more than twice are bit for bit those of a launch with these rows alone."""
+    import torch
+    rng = np.random.default_rng([n_units, width, k_max])
+    K, N = 1040, n_units * width
+    M = 32 * (2 * 256 * 2 // (n_units * 2) + 1)
+    B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    tiles = [dict(col0=t * width, width=width,
+                  kept_k=np.sort(rng.choice(K, size=k_max if t == 0 else int(rng.integers(0, k_max)),
+                                            replace=False)).astype(np.int32),
+                  kept_n=np.sort(rng.choice(width, size=int(rng.integers(1, width + 1)),
+                                            replace=False)).astype(np.int32)) for t in range(n_units)]
+    layout = tw.ROWMAJOR if row_major else tw.KMAJOR
+    Ab = oracle.cast_bits(rng.standard_normal((M, K)).astype(np.float32), dtype).reshape(M, K)
+    bias = torch.randn(N, device="cuda")
+    outs = []
+    try:
+        tw.set_option(tw.OPT_SHAPE, tw.SHAPE_SKINNY)
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            for m in (rows, M):
+                ld = round_up(m, 8)
+                host = Ab[:m] if row_major else np.zeros((K, ld), np.uint16)
+                if not row_major:
+                    host[:, :m] = Ab[:m].T
+                dA = to_device_bits(host, host.shape)
+                dC = torch.zeros((m, N) if row_major else (N, ld), dtype=torch.int16, device="cuda")
+                print("skinny pieces", n_units, width, k_max, m, dtype, row_major, flush=True)
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), m, lda=host.shape[1], ldc=dC.shape[1], a_layout=layout, c_layout=layout,
+                          pruned_cols=tw.PRUNED_ZERO, bias_ptr=bias.data_ptr(), activation=tw.ACT_RELU)
+                torch.cuda.synchronize()
+                outs.append(from_device_bits(dC)[:rows] if row_major else from_device_bits(dC)[:, :rows])
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+    assert np.array_equal(outs[0], outs[1])
+
+
 @pytest.mark.parametrize("n_units", [1, 2, 3, 4, 5, 7, 8, 11])
 @pytest.mark.parametrize("M", [1, 33, 500])
 @pytest.mark.parametrize("k_max, width", [(256, 128), (700, 128), (256, 64)])

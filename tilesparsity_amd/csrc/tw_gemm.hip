@@ -1911,24 +1911,24 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 // Skinny kernel for few rows of A (one time step of a recurrent cell: M = 128; a small batch): the
 // launch is then a chain of dependent trips to memory on an almost empty chip, and the streaming
 // kernels walk a tile's kept rows 64 at a time, one trip per step.  Here a workgroup takes 32 rows m
-// of one half of a unit (up to 64 compact columns) and its NW waves split the kept rows between them:
+// of one piece of a unit (64 compact columns, or 32: NB blocks) and its NW waves split the kept rows between them:
 // wave w takes the steps w, w + NW, ... of 64 kept rows: it fetches their row numbers, then their 4 KB
-// of A and 8 KB of weight fragments in one go, turns A through its own piece of LDS (no barrier:
+// of A and 8 (4) KB of weight fragments in one go, turns A through its own piece of LDS (no barrier:
 // nobody else reads it) and multiplies, each fragment's registers taking the next step's as soon as it
 // is used.  The NW partial products meet in LDS once, are added in wave order (so the result does not
 // depend on timing) and leave through one rounding.  With eight waves a tile of 512 kept rows is one
 // trip to memory for the numbers and one for the operands, and at 128 registers a wave two workgroups
 // share a compute unit.
 //   work:  workgroup b runs on die b % 8.  Units in whole groups of eight have a die each, where their
-//          halves and row blocks share their rows of A and their weight in the L2.  The units left
+//          pieces and row blocks share their rows of A and their weight in the L2.  The units left
 //          over (all of them, in a plan of fewer than eight) get as many dies each as there are, a
 //          row block in turn on each of them: with one die each and the others idle the 512 columns
 //          of VGG16 conv4_1 at M 980 took 14.4 us, on all dies 7.7;
 //          the unit comes from the kernel arguments at an offset that depends on the workgroup
-//          number alone, so that it arrives with the other arguments; workgroups of a half the
+//          number alone, so that it arrives with the other arguments; workgroups of a piece the
 //          unit does not have fill pruned columns (TW_PRUNED_ZERO) or leave
 //   stage: per wave 64 rows k of 32 rows m (64 bytes each), then reused for the wave's
-//          partial product [64 columns][32 + 4 rows m] in fp32
+//          partial product [its columns][32 + 4 rows m] in fp32
 // K-major A and C, or (RM) row-major ones; any beta.  A kept row of a row-major A is one 2-byte element
 // per m: a lane then takes one kept row of the step and fetches its 32 elements, 64 lanes together a few
 // neighbouring lines of each row m (a quarter kept: four), packs them into the same 64 bytes of the stage,
@@ -1936,11 +1936,11 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 //   The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
 constexpr int kSkRows = 32;                            // rows m of a workgroup
-constexpr int kSkCols = 64;                            // compact columns of a workgroup
+constexpr int kSkCols = 64;                            // compact columns of a workgroup, or half of them
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
-constexpr int kSkStage = kSkCols * kSkPitch * 4;       // 9216 bytes >= 64 * 64
 struct SkinnyWork {
-    int32_t n_units, halves, n_rowblk;
+    int32_t n_units, n_rowblk;
+    int32_t pieces, piece_shift; // of a unit: 1, 2 or 4, and its logarithm
     int32_t grouped;       // items of a row block in whole groups of eight units
     int32_t grouped_items; // n_rowblk times that
     uint32_t magic;        // 2^32 / grouped, rounded up
@@ -1948,28 +1948,31 @@ struct SkinnyWork {
     int32_t dies_per_unit; // kXcd / left
 };
 
-template <int DT, int NW, bool RM>
+template <int DT, int NW, bool RM, int NB>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
 {
     constexpr int NT = 64 * NW;
-    constexpr int RPT = kSkRows * kSkCols / NT; // rows of a column a thread adds up and stores: 8 or 4
+    constexpr int COLS = 32 * NB; // compact columns of a workgroup
+    constexpr int STAGE = COLS * kSkPitch * 4;
+    static_assert(STAGE >= 64 * 64, "a step of A fits the stage");
+    constexpr int RPT = kSkRows * COLS / NT; // rows of a column a thread adds up and stores: 8, 4 or 2
     using E = Elem<DT>;
-    __shared__ __align__(16) unsigned char sk_smem[NW * kSkStage];
+    __shared__ __align__(16) unsigned char sk_smem[NW * STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // (w.halves: 2, or 1 for a plan whose units all have at most 64 compact columns)
+    // (w.pieces of a unit: a power of two, COLS columns each)
     const int die = blockIdx.x % kXcd;
     int half, ui, yblk;
     bool in_range = true;
     if ((int)blockIdx.x < w.grouped_items) {
         yblk = (int)__umulhi(blockIdx.x, w.magic);
         const int rest = ((int)blockIdx.x - yblk * w.grouped) / kXcd;
-        half = w.halves == 2 ? rest & 1 : 0;
-        ui = (w.halves == 2 ? rest >> 1 : rest) * kXcd + die;
+        half = rest & (w.pieces - 1);
+        ui = (rest >> w.piece_shift) * kXcd + die;
     } else {
         const int rest = ((int)blockIdx.x - w.grouped_items) / kXcd;
-        half = w.halves == 2 ? rest & 1 : 0;
-        yblk = (w.halves == 2 ? rest >> 1 : rest) * w.dies_per_unit;
+        half = rest & (w.pieces - 1);
+        yblk = (rest >> w.piece_shift) * w.dies_per_unit;
         int v = die; // unit v of those left over, and which of its dies this is
         for (; v >= w.left; v -= w.left)
             ++yblk;
@@ -2017,19 +2020,19 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
 
     if (!in_range)
         return;
-    if (half * 2 < u.nb_cnt) {
+    if (half * NB < u.nb_cnt) {
         const int nsteps = u.k_pad / kBlockK;
-        const bool two_blocks = half * 2 + 1 < u.nb_cnt;
-        unsigned char *const stage = sk_smem + wave * kSkStage;
+        const bool two_blocks = NB == 2 && half * 2 + 1 < u.nb_cnt;
+        unsigned char *const stage = sk_smem + wave * STAGE;
         // the reducing role of this lane: column jj of the half, rows mr .. mr + RPT - 1
-        const int jj = RM ? lane : tid / (kSkRows / RPT), mr = RM ? wave * RPT : tid % (kSkRows / RPT) * RPT;
-        const int cnt = min(kSkCols, u.n_cnt - half * kSkCols);
+        const int jj = RM ? tid % COLS : tid / (kSkRows / RPT), mr = RM ? tid / COLS * RPT : tid % (kSkRows / RPT) * RPT;
+        const int cnt = min(COLS, u.n_cnt - half * COLS);
 
         struct Numbers {
             int row[RM ? 1 : 4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of the step (RM: kept row `lane`)
         };
         TW_GLOBAL(const unsigned char) const bsrc = Bp + u.b_off * 2 +
-                                          (int64_t)(u.nb0 + half * 2) * 4096 + lane * 16;
+                                          (int64_t)(u.nb0 + half * NB) * 4096 + lane * 16;
         const int64_t step_b = (int64_t)u.nblk * 4096;
         const int ch = lane & 3, row16 = lane >> 2;
         // Nothing on the way to the operands is conditional, so that the waits between the loads
@@ -2038,7 +2041,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         // have repeats the first (and is not stored).
         TW_GLOBAL(const uint16_t) const a_lane = A + m0 + (m0 + ch * 8 < M ? ch * 8 : 0);
         const int cb_off = two_blocks ? 4096 : 0;
-        u32x4 av[RM ? 1 : 4], bv[2][4];
+        u32x4 av[RM ? 1 : 4], bv[NB][4];
         uint32_t ae[RM ? kSkRows : 1];
         auto numbers = [&](int s) {
             Numbers n;
@@ -2053,7 +2056,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         };
         auto load_b = [&](int s, int k16) {
 #pragma unroll
-            for (int cb = 0; cb < 2; ++cb)
+            for (int cb = 0; cb < NB; ++cb)
                 bv[cb][k16] = *(TW_GLOBAL(const u32x4))(bsrc + s * step_b + cb * cb_off + k16 * 1024);
         };
         auto load_a = [&](const Numbers &n) {
@@ -2067,9 +2070,9 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                     av[i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[i] * lda);
             }
         };
-        f32x16 acc[2];
+        f32x16 acc[NB];
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
+        for (int cb = 0; cb < NB; ++cb)
 #pragma unroll
             for (int r = 0; r < 16; ++r)
                 acc[cb][r] = 0.0f;
@@ -2116,8 +2119,9 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                 const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + k16 * 1024 + 256));
                 const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
                 const u32x4 af = u32x4{l2.x, l2.y, h2.x, h2.y};
-                acc[0] = E::mfma(af, bv[0][k16], acc[0]);
-                acc[1] = E::mfma(af, bv[1][k16], acc[1]);
+#pragma unroll
+                for (int cb = 0; cb < NB; ++cb)
+                    acc[cb] = E::mfma(af, bv[cb][k16], acc[cb]);
                 if (MORE)
                     load_b(s + NW, k16);
             }
@@ -2126,7 +2130,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         int s = wave;
         Numbers n{};
         // where this lane's sums go, and the bias there: asked for ahead of what takes as long
-        const int out_n = kept_n[u.kn_off + half * kSkCols + (jj < cnt ? jj : 0)];
+        const int out_n = kept_n[u.kn_off + half * COLS + (jj < cnt ? jj : 0)];
         if (s < nsteps) {
             // (the weight fragments first: they do not wait for the row numbers)
             n = numbers(s);
@@ -2148,7 +2152,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         // the partial product of this wave: column cb * 32 + lane % 32, rows r4 * 8 + (lane / 32) * 4 + e
         float *const part = reinterpret_cast<float *>(stage);
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
+        for (int cb = 0; cb < NB; ++cb)
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
                 float *const dst = part + (cb * 32 + (lane & 31)) * kSkPitch + r4 * 8 + (lane >> 5) * 4;
@@ -2164,7 +2168,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             sum[e] = 0.0f;
 #pragma unroll
         for (int v = 0; v < NW; ++v) {
-            const float *const src = reinterpret_cast<const float *>(sk_smem + v * kSkStage) + jj * kSkPitch + mr;
+            const float *const src = reinterpret_cast<const float *>(sk_smem + v * STAGE) + jj * kSkPitch + mr;
 #pragma unroll
             for (int e = 0; e < RPT; ++e)
                 sum[e] += src[e];
@@ -2198,8 +2202,10 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             } else if (m0 + mr + RPT <= m_end) {
                 if constexpr (RPT == 8)
                     *reinterpret_cast<u32x4 *>(dst) = u32x4{h[0], h[1], h[2], h[3]};
-                else
+                else if constexpr (RPT == 4)
                     *reinterpret_cast<u32x2 *>(dst) = u32x2{h[0], h[1]};
+                else
+                    *reinterpret_cast<uint32_t *>(dst) = h[0];
             } else {
                 for (int e = 0; m0 + mr + e < m_end; ++e)
                     dst[e] = (uint16_t)(h[e >> 1] >> ((e & 1) * 16));
@@ -2209,7 +2215,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
 
     // ---- TW_PRUNED_ZERO: pruned columns receive act(beta * C + bias); shared out over the
     // workgroups of a row block
-    for (int z = p.n_gemm_u + ui * w.halves + half; z < p.n_all_u; z += w.n_units * w.halves) {
+    for (int z = p.n_gemm_u + ui * w.pieces + half; z < p.n_all_u; z += w.n_units * w.pieces) {
         const TileDev t = p.tiles[z - p.n_gemm_u];
         if constexpr (RM) {
             for (int i = tid; i < t.n_pruned * kSkRows; i += NT) {
@@ -2537,18 +2543,19 @@ int get_option(int option_id) { return option(option_id); }
 
 constexpr int kSkFewSteps = 4; // steps of the longest tile up to which the skinny kernel runs with four waves
 
-// The skinny kernel's work on M rows and its number of workgroups, or -1 where that is more than it
+// The skinny kernel's work on M rows in pieces of `cols` columns (64 or 32) and its number of workgroups, or -1 where that is more than it
 // numbers: it divides a workgroup's number by `grouped` with a multiplication, exact while number *
 // grouped stays below 2^32.
-static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w)
+static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w, int cols = kSkCols)
 {
     w->n_units = plan->n_units;
-    w->halves = plan->max_unit_n > kSkCols ? 2 : 1;
+    w->piece_shift = plan->max_unit_n > 2 * cols ? 2 : plan->max_unit_n > cols ? 1 : 0;
+    w->pieces = 1 << w->piece_shift;
     w->n_rowblk = (M + kSkRows - 1) / kSkRows;
     w->left = plan->n_units % kXcd;
     w->dies_per_unit = w->left ? kXcd / w->left : 1;
-    const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->halves, grouped_items = grouped * w->n_rowblk;
-    const int64_t left_items = w->left ? (int64_t)kXcd * w->halves * ((w->n_rowblk + w->dies_per_unit - 1) / w->dies_per_unit) : 0;
+    const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->pieces, grouped_items = grouped * w->n_rowblk;
+    const int64_t left_items = w->left ? (int64_t)kXcd * w->pieces * ((w->n_rowblk + w->dies_per_unit - 1) / w->dies_per_unit) : 0;
     if ((grouped_items + left_items) * 64 * 8 > kMaxGridThreads || grouped_items * grouped >= (1ll << 32))
         return -1;
     w->grouped = (int32_t)grouped;
@@ -2557,12 +2564,17 @@ static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w)
     return grouped_items + left_items;
 }
 
+// Workgroups on the die that has most of them.
+static int64_t skinny_per_die(const SkinnyWork &w)
+{
+    return (int64_t)w.grouped / kXcd * w.n_rowblk + (w.left ? (int64_t)w.pieces * ((w.n_rowblk + w.dies_per_unit - 1) / w.dies_per_unit) : 0);
+}
+
 // Its workgroups to a compute unit of the die that has most of them (second halves that a unit narrower than the
 // others does not have leave at once and are not counted).
 static double skinny_load(const tw_plan *plan, const SkinnyWork &w)
 {
-    const int per_die = w.grouped / kXcd * w.n_rowblk + (w.left ? w.halves * ((w.n_rowblk + w.dies_per_unit - 1) / w.dies_per_unit) : 0);
-    return (double)per_die * kXcd / plan->cu_count * plan->n_halves / (plan->n_units * w.halves);
+    return (double)skinny_per_die(w) * kXcd / plan->cu_count * plan->n_halves / (plan->n_units * w.pieces);
 }
 
 static int round_up32(int v) { return (v + 31) / 32 * 32; }
@@ -2877,10 +2889,24 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     const int64_t items = skinny_work(plan, a.M, &w);
     if (items < 0)
         return fail(TW_ERR_SHAPE, "M=%d: more row blocks than the skinny kernel numbers", a.M);
-    if (plan->max_k_pad <= kSkFewSteps * kBlockK)
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
-    else
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
+    const bool few = plan->max_k_pad <= kSkFewSteps * kBlockK;
+    // Pieces of 32 columns while no compute unit gets two workgroups: a workgroup on a compute unit of its own is bound by what
+    // that fetches (50 bytes a clock, 12 KB a step of 64 columns, 8 KB of 32), and the other compute units are idle.  us with
+    // pieces of 64 and of 32, K-major and row-major: M 64, K 4608, N 512, half the rows kept 6.5 and 5.0, 12.9 and 12.3; M 64,
+    // K 2304, N 256 4.6 and 3.8, 8.1 and 7.7; M 256, K 4096, N 1024 (256 workgroups) 5.1 and 4.7, 9.5 and 9.5; four waves,
+    // M 128, K 768, N 768 3.1 and 2.8, 4.5 and 4.1.  From 288 workgroups on 1.02 - 1.20 of the time, and 1.05 - 1.49.
+    SkinnyWork narrow;
+    const int64_t narrow_items = skinny_work(plan, a.M, &narrow, kSkCols / 2);
+    if (narrow_items >= 0 && skinny_per_die(narrow) * kXcd <= plan->cu_count) {
+        if (few)
+            hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 1>), dim3((unsigned)narrow_items), dim3(64 * 4), 0, s, a, narrow);
+        else
+            hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 1>), dim3((unsigned)narrow_items), dim3(64 * 8), 0, s, a, narrow);
+    } else if (few) {
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 2>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
+    } else {
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 2>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
+    }
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
