@@ -146,9 +146,27 @@ __device__ __forceinline__ float tw_finish(float v, const float *bias, int c, in
 // w = 32 * piece_nb and j = uv % n_split.  A piece beyond the unit's columns keeps valid
 // offsets and has n_cnt == 0: it runs like any other and stores nothing.  The descriptor is
 // workgroup-uniform and ends up in scalar registers.
-__device__ __forceinline__ UnitDev load_unit(const GemmArgs &p, int uv)
+__device__ __forceinline__ UnitDev unit_piece(const GemmArgs &p, int uv, int ui, const int32_t (&w)[12])
 {
     static_assert(sizeof(UnitDev) == 48, "UnitDev is read as 12 words");
+    UnitDev u;
+    __builtin_memcpy(&u, w, sizeof(UnitDev));
+    if (p.n_split > 1) {
+        const int j = uv - ui * p.n_split;
+        const int bps = p.piece_nb; // 32-column blocks per piece
+        const int nb = min(max(u.nb_cnt - j * bps, 0), bps);
+        const int nc = min(max(u.n_cnt - j * bps * kMfmaN, 0), bps * kMfmaN);
+        if (nb > 0) {
+            u.nb0 += j * bps;
+            u.kn_off += j * bps * kMfmaN;
+        }
+        u.nb_cnt = nb;
+        u.n_cnt = nc;
+    }
+    return u;
+}
+__device__ __forceinline__ UnitDev load_unit(const GemmArgs &p, int uv)
+{
     const int ui = uv / p.n_split;
     int32_t w[12];
     if (p.n_arg_units) {
@@ -168,21 +186,21 @@ __device__ __forceinline__ UnitDev load_unit(const GemmArgs &p, int uv)
 #pragma unroll
     for (int i = 0; i < 12; ++i)
         w[i] = __builtin_amdgcn_readfirstlane(w[i]);
-    UnitDev u;
-    __builtin_memcpy(&u, w, sizeof(UnitDev));
-    if (p.n_split > 1) {
-        const int j = uv - ui * p.n_split;
-        const int bps = p.piece_nb; // 32-column blocks per piece
-        const int nb = min(max(u.nb_cnt - j * bps, 0), bps);
-        const int nc = min(max(u.n_cnt - j * bps * kMfmaN, 0), bps * kMfmaN);
-        if (nb > 0) {
-            u.nb0 += j * bps;
-            u.kn_off += j * bps * kMfmaN;
-        }
-        u.nb_cnt = nb;
-        u.n_cnt = nc;
-    }
-    return u;
+    return unit_piece(p, uv, ui, w);
+}
+// The same in two parts: word `lane` of the unit of piece `uv`, by a vector load, and the piece out of the wave's words.
+__device__ __forceinline__ int unit_word(const GemmArgs &p, int uv, int lane)
+{
+    const int ui = uv / p.n_split;
+    return reinterpret_cast<const int32_t *>(p.units + ui)[lane < 12 ? lane : 0];
+}
+__device__ __forceinline__ UnitDev unit_of_words(const GemmArgs &p, int uv, int words)
+{
+    int32_t w[12];
+#pragma unroll
+    for (int i = 0; i < 12; ++i)
+        w[i] = __builtin_amdgcn_readlane(words, i);
+    return unit_piece(p, uv, uv / p.n_split, w);
 }
 
 // Workgroup barrier for hand-overs through LDS only: waits for this wave's LDS operations, not

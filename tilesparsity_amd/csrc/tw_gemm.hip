@@ -648,12 +648,16 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
         int m0, m_end; // rows [m0, m_end) of A and C, at most BM of them
         UnitDev u;     // col < n_gemm_u
     };
-    auto make_item = [&](int ticket) {
+    auto place_item = [&](int ticket) { // (without its unit)
         Item it;
         const Work w = queue_entry(p, qx, ticket, BM);
         it.col = w.kind == ITEM_END ? p.n_all_u : w.u;
         it.m0 = w.m0;
         it.m_end = it.m0 + w.rows < p.M ? it.m0 + w.rows : p.M;
+        return it;
+    };
+    auto make_item = [&](int ticket) {
+        Item it = place_item(ticket);
         if (it.col < p.n_gemm_u)
             it.u = load_unit(p, it.col);
         return it;
@@ -672,13 +676,21 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
     bool closed = false;    // thread 0: no claim of this workgroup is in flight, none will follow
     bool announced = false; // thread 0: the workgroup has been counted as done with the counter
     int t_done = -1;        // thread 0: workgroups counted before this one (atomic's result)
+    // One more for counter i of the slot.  (To an address that the compiler cannot take for the same in all lanes: it would add
+    // up the wave's ones first and hand the result out through a scalar register, waiting on the spot for the atomic's way
+    // to memory and back, about 1000 cycles at every item's end.)
+    auto count = [&](int i) {
+        int none;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(none));
+        return atomicAdd(&p.ticket[i + none], 1);
+    };
     if (tid == 0) {
         if (qi < qlen) {
-            t_pending = atomicAdd(&p.ticket[qx], 1);
+            t_pending = count(qx);
         } else { // nothing for this workgroup: it only counts itself as done
             closed = true;
             announced = true;
-            t_done = atomicAdd(&p.ticket[kXcd], 1);
+            t_done = count(kXcd);
         }
     }
     // Picks up the claim in flight and starts the one after it, unless the queue is exhausted.
@@ -693,7 +705,7 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                 t_next = ticket_base + t_pending;
                 asm volatile("" : "+v"(t_next)); // here, not where it is published
                 if (t_next < qlen)
-                    t_pending = atomicAdd(&p.ticket[qx], 1);
+                    t_pending = count(qx);
                 else
                     closed = true;
             }
@@ -710,7 +722,7 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                 asm volatile("" ::"v"(t_pending));
                 closed = true;
             }
-            t_done = atomicAdd(&p.ticket[kXcd], 1);
+            t_done = count(kXcd);
             announced = true;
         }
     };
@@ -725,6 +737,7 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
         }
     };
     auto published = [&]() { return make_item(__builtin_amdgcn_readfirstlane(s_tk[0])); };
+    auto published_place = [&]() { return place_item(__builtin_amdgcn_readfirstlane(s_tk[0])); };
     auto claim = [&]() { // two barriers of its own: items without steps
         publish();
         TW_LDS_BARRIER();
@@ -981,18 +994,27 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                     if (deferred)
                         store_deferred();
                     meet_wide(deferred); // time slot 0: step 0 has landed
-                    if (!have_next) {
+                    // The next item, and its first index words, for the loads that the last time slot
+                    // issues on its behalf: fetched early, so that nobody waits for them there, and in two parts behind
+                    // the loads of the time slots 1 and 2, where the multiplying waves do not wait for these waves (both in
+                    // time slot 0: 2000 cycles until the next loads leave, half of them waited for)
+                    bool chain = false;
+                    Ctx cn = c;
+                    auto learn = [&]() {
                         nxt = published();
                         have_next = true;
-                    }
-                    // the next item's first index words, for the loads that the last time slot
-                    // issues on its behalf: fetched now, so that nobody waits for them there
-                    const bool chain = nsteps >= 2 && has_steps(nxt);
-                    Ctx cn = c;
-                    if (chain) {
-                        cn = ctx_of(nxt);
-                        load_idx_scalar(cn, 0, n0);
-                        load_idx_scalar(cn, 1, n1);
+                        chain = nsteps >= 2 && has_steps(nxt);
+                    };
+                    auto look_ahead = [&]() {
+                        if (chain) {
+                            cn = ctx_of(nxt);
+                            load_idx_scalar(cn, 0, n0);
+                            load_idx_scalar(cn, 1, n1);
+                        }
+                    };
+                    if (nsteps < 4) {
+                        learn();
+                        look_ahead();
                     }
                     // time slots 1 .. nsteps - 2 issue the steps 2 .. nsteps - 1 (odd slots out
                     // of i0, even ones out of i1)
@@ -1001,10 +1023,14 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                         load_idx(c, j + 2, i1);
                         fence();
                         issue(c, j + 1, (gs + j + 1) % NST, i0);
+                        if (j == 1)
+                            learn();
                         meet_wide(deferred && j == 1);
                         load_idx(c, j + 3, i0);
                         fence();
                         issue(c, j + 2, (gs + j + 2) % NST, i1);
+                        if (j == 1)
+                            look_ahead();
                         meet();
                     }
                     if (j + 1 < nsteps) {
@@ -1301,9 +1327,15 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                 if (!have_next)
                     publish();
                 TW_LDS_BARRIER(); // time slot 0: step 0 is being staged
-                if (!have_next) {
-                    nxt = published();
+                // (the next item's unit on its way to vector registers, a word a lane, for the end of the steps: scalar loads
+                // would be waited for by the first read of a stage, 1100 cycles of every item)
+                int next_unit = 0;
+                const bool new_next = !have_next;
+                if (new_next) {
+                    nxt = published_place();
                     have_next = true;
+                    if (nxt.col < p.n_gemm_u)
+                        next_unit = unit_word(p, nxt.col, lane);
                 }
                 for (int s = 0; s < nsteps; ++s) {
                     if (w_active) {
@@ -1333,6 +1365,9 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
                     }
                     TW_LDS_BARRIER();
                 }
+
+                if (new_next && nxt.col < p.n_gemm_u)
+                    nxt.u = unit_of_words(p, nxt.col, next_unit);
 
                 // epilogue: alpha/beta in fp32, round, hand the tile over through LDS
                 float scale = p.alpha;
