@@ -53,6 +53,20 @@ def test_plan_from_mask_bit_exact(tw, oracle, K, N, G, dtype):
         check_export(oracle, plan, expect, B, dtype)
 
 
+@pytest.mark.parametrize("K,N,G", [(1300, 2048, 2048), (1025, 2049, 2049), (1300, 4100, 4100), (2100, 64, 1),
+                                   (130, 192, 3), (130, 195, 3), (9000, 5, 5), (1, 513, 513)])
+def test_lists_at_the_edges_of_their_windows(tw, oracle, K, N, G):
+    """Tables of 64 tiles (in the kernel arguments) and of 65, tiles of one window of columns, of a column more and of
+    two, more slabs of rows than one pass of a window's threads takes."""
+    rng = np.random.default_rng(K * 7 + N)
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    tiles = random_tiles(rng, K, N, G, k_keep=0.2, n_keep=0.6, empty_every=6)
+    mask = oracle.plan_mask(K, N, tiles)
+    print("lists at the edges", K, N, G, flush=True)
+    with tw.Plan.from_mask(mask, G, "f16", B) as plan:
+        check_export(oracle, plan, oracle.plan_from_mask(mask, G), B, "f16")
+
+
 @pytest.mark.parametrize("name", ["vgg16_conv4_2", "imbalance_stress"])
 def test_plan_from_mask_full_size_configurations(tw, oracle, name):
     """The mask -> kept lists -> relative offsets -> compaction pre-pass at the full size of the

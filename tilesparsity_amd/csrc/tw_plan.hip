@@ -247,15 +247,27 @@ __global__ void unpack_stream_kernel(const PlanTile *tiles, const uint16_t *Bp, 
 // Rows of one tile and slab, and what a slab of kFlagRows rows of it says about the columns.
 constexpr int kFlagRows = 128, kFlagPasses = kFlagRows / 8; // passes over the rows at 32 lanes a row
 constexpr int kMaxTileRows = 32768; // tiles of one launch, where they are the rows of its grid
+constexpr int kFlagArgTiles = 64;   // tiles whose first columns fit the kernel arguments
 struct FlagArgs {
     const uint8_t *mask;
-    const int32_t *tcol0; // host memory (pinned): first column of each tile, N behind the last
+    const int32_t *tcol0; // host memory (pinned): first column of each tile, N behind the last; null: arg_tcol0
     int32_t K, N, n_slabs, tile0;
     uint8_t *rowflag;     // [tile][K]
     uint8_t *colpart;     // per tile [slab][width, rounded up to 4], see colpart_at
     uint32_t *nnz;        // [tile][slab]: non-zero elements
+    int32_t arg_tcol0[kFlagArgTiles + 1];
     __device__ int64_t colpart_at(int t, int c0) const { return (int64_t)(((int64_t)c0 + 3 * t + 3) & ~(int64_t)3) * n_slabs; }
 };
+
+// First column of tile t (uniform), out of the arguments of a kernel whose first one is `a`: a read of the host's memory across
+// the bus, at the head of both kernels, takes 1.5 us.
+__device__ __forceinline__ int flag_col0(const FlagArgs &a, int t)
+{
+    if (a.tcol0)
+        return a.tcol0[t];
+    const auto *ka = (const __attribute__((address_space(4))) int32_t *)__builtin_amdgcn_kernarg_segment_ptr();
+    return ka[offsetof(FlagArgs, arg_tcol0) / 4 + t];
+}
 
 // Workgroup (slab, tile): kFlagRows rows of one tile, so every flag has one writer and nothing has to
 // be cleared first.  Each row is taken by 8, 16 or 32 lanes of 16 bytes (windows of 32 lanes for wider
@@ -266,7 +278,7 @@ __global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
     __shared__ uint32_t s_col[4][128]; // per wave, a window's columns
     __shared__ uint32_t s_nnz;
     const int slab = (int)blockIdx.x, t = a.tile0 + (int)blockIdx.y;
-    const int c0 = a.tcol0[t], w = a.tcol0[t + 1] - c0;
+    const int c0 = flag_col0(a, t), w = flag_col0(a, t + 1) - c0;
     const int k0 = slab * kFlagRows, nr = min(kFlagRows, a.K - k0);
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // the widest aligned load the mask allows: 16 bytes, 4 or 1
@@ -367,12 +379,11 @@ __global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
         a.nnz[(int64_t)t * a.n_slabs + slab] = s_nnz;
 }
 
-// What the host needs to know of a tile before it can lay the plan out, in pinned memory.
+// What the host needs to know of a tile before it can lay the plan out, in pinned memory: kept rows, kept columns, the low and
+// the high half of the number of non-zero elements, each with the build's number above it.  A word is written
+// at once, so none of them has to wait for another on its way across the bus.
 struct TileCounts {
-    unsigned long long nnz;
-    int32_t k_kept, n_kept;
-    uint32_t stamp; // the build's number, written last
-    uint32_t pad_[3];
+    unsigned long long word[4];
 };
 
 // One workgroup per tile: ascending lists of the kept rows (at kk + t * K), of the kept columns and of
@@ -384,10 +395,10 @@ __global__ void __launch_bounds__(kListThreads)
 {
     constexpr int NW = kListThreads / 64;
     __shared__ int s_wave[NW];
-    __shared__ uint32_t s_cols[1024]; // flags of a window of 4096 columns
+    __shared__ uint32_t s_cols[kListThreads]; // flags of a window of four times as many columns
     __shared__ unsigned long long s_nnz;
     const int t = (int)blockIdx.x, tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c0 = a.tcol0[t], w = a.tcol0[t + 1] - c0;
+    const int c0 = flag_col0(a, t), w = flag_col0(a, t + 1) - c0;
     // position of this thread's first one among all ones of the workgroup, and their number
     auto scan = [&](int mine, int &total) {
         int incl = mine;
@@ -411,6 +422,29 @@ __global__ void __launch_bounds__(kListThreads)
     };
     if (tid == 0)
         s_nnz = 0;
+    // What the slabs say about a window's columns: four of them a thread, 2^lg threads side by side, the slabs dealt out over the
+    // groups.  All loads of eight slabs are in flight at once, and the first window's fly over the rows' part (one slab after
+    // another behind it: K 4608 in two tiles 7.9 us).
+    const int words = ((w + 3) & ~3) >> 2;
+    const uint32_t *const part = reinterpret_cast<const uint32_t *>(a.colpart + a.colpart_at(t, c0));
+    const int lg = words >= kListThreads ? 9 : words > 1 ? 32 - __clz(words - 1) : 0, groups = kListThreads >> lg;
+    static_assert(kListThreads == 512, "a window is at most 2^9 words");
+    const int cj = tid & ((1 << lg) - 1);
+    auto slabs_of = [&](int base) {
+        uint32_t x = 0;
+        const uint32_t *const src = part + min(base + cj, words - 1);
+        for (int slab = tid >> lg; slab < a.n_slabs; slab += 8 * groups) {
+            uint32_t v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                v[i] = src[(int64_t)min(slab + i * groups, a.n_slabs - 1) * words];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                x |= v[i];
+        }
+        return x;
+    };
+    uint32_t cols = slabs_of(0);
     unsigned long long nnz = 0;
     for (int i = tid; i < a.n_slabs; i += kListThreads)
         nnz += a.nnz[(int64_t)t * a.n_slabs + i];
@@ -439,49 +473,36 @@ __global__ void __launch_bounds__(kListThreads)
         atomicAdd(&s_nnz, nnz);
 
     // columns: kept where any slab says so
-    const int words = ((w + 3) & ~3) >> 2;
-    const uint32_t *const part = reinterpret_cast<const uint32_t *>(a.colpart + a.colpart_at(t, c0));
     int n_kept = 0;
-    for (int base = 0; base < words; base += 1024) {
-        const int nw = min(1024, words - base);
-        for (int i = tid; i < nw; i += kListThreads)
-            s_cols[i] = 0;
+    for (int base = 0; base < words; base += kListThreads) {
+        const int nw = min(kListThreads, words - base);
+        if (base > 0)
+            cols = slabs_of(base);
+        s_cols[tid] = 0;
         __syncthreads();
-        for (int i = tid; i < nw * a.n_slabs; i += kListThreads) {
-            const int slab = i / nw, j = i - slab * nw;
-            const uint32_t x = part[(int64_t)slab * words + base + j];
-            if (x)
-                atomicOr(&s_cols[j], x);
-        }
+        if (cj < nw && cols)
+            atomicOr(&s_cols[cj], cols);
         __syncthreads();
-        // (four columns, one word, per thread and round)
-        for (int r = 0; r < nw; r += kListThreads) {
-            const int j = r + tid;
-            const int here = min(max(w - (base + j) * 4, 0), 4); // columns of this word (what lies behind them was not written)
-            const uint32_t x = (j < nw ? s_cols[j] : 0u) & (uint32_t)((1ull << (here * 8)) - 1ull);
-            int total;
-            int at = n_kept + scan(__popc(x), total);
-            const int col = (base + j) * 4;
-            int pruned = col - at; // pruned columns before this word
+        const int here = min(max(w - (base + tid) * 4, 0), 4); // columns of this word (what lies behind them was not written)
+        const uint32_t x = (tid < nw ? s_cols[tid] : 0u) & (uint32_t)((1ull << (here * 8)) - 1ull);
+        int total;
+        int at = n_kept + scan(__popc(x), total);
+        const int col = (base + tid) * 4;
+        int pruned = col - at; // pruned columns before this word
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (j >= nw || col + e >= w)
-                    break;
-                if (x >> (e * 8) & 0xFFu)
-                    kn[c0 + at++] = col + e;
-                else
-                    pn[c0 + pruned++] = col + e;
-            }
-            n_kept += total;
+        for (int e = 0; e < 4; ++e) {
+            if (tid >= nw || col + e >= w)
+                break;
+            if (x >> (e * 8) & 0xFFu)
+                kn[c0 + at++] = col + e;
+            else
+                pn[c0 + pruned++] = col + e;
         }
+        n_kept += total;
     }
-    if (tid == 0) {
-        volatile TileCounts *const c = counts + t;
-        c->nnz = s_nnz;
-        c->k_kept = k_kept;
-        c->n_kept = n_kept;
-        __threadfence_system(); // the counts are in host memory before the stamp that announces them
-        c->stamp = stamp;
+    if (tid < 4) {
+        const uint32_t v = tid == 0 ? (uint32_t)k_kept : tid == 1 ? (uint32_t)n_kept : tid == 2 ? (uint32_t)s_nnz : (uint32_t)(s_nnz >> 32);
+        reinterpret_cast<volatile TileCounts *>(counts)[t].word[tid] = (unsigned long long)stamp << 32 | v;
     }
 }
 
@@ -1208,17 +1229,18 @@ static int plan_from_device_mask(int K, int N, int dtype, int n_tiles, const int
     char *const ws = static_cast<char *>(ws_owner.ptr);
     volatile TileCounts *const counts = static_cast<volatile TileCounts *>(pinned.ptr);
     int32_t *const h_tcol0 = reinterpret_cast<int32_t *>(static_cast<char *>(pinned.ptr) + counts_bytes);
-    std::memcpy(h_tcol0, tcol0.data(), sizeof(int32_t) * (nt + 1));
+    FlagArgs fa;
+    fa.tcol0 = nt <= kFlagArgTiles ? nullptr : h_tcol0;
+    std::memcpy(nt <= kFlagArgTiles ? fa.arg_tcol0 : h_tcol0, tcol0.data(), sizeof(int32_t) * (nt + 1));
     // (never 0, and another number for every build, so that a stamp an earlier build left is not taken for this one's)
     static std::atomic<uint32_t> builds{0};
     uint32_t stamp = ++builds;
     if (stamp == 0)
         stamp = ++builds;
     for (int t = 0; t < nt; ++t)
-        counts[t].stamp = 0;
-    FlagArgs fa;
+        for (int i = 0; i < 4; ++i)
+            counts[t].word[i] = 0;
     fa.mask = d_mask;
-    fa.tcol0 = h_tcol0;
     fa.K = K;
     fa.N = N;
     fa.n_slabs = n_slabs;
@@ -1260,18 +1282,22 @@ static int plan_from_device_mask(int K, int N, int dtype, int n_tiles, const int
     unsigned long long mismatch = 0;
     int64_t sum_k = 0;
     for (int t = 0; t < nt; ++t) {
-        for (long spin = 0; counts[t].stamp != stamp; ++spin) {
-            if (spin < 200000) {
-                __builtin_ia32_pause();
-                continue;
+        uint32_t count[4];
+        for (int i = 0; i < 4; ++i) {
+            unsigned long long word;
+            for (long spin = 0; (word = counts[t].word[i]) >> 32 != stamp; ++spin) {
+                if (spin < 200000) {
+                    __builtin_ia32_pause();
+                    continue;
+                }
+                TW_HIP(hipStreamSynchronize(s));
+                if (counts[t].word[i] >> 32 != stamp)
+                    return fail(TW_ERR_DEVICE, "the pre-pass left no counts for tile %d", t);
             }
-            TW_HIP(hipStreamSynchronize(s));
-            if (counts[t].stamp != stamp)
-                return fail(TW_ERR_DEVICE, "the pre-pass left no counts for tile %d", t);
+            count[i] = (uint32_t)word;
         }
-        std::atomic_thread_fence(std::memory_order_acquire);
-        const int32_t rows = counts[t].k_kept, cols = counts[t].n_kept;
-        mismatch += (unsigned long long)rows * (unsigned long long)cols - counts[t].nnz;
+        const int32_t rows = (int32_t)count[0], cols = (int32_t)count[1];
+        mismatch += (unsigned long long)rows * (unsigned long long)cols - ((unsigned long long)count[3] << 32 | count[2]);
         sum_k += rows;
         p->kept_k_ptr[t + 1] = (int32_t)std::min<int64_t>(sum_k, INT32_MAX);
         p->kept_n_ptr[t + 1] = p->kept_n_ptr[t] + cols;
