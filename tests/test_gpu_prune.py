@@ -113,6 +113,25 @@ def test_2d_matches_oracle(twprune, po, shapes, g, sparsity, transform):
     assert got_tables == tables
 
 
+@pytest.mark.parametrize("widths, g", [
+    ([64, 65, 1, 63, 128, 4097], 1),             # tiles that end at every kept column, groups of one column
+    ([140000, 7], 100),                          # more groups of 64 columns than are taken at a time, one layer across the line
+    ([200] * 700, 33),                           # more of them over many layers
+    ([40, 3] * 600, 5),                          # more layers than are taken at a time
+    ([12288], 128), ([12289], 5000),             # columns kept in LDS, and one too many
+])
+def test_2d_groups_of_columns(twprune, po, widths, g):
+    """The step between the stages of the 2-D producer takes the columns of all layers in groups of 64."""
+    rng = np.random.default_rng(sum(widths) + g)
+    scores = [np.abs(rng.standard_normal((3, n))).astype(np.float32) for n in widths]
+    print("2d groups", len(widths), sum(widths), g, flush=True)
+    want, _, tables, _ = po.tiled_wise_2d(scores, 60, g)
+    got, got_tables = twprune.tiled_wise_2d(scores, 60, g, return_tiles=True)
+    for a, b, t, u in zip(want, got, tables, got_tables):
+        assert np.array_equal(a, b)
+        assert [tuple(x) for x in t] == [tuple(x) for x in u]
+
+
 def test_ties_and_extremes(twprune, po):
     rng = np.random.default_rng(21)
     # scores on a coarse grid: many rows share a norm, some tie with the threshold

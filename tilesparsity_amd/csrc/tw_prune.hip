@@ -507,8 +507,9 @@ template <int NT, int NB, bool NEXT = false, class T> __device__ Digit find_digi
     if (tid == 0)
         s_d = Digit{kLostRank, 1, (uint32_t)NB - 1u, 0xFFFFFFFFu};
     __syncthreads();
-    for (int w = 0; w < wave; ++w)
-        incl += s_wave[w];
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) // (all of them at once, not one after another)
+        incl += w < wave ? s_wave[w] : 0ull;
     unsigned long long before = incl - sum;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
@@ -694,7 +695,7 @@ template <int PASS> __global__ void __launch_bounds__(256) select_hist_kernel(co
 // The selection in one workgroup and its LDS, for a few ten thousand values (the columns of a network, a
 // sample).  The digits are those of the keys' own range, so that the values spread over all counters:
 // lanes of a wave that meet in one LDS counter take turns.
-template <int NT, class V> __device__ KeyRange key_range_in_block(V key, int n)
+template <class V> __device__ KeyRange key_range_in_block(V each)
 {
     __shared__ uint32_t s_lo, s_hi;
     if (threadIdx.x == 0) {
@@ -703,11 +704,10 @@ template <int NT, class V> __device__ KeyRange key_range_in_block(V key, int n)
     }
     __syncthreads();
     uint32_t lo = 0xFFFFFFFFu, hi = 0;
-    for (int i = (int)threadIdx.x; i < n; i += NT) {
-        const uint32_t k = key(i);
+    each([&](uint32_t k) {
         lo = min(lo, k);
         hi = max(hi, k);
-    }
+    });
     for (int off = 32; off > 0; off >>= 1) {
         lo = min(lo, (uint32_t)__shfl_down(lo, off));
         hi = max(hi, (uint32_t)__shfl_down(hi, off));
@@ -721,34 +721,33 @@ template <int NT, class V> __device__ KeyRange key_range_in_block(V key, int n)
 }
 // one pass: rank becomes the rank among the values that share the digits so far
 template <int PASS, int NT, class V>
-__device__ Digit count_in_block(V key, int n, const KeyRange &range, unsigned long long &rank, uint32_t &prefix, unsigned int *s_h,
+__device__ Digit count_in_block(V each, const KeyRange &range, unsigned long long &rank, uint32_t &prefix, unsigned int *s_h,
                                 uint32_t &mn)
 {
     for (int i = (int)threadIdx.x; i < kSelBins; i += NT)
         s_h[i] = 0;
     __syncthreads();
-    for (int i = (int)threadIdx.x; i < n; i += NT)
-        select_count<PASS>(key(i), range, prefix, s_h, mn);
+    each([&](uint32_t k) { select_count<PASS>(k, range, prefix, s_h, mn); });
     __syncthreads();
     const Digit d = find_digit<NT, PASS == 2 ? 1024 : kSelBins, PASS != 0>(s_h, rank);
     prefix = PASS == 0 ? d.digit : prefix << (range.lead_shift(PASS) - range.shift[PASS]) | d.digit;
     rank = d.rest;
     return d;
 }
-template <int NT, class V> __device__ Threshold select_in_block(V key, const SelectHead *h, unsigned int *s_h)
+// (each(f): f of every key of this thread's)
+template <int NT, class V> __device__ Threshold select_in_block(V each, const SelectHead *h, unsigned int *s_h)
 {
     __shared__ uint32_t s_min;
     __shared__ Threshold s_t;
     if (threadIdx.x == 0)
         s_min = 0xFFFFFFFFu;
-    const int n = (int)h->n;
-    const KeyRange range = key_range_in_block<NT>(key, n);
+    const KeyRange range = key_range_in_block(each);
     uint32_t prefix = 0, mn = 0xFFFFFFFFu;
     unsigned long long rank = h->rank0;
-    count_in_block<0, NT>(key, n, range, rank, prefix, s_h, mn);
-    Digit d = count_in_block<1, NT>(key, n, range, rank, prefix, s_h, mn);
+    count_in_block<0, NT>(each, range, rank, prefix, s_h, mn);
+    Digit d = count_in_block<1, NT>(each, range, rank, prefix, s_h, mn);
     if (range.shift[1] > 0) // (else two digits hold all of the range)
-        d = count_in_block<2, NT>(key, n, range, rank, prefix, s_h, mn);
+        d = count_in_block<2, NT>(each, range, rank, prefix, s_h, mn);
     for (int off = 32; off > 0; off >>= 1)
         mn = min(mn, (uint32_t)__shfl_down(mn, off));
     if ((threadIdx.x & 63) == 0)
@@ -806,7 +805,12 @@ template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(c
     if (tid == 0)
         select_rank(&s_head, K, q, q_is_f64);
     __syncthreads();
-    const Threshold t = select_in_block<256>([&](int i) { return sort_key(s_v[i]); }, &s_head, s_h);
+    const Threshold t = select_in_block<256>(
+        [&](auto f) {
+            for (int i = tid; i < K; i += 256)
+                f(sort_key(s_v[i]));
+        },
+        &s_head, s_h);
     if (tid == 0) {
         out[blockIdx.x] = t;
         if (t.lost)
@@ -818,8 +822,13 @@ template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(c
 // all column norms, the column masks, every layer's tiles (they end after every `granularity` kept
 // columns) and where its norms and its row-norm items begin, and the state of the row selection.
 // All on the device, so that the call needs no trip to the host between its stages.
+// What bounds it is the chain of LDS trips and barriers of one workgroup: the keys stay in registers over the selection's
+// passes, and all layers' columns are taken together in groups of 64, the waves a run of groups each, and then every group's
+// tiles by a thread of its own from the sums of the groups before it.  VGG16's layers (8832 columns) 31 -> 22 us; in front of
+// that a wave took a layer, group after group (N 4096: 64 times 570 cycles, 15 us).
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanStage = 12288; // column norms kept in LDS; more of them are read from memory in every pass
+constexpr int kPlanGroups = 2 * kPlanThreads; // groups of 64 columns at a time
 __global__ void __launch_bounds__(kPlanThreads)
     plan_2d_kernel(PruneLayer *layers, int n_layers, const float *cnorm, int64_t n_cols, float *norms,
                    SelectState *st_rows, int64_t *n_items, double q, int q_is_f64, Mail *mail)
@@ -828,15 +837,19 @@ __global__ void __launch_bounds__(kPlanThreads)
     __shared__ SelectHead s_head;
     __shared__ int64_t s_norm[kPlanThreads], s_item[kPlanThreads];
     __shared__ float s_cn[kPlanStage];
-    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ unsigned long long s_bits[kPlanGroups]; // which columns of a group are kept
+    __shared__ uint16_t s_layer[kPlanGroups];
+    __shared__ uint32_t s_first[kPlanThreads + 1];     // first group of each layer
+    __shared__ uint32_t s_start[kPlanThreads];         // kept columns of the layers before it
+    __shared__ uint32_t s_sum[kPlanThreads / 64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool staged = n_cols <= kPlanStage;
+    constexpr int PER = kPlanStage / kPlanThreads;
+    float v[PER];
     if (staged) {
-        constexpr int PER = kPlanStage / kPlanThreads;
-        float v[PER];
 #pragma unroll
         for (int i = 0; i < PER; ++i)
-            if (tid + i * kPlanThreads < n_cols)
-                v[i] = cnorm[tid + i * kPlanThreads];
+            v[i] = cnorm[min((int64_t)tid + i * kPlanThreads, n_cols - 1)];
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (tid + i * kPlanThreads < n_cols)
@@ -850,53 +863,142 @@ __global__ void __launch_bounds__(kPlanThreads)
             return s_cn[i];
         return as_global(cnorm)[i];
     };
-    const Threshold thr = select_in_block<kPlanThreads>([&](int i) { return sort_key(norm_of(i)); }, &s_head, s_h);
+    const Threshold thr = select_in_block<kPlanThreads>(
+        [&](auto f) {
+            if (staged) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i)
+                    if (tid + i * kPlanThreads < n_cols)
+                        f(sort_key(v[i]));
+            } else {
+                for (int i = tid; i < (int)n_cols; i += kPlanThreads)
+                    f(sort_key(as_global(cnorm)[i]));
+            }
+        },
+        &s_head, s_h);
     if (tid == 0) {
         mail->thr_cols = thr.v64;
         if (thr.lost)
             mail->lost = 1;
     }
+    // sums over the threads up to this one (modulo 2^32: only differences are used), and over all
+    auto scan = [&](uint32_t mine, uint32_t &total) {
+        uint32_t incl = mine;
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t up = __shfl_up(incl, off);
+            incl += lane >= off ? up : 0u;
+        }
+        if (lane == 63)
+            s_sum[wave] = incl;
+        __syncthreads();
+        total = 0;
+#pragma unroll
+        for (int w = 0; w < kPlanThreads / 64; ++w) {
+            incl += w < wave ? s_sum[w] : 0u;
+            total += s_sum[w];
+        }
+        __syncthreads();
+        return incl;
+    };
     int64_t norm_carry = 0, item_carry = 0;
     for (int base = 0; base < n_layers; base += kPlanThreads) {
         const int cnt = min(kPlanThreads, n_layers - base);
-        for (int l = wave; l < cnt; l += kPlanThreads / 64) {
-            PruneLayer &L = layers[base + l];
-            const int64_t first = L.col_begin;
-            TW_GLOBAL(uint8_t) const colkeep = as_global(L.colkeep);
-            TW_GLOBAL(uint8_t) const colout = as_global(L.colout);
-            TW_GLOBAL(int32_t) const tcol0 = as_global(L.tcol0);
-            const int N = L.N, G = L.granularity;
-            int kept = 0;           // columns kept before this group of 64
-            int tile = 1, end = G;  // the next tile starts behind kept column number `end`
-            for (int c0 = 0; c0 < N; c0 += 64) {
-                const int c = c0 + lane;
-                const float v = c < N ? norm_of(first + c) : 0.0f;
-                const bool keep = c < N && thr.passed_by(v);
-                const unsigned long long b = __ballot(keep);
-                const int mine = kept + __popcll(b & ((2ull << lane) - 1ull)); // kept columns up to this one
-                if (c < N) {
-                    colkeep[c] = keep ? 1 : 0;
-                    if (colout)
-                        colout[c] = keep ? 1 : 0;
-                }
-                kept += __popcll(b);
-                for (; end <= kept; end += G, ++tile)
-                    if (keep && mine == end && c + 1 < N)
-                        tcol0[tile] = c + 1;
-            }
-            if (lane == 0) {
-                // tiles that ended before the last column, and the one that takes the rest
-                const bool last_col_ends = kept > 0 && kept % G == 0 &&
-                                           thr.passed_by(norm_of(first + N - 1));
-                const int nt = kept / G - (last_col_ends ? 1 : 0) + 1;
-                tcol0[0] = 0;
-                tcol0[nt] = N;
-                L.n_tiles = nt;
-                s_norm[l] = (int64_t)L.K * nt;
-                s_item[l] = (int64_t)((L.K + kNormRows - 1) / kNormRows) * nt;
-            }
-        }
+        uint32_t n_groups;
+        s_first[tid + 1] = scan(tid < cnt ? ((uint32_t)layers[base + tid].N + 63u) / 64u : 0u, n_groups);
+        if (tid == 0)
+            s_first[0] = 0;
         __syncthreads();
+        uint32_t carry = 0; // kept columns of the groups before these
+        for (uint32_t g0 = 0; g0 < n_groups; g0 += kPlanGroups) {
+            const uint32_t ng = min((uint32_t)kPlanGroups, n_groups - g0);
+            // ---- which columns are kept: a run of groups a wave
+            const uint32_t run = (ng + kPlanThreads / 64 - 1) / (kPlanThreads / 64);
+            const uint32_t begin = g0 + wave * run, stop = min(begin + run, g0 + ng);
+            int l = 0;
+            for (int step = kPlanThreads / 2; step > 0 && begin < stop; step >>= 1) // the layer of its first group
+                l += l + step < cnt && s_first[l + step] <= begin ? step : 0;
+            for (uint32_t g = begin; g < stop; ++l) {
+                l = __builtin_amdgcn_readfirstlane(l);
+                const PruneLayer &L = layers[base + l];
+                const int64_t first = L.col_begin;
+                TW_GLOBAL(uint8_t) const colkeep = as_global(L.colkeep);
+                TW_GLOBAL(uint8_t) const colout = as_global(L.colout);
+                const int N = L.N;
+                const uint32_t l0 = s_first[l], l1 = min(s_first[l + 1], stop);
+                for (; g < l1; ++g) {
+                    const int c = (int)(g - l0) * 64 + lane;
+                    const float x = c < N ? norm_of(first + c) : 0.0f;
+                    const bool keep = c < N && thr.passed_by(x);
+                    const unsigned long long b = __ballot(keep);
+                    if (c < N) {
+                        colkeep[c] = keep ? 1 : 0;
+                        if (colout)
+                            colout[c] = keep ? 1 : 0;
+                    }
+                    if (lane == 0) {
+                        s_bits[g - g0] = b;
+                        s_layer[g - g0] = (uint16_t)l;
+                    }
+                }
+            }
+            __syncthreads();
+            // ---- kept columns before each group
+            uint32_t at[2], in[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                in[e] = (uint32_t)tid * 2 + e < ng ? (uint32_t)__popcll(s_bits[tid * 2 + e]) : 0u;
+            uint32_t all;
+            at[0] = carry + scan(in[0] + in[1], all) - in[0] - in[1];
+            at[1] = at[0] + in[0];
+            carry += all;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                if ((uint32_t)tid * 2 + e < ng) {
+                    const int gl = s_layer[tid * 2 + e];
+                    if (s_first[gl] == g0 + tid * 2 + e)
+                        s_start[gl] = at[e];
+                }
+            __syncthreads();
+            // ---- the tiles that end in each group
+#pragma unroll 1
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t g = g0 + tid * 2 + e;
+                if (g >= g0 + ng)
+                    break;
+                const int gl = s_layer[g - g0];
+                PruneLayer &L = layers[base + gl];
+                const int N = L.N, G = L.granularity, K = L.K;
+                TW_GLOBAL(int32_t) const tcol0 = as_global(L.tcol0);
+                const unsigned long long bits = s_bits[g - g0];
+                const int before = (int)(at[e] - s_start[gl]), here = (int)in[e];
+                int tile = before / G;
+                for (int64_t need = (int64_t)(tile + 1) * G - before; need <= here; need += G) {
+                    int pos = 0, n = (int)need; // the n-th kept column of the group
+#pragma unroll
+                    for (int half = 32; half > 0; half >>= 1) {
+                        const int low = __popcll(bits >> pos & ((1ull << half) - 1ull));
+                        pos += n > low ? half : 0;
+                        n -= n > low ? low : 0;
+                    }
+                    ++tile;
+                    const int c = (int)(g - s_first[gl]) * 64 + pos;
+                    if (c + 1 < N)
+                        tcol0[tile] = c + 1;
+                }
+                if (g + 1 == s_first[gl + 1]) {
+                    // tiles that ended before the last column, and the one that takes the rest
+                    const int kept = before + here;
+                    const bool last_col_ends = kept > 0 && kept % G == 0 && (bits >> ((N - 1) & 63) & 1ull);
+                    const int nt = kept / G - (last_col_ends ? 1 : 0) + 1;
+                    tcol0[0] = 0;
+                    tcol0[nt] = N;
+                    L.n_tiles = nt;
+                    s_norm[gl] = (int64_t)K * nt;
+                    s_item[gl] = (int64_t)((K + kNormRows - 1) / kNormRows) * nt;
+                }
+            }
+            __syncthreads();
+        }
         const int64_t my_norm = tid < cnt ? s_norm[tid] : 0, my_item = tid < cnt ? s_item[tid] : 0;
         for (int off = 1; off < cnt; off <<= 1) { // inclusive sums over the layers
             const int64_t a = tid >= off && tid < cnt ? s_norm[tid - off] : 0;
@@ -1426,8 +1528,11 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
     const double f = (double)st->head.rank0 / (double)st->head.n;
     const double mid = f * kMixSamples, dev = 5.0 * sqrt((double)kMixSamples * f * (1.0 - f)) + 2.0;
     const double want[2] = {mid - dev, mid + dev};
-    auto key_of = [&](int i) { return s_key[i]; };
-    const KeyRange range = key_range_in_block<kBracketThreads>(key_of, kMixSamples); // (its barrier: s_key is whole)
+    const KeyRange range = key_range_in_block([&](auto f) { // (its barrier: s_key is whole)
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+            f(key[i]);
+    });
     // both edges out of one count of the first digit and one of the second, with counters for each: an edge is a chain of trips
     // through LDS and barriers, which is all that this kernel waits for (one edge after the other: 14.6 us, so 11)
     __shared__ unsigned int s_h2[kSelBins];
