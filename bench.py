@@ -32,10 +32,10 @@ MFMA_PEAK_TFLOPS = 2500.0   # MI355X dense fp16 / bf16
 PREWARM_SECONDS = 0.03  # untimed launches before a configuration's warm-up steps (clock ramp-up)
 
 MEASURED_TRAFFIC = {
-    "vgg16_conv4_2_im2col": ((2 * 62014 + 11282) * 1024, "profiles/tw_gemm_ws_kernel__vgg16_conv4_2.md (tw_gemm_ws_kernel 256x128)"),
+    "vgg16_conv4_2_im2col": ((2 * 46243 + 11282) * 1024, "profiles/tw_gemm_ws_kernel__vgg16_conv4_2.md (tw_gemm_ws_kernel 256x128)"),
     "bert_base_ffn_in": ((2 * 7880 + 24576) * 1024, "profiles/tw_gemm_bw_kernel__bert_large_ffn1_75.md (tw_gemm_bw_kernel)"),
     "nmt_lstm_gates": ((2 * 3558.5 + 1024) * 1024, "profiles/tw_gemm_skinny_kernel__nmt_lstm_gates.md (tw_gemm_skinny_kernel)"),
-    "imbalance_stress": ((2 * 922921 + 209150) * 1024, "profiles/tw_gemm_ws_kernel__imbalance_stress.md (tw_gemm_ws_kernel 256x64)"),
+    "imbalance_stress": ((2 * 754156 + 209152) * 1024, "profiles/tw_gemm_ws_kernel__imbalance_stress.md (tw_gemm_ws_kernel 256x64)"),
     "bert_large_ffn1_keep50": ((2 * 25220 + 65570) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn1_50.md (tw_gemm_ws_kernel 256x128)"),
     "bert_large_ffn2_keep10": ((2 * 22280 + 16400) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn2.md (tw_gemm_ws_kernel 256x128)"),
     "bert_large_ffn2_keep50": ((2 * 49480 + 16400) * 1024, "profiles/tw_gemm_ws_kernel__bert_large_ffn2.md (tw_gemm_ws_kernel 256x128)"),
