@@ -211,8 +211,8 @@ int tw_plan_destroy(tw_plan *plan);
 
 /* Gives back to the device all memory that no plan and no call holds, for a host program that needs
  * it elsewhere.  Waits for what is queued on the memory of destroyed plans.  May be called at any time, by any
- * thread, beside calls of other threads; the next builds and producer calls allocate anew.  No
- * counterpart in the reference. */
+ * thread, beside calls of other threads and in a tw_masks_ready; the next builds and producer calls allocate anew.
+ * What a running producer call holds is given back when that call ends.  No counterpart in the reference. */
 int tw_release_memory(void);
 
 /* ---- the GEMM ------------------------------------------------------------------ */
@@ -529,8 +529,9 @@ int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N,
 
 /* The three with masks that the caller allocates while the first kernels run: `ready(user)` is called once,
  * on the calling thread, when those are queued, and has put the masks' addresses into `masks` when it
- * returns 0; any other value ends the call with TW_ERR_ALLOC.  It calls no producer itself.  ready ==
- * NULL: as above. */
+ * returns 0; any other value ends the call with TW_ERR_ALLOC.  It may call this library, and may wait for
+ * other threads that do: no call waits for one that is in its `ready`.  The current device is as before when
+ * it returns.  ready == NULL: as above. */
 typedef int (*tw_masks_ready)(void *user);
 int tw_prune_tiled_wise_1d_late(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores,
                                 double sparsity, int q_type, int granularity, uint8_t *const *masks,

@@ -293,6 +293,78 @@ def test_masks_that_cannot_be_made_end_the_call(tw, twprune, monkeypatch, fn):
     assert all(np.array_equal(a, b) for a, b in zip(want, getattr(twprune, fn)(scores, 50, 32)))
 
 
+@pytest.mark.parametrize("fn", ["tiled_wise_1d", "tiled_wise_2d", "tiled_wise_1d_mix"])
+@pytest.mark.parametrize("n_layers", [3, 129])
+def test_nothing_waits_for_a_call_that_makes_its_masks(tw, twprune, po, monkeypatch, fn, n_layers):
+    """While the masks are made, the library gives back its memory, another thread's producer call comes to an end,
+    and so do one of this thread and, within that, one more (more calls than there are kept buffers for): every
+    call's masks are the oracle's, and so are those of the next ones."""
+    import threading
+    rng = np.random.default_rng(n_layers)
+    scores = [rng.random((int(rng.integers(3, 90)), int(rng.integers(16, 200)))).astype(np.float32) for _ in range(n_layers)]
+    want = getattr(po, fn)(scores, 60, 16)
+    want = want[0] if fn != "tiled_wise_1d_mix" else want
+    make, depth, results = twprune._DeviceLayers.make_masks, threading.local(), []
+
+    def call():
+        results.append(getattr(twprune, fn)(scores, 60, 16))
+
+    def busy(self):
+        at = getattr(depth, "at", 0)
+        depth.at = at + 1
+        print("masks", fn, n_layers, "call", at, flush=True)
+        tw.release_memory()
+        if at == 0:
+            other = threading.Thread(target=plain)
+            other.start()
+            other.join(60)
+            assert not other.is_alive()
+        if at < 2:
+            call()
+        tw.release_memory()
+        depth.at = at
+        return make(self)
+
+    def plain():
+        depth.at = 2  # (its masks are made without further calls)
+        call()
+    with monkeypatch.context() as m:
+        m.setattr(twprune._DeviceLayers, "make_masks", busy)
+        call()
+    call()
+    call()
+    assert len(results) == 6
+    for got in results:
+        assert all(np.array_equal(a, b) for a, b in zip(want, got))
+
+
+@pytest.mark.parametrize("fn", ["tiled_wise_1d", "tiled_wise_2d", "tiled_wise_1d_mix"])
+def test_calls_of_several_threads(tw, twprune, po, fn):
+    """Threads in producer calls side by side, the library's memory given back now and then."""
+    import threading
+    rng = np.random.default_rng(8)
+    jobs = [[rng.random((int(rng.integers(3, 300)), int(rng.integers(16, 400)))).astype(np.float32) for _ in range(n)] for n in (1, 3, 2, 5)]
+    wants = [getattr(po, fn)(s, 60, 16) for s in jobs]
+    wants = [w if fn == "tiled_wise_1d_mix" else w[0] for w in wants]
+    wrong = []
+
+    def work(i):
+        try:
+            for r in range(20):
+                got = getattr(twprune, fn)(jobs[i], 60, 16)
+                assert all(np.array_equal(a, b) for a, b in zip(wants[i], got))
+                if r % 7 == i:
+                    tw.release_memory()
+        except BaseException as e:
+            wrong.append((i, e))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(90)
+    assert not wrong and not any(t.is_alive() for t in threads)
+
+
 @pytest.mark.parametrize("shapes", [[(8448, 4096)], [(4224, 8192), (33, 4)], [(8448, 4099)]])
 def test_scores_beyond_the_caches(twprune, shapes):
     """More than 128 MB of scores are read past the caches, by either kernel of the row norms: the same masks

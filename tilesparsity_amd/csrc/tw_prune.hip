@@ -20,7 +20,9 @@
 #include "tw_device.h"
 
 #include <cmath>
+#include <condition_variable>
 #include <cstring>
+#include <iterator>
 #include <mutex>
 
 #pragma clang fp contract(off)
@@ -1876,28 +1878,60 @@ __global__ void __launch_bounds__(256)
 
 namespace {
 
-// Temporaries of one producer call come from a process-wide device buffer that grows (until
+// Temporaries of one producer call come from a device buffer that is kept and grows (until
 // tw_release_memory gives it back), so that a steady stream of calls does not pay for hipMalloc / hipFree,
-// and its thresholds come back through a page of pinned host memory that its last kernel writes.  The arena
-// holds the lock of both for the duration of the call (producer calls are serialised).
-std::mutex g_ws_mutex;
-void *g_ws = nullptr;
-size_t g_ws_size = 0;
-int g_ws_device = -1; // the device the buffer lives on; calls on another device do not use it
-Mail *g_mail = nullptr;
+// and its thresholds come back through a page of pinned host memory that its last kernel writes.  A call holds
+// both for its duration, and one that finds them held waits (producer calls are serialised) - but never for a
+// call that is in its caller's `ready`: that code may itself wait for this call (a lock of an interpreter), make
+// a producer call or give memory back.  The second set is for a call that comes by then.
+struct Kept {
+    void *ws = nullptr;
+    size_t size = 0;
+    int device = -1; // the device the buffer lives on; calls on another device do not use it
+    Mail *mail = nullptr;
+    bool held = false;
+    bool away = false; // held by a call that is in its caller's `ready`
+    bool drop = false; // given back by tw_release_memory while it was held: freed when the call ends
+
+    void give_back()
+    {
+        if (ws && hipFree(ws) != hipSuccess)
+            (void)hipGetLastError();
+        ws = nullptr;
+        size = 0;
+        device = -1; // the device of the next call
+    }
+};
+std::mutex g_kept_mutex; // (held for a look at `g_kept` only)
+std::condition_variable g_kept_free;
+Kept g_kept[2];
 
 class Arena {
 public:
     // `s`: the stream the call queues its kernels on; the buffer is not handed to the next call
     // before that stream has run dry, whichever way the call ends (an error return after kernels
     // were queued included).
-    explicit Arena(hipStream_t s) : lock_(g_ws_mutex), stream_(s)
+    explicit Arena(hipStream_t s) : stream_(s)
     {
         if (hipGetDevice(&device_) != hipSuccess)
             device_ = -2;
-        if (g_ws_device < 0)
-            g_ws_device = device_;
-        usable_ = device_ == g_ws_device;
+        std::unique_lock<std::mutex> lock(g_kept_mutex);
+        for (;;) {
+            Kept *k = g_kept, *const end = std::end(g_kept);
+            while (k != end && k->held && k->away)
+                ++k;
+            if (k == end) // (a producer in the `ready` of one in the `ready` of another: memory of its own)
+                break;
+            if (!k->held) {
+                kept_ = k;
+                break;
+            }
+            g_kept_free.wait(lock);
+        }
+        kept_->held = true;
+        if (kept_->device < 0)
+            kept_->device = device_;
+        usable_ = device_ == kept_->device;
     }
     ~Arena()
     {
@@ -1905,25 +1939,62 @@ public:
             (void)hipStreamSynchronize(stream_);
         for (void *p : extras_)
             (void)hipFree(p);
-        if (usable_ && need_ > g_ws_size) { // grow for the next call
-            (void)hipFree(g_ws);
-            g_ws = nullptr;
-            g_ws_size = 0;
+        if (kept_ == &own_) {
+            if (own_.mail)
+                (void)hipHostFree(own_.mail);
+            return;
+        }
+        std::unique_lock<std::mutex> lock(g_kept_mutex);
+        if (!kept_->drop && usable_ && need_ > kept_->size) { // grow for the next call
+            lock.unlock();
+            (void)hipFree(kept_->ws);
+            kept_->ws = nullptr;
+            kept_->size = 0;
             const size_t want = need_ + need_ / 2;
-            if (hipMalloc(&g_ws, want) == hipSuccess) {
-                g_ws_size = want;
+            if (hipMalloc(&kept_->ws, want) == hipSuccess) {
+                kept_->size = want;
             } else {
                 (void)hipGetLastError();
-                g_ws = nullptr;
+                kept_->ws = nullptr;
             }
+            lock.lock();
         }
+        if (kept_->drop)
+            kept_->give_back();
+        kept_->held = kept_->drop = false;
+        lock.unlock();
+        g_kept_free.notify_all();
     }
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    // while code of the caller's runs: nobody waits for this call
+    class Away {
+    public:
+        explicit Away(Arena *a) : kept_(a ? a->kept_ : nullptr) { set(true); }
+        ~Away() { set(false); }
+        Away(const Away &) = delete;
+        Away &operator=(const Away &) = delete;
+
+    private:
+        void set(bool away)
+        {
+            if (!kept_)
+                return;
+            {
+                std::lock_guard<std::mutex> lock(g_kept_mutex);
+                kept_->away = away;
+            }
+            if (away)
+                g_kept_free.notify_all();
+        }
+        Kept *const kept_;
+    };
     void *alloc(size_t bytes)
     {
         bytes = (bytes + 255) / 256 * 256;
         need_ += bytes;
-        if (usable_ && off_ + bytes <= g_ws_size) {
-            void *p = static_cast<char *>(g_ws) + off_;
+        if (usable_ && off_ + bytes <= kept_->size) {
+            void *p = static_cast<char *>(kept_->ws) + off_;
             off_ += bytes;
             return p;
         }
@@ -1939,11 +2010,11 @@ public:
     // the pinned page for this call, or nullptr
     Mail *mail()
     {
-        if (!g_mail && hipHostMalloc((void **)&g_mail, 4096, hipHostMallocPortable) != hipSuccess) {
+        if (!kept_->mail && hipHostMalloc((void **)&kept_->mail, 4096, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
-            g_mail = nullptr;
+            kept_->mail = nullptr;
         }
-        mail_ = g_mail;
+        mail_ = kept_->mail;
         if (mail_)
             mail_->lost = 0;
         return mail_;
@@ -1959,8 +2030,8 @@ public:
     }
 
 private:
-    std::lock_guard<std::mutex> lock_;
     hipStream_t stream_;
+    Kept own_, *kept_ = &own_;
     int device_ = -1;
     bool usable_ = false, idle_ = false;
     Mail *mail_ = nullptr;
@@ -2018,11 +2089,14 @@ struct Masks {
     tw_masks_ready ready = nullptr;
     void *user = nullptr;
 
-    // asks for them and checks them
-    int get(int n_layers)
+    // asks for them and checks them; `ar`: what the call holds
+    int get(int n_layers, Arena *ar)
     {
-        if (ready && ready(user))
-            return fail(TW_ERR_ALLOC, "the caller has no masks");
+        if (ready) {
+            const Arena::Away away(ar);
+            if (ready(user))
+                return fail(TW_ERR_ALLOC, "the caller has no masks");
+        }
         ready = nullptr;
         for (int l = 0; l < n_layers; ++l)
             if (!m[l])
@@ -2110,16 +2184,16 @@ int early_masks(CallTable &c, Masks &masks)
     const int n_layers = (int)c.layers.size();
     if (n_layers <= kLateMasks)
         return TW_OK;
-    const int st = masks.get(n_layers);
+    const int st = masks.get(n_layers, nullptr);
     for (int l = 0; !st && l < n_layers; ++l)
         c.layers[l].mask = masks.m[l];
     return st;
 }
-int queue_fill(const CallTable &c, Masks &masks, const PruneLayer *d_table, const SelectState *d_st, const Threshold *d_tile_thr, Mail *mail,
+int queue_fill(const CallTable &c, Masks &masks, Arena &ar, const PruneLayer *d_table, const SelectState *d_st, const Threshold *d_tile_thr, Mail *mail,
                hipStream_t s)
 {
     const int n_layers = (int)c.layers.size();
-    const int st = masks.get(n_layers);
+    const int st = masks.get(n_layers, &ar);
     if (st)
         return st;
     MaskTable m;
@@ -2182,7 +2256,7 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
         if (per_tile)
             hipLaunchKernelGGL(select_finish_kernel, dim3(n_seg), dim3(256), 0, s, d_st, d_tile_thr, mail);
     }
-    st = queue_fill(c, masks, d_table, d_st, d_tile_thr, mail, s);
+    st = queue_fill(c, masks, ar, d_table, d_st, d_tile_thr, mail, s);
     if (st)
         return st;
     st = ar.wait();
@@ -2291,12 +2365,13 @@ private:
 
 void release_producer_memory()
 {
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    if (g_ws && hipFree(g_ws) != hipSuccess)
-        (void)hipGetLastError();
-    g_ws = nullptr;
-    g_ws_size = 0;
-    g_ws_device = -1; // the device of the next call
+    std::lock_guard<std::mutex> lock(g_kept_mutex);
+    for (Kept &k : g_kept) {
+        if (k.held)
+            k.drop = true;
+        else
+            k.give_back();
+    }
 }
 
 } // namespace tw
@@ -2560,7 +2635,7 @@ try {
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
-    st = queue_fill(c, m, d_table, d_st, nullptr, mail, s);
+    st = queue_fill(c, m, ar, d_table, d_st, nullptr, mail, s);
     if (st)
         return st;
     st = ar.wait();
@@ -2623,7 +2698,7 @@ try {
         return fail(TW_ERR_LAYOUT, "q_type=%d, %d: unknown", q_type, g1_q_type);
     for (int l = 0; l < n_layers; ++l)
         if (N[l] > kMixMaxN || K[l] > kMixMaxK || (N[l] + (int64_t)granularity - 1) / granularity * K[l] > kMixMaxNorms) { // one stage after the other
-            st = m.get(n_layers);
+            st = m.get(n_layers, nullptr);
             if (!st)
                 st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, m, nullptr, (hipStream_t)stream, 0);
             return st ? st : tw_prune_mix(n_layers, K, N, scores, masks, g1percent, g1_q_type, masks, threshold, stream);
@@ -2661,7 +2736,7 @@ try {
     queue_norms(c, d_table, nullptr, false, s);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (!st)
-        st = m.get(n_layers);
+        st = m.get(n_layers, &ar);
     if (st)
         return st;
     mix.write_to(masks);
