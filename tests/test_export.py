@@ -185,3 +185,31 @@ def test_img2col_forward_shapes_and_sign():
     assert np.array_equal(out[0], po.img2col(conv)) and np.array_equal(out[1], np.abs(dense))
     # HWIO -> (H*W*I) x O keeps the output channel as the column
     assert np.array_equal(out[0][:, 3], np.abs(conv[..., 3]).ravel())
+
+
+def test_a_failed_producer_call_keeps_no_tensors():
+    """The scores and masks of a call whose masks could not be made go with its exception, not with the next
+    run of the garbage collector."""
+    import gc
+    import weakref
+    from tilesparsity_amd import twprune
+
+    class NoMasks(twprune._DeviceLayers):
+        def __init__(self):
+            self.error = None
+
+        def make_masks(self):
+            raise MemoryError("no masks")
+
+    def call():
+        d = NoMasks()
+        refs.append(weakref.ref(d))
+        d.check(twprune._masks_ready(d))
+    refs = []
+    gc.disable()
+    try:
+        with pytest.raises(MemoryError):
+            call()
+        assert refs[0]() is None
+    finally:
+        gc.enable()

@@ -77,8 +77,13 @@ class _DeviceLayers:
         return self
 
     def check(self, status):
-        if self.error is not None:
-            raise self.error
+        # (its traceback leads back to this object: kept here, or in this frame, it would keep the tensors)
+        error, self.error = self.error, None
+        try:
+            if error is not None:
+                raise error
+        finally:
+            del error
         tw._check(status)
 
     def _make_cols(self):
