@@ -365,9 +365,9 @@ def test_calls_of_several_threads(tw, twprune, po, fn):
     assert not wrong and not any(t.is_alive() for t in threads)
 
 
-@pytest.mark.parametrize("shapes", [[(8448, 4096)], [(4224, 8192), (33, 4)], [(8448, 4099)]])
+@pytest.mark.parametrize("shapes", [[(20992, 4096)], [(10496, 8192), (33, 4)], [(20992, 4099)]])
 def test_scores_beyond_the_caches(twprune, shapes):
-    """More than 128 MB of scores are read past the caches, by either kernel of the row norms: the same masks
+    """More than 320 MB of scores are read past the caches, by either kernel of the row norms: the same masks
     as from the norms and the percentile one at a time."""
     import torch
     gen = torch.Generator(device="cuda").manual_seed(5)

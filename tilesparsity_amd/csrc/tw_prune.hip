@@ -251,7 +251,7 @@ __global__ void __launch_bounds__(256, 6)
 }
 
 // The same where every tile of every layer is one block of the sum whose rows are made of whole pieces of 16 bytes
-// (queue_norms): the second item's rows are on their way while the first is added up (226 MB of BERT-base, read past the
+// (queue_norms): the second item's rows are on their way while the first is added up (226 MB of BERT-base read past the
 // caches: 37 us, 6.1 TB/s; four items 38, the kernel above 40; through the caches 43, 45 and 46).
 constexpr int kNormItems = 2; // of a workgroup, in a row
 template <bool ONCE>
@@ -2154,11 +2154,12 @@ CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const flo
 }
 
 // The row norms of all layers' tiles; n_items: tiles of kept columns, *n_items items of them.  `last`: the call does not read the
-// scores again.  Scores of more than half the memory-side cache (256 MB) are then read past it: they would not stay
-// there beside what comes next (226 MB of BERT-base: 43 -> 37 us; but where the call reads them again, or the next one
-// builds plans out of the same matrices, they have to stay: narrowing VGG16's 126 MB 42.5 -> 46.7 us, fourteen plans 93 ->
-// 111).
-constexpr int64_t kStayingBytes = 128 << 20;
+// scores again.  Scores that go far beyond the memory-side cache (256 MB) are then read past it: most of them would not stay there for
+// whoever comes next.  The line is where that next one, a build of the layers' plans out of the same matrices, no longer loses what the
+// masks gain (BERT-base layers, us with the loads through the caches and past them, masks and plans): 283 MB 146 + 1265 and 133 + 1282, 321 MB
+// 160 + 1433 and 143 + 1449, 340 MB 166 + 1520 and 148 + 1530, 377 MB 178 + 1705 and 158 + 1705.  Below it the plans lose more (226 MB 112 + 988 and
+// 113 + 1022), though masks of scores that were written just before gain from 208 MB on (226 MB 144 and 129).
+constexpr int64_t kStayingBytes = 320 << 20;
 void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n_items, bool last, hipStream_t s)
 {
     bool blocks = n_items == nullptr;
