@@ -365,6 +365,25 @@ def test_calls_of_several_threads(tw, twprune, po, fn):
     assert not wrong and not any(t.is_alive() for t in threads)
 
 
+def test_more_workgroups_than_a_launch_takes(tw, twprune):
+    """2^24 workgroups of 256 threads, which one launch does not run: row norms of as many items, and thresholds of as
+    many tiles."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    s = torch.rand((1 << 23, 64), generator=gen, device="cuda")  # 2^24 items of 32 rows of one column
+    mask = twprune.tiled_wise_1d([s], 75, 1, return_device=True)[0].bool()
+    assert s.masked_fill(~mask, 2.0).min() > s.masked_fill(mask, -1.0).max()
+    assert abs(int(mask.sum()) - (1 << 27)) < 1000  # (equal values: some 32 of each)
+    del s, mask
+    tw.release_memory()
+    s = np.random.default_rng(6).random((4, (1 << 24) + 3), dtype=np.float32)
+    half = 1 << 23
+    got = twprune.granularity_pruning(s, 40, 1)
+    for part in (slice(0, half), slice(half, 2 * half), slice(2 * half, None)):
+        assert np.array_equal(got[:, part], twprune.granularity_pruning(s[:, part], 40, 1))
+    tw.release_memory()
+
+
 @pytest.mark.parametrize("shapes", [[(20992, 4096)], [(10496, 8192), (33, 4)], [(20992, 4099)]])
 def test_scores_beyond_the_caches(twprune, shapes):
     """More than 320 MB of scores are read past the caches, by either kernel of the row norms: the same masks

@@ -183,15 +183,15 @@ constexpr int kNormRows = 32;     // rows of an item: eight lanes each
 constexpr int kNormPitch = 136;   // floats; a block of 128 columns with up to 3 before it
 template <bool ONCE>
 __global__ void __launch_bounds__(256, 6)
-    tile_row_norms_kernel(const PruneLayer *layers, int n_layers, const int64_t *n_items)
+    tile_row_norms_kernel(const PruneLayer *layers, int n_layers, const int64_t *n_items, int64_t first_item)
 {
     __shared__ __align__(16) float stage[kNormRows * kNormPitch];
     __shared__ float s_left[kNormRows][kPairDepth];
-    const int64_t item = blockIdx.x;
+    const int64_t item = first_item + blockIdx.x;
     if (n_items && item >= *n_items)
         return; // (a grid sized for the most tiles the layers can have)
     const PruneLayer L = layers[LayerFinder(&layers->rt_begin, sizeof(PruneLayer), n_layers)(item)];
-    const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a launch has fewer than 2^31 items)
+    const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a call has fewer than 2^31 items)
     const int rblk = (int)(idx / (uint32_t)L.n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)L.n_tiles);
     const int k0 = rblk * kNormRows, nr = min(kNormRows, L.K - k0);
     const int c0 = tile_begin(L, t), w = tile_begin(L, t + 1) - c0;
@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(256, 6)
 constexpr int kNormItems = 2; // of a workgroup, in a row
 template <bool ONCE>
 __global__ void __launch_bounds__(256, 5)
-    block_row_norms_kernel(const PruneLayer *layers, int n_layers, int64_t n_items)
+    block_row_norms_kernel(const PruneLayer *layers, int n_layers, int64_t n_items, int64_t first_wg)
 {
     __shared__ __align__(16) float stage[kNormRows * kNormPitch];
     const LayerFinder find(&layers->rt_begin, sizeof(PruneLayer), n_layers);
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(256, 5)
     auto fetch = [&](int64_t item, Item &d) {
         const PruneLayer &L = layers[find(item)];
         const int K = L.K, N = L.N, G = L.granularity, n_tiles = L.n_tiles;
-        const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a launch has fewer than 2^31 items)
+        const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a call has fewer than 2^31 items)
         const int rblk = (int)(idx / (uint32_t)n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)n_tiles);
         const int k0 = rblk * kNormRows, c0 = t * G;
         d.nr = min(kNormRows, K - k0);
@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(256, 5)
             d.out[grp] = d.divide ? sqrtf(s) / (float)d.w : sqrtf(s);
         TW_LDS_BARRIER(); // the stage is written again
     };
-    const int64_t first = (int64_t)blockIdx.x * kNormItems, last = n_items - 1;
+    const int64_t first = (first_wg + blockIdx.x) * kNormItems, last = n_items - 1;
     Item a, b;
     fetch(first, a);
     fetch(min(first + 1, last), b);
@@ -316,11 +316,11 @@ struct ColLayer {
 };
 constexpr int kColRows = 64, kColCols = 32, kColPitch = kColRows + 4, kColDeep = 8;
 constexpr int kColThreads = 320; // four waves that load, one that adds
-__global__ void __launch_bounds__(kColThreads) col_norms_kernel(const ColLayer *layers, int n_layers, float *cnorm)
+__global__ void __launch_bounds__(kColThreads) col_norms_kernel(const ColLayer *layers, int n_layers, float *cnorm, int64_t first_blk)
 {
     __shared__ __align__(16) float sq[2][kColCols * kColPitch];
-    const ColLayer L = layers[LayerFinder(&layers->blk_begin, sizeof(ColLayer), n_layers)(blockIdx.x)];
-    const int c0 = (int)((int64_t)blockIdx.x - L.blk_begin) * kColCols;
+    const ColLayer L = layers[LayerFinder(&layers->blk_begin, sizeof(ColLayer), n_layers)(first_blk + blockIdx.x)];
+    const int c0 = (int)(first_blk + blockIdx.x - L.blk_begin) * kColCols;
     const int tid = (int)threadIdx.x, col = tid & 31;
     const int K = L.K, N = L.N;
     const int n_grp = (K + kColRows * kColDeep - 1) / (kColRows * kColDeep) * kColDeep; // in whole rounds of kColDeep
@@ -787,12 +787,13 @@ __global__ void __launch_bounds__(256) select_finish_kernel(const SelectState *s
 // eight 63 against 145.  They remain for tiles of more than kTileSelect norms.
 constexpr int kTileSelect = 8192;
 template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(const float *norms, int K, double q, int q_is_f64,
-                                                                               Threshold *out, Mail *mail)
+                                                                               Threshold *out, Mail *mail, int64_t first_tile)
 {
     __shared__ unsigned int s_h[kSelBins];
     __shared__ SelectHead s_head;
     __shared__ float s_v[STAGE];
-    const float *const v = norms + (int64_t)blockIdx.x * K;
+    const int64_t tile = first_tile + blockIdx.x;
+    const float *const v = norms + tile * K;
     const int tid = (int)threadIdx.x;
     for (int i0 = tid; i0 < K; i0 += 256 * 4) { // four loads in flight
         float x[4];
@@ -814,7 +815,7 @@ template <int STAGE> __global__ void __launch_bounds__(256) tile_select_kernel(c
         },
         &s_head, s_h);
     if (tid == 0) {
-        out[blockIdx.x] = t;
+        out[tile] = t;
         if (t.lost)
             mail->lost = 1;
     }
@@ -2128,6 +2129,15 @@ struct CallTable {
     std::vector<PruneLayer> layers;
     int64_t n_norms = 0, n_items = 0, n_fill = 0, n_tcol = 0, n_cols = 0; // sums over the layers (upper bounds)
 };
+// A launch of 2^32 threads or more reports no error and runs nothing: as many launches as that asks for.
+// launch(first workgroup, workgroups)
+template <class F> void in_launches(int64_t workgroups, int threads, F launch)
+{
+    const int64_t most = kMaxGridThreads / threads;
+    for (int64_t first = 0; first < workgroups; first += most)
+        launch(first, dim3((unsigned)std::min(most, workgroups - first)));
+}
+
 CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, int granularity, int flags)
 {
     CallTable c;
@@ -2172,10 +2182,14 @@ void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n
     const int n_layers = (int)c.layers.size();
     if (blocks) {
         auto kernel = once ? block_row_norms_kernel<true> : block_row_norms_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)((c.n_items + kNormItems - 1) / kNormItems)), dim3(256), 0, s, d_table, n_layers, c.n_items);
+        in_launches((c.n_items + kNormItems - 1) / kNormItems, 256, [&](int64_t first, dim3 grid) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, d_table, n_layers, c.n_items, first);
+        });
     } else {
         auto kernel = once ? tile_row_norms_kernel<true> : tile_row_norms_kernel<false>;
-        hipLaunchKernelGGL(kernel, dim3((unsigned)c.n_items), dim3(256), 0, s, d_table, n_layers, n_items);
+        in_launches(c.n_items, 256, [&](int64_t first, dim3 grid) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, d_table, n_layers, n_items, first);
+        });
     }
 }
 
@@ -2249,7 +2263,9 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
     // per-tile thresholds (one layer): every tile's K norms are one segment
     if (in_blocks) {
         auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
-        hipLaunchKernelGGL(kernel, dim3(n_seg), dim3(256), 0, s, d_norms, K[0], q, q_is_f64, d_tile_thr, mail);
+        in_launches(n_seg, 256, [&](int64_t first, dim3 grid) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, d_norms, K[0], q, q_is_f64, d_tile_thr, mail, first);
+        });
     } else {
         st = queue_select(d_norms, c.n_norms / n_seg, d_st, n_seg, s);
         if (st)
@@ -2464,7 +2480,9 @@ try {
         st = put_table(&e, sizeof(e), d_table, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(tile_row_norms_kernel<false>, dim3((unsigned)n_items), dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr);
+    in_launches(n_items, 256, [&](int64_t first, dim3 grid) {
+        hipLaunchKernelGGL(tile_row_norms_kernel<false>, grid, dim3(256), 0, s, d_table, 1, (const int64_t *)nullptr, first);
+    });
     TW_HIP(hipGetLastError());
     return ar.wait();
 }
@@ -2485,7 +2503,9 @@ try {
     const int st = put_table(&cl, sizeof(cl), d_cl, setup_of(nullptr, 0, 0, 0.0, 0), SetupSelect{}, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(col_norms_kernel, dim3((N + kColCols - 1) / kColCols), dim3(kColThreads), 0, s, d_cl, 1, norms);
+    in_launches(((int64_t)N + kColCols - 1) / kColCols, kColThreads, [&](int64_t first, dim3 grid) {
+        hipLaunchKernelGGL(col_norms_kernel, grid, dim3(kColThreads), 0, s, d_cl, 1, norms, first);
+    });
     TW_HIP(hipGetLastError());
     return ar.wait();
 }
@@ -2629,7 +2649,9 @@ try {
     st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, 0, q, q_type), SetupSelect{}, s);
     if (st)
         return st;
-    hipLaunchKernelGGL(col_norms_kernel, dim3((unsigned)n_blk), dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm);
+    in_launches(n_blk, kColThreads, [&](int64_t first, dim3 grid) {
+        hipLaunchKernelGGL(col_norms_kernel, grid, dim3(kColThreads), 0, s, d_cl, n_layers, d_cnorm, first);
+    });
     hipLaunchKernelGGL(plan_2d_kernel, dim3(1), dim3(kPlanThreads), 0, s, d_table, n_layers, d_cnorm, c.n_cols, d_norms,
                        d_st, d_items, q, q_type, mail);
     queue_norms(c, d_table, d_items, false, s);
