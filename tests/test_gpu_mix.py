@@ -355,3 +355,23 @@ def test_1d_mix_in_one_call(twprune, po, granularity, values):
         for a, b in zip(want, got):
             assert np.array_equal(np.asarray(a, bool), b.cpu().numpy().astype(bool)), (sp, g1, a.shape)
             assert b.max() <= 1
+
+
+@pytest.mark.parametrize("K,N,granularity", [(5, 1 << 21, 128), (5, 1 << 21, 3), (4, (1 << 21) - 1, 3), (4, (1 << 21) - 2, 3),
+                                             (3, (1 << 21) + 8, 128), (1 << 23, 4, 4), (1 << 23, 3, 2), ((1 << 23) + 1, 4, 4),
+                                             (1 << 23, 64, 1)])
+def test_1d_mix_at_its_limits(tw, twprune, K, N, granularity):
+    """The widest and the tallest layer whose elements are placed in rows and tiles by a multiplication in float and by
+    24-bit products, the most norms, and the first layers beyond, where one stage follows the other with the masks as
+    input and output: the masks of the two calls, whose kernels divide."""
+    import torch
+    gen = torch.Generator(device="cuda").manual_seed(K + N)
+    scores = [torch.rand((K, N), generator=gen, device="cuda"), torch.rand((64, 100), generator=gen, device="cuda")]
+    for sp, g1 in ((75, 5), (40, 0.5)):
+        want = twprune.tw_mix_fn(scores, g1, twprune.tiled_wise_1d(scores, sp + g1, granularity, return_device=True), return_device=True)
+        threshold = twprune.tw_mix_fn.last_threshold
+        got = twprune.tiled_wise_1d_mix(scores, sp, granularity, g1, return_device=True)
+        assert twprune.tw_mix_fn.last_threshold == threshold
+        assert all(torch.equal(a, b) for a, b in zip(want, got)), (sp, g1)
+        del want, got
+    tw.release_memory()

@@ -2227,9 +2227,9 @@ int too_large(int64_t workgroups)
 }
 
 // tiles of `granularity` columns: norms of all layers into one pooled vector, one threshold (or, with
-// kPerTileThreshold, one per tile of the only layer), masks.  *threshold receives it.
+// kPerTileThreshold, one per tile of the only layer), masks.  *threshold receives it.  `last`: nobody reads the scores right after.
 int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *const *scores, double q, int q_is_f64,
-                 int granularity, Masks masks, double *threshold, hipStream_t s, int flags)
+                 int granularity, Masks masks, double *threshold, hipStream_t s, int flags, bool last = true)
 {
     CallTable c = make_table(n_layers, K, N, scores, granularity, flags);
     const bool per_tile = (flags & kPerTileThreshold) != 0;
@@ -2259,7 +2259,7 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
                    setup_of(d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q, q_is_f64), SetupSelect{}, s);
     if (st)
         return st;
-    queue_norms(c, d_table, nullptr, true, s);
+    queue_norms(c, d_table, nullptr, last, s);
     // per-tile thresholds (one layer): every tile's K norms are one segment
     if (in_blocks) {
         auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
@@ -2723,7 +2723,7 @@ try {
         if (N[l] > kMixMaxN || K[l] > kMixMaxK || (N[l] + (int64_t)granularity - 1) / granularity * K[l] > kMixMaxNorms) { // one stage after the other
             st = m.get(n_layers, nullptr);
             if (!st)
-                st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, m, nullptr, (hipStream_t)stream, 0);
+                st = uniform_rows(n_layers, K, N, scores, sparsity, q_type, granularity, m, nullptr, (hipStream_t)stream, 0, false);
             return st ? st : tw_prune_mix(n_layers, K, N, scores, masks, g1percent, g1_q_type, masks, threshold, stream);
         }
     hipStream_t s = (hipStream_t)stream;
