@@ -316,8 +316,9 @@ int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda
  *   TW_OPT_SHAPE        one of the TW_SHAPE_* kernels below
  *   TW_OPT_WGS_PER_CU   workgroups launched per compute unit, 1..8
  *   TW_OPT_PIECE        columns of a tile handed out as one work item: 128, 64 or 32
- *   TW_OPT_XCD_QUEUES   1 and automatic: one work queue per accelerator die, each owning whole row
- *                       blocks of A (the workgroups of a die then share those rows in their L2);
+ *   TW_OPT_XCD_QUEUES   1 and automatic (unless TW_OPT_BALANCE is 1): one work queue per accelerator
+ *                       die, each owning whole row blocks of A (the workgroups of a die then share
+ *                       those rows in their L2);
  *                       0: the work items are dealt out over the dies in turn, tile after tile;
  *                       2: dealt out over the dies in turn, row block after row block (all tiles
  *                       of a row block before the next)
@@ -357,7 +358,7 @@ int tw_gemm_staged(const tw_plan *plan, const void *A, int a_layout, int64_t lda
 #define TW_N_SHAPES 14
 /* What a K-major launch of `plan` on M rows would run with, under the options in force:
  * choice[0] the TW_SHAPE_* kernel, [1] the columns of a unit piece, [2] workgroups per compute
- * unit, [3] 1 for one work queue per die.  (No counterpart in the reference, whose kernel is
+ * unit, [3] 1 for one work queue per die (of the kernels that have queues).  (No counterpart in the reference, whose kernel is
  * fixed at compile time, basic_nn.cu:250-259; benchmarks name the kernel they timed with it.) */
 int tw_gemm_choice(const tw_plan *plan, int M, int64_t lda, int64_t ldc, float beta, int32_t *choice);
 /* Name of the kernel tw_gemm_ex runs for these arguments, in any layout, under the options in force (a static string; NULL

@@ -1482,3 +1482,29 @@ def test_queues_of_the_dies_hand_out_every_item_once(tw, oracle, blocks, pruned)
     want = got[1, 0]
     assert (want[:, :M] != 0x1234).any(1).sum() >= (N if pruned == "zero" else 1)
     assert all(torch.equal(want, g) for g in got.values())
+
+
+def test_choice_names_queues_of_kernels_that_have_them(tw, oracle):
+    """choice()'s xcd_queues: only for a kernel that draws its items from queues, and as the options ask."""
+    rng = np.random.default_rng(9)
+    tiles = random_tiles(rng, 256, 512, 64, k_keep=0.3)
+    B = rng.standard_normal((256, 512)).astype(np.float32)
+    queued = {tw.SHAPE_WIDE, tw.SHAPE_128x128, tw.SHAPE_512x64, tw.SHAPE_128x64, tw.SHAPE_256x128, tw.SHAPE_128x32, tw.SHAPE_256x64}
+    seen = set()
+    try:
+        with tw.Plan.create(256, 512, "f16", tiles, B) as plan:
+            for shape in range(13):
+                tw.set_option(tw.OPT_SHAPE, shape)
+                for xcd in (-1, 0, 1, 2):
+                    tw.set_option(tw.OPT_XCD_QUEUES, xcd)
+                    c = plan.choice(4096)
+                    seen.add(c["shape"])
+                    assert c["xcd_queues"] == (c["shape"] in queued and xcd in (-1, 1)), (shape, xcd, c)
+                tw.set_option(tw.OPT_XCD_QUEUES, -1)
+                tw.set_option(tw.OPT_BALANCE, 1)
+                assert not plan.choice(4096)["xcd_queues"]
+                tw.set_option(tw.OPT_BALANCE, -1)
+    finally:
+        for opt in (tw.OPT_SHAPE, tw.OPT_XCD_QUEUES, tw.OPT_BALANCE):
+            tw.set_option(opt, -1)
+    assert len(seen & queued) >= 5 and len(seen - queued) >= 3

@@ -3417,7 +3417,7 @@ int tw_gemm_choice(const tw_plan *plan, int M, int64_t lda, int64_t ldc, float b
     choice[0] = c.shape;
     choice[1] = c.piece;
     choice[2] = c.per_cu;
-    choice[3] = c.xcd ? 1 : 0;
+    choice[3] = c.xcd && !is_queueless_shape(c.shape) ? 1 : 0;
     return TW_OK;
 }
 
