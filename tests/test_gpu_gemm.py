@@ -1444,44 +1444,62 @@ def test_row_major_operands_with_more_rows_than_a_grid_takes_threads(tw, beta):
     assert int((C != 1.5 + beta).sum(dtype=torch.int64)) == 3 * N
 
 
-@pytest.mark.parametrize("blocks", [7, 40, 43])
+@pytest.mark.parametrize("shape,G,blocks", [("128x32", 32, 7), ("128x32", 32, 40), ("128x32", 32, 43), ("256x64", 64, 43)])
 @pytest.mark.parametrize("pruned", ["untouched", "zero"])
-def test_queues_of_the_dies_hand_out_every_item_once(tw, oracle, blocks, pruned):
-    """Row blocks owned by the dies give bit for bit what items dealt out in turn give: fewer row blocks
+def test_queues_of_the_dies_hand_out_every_item_once(tw, oracle, shape, G, blocks, pruned):
+    """Row blocks owned by the dies, items dealt out tile after tile and row block after row block: fewer row blocks
     than dies (nobody owns one), five to a die in a group of two and one of three, the same with three
-    left over, each with one to a die's share of a launch and with twelve items and more to a workgroup,
-    tiles without kept rows and pruned columns to fill among them."""
+    left over, each with one to a die's share of a launch and with twelve items and more to a workgroup (the
+    256-row items only in fewer workgroups), tiles without kept rows and pruned columns to fill among them.  Every
+    launch starts from the same C and adds half of it, so that an item left out, or taken up again after it was
+    stored, differs from the oracle; nothing but the products' columns is written."""
     import torch
     rng = np.random.default_rng(5 + blocks)
-    K, N, G = 96, 2688, 32
+    K, N = 96, 2688
+    rows = int(shape.split("x")[0])
     tiles = random_tiles(rng, K, N, G, k_keep=0.4, n_keep=0.7, empty_every=20)
     B = (rng.standard_normal((K, N)) * 0.1).astype(np.float32)
-    code = tw.PRUNED_ZERO if pruned == "zero" else tw.PRUNED_UNTOUCHED
-    M = blocks * 128 - 5
+    M = blocks * rows - 5
     ld = round_up(M, 8)
-    dA = torch.from_numpy(oracle.cast_bits(rng.standard_normal((K, ld)).astype(np.float32), "f16").view(np.int16).reshape(K, ld)).cuda()
-    got = {}
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    C0 = rng.standard_normal((M, N)).astype(np.float32)
+    want = reference(oracle, A, B, tiles, "f16", beta=0.5, C0=C0).T
+    start = np.full((N, ld), SENTINEL, np.uint16)
+    start[:, :M] = oracle.cast_bits(C0, "f16").reshape(M, N).T
+    At = np.zeros((K, ld), np.uint16)
+    At[:, :M] = oracle.cast_bits(A, "f16").reshape(M, K).T
+    dA, dstart = to_device_bits(At, At.shape), to_device_bits(start, start.shape)
+    keep = kept_columns(tiles, N)
+    if pruned == "zero":
+        want[~keep] = 0.5 * oracle.quantize(C0, "f16").T[~keep]
+    got = []
     try:
         with tw.Plan.create(K, N, "f16", tiles, B) as plan:
-            tw.set_option(tw.OPT_SHAPE, tw.SHAPE_128x32)
+            tw.set_option(tw.OPT_SHAPE, getattr(tw, "SHAPE_" + shape))
             tw.set_option(tw.OPT_PIECE, 32)
             for per_cu in (1, 8):
                 tw.set_option(tw.OPT_WGS_PER_CU, per_cu)
-                for xcd in (0, 1, -1):
+                for xcd in (0, 1, 2, -1):
                     tw.set_option(tw.OPT_XCD_QUEUES, xcd)
-                    print("queues", blocks, pruned, per_cu, xcd, flush=True)
-                    dC = torch.full((N, ld), 0x1234, dtype=torch.int16, device="cuda")
+                    print("queues", shape, blocks, pruned, per_cu, xcd, flush=True)
                     for _ in range(2):  # (the second launch finds the counters as the first left them)
-                        plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=ld, ldc=ld, pruned_cols=code,
+                        dC = dstart.clone()
+                        plan.gemm(dA.data_ptr(), dC.data_ptr(), M, lda=ld, ldc=ld, beta=0.5,
+                                  pruned_cols=tw.PRUNED_ZERO if pruned == "zero" else tw.PRUNED_UNTOUCHED,
                                   stream=torch.cuda.current_stream().cuda_stream)
-                    torch.cuda.synchronize()
-                    got[per_cu, xcd] = dC.cpu()
+                        got.append(dC)
     finally:
         for opt in (tw.OPT_SHAPE, tw.OPT_PIECE, tw.OPT_WGS_PER_CU, tw.OPT_XCD_QUEUES):
             tw.set_option(opt, -1)
-    want = got[1, 0]
-    assert (want[:, :M] != 0x1234).any(1).sum() >= (N if pruned == "zero" else 1)
-    assert all(torch.equal(want, g) for g in got.values())
+    first = from_device_bits(got[0])
+    written = oracle.bits_to_f32(first[:, :M], "f16").reshape(N, M)
+    assert (first[:, M:] == SENTINEL).all()
+    if pruned == "untouched":
+        assert np.array_equal(first[~keep], start[~keep])
+        written, want = written[keep], want[keep]
+    # one rounding to 16 bits (2^-11 of the result), and 39 kept rows' products added in 32 bits
+    assert (np.abs(written - want) <= 2.0 ** -11 * np.abs(want) + 1e-5).all()
+    assert all(torch.equal(got[0], g) for g in got)
 
 
 def test_choice_names_queues_of_kernels_that_have_them(tw, oracle):
