@@ -1,4 +1,5 @@
-"""GPU parity of the TW mask producers (tw_prune_tiled_wise_1d / _2d through the C ABI)
+"""GPU parity of the TW mask producers (twprune, whose calls are tw_prune_tiled_wise_1d_late and its
+kin; the entry points that take masks from the start in test_entry_points_with_masks_from_the_start)
 against the CPU oracle and the golden vectors of the reference's prune_algo.py.
 
 Masks are integer results: the bar is bit-exact.  The oracle computes with NumPy itself
@@ -363,6 +364,49 @@ def test_calls_of_several_threads(tw, twprune, po, fn):
     for t in threads:
         t.join(90)
     assert not wrong and not any(t.is_alive() for t in threads)
+
+
+@pytest.mark.parametrize("n_layers", [3, 129])
+def test_entry_points_with_masks_from_the_start(tw, twprune, n_layers):
+    """tw_prune_tiled_wise_1d, _2d and _1d_mix as a C program calls them: the masks and thresholds of the calls that
+    ask for their masks; a mask that is NULL, there or when it has been asked for, and a `ready` that has none
+    are errors, and the next call is as ever."""
+    import ctypes
+    import torch
+    rng = np.random.default_rng(n_layers)
+    scores = [torch.from_numpy(rng.random((int(rng.integers(3, 60)), int(rng.integers(16, 70)))).astype(np.float32)).cuda()
+              for _ in range(n_layers)]
+    L, pp, i32 = tw.lib(), ctypes.POINTER(ctypes.c_void_p), ctypes.c_int32
+    d = twprune._DeviceLayers(scores).make_masks()
+    head = (n_layers, tw._ptr(d.K, i32), tw._ptr(d.N, i32), ctypes.cast(d.p_scores, pp))
+    masks, thr, thr2 = ctypes.cast(d.p_masks, pp), ctypes.c_double(), (ctypes.c_double * 2)()
+    never = tw.MASKS_READY(lambda d: 7)
+    nothing = tw.MASKS_READY(lambda d: 0)
+    calls = {  # entry point: its arguments, how they go on behind the masks, and how those of the _late form do
+        "tiled_wise_1d": ((60.0, 0, 16), lambda ready: (masks, *ready, ctypes.byref(thr), d.stream)),
+        "tiled_wise_2d": ((60.0, 0, 1, 16), lambda ready: (masks, *ready, None, thr2, d.stream)),
+        "tiled_wise_1d_mix": ((65.0, 0, 16, 5.0, 0), lambda ready: (masks, *ready, ctypes.byref(thr), d.stream)),
+    }
+    for name, (args, rest) in calls.items():
+        print("entry point", name, n_layers, flush=True)
+        plain, late = getattr(L, "tw_prune_" + name), getattr(L, "tw_prune_" + name + "_late")
+        want = getattr(twprune, name)(scores, 60, 16, return_device=True)
+        for m in d.d_masks:
+            m.fill_(9)
+        assert plain(*head, *args, *rest(())) == 0
+        assert all(torch.equal(a, b) for a, b in zip(want, d.d_masks))
+        last = {"tiled_wise_1d": lambda: twprune.tiled_wise_1d.last_threshold, "tiled_wise_1d_mix": lambda: twprune.tw_mix_fn.last_threshold,
+                "tiled_wise_2d": lambda: twprune.tiled_wise_2d.last_thresholds}[name]()
+        assert last == (tuple(thr2) if name == "tiled_wise_2d" else thr.value)
+        kept, d.p_masks[n_layers - 1] = d.p_masks[n_layers - 1], None
+        assert plain(*head, *args, *rest(())) == tw.ERR_NULL
+        assert late(*head, *args, *rest((nothing, None))) == tw.ERR_NULL
+        d.p_masks[n_layers - 1] = kept
+        assert late(*head, *args, *rest((never, None))) == tw.ERR_ALLOC
+        for m in d.d_masks:
+            m.fill_(9)
+        assert plain(*head, *args, *rest(())) == 0
+        assert all(torch.equal(a, b) for a, b in zip(want, d.d_masks))
 
 
 def test_more_workgroups_than_a_launch_takes(tw, twprune):
