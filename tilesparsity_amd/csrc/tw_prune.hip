@@ -1519,19 +1519,15 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
 {
     constexpr int PER = kMixSamples / kBracketThreads;
     __shared__ unsigned int s_h[kSelBins];
-    __shared__ uint32_t s_key[kMixSamples];
     const int tid = (int)threadIdx.x;
     uint32_t key[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i)
         key[i] = sample[tid + i * kBracketThreads];
-#pragma unroll
-    for (int i = 0; i < PER; ++i)
-        s_key[tid + i * kBracketThreads] = key[i];
     const double f = (double)st->head.rank0 / (double)st->head.n;
     const double mid = f * kMixSamples, dev = 5.0 * sqrt((double)kMixSamples * f * (1.0 - f)) + 2.0;
     const double want[2] = {mid - dev, mid + dev};
-    const KeyRange range = key_range_in_block([&](auto f) { // (its barrier: s_key is whole)
+    const KeyRange range = key_range_in_block([&](auto f) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             f(key[i]);
