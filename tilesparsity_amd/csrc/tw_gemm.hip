@@ -25,6 +25,7 @@
 //   * epilogue: alpha/beta in fp32, round to the 16-bit type, transpose through
 //     LDS, then scatter whole C columns (col0 + kept_n[j]) with 16-byte stores.
 #include "tw_device.h"
+#include "tw_queue.h"
 
 #include <algorithm>
 #include <atomic>
@@ -35,104 +36,6 @@
 #include <cstdlib>
 
 namespace tw {
-
-// ---------------------------------------------------------------------------------
-// Work queue (see GemmArgs): entry q of queue x names one item, or nothing past the end.
-enum ItemKind { ITEM_PIPE = 0, ITEM_NOSTEP = 1, ITEM_ZERO = 2, ITEM_END = 3 };
-
-struct Work {
-    int kind; // ItemKind
-    int u;    // column of the item matrix: piece of a unit, or n_gemm_u + tile to fill
-    int m0;   // first row
-    int rows; // rows [m0, m0 + rows) of A and C, cut at M by the caller
-};
-
-// (queue x's share of the first `n` of the items that are dealt out over the queues in turn)
-__device__ __forceinline__ int dealt_to(int n, int x)
-{
-    return (n + kXcd - 1 - x) / kXcd;
-}
-
-// where column `u` starts in the part of queue x that is ordered column after column
-__device__ __forceinline__ int column_start(const GemmArgs &p, int x, int u)
-{
-    return u * p.n_last + dealt_to(u * p.n_tail_mblk, x);
-}
-
-__device__ __forceinline__ int queue_length(const GemmArgs &p, int x)
-{
-    if (p.n_list_items)
-        return dealt_to(p.n_list_items, x);
-    return p.n_lead_items + column_start(p, x, p.n_pipe_u) + dealt_to((p.n_all_u - p.n_pipe_u) * p.n_mblk, x);
-}
-
-// (bm: rows of a row block of this launch)
-__device__ __forceinline__ Work queue_entry(const GemmArgs &p, int x, int q, int bm)
-{
-    Work w;
-    w.kind = ITEM_END;
-    w.u = 0;
-    w.m0 = 0;
-    w.rows = bm;
-    if (p.n_list_items) {
-        const int j = q * kXcd + x;
-        if (j >= p.n_list_items)
-            return w;
-        if (p.n_bal > 0) {
-            // columns with row blocks of their own height: column u owns the items
-            // bal_first[u] .. bal_first[u + 1] - 1 of the list
-            int u = 0;
-#pragma unroll
-            for (int i = 1; i < kBalColumns; ++i)
-                u += i < p.n_bal && j >= p.bal_first[i];
-            w.u = u;
-            w.rows = p.bal_rows[u];
-            w.m0 = (j - p.bal_first[u]) * w.rows;
-        } else {
-            // all columns of a row block (heaviest first) before the next row block
-            const int mb = j / p.n_all_u;
-            w.u = j - mb * p.n_all_u;
-            w.m0 = mb * bm;
-        }
-    } else if (q < p.n_lead_items) {
-        const int per = p.n_grp * p.n_pipe_u, g = q / per, r = q - g * per;
-        w.u = r / p.n_grp;
-        w.m0 = (x * p.n_own + g * p.n_grp + (r - w.u * p.n_grp)) * bm;
-    } else {
-        const int r = q - p.n_lead_items;
-        int end;
-        if (r < (end = column_start(p, x, p.n_pipe_u))) {
-            int u, off;
-            if (p.n_last > 0) { // (a column starts within one entry of its mean place)
-                u = r * kXcd / (p.n_last * kXcd + p.n_tail_mblk);
-                if (column_start(p, x, u) > r)
-                    --u;
-                else if (column_start(p, x, u + 1) <= r)
-                    ++u;
-                off = r - column_start(p, x, u);
-            } else {
-                u = (r * kXcd + x) / p.n_tail_mblk;
-                off = r - column_start(p, x, u);
-            }
-            w.u = u;
-            if (off < p.n_last) {
-                w.m0 = (x * p.n_own + p.n_own - p.n_last + off) * bm;
-            } else {
-                const int j = (dealt_to(u * p.n_tail_mblk, x) + off - p.n_last) * kXcd + x;
-                w.m0 = (kXcd * p.n_own + j - u * p.n_tail_mblk) * bm;
-            }
-        } else {
-            const int j = (r - end) * kXcd + x;
-            if (j >= (p.n_all_u - p.n_pipe_u) * p.n_mblk)
-                return w;
-            w.u = j / p.n_mblk;
-            w.m0 = (j - w.u * p.n_mblk) * bm;
-            w.u += p.n_pipe_u;
-        }
-    }
-    w.kind = w.u < p.n_pipe_u ? ITEM_PIPE : (w.u < p.n_gemm_u ? ITEM_NOSTEP : ITEM_ZERO);
-    return w;
-}
 
 // WM x WN waves of 64 x 64 outputs each: workgroup tile BM = 64*WM rows by BN = 64*WN
 // compact columns.  WGS is the number of workgroups meant to share a CU.
@@ -195,8 +98,8 @@ __global__ void __launch_bounds__(64 * WM * WN, (WM * WN * WGS) / 4)
     };
     auto make_item = [&](int ticket) {
         Item it;
-        const Work w = queue_entry(p, qx, ticket, BM);
-        it.col = w.kind == ITEM_END ? p.n_all_u : w.u;
+        const Work w = queue_entry(p, qx, ticket, qlen, BM);
+        it.col = w.col;
         it.m0 = w.m0;
         if (it.col < p.n_gemm_u)
             it.u = load_unit(p, it.col);
@@ -650,8 +553,8 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
     };
     auto place_item = [&](int ticket) { // (without its unit)
         Item it;
-        const Work w = queue_entry(p, qx, ticket, BM);
-        it.col = w.kind == ITEM_END ? p.n_all_u : w.u;
+        const Work w = queue_entry(p, qx, ticket, qlen, BM);
+        it.col = w.col;
         it.m0 = w.m0;
         it.m_end = it.m0 + w.rows < p.M ? it.m0 + w.rows : p.M;
         return it;
@@ -3097,14 +3000,15 @@ constexpr int64_t kMaxItems = 0x7fffffff;
 // workgroups.  `xcd`: every die owns an eighth of the row blocks, whatever is left over is dealt out in turn.
 // Dealt out all in turn, tile after tile, a row block's items meet on one die only where the row blocks are a
 // multiple of eight: a die then fetched most of A (VGG16 conv4_2, 49 row blocks: 126 MB instead of 95).  Over
-// 15000 random problems (M 300 .. 16384, K 512 .. 4608, N 256 .. 8192, 10 - 95 % of the rows kept) owned row
-// blocks take 0.96 of the time at half an item to one item a workgroup, 0.93 to two, 0.91 to three, 0.88 from
-// four to six, 0.83 from there on; 131 of them lose 3 % and more, four a tenth (to 1.19).
+// 8691 random problems (M 300 .. 16384, K 512 .. 4608, N 256 .. 8192, 10 - 95 % of the rows kept) owned row
+// blocks take 0.94 of the time at half an item to one item a workgroup, 0.92 to two, 0.88 to three, 0.84 from
+// three to six, 0.79 to twelve, 0.68 from there on, and lose 3 % in two of them.  (Where the row blocks are a multiple of
+// eight both are the same up to the groups: 1.01 of the time, and single timings from 0.98 to 1.12.)
 // Within a die the items go tile after tile, the longest first, so that a workgroup's last item is a short one:
 // row block after row block instead (the same rows for all workgroups of the die at a time) loses 10 % and more
 // in one problem of twenty between one and six items a workgroup (to 1.56).  Where there are twelve and more the
-// last items no longer count and two row blocks at a time are ahead of all at once: 0.80 of the time of dealt-out
-// items against 0.83 from twelve to eighteen, 0.78 against 0.81 above (load-imbalance stress, 29: 320 -> 293 us).
+// last items no longer count and two row blocks at a time are ahead of all at once: 0.98 of the time to fifteen, 0.97 to
+// eighteen, 0.95 above, three problems of 117 slower by 3 %; from four to six 1.00, to twelve 0.99, 22 of 383 slower (to 1.13).
 void fill_queues(GemmArgs &a, const tw_plan *plan, int M, int bm, int piece, int pruned_cols, bool xcd, int64_t wgs)
 {
     const int width = std::max(32, round_up32(plan->max_unit_n));
@@ -3114,14 +3018,7 @@ void fill_queues(GemmArgs &a, const tw_plan *plan, int M, int bm, int piece, int
     a.n_pipe_u = plan->n_pipe_units * a.n_split;
     a.n_gemm_u = plan->n_units * a.n_split;
     a.n_all_u = a.n_gemm_u + (pruned_cols == TW_PRUNED_ZERO ? plan->n_zero_tiles : 0);
-    a.n_own = xcd ? a.n_mblk / kXcd : 0;
-    a.n_grp = (int64_t)a.n_pipe_u * a.n_mblk >= 12 * wgs ? 2 : a.n_own;
-    a.n_grp = std::max(1, std::min(a.n_grp, a.n_own));
-    const int groups = std::max(1, a.n_own / a.n_grp);
-    a.n_last = a.n_own - (groups - 1) * a.n_grp;
-    a.n_lead_items = (groups - 1) * a.n_grp * a.n_pipe_u;
-    a.n_tail_mblk = a.n_mblk - kXcd * a.n_own;
-    a.n_list_items = 0;
+    lay_queues(a, xcd, wgs);
 }
 
 // Row blocks sized per column of the item matrix, for launches whose items do not fill the chip
@@ -3176,7 +3073,7 @@ bool balance_items(GemmArgs &a, const tw_plan *plan, int M, int bm, int64_t wgs)
     }
     for (int u = a.n_all_u; u <= kBalColumns; ++u)
         a.bal_first[u] = first;
-    a.n_list_items = first;
+    a.n_rest_items = first;
     return true;
 }
 
@@ -3201,9 +3098,7 @@ int launch_gemm(const tw_plan *plan, GemmArgs &a, const Choice &c, int32_t *tick
     if (c.shape == TW_SHAPE_BS || c.shape == TW_SHAPE_BS4 || c.shape == TW_SHAPE_BS8)
         return launch_bs(plan, a, option(TW_OPT_WGS_PER_CU), c.shape == TW_SHAPE_BS ? bs_wide(plan, a.M, a.C, a.ldc, a.act) : c.shape == TW_SHAPE_BS8, s);
     // queue 0 is the longest: one workgroup per entry, up to the chip's share of a queue
-    const int64_t qlen0 = a.n_list_items ? (a.n_list_items + kXcd - 1) / kXcd
-                                         : (int64_t)a.n_own * a.n_pipe_u + ((int64_t)a.n_tail_mblk * a.n_pipe_u + kXcd - 1) / kXcd +
-                                               ((int64_t)(a.n_all_u - a.n_pipe_u) * a.n_mblk + kXcd - 1) / kXcd;
+    const int64_t qlen0 = a.n_lead_items + ((int64_t)a.n_rest_items + kXcd - 1) / kXcd;
     const int64_t per_queue = std::max<int64_t>(1, (int64_t)plan->cu_count * c.per_cu / kXcd);
     const int grid = (int)(kXcd * std::min(qlen0, per_queue));
     if (plan->dtype == TW_F16)
@@ -3350,7 +3245,7 @@ int gemm_impl(const tw_plan *plan, const void *A, int a_layout, int64_t lda, voi
     const Choice c = choose_shape(plan, M, lda, ldc, beta != 0.0f);
     fill_queues(a, plan, M, kShapes[c.shape].bm, c.piece, pruned_cols, c.xcd, (int64_t)plan->cu_count * c.per_cu);
     if (option(TW_OPT_XCD_QUEUES) == 2)
-        a.n_list_items = (int)std::min<int64_t>((int64_t)a.n_all_u * a.n_mblk, kMaxItems);
+        order_by_row_blocks(a);
     // 256-row items whose loads write LDS directly (measured faster on every shape tried, with
     // one item per workgroup and with several)
     if ((c.shape == TW_SHAPE_256x128 || c.shape == TW_SHAPE_256x64) && option(TW_OPT_LDS_DMA) != 0 && (uint64_t)plan->packed_elems * 2u < (1ull << 32)) {

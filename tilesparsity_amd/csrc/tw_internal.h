@@ -49,16 +49,7 @@ struct TileDev {
     int32_t pad_;
 };
 
-// The work of one launch is a matrix of items: `n_all_u` columns (pieces of units that have kept
-// K rows first, heaviest first; then pieces of units without; then, with TW_PRUNED_ZERO, the tiles
-// whose pruned columns are filled) by `n_mblk` blocks of BM rows.  It is handed out through
-// kXcd queues, one per accelerator die: workgroup b runs on die b % kXcd and draws from that
-// die's queue only, so the workgroups that share an L2 work on the same rows of A.  Queue x owns
-// the row blocks [x * n_own, (x + 1) * n_own): first, in groups of n_grp row blocks, column after
-// column of a group; then column after column over the n_last row blocks left of its own and every
-// kXcd-th item of the `n_tail_mblk` row blocks that nobody owns; then every kXcd-th item of the
-// columns without steps.
-constexpr int kXcd = 8;
+constexpr int kXcd = 8;         // accelerator dies: workgroup b runs on die b % kXcd
 constexpr int kTicketInts = 16; // per slot: [0, kXcd) next index of each queue, [kXcd] workgroups done
 
 // Threads of a grid's first dimension: a launch of more reports no error and runs nothing.
@@ -89,18 +80,19 @@ struct GemmArgs {
     int32_t n_gemm_u;     // + pieces of units without (their columns receive beta * C)
     int32_t n_all_u;      // + tiles with pruned columns to fill
     int32_t n_own;        // row blocks owned by each queue
-    int32_t n_grp;        // ... worked off in groups of so many, tile after tile within a group
-    int32_t n_last;       // ... of which the last group has so many
-    int32_t n_lead_items; // (n_own - n_last) * n_pipe_u
-    int32_t n_tail_mblk;  // n_mblk - kXcd * n_own
-    int32_t n_list_items; // > 0: one list of so many items is dealt out over the queues instead
+    int32_t n_last;       // ... of which so many come behind the groups
+    int32_t n_lead_items; // items of a queue's groups: (n_own - n_last) * n_pipe_u
+    int32_t n_col_mblk;   // entries of a column in the list behind them
+    int32_t n_col_items;  // ... of all columns with steps: n_pipe_u * n_col_mblk
+    int32_t n_rest_items; // ... and of the columns without
+    int32_t rb_major;     // the list goes row block after row block (n_own == 0, n_col_mblk == n_all_u)
     float alpha, beta;
     const float *bias;    // fp32 [N] added to every written column before the activation, or null
     int32_t act;          // TW_ACT_*
     int32_t store_through; // output stores write through to memory (large outputs) or stay in L2
     int32_t *ticket;      // kTicketInts counters, zero between launches
     // Row blocks sized per column of the item matrix (n_bal > 0: one list of items for all
-    // queues, n_own == 0, n_tail_items items): column u has items of bal_rows[u] rows, the items
+    // queues, n_own == 0, n_rest_items items): column u has items of bal_rows[u] rows, the items
     // bal_first[u] .. bal_first[u + 1] - 1 of the list.  See balance_items.
     int32_t n_bal;
     // The 256 x 128 kernel in its direct-to-LDS form: bytes of A (K * lda elements) and
