@@ -390,6 +390,48 @@ def test_multi_step_launch_places(tw, oracle, M, H):
     assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M,shortest", [(32, 512), (33, 512), (100, 449), (64, 448), (40, 100)])
+def test_multi_step_launch_of_long_tiles(tw, oracle, M, shortest, dtype):
+    """Tiles of as many kept rows as a wave's registers take, so that steps are multiplied in pairs (from 449 rows on and
+    with more than one row block), next to one tile that ends the pairs: bit for bit what the form without the
+    first look computes step by step, and the single-step launches' states."""
+    import torch
+    rng = np.random.default_rng(M + shortest)
+    I, H, G, T = 320, 256, 128, 4
+    K, ld = I + H, (M + 7) // 8 * 8
+    W, bias, tiles, xs, h0, c0, A, c = _sequence_problem(rng, oracle, M, I, H, G, 0.5, T, dtype, ld)
+    for i, t in enumerate(tiles):
+        n = shortest if i == 3 else int(rng.integers(449, 513))
+        t["kept_k"] = np.sort(rng.choice(K, n, replace=False)).astype(np.int32)
+    dbias = torch.from_numpy(bias).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    got = []
+    with tw.Plan.create(K, 4 * H, dtype, tiles, W) as plan:
+        for look in (-1, 0):
+            print("long tiles", M, shortest, dtype, look, flush=True)
+            tw.set_option(tw.OPT_LSTM_LOOK, look)
+            try:
+                dA, dC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+                plan.lstm_steps(T, dA.data_ptr(), M, dC.data_ptr(), lda=ld, a_step=K * ld, ldc=ld,
+                                bias_ptr=dbias.data_ptr(), stream=s)
+                plan.lstm_steps_status(s)
+            finally:
+                tw.set_option(tw.OPT_LSTM_LOOK, -1)
+            got.append((dA, dC))
+        assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+        oA, oC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        for t in range(T):
+            plan.lstm_step(oA[t].data_ptr(), M, oC.data_ptr(), oC.data_ptr(), oA[t + 1, I].data_ptr(), lda=ld,
+                           ldc_prev=ld, ldc_new=ld, ldh=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        torch.cuda.synchronize()
+        dA, dC = got[0]
+        h = oracle.bits_to_f32(dA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+        want = oracle.bits_to_f32(oA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+    assert oracle.rel_error(h, want) <= 2 * TOL[dtype]
+    assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
+
+
 def test_multi_step_launch_in_a_graph(tw, oracle):
     """tw_lstm_steps records into a HIP graph (its fill of the rows of h is a kernel, not a memset):
     the graph is replayed four times on inputs restored in between, with eager launches of the same

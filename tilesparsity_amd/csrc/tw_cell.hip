@@ -383,14 +383,14 @@ struct LstmSeqArgs {
     float forget_bias;
     int32_t spin_limit;
     uint32_t a_bytes; // K * lda * 2
-    int32_t pad_;
+    int32_t per_hb;   // 2^20 / (H / 32), rounded up: exact quotients of the workgroups' numbers
     LstmBlk blk[kLstmMaxBlks];
 };
 static_assert(sizeof(LstmSeqArgs) <= 4096, "kernel arguments");
 
 // RB rows m of A per workgroup (32 is what the launch uses).  LOOK false: without the first look at
-// one word per writing workgroup (the fall-back path alone; TW_OPT_LSTM_LOOK = 0).
-template <int DT, int RB, bool LOOK>
+// one word per writing workgroup (the fall-back path alone; TW_OPT_LSTM_LOOK = 0).  PAIRS: see multiply_steps.
+template <int DT, int RB, bool LOOK, bool PAIRS>
 __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const LstmSeqArgs p)
 {
     static_assert(RB == 32 || RB == 16, "rows of a workgroup");
@@ -409,7 +409,7 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const
     const int n_hb = p.H / 32;
     const int die = blockIdx.x % kXcd, each = gridDim.x / kXcd, more = gridDim.x % kXcd;
     const int place = die * each + min(die, more) + (int)(blockIdx.x / kXcd);
-    const int hb = place % n_hb, m0 = place / n_hb * RB;
+    const int rb = place * p.per_hb >> 20, hb = place - rb * n_hb, m0 = rb * RB;
     const LstmBlk blk = p.blk[hb * 4 + gate];
     const int nsteps = (blk.k_kept + kBlockK - 1) / kBlockK;
     unsigned char *const stage = smem + wave * kLstmStage;
@@ -516,25 +516,48 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const
                                         : __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)voff[i][r], 0, 0));
             }
     };
-    // multiplies them: two steps through the two halves of the wave's stage, both written before either is read, so that
-    // the second one's reads follow the first one's products without a wait (M 128, 50 steps 228 -> 224 us)
+    // multiplies them: a step through one half of the wave's stage (the halves in turn, so that a
+    // step's rows are written while the step before is still being read); PAIRS: two steps through both halves, both
+    // written before either is read, so that the second one's reads follow the first one's products without a wait
     auto multiply_steps = [&](int lo, int hi) {
+        if constexpr (PAIRS) {
 #pragma unroll
-        for (int pair = 0; pair < kSeqSteps; pair += 2) {
-            if (pair + 2 <= lo || pair >= hi)
-                continue;
+            for (int pair = 0; pair < kSeqSteps; pair += 2) {
+                if (pair + 2 <= lo || pair >= hi)
+                    continue;
 #pragma unroll
-            for (int i = pair; i < pair + 2; ++i)
+                for (int i = pair; i < pair + 2; ++i)
+                    if (i >= lo && i < hi) {
+#pragma unroll
+                        for (int r = 0; r < LPS; ++r)
+                            *reinterpret_cast<u32x4 *>(stage + (i & 1) * STEPB + (r * RPL + rowl) * PITCH + ch * 16) = av[i][r];
+                    }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+                for (int i = pair; i < pair + 2; ++i)
+                    if (i >= lo && i < hi) {
+                        TW_LDS(unsigned char) lds_lane = (TW_LDS(unsigned char))stage + (i & 1) * STEPB + lane_b;
+#pragma unroll
+                        for (int k16 = 0; k16 < 4; ++k16) {
+                            const uint32_t r_lo = r_first + k16 * 16, r_hi = r_lo + 4;
+                            const s16x4 lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + r_lo * PITCH));
+                            const s16x4 hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds_lane + r_hi * PITCH));
+                            const u32x2 l2 = __builtin_bit_cast(u32x2, lo4), h2 = __builtin_bit_cast(u32x2, hi4);
+                            acc = mfma16<DT>(u32x4{l2.x, l2.y, h2.x, h2.y}, bq[i][k16], acc);
+                        }
+                    }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kSeqSteps; ++i)
                 if (i >= lo && i < hi) {
+                    unsigned char *const half = stage + (i & 1) * STEPB;
 #pragma unroll
                     for (int r = 0; r < LPS; ++r)
-                        *reinterpret_cast<u32x4 *>(stage + (i & 1) * STEPB + (r * RPL + rowl) * PITCH + ch * 16) = av[i][r];
-                }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int i = pair; i < pair + 2; ++i)
-                if (i >= lo && i < hi) {
-                    TW_LDS(unsigned char) lds_lane = (TW_LDS(unsigned char))stage + (i & 1) * STEPB + lane_b;
+                        *reinterpret_cast<u32x4 *>(half + (r * RPL + rowl) * PITCH + ch * 16) = av[i][r];
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                    TW_LDS(unsigned char) lds_lane = (TW_LDS(unsigned char))half + lane_b;
 #pragma unroll
                     for (int k16 = 0; k16 < 4; ++k16) {
                         const uint32_t r_lo = r_first + k16 * 16, r_hi = r_lo + 4;
@@ -871,6 +894,7 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
     const int limit = get_option(TW_OPT_SPIN_LIMIT);
     a.spin_limit = limit >= 0 ? limit : (1 << 20);
     a.a_bytes = (uint32_t)((uint64_t)K * (uint64_t)lda * 2u);
+    a.per_hb = ((1 << 20) + H / 32 - 1) / (H / 32);
     lstm_fill_blocks(plan, H, a.blk);
     // the rows of h the steps will hand to each other start out as "not written yet"
     if (T > 1) {
@@ -879,18 +903,21 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
                            A16, lda, a_step, M, H, K, T);
     }
     const dim3 grid((unsigned)(H / 32 * row_blocks)), block(64 * kLstmWaves);
+    // Pairs of steps where every wave has all of its four and there is more than one row block.  us for 50 steps one by one and in
+    // pairs: H 1024, tiles of 512 kept rows, M 128 223.9 and 219.7, M 256 223.3 and 218.6, M 32 207.9 and 208.3; H 512, M 256 202.9
+    // and 201.5, M 8 189.7 and 191.6; 410 kept rows 228.3 and 230.2 (M 128), fewer 1 - 3 % more in pairs (H 256, 128 kept rows, M 32 136.2
+    // and 139.1).
     const bool first_look = get_option(TW_OPT_LSTM_LOOK) != 0;
-    if (plan->dtype == TW_F16) {
-        if (first_look)
-            hipLaunchKernelGGL((tw_lstm_steps_kernel<TW_F16, 32, true>), grid, block, 0, (hipStream_t)stream, a);
-        else
-            hipLaunchKernelGGL((tw_lstm_steps_kernel<TW_F16, 32, false>), grid, block, 0, (hipStream_t)stream, a);
-    } else {
-        if (first_look)
-            hipLaunchKernelGGL((tw_lstm_steps_kernel<TW_BF16, 32, true>), grid, block, 0, (hipStream_t)stream, a);
-        else
-            hipLaunchKernelGGL((tw_lstm_steps_kernel<TW_BF16, 32, false>), grid, block, 0, (hipStream_t)stream, a);
-    }
+    bool pairs = first_look && row_blocks > 1;
+    for (int b = 0; b < H / 32 * 4; ++b)
+        pairs &= a.blk[b].k_kept > (2 * kSeqSteps - 1) * kBlockK;
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, (hipStream_t)stream, a); };
+    if (plan->dtype == TW_F16)
+        launch(pairs ? tw_lstm_steps_kernel<TW_F16, 32, true, true>
+                     : first_look ? tw_lstm_steps_kernel<TW_F16, 32, true, false> : tw_lstm_steps_kernel<TW_F16, 32, false, false>);
+    else
+        launch(pairs ? tw_lstm_steps_kernel<TW_BF16, 32, true, true>
+                     : first_look ? tw_lstm_steps_kernel<TW_BF16, 32, true, false> : tw_lstm_steps_kernel<TW_BF16, 32, false, false>);
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
