@@ -16,7 +16,7 @@ namespace tw { constexpr int kXcd = 8, kBalColumns = 4; }
 #include "tw_queue.h"
 using namespace tw;
 struct Args {
-    int32_t n_mblk, n_pipe_u, n_all_u, n_own, n_last, n_lead_items, n_col_mblk, n_col_items, n_rest_items, rb_major;
+    int32_t n_mblk, n_pipe_u, n_all_u, n_own, n_last, last_x, last_r, n_lead_items, n_col_mblk, n_col_items, n_rest_items, rb_major;
     int32_t n_bal, bal_first[kBalColumns + 1], bal_rows[kBalColumns];
 };
 static int walk(const Args &a, bool owned, bool by_rows)

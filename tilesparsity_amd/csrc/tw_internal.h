@@ -80,7 +80,8 @@ struct GemmArgs {
     int32_t n_gemm_u;     // + pieces of units without (their columns receive beta * C)
     int32_t n_all_u;      // + tiles with pruned columns to fill
     int32_t n_own;        // row blocks owned by each queue
-    int32_t n_last;       // ... of which so many come behind the groups
+    int32_t n_last;       // ... of which so many come behind the groups:
+    int32_t last_x, last_r; // the r-th of queue x is number x * last_x + r * last_r of those behind all groups
     int32_t n_lead_items; // items of a queue's groups: (n_own - n_last) * n_pipe_u
     int32_t n_col_mblk;   // entries of a column in the list behind them
     int32_t n_col_items;  // ... of all columns with steps: n_pipe_u * n_col_mblk
