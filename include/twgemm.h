@@ -528,7 +528,7 @@ int tw_prune_tiled_wise_1d_mix(int n_layers, const int32_t *K, const int32_t *N,
                                double sparsity, int q_type, int granularity, double g1percent, int g1_q_type,
                                uint8_t *const *masks, double *threshold, void *stream);
 
-/* The three with masks that the caller allocates while the first kernels run: `ready(user)` is called once,
+/* The three producers with masks that the caller allocates while the first kernels run: `ready(user)` is called once,
  * on the calling thread, when those are queued, and has put the masks' addresses into `masks` when it
  * returns 0; any other value ends the call with TW_ERR_ALLOC.  It may call this library, and may wait for
  * other threads that do: no call waits for one that is in its `ready`.  The current device is as before when

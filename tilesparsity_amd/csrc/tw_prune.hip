@@ -1472,7 +1472,7 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // elements.  The narrowing pass also writes the masks: what lies outside the bracket is decided
 // already, and the few per cent inside are marked one by one when the threshold is known, from the places kept
 // beside their values.
-// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 42 + 27 + 10 us; with those masks
+// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 40 + 26 + 10 us; with those masks
 // written and read and the elements read once more at the end 13 + 4 + 11 + 31 + 31 + 32, and the host's wait between the stages.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
@@ -1742,8 +1742,8 @@ __global__ void __launch_bounds__(256)
     }
     if (narrowed) {
         // four pieces at a time, sixteen loads in flight: a piece holds some two hundred values, and one piece after the other,
-        // each behind the load of its count, was eleven pairs of trips to memory (the three passes 18 + 12 + 12 us, so 9 + 11 +
-        // 11; what is left are the counts of all waves, the digits so far and the counters' atomics: 48 workgroups 12 + 15 + 15,
+        // each behind the load of its count, was eleven pairs of trips to memory (the three passes 18 + 12 + 12 us, so 11 + 10 +
+        // 11, and 5 for the third where two digits hold the bracket's range; what is left are the counts of all waves, the digits so far and the counters' atomics: 48 workgroups 12 + 15 + 15,
         // 192 10 + 10 + 10, 256 12 + 10 + 10)
         for (int q0 = 0; q0 < mine; q0 += 4) {
             TW_GLOBAL(const u32x2) v[4];

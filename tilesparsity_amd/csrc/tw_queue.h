@@ -66,8 +66,8 @@ template <class Args> TW_QUEUE_FN int queue_length(const Args &p, int x)
 // Entry q of queue x, of `len` entries; bm: rows of a row block.  Every workgroup works its first entry out before its
 // first load leaves, by code that comes from memory then: one division, whatever the part of the queue, and the end
 // without it.  With a division for each part and the starts of the columns counted die by die, launches of one item a
-// workgroup took up to a tenth longer (a quarter of the rows kept: M 4096, K 3072, N 768 15.3 us, now 14.6; M 8192, K 4096, N 1024
-// 28.5 and 27.8; M 8192, K 4096, N 512 with a tenth 12.7 and 11.8), longer ones 1 - 3 % (VGG16 conv4_2 29.4 and 28.7).
+// workgroup took up to a tenth longer (a quarter of the rows kept: M 4096, K 3072, N 768 15.4 us, 14.6 by this; M 8192, K 4096, N 1024
+// 28.6 and 27.4; M 8192, K 4096, N 512 with a tenth 12.7 and 11.8), longer ones 1 - 3 % (VGG16 conv4_2 29.3 and 28.6).
 template <class Args> TW_QUEUE_FN Work queue_entry(const Args &p, int x, int q, int len, int bm)
 {
     Work w;
