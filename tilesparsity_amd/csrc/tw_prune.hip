@@ -1899,8 +1899,9 @@ struct Kept {
         device = -1; // the device of the next call
     }
 };
-std::mutex g_kept_mutex; // (held for a look at `g_kept` only)
-std::condition_variable g_kept_free;
+// (held for a look at `g_kept` only; neither is destroyed when the process ends, whose other threads may still wait)
+std::mutex &g_kept_mutex = *new std::mutex;
+std::condition_variable &g_kept_free = *new std::condition_variable;
 Kept g_kept[2];
 
 class Arena {
