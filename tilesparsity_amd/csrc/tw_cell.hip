@@ -862,7 +862,8 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
     // number of row pieces of half the size, and a step takes 8.5 us instead of 5.9.)
     const int rb = 32;
     const int64_t row_blocks = ((int64_t)M + rb - 1) / rb;
-    const bool persistent = lstm_fused_plan(plan, H) && plan->max_k_pad <= 2 * kSeqSteps * kBlockK &&
+    const int64_t marks = (int64_t)(T - 1) * H * ((M + 7) / 8); // pieces of h to mark, a thread each
+    const bool persistent = marks <= kMaxGridThreads / 256 * 256 && lstm_fused_plan(plan, H) && plan->max_k_pad <= 2 * kSeqSteps * kBlockK &&
                             (int64_t)(H / 32) * row_blocks <= plan->cu_count &&
                             (uint64_t)K * (uint64_t)lda * 2u < (1ull << 32) && T > 1 && plan->d_tickets;
     if (!persistent) {
@@ -898,8 +899,7 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
     lstm_fill_blocks(plan, H, a.blk);
     // the rows of h the steps will hand to each other start out as "not written yet"
     if (T > 1) {
-        const int64_t n = (int64_t)(T - 1) * H * ((M + 7) / 8);
-        hipLaunchKernelGGL(lstm_mark_unwritten_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+        hipLaunchKernelGGL(lstm_mark_unwritten_kernel, dim3((unsigned)((marks + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
                            A16, lda, a_step, M, H, K, T);
     }
     const dim3 grid((unsigned)(H / 32 * row_blocks)), block(64 * kLstmWaves);
