@@ -432,6 +432,73 @@ def test_multi_step_launch_of_long_tiles(tw, oracle, M, shortest, dtype):
     assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
 
 
+@pytest.mark.parametrize("M,I,H,k_keep,T,dtype", [(2, 64, 1024, 0.25, 24, "f16"), (33, 1000, 1024, 0.2, 25, "bf16"),
+                                                  (100, 1024, 1024, 0.25, 24, "f16"), (43, 100, 512, 0.4, 32, "bf16"),
+                                                  (64, 1023, 1024, 0.12, 24, "f16")])
+def test_multi_step_launch_with_its_rows_in_lds(tw, oracle, M, I, H, k_keep, T, dtype):
+    """Sequences long and wide enough for the form that keeps the rows of A in LDS, next to a tile without a kept row, one
+    of 512, one that keeps rows of x only and one that keeps rows of h only: the single-step launches' states
+    within the tolerance of a step's h, the same bits a second time and without the first look, nothing
+    written beyond M or into the rows of x, and a launch without any polls reported as given up."""
+    import torch
+    rng = np.random.default_rng(M + I + T)
+    K, G, ld = I + H, 128, (M + 7) // 8 * 8
+    W, bias, tiles, xs, h0, c0, A, c = _sequence_problem(rng, oracle, M, I, H, G, k_keep, T, dtype, ld)
+    # Weights of 0.02: a hidden unit's gates then answer to h with 0.02 * sqrt(512) = 0.45 at most (in the 2-norm, derivatives of the
+    # activations left at their limit of 1), so that the differences of 24 - 32 steps add up to less than two of one step's
+    # (of 0.08 they would grow 1.8 times a step instead).
+    W *= 0.25
+    per_gate = H // G
+    for t, rows in ((0, np.arange(0)), (per_gate + 1, np.sort(rng.choice(K, 512, replace=False))),
+                    (1, np.sort(rng.choice(I, min(I, 200), replace=False))),
+                    (2 * per_gate, I + np.sort(rng.choice(H, 333, replace=False)))):
+        tiles[t]["kept_k"] = rows.astype(np.int32)
+    for t in tiles:
+        if len(t["kept_k"]) > 512:
+            t["kept_k"] = np.sort(rng.choice(t["kept_k"], 511, replace=False)).astype(np.int32)
+    assert np.mean([len(t["kept_k"]) for t in tiles]) >= 151  # (what the launch asks for, and no tile beyond 512)
+    dbias = torch.from_numpy(bias).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+
+    def steps(plan):
+        dA, dC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        plan.lstm_steps(T, dA.data_ptr(), M, dC.data_ptr(), lda=ld, a_step=K * ld, ldc=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        return dA, dC
+    with tw.Plan.create(K, 4 * H, dtype, tiles, W) as plan:
+        outs = []
+        for look in (-1, -1, 0):
+            print("rows in LDS", M, I, H, dtype, look, flush=True)
+            tw.set_option(tw.OPT_LSTM_LOOK, look)
+            try:
+                outs.append(steps(plan))
+                plan.lstm_steps_status(s)
+            finally:
+                tw.set_option(tw.OPT_LSTM_LOOK, -1)
+        for got in outs[1:]:
+            assert torch.equal(got[0], outs[0][0]) and torch.equal(got[1], outs[0][1])
+        oA, oC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        for t in range(T):
+            plan.lstm_step(oA[t].data_ptr(), M, oC.data_ptr(), oC.data_ptr(), oA[t + 1, I].data_ptr(), lda=ld,
+                           ldc_prev=ld, ldc_new=ld, ldh=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        torch.cuda.synchronize()
+        try:
+            tw.set_option(tw.OPT_SPIN_LIMIT, 0)
+            steps(plan)
+            with pytest.raises(tw.TwError) as e:
+                plan.lstm_steps_status(s)
+            assert e.value.status == tw.ERR_DEVICE
+        finally:
+            tw.set_option(tw.OPT_SPIN_LIMIT, -1)
+    dA, dC = outs[0]
+    a = from_device_bits(dA)
+    assert np.array_equal(a[:, :I], A[:, :I]) and np.array_equal(a[:, :, M:], A[:, :, M:])
+    assert np.array_equal(dC.cpu().numpy()[:, M:], c[:, M:])
+    got = oracle.bits_to_f32(dA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+    want = oracle.bits_to_f32(oA[1:, I:, :M].contiguous().cpu().numpy().view(np.uint16), dtype)
+    assert oracle.rel_error(got, want) <= 2 * TOL[dtype]
+    assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
+
+
 def test_multi_step_launch_in_a_graph(tw, oracle):
     """tw_lstm_steps records into a HIP graph (its fill of the rows of h is a kernel, not a memset):
     the graph is replayed four times on inputs restored in between, with eager launches of the same

@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstring>
+#include <type_traits>
 
 namespace tw {
 namespace {
@@ -701,6 +702,422 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const
             p.c[(int64_t)hu * p.ldc + m0 + mt + e] = c2[e];
 }
 
+#define TW_LDS_MEET() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
+
+// ---------------------------------------------------------------------------------
+// The same launch with the rows of A in LDS: where the rows of x and of h are at most 1024 each, a workgroup keeps one
+// copy of every row that any of its four gates keeps (the union of four lists: 700 of 1024 rows of either where each keeps a
+// quarter) and the waves gather their lists' rows there, with the transposed read's address per lane.
+// What bounds the kernel above is its row pieces on their way through a compute unit's vector memory path (64 bytes each, 45 bytes
+// a clock with sixteen workgroups on a die, and a wave that issues loads stands until they are taken): 2048 of them a step at four lists
+// of 512 kept rows, and the chain of its slowest wave, which has three of the five steps of 64 kept rows that hold rows of h.  Here a step
+// fetches 1400, no wave turns its rows through a stage of its own, and a list is dealt out in groups of 16 kept rows, the groups of
+// x and those of h in halves each.
+//   panel:  row s of the union at s * 64 bytes: the rows of x, ascending, then from a multiple of 128 on the rows of h; a load of a
+//           wave brings 16 rows straight into LDS.  The 32-byte halves of rows 4 .. 7 of eight are swapped, against bank conflicts.
+//   step:   look (as above); rows of h into the panel; meeting; products of the groups with rows of h; partial products, and the
+//           next step's rows of x leave, from the waves that have a group less; meeting; cell, h stored; meeting; products of the
+//           groups with rows of x while h travels.
+//   groups: a wave's weight fragments stay in registers, its groups with rows of x in blocks of four from the first slot on, those with rows
+//           of h from the last on; a group with both is in either, each time with zeros for the other's rows.
+//   edges:  a row of zeros stands for the padding of a list and for a slot without a group; rows and pieces that are not there get
+//           an offset beyond the buffer and arrive as zeros.
+// A row of h is looked at by its dwords: a thread stores two rows m of a hidden unit as one dword, and neither half of a stored
+// one is the pattern, so what is not written yet shows as a dword of all ones.
+// Cycles of a step, first / last wave (M 128, H 1024, 512 kept rows; the kernel above): look 1090 / 1100 (1040 / 1070), rows of h 1310 / 1550 (3190 / 4140),
+// looked at 590, meeting 810 / 290, products 990 / 1330 (2040 / 2430 with the loads of x), partial products, loads of x and meeting 1560 / 1210 (1960 / 590), cell
+// 780 / 1080 (850 / 1180), meeting 420 / 120 (400 / 70), products of x 1230 / 1490 (1490 / 1500): 8770 (10970).  Tried and slower: the loads
+// of x by all waves behind those of h (9770: the waves stand until all are taken before they can look at the rows of h), before the
+// look (9430), ahead of the products (9700), through registers between the products (10360).
+constexpr int kPanRows = 1024;   // most rows of x, and of h
+constexpr int kPanList = 2 * kSeqSteps * kBlockK; // most kept rows of a tile
+constexpr int kPanBlocks = 5;    // blocks of four groups of 16 kept rows a wave multiplies: 16 groups (tiles of at most 512 kept rows), no block with both kinds
+constexpr int kPanLoads = kPanRows / (16 * kLstmWaves); // loads of either kind a wave has
+constexpr int kPanPartial = 32 * 32 * 4;                // bytes of a wave's partial product
+constexpr int64_t pan_rows_up(int64_t rows) { return (rows + 127) / 128 * 128; }
+constexpr int64_t pan_lds_bytes(int64_t K, int64_t H)
+{
+    return kLstmWaves * kPanPartial + (pan_rows_up(K - H) + pan_rows_up(H)) * 64;
+}
+static_assert(pan_lds_bytes(2 * kPanRows, kPanRows) <= 160 * 1024, "the panel and the partial products fit a compute unit's LDS");
+
+template <int DT, bool LOOK>
+__global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_panel_kernel(const LstmSeqArgs p)
+{
+    extern __shared__ __align__(16) unsigned char lds[];
+    constexpr uint32_t kGone = 0xFFFFFFF0u;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int gate = wave >> 1, kh = wave & 1;
+    // (places as above)
+    const int n_hb = p.H / 32;
+    const int die = blockIdx.x % kXcd, each = gridDim.x / kXcd, more = gridDim.x % kXcd;
+    const int place = die * each + min(die, more) + (int)(blockIdx.x / kXcd);
+    const int rb = place * p.per_hb >> 20, hb = place - rb * n_hb, m0 = rb * 32;
+    const LstmBlk blk = p.blk[hb * 4 + gate];
+    const int32_t *const list = p.kept_k + blk.kk_off;
+    const int n = blk.k_kept, first_h = p.K - p.H;
+    float *const part0 = reinterpret_cast<float *>(lds); // eight partial products
+    unsigned char *const panel = lds + kLstmWaves * kPanPartial;
+    TW_LDS(unsigned char) const panel_lds = (TW_LDS(unsigned char))panel;
+
+    // ---- the union of the four lists: a flag per row of A, ranks by a scan, in LDS that the panel takes over
+    unsigned char *const flag = lds;                                            // 2048 bytes
+    uint16_t *const rank = reinterpret_cast<uint16_t *>(lds + 2048);            // row -> place in the union
+    uint16_t *const rows = reinterpret_cast<uint16_t *>(lds + 2048 + 4096);     // ... and back
+    int *const sums = reinterpret_cast<int *>(lds + 2048 + 8192);               // a wave's flags; [8]: rows of x; [9]: all
+    uint16_t *const list16 = reinterpret_cast<uint16_t *>(lds + 2048 + 8192 + 64) + gate * kPanList; // the gate's list once more
+    reinterpret_cast<uint32_t *>(flag)[tid] = 0;
+    int n_xrows = 0; // of this gate's list
+    {
+        int row[kPanList / 64];
+#pragma unroll
+        for (int i = 0; i < kPanList / 64; ++i) // (all on their way at once; the first again beyond the list's padding)
+            row[i] = list[i * 64 < n ? i * 64 + lane : lane];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kPanList / 64; ++i) {
+            const bool real = i * 64 + lane < n;
+            n_xrows += __builtin_popcountll(__builtin_amdgcn_ballot_w64(real && row[i] < first_h));
+            if (real) {
+                flag[row[i]] = 1;
+                list16[i * 64 + lane] = (uint16_t)row[i];
+            }
+        }
+    }
+    __syncthreads();
+    {
+        const uint32_t f = reinterpret_cast<uint32_t *>(flag)[tid]; // rows 4 tid .. + 3
+        const int mine = __popc(f);
+        int upto = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(upto, d);
+            upto += lane >= d ? v : 0;
+        }
+        if (lane == 63)
+            sums[wave] = upto;
+        __syncthreads();
+        int at = upto - mine;
+        for (int w = 0; w < wave; ++w)
+            at += sums[w];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = tid * 4 + e;
+            if (row == first_h)
+                sums[8] = at;
+            if (row < p.K)
+                rank[row] = (uint16_t)at;
+            if (f >> (8 * e) & 1u)
+                rows[at++] = (uint16_t)row;
+        }
+        if (tid == 64 * kLstmWaves - 1)
+            sums[9] = at;
+    }
+    __syncthreads();
+    const int ux = __builtin_amdgcn_readfirstlane(sums[8]), uh = __builtin_amdgcn_readfirstlane(sums[9]) - ux;
+    const int h_base = (ux + 127) / 128 * 128;             // first row of h of the panel
+    const int lh = (uh + 127) / 128; // loads of rows of h a wave has
+    // ---- this wave's groups and their rows' places in the panel
+    const int groups = (n + 15) / 16, gx = (n_xrows + 15) / 16, gh = groups - n_xrows / 16;
+    const int nx = kh ? gx / 2 : (gx + 1) / 2, nh = kh ? (gh + 1) / 2 : gh / 2; // <= 17 together
+    const int x0 = kh ? (gx + 1) / 2 : 0, h0 = groups - gh + (kh ? gh / 2 : 0);
+    const int L = lane & 15;
+    const int pos = (lane >> 5) * 8 + (L >> 2); // of this lane's row in the first transposed read of a group, + 4 in the second
+    const uint32_t lane_b = (uint32_t)(((lane >> 4) & 1) * 32 + (L & 3) * 8);
+    u32x4 bq[kPanBlocks][4];
+    uint32_t at[kPanBlocks][4]; // of a group's two reads: places in LDS in units of 8 bytes, 16 bits each
+    {
+        TW_GLOBAL(const unsigned char) const bsrc = (TW_GLOBAL(const unsigned char))p.Bp + blk.b_first + lane * 16;
+        const uint32_t panel_at = kLstmWaves * kPanPartial, zeros_at = (uint32_t)wave * kPanPartial;
+#pragma unroll
+        for (int b = 0; b < kPanBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int x = b * 4 + i, j = (kPanBlocks - 1 - b) * 4 + i;
+                const bool of_x = x < nx;
+                const int g = of_x ? x0 + x : j < nh ? h0 + j : -1;
+                bq[b][i] = u32x4{0u, 0u, 0u, 0u};
+                if (g >= 0)
+                    bq[b][i] = *(TW_GLOBAL(const u32x4))(bsrc + (g >> 2) * blk.step_b + (g & 3) * 1024);
+                at[b][i] = 0;
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const int e = g * 16 + pos + q * 4;
+                    uint32_t byte = zeros_at + lane_b;
+                    const int row = g >= 0 && e < n ? list16[e] : p.K;
+                    if (row < p.K && (row < first_h) == of_x) {
+                        const int place_of = rank[row] + (of_x ? 0 : h_base - ux);
+                        byte = panel_at + (uint32_t)place_of * 64u + (lane_b ^ (place_of >> 2 & 1) * 32u);
+                    }
+                    at[b][i] |= byte / 8u << (16 * q);
+                }
+            }
+    }
+    const int xb = (nx + 3) / 4, hb4 = (nh + 3) / 4; // blocks of either kind: together 5 at most
+    // ---- this wave's loads: 16 rows of the panel each, four lanes of 16 bytes a row
+    const int ch = (lane & 3) ^ (lane >> 4 & 1) * 2; // (the halves of rows 4 .. 7 of eight swapped)
+    const bool m_ok = m0 + ch * 8 < p.M;
+    uint32_t vx[2 * kPanLoads], vh[kPanLoads]; // (the rows of x: by the waves of the list's first halves alone)
+#pragma unroll
+    for (int l = 0; l < 2 * kPanLoads; ++l) {
+        const int u = (l * (kLstmWaves / 2) + gate) * 16 + (lane >> 2);
+        vx[l] = u < ux && m_ok ? (uint32_t)rows[u] * ((uint32_t)p.lda * 2u) + (uint32_t)(m0 + ch * 8) * 2u : kGone;
+    }
+#pragma unroll
+    for (int l = 0; l < kPanLoads; ++l) {
+        const int u = (l * kLstmWaves + wave) * 16 + (lane >> 2);
+        vh[l] = u < uh && m_ok ? (uint32_t)rows[ux + u] * ((uint32_t)p.lda * 2u) + (uint32_t)(m0 + ch * 8) * 2u : kGone;
+    }
+    // the cell's share of this thread: two rows of hidden unit hb * 32 + tid / 16
+    const int ju = tid >> 4, mt = (tid & 15) * 2;
+    const int hu = hb * 32 + ju;
+    bool row_ok[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        row_ok[e] = m0 + mt + e < p.M;
+    float bias4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (p.bias) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            bias4[g] = p.bias[g * p.H + hu];
+    }
+    float c2[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        c2[e] = row_ok[e] ? p.c[(int64_t)hu * p.ldc + m0 + mt + e] : 0.0f;
+    // (here, not at their first use: the wait there would be one for the rows of x on their way, at every step)
+    asm volatile("" : "+v"(bias4[0]), "+v"(bias4[1]), "+v"(bias4[2]), "+v"(bias4[3]), "+v"(c2[0]), "+v"(c2[1]));
+    const uint16_t *const A0 = reinterpret_cast<const uint16_t *>(p.A);
+    auto step_rsrc = [&](int t) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(A0 + (int64_t)t * p.a_step), 0, (int)p.a_bytes, kSeqRsrcFlags);
+    };
+    // the rows of x of A_t, straight into the panel
+    const int lx4 = (ux + 63) / 64;
+    TW_LDS(unsigned char) const lds_x = panel_lds + gate * 1024;
+    auto load_x = [&](int t) {
+        const __amdgpu_buffer_rsrc_t rsrc = step_rsrc(t);
+        int cnt = lx4;
+        asm volatile("" : "+s"(cnt));
+#pragma unroll
+        for (int l = 0; l < 2 * kPanLoads; ++l)
+            if (l < cnt)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TW_LDS(void))(lds_x + l * (kLstmWaves / 2 * 1024)), 16, (int)vx[l], 0, 0, 0);
+    };
+    // the rows of h go straight into the panel; once they are there a lane looks at its own pieces of them
+    TW_LDS(unsigned char) const lds_h = panel_lds + h_base * 64 + wave * 1024;
+    auto load_h = [&](int t, bool coherent) {
+        const __amdgpu_buffer_rsrc_t rsrc = step_rsrc(t);
+        int cnt = lh;
+        asm volatile("" : "+s"(cnt));
+#pragma unroll
+        for (int l = 0; l < kPanLoads; ++l)
+            if (l < cnt) {
+                if (coherent)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TW_LDS(void))(lds_h + l * (kLstmWaves * 1024)), 16, (int)vh[l], 0, 0, kSeqAuxCoherent);
+                else
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (TW_LDS(void))(lds_h + l * (kLstmWaves * 1024)), 16, (int)vh[l], 0, 0, 0);
+            }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    };
+    // (a row's last piece, where M is no multiple of 8: a dword with one element below M shows the pattern there, one with none is let pass)
+    const bool ragged = p.M - m0 < 32 && (p.M & 7);
+    auto unwritten = [&]() {
+        u32x4 v[kPanLoads];
+        int cnt = lh;
+        asm volatile("" : "+s"(cnt));
+#pragma unroll
+        for (int l = 0; l < kPanLoads; l += 2) {
+            v[l] = v[l + 1] = u32x4{0u, 0u, 0u, 0u};
+            if (l < cnt) {
+                v[l] = *(TW_LDS(const u32x4))(lds_h + l * (kLstmWaves * 1024) + lane * 16);
+                v[l + 1] = *(TW_LDS(const u32x4))(lds_h + min(l + 1, cnt - 1) * (kLstmWaves * 1024) + lane * 16);
+            }
+        }
+        if (ragged) {
+#pragma unroll
+            for (int l = 0; l < kPanLoads; ++l)
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const int m = m0 + ch * 8 + 2 * d;
+                    v[l][d] = m + 1 < p.M ? v[l][d] : m < p.M ? v[l][d] | 0xFFFF0000u : 0u;
+                }
+        }
+        uint32_t most[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int l = 0; l < kPanLoads; ++l)
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                most[d] = max(most[d], v[l][d]);
+        return __builtin_amdgcn_ballot_w64(max(max(most[0], most[1]), max(most[2], most[3])) == 0xFFFFFFFFu) != 0;
+    };
+    f32x16 acc;
+    auto clear = [&]() {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+            acc[e] = 0.0f;
+    };
+    // products of `cnt` blocks: UP: blocks 0, 1, .. (rows of x), else kPanBlocks - 1, .. (with rows of h), all reads of a block, and of the
+    // next one, ahead of its products; `also(i)` goes in front of the i-th
+    TW_LDS(unsigned char) const lds0 = (TW_LDS(unsigned char))lds;
+    auto multiply = [&](auto up_tag, int cnt, auto also) {
+        constexpr bool UP = decltype(up_tag)::value;
+        asm volatile("" : "+s"(cnt)); // (compared anew each time: the tests' results kept for all steps would not fit the scalar registers)
+        u32x4 op[2][4];
+        auto fetch = [&](int b, u32x4(&o)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint32_t w = at[b][i];
+                asm volatile("" : "+v"(w)); // (taken apart anew each time: the addresses kept for all steps would not fit the registers)
+                const u32x2 lo4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds0 + (w & 0xFFFFu) * 8u)));
+                const u32x2 hi4 = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((TW_LDS(s16x4))(lds0 + (w >> 16) * 8u)));
+                o[i] = u32x4{lo4.x, lo4.y, hi4.x, hi4.y};
+            }
+        };
+        if (cnt > 0)
+            fetch(UP ? 0 : kPanBlocks - 1, op[0]);
+#pragma unroll
+        for (int k = 0; k < kPanBlocks; ++k) {
+            also(k);
+            if (k + 1 < kPanBlocks && k + 1 < cnt)
+                fetch(UP ? k + 1 : kPanBlocks - 2 - k, op[(k + 1) & 1]);
+            if (k < cnt) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    acc = mfma16<DT>(op[k & 1][i], bq[UP ? k : kPanBlocks - 1 - k][i], acc);
+            }
+        }
+    };
+    auto nothing = [](int) {};
+    // the row of zeros that the padding of a list names, in this wave's place for partial products, which it does not need before its
+    // last read of the step
+    auto put_zeros = [&]() {
+        if (lane < 4)
+            *reinterpret_cast<u32x4 *>(lds + wave * kPanPartial + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    };
+    // the word lane l looks at, as above
+    const int probe_m = m0 + ((min(p.M - m0, 32) - 1) & ~1);
+    const uint32_t probe_off = lane < n_hb ? (uint32_t)(first_h + 32 * lane + 31) * ((uint32_t)p.lda * 2u) + (uint32_t)probe_m * 2u : kGone;
+    const uint32_t probe_mask = probe_m + 1 < p.M ? 0xFFFFFFFFu : 0xFFFFu;
+
+    __syncthreads(); // (the tables have been read)
+    if (kh == 0)
+        load_x(0);
+    put_zeros();
+    clear();
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    multiply(std::true_type(), xb, nothing);
+    // stores of h a wave has on its way when it waits for its rows of x, which left before them: one of dwords, or of the odd last row, or both
+    const int rows_m = min(p.M - m0, 32);
+    const bool two_stores = rows_m > 1 && (rows_m & 1);
+    bool gave_up = false;
+    for (int t = 0; t < p.T; ++t) {
+        // ---- rows of h of the step before: the look and the fetch as above
+        bool look = t > 0 && !gave_up && lh > 0; // (A_0 holds the caller's h)
+        int left = p.spin_limit;
+        if (look && LOOK) {
+            const __amdgpu_buffer_rsrc_t rsrc = step_rsrc(t);
+            for (;;) {
+                if (left <= 0)
+                    break;
+                --left;
+                const uint32_t w = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)probe_off, 0, kSeqAuxCoherent);
+                const uint32_t x = ~(w & probe_mask);
+                const bool fresh = ((x - 0x00010001u) & ~x & 0x80008000u) != 0;
+                if (__builtin_amdgcn_ballot_w64(fresh) == 0)
+                    break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+        }
+        load_h(t, !LOOK && look);
+        if (look) {
+            for (;;) {
+                if (left <= 0) {
+                    gave_up = true;
+                    if (lane == 0)
+                        __hip_atomic_store(p.status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    break;
+                }
+                if (!unwritten())
+                    break;
+                --left;
+                __builtin_amdgcn_s_sleep(1);
+                load_h(t, true);
+            }
+        }
+        TW_LDS_MEET();
+        multiply(std::false_type(), hb4, nothing);
+        // the partial product of this wave: column lane % 32, rows r4 * 8 + (lane / 32) * 4 + e; the 16-byte pieces of a column in another
+        // order in each of eight columns, against bank conflicts
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        {
+            const int col = lane & 31;
+            float *const part = part0 + wave * (kPanPartial / 4) + col * 32;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4)
+                *reinterpret_cast<f32x4 *>(part + ((r4 * 2 + (lane >> 5)) ^ (col & 7)) * 4) =
+                    f32x4{acc[r4 * 4], acc[r4 * 4 + 1], acc[r4 * 4 + 2], acc[r4 * 4 + 3]};
+        }
+        // the next step's rows of x leave
+        if (kh == 0 && t + 1 < p.T)
+            load_x(t + 1);
+        TW_LDS_MEET();
+        {
+            const float *const mine = part0 + ju * 32 + ((mt >> 2) ^ (ju & 7)) * 4 + (mt & 3);
+            // (read in asm: the compiler would wait for the rows of x on their way into LDS first)
+            float pre[4][2];
+            {
+                f32x4 v[4]; // of a gate: two rows of either partial product
+                static_assert(kPanPartial == 4096, "the reads' offsets, in pieces of 512 bytes");
+                asm volatile("ds_read2st64_b64 %0, %4 offset0:0 offset1:8\n\tds_read2st64_b64 %1, %4 offset0:16 offset1:24\n\t"
+                             "ds_read2st64_b64 %2, %4 offset0:32 offset1:40\n\tds_read2st64_b64 %3, %4 offset0:48 offset1:56\n\t"
+                             "s_waitcnt lgkmcnt(0)"
+                             : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+                             : "v"((uint32_t)(uintptr_t)(TW_LDS(const float))mine)
+                             : "memory");
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    pre[g][0] = (v[g].x + v[g].z) + bias4[g];
+                    pre[g][1] = (v[g].y + v[g].w) + bias4[g];
+                }
+            }
+            float h2[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                cell_update(pre[0][e], pre[1][e], pre[2][e], pre[3][e], p.forget_bias, c2[e], h2[e]);
+            uint16_t *const hdst = const_cast<uint16_t *>(A0) + (int64_t)(t + 1) * p.a_step + (int64_t)(first_h + hu) * p.lda + m0 + mt;
+            uint32_t h16[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                h16[e] = to16(h2[e], DT);
+                h16[e] = h16[e] == kSeqUnwritten ? kSeqUnwritten - 1u : h16[e];
+            }
+            asm volatile("" : "+v"(h16[0]), "+v"(h16[1])); // (side by side: left alone the second row waits for the first one's store)
+            if (row_ok[1]) {
+                const uint32_t w = h16[0] | (h16[1] << 16);
+                asm volatile("global_store_dword %0, %1, off sc0 sc1" ::"v"(hdst), "v"(w) : "memory");
+            } else if (row_ok[0]) {
+                const uint32_t w = h16[0];
+                asm volatile("global_store_short %0, %1, off sc0 sc1" ::"v"(hdst), "v"(w) : "memory");
+            }
+        }
+        if (t + 1 == p.T)
+            break;
+        // ---- the next step's rows of x, multiplied while h_t travels
+        clear();
+        if (two_stores)
+            asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else
+            asm volatile("s_waitcnt vmcnt(1) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        put_zeros();
+        multiply(std::true_type(), xb, nothing);
+    }
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+        if (row_ok[e])
+            p.c[(int64_t)hu * p.ldc + m0 + mt + e] = c2[e];
+}
+
 // Fills the rows of h of A_1 .. A_(T-1), rows m below M, with the pattern tw_lstm_steps_kernel
 // takes for "not written yet".  One thread per 16-byte piece (8 rows m) of a row.
 __global__ void lstm_mark_unwritten_kernel(uint16_t *A, int64_t lda, int64_t a_step, int M, int H, int K, int T)
@@ -746,6 +1163,14 @@ void lstm_fill_blocks(const tw_plan *plan, int H, LstmBlk *blk)
     }
 }
 } // namespace
+
+int prepare_cell()
+{
+    for (const void *k : {(const void *)tw_lstm_panel_kernel<TW_F16, true>, (const void *)tw_lstm_panel_kernel<TW_F16, false>,
+                          (const void *)tw_lstm_panel_kernel<TW_BF16, true>, (const void *)tw_lstm_panel_kernel<TW_BF16, false>})
+        TW_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)pan_lds_bytes(2 * kPanRows, kPanRows)));
+    return TW_OK;
+}
 } // namespace tw
 
 using namespace tw;
@@ -903,6 +1328,27 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
                            A16, lda, a_step, M, H, K, T);
     }
     const dim3 grid((unsigned)(H / 32 * row_blocks)), block(64 * kLstmWaves);
+    // The form with the rows of A in LDS.  It saves up to a fifth of a step and needs 4 - 6 us more to begin with.  us for 50 steps, above
+    // and in LDS, inputs as many as units: H 1024, a quarter kept, M 8 204 and 182, M 128 228 and 200, M 200 275 and 228, M 256 225 and 211; a tenth
+    // M 8 182 and 154, M 128 194 and 159; M 1 a quarter 201 and 195, a tenth 168 and 163; H 512, a quarter, M 128 176 and 158, half 210 and 178, a tenth 147 and 146; H 256
+    // 138 and 145.  24 steps: H 1024, 512 inputs, 154 kept rows, M 2 91 and 85, M 128 97 and 85; 64 inputs, 109 kept 79 and 83.  Below H 1024 with few rows or
+    // few kept rows of h: H 512, 1024 inputs, M 16, 102 of h 77 and 84, M 128, 51 of h 79 and 78; H 768, 768 inputs, M 4, 154 of h 90 and 94.
+    const int64_t kept = plan->n_tiles ? plan->kept_k_ptr[plan->n_tiles] / plan->n_tiles : 0; // rows of a tile, in the mean
+    const bool panel = K > H && K - H <= kPanRows && H <= kPanRows && M >= 2 && kept >= 150 &&
+                       (H >= 1024 ? T >= 24 : H >= 512 && T >= 32 && M > 32 && kept * H >= 100 * (int64_t)K);
+    if (panel) {
+        const int pst = prepare_device();
+        if (pst != TW_OK)
+            return pst;
+        const bool look = get_option(TW_OPT_LSTM_LOOK) != 0;
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, (size_t)pan_lds_bytes(K, H), (hipStream_t)stream, a); };
+        if (plan->dtype == TW_F16)
+            go(look ? tw_lstm_panel_kernel<TW_F16, true> : tw_lstm_panel_kernel<TW_F16, false>);
+        else
+            go(look ? tw_lstm_panel_kernel<TW_BF16, true> : tw_lstm_panel_kernel<TW_BF16, false>);
+        TW_HIP(hipGetLastError());
+        return TW_OK;
+    }
     // Pairs of steps where every wave has all of its four and there is more than one row block.  us for 50 steps one by one and in
     // pairs: H 1024, tiles of 512 kept rows, M 128 223.9 and 219.7, M 256 223.3 and 218.6, M 32 207.9 and 208.3; H 512, M 256 202.9
     // and 201.5, M 8 189.7 and 191.6; 410 kept rows 228.3 and 230.2 (M 128), fewer 1 - 3 % more in pairs (H 256, 128 kept rows, M 32 136.2

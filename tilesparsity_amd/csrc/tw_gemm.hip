@@ -2892,7 +2892,9 @@ int prepare_device()
     };
     for (const void *k : as_kernels)
         TW_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
-    const int rst = prepare_rm();
+    int rst = prepare_rm();
+    if (rst == TW_OK)
+        rst = prepare_cell();
     if (rst != TW_OK)
         return rst;
     void *p = nullptr;

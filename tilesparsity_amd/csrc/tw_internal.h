@@ -198,6 +198,7 @@ int rm_groups(const tw_plan *p);
 bool rm_takes(const tw_plan *p, int M, int64_t lda);
 int launch_rm(const tw_plan *p, const GemmArgs &a, hipStream_t s);
 int prepare_rm();
+int prepare_cell(); // the LSTM kernels' set-up per device
 // the kernel that takes a row-major A and a row-major C as they are, ahead of copies around a K-major one; NONE: none does
 enum class RowMajor { NONE, STREAM, SKINNY, PANEL };
 RowMajor row_major_kernel(const tw_plan *p, int M, int64_t lda, float beta);
