@@ -1,4 +1,4 @@
-"""Build recipe of libtwgemm.so (HIP, gfx950 only) and of the C++ perf driver.
+"""Build recipe of libtwgemm.so (HIP, gfx950 only), of the module that calls it from Python's inner loops, and of the C++ perf driver.
 
     python -m tilesparsity_amd.build            # compile everything in-tree
 
@@ -8,12 +8,14 @@ file so that it travels with the source tree.
 import os
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libtwgemm.so")
 PERF_PATH = os.path.join(PKG_DIR, "test_basic_nn")
+CALL_PATH = os.path.join(PKG_DIR, "_twcall.so")  # the calls of an inner loop, for twgemm.py
 
 SOURCES = ["tw_host.cpp", "tw_plan.hip", "tw_gemm.hip", "tw_gemm_bs.hip", "tw_gemm_rm.hip", "tw_prune.hip", "tw_cell.hip", "tw_layout.hip", "tw_side.hip"]
 
@@ -86,8 +88,18 @@ def build_perf_driver(verbose=False):
     return PERF_PATH
 
 
+def build_call_module(verbose=False):
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", os.path.join(ROOT, "include"),
+           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "tw_call.cpp"), "-o", CALL_PATH]
+    if verbose:
+        print(" ".join(cmd))
+    _run(cmd)
+    return CALL_PATH
+
+
 def build_all(verbose=False, force=True):
     build_library(verbose, force)
+    build_call_module(verbose)
     build_perf_driver(verbose)
 
 

@@ -77,6 +77,13 @@ MASKS_READY = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.py_object)
 _lib = None
 
 
+def _call_gemm(*args):
+    """Until the library is loaded: the call goes through ctypes, which loads it."""
+
+
+_call_lstm_step = _call_gemm
+
+
 def _share_torch_hip_runtime():
     """A process must hold ONE HIP runtime.  PyTorch wheels bundle their own
     libamdhip64 (same soname as the system one); if it is loaded after the system copy
@@ -188,6 +195,14 @@ def lib():
         fn = getattr(L, name)
         fn.restype = res
         fn.argtypes = args
+    try:
+        from tilesparsity_amd import _twcall
+    except ImportError as e:
+        raise ImportError("%s: build it with `python -m tilesparsity_amd.build`" % e)
+    _twcall.bind(*(ctypes.cast(getattr(L, name), vp).value
+                   for name in ("tw_gemm_ex", "tw_gemm_static", "tw_gemm_staged", "tw_lstm_step")))
+    global _call_gemm, _call_lstm_step
+    _call_gemm, _call_lstm_step = _twcall.gemm, _twcall.lstm_step
     _lib = L
     return L
 
@@ -304,6 +319,7 @@ class Plan:
 
     def __init__(self, handle, K, N, dtype):
         self._h = ctypes.c_void_p(handle)
+        self._at = self._h.value  # (the same as an int, None once destroyed)
         self.K, self.N, self.dtype = K, N, dtype
 
     # -- constructors
@@ -422,7 +438,14 @@ class Plan:
         """One LSTM time step on K-major device buffers (see tw_lstm_step): the gate GEMM of this
         plan (N = 4H) and the cell arithmetic in one launch where the plan allows it, else
         tw_gemm_ex into `gates_ptr` followed by tw_lstm_gates."""
-        vp = ctypes.c_void_p
+        st = _call_lstm_step(self._at, A_ptr, M if lda is None else lda, M, bias_ptr, forget_bias, c_prev_ptr,
+                             M if ldc_prev is None else ldc_prev, c_new_ptr, M if ldc_new is None else ldc_new, h_new_ptr,
+                             M if ldh is None else ldh, gates_ptr, M if ldg is None else ldg, stream)
+        if st is not None:
+            if st:
+                _check(st)
+            return
+        vp = ctypes.c_void_p  # (arguments that are no plain ints, floats or None)
         ld = lambda v: M if v is None else v
         _check(lib().tw_lstm_step(self._h, vp(int(A_ptr or 0)), ld(lda), M, vp(int(bias_ptr or 0)),
                                   forget_bias, vp(int(c_prev_ptr or 0)), ld(ldc_prev),
@@ -517,7 +540,13 @@ class Plan:
             lda = M if a_layout == KMAJOR else self.K
         if ldc is None:
             ldc = M if c_layout == KMAJOR else self.N
-        if workspace_ptr is not None:
+        st = _call_gemm(self._at, A_ptr, a_layout, lda, C_ptr, c_layout, ldc, M, alpha, beta, pruned_cols, stream, bias_ptr,
+                        activation, static, workspace_ptr, workspace_bytes)
+        if st is not None:
+            if st:
+                _check(st)
+            return
+        if workspace_ptr is not None:  # (arguments that are no plain ints, floats, truth values or None)
             ep = Epilogue(ctypes.c_void_p(int(bias_ptr or 0)), int(activation))
             _check(lib().tw_gemm_staged(self._h, ctypes.c_void_p(int(A_ptr or 0)), a_layout, lda,
                                         ctypes.c_void_p(int(C_ptr or 0)), c_layout, ldc, M, alpha, beta,
@@ -539,7 +568,7 @@ class Plan:
     def destroy(self):
         if self._h is not None and self._h.value:
             lib().tw_plan_destroy(self._h)
-        self._h = None
+        self._h = self._at = None
 
     def __del__(self):
         try:
