@@ -510,9 +510,11 @@ __global__ void __launch_bounds__(kListThreads)
 
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-// Device memory of plans and of builds.  The runtime hands out and takes back pieces of up to a
-// megabyte in half a microsecond, but maps and unmaps larger ones anew: 25 us for a hipMalloc of 4 MB,
-// 20 - 240 for its hipFree.  Those are kept here when they are given back, up to kPoolBytes a process,
+// Device memory of plans and of builds.  The runtime maps and unmaps pieces of more than a megabyte anew (25 us for a hipMalloc of 4 MB,
+// 20 - 240 for its hipFree), and hipFree waits for the device whatever the size: a program that replaces its plans and has
+// products of the new ones on their way stood there until they had run (14 VGG16 layers, masks, plans and first products
+// 1027 us a pass with pieces of up to a megabyte left to the runtime, 873 this way).  So they are kept here when they are given back, up to
+// kPoolBytes and kPoolPieces a process,
 // and go to the next that asks for about as much on that device; what does not fit is freed, and all
 // of it when an allocation fails or the host program asks for it (tw_release_memory).  Kernels of a plan that is destroyed may still be queued, on any
 // stream or in a graph: its piece is handed out again only behind a wait for the whole device, made by
@@ -521,12 +523,12 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // in the process, whichever thread and mode it was begun in, and another thread may be capturing while
 // this one builds.  hipFree waits for the device as well, by contract, and leaves the captures of other
 // threads (and relaxed ones) alone, so the wait is the freeing of a small piece.
-constexpr size_t kPoolFrom = 1 << 20, kPoolBytes = 256u << 20;
+constexpr size_t kPoolBytes = 256u << 20, kPoolPieces = 512;
 class DevicePool {
 public:
     void *get(size_t bytes, int device)
     {
-        if (bytes > kPoolFrom) {
+        {
             std::unique_lock<std::mutex> lock(mu_);
             size_t best = free_.size();
             for (size_t i = 0; i < free_.size(); ++i)
@@ -560,10 +562,8 @@ public:
             if (hipMalloc(&p, bytes) != hipSuccess)
                 return nullptr;
         }
-        if (bytes > kPoolFrom) {
-            std::lock_guard<std::mutex> lock(mu_);
-            used_[p] = bytes;
-        }
+        std::lock_guard<std::mutex> lock(mu_);
+        used_[p] = bytes;
         return p;
     }
     // `device` is p's; no kernel uses `p` any more, or (idle == false) what is queued on the device may
@@ -582,7 +582,7 @@ public:
         }
         if (bytes) {
             std::lock_guard<std::mutex> lock(mu_);
-            if (held_ + bytes <= kPoolBytes) {
+            if (held_ + bytes <= kPoolBytes && free_.size() < kPoolPieces) {
                 free_.push_back(Piece{p, bytes, device, idle, waits_});
                 held_ += bytes;
                 return;
