@@ -357,6 +357,44 @@ def test_1d_mix_in_one_call(twprune, po, granularity, values):
             assert b.max() <= 1
 
 
+@pytest.mark.parametrize("granularity", [4, 100, 128])
+@pytest.mark.parametrize("values", ["normal", "tiny", "huge", "no_numbers"])
+def test_mix_bracket_of_whole_fours(twprune, granularity, values):
+    """Four neighbours in one row of one tile (no layer asks for the kernel that looks at two), items in vectors and
+    without, and scores that the bracket is compared with as bits: below and above the range where sqrt(x x) is |x| again,
+    infinite ones and NaNs, which rank above everything and are in no mask.  The expectation is NumPy's float32 arithmetic on the
+    masks of the first stage."""
+    import torch
+    rng = np.random.default_rng(47)
+    scores = [np.abs(rng.standard_normal(s)).astype(np.float32) for s in ((512, 384), (577, 300), (64, 1000), (9, 8))]
+    with np.errstate(all="ignore"):
+        if values == "tiny":
+            scores = [(x * 10.0 ** rng.integers(-26, -16, x.shape)).astype(np.float32) for x in scores]
+        elif values == "huge":
+            scores = [(x * 10.0 ** rng.integers(16, 22, x.shape)).astype(np.float32) for x in scores]
+        elif values == "no_numbers":
+            for x in scores[:3]:
+                at = rng.permutation(x.size)[:60]
+                x.reshape(-1)[at[:30]], x.reshape(-1)[at[30:]] = np.inf, np.nan
+    dev = [torch.from_numpy(x).cuda() for x in scores]
+    for sp, g1 in ((75, 5), (60, 1), (50, 40)):
+        first = twprune.tiled_wise_1d(dev, sp + g1 if sp + g1 <= 100 else 100, granularity, return_device=True)
+        masks = [m.cpu().numpy() != 0 for m in first]
+        with np.errstate(all="ignore"):
+            own = [np.sqrt(x * x) - m.astype(np.float32) for x, m in zip(scores, masks)]
+            s = np.sort(np.concatenate([v.reshape(-1) for v in own]))  # (NaNs last)
+            virt = np.float32(s.size - 1) * (np.float32(100 - g1) / np.float32(100))
+            k = int(np.floor(virt))
+            g, a, b = np.float32(virt - np.floor(virt)), s[k], s[k + 1]
+            thr = b - (b - a) * (np.float32(1) - g) if g >= 0.5 else a + (b - a) * g
+            want = [m | (v > thr) for m, v in zip(masks, own)]
+        for got in (twprune.tiled_wise_1d_mix(dev, sp, granularity, g1, return_device=True),
+                    twprune.tw_mix_fn(dev, g1, first, return_device=True)):
+            assert np.array_equal(np.float64(thr), np.float64(twprune.tw_mix_fn.last_threshold), equal_nan=True), (sp, g1)
+            for x, y in zip(want, got):
+                assert np.array_equal(x.astype(np.uint8), y.cpu().numpy()), (sp, g1, x.shape)
+
+
 @pytest.mark.parametrize("K,N,granularity", [(5, 1 << 21, 128), (5, 1 << 21, 3), (4, (1 << 21) - 1, 3), (4, (1 << 21) - 2, 3),
                                              (3, (1 << 21) + 8, 128), (1 << 23, 4, 4), (1 << 23, 3, 2), ((1 << 23) + 1, 4, 4),
                                              (1 << 23, 64, 1)])

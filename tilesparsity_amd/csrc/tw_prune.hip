@@ -42,6 +42,20 @@ template <bool ONCE, class T> __device__ __forceinline__ T load_global(TW_GLOBAL
         return *p;
 }
 
+// An entry, the same for all lanes, of a table that nobody writes while the kernel runs, through the scalar cache.  (In a kernel that
+// stores, the compiler takes the vector path for it, and the wait for it there is one for every load in flight.)
+template <class T> __device__ __forceinline__ T load_entry(const T *p)
+{
+    struct Words {
+        uint32_t w[sizeof(T) / 4];
+    } a;
+    const auto *const src = (const __attribute__((address_space(4))) uint32_t *)(uintptr_t)p;
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i)
+        a.w[i] = src[i];
+    return __builtin_bit_cast(T, a);
+}
+
 // NumPy's pairwise sum of the squares of n <= 128 terms, by a group of 8 adjacent lanes: lane j keeps
 // NumPy's running sum r[j] (terms j, j+8, j+16, ...), the three shuffle steps are NumPy's
 // ((r0+r1)+(r2+r3)) + ((r4+r5)+(r6+r7)), lane 0 then adds the n % 8 trailing terms.  The result
@@ -400,6 +414,7 @@ __device__ __forceinline__ float key_to_float(uint32_t key)
 // worked out of the histogram by every workgroup of the next pass, and the threshold out of the
 // last one by whatever uses it (threshold_of).
 constexpr int kSelBins = 2048;
+constexpr uint32_t kNanFrom = 0x7F800001u; // |x| from here on is no number
 struct SelectHead {               // the wanted rank and the interpolation above it
     int64_t n;                    // number of values
     unsigned long long rank0;     // 0-based rank of the wanted value
@@ -417,6 +432,7 @@ struct SelectState {
     uint32_t min_gt;              // smallest key above the group the passes so far narrowed down to (0xFFFFFFFF: none)
     // mixed masks: the selection first narrows the elements down to those between two values
     float lo, hi;                 // the bracket
+    uint32_t cut[2][2];           // of an element without and with a mask byte: the first |x| whose score is inside it, the first beyond (as bits)
     uint32_t room;                // values inside it that a wave can keep aside
     uint32_t key_base;            // the passes' digits are those of key - key_base,
     int32_t key_bits;             // which has this many bits (up to 22: two passes hold them all, the third has nothing to do)
@@ -457,6 +473,8 @@ __device__ void select_begin(SelectState *st, int64_t n, double q, int q_is_f64)
     st->min_gt = 0xFFFFFFFFu;
     st->lo = -INFINITY;
     st->hi = INFINITY;
+    st->cut[0][0] = st->cut[1][0] = 0;
+    st->cut[0][1] = st->cut[1][1] = kNanFrom;
     st->key_base = 0;
     st->key_bits = 32;
 }
@@ -548,6 +566,12 @@ struct Threshold {
     bool f64;
     bool lost; // no value had the wanted rank
     __device__ bool passed_by(float v) const { return f64 ? (double)v > v64 : v > v32; }
+    // the float that the same floats are above
+    __device__ float in_float() const
+    {
+        const float near = (float)v64;
+        return !f64 ? v32 : (double)near > v64 ? nextafterf(near, -INFINITY) : near;
+    }
 };
 
 // NumPy's two-sided linear interpolation between the k-th smallest value a and its upper
@@ -1241,7 +1265,9 @@ struct MixLayer {
 
 // Where the mask bytes of the elements come from: the caller's masks; the norms of the tiles' rows and
 // their threshold, for masks that nobody has written yet; a bit each that the narrowing pass has left.
-enum MixSource { MIX_BYTES, MIX_NORMS, MIX_BITS };
+// MIX_SPLIT: norms where four elements that are worked off together can lie in two tiles or rows (a kernel of its own, since a load on a
+// condition is waited for on the spot).
+enum MixSource { MIX_BYTES, MIX_NORMS, MIX_SPLIT, MIX_BITS };
 
 // ||x|| of a single element (sqrt(x*x) / 1, the reference's norm over a tile of one column) minus 1
 // where the TW mask already keeps it (prune_algo.py:159-161).  The square root of a rounded square
@@ -1261,8 +1287,8 @@ __device__ __forceinline__ float mix_value(float x, uint32_t m0)
 // The kernels of the mixed producer walk items of 4096 consecutive elements of a layer, sixteen per
 // thread, as vectors where the layer allows it.  The element scores are worked
 // out anew from weight and mask wherever they are needed rather than written to a pool and read back.  At
-// four or five bytes an element the vector instructions count as much as the memory: a dozen per element
-// are 10 us for 31.5 M elements.
+// four or five bytes an element the vector instructions count as much as the memory: ten per element
+// are 8 us for 31.5 M elements.
 constexpr int kMixItem = 4096;
 struct MixFetched {
     TW_GLOBAL(const float) sc;
@@ -1271,12 +1297,11 @@ struct MixFetched {
     int n;
     bool vec;
     float4 x[4];
-    uint32_t m[4];   // mask bytes, any value but 0 counting as 1 (MIX_NORMS: how many of the four have the first norm)
-    float nv[4][2];  // MIX_NORMS: the norm of the first and of the last of four elements
+    uint32_t m[4];   // mask bytes, any value but 0 counting as 1 (MIX_SPLIT: how many of the four have the first norm)
+    float nv[4][2];  // MIX_NORMS: the norm of four elements; MIX_SPLIT: of the first and of the last
     uint32_t bits;   // MIX_BITS: the thread's sixteen elements
     const MixLayer *layer;
     int64_t e0;      // the item's first element
-    bool split;      // MIX_NORMS: four elements can lie in two tiles or rows
 };
 __device__ __forceinline__ bool mix_in_vectors(const MixLayer &L, int64_t e0) { return L.in_fours && L.n - e0 >= kMixItem; }
 // Layers whose elements are placed in rows and tiles with a multiplication in float: (x + 0.5) / N is off by less than
@@ -1314,8 +1339,9 @@ struct MixCell {
     __device__ uint32_t norm(const MixLayer &L, uint32_t t) const { return __umul24(t, (uint32_t)L.K) + k; }
 };
 template <int SRC>
-__device__ __forceinline__ void mix_fetch(const MixLayer &L, int64_t item, const uint16_t *bits, const float *safe, MixFetched &d)
+__device__ __forceinline__ void mix_fetch(const MixLayer *layer, int64_t item, const uint16_t *bits, const float *safe, MixFetched &d)
 {
+    const MixLayer L = load_entry(layer);
     const int64_t e0 = (item - L.item_begin) * kMixItem;
     d.n = (int)min((int64_t)kMixItem, L.n - e0);
     d.sc = as_global(L.score) + e0;
@@ -1336,28 +1362,25 @@ __device__ __forceinline__ void mix_fetch(const MixLayer &L, int64_t item, const
     } else if constexpr (SRC == MIX_BITS) {
         d.bits = as_global(bits)[item * 256 + threadIdx.x];
     } else {
-        d.layer = &L;
+        d.layer = layer;
         d.e0 = e0;
-        d.split = L.in_fours != 2;
         TW_GLOBAL(const float) const nm = as_global(L.norms);
         MixCell p(L, e0, d.vec ? threadIdx.x * 4 : 0u);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const uint32_t t = p.tile(L), at = p.norm(L, t);
+            const uint32_t t = p.tile(L), at = d.vec ? p.norm(L, t) : 0u; // (no branch: any norm will do)
             d.nv[i][0] = nm[at];
-            if (d.split) {
+            if constexpr (SRC == MIX_SPLIT) {
                 const uint32_t end = min((t + 1) * (uint32_t)L.G, (uint32_t)L.N); // of the tile
                 d.m[i] = min(end - p.c, 4u);
                 d.nv[i][1] = nm[d.vec && d.m[i] < 4 ? (end == (uint32_t)L.N ? p.k + 1 : at + L.K) : at];
             }
-            if (d.vec && i < 3)
-                p.on_1024(L);
+            p.on_1024(L);
         }
     }
 }
-// f(values, mask bytes, output, count, place) per four (or single) elements; `place` and what is in sixty-fourths of it
-// tell the first one's place among the wave's elements of the item (see mix_place)
-template <int SRC, class F> __device__ __forceinline__ void mix_apply(const MixFetched &d, const Threshold &rows, F f)
+// MIX_BITS: f(values, mask bytes, output, count) per four (or single) elements
+template <class F> __device__ __forceinline__ void mix_apply(const MixFetched &d, F f)
 {
     if (d.vec) {
         float ax[4][4];
@@ -1388,41 +1411,17 @@ template <int SRC, class F> __device__ __forceinline__ void mix_apply(const MixF
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             float v[4];
-            uint32_t m;
-            if constexpr (SRC == MIX_NORMS) {
-                const bool in = rows.passed_by(d.nv[i][0]);
-                m = in ? 0x01010101u : 0u;
-                if (d.split) {
-                    const uint32_t first = (uint32_t)((1ull << (d.m[i] * 8)) - 1ull); // bytes of the first tile
-                    m = (m & first) | (rows.passed_by(d.nv[i][1]) ? ~first & 0x01010101u : 0u);
-                }
-            } else if constexpr (SRC == MIX_BITS) {
-                m = ((d.bits >> (i * 4) & 15u) * 0x204081u) & 0x01010101u;
-            } else {
-                m = d.m[i];
-            }
+            const uint32_t m = ((d.bits >> (i * 4) & 15u) * 0x204081u) & 0x01010101u;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) { // (the mask byte, any value but 0 counting as 1)
-                const float one = (float)(m >> (e * 8) & 255u);
-                v[e] = ax[i][e] - (SRC == MIX_BYTES ? fminf(one, 1.0f) : one);
-            }
-            f(v, m, d.out + (threadIdx.x + i * 256) * 4, 4, i << 8);
+            for (int e = 0; e < 4; ++e)
+                v[e] = ax[i][e] - (float)(m >> (e * 8) & 255u);
+            f(v, m, d.out + (threadIdx.x + i * 256) * 4, 4);
         }
     } else {
-        // (whole waves make every round: f may look at its wave)
-        for (int i0 = 0; i0 < d.n; i0 += 256) {
-            const int i = i0 + (int)threadIdx.x, j = min(i, d.n - 1);
-            uint32_t m0;
-            if constexpr (SRC == MIX_NORMS) {
-                const MixCell p(*d.layer, d.e0, (uint32_t)j);
-                m0 = rows.passed_by(as_global(d.layer->norms)[p.norm(*d.layer, p.tile(*d.layer))]) ? 1u : 0u;
-            } else if constexpr (SRC == MIX_BITS) {
-                m0 = d.bits >> (i0 >> 8) & 1u;
-            } else {
-                m0 = d.mk[j];
-            }
-            float v[4] = {mix_value(d.sc[j], m0), 0.0f, 0.0f, 0.0f};
-            f(v, m0, d.out + j, i < d.n ? 1 : 0, i0 >> 2);
+        for (int i = (int)threadIdx.x, slot = 0; i < d.n; i += 256, ++slot) {
+            const uint32_t m0 = d.bits >> slot & 1u;
+            const float v[4] = {mix_value(d.sc[i], m0), 0.0f, 0.0f, 0.0f};
+            f(v, m0, d.out + i, 1);
         }
     }
 }
@@ -1434,28 +1433,26 @@ __device__ __forceinline__ int mix_place(bool vec, int wave, uint32_t code)
     return vec ? (thread + (int)(code >> 8 & 3u) * 256) * 4 + (int)(code >> 6 & 3u) : (int)(code >> 6 & 15u) * 256 + thread;
 }
 // All items of a launch, shared out over its workgroups, the next item's loads in flight while one is
-// worked on.  done(item) after every item;
-// bits: MIX_BITS; safe: 16 KB of device memory that can be read; rows(): MIX_NORMS, asked for once, after the first loads.
-template <int SRC, class R, class F, class D>
+// worked on: work(item, what was fetched for it).
+// bits: MIX_BITS; safe: 16 KB of device memory that can be read; fetched(): once, after the first loads.
+template <int SRC, class R, class F>
 __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layers, int64_t n_items, const uint16_t *bits, const float *safe,
-                                             R rows_of, F f, D done)
+                                             R fetched, F work)
 {
     const LayerFinder find(&layers->item_begin, sizeof(MixLayer), n_layers);
     MixFetched a, b;
     const int64_t step = gridDim.x, last = n_items - 1;
     int64_t item = blockIdx.x; // (a launch has at most n_items workgroups)
-    mix_fetch<SRC>(layers[find(item)], item, bits, safe, a);
-    const Threshold rows = rows_of();
+    mix_fetch<SRC>(layers + find(item), item, bits, safe, a);
+    fetched();
     for (;;) {
         const int64_t i1 = min(item + step, last), i2 = min(item + 2 * step, last);
-        mix_fetch<SRC>(layers[find(i1)], i1, bits, safe, b);
-        mix_apply<SRC>(a, rows, f);
-        done(item);
+        mix_fetch<SRC>(layers + find(i1), i1, bits, safe, b);
+        work(item, a);
         if (item + step > last)
             break;
-        mix_fetch<SRC>(layers[find(i2)], i2, bits, safe, a);
-        mix_apply<SRC>(b, rows, f);
-        done(item + step);
+        mix_fetch<SRC>(layers + find(i2), i2, bits, safe, a);
+        work(item + step, b);
         item += 2 * step;
         if (item > last)
             break;
@@ -1472,7 +1469,7 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // elements.  The narrowing pass also writes the masks: what lies outside the bracket is decided
 // already, and the few per cent inside are marked one by one when the threshold is known, from the places kept
 // beside their values.
-// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 40 + 26 + 10 us; with those masks
+// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 33 + 26 + 10 us; with those masks
 // written and read and the elements read once more at the end 13 + 4 + 11 + 31 + 31 + 32, and the host's wait between the stages.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
@@ -1571,9 +1568,28 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
         const unsigned long long at = ((unsigned long long)both + w) << range.shift[1];
         edge[w] = inside[w] ? (uint32_t)min((unsigned long long)range.base + at - w, 0xFFFFFFFFull) : w ? 0xFFFFFFFFu : 0u;
     }
+    const float lo = edge[0] == 0u ? -INFINITY : key_to_float(edge[0]);
+    const float hi = edge[1] == 0xFFFFFFFFu ? INFINITY : key_to_float(edge[1]);
     if (tid == 0) {
-        st->lo = edge[0] == 0u ? -INFINITY : key_to_float(edge[0]);
-        st->hi = edge[1] == 0xFFFFFFFFu ? INFINITY : key_to_float(edge[1]);
+        st->lo = lo;
+        st->hi = hi;
+    }
+    // (a score grows with |x|: which |x| are inside is one range for elements without a mask byte and one for those with.  A wave looks for
+    // one end of one of them, 64 places at a time)
+    const int wave = tid >> 6, lane = tid & 63;
+    if (wave < 4) {
+        const uint32_t m0 = wave & 1;
+        auto from = [&](uint32_t u) {
+            const float v = mix_value(__uint_as_float(u), m0);
+            return u >= kNanFrom || !(wave >> 1 ? v <= hi : v < lo);
+        };
+        uint32_t first = 0;
+#pragma unroll 1
+        for (int s = 25; s >= 1; s -= 6)
+            first += (uint32_t)__popcll(__ballot(!from(first + ((uint32_t)(lane + 1) << s) - 1u))) << s;
+        first += (uint32_t)__popcll(__ballot(lane < 2 && !from(first + lane)));
+        if (lane == 0)
+            st->cut[m0][wave >> 1] = first;
     }
 }
 
@@ -1583,6 +1599,9 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
 // kernel, one per wave 90).  The masks leave with it, as if nothing between were above the threshold; and a bit for
 // each element's mask0, which nobody can read any more where the masks are written in place, should the
 // bracket have missed.
+// The 31.5 M elements of VGG16 with masks out of norms 39 -> 33 us: reading them takes 22 (5.7 TB/s), the norms of their rows 2, the
+// threshold of those norms 3, the masks 3 and the candidates 3; before, every item waited for the next one's loads (its layer's entry
+// and conditional loads of norms behind them), and 29 vector instructions an element were 24 us of every SIMD's time (17 now).
 constexpr int kMixWgs = 1024, kMixWaves = kMixWgs * 4; // most workgroups and waves of a pass over the elements
 struct MixCounts {
     uint32_t between, below;
@@ -1593,52 +1612,113 @@ __global__ void __launch_bounds__(256, 4)
                       MixCounts *counts, uint16_t *bits, Mail *mail)
 {
     const float lo = st->lo, hi = st->hi;
+    const uint32_t in0 = st->cut[0][0], up0 = st->cut[0][1], in1 = st->cut[1][0], up1 = st->cut[1][1];
     const uint32_t room = st->room;
     const int lane = (int)(threadIdx.x & 63);
     const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     TW_GLOBAL(u32x2) const keep = as_global(cand) + (int64_t)w * room;
     __shared__ __align__(16) float s_v[kMixItem];
-    uint32_t kept = 0, below = 0, round = 0; // wave-uniform
+    constexpr uint32_t kFrom = 0x22000000u, kTo = 0x5D000000u; // 2^-59 and 2^59, as bits
+    const bool plain = min(in0, in1) >= kFrom && max(up0, up1) <= kTo; // every candidate is: see mix_plain
+    static_assert(kMixPlainMin < 0x1p-59f && kMixPlainMax > 0x1p59f, "within mix_plain's");
+    uint32_t kept = 0, round = 0;            // wave-uniform
+    uint32_t below = 0;                      // of the lane's elements
     uint32_t mine = 0, inside = 0;           // mask0 of the thread's sixteen elements of the item; which are candidates
+    float rows = 0.0f;
     auto rows_of = [&]() {
-        if constexpr (SRC == MIX_NORMS) {
+        if constexpr (SRC != MIX_BYTES) {
             const Threshold t = threshold_of<256>(st_rows);
             if (blockIdx.x == 0 && threadIdx.x == 0 && t.lost)
                 mail->lost = 1;
-            return t;
-        } else {
-            return Threshold{};
+            rows = t.in_float();
         }
     };
-    auto narrow = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt, int at0) {
-        const int slot = at0 >> 6; // of the thread's sixteen
-        float *const sv = s_v + ((slot >> 2) * 256 + (int)threadIdx.x) * 4;
-        if (cnt == 4) {
-            *reinterpret_cast<float4 *>(sv) = float4{v[0], v[1], v[2], v[3]};
-            uint32_t in = 0, over = 0; // a bit an element, the last one lowest
+    // Sixteen elements of a thread: |x|, as whole numbers, against the two ends of the bracket for an element of its kind.  A bit of
+    // two registers for each, the last element first, and everything else out of those.
+    auto narrow = [&](const MixFetched &d) {
+        if (d.vec) {
+            uint32_t mask[4], under_in = 0, under_up = 0, top = 0;
+            mine = 0;
+            auto test = [&](float x, uint32_t in, uint32_t up) { // (all three below 2^31: the difference's sign)
+                const uint32_t u = __float_as_uint(x) & 0x7FFFFFFFu;
+                under_in = __builtin_amdgcn_alignbit(under_in, u - in, 31);
+                under_up = __builtin_amdgcn_alignbit(under_up, u - up, 31);
+                top = max(top, u);
+            };
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                below += __popcll(__ballot(v[e] < lo));
-                in = in + in + (v[e] >= lo && v[e] <= hi ? 1u : 0u);
-                over = over + over + (v[e] > hi ? 1u : 0u);
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<float4 *>(s_v + (i * 256 + (int)threadIdx.x) * 4) = d.x[i];
+            if constexpr (SRC == MIX_NORMS) { // four elements of one kind
+#pragma unroll
+                for (int i = 3; i >= 0; --i) {
+                    const bool row = d.nv[i][0] > rows;
+                    const uint32_t in = row ? in1 : in0, up = row ? up1 : up0;
+                    mask[i] = row ? 0x01010101u : 0u;
+                    mine = mine << 4 | (row ? 15u : 0u);
+                    test(d.x[i].w, in, up);
+                    test(d.x[i].z, in, up);
+                    test(d.x[i].y, in, up);
+                    test(d.x[i].x, in, up);
+                }
+            } else {
+#pragma unroll
+                for (int i = 3; i >= 0; --i) {
+                    uint32_t m;
+                    if constexpr (SRC == MIX_SPLIT) {
+                        const uint32_t first = (uint32_t)((1ull << (d.m[i] * 8)) - 1ull); // bytes of the first tile
+                        m = (d.nv[i][0] > rows ? first & 0x01010101u : 0u) | (d.nv[i][1] > rows ? ~first & 0x01010101u : 0u);
+                    } else {
+                        m = ((d.m[i] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu | d.m[i]) >> 7 & 0x01010101u; // mask bytes that are not 0
+                    }
+                    mask[i] = m;
+                    mine = mine << 4 | m * 0x10204080u >> 28;
+                    const float x[4] = {d.x[i].x, d.x[i].y, d.x[i].z, d.x[i].w};
+#pragma unroll
+                    for (int e = 3; e >= 0; --e) {
+                        const bool one = m >> (e * 8) & 1u;
+                        test(x[e], one ? in1 : in0, one ? up1 : up0);
+                    }
+                }
             }
-            inside |= (__brev(in) >> 28) << slot;
-            const uint32_t o = SRC == MIX_NORMS ? m : ((m & 0x7F7F7F7Fu) + 0x7F7F7F7Fu | m) >> 7 & 0x01010101u; // mask bytes that are not 0
-            mine |= (o * 0x10204080u >> 28) << slot;
-            *(TW_GLOBAL(uint32_t))out = o | (((__brev(over) >> 28) * 0x204081u) & 0x01010101u);
+            below += (uint32_t)__popc(under_in);
+            inside = under_up & ~under_in;
+            uint32_t above = ~under_up;
+            if (top >= kNanFrom) { // (what is no number is neither below nor inside nor above)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float x[4] = {d.x[i].x, d.x[i].y, d.x[i].z, d.x[i].w};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        above &= ~((x[e] != x[e] ? 1u : 0u) << (i * 4 + e));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                *(TW_GLOBAL(uint32_t))(d.out + (threadIdx.x + i * 256) * 4) = mask[i] | __umul24(above >> (i * 4) & 15u, 0x204081u) & 0x01010101u;
         } else {
-            sv[slot & 3] = v[0];
-            below += __popcll(__ballot(cnt && v[0] < lo));
-            inside |= (cnt && v[0] >= lo && v[0] <= hi ? 1u : 0u) << slot;
-            mine |= (m ? 1u : 0u) << slot;
-            if (cnt)
-                *as_global(out) = m || v[0] > hi ? 1 : 0;
+            mine = inside = 0;
+            for (int i = (int)threadIdx.x, slot = 0; i < d.n; i += 256, ++slot) {
+                uint32_t m0;
+                if constexpr (SRC != MIX_BYTES) {
+                    const MixCell p(*d.layer, d.e0, (uint32_t)i);
+                    m0 = as_global(d.layer->norms)[p.norm(*d.layer, p.tile(*d.layer))] > rows ? 1u : 0u;
+                } else {
+                    m0 = d.mk[i] ? 1u : 0u;
+                }
+                const float x = d.sc[i], v = mix_value(x, m0);
+                s_v[((slot >> 2) * 256 + (int)threadIdx.x) * 4 + (slot & 3)] = x;
+                below += v < lo ? 1u : 0u;
+                inside |= (v >= lo && v <= hi ? 1u : 0u) << slot;
+                mine |= m0 << slot;
+                as_global(d.out)[i] = m0 || v > hi ? 1 : 0;
+            }
         }
     };
     // The candidates of an item, one of every lane that has one left at a time: a lane has half of one among its
-    // sixteen elements, so that three or four rounds do for sixteen tests and as many stores (42 us for the 31.5 M elements
-    // of VGG16 with masks out of norms, 46 with a test behind each element).
-    auto item_done = [&](int64_t item) {
+    // sixteen elements, so that three or four rounds do for sixteen tests and as many stores (4 us less than a test behind each of
+    // VGG16's 31.5 M elements).
+    auto work = [&](int64_t item, const MixFetched &d) {
+        narrow(d);
         for (;;) {
             const bool some = inside != 0;
             const unsigned long long in = __ballot(some);
@@ -1646,16 +1726,21 @@ __global__ void __launch_bounds__(256, 4)
                 break;
             const uint32_t slot = some ? (uint32_t)__builtin_ctz(inside) : 0u;
             const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, kept));
-            if (some && at < room) // (the count tells of an overflow)
-                keep[at] = u32x2{__float_as_uint(s_v[((slot >> 2) * 256 + threadIdx.x) * 4 + (slot & 3)]), round << 10 | slot << 6 | (uint32_t)lane};
+            if (some && at < room) { // (the count tells of an overflow)
+                const float x = s_v[((slot >> 2) * 256 + threadIdx.x) * 4 + (slot & 3)];
+                const uint32_t one = mine >> slot & 1u;
+                const float v = plain ? fabsf(x) - (float)one : mix_value(x, one);
+                keep[at] = u32x2{__float_as_uint(v), round << 10 | slot << 6 | (uint32_t)lane};
+            }
             kept += __popcll(in);
             inside &= inside - 1;
         }
         as_global(bits)[item * 256 + threadIdx.x] = (uint16_t)mine;
-        mine = 0;
         ++round;
     };
-    mix_for_each<SRC>(layers, n_layers, n_items, nullptr, reinterpret_cast<const float *>(cand), rows_of, narrow, item_done);
+    mix_for_each<SRC>(layers, n_layers, n_items, nullptr, reinterpret_cast<const float *>(cand), rows_of, work);
+    for (int off = 32; off > 0; off >>= 1)
+        below += (uint32_t)__shfl_down((int)below, off);
     if (lane == 0)
         counts[w] = MixCounts{kept, below};
 }
@@ -1776,13 +1861,14 @@ __global__ void __launch_bounds__(256)
             }
         }
     } else {
-        auto count = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt, int) {
+        auto count = [&](const float (&v)[4], uint32_t, uint8_t *, int cnt) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 if (e < cnt)
                     select_count<PASS>(sort_key(v[e]), range, prefix, s_h, mn);
         };
-        mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() { return Threshold{}; }, count, [](int64_t) {});
+        mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() {},
+                               [&](int64_t, const MixFetched &d) { mix_apply(d, count); });
     }
     select_leave<PASS, 256>(st, s_h, &s_min, mn);
 }
@@ -1857,17 +1943,18 @@ __global__ void __launch_bounds__(256)
         }
         return;
     }
-    auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt, int) {
+    auto mark = [&](const float (&v)[4], uint32_t m, uint8_t *out, int cnt) {
         if (cnt == 4) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 m |= thr.passed_by(v[e]) ? 1u << (e * 8) : 0u;
             *(TW_GLOBAL(uint32_t))out = m;
-        } else if (cnt == 1) {
+        } else {
             *as_global(out) = (m || thr.passed_by(v[0])) ? 1 : 0;
         }
     };
-    mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() { return Threshold{}; }, mark, [](int64_t) {});
+    mix_for_each<MIX_BITS>(layers, n_layers, n_items, bits, reinterpret_cast<const float *>(cand), []() {},
+                           [&](int64_t, const MixFetched &d) { mix_apply(d, mark); });
 }
 
 // ---------------------------------------------------------------------------------
@@ -2347,7 +2434,11 @@ public:
                                d_sample_);
             hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample_, d_st_);
         }
-        hipLaunchKernelGGL(mix_narrow_kernel<SRC>, dim3(wgs_), dim3(256), 0, s, d_layers, n_layers, n_items_, st_rows, d_st_, d_cand_,
+        bool split = false;
+        for (const MixLayer &e : layers_)
+            split |= e.in_fours == 1;
+        auto narrow = SRC == MIX_NORMS && split ? mix_narrow_kernel<MIX_SPLIT> : mix_narrow_kernel<SRC>;
+        hipLaunchKernelGGL(narrow, dim3(wgs_), dim3(256), 0, s, d_layers, n_layers, n_items_, st_rows, d_st_, d_cand_,
                            d_counts_, d_bits_, mail);
         const dim3 grid((unsigned)std::min<int64_t>(n_items_, 512));
         hipLaunchKernelGGL(mix_hist_kernel<0>, grid, dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_, d_counts_, waves,
