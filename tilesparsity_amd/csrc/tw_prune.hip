@@ -433,6 +433,7 @@ struct SelectState {
     // mixed masks: the selection first narrows the elements down to those between two values
     float lo, hi;                 // the bracket
     uint32_t cut[2][2];           // of an element without and with a mask byte: the first |x| whose score is inside it, the first beyond (as bits)
+    float row_norm;               // what the norms of kept rows are above (masks out of norms; the sample's kernel leaves it)
     uint32_t room;                // values inside it that a wave can keep aside
     uint32_t key_base;            // the passes' digits are those of key - key_base,
     int32_t key_bits;             // which has this many bits (up to 22: two passes hold them all, the third has nothing to do)
@@ -502,26 +503,63 @@ struct Digit {
     unsigned long long rest, count;
     uint32_t digit, next;
 };
+// Over the lanes of a wave, in registers: a step through LDS (__shfl) is some 60 cycles, and a selection is a chain of them.
+// (row_shr 1, 2, 4, 8 inside rows of 16 lanes, then the last lane of a row to the next row, of the second row to the upper half; a lane
+// that gets nothing keeps `none`)
+template <class F> __device__ __forceinline__ uint32_t wave_steps(uint32_t x, uint32_t none, F f)
+{
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x111, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x112, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x114, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x118, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x142, 0xA, 0xF, false));
+    return f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x143, 0xC, 0xF, false));
+}
+__device__ __forceinline__ uint32_t last_lane(uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, 63); }
+__device__ __forceinline__ uint32_t wave_min(uint32_t x)
+{
+    return last_lane(wave_steps(x, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); }));
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    return last_lane(wave_steps(x, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }));
+}
+// sums over the lanes up to this one
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x)
+{
+    return wave_steps(x, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long x)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        x += (unsigned long long)hi << 32 | lo;
+    };
+    step(std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xA>());
+    step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xC>());
+    return x;
+}
+
+// (T: what the counts are and, counts of a launch's values fitting one or the other, what they add up to)
 template <int NT, int NB, bool NEXT = false, class T> __device__ Digit find_digit(const T *hist, unsigned long long rank)
 {
     constexpr int PER = NB / NT;
-    __shared__ unsigned long long s_wave[NT / 64];
+    __shared__ T s_wave[NT / 64];
     __shared__ Digit s_d;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    T c[PER];
-    unsigned long long sum = 0;
+    T c[PER], sum = 0;
 #pragma unroll
     for (int i = 0; i < PER; ++i)
         c[i] = hist[tid * PER + i];
 #pragma unroll
     for (int i = 0; i < PER; ++i)
         sum += c[i];
-    unsigned long long incl = sum;
-    for (int off = 1; off < 64; off <<= 1) {
-        const unsigned long long up = __shfl_up(incl, off);
-        if (lane >= off)
-            incl += up;
-    }
+    T incl = wave_scan(sum);
     if (lane == 63)
         s_wave[wave] = incl;
     if (tid == 0)
@@ -529,31 +567,26 @@ template <int NT, int NB, bool NEXT = false, class T> __device__ Digit find_digi
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < NT / 64; ++w) // (all of them at once, not one after another)
-        incl += w < wave ? s_wave[w] : 0ull;
-    unsigned long long before = incl - sum;
+        incl += w < wave ? s_wave[w] : 0;
+    T before = incl - sum;
+    uint32_t next = 0xFFFFFFFFu; // the first digit with a value and more than `rank` values before it
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-        if (before <= rank && rank < before + c[i]) { // exactly one digit
+        if (before <= rank && rank < (unsigned long long)before + c[i]) { // exactly one digit
             s_d.digit = tid * PER + i;
             s_d.rest = rank - before;
             s_d.count = c[i];
         }
+        if (NEXT && before > rank && c[i])
+            next = min(next, (uint32_t)(tid * PER + i));
         before += c[i];
     }
-    __syncthreads();
     if (NEXT) { // (one LDS atomic per wave: hundreds on one word take microseconds)
-        const uint32_t digit = s_d.digit;
-        uint32_t next = 0xFFFFFFFFu;
-#pragma unroll
-        for (int i = PER - 1; i >= 0; --i)
-            if (c[i] && (uint32_t)(tid * PER + i) > digit)
-                next = tid * PER + i;
-        for (int off = 32; off > 0; off >>= 1)
-            next = min(next, (uint32_t)__shfl_down(next, off));
-        if (lane == 0)
+        next = wave_min(next);
+        if (lane == 0 && next != 0xFFFFFFFFu)
             atomicMin(&s_d.next, next);
-        __syncthreads();
     }
+    __syncthreads();
     const Digit d = s_d;
     __syncthreads(); // the shared words are written again by the next call
     return d;
@@ -688,8 +721,7 @@ __device__ void select_enter(SelectState *st, const KeyRange &range, unsigned in
 template <int PASS, int NT> __device__ void select_leave(SelectState *st, unsigned int *s_h, uint32_t *s_min, uint32_t mn)
 {
     if (PASS > 0) {
-        for (int off = 32; off > 0; off >>= 1)
-            mn = min(mn, (uint32_t)__shfl_down(mn, off));
+        mn = wave_min(mn);
         if ((threadIdx.x & 63) == 0 && mn != 0xFFFFFFFFu)
             atomicMin(s_min, mn);
     }
@@ -734,10 +766,8 @@ template <class V> __device__ KeyRange key_range_in_block(V each)
         lo = min(lo, k);
         hi = max(hi, k);
     });
-    for (int off = 32; off > 0; off >>= 1) {
-        lo = min(lo, (uint32_t)__shfl_down(lo, off));
-        hi = max(hi, (uint32_t)__shfl_down(hi, off));
-    }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
     if ((threadIdx.x & 63) == 0) {
         atomicMin(&s_lo, lo);
         atomicMax(&s_hi, hi);
@@ -774,8 +804,7 @@ template <int NT, class V> __device__ Threshold select_in_block(V each, const Se
     Digit d = count_in_block<1, NT>(each, range, rank, prefix, s_h, mn);
     if (range.shift[1] > 0) // (else two digits hold all of the range)
         d = count_in_block<2, NT>(each, range, rank, prefix, s_h, mn);
-    for (int off = 32; off > 0; off >>= 1)
-        mn = min(mn, (uint32_t)__shfl_down(mn, off));
+    mn = wave_min(mn);
     if ((threadIdx.x & 63) == 0)
         atomicMin(&s_min, mn);
     __syncthreads();
@@ -910,11 +939,7 @@ __global__ void __launch_bounds__(kPlanThreads)
     }
     // sums over the threads up to this one (modulo 2^32: only differences are used), and over all
     auto scan = [&](uint32_t mine, uint32_t &total) {
-        uint32_t incl = mine;
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t up = __shfl_up(incl, off);
-            incl += lane >= off ? up : 0u;
-        }
+        uint32_t incl = wave_scan(mine);
         if (lane == 63)
             s_sum[wave] = incl;
         __syncthreads();
@@ -1469,13 +1494,13 @@ __device__ __forceinline__ void mix_for_each(const MixLayer *layers, int n_layer
 // elements.  The narrowing pass also writes the masks: what lies outside the bracket is decided
 // already, and the few per cent inside are marked one by one when the threshold is known, from the places kept
 // beside their values.
-// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 6 + 11 + 33 + 26 + 10 us; with those masks
+// Over the elements of VGG16, masks out of norms: sample, bracket, narrowing, passes, marking 5 + 8 + 30 + 23 + 9 us; with those masks
 // written and read and the elements read once more at the end 13 + 4 + 11 + 31 + 31 + 32, and the host's wait between the stages.
 constexpr int kMixSamples = 8192;
 constexpr int64_t kMixSampleFrom = 1 << 17; // fewer elements than this are all kept aside
 template <int SRC>
 __global__ void __launch_bounds__(256)
-    mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, const SelectState *st_rows, uint32_t *sample)
+    mix_sample_kernel(const MixLayer *layers, int n_layers, int64_t total, const SelectState *st_rows, SelectState *st, uint32_t *sample, Mail *mail)
 {
     const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x); // kMixSamples threads
     const int64_t at = total / kMixSamples * i;
@@ -1502,7 +1527,14 @@ __global__ void __launch_bounds__(256)
         else if ((k + 1) * L.N <= j)
             ++k;
         const float norm = as_global(L.norms)[(int64_t)((int)(j - k * L.N) / L.G) * L.K + k];
-        m0 = threshold_of<256>(st_rows).passed_by(norm) ? 1u : 0u;
+        const Threshold t = threshold_of<256>(st_rows);
+        const float rows = t.in_float();
+        m0 = norm > rows ? 1u : 0u;
+        if (i == 0) {
+            st->row_norm = rows;
+            if (t.lost)
+                mail->lost = 1;
+        }
     } else {
         m0 = L.mask0[j];
     }
@@ -1530,7 +1562,7 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
             f(key[i]);
     });
     // both edges out of one count of the first digit and one of the second, with counters for each: an edge is a chain of trips
-    // through LDS and barriers, which is all that this kernel waits for (one edge after the other: 14.6 us, so 11)
+    // through LDS and barriers, which is all that this kernel waits for (one edge after the other: 14.6 us, so 11, and 8 with the steps over a wave's lanes in registers)
     __shared__ unsigned int s_h2[kSelBins];
     bool inside[2];
     uint32_t prefix[2], edge[2];
@@ -1599,8 +1631,8 @@ __global__ void __launch_bounds__(kBracketThreads) mix_bracket_kernel(const uint
 // kernel, one per wave 90).  The masks leave with it, as if nothing between were above the threshold; and a bit for
 // each element's mask0, which nobody can read any more where the masks are written in place, should the
 // bracket have missed.
-// The 31.5 M elements of VGG16 with masks out of norms 39 -> 33 us: reading them takes 22 (5.7 TB/s), the norms of their rows 2, the
-// threshold of those norms 3, the masks 3 and the candidates 3; before, every item waited for the next one's loads (its layer's entry
+// The 31.5 M elements of VGG16 with masks out of norms 39 -> 30 us: reading them takes 22 (5.7 TB/s), the norms of their rows 2, the masks 3
+// and the candidates 3 (and the norms' threshold 3 more where no sample's kernel has left it); before, every item waited for the next one's loads (its layer's entry
 // and conditional loads of norms behind them), and 29 vector instructions an element were 24 us of every SIMD's time (17 now).
 constexpr int kMixWgs = 1024, kMixWaves = kMixWgs * 4; // most workgroups and waves of a pass over the elements
 struct MixCounts {
@@ -1609,7 +1641,7 @@ struct MixCounts {
 template <int SRC>
 __global__ void __launch_bounds__(256, 4)
     mix_narrow_kernel(const MixLayer *layers, int n_layers, int64_t n_items, const SelectState *st_rows, const SelectState *st, u32x2 *cand,
-                      MixCounts *counts, uint16_t *bits, Mail *mail)
+                      MixCounts *counts, uint16_t *bits, Mail *mail, int sampled)
 {
     const float lo = st->lo, hi = st->hi;
     const uint32_t in0 = st->cut[0][0], up0 = st->cut[0][1], in1 = st->cut[1][0], up1 = st->cut[1][1];
@@ -1627,10 +1659,14 @@ __global__ void __launch_bounds__(256, 4)
     float rows = 0.0f;
     auto rows_of = [&]() {
         if constexpr (SRC != MIX_BYTES) {
-            const Threshold t = threshold_of<256>(st_rows);
-            if (blockIdx.x == 0 && threadIdx.x == 0 && t.lost)
-                mail->lost = 1;
-            rows = t.in_float();
+            if (sampled) {
+                rows = st->row_norm;
+            } else {
+                const Threshold t = threshold_of<256>(st_rows);
+                if (blockIdx.x == 0 && threadIdx.x == 0 && t.lost)
+                    mail->lost = 1;
+                rows = t.in_float();
+            }
         }
     };
     // Sixteen elements of a thread: |x|, as whole numbers, against the two ends of the bracket for an element of its kind.  A bit of
@@ -1739,8 +1775,7 @@ __global__ void __launch_bounds__(256, 4)
         ++round;
     };
     mix_for_each<SRC>(layers, n_layers, n_items, nullptr, reinterpret_cast<const float *>(cand), rows_of, work);
-    for (int off = 32; off > 0; off >>= 1)
-        below += (uint32_t)__shfl_down((int)below, off);
+    below = last_lane(wave_scan(below));
     if (lane == 0)
         counts[w] = MixCounts{kept, below};
 }
@@ -1766,12 +1801,10 @@ __device__ bool mix_totals(const MixCounts *counts, int waves, uint32_t room, un
         b += w < waves ? c.below : 0u;
         most = max(most, c.between);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        a += __shfl_down(a, off);
-        b += __shfl_down(b, off);
-        most = max(most, (uint32_t)__shfl_down(most, off));
-    }
-    if ((threadIdx.x & 63) == 0) {
+    a = wave_scan(a);
+    b = wave_scan(b);
+    most = wave_max(most);
+    if ((threadIdx.x & 63) == 63) {
         atomicAdd(&s_sum[0], a);
         atomicAdd(&s_sum[1], b);
         atomicMax(&s_most, most);
@@ -1783,6 +1816,11 @@ __device__ bool mix_totals(const MixCounts *counts, int waves, uint32_t room, un
 }
 
 constexpr int kMixHistWgs = 96; // workgroups that count what was kept (each adds up to 2048 counters to the others')
+// A piece holds some two hundred values, and one piece after the other, each behind the load of its count, was eleven pairs of trips to memory.
+// (What is left of a pass are the counts of all waves, the digits so far and the counters' atomics: with 48 workgroups 12 + 15 + 15 us,
+// 96 11 + 10 + 11, and 5 for the third where two digits hold the bracket's range, 192 10 + 10 + 10, 256 12 + 10 + 10;
+// with 96 and the first pieces on their way while those are looked at 9.5 + 9.)
+constexpr int kMixPieces = 4; // at a time
 static_assert(kMixWaves <= 64 * 4 * kMixHistWgs, "a lane for each piece of a wave");
 template <int PASS>
 __global__ void __launch_bounds__(256)
@@ -1801,6 +1839,22 @@ __global__ void __launch_bounds__(256)
     const int per = min((int)gridDim.x, kMixHistWgs) * 4, w0 = (int)(blockIdx.x * 4 + (threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
     const int mine = w0 < min(per, waves) ? (waves - w0 + per - 1) / per : 0;
     const uint32_t held = lane < mine ? counts[w0 + lane * per].between : 0u;
+    // Four pieces at a time, sixteen loads in flight; the first of them ahead of the counts of all waves and the digits so far
+    TW_GLOBAL(const u32x2) v[kMixPieces];
+    uint32_t n[kMixPieces];
+    float x[kMixPieces][4];
+    auto fetch = [&](int q0) {
+#pragma unroll
+        for (int q = 0; q < kMixPieces; ++q) {
+            n[q] = q0 + q < mine ? (uint32_t)__builtin_amdgcn_readlane((int)held, q0 + q) : 0u;
+            v[q] = as_global(cand) + (int64_t)(mine ? w0 + min(q0 + q, mine - 1) * per : 0) * room;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) // (a piece that did not hold all of its values is not looked at)
+                x[q][e] = __uint_as_float(v[q][min((uint32_t)(lane + e * 64), min(max(n[q], 1u), room) - 1u)].x);
+        }
+    };
+    if (blockIdx.x < kMixHistWgs)
+        fetch(0);
     unsigned long long n_cand, below;
     bool narrowed;
     if (PASS == 0) {
@@ -1826,24 +1880,11 @@ __global__ void __launch_bounds__(256)
         st->narrowed = narrowed;
     }
     if (narrowed) {
-        // four pieces at a time, sixteen loads in flight: a piece holds some two hundred values, and one piece after the other,
-        // each behind the load of its count, was eleven pairs of trips to memory (the three passes 18 + 12 + 12 us, so 11 + 10 +
-        // 11, and 5 for the third where two digits hold the bracket's range; what is left are the counts of all waves, the digits so far and the counters' atomics: 48 workgroups 12 + 15 + 15,
-        // 192 10 + 10 + 10, 256 12 + 10 + 10)
-        for (int q0 = 0; q0 < mine; q0 += 4) {
-            TW_GLOBAL(const u32x2) v[4];
-            uint32_t n[4];
-            float x[4][4];
+        for (int q0 = 0; q0 < mine; q0 += kMixPieces) {
+            if (q0)
+                fetch(q0);
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                n[q] = q0 + q < mine ? (uint32_t)__builtin_amdgcn_readlane((int)held, q0 + q) : 0u;
-                v[q] = as_global(cand) + (int64_t)(w0 + min(q0 + q, mine - 1) * per) * room;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    x[q][e] = __uint_as_float(v[q][min((uint32_t)(lane + e * 64), max(n[q], 1u) - 1u)].x);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < kMixPieces; ++q) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if ((uint32_t)(lane + e * 64) < n[q])
@@ -2412,7 +2453,7 @@ public:
         // room for the values inside the bracket: an eighth of the elements, and all of a small network's
         wgs_ = (int)std::min<int64_t>(n_items_, kMixWgs);
         const int64_t share = (n_items_ + wgs_ - 1) / wgs_ * (kMixItem / 4); // elements of a wave
-        room_ = (uint32_t)(total_ > kMixSampleFrom ? std::max<int64_t>(share / 8, 512) : share);
+        room_ = (uint32_t)(sampled() ? std::max<int64_t>(share / 8, 512) : share);
         d_cand_ = ar.alloc_n<u32x2>((size_t)wgs_ * 4 * room_);
         d_counts_ = ar.alloc_n<MixCounts>(wgs_ * 4);
         d_bits_ = ar.alloc_n<uint16_t>((size_t)n_items_ * 256);
@@ -2422,24 +2463,30 @@ public:
             return fail(TW_ERR_ALLOC, "allocation for %lld element scores failed", (long long)total_);
         return TW_OK;
     }
+    bool sampled() const { return total_ > kMixSampleFrom; }
     size_t table_bytes() const { return sizeof(MixLayer) * layers_.size(); }
     std::vector<MixLayer> &table() { return layers_; }
     SetupSelect setup() const { return setup_of(d_st_, 1, total_, q_, q_type_, room_); }
-    // behind put_table of the table (at d_layers on the device) and, with SRC == MIX_NORMS, the passes of the selection of `st_rows`
+    // behind put_table of the table (at d_layers on the device; where the masks are is not looked at) and, with SRC == MIX_NORMS, the
+    // passes of the selection of `st_rows`
+    template <int SRC> void queue_bracket(const MixLayer *d_layers, const SelectState *st_rows, Mail *mail, hipStream_t s)
+    {
+        if (!sampled())
+            return;
+        hipLaunchKernelGGL(mix_sample_kernel<SRC>, dim3(kMixSamples / 256), dim3(256), 0, s, d_layers, (int)layers_.size(), total_, st_rows,
+                           d_st_, d_sample_, mail);
+        hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample_, d_st_);
+    }
+    // behind that, and put_table of the table with the masks' places
     template <int SRC> int queue(const MixLayer *d_layers, const SelectState *st_rows, Mail *mail, hipStream_t s)
     {
         const int n_layers = (int)layers_.size(), waves = wgs_ * 4;
-        if (total_ > kMixSampleFrom) {
-            hipLaunchKernelGGL(mix_sample_kernel<SRC>, dim3(kMixSamples / 256), dim3(256), 0, s, d_layers, n_layers, total_, st_rows,
-                               d_sample_);
-            hipLaunchKernelGGL(mix_bracket_kernel, dim3(1), dim3(kBracketThreads), 0, s, d_sample_, d_st_);
-        }
         bool split = false;
         for (const MixLayer &e : layers_)
             split |= e.in_fours == 1;
         auto narrow = SRC == MIX_NORMS && split ? mix_narrow_kernel<MIX_SPLIT> : mix_narrow_kernel<SRC>;
         hipLaunchKernelGGL(narrow, dim3(wgs_), dim3(256), 0, s, d_layers, n_layers, n_items_, st_rows, d_st_, d_cand_,
-                           d_counts_, d_bits_, mail);
+                           d_counts_, d_bits_, mail, sampled() ? 1 : 0);
         const dim3 grid((unsigned)std::min<int64_t>(n_items_, 512));
         hipLaunchKernelGGL(mix_hist_kernel<0>, grid, dim3(256), 0, s, d_layers, n_layers, n_items_, d_st_, d_cand_, d_counts_, waves,
                            d_bits_);
@@ -2786,8 +2833,10 @@ try {
         st = fail(TW_ERR_ALLOC, "allocation for %d layers failed", n_layers);
     if (!st)
         st = put_table(mix.table().data(), mix.table_bytes(), d_layers, mix.setup(), SetupSelect{}, s);
-    if (!st)
+    if (!st) {
+        mix.queue_bracket<MIX_BYTES>(d_layers, nullptr, mail, s);
         st = mix.queue<MIX_BYTES>(d_layers, nullptr, mail, s);
+    }
     if (st)
         return st;
     st = ar.wait();
@@ -2827,10 +2876,11 @@ try {
     Arena ar(s);
     float *d_norms = ar.alloc_n<float>(c.n_norms);
     SelectState *d_st = ar.alloc_n<SelectState>(1);
-    PruneLayer *d_table = ar.alloc_n<PruneLayer>(n_layers);
-    MixLayer *d_layers = ar.alloc_n<MixLayer>(n_layers);
+    // both layer tables in one buffer: one upload
+    const size_t table_bytes = sizeof(PruneLayer) * n_layers;
+    char *d_tables = static_cast<char *>(ar.alloc(table_bytes + mix.table_bytes()));
     Mail *mail = ar.mail();
-    if (!d_norms || !d_st || !d_table || !d_layers || !mail)
+    if (!d_norms || !d_st || !d_tables || !mail)
         return fail(TW_ERR_ALLOC, "allocation of %lld norms failed", (long long)c.n_norms);
     st = mix.alloc(ar);
     if (st)
@@ -2841,13 +2891,21 @@ try {
         mix.table()[l].norms = d_norms + off;
         off += (int64_t)K[l] * c.layers[l].n_tiles;
     }
-    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
+    PruneLayer *d_table = reinterpret_cast<PruneLayer *>(d_tables);
+    MixLayer *d_layers = reinterpret_cast<MixLayer *>(d_tables + table_bytes);
+    std::vector<char> both(table_bytes + mix.table_bytes());
+    std::memcpy(both.data(), c.layers.data(), table_bytes);
+    std::memcpy(both.data() + table_bytes, mix.table().data(), mix.table_bytes());
+    st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
     if (st)
         return st;
     queue_norms(c, d_table, nullptr, false, s);
     st = queue_select(d_norms, c.n_norms, d_st, 1, s);
-    if (!st)
-        st = m.get(n_layers, &ar);
+    if (st)
+        return st;
+    // (everything that the masks' places are not needed for is on its way when the caller allocates them)
+    mix.queue_bracket<MIX_NORMS>(d_layers, d_st, mail, s);
+    st = m.get(n_layers, &ar);
     if (st)
         return st;
     mix.write_to(masks);
