@@ -124,6 +124,33 @@ def test_plan_from_device_mask_tile_edges(tw, oracle, K, N, widths, offset):
             check_export(oracle, plan, tiles, B, "bf16")
 
 
+@pytest.mark.parametrize("K,N,widths,offset", [
+    (1, 1, [1], 0), (3, 5, [2, 3], 1), (1, 15, [15], 3),     # less than sixteen bytes of mask
+    (1, 16, [7, 9], 1), (1, 17, [17], 0), (5, 7, [3, 4], 2),  # the last row's pieces start before their place
+    (129, 131, [1, 130], 1), (257, 301, [301], 3),            # ... of a slab of one row, of lanes of 16 and 32 a row
+])
+def test_masks_of_a_few_bytes(tw, oracle, K, N, widths, offset):
+    """Masks at any address, to their last byte, of which nothing behind them may be read: tiles without rows, without columns
+    and with none pruned, by the oracle's lists."""
+    import torch
+    rng = np.random.default_rng(K * 31 + N)
+    table = [(sum(widths[:i]), w) for i, w in enumerate(widths)]
+    B = rng.standard_normal((K, N)).astype(np.float32)
+    dB = torch.from_numpy(B).cuda()
+    for keep in (0.0, 0.4, 1.0):
+        tiles = [dict(col0=c, width=w, kept_k=np.flatnonzero(rng.random(K) < keep).astype(np.int32),
+                      kept_n=np.flatnonzero(rng.random(w) < max(keep, 0.5)).astype(np.int32)) for c, w in table]
+        mask = oracle.plan_mask(K, N, tiles)
+        for t in tiles:  # (a mask holds no lists of a tile without elements)
+            if len(t["kept_k"]) == 0 or len(t["kept_n"]) == 0:
+                t["kept_k"] = t["kept_n"] = np.zeros(0, np.int32)
+        buf = torch.full((offset + K * N + 64,), 7, dtype=torch.uint8, device="cuda")
+        buf[offset:offset + K * N] = torch.from_numpy(np.ascontiguousarray(mask, np.uint8)).cuda().reshape(-1)
+        with tw.Plan.from_device_mask(K, N, buf.data_ptr() + offset, table, "f16", dB.data_ptr(),
+                                      stream=torch.cuda.current_stream().cuda_stream) as plan:
+            check_export(oracle, plan, tiles, B, "f16")
+
+
 def test_plan_from_mask_rejects_non_tw_mask(tw):
     K, N, G = 64, 128, 32
     mask = np.zeros((K, N), np.uint8)

@@ -208,4 +208,46 @@ __device__ __forceinline__ UnitDev unit_of_words(const GemmArgs &p, int uv, int 
 // and atomics), so prefetched loads, the item's output stores and the ticket atomic keep flying.
 #define TW_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
+// Over the lanes of a wave, in registers: a step through LDS (__shfl) is some 60 cycles, and a selection or an ordered list is a chain of them.
+// (row_shr 1, 2, 4, 8 inside rows of 16 lanes, then the last lane of a row to the next row, of the second row to the upper half; a lane
+// that gets nothing keeps `none`)
+template <class F> __device__ __forceinline__ uint32_t wave_steps(uint32_t x, uint32_t none, F f)
+{
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x111, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x112, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x114, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x118, 0xF, 0xF, false));
+    x = f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x142, 0xA, 0xF, false));
+    return f(x, (uint32_t)__builtin_amdgcn_update_dpp((int)none, (int)x, 0x143, 0xC, 0xF, false));
+}
+__device__ __forceinline__ uint32_t last_lane(uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, 63); }
+__device__ __forceinline__ uint32_t wave_min(uint32_t x)
+{
+    return last_lane(wave_steps(x, 0xFFFFFFFFu, [](uint32_t a, uint32_t b) { return min(a, b); }));
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x)
+{
+    return last_lane(wave_steps(x, 0u, [](uint32_t a, uint32_t b) { return max(a, b); }));
+}
+// sums over the lanes up to this one
+__device__ __forceinline__ uint32_t wave_scan(uint32_t x)
+{
+    return wave_steps(x, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ unsigned long long wave_scan(unsigned long long x)
+{
+    auto step = [&](auto ctrl, auto rows) {
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+        x += (unsigned long long)hi << 32 | lo;
+    };
+    step(std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xF>());
+    step(std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xA>());
+    step(std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xC>());
+    return x;
+}
+
 } // namespace tw

@@ -9,6 +9,7 @@
 // i.e. one MFMA B operand is 16 bytes per lane, 1 KiB contiguous per wave, and the whole
 // block a 64-row main-loop step needs is one contiguous run of nblk * 4 KiB.
 #include "tw_internal.h"
+#include "tw_device.h"
 
 #include <algorithm>
 #include <atomic>
@@ -91,21 +92,31 @@ __device__ __forceinline__ void pack_dense(const PlanTile &t, int64_t g, const i
     const PackPos q = pack_pos(t, g);
     if (!q.any)
         return;
-    const int col = q.n < t.n_kept ? t.col0 + kept_n[t.kn_src + q.n] : -1;
-    int64_t src[8];
+    // (what lies past the lists' ends repeats their last entry: no load is on a condition, so the eight rows' numbers are on their way
+    // together and then the eight weights; VGG16's layers 3.4 - 4.2 us, 6.6 - 7.4 with each behind the one before)
+    const bool in = q.n < t.n_kept;
+    const int64_t col = t.col0 + kept_n[t.kn_src + min(q.n, t.n_kept - 1)];
+    int32_t row[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int kk = q.kk0 + e;
-        src[e] = col >= 0 && kk < t.k_kept ? (int64_t)kept_k[t.kk_src + kk] * N + col : -1;
+    for (int e = 0; e < 8; ++e)
+        row[e] = kept_k[t.kk_src + min(q.kk0 + e, t.k_kept - 1)];
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        f[e] = B[(int64_t)row[e] * N + col];
+    if (mask) {
+        uint8_t m[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            m[e] = mask[(int64_t)row[e] * N + col];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            f[e] = m[e] ? f[e] : 0.0f;
     }
     uint16_t v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        float f = 0.0f;
-        if (src[e] >= 0 && (!mask || mask[src[e]]))
-            f = B[src[e]];
-        v[e] = cast16(f, dtype);
-    }
+    for (int e = 0; e < 8; ++e)
+        v[e] = cast16(in && q.kk0 + e < t.k_kept ? f[e] : 0.0f, dtype);
     pack_put(Bp, t, g, v);
 }
 
@@ -116,12 +127,14 @@ __device__ __forceinline__ void pack_stream(const PlanTile &t, int64_t g, const 
     const PackPos q = pack_pos(t, g);
     if (!q.any)
         return;
+    const uint16_t *const src = Bs + t.src_off + (int64_t)min(q.n, t.n_kept - 1) * K;
     uint16_t v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const int kk = q.kk0 + e;
-        v[e] = (q.n < t.n_kept && kk < t.k_kept) ? Bs[t.src_off + (int64_t)q.n * K + kk] : (uint16_t)0;
-    }
+    for (int e = 0; e < 8; ++e)
+        v[e] = src[min(q.kk0 + e, t.k_kept - 1)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        v[e] = q.n < t.n_kept && q.kk0 + e < t.k_kept ? v[e] : (uint16_t)0;
     pack_put(Bp, t, g, v);
 }
 
@@ -191,33 +204,36 @@ __global__ void __launch_bounds__(256) plan_build_kernel(const BuildArgs a)
             a.tickets[i] = 0;
         return;
     }
+    // All lists of the tile together, an entry of each a thread, out of loads that wait for nothing but each other's addresses (a list
+    // after the other was as many trips to memory).  An empty list's entry comes from another one and is dropped.
     const PlanTile t = build_tile(a, y - a.n_tiles);
-    for (int64_t i = i0; i < t.k_kept; i += step) {
-        const int k = a.kk[t.kk_src + i];
-        a.kept_k[t.kk_dst + i] = k;
-        a.rel_k[t.kk_dst + i] = k - (int)i;
-    }
-    for (int64_t i = i0; i < t.n_kept; i += step) {
-        const int c = a.kn[t.kn_src + i];
-        a.kept_n[t.kn_dst + i] = c;
-        a.rel_n[t.kn_dst + i] = c - (int)i;
-    }
-    for (int64_t i = i0; i < t.n_pruned; i += step)
-        a.pruned_n[t.pn_dst + i] = a.pn[t.pn_src + i];
-    for (int64_t i = i0; i < t.kkp_len; i += step)
-        a.kept_k_pad[t.kkp_dst + i] = i < t.k_kept ? a.kk[t.kk_src + i] : 0;
-    // pairs of rows (GemmArgs::kept_pairs); the padding names row K there (a row of zeros behind the
-    // A-stationary kernel's panel), not row 0.  A tile without columns has no unit and its list
-    // counts as padding.
-    if (a.kept_pairs) {
-        const int kept = t.n_kept > 0 ? t.k_kept : 0;
-        for (int64_t i = i0; i < t.kkp_len / 2; i += step) {
-            const int in = (int)(i & 31), e = in >> 2, g16 = in & 3;
-            const int lo = (int)(i >> 5) * 64 + g16 * 16 + (e >> 2) * 8 + (e & 3);
-            const uint32_t r_lo = lo < kept ? (uint32_t)a.kk[t.kk_src + lo] : (uint32_t)a.K;
-            const uint32_t r_hi = lo + 4 < kept ? (uint32_t)a.kk[t.kk_src + lo + 4] : (uint32_t)a.K;
-            a.kept_pairs[t.kkp_dst / 2 + i] = r_lo | r_hi << 16;
+    const int32_t *const kk = t.k_kept > 0 ? a.kk + t.kk_src : t.n_kept > 0 ? a.kn + t.kn_src : a.pn + t.pn_src;
+    const int32_t *const kn = t.n_kept > 0 ? a.kn + t.kn_src : kk, *const pn = t.n_pruned > 0 ? a.pn + t.pn_src : kk;
+    const int last_k = max(t.k_kept, 1) - 1, last_n = max(t.n_kept, 1) - 1, last_p = max(t.n_pruned, 1) - 1;
+    const int kept = t.n_kept > 0 ? t.k_kept : 0; // of the pairs
+    const int64_t longest = max(max(t.k_kept, t.kkp_len), max(t.n_kept, t.n_pruned));
+    for (int64_t i = i0; i < longest; i += step) {
+        // pairs of rows (GemmArgs::kept_pairs); the padding names row K there (a row of zeros behind the
+        // A-stationary kernel's panel), not row 0.  A tile without columns has no unit and its list
+        // counts as padding.
+        const int in = (int)(i & 31), e = in >> 2, g16 = in & 3;
+        const int lo = (int)(i >> 5) * 64 + g16 * 16 + (e >> 2) * 8 + (e & 3);
+        const int k = kk[min(i, (int64_t)last_k)], c = kn[min(i, (int64_t)last_n)], z = pn[min(i, (int64_t)last_p)];
+        const int k_lo = kk[min(lo, last_k)], k_hi = kk[min(lo + 4, last_k)];
+        if (i < t.k_kept) {
+            a.kept_k[t.kk_dst + i] = k;
+            a.rel_k[t.kk_dst + i] = k - (int)i;
         }
+        if (i < t.n_kept) {
+            a.kept_n[t.kn_dst + i] = c;
+            a.rel_n[t.kn_dst + i] = c - (int)i;
+        }
+        if (i < t.n_pruned)
+            a.pruned_n[t.pn_dst + i] = z;
+        if (i < t.kkp_len)
+            a.kept_k_pad[t.kkp_dst + i] = i < t.k_kept ? k : 0;
+        if (a.kept_pairs && i < t.kkp_len / 2)
+            a.kept_pairs[t.kkp_dst / 2 + i] = (lo < kept ? (uint32_t)k_lo : (uint32_t)a.K) | (lo + 4 < kept ? (uint32_t)k_hi : (uint32_t)a.K) << 16;
     }
 }
 // Inverse of the packing into the reference's compacted layout at K*col0.
@@ -245,7 +261,7 @@ __global__ void unpack_stream_kernel(const PlanTile *tiles, const uint16_t *Bp, 
 // elements lie in that product, so it is exactly when they are as many as rows times columns.
 
 // Rows of one tile and slab, and what a slab of kFlagRows rows of it says about the columns.
-constexpr int kFlagRows = 128, kFlagPasses = kFlagRows / 8; // passes over the rows at 32 lanes a row
+constexpr int kFlagRows = 128;
 constexpr int kMaxTileRows = 32768; // tiles of one launch, where they are the rows of its grid
 constexpr int kFlagArgTiles = 64;   // tiles whose first columns fit the kernel arguments
 struct FlagArgs {
@@ -269,25 +285,25 @@ __device__ __forceinline__ int flag_col0(const FlagArgs &a, int t)
     return ka[offsetof(FlagArgs, arg_tcol0) / 4 + t];
 }
 
+typedef uint32_t Flags __attribute__((ext_vector_type(4), aligned(1))); // sixteen bytes at any address
+
 // Workgroup (slab, tile): kFlagRows rows of one tile, so every flag has one writer and nothing has to
-// be cleared first.  Each row is taken by 8, 16 or 32 lanes of 16 bytes (windows of 32 lanes for wider
+// be cleared first.  Each row is taken by 8, 16 or 32 lanes (LG: 3, 4, 5) of 16 bytes (windows of 32 lanes for wider
 // tiles), all loads of a window in flight at once; a row's lanes vote, the rows of a column are
-// joined with shuffles and through LDS.
-__global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
+// joined with shuffles and through LDS.  What the mask's rows are aligned to (UNIT bytes) and the lanes of a row are constants of each copy, and
+// what lies past a row's end repeats its last bytes: with a branch around a load the compiler waits for each of them (VGG16's layers 3.8 -
+// 6.2 us, 3.8 - 9 with those, and a mask off 4 bytes 256 loads of a byte).
+template <int UNIT, int LG> __device__ __forceinline__ void flags_of_slab(const FlagArgs &a, int t, int c0, int w)
 {
     __shared__ uint32_t s_col[4][128]; // per wave, a window's columns
     __shared__ uint32_t s_nnz;
-    const int slab = (int)blockIdx.x, t = a.tile0 + (int)blockIdx.y;
-    const int c0 = flag_col0(a, t), w = flag_col0(a, t + 1) - c0;
+    constexpr int lpr = 1 << LG, rpp = 256 >> LG, kPasses = kFlagRows / rpp; // rows the workgroup takes at a time
+    const int slab = (int)blockIdx.x;
     const int k0 = slab * kFlagRows, nr = min(kFlagRows, a.K - k0);
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // the widest aligned load the mask allows: 16 bytes, 4 or 1
-    const int unit = (a.N & 15) == 0 && ((uintptr_t)a.mask & 15) == 0 ? 16 : (a.N & 3) == 0 && ((uintptr_t)a.mask & 3) == 0 ? 4 : 1;
-    const int a0 = c0 & -unit, chunks = (c0 + w - a0 + 15) >> 4;
-    const int lpr = chunks <= 8 ? 8 : chunks <= 16 ? 16 : 32; // lanes of a row
-    const int lg = lpr == 8 ? 3 : lpr == 16 ? 4 : 5;
-    const int rpp = 256 >> lg;                                // rows the workgroup takes at a time
-    const int l = tid & (lpr - 1), r0 = tid >> lg;
+    const int a0 = UNIT == 0 ? c0 : c0 & -UNIT, chunks = (c0 + w - a0 + 15) >> 4;
+    const int64_t last16 = (int64_t)a.K * a.N - 16; // the mask's last sixteen bytes
+    const int l = tid & (lpr - 1), r0 = tid >> LG;
     const uint8_t *const base = a.mask + (int64_t)k0 * a.N;
     uint32_t row_any = 0; // bit p: row r0 + p * rpp has an element (this lane's chunks)
     uint32_t nnz = 0;
@@ -295,27 +311,41 @@ __global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
         s_nnz = 0;
     for (int win = 0; win * lpr < chunks; ++win) {
         const int cc = a0 + (win * lpr + l) * 16; // first column of this lane's chunk
-        uint32_t v[kFlagPasses][4];
+        uint32_t v[kPasses][4];
 #pragma unroll
-        for (int p = 0; p < kFlagPasses; ++p) {
-            if (p * rpp >= kFlagRows)
-                break;
-            const uint8_t *const src = base + (int64_t)min(r0 + p * rpp, nr - 1) * a.N + cc;
-            if (unit == 16) {
-                const uint4 x = cc < a.N ? *reinterpret_cast<const uint4 *>(src) : uint4{0u, 0u, 0u, 0u};
+        for (int p = 0; p < kPasses; ++p) {
+            const uint8_t *const row = base + (int64_t)min(r0 + p * rpp, nr - 1) * a.N;
+            if constexpr (UNIT == 16) {
+                const uint4 x = *reinterpret_cast<const uint4 *>(row + min(cc, a.N - 16));
                 v[p][0] = x.x, v[p][1] = x.y, v[p][2] = x.z, v[p][3] = x.w;
-            } else if (unit == 4) {
+            } else if constexpr (UNIT == 4) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    v[p][j] = cc + j * 4 < a.N ? *reinterpret_cast<const uint32_t *>(src + j * 4) : 0u;
-            } else {
+                    v[p][j] = *reinterpret_cast<const uint32_t *>(row + min(cc + j * 4, a.N - 4));
+            } else if constexpr (UNIT == 1) {
+                const int64_t at = row - a.mask + cc;
+                const Flags x = *reinterpret_cast<const Flags *>(a.mask + min(at, last16));
+                v[p][0] = x.x, v[p][1] = x.y, v[p][2] = x.z, v[p][3] = x.w;
+            } else { // (less than 16 bytes of mask)
+                uint32_t x[16];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    v[p][j] = 0u;
+                for (int e = 0; e < 16; ++e)
+                    x[e] = row[min(cc + e, a.N - 1)];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (cc + j * 4 + e < a.N)
-                            v[p][j] |= (uint32_t)src[j * 4 + e] << (e * 8);
+                for (int j = 0; j < 4; ++j)
+                    v[p][j] = x[j * 4] | x[j * 4 + 1] << 8 | x[j * 4 + 2] << 16 | x[j * 4 + 3] << 24;
+            }
+        }
+        if (UNIT == 1 && k0 + nr == a.K) { // what was read before its place, the mask ending there, moves down
+#pragma unroll
+            for (int p = 0; p < kPasses; ++p) {
+                const int64_t over = (int64_t)(k0 + min(r0 + p * rpp, nr - 1)) * a.N + cc - last16;
+                if (over > 0) {
+                    const int by = (int)min(over, (int64_t)16) * 8;
+                    unsigned long long lo = (unsigned long long)v[p][1] << 32 | v[p][0], hi = (unsigned long long)v[p][3] << 32 | v[p][2];
+                    lo = by >= 64 ? (by >= 128 ? 0ull : hi >> (by - 64)) : lo >> by | hi << 1 << (63 - by);
+                    hi = by >= 64 ? 0ull : hi >> by;
+                    v[p][0] = (uint32_t)lo, v[p][1] = (uint32_t)(lo >> 32), v[p][2] = (uint32_t)hi, v[p][3] = (uint32_t)(hi >> 32);
                 }
             }
         }
@@ -326,9 +356,7 @@ __global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
             in_tile[j] = (uint32_t)((1ull << (hi * 8)) - 1ull) & ~(uint32_t)((1ull << (lo * 8)) - 1ull);
         }
 #pragma unroll
-        for (int p = 0; p < kFlagPasses; ++p) {
-            if (p * rpp >= kFlagRows)
-                break;
+        for (int p = 0; p < kPasses; ++p) {
             uint32_t any = 0;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -362,21 +390,41 @@ __global__ void __launch_bounds__(256) mask_flags_kernel(const FlagArgs a)
         __syncthreads();
     }
 #pragma unroll
-    for (int p = 0; p < kFlagPasses; ++p) {
-        if (p * rpp >= kFlagRows)
-            break;
+    for (int p = 0; p < kPasses; ++p) {
         const unsigned long long votes = __ballot(row_any >> p & 1u);
         const unsigned long long mine = (lpr == 32 ? 0xFFFFFFFFull : (1ull << lpr) - 1ull) << (lane & -lpr);
         if (l == 0 && r0 + p * rpp < nr)
             a.rowflag[(int64_t)t * a.K + k0 + r0 + p * rpp] = (votes & mine) != 0ull;
     }
-    for (int off = 32; off > 0; off >>= 1)
-        nnz += __shfl_down(nnz, off);
-    if (lane == 0)
+    nnz = wave_scan(nnz);
+    if (lane == 63)
         atomicAdd(&s_nnz, nnz);
     __syncthreads();
     if (tid == 0)
         a.nnz[(int64_t)t * a.n_slabs + slab] = s_nnz;
+}
+__global__ void __launch_bounds__(256, 3) mask_flags_kernel(const FlagArgs a)
+{
+    const int t = a.tile0 + (int)blockIdx.y;
+    const int c0 = flag_col0(a, t), w = flag_col0(a, t + 1) - c0;
+    auto lanes_of = [&](auto unit) { // loads of 16 bytes, 4 or, at any address, 16 again
+        constexpr int UNIT = decltype(unit)::value;
+        const int chunks = (c0 + w - (c0 & -UNIT) + 15) >> 4;
+        if (chunks <= 8)
+            flags_of_slab<UNIT, 3>(a, t, c0, w);
+        else if (chunks <= 16)
+            flags_of_slab<UNIT, 4>(a, t, c0, w);
+        else
+            flags_of_slab<UNIT, 5>(a, t, c0, w);
+    };
+    if ((a.N & 15) == 0 && ((uintptr_t)a.mask & 15) == 0)
+        lanes_of(std::integral_constant<int, 16>());
+    else if ((a.N & 3) == 0 && ((uintptr_t)a.mask & 3) == 0)
+        lanes_of(std::integral_constant<int, 4>());
+    else if ((int64_t)a.K * a.N >= 16)
+        lanes_of(std::integral_constant<int, 1>());
+    else
+        flags_of_slab<0, 3>(a, t, c0, w);
 }
 
 // What the host needs to know of a tile before it can lay the plan out, in pinned memory: kept rows, kept columns, the low and
@@ -401,12 +449,7 @@ __global__ void __launch_bounds__(kListThreads)
     const int c0 = flag_col0(a, t), w = flag_col0(a, t + 1) - c0;
     // position of this thread's first one among all ones of the workgroup, and their number
     auto scan = [&](int mine, int &total) {
-        int incl = mine;
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(incl, off);
-            if (lane >= off)
-                incl += up;
-        }
+        const int incl = (int)wave_scan((uint32_t)mine);
         if (lane == 63)
             s_wave[wave] = incl;
         __syncthreads();
@@ -422,54 +465,69 @@ __global__ void __launch_bounds__(kListThreads)
     };
     if (tid == 0)
         s_nnz = 0;
+    // The first loads of everything leave together, none of them on a condition (VGG16's layers 4.0 - 5.5 us, 4.1 - 6.5 with one part's
+    // behind another's and a flag at a time, each behind the one before).
+    // sixteen rows' flags a thread (what lies behind a tile's last one stays inside the workspace)
+    const uint8_t *const flag = a.rowflag + (int64_t)t * a.K;
+    auto rows_per_thread = [&](int base) { return min(16, (a.K - base + kListThreads - 1) / kListThreads); };
+    auto flags_of = [&](int base) { return *reinterpret_cast<const Flags *>(flag + min(base + tid * rows_per_thread(base), a.K - 1)); };
+    Flags f = flags_of(0);
+    const uint32_t nnz0 = a.nnz[(int64_t)t * a.n_slabs + min(tid, a.n_slabs - 1)];
     // What the slabs say about a window's columns: four of them a thread, 2^lg threads side by side, the slabs dealt out over the
-    // groups.  All loads of eight slabs are in flight at once, and the first window's fly over the rows' part (one slab after
-    // another behind it: K 4608 in two tiles 7.9 us).
+    // groups, eight of them at a time.
     const int words = ((w + 3) & ~3) >> 2;
     const uint32_t *const part = reinterpret_cast<const uint32_t *>(a.colpart + a.colpart_at(t, c0));
     const int lg = words >= kListThreads ? 9 : words > 1 ? 32 - __clz(words - 1) : 0, groups = kListThreads >> lg;
     static_assert(kListThreads == 512, "a window is at most 2^9 words");
     const int cj = tid & ((1 << lg) - 1);
-    auto slabs_of = [&](int base) {
-        uint32_t x = 0;
+    auto eight_slabs = [&](int base, int slab, uint32_t (&v)[8]) {
         const uint32_t *const src = part + min(base + cj, words - 1);
-        for (int slab = tid >> lg; slab < a.n_slabs; slab += 8 * groups) {
-            uint32_t v[8];
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                v[i] = src[(int64_t)min(slab + i * groups, a.n_slabs - 1) * words];
+        for (int i = 0; i < 8; ++i)
+            v[i] = src[(int64_t)min(slab + i * groups, a.n_slabs - 1) * words];
+    };
+    uint32_t v0[8];
+    eight_slabs(0, tid >> lg, v0);
+    auto slabs_of = [&](int base, uint32_t x, int slab) {
+        for (; slab < a.n_slabs; slab += 8 * groups) {
+            uint32_t v[8];
+            eight_slabs(base, slab, v);
 #pragma unroll
             for (int i = 0; i < 8; ++i)
                 x |= v[i];
         }
         return x;
     };
-    uint32_t cols = slabs_of(0);
-    unsigned long long nnz = 0;
-    for (int i = tid; i < a.n_slabs; i += kListThreads)
-        nnz += a.nnz[(int64_t)t * a.n_slabs + i];
-    for (int off = 32; off > 0; off >>= 1)
-        nnz += __shfl_down(nnz, off);
 
     // rows
-    const uint8_t *const flag = a.rowflag + (int64_t)t * a.K;
     int32_t *const rows = kk + (int64_t)t * a.K;
     int k_kept = 0;
     for (int base = 0; base < a.K; base += kListThreads * 16) { // sixteen rows a thread at a time
-        const int run = min(16, (a.K - base + kListThreads - 1) / kListThreads);
+        const int run = rows_per_thread(base);
         const int first = base + tid * run;
+        if (base > 0)
+            f = flags_of(base);
         uint32_t bits = 0;
 #pragma unroll
         for (int i = 0; i < 16; ++i)
-            if (i < run && first + i < a.K)
-                bits |= (flag[first + i] ? 1u : 0u) << i;
+            bits |= (f[i >> 2] >> (i & 3) * 8 & 1u) << i;
+        bits &= (1u << max(min(run, a.K - first), 0)) - 1u;
         int total;
         int at = k_kept + scan(__popc(bits), total);
         for (; bits; bits &= bits - 1u)
             rows[at++] = first + __ffs(bits) - 1;
         k_kept += total;
     }
-    if (lane == 0)
+    uint32_t cols = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        cols |= v0[i];
+    cols = slabs_of(0, cols, (tid >> lg) + 8 * groups);
+    unsigned long long nnz = tid < a.n_slabs ? nnz0 : 0u;
+    for (int i = tid + kListThreads; i < a.n_slabs; i += kListThreads)
+        nnz += a.nnz[(int64_t)t * a.n_slabs + i];
+    nnz = wave_scan(nnz);
+    if (lane == 63)
         atomicAdd(&s_nnz, nnz);
 
     // columns: kept where any slab says so
@@ -477,7 +535,7 @@ __global__ void __launch_bounds__(kListThreads)
     for (int base = 0; base < words; base += kListThreads) {
         const int nw = min(kListThreads, words - base);
         if (base > 0)
-            cols = slabs_of(base);
+            cols = slabs_of(base, 0u, tid >> lg);
         s_cols[tid] = 0;
         __syncthreads();
         if (cj < nw && cols)
