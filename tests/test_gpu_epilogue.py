@@ -111,6 +111,41 @@ def test_row_major_epilogue(tw, oracle, act_name, act):
         assert oracle.rel_error(C, reference(oracle, A, B, tiles, "f16", bias, act_name)) <= 1e-2
 
 
+@pytest.mark.parametrize("row_major", [False, True])
+@pytest.mark.parametrize("M,beta", [(1, 0.0), (7, 0.5), (33, 0.0), (64, 0.5), (65, 0.0), (130, 0.5), (130, 0.0)])
+def test_pruned_columns_beside_few_rows(tw, oracle, M, beta, row_major):
+    """The kernel for few rows fills pruned columns by workgroups of their own: a row block's last piece of one row, tiles of one
+    pruned column, of all but one and of nothing kept, a tile of one column.  Bit for bit: nothing is added up in them, and the scale is a
+    power of two."""
+    rng = np.random.default_rng(M * 2 + row_major)
+    K, widths = 640, [128, 128, 1, 100, 128, 3]
+    kept = [127, 1, 1, 100, 0, 2]
+    N, tiles, c = sum(widths), [], 0
+    for w, n in zip(widths, kept):
+        tiles.append(dict(col0=c, width=w, kept_k=np.sort(rng.choice(K, 150 if n else 0, replace=False)).astype(np.int32),
+                          kept_n=np.sort(rng.choice(w, n, replace=False)).astype(np.int32)))
+        c += w
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.08).astype(np.float32)
+    C0, bias = rng.standard_normal((M, N)).astype(np.float32), rng.standard_normal(N).astype(np.float32)
+    keep = kept_columns(tiles, N)
+    try:
+        tw.set_option(tw.OPT_SHAPE, tw.SHAPE_SKINNY)
+        with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+            lay = tw.ROWMAJOR if row_major else tw.KMAJOR
+            assert "skinny" in plan.kernel_name(M, lda=round_up(K if row_major else M, 8), ldc=round_up(N if row_major else M, 8),
+                                                a_layout=lay, c_layout=lay, beta=beta)
+            for b in (bias, None):
+                C = run(tw, oracle, plan, A, "f16", N, b, 1, beta=beta, C0=C0, row_major=row_major)
+                old = np.float32(beta) * oracle.quantize(C0, "f16").astype(np.float32)
+                want = oracle.quantize(np.maximum(old + (0 if b is None else b), 0).astype(np.float32), "f16")
+                assert np.array_equal(C[:, ~keep], want.reshape(M, N)[:, ~keep])
+                ref = reference(oracle, A, B, tiles, "f16", b, "relu", beta=beta, C0=C0)
+                assert oracle.rel_error(C[:, keep], ref[:, keep]) <= TOL["f16"]
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+
+
 def test_untouched_columns_stay_untouched(tw, oracle):
     rng = np.random.default_rng(32)
     M, K, N, G = 256, 128, 256, 128

@@ -1865,7 +1865,10 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 //          of VGG16 conv4_1 at M 980 took 14.4 us, on all dies 7.7;
 //          the unit comes from the kernel arguments at an offset that depends on the workgroup
 //          number alone, so that it arrives with the other arguments; workgroups of a piece the
-//          unit does not have fill pruned columns (TW_PRUNED_ZERO) or leave
+//          unit does not have leave.  Pruned columns (TW_PRUNED_ZERO) have workgroups of their own behind all others: behind
+//          the products of the same workgroups their chain of tile, column and bias was a third of the launch (M 64,
+//          K 4608, N 512, a quarter of the rows and half of the columns kept 6.2 us, 4.3 this way; M 256, K 768, N 3072, a tenth pruned 5.9 and 4.2;
+//          53 problems, M 1 - 980, K-major and row-major: 0.77 of the time in the mean, 1.0 at most)
 //   stage: per wave 64 rows k of 32 rows m (64 bytes each), then reused for the wave's
 //          partial product [its columns][32 + 4 rows m] in fp32
 // K-major A and C, or (RM) row-major ones; any beta.  A kept row of a row-major A is one 2-byte element
@@ -1877,6 +1880,7 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 constexpr int kSkRows = 32;                            // rows m of a workgroup
 constexpr int kSkCols = 64;                            // compact columns of a workgroup, or half of them
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
+constexpr int sk_fill_rows(bool rm) { return rm ? 32 : 64; } // rows m of a tile's pruned columns that a workgroup fills
 struct SkinnyWork {
     int32_t n_units, n_rowblk;
     int32_t pieces, piece_shift; // of a unit: 1, 2 or 4, and its logarithm
@@ -1885,7 +1889,59 @@ struct SkinnyWork {
     uint32_t magic;        // 2^32 / grouped, rounded up
     int32_t left;          // units left over
     int32_t dies_per_unit; // kXcd / left
+    int32_t gemm_wgs;      // workgroups that multiply; those behind them fill pruned columns
+    int32_t fill_wgs, n_fillblk; // so many, sk_fill_rows rows of a tile at a time
 };
+
+// Pruned columns receive act(beta * C + bias).  The tile, its columns and their bias are a chain of three trips to memory, which four
+// pieces of a thread take together.
+template <int DT, int NT, bool RM> __device__ __forceinline__ void skinny_fill(const GemmArgs &p, const SkinnyWork &w, int first)
+{
+    using E = Elem<DT>;
+    constexpr int ROWS = sk_fill_rows(RM), PIECE = RM ? 1 : 8; // rows of a piece
+    uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
+    const int tid = threadIdx.x, items = (p.n_all_u - p.n_gemm_u) * w.n_fillblk;
+    for (int item = first; item < items; item += w.fill_wgs) {
+        const int z = item / w.n_fillblk, m0 = (item - z * w.n_fillblk) * ROWS;
+        const int m_end = min(m0 + ROWS, p.M);
+        const TileDev t = p.tiles[z];
+        const int per_col = (m_end - m0 + PIECE - 1) / PIECE, pieces = t.n_pruned * per_col;
+        for (int i0 = tid; i0 < pieces; i0 += NT * 4) {
+            int c[4], m[4];
+            float b[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) { // (row-major: neighbouring lanes in neighbouring columns)
+                const int i = min(i0 + j * NT, pieces - 1), q = RM ? i / t.n_pruned : i / per_col;
+                c[j] = t.col0 + p.pruned_n[t.pn_off + (RM ? i - q * t.n_pruned : q)];
+                m[j] = m0 + (RM ? q : (i - q * per_col) * 8);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                b[j] = p.bias ? p.bias[c[j]] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (i0 + j * NT >= pieces)
+                    break;
+                uint16_t *const dst = RM ? C + (int64_t)m[j] * p.ldc + c[j] : C + (int64_t)c[j] * p.ldc + m[j];
+                if constexpr (RM) {
+                    const float old = p.beta != 0.0f ? p.beta * E::from_bits(*dst) : 0.0f;
+                    *dst = (uint16_t)E::to_bits(tw_activate(old + b[j], p.act));
+                } else {
+                    uint32_t h[4];
+                    if (p.beta == 0.0f) {
+                        const uint32_t v = E::to_bits(tw_activate(0.0f + b[j], p.act));
+                        h[0] = h[1] = h[2] = h[3] = v | v << 16;
+                    } else {
+                        h[0] = h[1] = h[2] = h[3] = 0u;
+                        for (int e = 0; e < 8 && m[j] + e < m_end; ++e)
+                            h[e >> 1] |= E::to_bits(tw_activate(p.beta * E::from_bits(dst[e]) + b[j], p.act)) << ((e & 1) * 16);
+                    }
+                    store_chunk(dst, u32x4{h[0], h[1], h[2], h[3]}, m[j], m_end, false);
+                }
+            }
+        }
+    }
+}
 
 template <int DT, int NW, bool RM, int NB>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
@@ -1900,6 +1956,10 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // (w.pieces of a unit: a power of two, COLS columns each)
+    if ((int)blockIdx.x >= w.gemm_wgs) {
+        skinny_fill<DT, NT, RM>(p, w, (int)blockIdx.x - w.gemm_wgs);
+        return;
+    }
     const int die = blockIdx.x % kXcd;
     int half, ui, yblk;
     bool in_range = true;
@@ -2149,35 +2209,6 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                 for (int e = 0; m0 + mr + e < m_end; ++e)
                     dst[e] = (uint16_t)(h[e >> 1] >> ((e & 1) * 16));
             }
-        }
-    }
-
-    // ---- TW_PRUNED_ZERO: pruned columns receive act(beta * C + bias); shared out over the
-    // workgroups of a row block
-    for (int z = p.n_gemm_u + ui * w.pieces + half; z < p.n_all_u; z += w.n_units * w.pieces) {
-        const TileDev t = p.tiles[z - p.n_gemm_u];
-        if constexpr (RM) {
-            for (int i = tid; i < t.n_pruned * kSkRows; i += NT) {
-                const int m = m0 + i / t.n_pruned;
-                if (m >= m_end)
-                    break;
-                const int c = t.col0 + p.pruned_n[t.pn_off + i % t.n_pruned];
-                uint16_t *const dst = C + (int64_t)m * ldc + c;
-                const float old = p.beta != 0.0f ? p.beta * E::from_bits(*dst) : 0.0f;
-                *dst = (uint16_t)E::to_bits(tw_finish(old, p.bias, c, p.act));
-            }
-            continue;
-        }
-        for (int i = tid; i < t.n_pruned * 4; i += NT) {
-            const int jz = i >> 2, m = m0 + (i & 3) * 8;
-            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
-            uint16_t *const dst = C + (int64_t)c * ldc + m;
-            uint32_t h[4] = {0u, 0u, 0u, 0u};
-            for (int e = 0; e < 8 && m + e < m_end; ++e) {
-                const float old = p.beta != 0.0f ? p.beta * E::from_bits(dst[e]) : 0.0f;
-                h[e >> 1] |= E::to_bits(tw_finish(old, p.bias, c, p.act)) << ((e & 1) * 16);
-            }
-            store_chunk(dst, u32x4{h[0], h[1], h[2], h[3]}, m, m_end, false);
         }
     }
 }
@@ -2836,16 +2867,23 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     // M 128, K 768, N 768 3.1 and 2.8, 4.5 and 4.1.  From 288 workgroups on 1.02 - 1.20 of the time, and 1.05 - 1.49.
     SkinnyWork narrow;
     const int64_t narrow_items = skinny_work(plan, a.M, &narrow, kSkCols / 2);
-    if (narrow_items >= 0 && skinny_per_die(narrow) * kXcd <= plan->cu_count) {
-        if (few)
-            hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 1>), dim3((unsigned)narrow_items), dim3(64 * 4), 0, s, a, narrow);
-        else
-            hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 1>), dim3((unsigned)narrow_items), dim3(64 * 8), 0, s, a, narrow);
-    } else if (few) {
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 2>), dim3((unsigned)items), dim3(64 * 4), 0, s, a, w);
-    } else {
-        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 2>), dim3((unsigned)items), dim3(64 * 8), 0, s, a, w);
-    }
+    const bool pieces_of_32 = narrow_items >= 0 && skinny_per_die(narrow) * kXcd <= plan->cu_count;
+    if (pieces_of_32)
+        w = narrow;
+    const int threads = few ? 256 : 512;
+    w.gemm_wgs = (int32_t)(pieces_of_32 ? narrow_items : items);
+    w.n_fillblk = (a.M + sk_fill_rows(RM) - 1) / sk_fill_rows(RM);
+    // (a launch of as many workgroups as it takes loops over the rest)
+    w.fill_wgs = (int32_t)std::min<int64_t>((int64_t)(a.n_all_u - a.n_gemm_u) * w.n_fillblk, kMaxGridThreads / threads - w.gemm_wgs);
+    const dim3 grid((unsigned)(w.gemm_wgs + w.fill_wgs));
+    if (pieces_of_32 && few)
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 1>), grid, dim3(threads), 0, s, a, w);
+    else if (pieces_of_32)
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 1>), grid, dim3(threads), 0, s, a, w);
+    else if (few)
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 2>), grid, dim3(threads), 0, s, a, w);
+    else
+        hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 2>), grid, dim3(threads), 0, s, a, w);
     TW_HIP(hipGetLastError());
     return TW_OK;
 }
