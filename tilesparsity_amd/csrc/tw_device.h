@@ -208,6 +208,119 @@ __device__ __forceinline__ UnitDev unit_of_words(const GemmArgs &p, int uv, int 
 // and atomics), so prefetched loads, the item's output stores and the ticket atomic keep flying.
 #define TW_LDS_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
+// Pruned columns (TW_PRUNED_ZERO) receive act(beta * C + bias).  A tile, its columns and their bias are a chain of three trips to memory, so
+// four of them go together: of four tiles, or four stretches of one.  (With a column at a time per thread, and its bias read again for
+// every row, what a fill added to the product was, in us, and is: M 6272, K 3072, N 768, half of the columns pruned, 256 x 64 streaming
+// kernel 10.9 and 3.8; K 768, N 3072 row-major, A-stationary 26.6 and 10.1; M 1024 7.1 and 3.2; M 6272, K 4096, N 8192, row-major streaming 85 and 28;
+// a tenth pruned, M 6272, K 3072, N 768 3.6 and 2.0.)
+// Tile z of the fill table, or, past the end, one without columns.
+__device__ __forceinline__ TileDev fill_tile(const GemmArgs &p, int z)
+{
+    const int last = p.n_all_u - p.n_gemm_u - 1;
+    const auto *const g = (const __attribute__((address_space(4))) int32_t *)(uintptr_t)(p.tiles + (z < last ? z : last));
+    return TileDev{g[0], z <= last ? g[1] : 0, g[2], 0};
+}
+// K-major C, rows [m_lo, m_hi): pieces first[j] + tid, + stride .. of tile t[j], a piece being eight rows of a column.
+template <int DT> __device__ __forceinline__ void fill_kmajor(const GemmArgs &p, int act, const TileDev (&t)[4], const int (&first)[4], int stride,
+                                                              int m_lo, int m_hi, int tid, bool through)
+{
+    using E = Elem<DT>;
+    if (m_hi <= m_lo)
+        return;
+    uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
+    const uint32_t per_col = (uint32_t)(m_hi - m_lo + 7) / 8;
+    int most = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        most = max(most, t[j].n_pruned * (int)per_col - first[j]);
+    for (int k = tid; k < most; k += stride) {
+        int c[4], m[4];
+        float b[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t i = (uint32_t)(first[j] + k), q = i / per_col;
+            const bool in = (int)q < t[j].n_pruned;
+            c[j] = in ? t[j].col0 + p.pruned_n[t[j].pn_off + (in ? (int)q : 0)] : -1;
+            m[j] = m_lo + (int)(i - q * per_col) * 8;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            b[j] = p.bias ? p.bias[max(c[j], 0)] : 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (c[j] < 0)
+                continue;
+            uint16_t *const dst = C + (int64_t)c[j] * p.ldc + m[j];
+            uint32_t h[4];
+            if (p.beta == 0.0f) {
+                const uint32_t v = E::to_bits(tw_activate(0.0f + b[j], act));
+                h[0] = h[1] = h[2] = h[3] = v | v << 16;
+            } else {
+                h[0] = h[1] = h[2] = h[3] = 0u;
+                for (int e = 0; e < 8 && m[j] + e < m_hi; ++e)
+                    h[e >> 1] |= E::to_bits(tw_activate(p.beta * E::from_bits(dst[e]) + b[j], act)) << ((e & 1) * 16);
+            }
+            store_chunk(dst, u32x4{h[0], h[1], h[2], h[3]}, m[j], m_hi, through);
+        }
+    }
+}
+// one tile, by NT threads
+template <int DT, int NT> __device__ __forceinline__ void fill_kmajor(const GemmArgs &p, int act, const TileDev &t, int m_lo, int m_hi, int tid, bool through)
+{
+    const TileDev same[4] = {t, t, t, t};
+    const int first[4] = {0, NT, 2 * NT, 3 * NT};
+    fill_kmajor<DT>(p, act, same, first, 4 * NT, m_lo, m_hi, tid, through);
+}
+// tiles z0, z0 + step, .. of the table
+template <int DT, int NT> __device__ __forceinline__ void fill_kmajor_tiles(const GemmArgs &p, int z0, int step, int m_lo, int m_hi, int tid, bool through)
+{
+    const int n = p.n_all_u - p.n_gemm_u;
+    const int first[4] = {0, 0, 0, 0};
+    for (int z = z0; z < n; z += 4 * step) {
+        const TileDev t[4] = {fill_tile(p, z), fill_tile(p, z + step), fill_tile(p, z + 2 * step), fill_tile(p, z + 3 * step)};
+        fill_kmajor<DT>(p, p.act, t, first, NT, m_lo, m_hi, tid, through);
+    }
+}
+// Row-major C, tiles z0, z0 + step, .. by NT threads: a lane keeps its column of each of four tiles, and with it the value where C is not
+// read, and walks down the rows.
+template <int DT, int NT> __device__ __forceinline__ void fill_rowmajor_tiles(const GemmArgs &p, int z0, int step, int m_lo, int m_hi, int tid)
+{
+    using E = Elem<DT>;
+    uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
+    const int n = p.n_all_u - p.n_gemm_u;
+    for (int z = z0; z < n; z += 4 * step) {
+        const TileDev t[4] = {fill_tile(p, z), fill_tile(p, z + step), fill_tile(p, z + 2 * step), fill_tile(p, z + 3 * step)};
+        const int most = max(max(t[0].n_pruned, t[1].n_pruned), max(t[2].n_pruned, t[3].n_pruned));
+        int lg = 0; // 2^lg columns side by side
+        while (lg < 6 && 1 << lg < most)
+            ++lg;
+        for (int base = 0; base < most; base += 1 << lg) {
+            const int q = base + (tid & ((1 << lg) - 1));
+            int c[4];
+            float b[4];
+            uint16_t v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                c[j] = q < t[j].n_pruned ? t[j].col0 + p.pruned_n[t[j].pn_off + q] : -1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                b[j] = p.bias ? p.bias[max(c[j], 0)] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = (uint16_t)E::to_bits(tw_activate(0.0f + b[j], p.act));
+            for (int m = m_lo + (tid >> lg); m < m_hi; m += NT >> lg) {
+                uint16_t *const row = C + (int64_t)m * p.ldc;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (c[j] < 0)
+                        continue;
+                    row[c[j]] = p.beta == 0.0f ? v[j] : (uint16_t)E::to_bits(tw_activate(p.beta * E::from_bits(row[c[j]]) + b[j], p.act));
+                }
+            }
+        }
+    }
+}
+
 // Over the lanes of a wave, in registers: a step through LDS (__shfl) is some 60 cycles, and a selection or an ordered list is a chain of them.
 // (row_shr 1, 2, 4, 8 inside rows of 16 lanes, then the last lane of a row to the next row, of the second row to the upper half; a lane
 // that gets nothing keeps `none`)

@@ -651,22 +651,23 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
     };
     // zero-fill item: pruned columns of one tile receive beta*C (all threads, no barrier)
     auto zero_fill = [&](const Item &it) {
+        // (a column at a time, not four as in fill_kmajor: what that keeps in scalar registers costs the item loop its own, 2 % of a launch)
         const int m = it.m0 + (tid % CPR) * 8;
         const TileDev t = p.tiles[it.col - p.n_gemm_u];
+#pragma unroll 1
         for (int j = tid / CPR; j < t.n_pruned; j += NT / CPR) {
             const int c = t.col0 + p.pruned_n[t.pn_off + j];
+            const float b = p.bias ? p.bias[c] : 0.0f;
             uint16_t *dst = C + (int64_t)c * p.ldc + m;
-            u32x4 v = {0u, 0u, 0u, 0u};
-            if ((p.beta != 0.0f || p.bias || p.act) && m < it.m_end) {
+            u32x4 v;
+            if (p.beta == 0.0f) {
+                const uint32_t h = E::to_bits(tw_activate(0.0f + b, p.act));
+                v.x = v.y = v.z = v.w = h | h << 16;
+            } else {
                 uint32_t w[4] = {0u, 0u, 0u, 0u};
-                for (int e = 0; e < 8 && m + e < it.m_end; ++e) {
-                    const float old = p.beta != 0.0f ? p.beta * E::from_bits(dst[e]) : 0.0f;
-                    w[e >> 1] |= E::to_bits(tw_finish(old, p.bias, c, p.act)) << ((e & 1) * 16);
-                }
-                v.x = w[0];
-                v.y = w[1];
-                v.z = w[2];
-                v.w = w[3];
+                for (int e = 0; e < 8 && m + e < it.m_end; ++e)
+                    w[e >> 1] |= E::to_bits(tw_activate(p.beta * E::from_bits(dst[e]) + b, p.act)) << ((e & 1) * 16);
+                v = u32x4{w[0], w[1], w[2], w[3]};
             }
             store_chunk(dst, v, m, it.m_end, p.store_through != 0);
         }
@@ -1824,26 +1825,10 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
     }
 
     // ---- TW_PRUNED_ZERO: the pruned columns of this group's tiles receive act(bias)
-    for (int z = p.n_gemm_u + group; z < p.n_all_u; z += n_groups) {
-        const TileDev t = p.tiles[z - p.n_gemm_u];
-        if (RM) {
-            for (int i = tid; i < t.n_pruned * BMS; i += NT) {
-                const int m = m0 + i / t.n_pruned;
-                const int c = t.col0 + p.pruned_n[t.pn_off + i % t.n_pruned];
-                if (m < m_end)
-                    C[(int64_t)m * p.ldc + c] = (uint16_t)E::to_bits(tw_finish(0.0f, p.bias, c, p.act));
-            }
-            continue;
-        }
-        for (int i = tid; i < t.n_pruned * CH; i += NT) {
-            const int jz = i / CH, ch = i % CH;
-            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
-            const uint32_t hb = E::to_bits(tw_finish(0.0f, p.bias, c, p.act));
-            const uint32_t w = hb | (hb << 16);
-            store_chunk(C + (int64_t)c * p.ldc + m0 + ch * 8, u32x4{w, w, w, w}, m0 + ch * 8, m_end,
-                        p.store_through != 0);
-        }
-    }
+    if constexpr (RM)
+        fill_rowmajor_tiles<DT, NT>(p, group, n_groups, m0, m_end, tid);
+    else
+        fill_kmajor_tiles<DT, NT>(p, group, n_groups, m0, m_end, tid, p.store_through != 0);
 }
 
 // ---------------------------------------------------------------------------------
@@ -1893,56 +1878,6 @@ struct SkinnyWork {
     int32_t fill_wgs, n_fillblk; // so many, sk_fill_rows rows of a tile at a time
 };
 
-// Pruned columns receive act(beta * C + bias).  The tile, its columns and their bias are a chain of three trips to memory, which four
-// pieces of a thread take together.
-template <int DT, int NT, bool RM> __device__ __forceinline__ void skinny_fill(const GemmArgs &p, const SkinnyWork &w, int first)
-{
-    using E = Elem<DT>;
-    constexpr int ROWS = sk_fill_rows(RM), PIECE = RM ? 1 : 8; // rows of a piece
-    uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
-    const int tid = threadIdx.x, items = (p.n_all_u - p.n_gemm_u) * w.n_fillblk;
-    for (int item = first; item < items; item += w.fill_wgs) {
-        const int z = item / w.n_fillblk, m0 = (item - z * w.n_fillblk) * ROWS;
-        const int m_end = min(m0 + ROWS, p.M);
-        const TileDev t = p.tiles[z];
-        const int per_col = (m_end - m0 + PIECE - 1) / PIECE, pieces = t.n_pruned * per_col;
-        for (int i0 = tid; i0 < pieces; i0 += NT * 4) {
-            int c[4], m[4];
-            float b[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) { // (row-major: neighbouring lanes in neighbouring columns)
-                const int i = min(i0 + j * NT, pieces - 1), q = RM ? i / t.n_pruned : i / per_col;
-                c[j] = t.col0 + p.pruned_n[t.pn_off + (RM ? i - q * t.n_pruned : q)];
-                m[j] = m0 + (RM ? q : (i - q * per_col) * 8);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                b[j] = p.bias ? p.bias[c[j]] : 0.0f;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (i0 + j * NT >= pieces)
-                    break;
-                uint16_t *const dst = RM ? C + (int64_t)m[j] * p.ldc + c[j] : C + (int64_t)c[j] * p.ldc + m[j];
-                if constexpr (RM) {
-                    const float old = p.beta != 0.0f ? p.beta * E::from_bits(*dst) : 0.0f;
-                    *dst = (uint16_t)E::to_bits(tw_activate(old + b[j], p.act));
-                } else {
-                    uint32_t h[4];
-                    if (p.beta == 0.0f) {
-                        const uint32_t v = E::to_bits(tw_activate(0.0f + b[j], p.act));
-                        h[0] = h[1] = h[2] = h[3] = v | v << 16;
-                    } else {
-                        h[0] = h[1] = h[2] = h[3] = 0u;
-                        for (int e = 0; e < 8 && m[j] + e < m_end; ++e)
-                            h[e >> 1] |= E::to_bits(tw_activate(p.beta * E::from_bits(dst[e]) + b[j], p.act)) << ((e & 1) * 16);
-                    }
-                    store_chunk(dst, u32x4{h[0], h[1], h[2], h[3]}, m[j], m_end, false);
-                }
-            }
-        }
-    }
-}
-
 template <int DT, int NW, bool RM, int NB>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
 {
@@ -1957,7 +1892,14 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // (w.pieces of a unit: a power of two, COLS columns each)
     if ((int)blockIdx.x >= w.gemm_wgs) {
-        skinny_fill<DT, NT, RM>(p, w, (int)blockIdx.x - w.gemm_wgs);
+        const int n = (p.n_all_u - p.n_gemm_u) * w.n_fillblk;
+        for (int item = (int)blockIdx.x - w.gemm_wgs; item < n; item += w.fill_wgs) {
+            const int z = item / w.n_fillblk, m_lo = (item - z * w.n_fillblk) * sk_fill_rows(RM), m_hi = min(m_lo + sk_fill_rows(RM), p.M);
+            if constexpr (RM)
+                fill_rowmajor_tiles<DT, NT>(p, z, p.n_all_u, m_lo, m_hi, tid);
+            else
+                fill_kmajor<DT, NT>(p, p.act, fill_tile(p, z), m_lo, m_hi, tid, false);
+        }
         return;
     }
     const int die = blockIdx.x % kXcd;

@@ -306,18 +306,8 @@ __global__ void __launch_bounds__(64 * kBsWaves, 4)
 
     // ---- TW_PRUNED_ZERO: the pruned columns of this unit's share of the tiles receive act(bias)
     // on the range's rows
-    for (int z = p.n_gemm_u + ui; z < p.n_all_u; z += n_units) {
-        const TileDev t = p.tiles[z - p.n_gemm_u];
-        const int chunks = (m_hi - m_lo + 7) / 8;
-        for (int i = tid; i < t.n_pruned * chunks; i += 64 * kBsMulWaves) {
-            const int jz = i / chunks, ch = i - jz * chunks;
-            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
-            const uint32_t hb = E::to_bits(tw_finish(0.0f, p.bias, c, p.act));
-            const uint32_t w = hb | (hb << 16);
-            store_chunk(C + (int64_t)c * p.ldc + m_lo + ch * 8, u32x4{w, w, w, w}, m_lo + ch * 8, m_hi,
-                        p.store_through != 0);
-        }
-    }
+    for (int z = ui; z < p.n_all_u - p.n_gemm_u; z += n_units)
+        fill_kmajor<DT, 64 * kBsMulWaves>(p, p.act, fill_tile(p, z), m_lo, m_hi, tid, p.store_through != 0);
 }
 
 // ---------------------------------------------------------------------------------
@@ -639,18 +629,8 @@ __global__ void __launch_bounds__(bw_threads(NS), 3)
         done[wave] = 0x7fffffff;
 
     // ---- TW_PRUNED_ZERO: the pruned columns of this unit's share of the tiles receive act(bias)
-    for (int z = p.n_gemm_u + ui; z < p.n_all_u; z += n_units) {
-        const TileDev t = p.tiles[z - p.n_gemm_u];
-        const int chunks = (m_hi - m_lo + 7) / 8;
-        for (int i = tid; i < t.n_pruned * chunks; i += 64 * kBwMulWaves) {
-            const int jz = i / chunks, ch = i - jz * chunks;
-            const int c = t.col0 + p.pruned_n[t.pn_off + jz];
-            const uint32_t hb = E::to_bits(tw_finish(0.0f, p.bias, c, ACT));
-            const uint32_t w = hb | (hb << 16);
-            store_chunk(C + (int64_t)c * p.ldc + m_lo + ch * 8, u32x4{w, w, w, w}, m_lo + ch * 8, m_hi,
-                        through && p.store_through);
-        }
-    }
+    for (int z = ui; z < p.n_all_u - p.n_gemm_u; z += n_units)
+        fill_kmajor<DT, 64 * kBwMulWaves>(p, ACT, fill_tile(p, z), m_lo, m_hi, tid, through && p.store_through);
 }
 
 bool bw_takes(const tw_plan *plan, int64_t lda, int64_t ldc, bool reads_c)

@@ -451,16 +451,7 @@ __global__ void __launch_bounds__(kRmThreads, 2)
     }
     // ---- TW_PRUNED_ZERO: pruned columns receive act(beta * C + bias); shared out over the
     // workgroups of a row block
-    for (int z = p.n_gemm_u + grp; z < p.n_all_u; z += gridDim.y) {
-        const TileDev t = p.tiles[z - p.n_gemm_u];
-        for (int i = tid; i < t.n_pruned * m_cnt; i += kRmThreads) {
-            const int m = i / t.n_pruned;
-            const int c = t.col0 + p.pruned_n[t.pn_off + i - m * t.n_pruned];
-            uint16_t *const dst = C + (int64_t)(m0 + m) * p.ldc + c;
-            const float old = p.beta != 0.0f ? p.beta * E::from_bits(*dst) : 0.0f;
-            *dst = (uint16_t)E::to_bits(tw_finish(old, p.bias, c, p.act));
-        }
-    }
+    fill_rowmajor_tiles<DT, kRmThreads>(p, grp, (int)gridDim.y, m0, m0 + m_cnt, tid);
 }
 
 int rm_groups(const tw_plan *plan)
