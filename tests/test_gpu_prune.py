@@ -278,6 +278,22 @@ def test_masks_of_many_layers_made_during_the_call(twprune, po, n_layers):
         assert len(got) == n_layers and all(np.array_equal(w, g) for w, g in zip(want, got)), fn
 
 
+@pytest.mark.parametrize("n_layers", [1, 20, 21, 40, 41])
+def test_tables_in_the_arguments_of_the_norms(twprune, po, n_layers):
+    """As many layers as go to the device with the launch that reads the scores (40, and 20 where a second stage's table goes along),
+    and one more; fewer workgroups than clear the counters and more; the calls before and after it with other tables."""
+    rng = np.random.default_rng(n_layers + 7)
+    for rows in (8, 200):
+        scores = twprune.img2col_forward([rng.standard_normal((int(rng.integers(3, rows)), 4 * int(rng.integers(1, 20)))).astype(np.float32)
+                                          for _ in range(n_layers)])
+        for g in (16, 12):
+            for fn in ("tiled_wise_1d", "tiled_wise_1d_mix", "tiled_wise_1d"):
+                want = getattr(po, fn)(scores, 60, g)
+                want = want[0] if fn != "tiled_wise_1d_mix" else want
+                got = getattr(twprune, fn)(scores, 60, g)
+                assert len(got) == n_layers and all(np.array_equal(w, x) for w, x in zip(want, got)), (fn, rows, g)
+
+
 @pytest.mark.parametrize("fn", ["tiled_wise_1d", "tiled_wise_2d", "tiled_wise_1d_mix"])
 def test_masks_that_cannot_be_made_end_the_call(tw, twprune, monkeypatch, fn):
     """An exception while the masks are made comes out of the producer, and the next call is as ever."""

@@ -264,56 +264,6 @@ __global__ void __launch_bounds__(256, 6)
     }
 }
 
-// The same where every tile of every layer is one block of the sum whose rows are made of whole pieces of 16 bytes
-// (queue_norms): the second item's rows are on their way while the first is added up (226 MB of BERT-base read past the
-// caches: 37 us, 6.1 TB/s; four items 38, the kernel above 40; through the caches 43, 45 and 46).
-constexpr int kNormItems = 2; // of a workgroup, in a row
-template <bool ONCE>
-__global__ void __launch_bounds__(256, 5)
-    block_row_norms_kernel(const PruneLayer *layers, int n_layers, int64_t n_items, int64_t first_wg)
-{
-    __shared__ __align__(16) float stage[kNormRows * kNormPitch];
-    const LayerFinder find(&layers->rt_begin, sizeof(PruneLayer), n_layers);
-    const int tid = (int)threadIdx.x, l8 = tid & 7, grp = tid >> 3, r0 = tid >> 5, q = tid & 31;
-    struct Item {
-        u32x4 v[4]; // the thread's pieces of rows r0 + 8 i
-        TW_GLOBAL(float) out;
-        int nr, w, divide;
-    };
-    auto fetch = [&](int64_t item, Item &d) {
-        const PruneLayer &L = layers[find(item)];
-        const int K = L.K, N = L.N, G = L.granularity, n_tiles = L.n_tiles;
-        const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a call has fewer than 2^31 items)
-        const int rblk = (int)(idx / (uint32_t)n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)n_tiles);
-        const int k0 = rblk * kNormRows, c0 = t * G;
-        d.nr = min(kNormRows, K - k0);
-        d.w = min(G, N - c0);
-        d.divide = !(L.flags & kNormNotDivided);
-        d.out = as_global(L.norms) + (int64_t)t * K + k0;
-        TW_GLOBAL(const float) const src = as_global(L.score) + (int64_t)k0 * N + c0 + min(q * 4, d.w - 4); // (pieces past the last repeat it)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) // (so do rows)
-            d.v[i] = load_global<ONCE>((TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, d.nr - 1) * N));
-    };
-    auto add = [&](const Item &d) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<u32x4 *>(stage + (r0 + i * 8) * kNormPitch + q * 4) = d.v[i];
-        TW_LDS_BARRIER();
-        const float s = pairwise_block(stage + grp * kNormPitch, d.w, l8);
-        if (l8 == 0 && grp < d.nr) // both operations correctly rounded
-            d.out[grp] = d.divide ? sqrtf(s) / (float)d.w : sqrtf(s);
-        TW_LDS_BARRIER(); // the stage is written again
-    };
-    const int64_t first = (first_wg + blockIdx.x) * kNormItems, last = n_items - 1;
-    Item a, b;
-    fetch(first, a);
-    fetch(min(first + 1, last), b);
-    add(a);
-    if (first < last)
-        add(b);
-}
-
 // cnorm[pooled c] = ||score[:, c]|| / K, the rows accumulated in order.  The chain of K additions
 // per column is sequential by definition; everything around it is not: a workgroup takes 32
 // columns; four waves load 64 rows at a time (eight such groups in flight in registers: 64 KB a
@@ -1050,11 +1000,11 @@ struct SetupSelect {
     uint32_t room;
     int32_t pad_;
 };
-__global__ void __launch_bounds__(256)
-    prune_setup_kernel(const Blob a, uint32_t *dst, int words, const SetupSelect first, const SetupSelect second)
+// (`a`, the words, is the kernel's first argument; by the launch's first `workgroups`)
+__device__ __forceinline__ void prune_setup(uint32_t *dst, int words, const SetupSelect &first, const SetupSelect &second, int workgroups)
 {
     const auto *src = (const __attribute__((address_space(4))) uint32_t *)__builtin_amdgcn_kernarg_segment_ptr();
-    const int gtid = (int)(blockIdx.x * blockDim.x + threadIdx.x), nthr = (int)(gridDim.x * blockDim.x);
+    const int gtid = (int)(blockIdx.x * blockDim.x + threadIdx.x), nthr = workgroups * (int)blockDim.x;
     for (int i = gtid; i < words; i += nthr)
         dst[i] = src[i];
     auto begin = [&](const SetupSelect &p) {
@@ -1069,6 +1019,83 @@ __global__ void __launch_bounds__(256)
     };
     begin(first);
     begin(second);
+}
+__global__ void __launch_bounds__(256)
+    prune_setup_kernel(const Blob a, uint32_t *dst, int words, const SetupSelect first, const SetupSelect second)
+{
+    prune_setup(dst, words, first, second, (int)gridDim.x);
+}
+
+// The same where every tile of every layer is one block of the sum whose rows are made of whole pieces of 16 bytes
+// (queue_norms): the second item's rows are on their way while the first is added up (226 MB of BERT-base read past the
+// caches: 37 us, 6.1 TB/s; four items 38, tile_row_norms_kernel 40; through the caches 43, 45 and 46).
+// SETUP: the call's tables are in the arguments, and the first workgroups do on the side what prune_setup_kernel does, so that the call's
+// first launch is the one that reads the scores (masks of twelve BERT-base feed-forward layers 119.6 -> 116.4 us; tables of more than kBlobWords
+// words, and many selections to clear, keep the launch of their own).
+constexpr int kNormItems = 2; // of a workgroup, in a row
+struct NormTable { // on the device
+    const PruneLayer *layers;
+};
+struct NormSetup {
+    Blob a;
+    uint32_t *dst;
+    int32_t words, pad_;
+    SetupSelect first, second;
+};
+constexpr int kNormSetupWgs = 16;
+template <bool ONCE, bool SETUP>
+__global__ void __launch_bounds__(256, 5)
+    block_row_norms_kernel(const std::conditional_t<SETUP, NormSetup, NormTable> from, int n_layers, int64_t n_items, int64_t first_wg)
+{
+    __shared__ __align__(16) float stage[kNormRows * kNormPitch];
+    const PruneLayer *layers;
+    if constexpr (SETUP)
+        layers = (const PruneLayer *)(uintptr_t)__builtin_amdgcn_kernarg_segment_ptr();
+    else
+        layers = from.layers;
+    const LayerFinder find(&layers->rt_begin, sizeof(PruneLayer), n_layers);
+    const int tid = (int)threadIdx.x, l8 = tid & 7, grp = tid >> 3, r0 = tid >> 5, q = tid & 31;
+    struct Item {
+        u32x4 v[4]; // the thread's pieces of rows r0 + 8 i
+        TW_GLOBAL(float) out;
+        int nr, w, divide;
+    };
+    auto fetch = [&](int64_t item, Item &d) {
+        const PruneLayer L = load_entry(layers + find(item));
+        const int K = L.K, N = L.N, G = L.granularity, n_tiles = L.n_tiles;
+        const uint32_t idx = (uint32_t)(item - L.rt_begin); // (a call has fewer than 2^31 items)
+        const int rblk = (int)(idx / (uint32_t)n_tiles), t = (int)(idx - (uint32_t)rblk * (uint32_t)n_tiles);
+        const int k0 = rblk * kNormRows, c0 = t * G;
+        d.nr = min(kNormRows, K - k0);
+        d.w = min(G, N - c0);
+        d.divide = !(L.flags & kNormNotDivided);
+        d.out = as_global(L.norms) + (int64_t)t * K + k0;
+        TW_GLOBAL(const float) const src = as_global(L.score) + (int64_t)k0 * N + c0 + min(q * 4, d.w - 4); // (pieces past the last repeat it)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) // (so do rows)
+            d.v[i] = load_global<ONCE>((TW_GLOBAL(const u32x4))(src + (int64_t)min(r0 + i * 8, d.nr - 1) * N));
+    };
+    auto add = [&](const Item &d) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<u32x4 *>(stage + (r0 + i * 8) * kNormPitch + q * 4) = d.v[i];
+        TW_LDS_BARRIER();
+        const float s = pairwise_block(stage + grp * kNormPitch, d.w, l8);
+        if (l8 == 0 && grp < d.nr) // both operations correctly rounded
+            d.out[grp] = d.divide ? sqrtf(s) / (float)d.w : sqrtf(s);
+        TW_LDS_BARRIER(); // the stage is written again
+    };
+    const int64_t first = (first_wg + blockIdx.x) * kNormItems, last = n_items - 1;
+    Item a, b;
+    fetch(first, a);
+    fetch(min(first + 1, last), b);
+    add(a);
+    if (first < last)
+        add(b);
+    if constexpr (SETUP) {
+        if (first_wg == 0 && blockIdx.x < kNormSetupWgs)
+            prune_setup(from.dst, from.words, from.first, from.second, min((int)gridDim.x, kNormSetupWgs));
+    }
 }
 
 // mask[k][c] = (norm of row k in c's tile > threshold) and column c kept.  A unit of work is 16
@@ -2253,7 +2280,14 @@ CallTable make_table(int n_layers, const int32_t *K, const int32_t *N, const flo
 // 160 + 1433 and 143 + 1449, 340 MB 166 + 1520 and 148 + 1530, 377 MB 178 + 1705 and 158 + 1705.  Below it the plans lose more (226 MB 112 + 988 and
 // 113 + 1022), though masks of scores that were written just before gain from 208 MB on (226 MB 144 and 129).
 constexpr int64_t kStayingBytes = 320 << 20;
-void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n_items, bool last, hipStream_t s)
+// Tables that are not on the device yet, the layers' first.
+struct Tables {
+    const void *host;
+    size_t bytes;
+    void *dev;
+    SetupSelect first, second;
+};
+int queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n_items, bool last, hipStream_t s, const Tables *tables = nullptr)
 {
     bool blocks = n_items == nullptr;
     int64_t bytes = 0;
@@ -2263,10 +2297,28 @@ void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n
     for (const PruneLayer &e : c.layers)
         blocks &= (e.N & 3) == 0 && (e.granularity & 3) == 0 && e.granularity <= 128 && ((uintptr_t)e.score & 15) == 0;
     const int n_layers = (int)c.layers.size();
-    if (blocks) {
-        auto kernel = once ? block_row_norms_kernel<true> : block_row_norms_kernel<false>;
+    if (blocks && tables && tables->bytes <= sizeof(Blob) && tables->first.n_states <= 4) { // (more of them want more workgroups to clear them)
+        NormSetup u;
+        std::memcpy(u.a.w, tables->host, tables->bytes);
+        u.dst = static_cast<uint32_t *>(tables->dev);
+        u.words = (int32_t)((tables->bytes + 3) / 4);
+        u.pad_ = 0;
+        u.first = tables->first;
+        u.second = tables->second;
+        auto kernel = once ? block_row_norms_kernel<true, true> : block_row_norms_kernel<false, true>;
         in_launches((c.n_items + kNormItems - 1) / kNormItems, 256, [&](int64_t first, dim3 grid) {
-            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, d_table, n_layers, c.n_items, first);
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, u, n_layers, c.n_items, first);
+        });
+        TW_HIP(hipGetLastError());
+        return TW_OK;
+    }
+    if (tables)
+        if (const int st = put_table(tables->host, tables->bytes, tables->dev, tables->first, tables->second, s))
+            return st;
+    if (blocks) {
+        auto kernel = once ? block_row_norms_kernel<true, false> : block_row_norms_kernel<false, false>;
+        in_launches((c.n_items + kNormItems - 1) / kNormItems, 256, [&](int64_t first, dim3 grid) {
+            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, NormTable{d_table}, n_layers, c.n_items, first);
         });
     } else {
         auto kernel = once ? tile_row_norms_kernel<true> : tile_row_norms_kernel<false>;
@@ -2274,6 +2326,8 @@ void queue_norms(const CallTable &c, const PruneLayer *d_table, const int64_t *n
             hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, d_table, n_layers, n_items, first);
         });
     }
+    TW_HIP(hipGetLastError());
+    return TW_OK;
 }
 
 // masks of more layers than a launch takes addresses: into the table, before it goes to the device
@@ -2338,11 +2392,11 @@ int uniform_rows(int n_layers, const int32_t *K, const int32_t *N, const float *
         e.norms = d_norms + off;
         off += (int64_t)e.K * e.n_tiles;
     }
-    st = put_table(c.layers.data(), sizeof(PruneLayer) * n_layers, d_table,
-                   setup_of(d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q, q_is_f64), SetupSelect{}, s);
+    const Tables tables{c.layers.data(), sizeof(PruneLayer) * n_layers, d_table,
+                        setup_of(d_st, in_blocks ? 0 : n_seg, c.n_norms / n_seg, q, q_is_f64), SetupSelect{}};
+    st = queue_norms(c, d_table, nullptr, last, s, &tables);
     if (st)
         return st;
-    queue_norms(c, d_table, nullptr, last, s);
     // per-tile thresholds (one layer): every tile's K norms are one segment
     if (in_blocks) {
         auto kernel = K[0] <= 1024 ? tile_select_kernel<1024> : tile_select_kernel<kTileSelect>;
@@ -2747,8 +2801,9 @@ try {
     });
     hipLaunchKernelGGL(plan_2d_kernel, dim3(1), dim3(kPlanThreads), 0, s, d_table, n_layers, d_cnorm, c.n_cols, d_norms,
                        d_st, d_items, q, q_type, mail);
-    queue_norms(c, d_table, d_items, false, s);
-    st = queue_select(d_norms, c.n_norms, d_st, 1, s);
+    st = queue_norms(c, d_table, d_items, false, s);
+    if (!st)
+        st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
     st = queue_fill(c, m, ar, d_table, d_st, nullptr, mail, s);
@@ -2854,11 +2909,10 @@ try {
     std::vector<char> both(table_bytes + mix.table_bytes());
     std::memcpy(both.data(), c.layers.data(), table_bytes);
     std::memcpy(both.data() + table_bytes, mix.table().data(), mix.table_bytes());
-    st = put_table(both.data(), both.size(), d_tables, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup(), s);
-    if (st)
-        return st;
-    queue_norms(c, d_table, nullptr, false, s);
-    st = queue_select(d_norms, c.n_norms, d_st, 1, s);
+    const Tables tables{both.data(), both.size(), d_tables, setup_of(d_st, 1, c.n_norms, sparsity, q_type), mix.setup()};
+    st = queue_norms(c, d_table, nullptr, false, s, &tables);
+    if (!st)
+        st = queue_select(d_norms, c.n_norms, d_st, 1, s);
     if (st)
         return st;
     // (everything that the masks' places are not needed for is on its way when the caller allocates them)
