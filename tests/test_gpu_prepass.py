@@ -128,6 +128,7 @@ def test_plan_from_device_mask_tile_edges(tw, oracle, K, N, widths, offset):
     (1, 1, [1], 0), (3, 5, [2, 3], 1), (1, 15, [15], 3),     # less than sixteen bytes of mask
     (1, 16, [7, 9], 1), (1, 17, [17], 0), (5, 7, [3, 4], 2),  # the last row's pieces start before their place
     (129, 131, [1, 130], 1), (257, 301, [301], 3),            # ... of a slab of one row, of lanes of 16 and 32 a row
+    (129, 1, [1], 1), (130, 3, [3], 0), (391, 2, [1, 1], 3),  # ... of rows in the slab before the last one
 ])
 def test_masks_of_a_few_bytes(tw, oracle, K, N, widths, offset):
     """Masks at any address, to their last byte, of which nothing behind them may be read: tiles without rows, without columns

@@ -336,7 +336,7 @@ template <int UNIT, int LG> __device__ __forceinline__ void flags_of_slab(const 
                     v[p][j] = x[j * 4] | x[j * 4 + 1] << 8 | x[j * 4 + 2] << 16 | x[j * 4 + 3] << 24;
             }
         }
-        if (UNIT == 1 && k0 + nr == a.K) { // what was read before its place, the mask ending there, moves down
+        if (UNIT == 1 && (int64_t)(a.K - k0 - nr) * a.N < 16) { // what was read before its place, the mask ending there, moves down
 #pragma unroll
             for (int p = 0; p < kPasses; ++p) {
                 const int64_t over = (int64_t)(k0 + min(r0 + p * rpp, nr - 1)) * a.N + cc - last16;
