@@ -1526,3 +1526,47 @@ def test_choice_names_queues_of_kernels_that_have_them(tw, oracle):
         for opt in (tw.OPT_SHAPE, tw.OPT_XCD_QUEUES, tw.OPT_BALANCE):
             tw.set_option(opt, -1)
     assert len(seen & queued) >= 5 and len(seen - queued) >= 3
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16, 17, 24, 33, 130])
+@pytest.mark.parametrize("K,k_keep", [(600, 0.3), (900, 0.4)])     # four waves, and eight
+def test_row_major_blocks_of_fewer_rows(tw, oracle, K, k_keep, M, dtype):
+    """The kernel for few rows takes 8, 16 or 32 rows of a row-major A a workgroup, by how many workgroups that makes: last blocks of one
+    row, whole ones, and a plan so wide that 32 remain.  A row that is no number stays in its own row of C, and no row behind
+    the last is written.  The same launch on a single row gives the same bits for every row (the sums do not depend on the block)."""
+    import torch
+    for N in (96, 2048):
+        rng = np.random.default_rng(K + M + N)
+        tiles = random_tiles(rng, K, N, 128, k_keep=k_keep, n_keep=0.9)
+        B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+        A = rng.standard_normal((M, K)).astype(np.float32)
+        lda, ldc, rows = round_up(K, 8), round_up(N, 8), M + 40
+        Ab = np.zeros((M, lda), np.uint16)
+        Ab[:, :K] = oracle.cast_bits(A, dtype).reshape(M, K)
+        if M > 4:
+            Ab[3, :K] = 0x7FFF  # NaN in either type
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+            assert "skinny" in plan.kernel_name(M, lda=lda, ldc=ldc, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR)
+            dA = to_device_bits(Ab, Ab.shape)
+
+            def run(first, m):
+                dC = to_device_bits(np.full((rows, ldc), 0x1234, np.uint16), (rows, ldc))
+                plan.gemm(dA.data_ptr() + first * lda * 2, dC.data_ptr(), m, lda=lda, ldc=ldc, a_layout=tw.ROWMAJOR, c_layout=tw.ROWMAJOR,
+                          pruned_cols=tw.PRUNED_ZERO, stream=torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                got = from_device_bits(dC)
+                assert (got[m:] == 0x1234).all()
+                return got[:m, :N]
+            got = run(0, M)
+            keep = kept_columns(tiles, N)
+            for m in sorted({0, M // 2, M - 1}):
+                if M > 4 and m == 3:
+                    continue
+                assert np.array_equal(got[m], run(m, 1)[0]), (N, m)
+            C = oracle.bits_to_f32(got, dtype).reshape(M, N)
+            good = [m for m in range(M) if not (M > 4 and m == 3)]
+            ref = oracle.quantize(A, dtype).astype(np.float64) @ (oracle.quantize(B, dtype) * oracle.plan_mask(K, N, tiles)).astype(np.float64)
+            assert oracle.rel_error(C[good], ref[good]) <= {"f16": 1e-2, "bf16": 2e-2}[dtype]
+            if M > 4:
+                assert np.isnan(C[3, keep]).all() and (C[3, ~keep] == 0).all()

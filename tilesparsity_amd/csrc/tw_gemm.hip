@@ -1862,7 +1862,7 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 // and everything behind it is the same, bit for bit.  C leaves with the lanes along its columns.
 //   The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
-constexpr int kSkRows = 32;                            // rows m of a workgroup
+constexpr int kSkRows = 32;                            // rows m of a workgroup (row-major: or eight or sixteen, ROWS)
 constexpr int kSkCols = 64;                            // compact columns of a workgroup, or half of them
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
 constexpr int sk_fill_rows(bool rm) { return rm ? 32 : 64; } // rows m of a tile's pruned columns that a workgroup fills
@@ -1878,14 +1878,15 @@ struct SkinnyWork {
     int32_t fill_wgs, n_fillblk; // so many, sk_fill_rows rows of a tile at a time
 };
 
-template <int DT, int NW, bool RM, int NB>
+template <int DT, int NW, bool RM, int NB, int ROWS = kSkRows>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
 {
     constexpr int NT = 64 * NW;
     constexpr int COLS = 32 * NB; // compact columns of a workgroup
     constexpr int STAGE = COLS * kSkPitch * 4;
     static_assert(STAGE >= 64 * 64, "a step of A fits the stage");
-    constexpr int RPT = kSkRows * COLS / NT; // rows of a column a thread adds up and stores: 8, 4 or 2
+    static_assert(ROWS == kSkRows || RM, "a chunk of a K-major row is eight rows m as it is");
+    constexpr int RPT = ROWS * COLS / NT < 2 ? 2 : ROWS * COLS / NT; // rows of a column a thread adds up and stores: 8, 4 or 2
     using E = Elem<DT>;
     __shared__ __align__(16) unsigned char sk_smem[NW * STAGE];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -1926,7 +1927,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     uintptr_t A_i = (uintptr_t)p.A, kk_i = (uintptr_t)p.kept_k, kn_i = (uintptr_t)p.kept_n, Bp_i = (uintptr_t)p.Bp;
     int64_t lda = p.lda, ldc = p.ldc;
     int M = p.M;
-    const int m0 = yblk * kSkRows;
+    const int m0 = yblk * ROWS;
     // the unit: asked for from the kernel arguments before anything else has arrived
     UnitDev u;
     {
@@ -1952,7 +1953,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             uw[i] = __builtin_amdgcn_readfirstlane(uw[i]);
         __builtin_memcpy(&u, uw, sizeof(UnitDev));
     }
-    const int m_end = m0 + kSkRows < M ? m0 + kSkRows : M;
+    const int m_end = m0 + ROWS < M ? m0 + ROWS : M;
     TW_GLOBAL(const uint16_t) const A = (TW_GLOBAL(const uint16_t))A_i;
     uint16_t *const C = reinterpret_cast<uint16_t *>(p.C);
     TW_GLOBAL(const int32_t) const kept_k = (TW_GLOBAL(const int32_t))kk_i;
@@ -1966,7 +1967,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         const bool two_blocks = NB == 2 && half * 2 + 1 < u.nb_cnt;
         unsigned char *const stage = sk_smem + wave * STAGE;
         // the reducing role of this lane: column jj of the half, rows mr .. mr + RPT - 1
-        const int jj = RM ? tid % COLS : tid / (kSkRows / RPT), mr = RM ? tid / COLS * RPT : tid % (kSkRows / RPT) * RPT;
+        const int jj = RM ? tid % COLS : tid / (ROWS / RPT), mr = RM ? tid / COLS * RPT : tid % (ROWS / RPT) * RPT;
         const int cnt = min(COLS, u.n_cnt - half * COLS);
 
         struct Numbers {
@@ -1983,7 +1984,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         TW_GLOBAL(const uint16_t) const a_lane = A + m0 + (m0 + ch * 8 < M ? ch * 8 : 0);
         const int cb_off = two_blocks ? 4096 : 0;
         u32x4 av[RM ? 1 : 4], bv[NB][4];
-        uint32_t ae[RM ? kSkRows : 1];
+        uint32_t ae[RM ? ROWS : 1];
         auto numbers = [&](int s) {
             Numbers n;
             if constexpr (RM) {
@@ -2003,7 +2004,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         auto load_a = [&](const Numbers &n) {
             if constexpr (RM) { // (rows past M repeat the last one; those of the product are not stored)
 #pragma unroll
-                for (int i = 0; i < kSkRows; ++i)
+                for (int i = 0; i < ROWS; ++i)
                     ae[i] = (A + (int64_t)(m0 + i < M ? m0 + i : M - 1) * lda)[(uint32_t)n.row[0]];
             } else {
 #pragma unroll
@@ -2033,12 +2034,12 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             constexpr bool MORE = decltype(more_tag)::value;
             if constexpr (RM) {
                 const uint32_t keep = s * kBlockK + lane < u.k_kept ? 0xFFFFFFFFu : 0u;
-                uint32_t w2[kSkRows / 2];
+                uint32_t w2[ROWS / 2];
 #pragma unroll
-                for (int i = 0; i < kSkRows / 2; ++i)
+                for (int i = 0; i < ROWS / 2; ++i)
                     w2[i] = (ae[2 * i] | (ae[2 * i + 1] << 16)) & keep;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < ROWS / 8; ++i) // (the others are of products that nobody stores)
                     *reinterpret_cast<u32x4 *>(stage + lane * 64 + i * 16) =
                         u32x4{w2[4 * i], w2[4 * i + 1], w2[4 * i + 2], w2[4 * i + 3]};
             } else
@@ -2095,7 +2096,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
 #pragma unroll
         for (int cb = 0; cb < NB; ++cb)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
+            for (int r4 = 0; r4 < ROWS / 8; ++r4) {
                 float *const dst = part + (cb * 32 + (lane & 31)) * kSkPitch + r4 * 8 + (lane >> 5) * 4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -2114,7 +2115,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             for (int e = 0; e < RPT; ++e)
                 sum[e] += src[e];
         }
-        if (jj < cnt && m0 + mr < m_end) {
+        if (jj < cnt && mr < ROWS && m0 + mr < m_end) {
             uint16_t *const dst = RM ? C + (int64_t)(m0 + mr) * ldc + out_col : C + (int64_t)out_col * ldc + m0 + mr;
             const int64_t step_m = RM ? ldc : 1;
             float v[RPT];
@@ -2455,15 +2456,15 @@ int get_option(int option_id) { return option(option_id); }
 
 constexpr int kSkFewSteps = 4; // steps of the longest tile up to which the skinny kernel runs with four waves
 
-// The skinny kernel's work on M rows in pieces of `cols` columns (64 or 32) and its number of workgroups, or -1 where that is more than it
+// The skinny kernel's work on M rows in blocks of `rows`, in pieces of `cols` columns (64 or 32), and its number of workgroups, or -1 where that is more than it
 // numbers: it divides a workgroup's number by `grouped` with a multiplication, exact while number *
 // grouped stays below 2^32.
-static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w, int cols = kSkCols)
+static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w, int cols = kSkCols, int rows = kSkRows)
 {
     w->n_units = plan->n_units;
     w->piece_shift = plan->max_unit_n > 2 * cols ? 2 : plan->max_unit_n > cols ? 1 : 0;
     w->pieces = 1 << w->piece_shift;
-    w->n_rowblk = (M + kSkRows - 1) / kSkRows;
+    w->n_rowblk = (M + rows - 1) / rows;
     w->left = plan->n_units % kXcd;
     w->dies_per_unit = w->left ? kXcd / w->left : 1;
     const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->pieces, grouped_items = grouped * w->n_rowblk;
@@ -2812,12 +2813,38 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     const bool pieces_of_32 = narrow_items >= 0 && skinny_per_die(narrow) * kXcd <= plan->cu_count;
     if (pieces_of_32)
         w = narrow;
+    int64_t wgs = pieces_of_32 ? narrow_items : items;
+    // Row-major A: eight or sixteen rows a workgroup instead of 32 while there is a compute unit for each workgroup.  A kept row of a row-major A
+    // is a load of its own for every m, so that a workgroup is as long as its rows are many (32 loads a step of 64 kept rows, of which each holds the
+    // address pipe as long as one of 1 KB), and the weight they share comes out of the L2.  us with 32 rows and this way: M 1, K 3072,
+    // N 768, a quarter kept 6.8 and 3.8, M 128 (sixteen rows) 7.3 and 5.2; M 64, K 4608, N 512, 0.6 kept 15.5 and 6.9; M 32, K 600, N 4096 4.0 and 3.3;
+    // 126 problems 0.66 of the time in the mean, 1.0 where 32 rows are kept.  The sums are the same, bit for bit.
+    int rows = kSkRows;
+    if (RM && pieces_of_32)
+        for (int fewer = 8; fewer < kSkRows && rows == kSkRows; fewer *= 2) {
+            SkinnyWork small;
+            const int64_t small_items = skinny_work(plan, a.M, &small, kSkCols / 2, fewer);
+            if (small_items >= 0 && skinny_per_die(small) * kXcd <= plan->cu_count) {
+                w = small;
+                wgs = small_items;
+                rows = fewer;
+            }
+        }
     const int threads = few ? 256 : 512;
-    w.gemm_wgs = (int32_t)(pieces_of_32 ? narrow_items : items);
+    w.gemm_wgs = (int32_t)wgs;
     w.n_fillblk = (a.M + sk_fill_rows(RM) - 1) / sk_fill_rows(RM);
     // (a launch of as many workgroups as it takes loops over the rest)
     w.fill_wgs = (int32_t)std::min<int64_t>((int64_t)(a.n_all_u - a.n_gemm_u) * w.n_fillblk, kMaxGridThreads / threads - w.gemm_wgs);
     const dim3 grid((unsigned)(w.gemm_wgs + w.fill_wgs));
+    if constexpr (RM) {
+        if (rows < kSkRows) {
+            auto kernel = rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
+                                    : (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 16> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 16>);
+            hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, a, w);
+            TW_HIP(hipGetLastError());
+            return TW_OK;
+        }
+    }
     if (pieces_of_32 && few)
         hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 1>), grid, dim3(threads), 0, s, a, w);
     else if (pieces_of_32)
