@@ -1570,3 +1570,46 @@ def test_row_major_blocks_of_fewer_rows(tw, oracle, K, k_keep, M, dtype):
             assert oracle.rel_error(C[good], ref[good]) <= {"f16": 1e-2, "bf16": 2e-2}[dtype]
             if M > 4:
                 assert np.isnan(C[3, keep]).all() and (C[3, ~keep] == 0).all()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 16, 17, 24, 33, 130])
+@pytest.mark.parametrize("K,k_keep", [(600, 0.3), (900, 0.4)])     # four waves, and eight
+def test_k_major_blocks_of_fewer_rows(tw, oracle, K, k_keep, M, dtype):
+    """The same of a K-major A, whose rows of a block are one, two or four pieces of a kept row: neither a column that is no number, nor
+    the padding behind the last, nor a row that no tile keeps reaches another's result, nothing behind the last column of C is written,
+    and a column alone gives the same bits as among the others."""
+    import torch
+    for N in (96, 1024, 4096):
+        rng = np.random.default_rng(K + M + N)
+        tiles = random_tiles(rng, K, N, 128, k_keep=k_keep, n_keep=0.9)
+        B = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+        A = rng.standard_normal((M, K)).astype(np.float32)
+        bits = oracle.cast_bits(A, dtype).reshape(M, K)
+        mask = oracle.plan_mask(K, N, tiles)
+        bits[:, ~mask.astype(bool).any(1)] = 0x7FFF  # NaN in either type
+        if M > 4:
+            bits[3] = 0x7FFF
+        with tw.Plan.create(K, N, dtype, tiles, B) as plan:
+
+            def run(rows):
+                m, ld = rows.shape[0], round_up(rows.shape[0], 8) + 8
+                assert "skinny" in plan.kernel_name(m, lda=ld, ldc=ld)
+                At = np.full((K, ld), 0x7FFF, np.uint16)
+                At[:, :m] = rows.T
+                dA, dC = to_device_bits(At, (K, ld)), to_device_bits(np.full((N, ld), 0x1234, np.uint16), (N, ld))
+                plan.gemm(dA.data_ptr(), dC.data_ptr(), m, lda=ld, ldc=ld, pruned_cols=tw.PRUNED_ZERO, stream=torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                got = from_device_bits(dC)
+                assert (got[:, m:] == 0x1234).all()
+                return np.ascontiguousarray(got[:, :m].T)
+            got = run(bits)
+            keep = kept_columns(tiles, N)
+            good = [m for m in range(M) if not (M > 4 and m == 3)]
+            for m in sorted({0, M // 2, M - 1} & set(good)):
+                assert np.array_equal(got[m], run(bits[m:m + 1])[0]), (N, m)
+            C = oracle.bits_to_f32(got, dtype).reshape(M, N)
+            ref = oracle.quantize(A, dtype).astype(np.float64) @ (oracle.quantize(B, dtype) * mask).astype(np.float64)
+            assert oracle.rel_error(C[good], ref[good]) <= {"f16": 1e-2, "bf16": 2e-2}[dtype]
+            if M > 4:
+                assert np.isnan(C[3, keep]).all() and (C[3, ~keep] == 0).all()

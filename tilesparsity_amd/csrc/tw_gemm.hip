@@ -1862,7 +1862,7 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 // and everything behind it is the same, bit for bit.  C leaves with the lanes along its columns.
 //   The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
-constexpr int kSkRows = 32;                            // rows m of a workgroup (row-major: or eight or sixteen, ROWS)
+constexpr int kSkRows = 32;                            // rows m of a workgroup (or eight or sixteen, ROWS)
 constexpr int kSkCols = 64;                            // compact columns of a workgroup, or half of them
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
 constexpr int sk_fill_rows(bool rm) { return rm ? 32 : 64; } // rows m of a tile's pruned columns that a workgroup fills
@@ -1885,7 +1885,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     constexpr int COLS = 32 * NB; // compact columns of a workgroup
     constexpr int STAGE = COLS * kSkPitch * 4;
     static_assert(STAGE >= 64 * 64, "a step of A fits the stage");
-    static_assert(ROWS == kSkRows || RM, "a chunk of a K-major row is eight rows m as it is");
+    constexpr int CH = ROWS / 8, KPL = 64 / CH; // K-major: pieces of eight rows m of a kept row, kept rows of a wave's load
     constexpr int RPT = ROWS * COLS / NT < 2 ? 2 : ROWS * COLS / NT; // rows of a column a thread adds up and stores: 8, 4 or 2
     using E = Elem<DT>;
     __shared__ __align__(16) unsigned char sk_smem[NW * STAGE];
@@ -1971,19 +1971,19 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         const int cnt = min(COLS, u.n_cnt - half * COLS);
 
         struct Numbers {
-            int row[RM ? 1 : 4]; // rows of A this lane fetches a chunk of: kept row i * 16 + lane / 4 of the step (RM: kept row `lane`)
+            int row[RM ? 1 : CH]; // rows of A this lane fetches a chunk of: kept row i * KPL + lane / CH of the step (RM: kept row `lane`)
         };
         TW_GLOBAL(const unsigned char) const bsrc = Bp + u.b_off * 2 +
                                           (int64_t)(u.nb0 + half * NB) * 4096 + lane * 16;
         const int64_t step_b = (int64_t)u.nblk * 4096;
-        const int ch = lane & 3, row16 = lane >> 2;
+        const int ch = lane % CH, row_of = lane / CH;
         // Nothing on the way to the operands is conditional, so that the waits between the loads
         // are exact counts: a chunk of rows past M is fetched from the row block's first chunk
         // instead (those rows of the product are never stored), and a second block the half does not
         // have repeats the first (and is not stored).
         TW_GLOBAL(const uint16_t) const a_lane = A + m0 + (m0 + ch * 8 < M ? ch * 8 : 0);
         const int cb_off = two_blocks ? 4096 : 0;
-        u32x4 av[RM ? 1 : 4], bv[NB][4];
+        u32x4 av[RM ? 1 : CH], bv[NB][4];
         uint32_t ae[RM ? ROWS : 1];
         auto numbers = [&](int s) {
             Numbers n;
@@ -1991,8 +1991,8 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                 n.row[0] = kept_k[u.kk_off + s * kBlockK + lane];
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    n.row[i] = kept_k[u.kk_off + s * kBlockK + i * 16 + row16];
+                for (int i = 0; i < CH; ++i)
+                    n.row[i] = kept_k[u.kk_off + s * kBlockK + i * KPL + row_of];
             }
             return n;
         };
@@ -2008,7 +2008,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                     ae[i] = (A + (int64_t)(m0 + i < M ? m0 + i : M - 1) * lda)[(uint32_t)n.row[0]];
             } else {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < CH; ++i)
                     av[i] = *(TW_GLOBAL(const u32x4))(a_lane + (int64_t)n.row[i] * lda);
             }
         };
@@ -2029,7 +2029,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
         // (the tile's list of kept rows is padded to whole steps with row 0: what was fetched for
         // the padding is replaced by zeros here, so that no value of a row the tile does not keep,
         // finite or not, ever reaches a product)
-        const int k_lim = u.k_kept - row16;
+        const int k_lim = u.k_kept - row_of;
         auto multiply = [&](int s, Numbers &n, auto more_tag) {
             constexpr bool MORE = decltype(more_tag)::value;
             if constexpr (RM) {
@@ -2044,10 +2044,10 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
                         u32x4{w2[4 * i], w2[4 * i + 1], w2[4 * i + 2], w2[4 * i + 3]};
             } else
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t keep = s * kBlockK + i * 16 < k_lim ? 0xFFFFFFFFu : 0u;
+            for (int i = 0; i < CH; ++i) {
+                const uint32_t keep = s * kBlockK + i * KPL < k_lim ? 0xFFFFFFFFu : 0u;
                 const u32x4 v = av[i];
-                *reinterpret_cast<u32x4 *>(stage + (i * 16 + row16) * 64 + ch * 16) =
+                *reinterpret_cast<u32x4 *>(stage + (i * KPL + row_of) * 64 + ch * 16) =
                     u32x4{v.x & keep, v.y & keep, v.z & keep, v.w & keep};
             }
             if (MORE) {
@@ -2110,7 +2110,7 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
             sum[e] = 0.0f;
 #pragma unroll
         for (int v = 0; v < NW; ++v) {
-            const float *const src = reinterpret_cast<const float *>(sk_smem + v * STAGE) + jj * kSkPitch + mr;
+            const float *const src = reinterpret_cast<const float *>(sk_smem + v * STAGE) + (jj < COLS ? jj : 0) * kSkPitch + mr;
 #pragma unroll
             for (int e = 0; e < RPT; ++e)
                 sum[e] += src[e];
@@ -2814,17 +2814,22 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     if (pieces_of_32)
         w = narrow;
     int64_t wgs = pieces_of_32 ? narrow_items : items;
-    // Row-major A: eight or sixteen rows a workgroup instead of 32 while there is a compute unit for each workgroup.  A kept row of a row-major A
-    // is a load of its own for every m, so that a workgroup is as long as its rows are many (32 loads a step of 64 kept rows, of which each holds the
-    // address pipe as long as one of 1 KB), and the weight they share comes out of the L2.  us with 32 rows and this way: M 1, K 3072,
+    // Eight or sixteen rows a workgroup instead of 32 while there is a compute unit for each workgroup.  The weight they share comes out of the L2.
+    // The sums are the same, bit for bit.
+    // Row-major A: a kept row is a load of its own for every m, so that a workgroup is as long as its rows are many (32 loads a step of 64 kept
+    // rows, of which each holds the address pipe as long as one of 1 KB).  us with 32 rows and this way: M 1, K 3072,
     // N 768, a quarter kept 6.8 and 3.8, M 128 (sixteen rows) 7.3 and 5.2; M 64, K 4608, N 512, 0.6 kept 15.5 and 6.9; M 32, K 600, N 4096 4.0 and 3.3;
-    // 126 problems 0.66 of the time in the mean, 1.0 where 32 rows are kept.  The sums are the same, bit for bit.
+    // 126 problems 0.66 of the time in the mean, 1.0 where 32 rows are kept.
+    // K-major A: a step of A is one or two loads instead of four, stored and read that much shorter.  us with 32 rows and this way:
+    // M 1, K 3072, N 768, 0.6 kept 5.3 and 4.05; M 16, K 768, N 768 3.3 and 3.0; M 32, K 8192, N 1024 8.2 and 7.2; M 48, K 4096, N 512, a quarter
+    // kept 4.2 and 3.8; 300 problems of M 1 - 250 0.94 in the mean, worst 1.01.  Here only up to 5/8 of the compute units: each workgroup asks for as many lines of A
+    // as one of 32 rows did, and with more of them the L2 falls behind: 192 workgroups 1.19 (M 64, K 3072, N 768), 256 1.25 (M 128, K 4608, N 512).
     int rows = kSkRows;
-    if (RM && pieces_of_32)
+    if (pieces_of_32)
         for (int fewer = 8; fewer < kSkRows && rows == kSkRows; fewer *= 2) {
             SkinnyWork small;
             const int64_t small_items = skinny_work(plan, a.M, &small, kSkCols / 2, fewer);
-            if (small_items >= 0 && skinny_per_die(small) * kXcd <= plan->cu_count) {
+            if (small_items >= 0 && skinny_per_die(small) * kXcd <= (RM ? plan->cu_count : plan->cu_count * 5 / 8)) {
                 w = small;
                 wgs = small_items;
                 rows = fewer;
@@ -2836,16 +2841,11 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
     // (a launch of as many workgroups as it takes loops over the rest)
     w.fill_wgs = (int32_t)std::min<int64_t>((int64_t)(a.n_all_u - a.n_gemm_u) * w.n_fillblk, kMaxGridThreads / threads - w.gemm_wgs);
     const dim3 grid((unsigned)(w.gemm_wgs + w.fill_wgs));
-    if constexpr (RM) {
-        if (rows < kSkRows) {
-            auto kernel = rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
-                                    : (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 16> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 16>);
-            hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, a, w);
-            TW_HIP(hipGetLastError());
-            return TW_OK;
-        }
-    }
-    if (pieces_of_32 && few)
+    if (rows < kSkRows) {
+        auto kernel = rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
+                                : (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 16> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 16>);
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, a, w);
+    } else if (pieces_of_32 && few)
         hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 4, RM, 1>), grid, dim3(threads), 0, s, a, w);
     else if (pieces_of_32)
         hipLaunchKernelGGL((tw_gemm_skinny_kernel<DT, 8, RM, 1>), grid, dim3(threads), 0, s, a, w);
