@@ -499,6 +499,66 @@ def test_multi_step_launch_with_its_rows_in_lds(tw, oracle, M, I, H, k_keep, T, 
     assert oracle.rel_error(dC[:, :M].cpu().numpy(), oC[:, :M].cpu().numpy()) <= 2 * TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_multi_step_launch_with_its_rows_in_lds_nonfinite(tw, oracle, dtype):
+    """The sixteen kept rows of a tile that go over from rows of x to rows of h take part in the products of both: an infinite weight on
+    either side of the border, in f16 also a finite one beyond its range, is multiplied by its own row alone, an infinite x reaches
+    the one gate that keeps its row and no other of the workgroup, and neither rows of x and h that no tile keeps nor those behind a list's
+    end reach anything.  The single-step launches are the measure; infinities saturate the gate i, so that all states but the
+    ones whose bias is a NaN stay finite."""
+    import torch
+    rng = np.random.default_rng(5)
+    M, I, H, G, T = 40, 256, 1024, 128, 24
+    K, ld = I + H, 40
+    W, bias, tiles, xs, h0, c0, A, c = _sequence_problem(rng, oracle, M, I, H, G, 0.25, T, dtype, ld)
+    W *= 0.25  # (as above)
+    no_x, no_h, unit = 17, I + 700, 700       # rows that no tile keeps; the hidden unit of the latter
+    inf_x = 33                                # kept by the first tile of gate i alone
+    border = (I - 1, I)                       # the last row of x and the first of h: both kept by every tile of gate i
+    for t, tile in enumerate(tiles):
+        rows = np.setdiff1d(tile["kept_k"], (no_x, no_h, inf_x) + border)
+        # 16 n + 3 .. 13 rows of x: the border lies inside a group of sixteen, in either half of it
+        x, h = rows[rows < I], rows[rows >= I]
+        x = x[:len(x) // 16 * 16 - 16 + (3, 8, 13, 7)[t % 4] - 1 - (t == 0)]
+        tile["kept_k"] = np.sort(np.concatenate([x, border, h, [inf_x] if t == 0 else []])).astype(np.int32)
+        assert (tile["kept_k"] < I).sum() % 16 == (3, 8, 13, 7)[t % 4]
+    assert 150 <= np.mean([len(t["kept_k"]) for t in tiles]) and max(len(t["kept_k"]) for t in tiles) <= 512
+    big = 7.0e4 if dtype == "f16" else np.inf
+    for j, col in enumerate(rng.choice(np.arange(G, H), 40, replace=False)):  # (gate i: sigmoid of +-inf is 0 or 1)
+        W[border[j & 1], col] = (np.inf, -np.inf, big, -big)[j >> 1 & 3]
+    A[:T, no_x, :M] = oracle.cast_bits(np.full(1, np.nan, np.float32), dtype)[0]
+    A[:T, inf_x, :M] = oracle.cast_bits(np.full(1, np.inf, np.float32), dtype)[0]
+    bias[unit] = np.nan
+    # (no zero meets an infinite weight, and no h whose sign its rounding could turn: unit 0 grows from above zero)
+    for t in range(T):
+        x = A[t, border[0], :M]
+        x[(x & 0x7FFF) == 0] = 0x3C00
+    bias[[0, H, 2 * H, 3 * H]] = 4.0
+    A[0, I, :M] &= 0x7FFF
+    A[0, I, :M] |= 0x3000
+    c[0, :M] = np.abs(c[0, :M]) + 0.5
+    dbias = torch.from_numpy(bias).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    with tw.Plan.create(K, 4 * H, dtype, tiles, W) as plan:
+        print("rows in LDS, nonfinite", dtype, flush=True)
+        dA, dC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        plan.lstm_steps(T, dA.data_ptr(), M, dC.data_ptr(), lda=ld, a_step=K * ld, ldc=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        plan.lstm_steps_status(s)
+        oA, oC = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+        for t in range(T):
+            plan.lstm_step(oA[t].data_ptr(), M, oC.data_ptr(), oC.data_ptr(), oA[t + 1, I].data_ptr(), lda=ld,
+                           ldc_prev=ld, ldc_new=ld, ldh=ld, bias_ptr=dbias.data_ptr(), stream=s)
+        torch.cuda.synchronize()
+    units = np.arange(H) != unit
+    got = oracle.bits_to_f32(np.ascontiguousarray(from_device_bits(dA)[1:, I:, :M]), dtype).reshape(T, H, M)
+    want = oracle.bits_to_f32(np.ascontiguousarray(from_device_bits(oA)[1:, I:, :M]), dtype).reshape(T, H, M)
+    assert np.isnan(want[:, unit]).all() and np.isnan(got[:, unit]).all()
+    assert np.isfinite(want[:, units]).all()
+    assert np.isfinite(got[:, units]).all()
+    assert oracle.rel_error(got[:, units], want[:, units]) <= 2 * TOL[dtype]
+    assert oracle.rel_error(dC.cpu().numpy()[units, :M], oC.cpu().numpy()[units, :M]) <= 2 * TOL[dtype]
+
+
 def test_multi_step_launch_in_a_graph(tw, oracle):
     """tw_lstm_steps records into a HIP graph (its fill of the rows of h is a kernel, not a memset):
     the graph is replayed four times on inputs restored in between, with eager launches of the same

@@ -719,7 +719,8 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const
 //           next step's rows of x leave, from the waves that have a group less; meeting; cell, h stored; meeting; products of the
 //           groups with rows of x while h travels.
 //   groups: a wave's weight fragments stay in registers, its groups with rows of x in blocks of four from the first slot on, those with rows
-//           of h from the last on; a group with both is in either, each time with zeros for the other's rows.
+//           of h from the last on; a group with both is in either, each time with zeros for the other's rows, of A and of the
+//           weight (zeros of A alone would make a NaN of an infinite weight).
 //   edges:  a row of zeros stands for the padding of a list and for a slot without a group; rows and pieces that are not there get
 //           an offset beyond the buffer and arrive as zeros.
 // A row of h is looked at by its dwords: a thread stores two rows m of a hidden unit as one dword, and neither half of a stored
@@ -838,8 +839,16 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_panel_kernel(const
                 const bool of_x = x < nx;
                 const int g = of_x ? x0 + x : j < nh ? h0 + j : -1;
                 bq[b][i] = u32x4{0u, 0u, 0u, 0u};
-                if (g >= 0)
-                    bq[b][i] = *(TW_GLOBAL(const u32x4))(bsrc + (g >> 2) * blk.step_b + (g & 3) * 1024);
+                if (g >= 0) {
+                    const u32x4 whole = *(TW_GLOBAL(const u32x4))(bsrc + (g >> 2) * blk.step_b + (g & 3) * 1024);
+                    // (of the lane's eight kept rows the first `with_x` are rows of x)
+                    const int with_x = min(max(n_xrows - (g * 16 + (lane >> 5) * 8), 0), 8);
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t x_rows = (with_x > 2 * d ? 0xFFFFu : 0u) | (with_x > 2 * d + 1 ? 0xFFFF0000u : 0u);
+                        bq[b][i][d] = whole[d] & (of_x ? x_rows : ~x_rows);
+                    }
+                }
                 at[b][i] = 0;
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
