@@ -146,6 +146,32 @@ def test_pruned_columns_beside_few_rows(tw, oracle, M, beta, row_major):
         tw.set_option(tw.OPT_SHAPE, -1)
 
 
+@pytest.mark.parametrize("shape,row_major", [(sh, False) for sh in (0, 1, 2, 3, 4, 5, 6, 9)] + [(9, True), (13, True)])
+def test_pruned_columns_keep_the_sign_of_a_zero(tw, oracle, shape, row_major):
+    """beta * C of a pruned column, without a bias, is what is stored: a zero of either sign stays one of that sign in every kernel that
+    fills pruned columns and reads C."""
+    rng = np.random.default_rng(shape)
+    M, K, N, G = 136, 320, 256, 128
+    A = rng.standard_normal((M, K)).astype(np.float32)
+    B = (rng.standard_normal((K, N)) * 0.08).astype(np.float32)
+    tiles = random_tiles(rng, K, N, G, k_keep=0.4, n_keep=0.5)
+    keep = kept_columns(tiles, N)
+    C0 = rng.choice(np.array([-0.0, 0.0, -1.5, 2.0], np.float32), (M, N))
+    lay = tw.ROWMAJOR if row_major else tw.KMAJOR
+    try:
+        tw.set_option(tw.OPT_SHAPE, shape)
+        with tw.Plan.create(K, N, "f16", tiles, B) as plan:
+            print(plan.kernel_name(M, lda=round_up(K if row_major else M, 8), ldc=round_up(N if row_major else M, 8),
+                                   a_layout=lay, c_layout=lay, beta=1.0), flush=True)
+            for beta in (1.0, -0.5):
+                C = run(tw, oracle, plan, A, "f16", N, None, 0, beta=beta, C0=C0, row_major=row_major)
+                want = np.float32(beta) * C0
+                assert np.array_equal(C[:, ~keep], want[:, ~keep])
+                assert np.array_equal(np.signbit(C[:, ~keep]), np.signbit(want[:, ~keep]))
+    finally:
+        tw.set_option(tw.OPT_SHAPE, -1)
+
+
 def test_untouched_columns_stay_untouched(tw, oracle):
     rng = np.random.default_rng(32)
     M, K, N, G = 256, 128, 256, 128

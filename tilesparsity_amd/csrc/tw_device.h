@@ -213,6 +213,10 @@ __device__ __forceinline__ UnitDev unit_of_words(const GemmArgs &p, int uv, int 
 // every row, what a fill added to the product was, in us, and is: M 6272, K 3072, N 768, half of the columns pruned, 256 x 64 streaming
 // kernel 10.9 and 3.8; K 768, N 3072 row-major, A-stationary 26.6 and 10.1; M 1024 7.1 and 3.2; M 6272, K 4096, N 8192, row-major streaming 85 and 28;
 // a tenth pruned, M 6272, K 3072, N 768 3.6 and 2.0.)
+
+// Added where there is no bias: the zero that leaves every value as it is, -0 too.
+constexpr float kNoBias = -0.0f;
+
 // Tile z of the fill table, or, past the end, one without columns.
 __device__ __forceinline__ TileDev fill_tile(const GemmArgs &p, int z)
 {
@@ -245,7 +249,7 @@ template <int DT> __device__ __forceinline__ void fill_kmajor(const GemmArgs &p,
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            b[j] = p.bias ? p.bias[max(c[j], 0)] : 0.0f;
+            b[j] = p.bias ? p.bias[max(c[j], 0)] : kNoBias;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (c[j] < 0)
@@ -304,7 +308,7 @@ template <int DT, int NT> __device__ __forceinline__ void fill_rowmajor_tiles(co
                 c[j] = q < t[j].n_pruned ? t[j].col0 + p.pruned_n[t[j].pn_off + q] : -1;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                b[j] = p.bias ? p.bias[max(c[j], 0)] : 0.0f;
+                b[j] = p.bias ? p.bias[max(c[j], 0)] : kNoBias;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 v[j] = (uint16_t)E::to_bits(tw_activate(0.0f + b[j], p.act));

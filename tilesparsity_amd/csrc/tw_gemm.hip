@@ -657,7 +657,7 @@ __global__ void __launch_bounds__(BM == 128 ? 256 : 512, 2) tw_gemm_ws_kernel(co
 #pragma unroll 1
         for (int j = tid / CPR; j < t.n_pruned; j += NT / CPR) {
             const int c = t.col0 + p.pruned_n[t.pn_off + j];
-            const float b = p.bias ? p.bias[c] : 0.0f;
+            const float b = p.bias ? p.bias[c] : kNoBias;
             uint16_t *dst = C + (int64_t)c * p.ldc + m;
             u32x4 v;
             if (p.beta == 0.0f) {
