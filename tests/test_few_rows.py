@@ -1,0 +1,91 @@
+"""The workgroups of the kernel for few rows, walked on the CPU: the header that the kernel and its launch are built from is
+compiled for the host with a program that enumerates what they take."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tilesparsity_amd", "csrc")
+HEAD = r"""
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+namespace tw { constexpr int kXcd = 8; constexpr int64_t kMaxGridThreads = 0xFFFFFFFFll; }
+#include "tw_few_rows.h"
+using namespace tw;
+"""
+
+FILLS = HEAD + r"""
+int main()
+{
+    // every item of a fill once, the launch as large as it likes and cut to a few workgroups
+    for (int n_tiles : {0, 1, 2, 7, 40})
+        for (int M : {1, 32, 33, 64, 65, 1000})
+            for (int rm = 0; rm < 2; ++rm)
+                for (int most : {0, 1, 3, 16, 17}) {
+                    SkinnyWork w{};
+                    skinny_fill(&w, n_tiles, M, rm, 512);
+                    if (most && w.fill_wgs > most) {
+                        w.fill_wgs = most;
+                        w.step_z = most / w.n_fillblk, w.step_blk = most % w.n_fillblk;
+                    }
+                    std::vector<int> seen((size_t)n_tiles * w.n_fillblk, 0);
+                    for (int wg = 0; wg < w.fill_wgs; ++wg)
+                        for (FillPlace at = fill_first(w, wg); at.z < n_tiles; at = fill_next(w, at))
+                            ++seen.at((size_t)at.z * w.n_fillblk + at.blk);
+                    for (int n : seen)
+                        if (n != 1)
+                            return std::printf("%d tiles, M %d, row-major %d, %d workgroups: %d\n", n_tiles, M, rm, w.fill_wgs, n);
+                }
+    // more than 2^31 items, and a product that leaves the fill seven workgroups: the places of some workgroups against their numbers
+    for (int rm = 0; rm < 2; ++rm)
+        for (int n_tiles : {16384, 65536, 1 << 20})
+            for (int M : {1 << 20, (8 << 20) + 1, 0x7fffffff})
+                for (int gemm : {0, 8, 8388600}) {
+                    SkinnyWork w{};
+                    w.gemm_wgs = gemm;
+                    skinny_fill(&w, n_tiles, M, rm, 512);
+                    const int64_t items = (int64_t)n_tiles * w.n_fillblk;
+                    if (w.fill_wgs < 1 || ((int64_t)gemm + w.fill_wgs) * 512 > kMaxGridThreads)
+                        return std::printf("%d workgroups left\n", w.fill_wgs);
+                    for (int wg : {0, w.fill_wgs / 2, w.fill_wgs - 1}) {
+                        int64_t i = wg;
+                        FillPlace at = fill_first(w, wg);
+                        for (int n = 0; n < 100000 && i < items; ++n, i += w.fill_wgs, at = fill_next(w, at))
+                            if (at.z != i / w.n_fillblk || at.blk != i % w.n_fillblk || at.z >= n_tiles)
+                                return std::printf("item %lld of %lld: %d %d\n", (long long)i, (long long)items, at.z, at.blk);
+                        if (i >= items && at.z < n_tiles)
+                            return std::printf("%lld items, and one more: %d %d\n", (long long)items, at.z, at.blk);
+                    }
+                }
+    // the workgroups that multiply never take all of a launch
+    for (int units = 1; units < 100; ++units)
+        for (int M = 1; M > 0 && M < 0x7fffffff - (M >> 3) - 1000; M += (M >> 3) + 997) {
+            SkinnyWork w{};
+            const int64_t wgs = skinny_work(units, 128, M, &w);
+            if (wgs >= 0 && (wgs % 8 || wgs * 512 > kMaxGridThreads || kMaxGridThreads / 512 - wgs < 1))
+                return std::printf("%d units, M %d: %lld\n", units, M, (long long)wgs);
+        }
+    std::printf("ok\n");
+    return 0;
+}
+"""
+
+
+def build(tmp_path, program):
+    compiler = shutil.which("g++")
+    if compiler is None:
+        pytest.skip("no host compiler")
+    src, exe = tmp_path / "few.cpp", tmp_path / "few"
+    src.write_text(program)
+    subprocess.run([compiler, "-std=c++17", "-O1", "-Wno-unknown-pragmas", "-fsanitize=undefined", "-fno-sanitize-recover=undefined",
+                    "-I", CSRC, "-o", str(exe), str(src)], check=True)
+    return str(exe)
+
+
+def test_every_block_of_pruned_columns_is_filled_once(tmp_path):
+    """Also where they number 2^31 and more, and beside a product of as many workgroups as a launch takes."""
+    res = subprocess.run([build(tmp_path, FILLS)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert res.returncode == 0 and res.stdout == "ok\n", res.stdout

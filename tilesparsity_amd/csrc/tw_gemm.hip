@@ -25,6 +25,7 @@
 //   * epilogue: alpha/beta in fp32, round to the 16-bit type, transpose through
 //     LDS, then scatter whole C columns (col0 + kept_n[j]) with 16-byte stores.
 #include "tw_device.h"
+#include "tw_few_rows.h"
 #include "tw_queue.h"
 
 #include <algorithm>
@@ -1862,21 +1863,7 @@ __global__ void __launch_bounds__(64 * as_waves(BMS, RM), 1)
 // and everything behind it is the same, bit for bit.  C leaves with the lanes along its columns.
 //   The sum over k runs in NW slices, so the result can differ from
 // the streaming kernels' in the last bit of fp32 before the rounding to 16 bits.
-constexpr int kSkRows = 32;                            // rows m of a workgroup (or eight or sixteen, ROWS)
-constexpr int kSkCols = 64;                            // compact columns of a workgroup, or half of them
 constexpr int kSkPitch = kSkRows + 4;                  // floats per column of a partial product
-constexpr int sk_fill_rows(bool rm) { return rm ? 32 : 64; } // rows m of a tile's pruned columns that a workgroup fills
-struct SkinnyWork {
-    int32_t n_units, n_rowblk;
-    int32_t pieces, piece_shift; // of a unit: 1, 2 or 4, and its logarithm
-    int32_t grouped;       // items of a row block in whole groups of eight units
-    int32_t grouped_items; // n_rowblk times that
-    uint32_t magic;        // 2^32 / grouped, rounded up
-    int32_t left;          // units left over
-    int32_t dies_per_unit; // kXcd / left
-    int32_t gemm_wgs;      // workgroups that multiply; those behind them fill pruned columns
-    int32_t fill_wgs, n_fillblk; // so many, sk_fill_rows rows of a tile at a time
-};
 
 template <int DT, int NW, bool RM, int NB, int ROWS = kSkRows>
 __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmArgs p, const SkinnyWork w)
@@ -1893,9 +1880,9 @@ __global__ void __launch_bounds__(64 * NW, 4) tw_gemm_skinny_kernel(const GemmAr
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // (w.pieces of a unit: a power of two, COLS columns each)
     if ((int)blockIdx.x >= w.gemm_wgs) {
-        const int n = (p.n_all_u - p.n_gemm_u) * w.n_fillblk;
-        for (int item = (int)blockIdx.x - w.gemm_wgs; item < n; item += w.fill_wgs) {
-            const int z = item / w.n_fillblk, m_lo = (item - z * w.n_fillblk) * sk_fill_rows(RM), m_hi = min(m_lo + sk_fill_rows(RM), p.M);
+        const int n_tiles = p.n_all_u - p.n_gemm_u;
+        for (FillPlace at = fill_first(w, (int)blockIdx.x - w.gemm_wgs); at.z < n_tiles; at = fill_next(w, at)) {
+            const int z = at.z, m_lo = at.blk * sk_fill_rows(RM), m_hi = m_lo + min(sk_fill_rows(RM), p.M - m_lo);
             if constexpr (RM)
                 fill_rowmajor_tiles<DT, NT>(p, z, p.n_all_u, m_lo, m_hi, tid);
             else
@@ -2456,31 +2443,9 @@ int get_option(int option_id) { return option(option_id); }
 
 constexpr int kSkFewSteps = 4; // steps of the longest tile up to which the skinny kernel runs with four waves
 
-// The skinny kernel's work on M rows in blocks of `rows`, in pieces of `cols` columns (64 or 32), and its number of workgroups, or -1 where that is more than it
-// numbers: it divides a workgroup's number by `grouped` with a multiplication, exact while number *
-// grouped stays below 2^32.
 static int64_t skinny_work(const tw_plan *plan, int M, SkinnyWork *w, int cols = kSkCols, int rows = kSkRows)
 {
-    w->n_units = plan->n_units;
-    w->piece_shift = plan->max_unit_n > 2 * cols ? 2 : plan->max_unit_n > cols ? 1 : 0;
-    w->pieces = 1 << w->piece_shift;
-    w->n_rowblk = (M + rows - 1) / rows;
-    w->left = plan->n_units % kXcd;
-    w->dies_per_unit = w->left ? kXcd / w->left : 1;
-    const int64_t grouped = (int64_t)(plan->n_units - w->left) * w->pieces, grouped_items = grouped * w->n_rowblk;
-    const int64_t left_items = w->left ? (int64_t)kXcd * w->pieces * ((w->n_rowblk + w->dies_per_unit - 1) / w->dies_per_unit) : 0;
-    if ((grouped_items + left_items) * 64 * 8 > kMaxGridThreads || grouped_items * grouped >= (1ll << 32))
-        return -1;
-    w->grouped = (int32_t)grouped;
-    w->grouped_items = (int32_t)grouped_items;
-    w->magic = grouped ? (uint32_t)(((1ull << 32) + grouped - 1) / grouped) : 0u;
-    return grouped_items + left_items;
-}
-
-// Workgroups on the die that has most of them.
-static int64_t skinny_per_die(const SkinnyWork &w)
-{
-    return (int64_t)w.grouped / kXcd * w.n_rowblk + (w.left ? (int64_t)w.pieces * ((w.n_rowblk + w.dies_per_unit - 1) / w.dies_per_unit) : 0);
+    return skinny_work(plan->n_units, plan->max_unit_n, M, w, cols, rows);
 }
 
 // Its workgroups to a compute unit of the die that has most of them (second halves that a unit narrower than the
@@ -2837,9 +2802,7 @@ template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const G
         }
     const int threads = few ? 256 : 512;
     w.gemm_wgs = (int32_t)wgs;
-    w.n_fillblk = (a.M + sk_fill_rows(RM) - 1) / sk_fill_rows(RM);
-    // (a launch of as many workgroups as it takes loops over the rest)
-    w.fill_wgs = (int32_t)std::min<int64_t>((int64_t)(a.n_all_u - a.n_gemm_u) * w.n_fillblk, kMaxGridThreads / threads - w.gemm_wgs);
+    skinny_fill(&w, a.n_all_u - a.n_gemm_u, a.M, RM, threads);
     const dim3 grid((unsigned)(w.gemm_wgs + w.fill_wgs));
     if (rows < kSkRows) {
         auto kernel = rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
