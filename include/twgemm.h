@@ -204,9 +204,9 @@ int tw_plan_export(const tw_plan *plan, int32_t *tile_col0, int32_t *tile_width,
                    uint16_t *B_stream);
 
 /* The device memory of a destroyed plan and of what its building needed is kept for the next plans that
- * are built, up to 256 MB a process, and so is the working memory of the mask producers below (as much as
- * the largest call has needed).  It is given back by tw_release_memory, and when an allocation of this library
- * fails.  A plan may be destroyed while products of it are queued, and while a stream is being captured. */
+ * are built, up to 256 MB and 512 pieces a process (then the oldest go), and so is the working memory of the
+ * mask producers below (as much as the largest call has needed).  It is given back by tw_release_memory, and when
+ * an allocation of this library fails.  A plan may be destroyed while products of it are queued, and while a stream is being captured. */
 int tw_plan_destroy(tw_plan *plan);
 
 /* Gives back to the device all memory that no plan and no call holds, for a host program that needs

@@ -520,3 +520,40 @@ def test_plan_memory_is_given_back(tw):
         torch.cuda.synchronize()
     assert torch.equal(last, want)
     tw.release_memory()
+
+
+def test_plan_memory_of_many_sizes_makes_room(tw):
+    """Plans of sizes that nobody builds again, more than the library keeps pieces of: the next plan's memory is kept all the same, the oldest
+    pieces go for it; and what is kept stays within its 256 MB."""
+    import torch
+    K, N = 4096, 8192
+    mask = torch.ones((K, N), dtype=torch.uint8, device="cuda")
+    W = torch.randn((K, N), device="cuda")
+    table = [(c, 128) for c in range(0, N, 128)]
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def build():
+        return tw.Plan.from_device_mask(K, N, mask.data_ptr(), table, "f16", W.data_ptr(), stream=stream)
+
+    def free():
+        torch.cuda.synchronize()
+        return torch.cuda.mem_get_info()[0]
+
+    tw.release_memory()
+    base = free()
+    B = np.ones((64, 32), np.float32)
+    tile = [dict(col0=0, width=32, kept_k=np.arange(64, dtype=np.int32), kept_n=np.arange(32, dtype=np.int32))]
+    small = [tw.Plan.create(64, 32, "f16", tile, B) for _ in range(520)]
+    for p in small:
+        p.destroy()
+    plan = build()
+    held = free()
+    plan.destroy()
+    assert free() - held < 32 << 20            # (64 MB of weight)
+    plans = [build() for _ in range(6)]
+    for p in plans:
+        p.destroy()
+    kept = base - free()
+    assert (128 << 20) <= kept <= (256 << 20) + (32 << 20)
+    tw.release_memory()
+    assert base - free() < 32 << 20

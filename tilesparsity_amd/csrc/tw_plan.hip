@@ -573,7 +573,8 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // products of the new ones on their way stood there until they had run (14 VGG16 layers, masks, plans and first products
 // 1027 us a pass with pieces of up to a megabyte left to the runtime, 873 this way).  So they are kept here when they are given back, up to
 // kPoolBytes and kPoolPieces a process,
-// and go to the next that asks for about as much on that device; what does not fit is freed, and all
+// and go to the next that asks for about as much on that device; at a bound the oldest are freed (a quarter of the pieces at a time: the first of
+// those frees waits for the device), and all
 // of it when an allocation fails or the host program asks for it (tw_release_memory).  Kernels of a plan that is destroyed may still be queued, on any
 // stream or in a graph: its piece is handed out again only behind a wait for the whole device, made by
 // the build that takes it (a build waits anyway) and not by the destruction, which may come in the
@@ -629,24 +630,30 @@ public:
     {
         if (!p)
             return;
-        size_t bytes = 0;
+        std::vector<Piece> gone;
         {
             std::lock_guard<std::mutex> lock(mu_);
             auto it = used_.find(p);
-            if (it != used_.end()) {
-                bytes = it->second;
+            const size_t bytes = it != used_.end() ? it->second : 0;
+            if (it != used_.end())
                 used_.erase(it);
-            }
-        }
-        if (bytes) {
-            std::lock_guard<std::mutex> lock(mu_);
-            if (held_ + bytes <= kPoolBytes && free_.size() < kPoolPieces) {
+            if (bytes && bytes <= kPoolBytes) {
+                // (the oldest: sizes that nobody asks for again would keep all others out)
+                const size_t most = free_.size() < kPoolPieces ? free_.size() : kPoolPieces - kPoolPieces / 4;
+                size_t n = 0;
+                for (; n < free_.size() && (held_ + bytes > kPoolBytes || free_.size() - n > most); ++n)
+                    held_ -= free_[n].bytes;
+                gone.assign(free_.begin(), free_.begin() + n);
+                free_.erase(free_.begin(), free_.begin() + n);
                 free_.push_back(Piece{p, bytes, device, idle, waits_});
                 held_ += bytes;
-                return;
+                p = nullptr;
             }
         }
-        free_now(p);
+        for (const Piece &q : gone)
+            free_now(q.ptr);
+        if (p)
+            free_now(p);
     }
     // what is kept goes back to the device (hipFree waits for work still queued on a destroyed plan: not
     // under the lock, other threads build and destroy plans meanwhile)
