@@ -1,6 +1,10 @@
 """The module that takes Plan.gemm and Plan.lstm_step to the library without ctypes (csrc/tw_call.cpp): plain arguments arrive
 as ctypes would hand them over, any other makes it stand aside."""
 import ctypes
+import os
+import subprocess
+import sys
+import sysconfig
 
 import numpy as np
 import pytest
@@ -73,3 +77,33 @@ def test_a_destroyed_plan_is_refused(tw):
         plan.lstm_step(16, 8, 16, 16, 16)
     with pytest.raises(ctypes.ArgumentError):
         plan.gemm(16, 16, 8.5, lda=8, ldc=8)
+
+
+def test_the_library_without_the_module(tw):
+    """A tree without the module, or with one that another interpreter built: all calls go through ctypes, as a warning says."""
+    code = r"""
+import sys, warnings
+sys.modules["tilesparsity_amd._twcall"] = None
+from tilesparsity_amd import twgemm as tw
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    assert tw.lib() is tw.lib()
+assert len(seen) == 1 and "ctypes" in str(seen[0].message), seen
+plan = tw.Plan(0, 64, 64, 0)
+for call in (lambda: plan.gemm(16, 16, 8), lambda: plan.gemm(16, 16, 8, workspace_ptr=16, workspace_bytes=64),
+             lambda: plan.gemm(16, 16, 8, static=True), lambda: plan.lstm_step(16, 8, 16, 16, 16)):
+    try:
+        call()
+    except tw.TwError as e:
+        assert e.status == tw.ERR_NULL
+    else:
+        raise AssertionError
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+
+
+def test_the_module_is_this_interpreters(tw):
+    """Its name says which interpreter it was built for: another one does not load it."""
+    from tilesparsity_amd import _twcall, build
+    assert _twcall.__file__ == build.CALL_PATH and _twcall.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    assert not os.path.exists(os.path.join(build.PKG_DIR, "_twcall.so"))

@@ -15,7 +15,8 @@ ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 LIB_PATH = os.path.join(PKG_DIR, "libtwgemm.so")
 PERF_PATH = os.path.join(PKG_DIR, "test_basic_nn")
-CALL_PATH = os.path.join(PKG_DIR, "_twcall.so")  # the calls of an inner loop, for twgemm.py
+# the calls of an inner loop, for twgemm.py; named after the interpreter, whose objects it looks into
+CALL_PATH = os.path.join(PKG_DIR, "_twcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 SOURCES = ["tw_host.cpp", "tw_plan.hip", "tw_gemm.hip", "tw_gemm_bs.hip", "tw_gemm_rm.hip", "tw_prune.hip", "tw_cell.hip", "tw_layout.hip", "tw_side.hip"]
 
@@ -90,8 +91,15 @@ def build_perf_driver(verbose=False):
 
 
 def build_call_module(verbose=False):
+    include = sysconfig.get_paths()["include"]
+    untagged = os.path.join(PKG_DIR, "_twcall.so")  # (any interpreter would take one of that name)
+    if os.path.exists(untagged):
+        os.remove(untagged)
+    if not os.path.exists(os.path.join(include, "Python.h")):
+        sys.stderr.write("%s has no Python.h: without _twcall all calls go through ctypes\n" % include)
+        return None
     cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", os.path.join(ROOT, "include"),
-           "-I", sysconfig.get_paths()["include"], os.path.join(CSRC, "tw_call.cpp"), "-o", CALL_PATH]
+           "-I", include, os.path.join(CSRC, "tw_call.cpp"), "-o", CALL_PATH]
     if verbose:
         print(" ".join(cmd))
     _run(cmd)

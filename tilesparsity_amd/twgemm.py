@@ -14,6 +14,7 @@ import ctypes
 import importlib.util
 import os
 import sys
+import warnings
 
 import numpy as np
 
@@ -78,7 +79,7 @@ _lib = None
 
 
 def _call_gemm(*args):
-    """Until the library is loaded: the call goes through ctypes, which loads it."""
+    """Until the library is loaded, and without the module that takes its place then: the call goes through ctypes."""
 
 
 _call_lstm_step = _call_gemm
@@ -198,11 +199,12 @@ def lib():
     try:
         from tilesparsity_amd import _twcall
     except ImportError as e:
-        raise ImportError("%s: build it with `python -m tilesparsity_amd.build`" % e)
-    _twcall.bind(*(ctypes.cast(getattr(L, name), vp).value
-                   for name in ("tw_gemm_ex", "tw_gemm_static", "tw_gemm_staged", "tw_lstm_step")))
-    global _call_gemm, _call_lstm_step
-    _call_gemm, _call_lstm_step = _twcall.gemm, _twcall.lstm_step
+        warnings.warn("%s: Plan.gemm and Plan.lstm_step go through ctypes (build the module with `python -m tilesparsity_amd.build`)" % e)
+    else:
+        _twcall.bind(*(ctypes.cast(getattr(L, name), vp).value
+                       for name in ("tw_gemm_ex", "tw_gemm_static", "tw_gemm_staged", "tw_lstm_step")))
+        global _call_gemm, _call_lstm_step
+        _call_gemm, _call_lstm_step = _twcall.gemm, _twcall.lstm_step
     _lib = L
     return L
 
