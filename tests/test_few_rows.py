@@ -73,6 +73,21 @@ int main()
 }
 """
 
+FORM = HEAD + r"""
+int main(int argc, char **argv) // units, columns of the widest, row-major, M ...: a line of columns and rows of a workgroup for each M
+{
+    for (int i = 4; i < argc; ++i) {
+        SkinnyWork w{};
+        int64_t wgs;
+        const SkinnyForm f = skinny_form(std::atoi(argv[1]), std::atoi(argv[2]), std::atoi(argv[i]), std::atoi(argv[3]), 256, &w, &wgs);
+        if (wgs < 0 || w.n_rowblk != (std::atoi(argv[i]) + f.rows - 1) / f.rows)
+            return 1;
+        std::printf("%d %d\n", f.cols, f.rows);
+    }
+    return 0;
+}
+"""
+
 
 def build(tmp_path, program):
     compiler = shutil.which("g++")
@@ -89,3 +104,25 @@ def test_every_block_of_pruned_columns_is_filled_once(tmp_path):
     """Also where they number 2^31 and more, and beside a product of as many workgroups as a launch takes."""
     res = subprocess.run([build(tmp_path, FILLS)], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     assert res.returncode == 0 and res.stdout == "ok\n", res.stdout
+
+
+def test_what_the_tests_on_the_gpu_launch(tmp_path):
+    """Row blocks of 8, 16 and 32 rows are each among the launches of test_gpu_gemm.py's
+    test_row_major_blocks_of_fewer_rows and test_k_major_blocks_of_fewer_rows, on the 256 compute units of an MI355X."""
+    exe = build(tmp_path, FORM)
+    rows = [1, 7, 8, 9, 16, 17, 24, 33, 130]
+    for row_major, widths in ((1, (96, 2048)), (0, (96, 1024, 4096))):
+        seen = set()
+        for N in widths:
+            cols = round(min(N, 128) * 0.9)
+            out = subprocess.run([exe, str(-(-N // 128)), str(cols), str(row_major)] + [str(m) for m in rows],
+                                 stdout=subprocess.PIPE, text=True, check=True).stdout
+            seen |= {tuple(map(int, line.split())) for line in out.splitlines()}
+        assert seen == {(32, 8), (32, 16), (64, 32)} | (set() if row_major else {(32, 32)}), (row_major, seen)
+
+
+@pytest.mark.gpu
+def test_compute_units_of_the_device(tw):
+    """What the forms above are worked out for."""
+    import torch
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256

@@ -602,6 +602,47 @@ def test_multi_step_launch_in_a_graph(tw, oracle):
     assert oracle.rel_error(got, want_h[-1]) <= 2 * TOL[dtype]
 
 
+def test_multi_step_launch_with_its_rows_in_lds_in_a_graph(tw, oracle):
+    """The same of a sequence that keeps its rows of A in LDS: recorded, replayed four times with eager launches of the plan between the
+    replays, each replay with the eager call's bits."""
+    import torch
+    rng = np.random.default_rng(78)
+    M, I, H, G, T, dtype = 72, 256, 1024, 128, 24, "f16"
+    K, ld = I + H, 72
+    W, bias, tiles, xs, h0, c0, A, c = _sequence_problem(rng, oracle, M, I, H, G, 0.2, T, dtype, ld)
+    assert np.mean([len(t["kept_k"]) for t in tiles]) >= 151 and max(len(t["kept_k"]) for t in tiles) <= 512
+    dbias = torch.from_numpy(bias).cuda()
+    s = torch.cuda.Stream()
+    with tw.Plan.create(K, 4 * H, dtype, tiles, W) as plan:
+        with torch.cuda.stream(s):
+            A0, C0 = to_device_bits(A, A.shape), torch.from_numpy(c.copy()).cuda()
+            dA, dC = A0.clone(), C0.clone()
+            other_a, other_c = A0.clone(), C0.clone()
+
+            def steps(a, cc):
+                plan.lstm_steps(T, a.data_ptr(), M, cc.data_ptr(), lda=ld, a_step=K * ld, ldc=ld,
+                                bias_ptr=dbias.data_ptr(), stream=s.cuda_stream)
+            print("multi-step launch with its rows in LDS, eager then in a graph", flush=True)
+            steps(dA, dC)
+            plan.lstm_steps_status(s.cuda_stream)
+            want_a, want_c = dA.clone(), dC.clone()
+            dA.copy_(A0)
+            dC.copy_(C0)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g, stream=s):
+                steps(dA, dC)
+            for rep in range(4):
+                dA.copy_(A0)
+                dC.copy_(C0)
+                other_c.copy_(C0 + rep)
+                steps(other_a, other_c)
+                s.synchronize()
+                g.replay()
+                plan.lstm_steps_status(s.cuda_stream)
+                assert torch.equal(dA, want_a) and torch.equal(dC, want_c), rep
+    assert not torch.equal(want_a, A0) and torch.isfinite(want_c[:, :M]).all()
+
+
 def test_multi_step_launch_without_the_first_look(tw, oracle):
     """TW_OPT_LSTM_LOOK = 0: the waves fetch a step's rows of h at once and again until none shows
     the fill pattern (the path a wave otherwise takes only for a line that was fetched too early).

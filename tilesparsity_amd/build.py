@@ -59,7 +59,7 @@ def build_library(verbose=False, force=True):
     objdir = os.path.join(PKG_DIR, "build")
     os.makedirs(objdir, exist_ok=True)
     headers = [os.path.join(CSRC, "tw_internal.h"), os.path.join(CSRC, "tw_device.h"), os.path.join(CSRC, "tw_queue.h"),
-               os.path.join(CSRC, "tw_few_rows.h"),
+               os.path.join(CSRC, "tw_few_rows.h"), os.path.join(CSRC, "tw_lstm_form.h"),
                os.path.join(ROOT, "include", "twgemm.h"),
                os.path.abspath(__file__)]
     newest_header = max(os.path.getmtime(h) for h in headers)

@@ -3,6 +3,7 @@
 // the K-major A of the next time step.  Elementwise, 18 bytes per (unit, row): at the sizes of a time step (M = 128, H = 1024: 2.4 MB)
 // the launch itself is most of its time.
 #include "tw_internal.h"
+#include "tw_lstm_form.h"
 
 #include <cstddef>
 #include <cstring>
@@ -730,7 +731,6 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_steps_kernel(const
 // 780 / 1080 (850 / 1180), meeting 420 / 120 (400 / 70), products of x 1230 / 1490 (1490 / 1500): 8770 (10970).  Tried and slower: the loads
 // of x by all waves behind those of h (9770: the waves stand until all are taken before they can look at the rows of h), before the
 // look (9430), ahead of the products (9700), through registers between the products (10360).
-constexpr int kPanRows = 1024;   // most rows of x, and of h
 constexpr int kPanList = 2 * kSeqSteps * kBlockK; // most kept rows of a tile
 constexpr int kPanBlocks = 5;    // blocks of four groups of 16 kept rows a wave multiplies: 16 groups (tiles of at most 512 kept rows), no block with both kinds
 constexpr int kPanLoads = kPanRows / (16 * kLstmWaves); // loads of either kind a wave has
@@ -1337,15 +1337,8 @@ extern "C" int tw_lstm_steps(const tw_plan *plan, int T, void *A, int64_t lda, i
                            A16, lda, a_step, M, H, K, T);
     }
     const dim3 grid((unsigned)(H / 32 * row_blocks)), block(64 * kLstmWaves);
-    // The form with the rows of A in LDS.  It saves up to a fifth of a step and needs 4 - 6 us more to begin with.  us for 50 steps, above
-    // and in LDS, inputs as many as units: H 1024, a quarter kept, M 8 204 and 182, M 128 228 and 200, M 200 275 and 228, M 256 225 and 211; a tenth
-    // M 8 182 and 154, M 128 194 and 159; M 1 a quarter 201 and 195, a tenth 168 and 163; H 512, a quarter, M 128 176 and 158, half 210 and 178, a tenth 147 and 146; H 256
-    // 138 and 145.  24 steps: H 1024, 512 inputs, 154 kept rows, M 2 91 and 85, M 128 97 and 85; 64 inputs, 109 kept 79 and 83.  Below H 1024 with few rows or
-    // few kept rows of h: H 512, 1024 inputs, M 16, 102 of h 77 and 84, M 128, 51 of h 79 and 78; H 768, 768 inputs, M 4, 154 of h 90 and 94.
     const int64_t kept = plan->n_tiles ? plan->kept_k_ptr[plan->n_tiles] / plan->n_tiles : 0; // rows of a tile, in the mean
-    const bool panel = K > H && K - H <= kPanRows && H <= kPanRows && M >= 2 && kept >= 150 &&
-                       (H >= 1024 ? T >= 24 : H >= 512 && T >= 32 && M > 32 && kept * H >= 100 * (int64_t)K);
-    if (panel) {
+    if (lstm_rows_in_lds(K, H, M, T, kept)) {
         const int pst = prepare_device();
         if (pst != TW_OK)
             return pst;

@@ -57,6 +57,49 @@ inline int64_t skinny_per_die(const SkinnyWork &w)
     return (int64_t)w.grouped / kXcd * w.n_rowblk + (w.left ? (int64_t)w.pieces * ((w.n_rowblk + w.dies_per_unit - 1) / w.dies_per_unit) : 0);
 }
 
+// The form a launch takes on `cu` compute units: columns and rows of a workgroup; `w` and the number of workgroups go with it (-1: too many).
+struct SkinnyForm {
+    int32_t cols, rows;
+};
+// Pieces of 32 columns while no compute unit gets two workgroups: a workgroup on a compute unit of its own is bound by what
+// that fetches (50 bytes a clock, 12 KB a step of 64 columns, 8 KB of 32), and the other compute units are idle.  us with
+// pieces of 64 and of 32, K-major and row-major: M 64, K 4608, N 512, half the rows kept 6.5 and 5.0, 12.9 and 12.3; M 64,
+// K 2304, N 256 4.6 and 3.8, 8.1 and 7.7; M 256, K 4096, N 1024 (256 workgroups) 5.1 and 4.7, 9.5 and 9.5; four waves,
+// M 128, K 768, N 768 3.1 and 2.8, 4.5 and 4.1.  From 288 workgroups on 1.02 - 1.20 of the time, and 1.05 - 1.49.
+// Eight or sixteen rows a workgroup instead of 32 while there is a compute unit for each workgroup.  The sums are the same, bit for bit.  us with
+// 32 rows and this way, one plan again and again, 80 plans in turn, and 600 (operands out of the L2s, beside them, and of memory):
+// Row-major A: a kept row is a load of its own for every m, so that a workgroup is as long as its rows are many (32 loads a step of 64 kept
+// rows, of which each holds the address pipe as long as one of 1 KB).  M 1, K 3072, N 768, a quarter kept 6.0 and 3.4, 6.9 and 3.8, 7.9 and 4.7; M 128 (sixteen
+// rows) 6.5 and 4.6, 7.3 and 5.1, 8.7 and 6.0; M 64, K 4608, N 512, 0.6 kept 14.0 and 6.2, 17.7 and 8.0, 18.1 and 8.0; 42 problems 0.58 of the time in the
+// mean and 0.74 at most, with 80 plans 0.62 and 0.79.
+// K-major A: a step of A is one or two loads instead of four, stored and read that much shorter.  M 1, K 3072, N 768, 0.6 kept 4.9 and 3.7, 6.7 and 6.0, 7.5 and 6.8;
+// M 32, K 8192, N 1024 7.6 and 6.8, 15.9 and 13.5, 15.8 and 13.4; M 48, K 4096, N 512, a quarter kept 3.6 and 3.4, 4.8 and 4.5, 6.3 and 5.8; 22 problems 0.89 in the
+// mean, worst 1.02, with 80 plans 0.94 and 1.03 (N 128, 0.1 kept: 3.32 and 3.41).  Here only up to 5/8 of the compute units: each workgroup asks for
+// as many lines of A as one of 32 rows did, and with more of them the L2 falls behind: M 64, K 3072, N 768 (256 workgroups) 4.6 and 5.5 from the L2s, 7.7 and 7.0
+// with 80 plans; 385 workgroups and more 1.3 - 1.8 and 1.1 - 1.5 of the time.
+inline SkinnyForm skinny_form(int n_units, int unit_cols, int M, bool rm, int cu, SkinnyWork *w, int64_t *wgs)
+{
+    SkinnyForm f{kSkCols, kSkRows};
+    *wgs = skinny_work(n_units, unit_cols, M, w);
+    SkinnyWork other;
+    const int64_t narrow = skinny_work(n_units, unit_cols, M, &other, kSkCols / 2);
+    if (*wgs < 0 || narrow < 0 || skinny_per_die(other) * kXcd > cu)
+        return f;
+    f.cols = kSkCols / 2;
+    *w = other;
+    *wgs = narrow;
+    for (int rows = 8; rows < kSkRows; rows *= 2) {
+        const int64_t n = skinny_work(n_units, unit_cols, M, &other, kSkCols / 2, rows);
+        if (n >= 0 && skinny_per_die(other) * kXcd <= (rm ? cu : cu * 5 / 8)) {
+            f.rows = rows;
+            *w = other;
+            *wgs = n;
+            break;
+        }
+    }
+    return f;
+}
+
 // The workgroups that fill the pruned columns of `n_tiles` tiles, behind w->gemm_wgs of `threads` threads.  A launch of as many workgroups as
 // it takes loops over the rest; some are always left, since those that multiply come in eights and 8 * n * 512 is never the limit itself.
 inline void skinny_fill(SkinnyWork *w, int n_tiles, int M, bool rm, int threads)

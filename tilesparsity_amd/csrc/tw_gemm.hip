@@ -2759,53 +2759,22 @@ template <int DT, int BMS, bool RM> static int launch_as(const tw_plan *plan, co
     return TW_OK;
 }
 
-// the skinny kernel: one workgroup per (half of a unit, 32-row block); four waves where no tile has
+// the skinny kernel: one workgroup per piece of a unit and block of rows (skinny_form); four waves where no tile has
 // more than four steps for them
 template <int DT, bool RM> static int launch_skinny(const tw_plan *plan, const GemmArgs &a, hipStream_t s)
 {
     SkinnyWork w;
-    const int64_t items = skinny_work(plan, a.M, &w);
-    if (items < 0)
+    int64_t wgs;
+    const SkinnyForm form = skinny_form(plan->n_units, plan->max_unit_n, a.M, RM, plan->cu_count, &w, &wgs);
+    if (wgs < 0)
         return fail(TW_ERR_SHAPE, "M=%d: more row blocks than the skinny kernel numbers", a.M);
-    const bool few = plan->max_k_pad <= kSkFewSteps * kBlockK;
-    // Pieces of 32 columns while no compute unit gets two workgroups: a workgroup on a compute unit of its own is bound by what
-    // that fetches (50 bytes a clock, 12 KB a step of 64 columns, 8 KB of 32), and the other compute units are idle.  us with
-    // pieces of 64 and of 32, K-major and row-major: M 64, K 4608, N 512, half the rows kept 6.5 and 5.0, 12.9 and 12.3; M 64,
-    // K 2304, N 256 4.6 and 3.8, 8.1 and 7.7; M 256, K 4096, N 1024 (256 workgroups) 5.1 and 4.7, 9.5 and 9.5; four waves,
-    // M 128, K 768, N 768 3.1 and 2.8, 4.5 and 4.1.  From 288 workgroups on 1.02 - 1.20 of the time, and 1.05 - 1.49.
-    SkinnyWork narrow;
-    const int64_t narrow_items = skinny_work(plan, a.M, &narrow, kSkCols / 2);
-    const bool pieces_of_32 = narrow_items >= 0 && skinny_per_die(narrow) * kXcd <= plan->cu_count;
-    if (pieces_of_32)
-        w = narrow;
-    int64_t wgs = pieces_of_32 ? narrow_items : items;
-    // Eight or sixteen rows a workgroup instead of 32 while there is a compute unit for each workgroup.  The weight they share comes out of the L2.
-    // The sums are the same, bit for bit.
-    // Row-major A: a kept row is a load of its own for every m, so that a workgroup is as long as its rows are many (32 loads a step of 64 kept
-    // rows, of which each holds the address pipe as long as one of 1 KB).  us with 32 rows and this way: M 1, K 3072,
-    // N 768, a quarter kept 6.8 and 3.8, M 128 (sixteen rows) 7.3 and 5.2; M 64, K 4608, N 512, 0.6 kept 15.5 and 6.9; M 32, K 600, N 4096 4.0 and 3.3;
-    // 126 problems 0.66 of the time in the mean, 1.0 where 32 rows are kept.
-    // K-major A: a step of A is one or two loads instead of four, stored and read that much shorter.  us with 32 rows and this way:
-    // M 1, K 3072, N 768, 0.6 kept 5.3 and 4.05; M 16, K 768, N 768 3.3 and 3.0; M 32, K 8192, N 1024 8.2 and 7.2; M 48, K 4096, N 512, a quarter
-    // kept 4.2 and 3.8; 300 problems of M 1 - 250 0.94 in the mean, worst 1.01.  Here only up to 5/8 of the compute units: each workgroup asks for as many lines of A
-    // as one of 32 rows did, and with more of them the L2 falls behind: 192 workgroups 1.19 (M 64, K 3072, N 768), 256 1.25 (M 128, K 4608, N 512).
-    int rows = kSkRows;
-    if (pieces_of_32)
-        for (int fewer = 8; fewer < kSkRows && rows == kSkRows; fewer *= 2) {
-            SkinnyWork small;
-            const int64_t small_items = skinny_work(plan, a.M, &small, kSkCols / 2, fewer);
-            if (small_items >= 0 && skinny_per_die(small) * kXcd <= (RM ? plan->cu_count : plan->cu_count * 5 / 8)) {
-                w = small;
-                wgs = small_items;
-                rows = fewer;
-            }
-        }
+    const bool few = plan->max_k_pad <= kSkFewSteps * kBlockK, pieces_of_32 = form.cols < kSkCols;
     const int threads = few ? 256 : 512;
     w.gemm_wgs = (int32_t)wgs;
     skinny_fill(&w, a.n_all_u - a.n_gemm_u, a.M, RM, threads);
     const dim3 grid((unsigned)(w.gemm_wgs + w.fill_wgs));
-    if (rows < kSkRows) {
-        auto kernel = rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
+    if (form.rows < kSkRows) {
+        auto kernel = form.rows == 8 ? (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 8> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 8>)
                                 : (few ? tw_gemm_skinny_kernel<DT, 4, RM, 1, 16> : tw_gemm_skinny_kernel<DT, 8, RM, 1, 16>);
         hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, s, a, w);
     } else if (pieces_of_32 && few)
