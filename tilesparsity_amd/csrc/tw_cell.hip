@@ -839,16 +839,8 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_panel_kernel(const
                 const bool of_x = x < nx;
                 const int g = of_x ? x0 + x : j < nh ? h0 + j : -1;
                 bq[b][i] = u32x4{0u, 0u, 0u, 0u};
-                if (g >= 0) {
-                    const u32x4 whole = *(TW_GLOBAL(const u32x4))(bsrc + (g >> 2) * blk.step_b + (g & 3) * 1024);
-                    // (of the lane's eight kept rows the first `with_x` are rows of x)
-                    const int with_x = min(max(n_xrows - (g * 16 + (lane >> 5) * 8), 0), 8);
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const uint32_t x_rows = (with_x > 2 * d ? 0xFFFFu : 0u) | (with_x > 2 * d + 1 ? 0xFFFF0000u : 0u);
-                        bq[b][i][d] = whole[d] & (of_x ? x_rows : ~x_rows);
-                    }
-                }
+                if (g >= 0)
+                    bq[b][i] = *(TW_GLOBAL(const u32x4))(bsrc + (g >> 2) * blk.step_b + (g & 3) * 1024);
                 at[b][i] = 0;
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
@@ -1015,6 +1007,33 @@ __global__ void __launch_bounds__(64 * kLstmWaves, 1) tw_lstm_panel_kernel(const
     put_zeros();
     clear();
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // the weights of a group with both kinds are cut to the kind of its slot (here, where the loads are through: 1.8 % of 50 steps where each
+    // fragment was cut behind its load)
+    if (n_xrows & 15) {
+        const int border = n_xrows >> 4, with_x = min(max((n_xrows & 15) - (lane >> 5) * 8, 0), 8); // (of the lane's eight kept rows)
+        int at_x = border - x0, at_h = border - h0; // its slots, if the wave has them
+        at_x = at_x < nx ? at_x : -1;
+        at_h = at_h < nh ? at_h : -1;
+        asm volatile("" : "+s"(at_x), "+s"(at_h)); // (compared here: kept from above the results would not fit the scalar registers)
+        uint32_t x_rows[4];
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+            x_rows[d] = (with_x > 2 * d ? 0xFFFFu : 0u) | (with_x > 2 * d + 1 ? 0xFFFF0000u : 0u);
+        auto cut = [&](int b, int i, bool of_x) {
+#pragma unroll
+            for (int d = 0; d < 4; ++d)
+                bq[b][i][d] &= of_x ? x_rows[d] : ~x_rows[d];
+        };
+#pragma unroll
+        for (int b = 0; b < kPanBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (b * 4 + i == at_x)
+                    cut(b, i, true);
+                if ((kPanBlocks - 1 - b) * 4 + i == at_h)
+                    cut(b, i, false);
+            }
+    }
     multiply(std::true_type(), xb, nothing);
     // stores of h a wave has on its way when it waits for its rows of x, which left before them: one of dwords, or of the odd last row, or both
     const int rows_m = min(p.M - m0, 32);
