@@ -429,7 +429,7 @@ def test_builds_beside_a_capture(tw, oracle, mode, threaded):
             p.destroy()
 
 
-@pytest.mark.parametrize("K", [256, 2048])     # a plan below the size whose memory is kept, and one above it
+@pytest.mark.parametrize("K", [256, 2048])     # memory of half a megabyte, and of four
 def test_plan_destroyed_with_products_queued(tw, oracle, K):
     """Products of a plan are still queued on another stream when it is destroyed and a plan of the same
     mask with another weight takes its memory: every queued product is the old plan's."""

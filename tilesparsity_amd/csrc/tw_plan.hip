@@ -571,10 +571,9 @@ static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 // Device memory of plans and of builds.  The runtime maps and unmaps pieces of more than a megabyte anew (25 us for a hipMalloc of 4 MB,
 // 20 - 240 for its hipFree), and hipFree waits for the device whatever the size: a program that replaces its plans and has
 // products of the new ones on their way stood there until they had run (14 VGG16 layers, masks, plans and first products
-// 1027 us a pass with pieces of up to a megabyte left to the runtime, 873 this way).  So they are kept here when they are given back, up to
-// kPoolBytes and kPoolPieces a process,
-// and go to the next that asks for about as much on that device; at a bound the oldest are freed (a quarter of the pieces at a time: the first of
-// those frees waits for the device), and all
+// 1066 us a pass with pieces of up to a megabyte left to the runtime, 912 this way).  So they are kept here when they are given back, up to
+// kPoolBytes and kPoolPieces a process, and go to the next that asks for about as much on that device; at a bound the oldest are freed (a
+// quarter of the pieces at a time: the first of those frees waits for the device), and all
 // of it when an allocation fails or the host program asks for it (tw_release_memory).  Kernels of a plan that is destroyed may still be queued, on any
 // stream or in a graph: its piece is handed out again only behind a wait for the whole device, made by
 // the build that takes it (a build waits anyway) and not by the destruction, which may come in the
