@@ -27,10 +27,8 @@ int main()
                 for (int most : {0, 1, 3, 16, 17}) {
                     SkinnyWork w{};
                     skinny_fill(&w, n_tiles, M, rm, 512);
-                    if (most && w.fill_wgs > most) {
+                    if (most && w.fill_wgs > most)
                         w.fill_wgs = most;
-                        w.step_z = most / w.n_fillblk, w.step_blk = most % w.n_fillblk;
-                    }
                     std::vector<int> seen((size_t)n_tiles * w.n_fillblk, 0);
                     for (int wg = 0; wg < w.fill_wgs; ++wg)
                         for (FillPlace at = fill_first(w, wg); at.z < n_tiles; at = fill_next(w, at))
